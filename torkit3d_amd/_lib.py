@@ -1,4 +1,6 @@
-"""ctypes loader for ``libtk3d.so`` (the hand-written HIP kernels behind a C ABI).
+"""ctypes access to ``libtk3d.so`` (the hand-written HIP kernels behind a C ABI), for callers of
+single entry points: the tests, the benchmark and the smoke run. The operators go through the
+extension module ``_native``.
 
 There is no CPU fallback: if the library is missing or a call fails, an exception
 is raised.
@@ -89,40 +91,12 @@ def chamfer_workspace_bytes(b, n1, n2, always=False):
     return int(_chamfer_workspace_fn(i64(b), i64(n1), i64(n2), ctypes.c_int(1 if always else 0)))
 
 
-ERR_UNSUPPORTED = -6  # TK3D_ERR_UNSUPPORTED
-
-
-def call(name, tensor_for_dtype, *args, may_decline=False):
-    """Call ``name`` + the dtype suffix and raise on an error code. With ``may_decline`` a
-    TK3D_ERR_UNSUPPORTED return (nothing was launched) is handed back as False instead."""
+def call(name, tensor_for_dtype, *args):
+    """Call ``name`` + the dtype suffix and raise on an error code."""
     key = (name, tensor_for_dtype.dtype)
     fn = _functions.get(key)
     if fn is None:
         fn = getattr(lib(), name + suffix(tensor_for_dtype))
         fn.restype = ctypes.c_int
         _functions[key] = fn
-    code = fn(*args)
-    if may_decline and code == ERR_UNSUPPORTED:
-        return False
-    check(code, name)
-    return True
-
-
-class _NoSwitch:
-    def __enter__(self):
-        return None
-
-    def __exit__(self, *exc):
-        return False
-
-
-_NO_SWITCH = _NoSwitch()
-
-
-def on_device_of(t):
-    """Context in which the tensor's GPU is current (kernels, allocations and streams
-    follow the current device). Switching costs a few microseconds per call, so nothing
-    is done when that GPU is current already."""
-    if t.device.index == torch.cuda.current_device():
-        return _NO_SWITCH
-    return torch.cuda.device(t.device)
+    check(fn(*args), name)

@@ -13,6 +13,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 REPO = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB_PATH = os.path.join(HERE, "libtk3d.so")
+NATIVE_PATH = os.path.join(HERE, "_host.so")
 
 # -ffp-contract=off: the only fused multiply-adds are the ones the sources spell.
 # -packed-fp32-ops is switched off for the device pass (the host pass does not
@@ -100,5 +101,39 @@ def build(verbose=False, jobs=None):
     return LIB_PATH
 
 
+def build_native(verbose=False):
+    """Compile the Python extension with the operators' host path (``csrc/native.cpp``) against
+    the installed torch and ``libtk3d.so``, which it finds beside itself."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared",
+           "-fvisibility=hidden", "-Wall", "-Wno-deprecated-declarations",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-DTORCH_EXTENSION_NAME=_host",
+           "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI),
+           "-I", os.path.join(REPO, "include"), "-I", sysconfig.get_paths()["include"]]
+    rocm = os.path.dirname(os.path.dirname(hipcc_path()))
+    for path in cpp_extension.include_paths() + [os.path.join(rocm, "include"),
+                                                 "/opt/rocm/include"]:
+        cmd += ["-isystem", path]
+    cmd += [os.path.join(CSRC, "native.cpp"), "-o", NATIVE_PATH + ".tmp", "-L", HERE,
+            "-l:" + os.path.basename(LIB_PATH),
+            "-L", torch_lib, "-ltorch_python", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10",
+            "-lc10_hip", "-Wl,-rpath,$ORIGIN"]
+    if verbose:
+        print(" ".join(cmd))
+    res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if res.returncode != 0:
+        raise RuntimeError("building _host.so failed:\n" + res.stdout)
+    if verbose and res.stdout.strip():
+        print(res.stdout)
+    os.replace(NATIVE_PATH + ".tmp", NATIVE_PATH)
+    return NATIVE_PATH
+
+
 if __name__ == "__main__":
     print(build(verbose="-v" in sys.argv))
+    print(build_native(verbose="-v" in sys.argv))

@@ -1,0 +1,667 @@
+// Host path of the operators: argument checks, output allocation, autograd nodes and the calls
+// into the C ABI (include/tk3d.h), as a Python extension module (torkit3d_amd/_host.so).
+// A small call is host work only: through ctypes and Python's autograd.Function a chamfer
+// forward + backward on 2 x 1024 points took 100 to 160 us around 27 us of kernels.
+#include <algorithm>
+#include <optional>
+#include <stdexcept>
+#include <string>
+#include <tuple>
+#include <vector>
+
+#include <ATen/ATen.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/core/GradMode.h>
+#include <c10/hip/HIPStream.h>
+#include <pybind11/pybind11.h>
+#include <pybind11/stl.h>
+#include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/utils/pybind.h>
+
+#include "tk3d.h"
+
+namespace py = pybind11;
+using at::Tensor;
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+namespace {
+
+// ---- checks (messages as the reference's TORCH_CHECKs give them; RuntimeError in Python) ----
+
+[[noreturn]] void fail(const std::string &message) { throw std::runtime_error(message); }
+
+void check(bool ok, const std::string &message)
+{
+    if (!ok)
+        fail(message);
+}
+
+void check_eq(int64_t a, int64_t b, const char *what)
+{
+    if (a != b)
+        fail("Check failed: " + std::string(what) + " (" + std::to_string(a) + " vs. " +
+             std::to_string(b) + ")");
+}
+
+Tensor tensor_arg(const char *name, py::handle h)
+{
+    if (!THPVariable_Check(h.ptr()))
+        fail(std::string(name) + " must be a tensor.");
+    return THPVariable_Unpack(h.ptr());
+}
+
+void check_cuda(const char *name, const Tensor &t)
+{
+    if (!t.is_cuda())
+        fail(std::string(name) + " must be a CUDA tensor.");
+}
+
+void check_contiguous_cuda(const char *name, const Tensor &t)
+{
+    check_cuda(name, t);
+    if (!t.is_contiguous())
+        fail(std::string(name) + " must be contiguous.");
+}
+
+void check_index(const char *name, const Tensor &t)
+{
+    if (t.scalar_type() != at::kLong)
+        fail(std::string(name) + " must be an int64 tensor.");
+}
+
+void check_same(const char *a_name, const Tensor &a, const char *b_name, const Tensor &b)
+{
+    if (a.scalar_type() != b.scalar_type())
+        fail(std::string(a_name) + " and " + b_name + " must have the same dtype.");
+    if (a.device() != b.device())
+        fail(std::string(a_name) + " and " + b_name + " must be on the same device.");
+}
+
+// float32 (true) or float64 (false); anything else is an error.
+bool is_f32(const Tensor &t)
+{
+    if (t.scalar_type() == at::kFloat)
+        return true;
+    if (t.scalar_type() != at::kDouble)
+        fail(std::string("torkit3d_amd supports float32 and float64 tensors, got ") +
+             c10::toString(t.scalar_type()));
+    return false;
+}
+
+void done(int code, const char *what)
+{
+    if (code != TK3D_OK)
+        fail(std::string(what) + " failed: " + tk3d_error_string(code) + " (code " +
+             std::to_string(code) + ")");
+}
+
+// ---- device pointers, outputs, stream ---------------------------------------------------------
+
+struct Ptr {  // becomes whatever pointer the entry point takes
+    void *p;
+    template <typename T> operator T *() const { return static_cast<T *>(p); }
+};
+
+Ptr ptr(const Tensor &t)
+{
+    return {t.defined() && t.numel() > 0 ? const_cast<void *>(t.const_data_ptr()) : nullptr};
+}
+
+Tensor like(const Tensor &t, at::IntArrayRef shape) { return at::empty(shape, t.options()); }
+
+Tensor index_like(const Tensor &t, at::IntArrayRef shape)
+{
+    return at::empty(shape, t.options().dtype(at::kLong));
+}
+
+Tensor scratch(const Tensor &t, size_t bytes)
+{
+    return bytes ? at::empty({(int64_t)bytes}, t.options().dtype(at::kByte)) : Tensor();
+}
+
+void *stream_of(const Tensor &t)
+{
+    return c10::hip::getCurrentHIPStream(t.device().index()).stream();
+}
+
+// Makes the tensor's GPU the current one (kernels, allocations and streams follow it).
+using OnDeviceOf = c10::OptionalDeviceGuard;
+
+#define TK3D_CALL(is32, name, ...)                                                             \
+    done((is32) ? name##_f32(__VA_ARGS__) : name##_f64(__VA_ARGS__), #name)
+
+// ---- operators ---------------------------------------------------------------------------------
+
+struct Cloud {
+    int64_t b, n;
+};
+
+Cloud cloud_dims(const char *name, const Tensor &t, bool channels_first)
+{
+    check_contiguous_cuda(name, t);
+    check_eq(t.dim(), 3, (std::string(name) + ".dim() == 3").c_str());
+    check_eq(t.size(channels_first ? 1 : 2), 3,
+             (std::string(name) + (channels_first ? ".size(1) == 3" : ".size(2) == 3")).c_str());
+    return {t.size(0), t.size(channels_first ? 2 : 1)};
+}
+
+std::tuple<Tensor, Tensor> fps(const Tensor &points, int64_t num_samples, bool channels_first,
+                               bool want_xyz)
+{
+    const Cloud c = cloud_dims("points", points, channels_first);
+    check(num_samples > 0,
+          "Check failed: num_samples > 0 (" + std::to_string(num_samples) + " vs. 0)");
+    check(c.n >= num_samples, "Check failed: points.size(1) >= num_samples (" +
+                                  std::to_string(c.n) + " vs. " + std::to_string(num_samples) + ")");
+    OnDeviceOf guard(points.device());
+    const Tensor index = index_like(points, {c.b, num_samples});
+    Tensor sampled;
+    if (want_xyz)
+        sampled = channels_first ? like(points, {c.b, 3, num_samples})
+                                 : like(points, {c.b, num_samples, 3});
+    const size_t bytes =
+        tk3d_sample_farthest_points_workspace_bytes(c.b, c.n, points.element_size());
+    const Tensor ws = scratch(points, bytes);
+    TK3D_CALL(is_f32(points), tk3d_sample_farthest_points_gather, ptr(points), channels_first, c.b,
+              c.n, num_samples, ptr(index), ptr(sampled), ptr(ws), bytes, stream_of(points));
+    return {index, sampled};
+}
+
+Tensor ball_query(const Tensor &query, const Tensor &key, double radius, int64_t max_neighbors,
+                  bool channels_first)
+{
+    const Cloud q = cloud_dims("query", query, channels_first);
+    const Cloud k = cloud_dims("key", key, channels_first);
+    check_eq(q.b, k.b, "query.size(0) == key.size(0)");
+    check_same("query", query, "key", key);
+    check(max_neighbors >= 0, "max_neighbors must be non-negative.");
+    OnDeviceOf guard(query.device());
+    const Tensor index = index_like(query, {q.b, q.n, max_neighbors});
+    if (channels_first)
+        TK3D_CALL(is_f32(query), tk3d_ball_query_bcn, ptr(query), ptr(key), q.b, q.n, k.n,
+                  (float)radius, max_neighbors, ptr(index), stream_of(query));
+    else
+        TK3D_CALL(is_f32(query), tk3d_ball_query, ptr(query), ptr(key), q.b, q.n, k.n,
+                  (float)radius, max_neighbors, ptr(index), stream_of(query));
+    return index;
+}
+
+// Empty when the library has no kernel for this k on [B,3,N] clouds (k > 64).
+std::vector<Tensor> knn(const Tensor &query, const Tensor &key, int64_t k, int64_t version,
+                        bool channels_first)
+{
+    const Cloud q = cloud_dims("query", query, channels_first);
+    const Cloud c = cloud_dims("key", key, channels_first);
+    check_eq(c.b, q.b, "key.size(0) == query.size(0)");
+    check(c.n >= k, "Check failed: key.size(1) >= k (" + std::to_string(c.n) + " vs. " +
+                        std::to_string(k) + ")");
+    check_same("query", query, "key", key);
+    check(version == 0 || version == 1, "Invalid version");
+    check(k >= 0, "k must be non-negative.");
+    if (channels_first && k > 64)
+        return {};
+    OnDeviceOf guard(query.device());
+    const Tensor distance = like(query, {q.b, q.n, k});
+    const Tensor index = index_like(query, {q.b, q.n, k});
+    if (k > 0 && channels_first) {
+        const int code =
+            is_f32(query)
+                ? tk3d_knn_distance_bcn_f32(ptr(query), ptr(key), q.b, q.n, c.n, k, (int)version,
+                                            ptr(distance), ptr(index), stream_of(query))
+                : tk3d_knn_distance_bcn_f64(ptr(query), ptr(key), q.b, q.n, c.n, k, (int)version,
+                                            ptr(distance), ptr(index), stream_of(query));
+        if (code == TK3D_ERR_UNSUPPORTED)
+            return {};
+        done(code, "tk3d_knn_distance_bcn");
+    } else if (k > 0) {
+        TK3D_CALL(is_f32(query), tk3d_knn_distance, ptr(query), ptr(key), q.b, q.n, c.n, k,
+                  (int)version, ptr(distance), ptr(index), stream_of(query));
+    }
+    return {distance, index};
+}
+
+std::tuple<Tensor, Tensor, Tensor> three_nn(const Tensor &query, const Tensor &key,
+                                            bool channels_first, double eps)
+{
+    const Cloud q = cloud_dims("query", query, channels_first);
+    const Cloud c = cloud_dims("key", key, channels_first);
+    check_eq(q.b, c.b, "query.size(0) == key.size(0)");
+    check_same("query", query, "key", key);
+    check(c.n >= 3, "Check failed: key.size(1) >= k (" + std::to_string(c.n) + " vs. 3)");
+    OnDeviceOf guard(query.device());
+    const Tensor distance = like(query, {q.b, q.n, 3});
+    const Tensor index = index_like(query, {q.b, q.n, 3});
+    const Tensor weight = like(query, {q.b, q.n, 3});
+    TK3D_CALL(is_f32(query), tk3d_three_nn, ptr(query), ptr(key), channels_first, q.b, q.n, c.n,
+              eps, ptr(distance), ptr(index), ptr(weight), stream_of(query));
+    return {distance, index, weight};
+}
+
+std::vector<Tensor> chamfer_forward(const Tensor &xyz1, const Tensor &xyz2, bool channels_first)
+{
+    const Cloud a = cloud_dims("xyz1", xyz1, channels_first);
+    const Cloud c = cloud_dims("xyz2", xyz2, channels_first);
+    check_eq(a.b, c.b, "xyz1.size(0) == xyz2.size(0)");
+    check_same("xyz1", xyz1, "xyz2", xyz2);
+    OnDeviceOf guard(xyz1.device());
+    const Tensor dist1 = like(xyz1, {a.b, a.n}), idx1 = index_like(xyz1, {a.b, a.n});
+    const Tensor dist2 = like(xyz1, {a.b, c.n}), idx2 = index_like(xyz1, {a.b, c.n});
+    void *stream = stream_of(xyz1);
+    if (is_f32(xyz1)) {
+        // Clouds of a few thousand points and more are sorted along a space-filling curve in a
+        // scratch buffer, and only key tiles near a wave's queries are swept. (On [B,3,N]
+        // clouds the sorted path goes up to 16384 points.)
+        const bool sortable = !channels_first || std::max(a.n, c.n) <= 16384;
+        const size_t bytes =
+            sortable ? tk3d_chamfer_distance_forward_workspace_bytes(a.b, a.n, c.n, 0) : 0;
+        const Tensor ws = scratch(xyz1, bytes);
+        const auto call = channels_first ? tk3d_chamfer_distance_forward_bcn_f32
+                                         : tk3d_chamfer_distance_forward_ws_f32;
+        done(call(ptr(xyz1), ptr(xyz2), a.b, a.n, c.n, ptr(dist1), ptr(idx1), ptr(dist2),
+                  ptr(idx2), ptr(ws), bytes, stream),
+             "tk3d_chamfer_distance_forward_f32");
+    } else {
+        const auto call = channels_first ? tk3d_chamfer_distance_forward_bcn_f64
+                                         : tk3d_chamfer_distance_forward_f64;
+        done(call(ptr(xyz1), ptr(xyz2), a.b, a.n, c.n, ptr(dist1), ptr(idx1), ptr(dist2),
+                  ptr(idx2), stream),
+             "tk3d_chamfer_distance_forward_f64");
+    }
+    return {dist1, idx1, dist2, idx2};
+}
+
+std::vector<Tensor> chamfer_backward(const Tensor &grad1, const Tensor &grad2, const Tensor &xyz1,
+                                     const Tensor &xyz2, const Tensor &idx1, const Tensor &idx2)
+{
+    check_contiguous_cuda("grad_dist1", grad1);
+    check_contiguous_cuda("grad_dist2", grad2);
+    check_contiguous_cuda("xyz1", xyz1);
+    check_contiguous_cuda("xyz2", xyz2);
+    check_contiguous_cuda("idx1", idx1);
+    check_contiguous_cuda("idx2", idx2);
+    check(grad1.dim() == 2 && grad2.dim() == 2, "grad_dist must be 2-D tensors.");
+    const int64_t b = grad1.size(0), n1 = grad1.size(1), n2 = grad2.size(1);
+    check_eq(grad2.size(0), b, "grad_dist2.size(0) == bs");
+    check(xyz1.dim() == 3 && xyz2.dim() == 3, "xyz1 and xyz2 must be 3-D tensors.");
+    check_eq(xyz1.size(0), b, "xyz1.size(0) == bs");
+    check_eq(xyz2.size(0), b, "xyz2.size(0) == bs");
+    check_eq(xyz1.size(1), n1, "xyz1.size(1) == n1");
+    check_eq(xyz2.size(1), n2, "xyz2.size(1) == n2");
+    check_eq(xyz1.size(2), 3, "xyz1.size(2) == 3");
+    check_eq(xyz2.size(2), 3, "xyz2.size(2) == 3");
+    check(idx1.dim() == 2 && idx2.dim() == 2, "idx1 and idx2 must be 2-D tensors.");
+    check_eq(idx1.size(0), b, "idx1.size(0) == bs");
+    check_eq(idx2.size(0), b, "idx2.size(0) == bs");
+    check_eq(idx1.size(1), n1, "idx1.size(1) == n1");
+    check_eq(idx2.size(1), n2, "idx2.size(1) == n2");
+    check_index("idx1", idx1);
+    check_index("idx2", idx2);
+    check_same("grad_dist1", grad1, "xyz1", xyz1);
+    check_same("grad_dist2", grad2, "xyz2", xyz2);
+    check_same("xyz1", xyz1, "xyz2", xyz2);
+    OnDeviceOf guard(xyz1.device());
+    const Tensor grad_xyz1 = like(xyz1, {b, n1, 3}), grad_xyz2 = like(xyz1, {b, n2, 3});
+    TK3D_CALL(is_f32(xyz1), tk3d_chamfer_distance_backward, ptr(grad1), ptr(grad2), ptr(xyz1),
+              ptr(xyz2), ptr(idx1), ptr(idx2), b, n1, n2, ptr(grad_xyz1), ptr(grad_xyz2),
+              stream_of(xyz1));
+    return {grad_xyz1, grad_xyz2};
+}
+
+// Like the reference (which goes through at::gather) non-contiguous tensors are accepted.
+Tensor group_forward(const Tensor &input_, const Tensor &index_)
+{
+    check_cuda("input", input_);
+    check_cuda("index", index_);
+    check_eq(input_.dim(), 3, "input.dim() == 3");
+    check_eq(index_.dim(), 3, "index.dim() == 3");
+    check_eq(input_.size(0), index_.size(0), "input.size(0) == index.size(0)");
+    check_index("index", index_);
+    OnDeviceOf guard(input_.device());
+    const Tensor input = input_.contiguous(), index = index_.contiguous();
+    const int64_t b = input.size(0), c = input.size(1), n2 = index.size(1), k = index.size(2);
+    const Tensor output = like(input, {b, c, n2, k});
+    TK3D_CALL(is_f32(input), tk3d_group_points_forward, ptr(input), ptr(index), b, c,
+              input.size(2), n2, k, ptr(output), stream_of(input));
+    return output;
+}
+
+void check_grouped_grad(const Tensor &grad, const Tensor &index)
+{
+    check_contiguous_cuda("grad_output", grad);
+    check_contiguous_cuda("index", index);
+    check_eq(grad.dim(), 4, "grad_output.dim() == 4");
+    check_eq(index.dim(), 3, "index.dim() == 3");
+    check_eq(index.size(0), grad.size(0), "index.size(0) == grad_output.size(0)");
+    check_eq(index.size(1), grad.size(2), "index.size(1) == grad_output.size(2)");
+    check_eq(index.size(2), grad.size(3), "index.size(2) == grad_output.size(3)");
+    check_index("index", index);
+}
+
+Tensor group_backward(const Tensor &grad, const Tensor &index, int64_t n1)
+{
+    check_grouped_grad(grad, index);
+    OnDeviceOf guard(grad.device());
+    const Tensor out = like(grad, {grad.size(0), grad.size(1), n1});
+    TK3D_CALL(is_f32(grad), tk3d_group_points_backward, ptr(grad), ptr(index), grad.size(0),
+              grad.size(1), n1, grad.size(2), grad.size(3), ptr(out), stream_of(grad));
+    return out;
+}
+
+Tensor group_concat_forward(const Tensor &feature, const Tensor &xyz, const Tensor &centre,
+                            const Tensor &index)
+{
+    const Cloud p = cloud_dims("xyz", xyz, true);
+    const Cloud m = cloud_dims("centre", centre, true);
+    check_eq(p.b, m.b, "xyz.size(0) == centre.size(0)");
+    check_same("xyz", xyz, "centre", centre);
+    check_contiguous_cuda("index", index);
+    check_index("index", index);
+    check_eq(index.dim(), 3, "index.dim() == 3");
+    check_eq(index.size(0), p.b, "index.size(0) == xyz.size(0)");
+    check_eq(index.size(1), m.n, "index.size(1) == centre.size(2)");
+    int64_t c = 0;
+    if (feature.defined()) {
+        check_contiguous_cuda("feature", feature);
+        check_eq(feature.dim(), 3, "feature.dim() == 3");
+        check_eq(feature.size(0), p.b, "feature.size(0) == xyz.size(0)");
+        check_eq(feature.size(2), p.n, "feature.size(2) == xyz.size(2)");
+        check_same("feature", feature, "xyz", xyz);
+        c = feature.size(1);
+    }
+    OnDeviceOf guard(xyz.device());
+    const Tensor out = like(xyz, {p.b, c + 3, m.n, index.size(2)});
+    TK3D_CALL(is_f32(xyz), tk3d_group_points_concat_forward, ptr(feature), ptr(xyz), ptr(centre),
+              ptr(index), p.b, c, p.n, m.n, index.size(2), ptr(out), stream_of(xyz));
+    return out;
+}
+
+std::tuple<Tensor, Tensor> group_concat_backward(const Tensor &grad, const Tensor &index,
+                                                 int64_t n1, bool want_feature, bool want_xyz)
+{
+    check_grouped_grad(grad, index);
+    const int64_t b = grad.size(0), c = grad.size(1) - 3;
+    check(c >= 0, "grad_output must have at least 3 channels.");
+    OnDeviceOf guard(grad.device());
+    Tensor feature, xyz;
+    if (want_feature && c > 0)
+        feature = like(grad, {b, c, n1});
+    if (want_xyz)
+        xyz = like(grad, {b, 3, n1});
+    if (feature.defined() || xyz.defined())
+        TK3D_CALL(is_f32(grad), tk3d_group_points_concat_backward, ptr(grad), ptr(index), b, c, n1,
+                  grad.size(2), grad.size(3), ptr(feature), ptr(xyz), stream_of(grad));
+    return {feature, xyz};
+}
+
+void check_interpolate(const char *name, const Tensor &first, const Tensor &index,
+                       const Tensor &weight)
+{
+    const std::string n(name);
+    check_contiguous_cuda(name, first);
+    check_contiguous_cuda("index", index);
+    check_contiguous_cuda("weight", weight);
+    check_eq(first.dim(), 3, (n + ".dim() == 3").c_str());
+    check_eq(index.dim(), 3, "index.dim() == 3");
+    check_eq(weight.dim(), 3, "weight.dim() == 3");
+    check_eq(first.size(0), index.size(0), (n + ".size(0) == index.size(0)").c_str());
+    check_eq(first.size(0), weight.size(0), (n + ".size(0) == weight.size(0)").c_str());
+    check_eq(index.size(1), weight.size(1), "index.size(1) == weight.size(1)");
+    check_eq(index.size(2), weight.size(2), "index.size(2) == weight.size(2)");
+    check_index("index", index);
+    check_same(name, first, "weight", weight);
+}
+
+Tensor interpolate_forward(const Tensor &input, const Tensor &index, const Tensor &weight)
+{
+    check_interpolate("input", input, index, weight);
+    check_eq(index.size(2), 3, "index.size(2) == 3");
+    OnDeviceOf guard(input.device());
+    const Tensor out = like(input, {input.size(0), input.size(1), index.size(1)});
+    TK3D_CALL(is_f32(input), tk3d_interpolate_forward, ptr(input), ptr(index), ptr(weight),
+              input.size(0), input.size(1), input.size(2), index.size(1), index.size(2), ptr(out),
+              stream_of(input));
+    return out;
+}
+
+Tensor interpolate_backward(const Tensor &grad, const Tensor &index, const Tensor &weight,
+                            int64_t n1)
+{
+    check_interpolate("grad_output", grad, index, weight);
+    check_eq(grad.size(2), index.size(1), "grad_output.size(2) == index.size(1)");
+    check(index.size(2) == 3, "Only support k=3.");
+    OnDeviceOf guard(grad.device());
+    const Tensor out = like(grad, {grad.size(0), grad.size(1), n1});
+    TK3D_CALL(is_f32(grad), tk3d_interpolate_backward, ptr(grad), ptr(index), ptr(weight),
+              grad.size(0), grad.size(1), n1, grad.size(2), index.size(2), ptr(out),
+              stream_of(grad));
+    return out;
+}
+
+// ---- autograd nodes ------------------------------------------------------------------------------
+
+bool tracked(const Tensor &t) { return t.defined() && t.requires_grad(); }
+
+struct ChamferNode : torch::autograd::Function<ChamferNode> {
+    static variable_list forward(AutogradContext *ctx, const Tensor &xyz1, const Tensor &xyz2,
+                                 bool channels_first)
+    {
+        const std::vector<Tensor> out =
+            chamfer_forward(xyz1.contiguous(), xyz2.contiguous(), channels_first);
+        ctx->save_for_backward({xyz1.contiguous(), xyz2.contiguous(), out[1], out[3]});
+        ctx->saved_data["channels_first"] = channels_first;
+        return {out[0], out[2]};
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grads)
+    {
+        const variable_list saved = ctx->get_saved_variables();
+        if (!ctx->saved_data["channels_first"].toBool()) {
+            const std::vector<Tensor> g =
+                chamfer_backward(grads[0].contiguous(), grads[1].contiguous(), saved[0], saved[1],
+                                 saved[2], saved[3]);
+            return {g[0], g[1], Tensor()};
+        }
+        // (the backward kernel works on [B,N,3])
+        const std::vector<Tensor> g = chamfer_backward(
+            grads[0].contiguous(), grads[1].contiguous(), saved[0].transpose(1, 2).contiguous(),
+            saved[1].transpose(1, 2).contiguous(), saved[2], saved[3]);
+        return {g[0].transpose(1, 2), g[1].transpose(1, 2), Tensor()};
+    }
+};
+
+std::tuple<Tensor, Tensor> chamfer(const Tensor &xyz1, const Tensor &xyz2, bool channels_first)
+{
+    if (c10::GradMode::is_enabled() && (tracked(xyz1) || tracked(xyz2))) {
+        const variable_list out = ChamferNode::apply(xyz1, xyz2, channels_first);
+        return {out[0], out[1]};
+    }
+    const std::vector<Tensor> out =
+        chamfer_forward(xyz1.contiguous(), xyz2.contiguous(), channels_first);
+    return {out[0], out[2]};
+}
+
+struct GroupNode : torch::autograd::Function<GroupNode> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &points, const Tensor &index)
+    {
+        ctx->save_for_backward({index});
+        ctx->saved_data["n"] = points.size(2);
+        return group_forward(points, index);
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grads)
+    {
+        const variable_list saved = ctx->get_saved_variables();
+        return {group_backward(grads[0].contiguous(), saved[0].contiguous(),
+                               ctx->saved_data["n"].toInt()),
+                Tensor()};
+    }
+};
+
+Tensor group_points(const Tensor &points, const Tensor &index)
+{
+    if (c10::GradMode::is_enabled() && tracked(points))
+        return GroupNode::apply(points, index);
+    return group_forward(points, index);
+}
+
+struct GroupConcatNode : torch::autograd::Function<GroupConcatNode> {
+    static Tensor forward(AutogradContext *ctx, const std::optional<Tensor> &maybe_feature,
+                          const Tensor &xyz, const Tensor &centre, const Tensor &index)
+    {
+        const Tensor feature = maybe_feature.value_or(Tensor());
+        ctx->save_for_backward({index});
+        ctx->saved_data["n"] = xyz.size(2);
+        ctx->saved_data["feature"] = feature.defined() && feature.requires_grad();
+        ctx->saved_data["xyz"] = xyz.requires_grad();
+        ctx->saved_data["centre"] = centre.requires_grad();
+        return group_concat_forward(feature.defined() ? feature.contiguous() : feature,
+                                    xyz.contiguous(), centre.contiguous(), index.contiguous());
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grads)
+    {
+        const variable_list saved = ctx->get_saved_variables();
+        const Tensor grad = grads[0].contiguous();
+        auto [feature, xyz] = group_concat_backward(
+            grad, saved[0].contiguous(), ctx->saved_data["n"].toInt(),
+            ctx->saved_data["feature"].toBool(), ctx->saved_data["xyz"].toBool());
+        Tensor centre;
+        if (ctx->saved_data["centre"].toBool())
+            centre = grad.narrow(1, grad.size(1) - 3, 3).sum(3).neg();
+        return {feature, xyz, centre, Tensor()};
+    }
+};
+
+Tensor group_points_with_xyz(const Tensor &feature, const Tensor &xyz, const Tensor &centre,
+                             const Tensor &index)
+{
+    if (c10::GradMode::is_enabled() && (tracked(feature) || tracked(xyz) || tracked(centre)))
+        return GroupConcatNode::apply(
+            feature.defined() ? std::optional<Tensor>(feature) : std::nullopt, xyz, centre, index);
+    return group_concat_forward(feature.defined() ? feature.contiguous() : feature,
+                                xyz.contiguous(), centre.contiguous(), index.contiguous());
+}
+
+struct InterpolateNode : torch::autograd::Function<InterpolateNode> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &feature, const Tensor &index,
+                          const Tensor &weight)
+    {
+        ctx->save_for_backward({index, weight});
+        ctx->saved_data["n"] = feature.size(2);
+        return interpolate_forward(feature.contiguous(), index.contiguous(), weight.contiguous());
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grads)
+    {
+        const variable_list saved = ctx->get_saved_variables();
+        return {interpolate_backward(grads[0].contiguous(), saved[0].contiguous(),
+                                     saved[1].contiguous(), ctx->saved_data["n"].toInt()),
+                Tensor(), Tensor()};
+    }
+};
+
+Tensor interpolate(const Tensor &feature, const Tensor &index, const Tensor &weight)
+{
+    if (c10::GradMode::is_enabled() && (tracked(feature) || tracked(weight)))
+        return InterpolateNode::apply(feature, index, weight);
+    return interpolate_forward(feature.contiguous(), index.contiguous(), weight.contiguous());
+}
+
+// ---- Python ----------------------------------------------------------------------------------------
+
+Tensor optional_arg(const char *name, py::handle h)
+{
+    return h.is_none() ? Tensor() : tensor_arg(name, h);
+}
+
+// Runs an operator without the interpreter lock.
+template <typename F> auto unlocked(F &&f)
+{
+    py::gil_scoped_release release;
+    return f();
+}
+
+}  // namespace
+
+PYBIND11_MODULE(_host, m)
+{
+    m.def("sample_farthest_points",
+          [](py::handle points, int64_t k, bool channels_first, bool want_xyz) {
+              const Tensor p = tensor_arg("points", points);
+              return unlocked([&] { return fps(p, k, channels_first, want_xyz); });
+          });
+    m.def("ball_query", [](py::handle query, py::handle key, double radius, int64_t k,
+                           bool channels_first) {
+        const Tensor q = tensor_arg("query", query), c = tensor_arg("key", key);
+        return unlocked([&] { return ball_query(q, c, radius, k, channels_first); });
+    });
+    m.def("knn", [](py::handle query, py::handle key, int64_t k, int64_t version,
+                    bool channels_first) {
+        const Tensor q = tensor_arg("query", query), c = tensor_arg("key", key);
+        return unlocked([&] { return knn(q, c, k, version, channels_first); });
+    });
+    m.def("three_nn", [](py::handle query, py::handle key, bool channels_first, double eps) {
+        const Tensor q = tensor_arg("query", query), c = tensor_arg("key", key);
+        return unlocked([&] { return three_nn(q, c, channels_first, eps); });
+    });
+    m.def("chamfer_forward", [](py::handle xyz1, py::handle xyz2, bool channels_first) {
+        const Tensor a = tensor_arg("xyz1", xyz1), c = tensor_arg("xyz2", xyz2);
+        return unlocked([&] { return chamfer_forward(a, c, channels_first); });
+    });
+    m.def("chamfer_backward", [](py::handle grad1, py::handle grad2, py::handle xyz1,
+                                 py::handle xyz2, py::handle idx1, py::handle idx2) {
+        const Tensor t[] = {tensor_arg("grad_dist1", grad1), tensor_arg("grad_dist2", grad2),
+                            tensor_arg("xyz1", xyz1),        tensor_arg("xyz2", xyz2),
+                            tensor_arg("idx1", idx1),        tensor_arg("idx2", idx2)};
+        return unlocked([&] { return chamfer_backward(t[0], t[1], t[2], t[3], t[4], t[5]); });
+    });
+    m.def("group_forward", [](py::handle input, py::handle index) {
+        const Tensor x = tensor_arg("input", input), i = tensor_arg("index", index);
+        return unlocked([&] { return group_forward(x, i); });
+    });
+    m.def("group_backward", [](py::handle grad, py::handle index, int64_t n1) {
+        const Tensor g = tensor_arg("grad_output", grad), i = tensor_arg("index", index);
+        return unlocked([&] { return group_backward(g, i, n1); });
+    });
+    m.def("group_concat_forward", [](py::handle feature, py::handle xyz, py::handle centre,
+                                     py::handle index) {
+        const Tensor f = optional_arg("feature", feature), x = tensor_arg("xyz", xyz),
+                     c = tensor_arg("centre", centre), i = tensor_arg("index", index);
+        return unlocked([&] { return group_concat_forward(f, x, c, i); });
+    });
+    m.def("group_concat_backward", [](py::handle grad, py::handle index, int64_t n1,
+                                      bool want_feature, bool want_xyz) {
+        const Tensor g = tensor_arg("grad_output", grad), i = tensor_arg("index", index);
+        return unlocked([&] { return group_concat_backward(g, i, n1, want_feature, want_xyz); });
+    });
+    m.def("interpolate_forward", [](py::handle input, py::handle index, py::handle weight) {
+        const Tensor x = tensor_arg("input", input), i = tensor_arg("index", index),
+                     w = tensor_arg("weight", weight);
+        return unlocked([&] { return interpolate_forward(x, i, w); });
+    });
+    m.def("interpolate_backward", [](py::handle grad, py::handle index, py::handle weight,
+                                     int64_t n1) {
+        const Tensor g = tensor_arg("grad_output", grad), i = tensor_arg("index", index),
+                     w = tensor_arg("weight", weight);
+        return unlocked([&] { return interpolate_backward(g, i, w, n1); });
+    });
+
+    // differentiable forms
+    m.def("chamfer", [](py::handle xyz1, py::handle xyz2, bool channels_first) {
+        const Tensor a = tensor_arg("xyz1", xyz1), c = tensor_arg("xyz2", xyz2);
+        return unlocked([&] { return chamfer(a, c, channels_first); });
+    });
+    m.def("group_points", [](py::handle points, py::handle index) {
+        const Tensor x = tensor_arg("input", points), i = tensor_arg("index", index);
+        return unlocked([&] { return group_points(x, i); });
+    });
+    m.def("group_points_with_xyz", [](py::handle feature, py::handle xyz, py::handle centre,
+                                      py::handle index) {
+        const Tensor f = optional_arg("feature", feature), x = tensor_arg("xyz", xyz),
+                     c = tensor_arg("centre", centre), i = tensor_arg("index", index);
+        return unlocked([&] { return group_points_with_xyz(f, x, c, i); });
+    });
+    m.def("interpolate", [](py::handle feature, py::handle index, py::handle weight) {
+        const Tensor x = tensor_arg("input", feature), i = tensor_arg("index", index),
+                     w = tensor_arg("weight", weight);
+        return unlocked([&] { return interpolate(x, i, w); });
+    });
+}

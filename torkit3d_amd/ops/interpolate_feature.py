@@ -1,7 +1,7 @@
 """Weighted feature interpolation (API of torkit3d/ops/interpolate_feature.py)."""
 import torch
 
-from .. import _C, _fused
+from .. import _C, _native
 
 
 class InterpolateFeature(torch.autograd.Function):
@@ -26,7 +26,7 @@ class InterpolateFeature(torch.autograd.Function):
 def interpolate_feature(feature, index, weight):
     """feature [B, C, N1], index [B, N2, K], weight [B, N2, K] -> [B, C, N2] with
     out[b, c, n] = sum_i feature[b, c, index[b, n, i]] * weight[b, n, i]."""
-    return InterpolateFeature.apply(feature, index, weight)
+    return _native.interpolate(feature, index, weight)
 
 
 def three_nn_weights(distance, eps=1e-10):
@@ -49,7 +49,7 @@ def three_nn_interpolation(query_xyz, key_xyz, transpose=False, eps=1e-10):
         distance [B, N1, 3] (squared, MinK slot order), index [B, N1, 3] int64,
         weight [B, N1, 3]. Not differentiable, as in the reference (``no_grad``).
     """
-    with torch.no_grad():
-        return _fused.three_nn(query_xyz.contiguous(), key_xyz.contiguous(), bool(transpose), eps)
+    return _native.three_nn(query_xyz.detach().contiguous(), key_xyz.detach().contiguous(),
+                            bool(transpose), float(eps))
 
 three_interpolate = interpolate_feature  # the spelling common elsewhere
