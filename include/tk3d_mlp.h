@@ -1,0 +1,165 @@
+/*
+ * tk3d_mlp.h - C ABI of the shared-MLP kernels (torkit3d_amd/csrc/mlp.hip): the pieces of
+ * "1x1 convolution, batch norm, ReLU" chains on [B, C, P] fp32 tensors, forward and backward,
+ * that the reference runs as stock torch modules (torkit3d/nn/modules/mlp.py,
+ * torkit3d/nn/modules/conv.py) on the tensors its ops produce (torkit3d/layers/pointnet2.py,
+ * torkit3d/ops/edge_conv.py). Conventions of tk3d.h: device pointers, dense tensors, outputs
+ * allocated by the caller and fully overwritten, nothing allocated or synchronised, 0 or an
+ * error code returned.
+ *
+ * A layer computes y = W x, then z = relu((y - mean) / sqrt(var + eps) * gamma + beta). The
+ * entry points hand y from layer to layer: the norm and the ReLU are applied where y is read.
+ * Backward, with g the gradient of z, e = g where z > 0 (or NaN) else 0:
+ *     dbeta = sum e,   dgamma = sum e (y - mean) / sqrt(var + eps),
+ *     dy = a e + b y + d  with (a, b, d) per channel (tk3d_mlp_grad_coefficients_f32).
+ *
+ * Pooled layers. Where only the maximum of z over groups of `group` consecutive positions is
+ * wanted, y itself is never stored: the product keeps the extreme of y over each group (the
+ * largest for gamma >= 0, else the smallest) and its place. In the backward e has one nonzero per
+ * group and channel, and with y = W x
+ *     W^T dy = W^T (a e) + (W^T diag(b) W) x + W^T d
+ *     dW     = (a e) x^T + diag(b) W (x x^T) + d (sum x)^T
+ * so the dense part needs only the input x.
+ */
+#ifndef TK3D_MLP_H
+#define TK3D_MLP_H
+
+#include <stddef.h>
+#include <stdint.h>
+
+#ifdef __cplusplus
+extern "C" {
+#endif
+
+typedef struct {
+    const float *mean, *var, *gamma, *beta; /* [C] each */
+    float eps;
+} tk3d_mlp_norm;
+
+typedef struct {
+    const float *x;        /* [B, K, P]; batch_stride elements from one batch element to the next */
+    const float *y;        /* same shape, for the gradient inputs */
+    const float *coef;     /* [K][4]: (a, b, d, -), for the gradient inputs */
+    const void *sel;       /* [B, K, M] of (float a e, int32 place in the group), sparse input */
+    const float *w;        /* weight of input channel k and output channel c: w[k * wk + c * wc] */
+    int64_t batch_stride;
+    int32_t K, wk, wc;
+} tk3d_mlp_source;
+
+/* What a product reads (in) and what it does with its result (out). */
+enum {
+    TK3D_MLP_IN_RAW = 0,      /* x */
+    TK3D_MLP_IN_RAW2 = 1,     /* the channels of src[0].x, then those of src[1].x */
+    TK3D_MLP_IN_ACT = 2,      /* relu(in_norm(x)) */
+    TK3D_MLP_IN_GRAD = 3,     /* a x + b y + d */
+    TK3D_MLP_IN_GRAD_OUT = 4, /* the same with x masked by relu(in_norm(y)) first */
+    TK3D_MLP_IN_POOL = 5,     /* the sparse src[0].sel, then relu(in_norm(src[1].x)) */
+    TK3D_MLP_OUT_STATS = 0,     /* out, and partial sums of it and of its square */
+    TK3D_MLP_OUT_PLAIN = 1,     /* out + bias, channels from C0 on in out2; either may be NULL */
+    TK3D_MLP_OUT_POINTS = 2,    /* out as [B, P, C] */
+    TK3D_MLP_OUT_EVAL = 3,      /* relu(out_norm(out)) */
+    TK3D_MLP_OUT_POOL = 4,      /* extreme over groups (out [B,C,M]), place (arg), partial sums */
+    TK3D_MLP_OUT_POOL_EVAL = 5, /* relu(out_norm(extreme over groups)) */
+    TK3D_MLP_OUT_MASK = 6       /* e = (out + bias) where relu(out_norm(yprev)) passes, and partial
+                                   sums of e and e (yprev - mean) */
+};
+
+typedef struct {
+    tk3d_mlp_source src[2];
+    tk3d_mlp_norm in_norm, out_norm;
+    float *out, *out2;
+    const float *yprev; /* [B, C, P] */
+    const float *bias;  /* [C] or NULL */
+    unsigned char *arg; /* [B, C, M] */
+    void *partial;      /* doubles [C][slots][2]; tk3d_mlp_product_slots gives slots */
+    int32_t B, C, C0, P;
+    int32_t group, M;   /* pooled forms: P == group * M, group 32 or 64 */
+} tk3d_mlp_product;
+
+/* One product. `slots` as tk3d_mlp_product_slots returns it for the same arguments. */
+int tk3d_mlp_product_slots(int in, int out, const tk3d_mlp_product *p);
+int tk3d_mlp_product_f32(int in, int out, const tk3d_mlp_product *p, void *stream);
+
+/* Weight gradient: out[r][c] = sum over (b, p) of row(r, p) * colv(c, p), r < R, c < C, in
+ * `splits` partial sums [splits][R][C]. Rows: raw x, gradient (a x + b y + d, masked or not),
+ * sparse, or activations; columns: raw x or activations. rowsum (NULL or [splits][R]) gets the
+ * sums of the rows themselves. */
+enum {
+    TK3D_MLP_ROW_RAW = 0,
+    TK3D_MLP_ROW_GRAD = 1,
+    TK3D_MLP_ROW_GRAD_OUT = 2,
+    TK3D_MLP_ROW_POOL = 3,
+    TK3D_MLP_ROW_ACT = 4,
+    TK3D_MLP_COL_RAW = 0,
+    TK3D_MLP_COL_ACT = 1
+};
+typedef struct {
+    tk3d_mlp_source row, col; /* K = R and C; weights unused */
+    tk3d_mlp_norm row_norm, col_norm;
+    float *partial, *rowsum;
+    int32_t B, P, group, M;
+} tk3d_mlp_outer;
+int tk3d_mlp_outer_splits(const tk3d_mlp_outer *p);
+int tk3d_mlp_outer_f32(int row, int col, const tk3d_mlp_outer *p, void *stream);
+
+/* out[r * ld + c] = sum of the partial sums [splits][R][C]; n of them in one launch. */
+typedef struct {
+    const float *partial;
+    float *out;
+    int32_t splits, R, C, ld;
+} tk3d_mlp_sum;
+int tk3d_mlp_sum_f32(const tk3d_mlp_sum *sums, int n, void *stream);
+
+/* Batch statistics of `n` values per channel from the partial sums: mean and (biased) variance,
+ * running statistics updated with `momentum` (unbiased variance) and *batches incremented where
+ * given (NULL otherwise). */
+int tk3d_mlp_statistics_f32(const void *partial, int slots, int64_t n, int C, float momentum,
+                            float *mean, float *var, float *running_mean, float *running_var,
+                            int64_t *batches, void *stream);
+
+/* (a, b, d) per channel from the partial sums of (e, e (y - mean)), and dgamma, dbeta.
+ * frozen: the statistics are constants (evaluation mode), b = d = 0. */
+int tk3d_mlp_grad_coefficients_f32(const void *partial, int slots, int64_t n, int C,
+                                   const tk3d_mlp_norm *norm, int frozen, float *coef,
+                                   float *dgamma, float *dbeta, void *stream);
+
+/* Partial sums of (e, e (y - mean)) with e = g masked by relu(norm(y)); g, y [B, C, P].
+ * slots of tk3d_mlp_mask_slots. */
+int tk3d_mlp_mask_slots(int B, int C, int P);
+int tk3d_mlp_mask_sums_f32(const float *g, const float *y, int B, int C, int P,
+                           const tk3d_mlp_norm *norm, void *partial, void *stream);
+
+/* z = relu(norm(y)), n rows of P values, channel = row modulo C. */
+int tk3d_mlp_activate_f32(const float *y, int64_t rows, int C, int P, const tk3d_mlp_norm *norm,
+                          float *z, void *stream);
+/* dy = a e + b y + d over e itself. */
+int tk3d_mlp_grad_apply_f32(float *e, const float *y, const float *coef, int B, int C, int P,
+                            void *stream);
+
+/* Backward of a pooled layer, before the products: from g [B,C,M], the extremes and their places
+ * the coefficients, dgamma, dbeta and sel (see tk3d_mlp_source); positions = B * group * M. */
+int tk3d_mlp_pool_grad_f32(const float *g, const float *extreme, const unsigned char *arg, int B,
+                           int C, int M, int64_t positions, const tk3d_mlp_norm *norm, int frozen,
+                           void *sel, float *coef, float *dgamma, float *dbeta, void *stream);
+/* gram[k][c] = sum_o W[o][k] b[o] W[o][c] and bias[c] = sum_o W[o][c] d[o]; W [O][I]. */
+int tk3d_mlp_pool_gram_f32(const float *w, const float *coef, int O, int I, float *gram, float *bias,
+                           void *stream);
+/* dW[o][i] = sparse[o][i] + b[o] (W xx)[o][i] + d[o] xsum[i]; sparse, xx, xsum as partial sums. */
+int tk3d_mlp_pool_weight_grad_f32(const float *sparse, int sparse_splits, const float *xx,
+                                  const float *xsum, int xx_splits, const float *w,
+                                  const float *coef, int O, int I, float *scratch, float *dw,
+                                  void *stream);
+
+/* First layer behind a grouping: y[b,c,m,s] = u[b,j,c] + sum_a wx[c][a] (xyz[b,a,j] -
+ * centre[b,a,m]), j = index[b,m,s] (an index outside [0,N) reads as zeros). u [B,N,C] (the product
+ * of the features with their weights, or NULL), wx rows ldw apart. rel (NULL or [B,3,M*S]) gets
+ * the centred coordinates. Partial sums as TK3D_MLP_OUT_STATS. */
+int tk3d_mlp_group_slots(int B, int C, int M, int S);
+int tk3d_mlp_group_f32(const float *u, const float *xyz, const float *centre, const int64_t *index,
+                       const float *wx, int ldw, int B, int C, int N, int M, int S, float *y,
+                       float *rel, void *partial, void *stream);
+
+#ifdef __cplusplus
+}
+#endif
+#endif /* TK3D_MLP_H */

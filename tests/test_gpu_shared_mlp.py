@@ -1,0 +1,164 @@
+"""The fused chains of ``SharedMLP`` (csrc/mlp.hip) against the same modules in stock torch.
+
+The oracle is the stock chain in float64. A float32 implementation may differ from it by what
+float32 gives, so every output, gradient and running statistic of the fused chain has to be
+about as close to float64 (2-norm of the difference over 2-norm of the result) as stock
+float32 is: within four times its error plus 2e-6 (a few rounding errors of 2^-24 through up
+to four layers)."""
+import copy
+
+import pytest
+import torch
+from torch import nn
+
+from torkit3d_amd.nn import SharedMLP, mlp1d_bn_relu, mlp2d_bn_relu
+from torkit3d_amd.ops.group_points import group_points_with_xyz
+
+pytestmark = pytest.mark.gpu
+
+
+def make(build, cin, widths, training, cuda):
+    torch.manual_seed(1)
+    mlp = build(cin, widths)
+    for m in mlp.modules():
+        if isinstance(m, (nn.BatchNorm1d, nn.BatchNorm2d)):
+            nn.init.uniform_(m.weight, -1.0, 1.5)  # both signs: maxima become minima
+            nn.init.uniform_(m.bias, -0.5, 0.5)
+            nn.init.uniform_(m.running_mean, -0.5, 0.5)
+            nn.init.uniform_(m.running_var, 0.5, 2.0)
+    return mlp.to(cuda).train(training)
+
+
+def stock(mlp, dtype):
+    """The same layers as a plain nn.Sequential."""
+    return nn.Sequential(*copy.deepcopy(mlp).to(dtype).children()).train(mlp.training)
+
+
+def everything(module, fn, inputs):
+    """Outputs, gradients (inputs that float, parameters) and buffers after one pass."""
+    leaves = [t.clone().requires_grad_() if t.is_floating_point() and g else t for t, g in inputs]
+    out = fn(module, *leaves)
+    grad = torch.linspace(-1.0, 1.0, out.numel(), device=out.device, dtype=torch.float64)
+    grad = grad[torch.randperm(out.numel(), generator=torch.Generator().manual_seed(3)).to(out.device)]
+    wanted = [t for t in leaves if t.requires_grad] + list(module.parameters())
+    grads = torch.autograd.grad(out, wanted, grad.view_as(out).to(out.dtype))
+    return [out.detach(), *grads, *[b.clone() for b in module.buffers()]]
+
+
+def check(mlp, fused, reference, inputs, monkeypatch):
+    used = []
+    real = SharedMLP._chain
+    monkeypatch.setattr(SharedMLP, "_chain",
+                        lambda self, *a, **k: used.append(real(self, *a, **k)) or used[-1])
+    plain32, plain64 = stock(mlp, torch.float32), stock(mlp, torch.float64)
+    got = everything(mlp, fused, inputs)
+    assert len(used) == 1 and used[0] is not None, "the fused chain did not run"
+    single = everything(plain32, reference, inputs)
+    exact = everything(plain64, reference, [(t.double() if t.is_floating_point() else t, g)
+                                            for t, g in inputs])
+    for i, (a, s, e) in enumerate(zip(got, single, exact)):
+        assert a.shape == e.shape
+        if not e.is_floating_point():
+            assert torch.equal(a, e)
+            continue
+        norm = float(e.norm()) + 1e-30
+        mine, theirs = float((a.double() - e).norm()) / norm, float((s.double() - e).norm()) / norm
+        assert mine <= 4 * theirs + 2e-6, (i, tuple(e.shape), mine, theirs)
+
+
+def randn(seed, *shape):
+    return torch.randn(*shape, generator=torch.Generator().manual_seed(seed)).cuda()
+
+
+# Positions and channels around the tiles (32 channels, 32/64/128 positions, 8 input channels a
+# step, weights in one piece or in several), row lengths that are multiples of 4 and not.
+@pytest.mark.parametrize("training", [True, False])
+@pytest.mark.parametrize("b,p,widths", [
+    (2, 1, (5, 7)), (1, 37, (3, 33, 65)), (3, 64, (8, 32)), (2, 130, (64, 31, 64)),
+    (1, 4, (9, 16, 8)), (5, 1000, (131, 128, 128)), (2, 1024, (16, 32, 64, 32)),
+    (1, 129, (300, 257)), (4, 36, (768, 256, 40)), (40, 4096, (6, 32, 64, 40)),
+])
+def test_dense(cuda, monkeypatch, b, p, widths, training):
+    mlp = make(mlp1d_bn_relu, widths[0], widths[1:], training, cuda)
+    check(mlp, lambda m, x: m(x), lambda m, x: m(x), [(randn(b + p, b, widths[0], p), True)],
+          monkeypatch)
+
+
+@pytest.mark.parametrize("c1,c2,p", [(5, 3, 37), (128, 3, 512), (64, 96, 1000)])
+def test_concatenated_input(cuda, monkeypatch, c1, c2, p):
+    mlp = make(mlp1d_bn_relu, c1 + c2, (32, 48), True, cuda)
+    check(mlp, lambda m, x, y: m.forward_cat(x, y), lambda m, x, y: m(torch.cat([x, y], 1)),
+          [(randn(1, 2, c1, p), True), (randn(2, 2, c2, p), True)], monkeypatch)
+
+
+# Groups of 32 and 64 in the three tile shapes; one and several channel tiles.
+@pytest.mark.parametrize("training", [True, False])
+@pytest.mark.parametrize("b,m,s,widths", [
+    (2, 5, 32, (6, 32, 32)), (1, 3, 32, (4, 20, 70)), (2, 2, 64, (9, 64, 33)),
+    (2, 1600, 32, (3, 32, 32)), (4, 600, 64, (16, 64, 96)), (8, 1024, 32, (7, 40, 64)),
+])
+def test_maximum_over_neighbours(cuda, monkeypatch, b, m, s, widths, training):
+    mlp = make(mlp2d_bn_relu, widths[0], widths[1:], training, cuda)
+    check(mlp, lambda n, x: n.forward_max(x), lambda n, x: n(x).max(dim=3)[0],
+          [(randn(m, b, widths[0], m, s), True)], monkeypatch)
+
+
+# Grouped input: with features (gradient wanted or not, few or many), without, indices outside.
+@pytest.mark.parametrize("training", [True, False])
+@pytest.mark.parametrize("features,tracked,n,m,s", [
+    (0, False, 100, 7, 64), (3, False, 333, 40, 32), (5, True, 333, 40, 32), (61, True, 64, 33, 64),
+    (64, False, 500, 30, 32), (64, True, 2048, 512, 32),
+])
+def test_grouped(cuda, monkeypatch, features, tracked, n, m, s, training):
+    g = torch.Generator().manual_seed(n)
+    mlp = make(mlp2d_bn_relu, features + 3, (36, 32, 64), training, cuda)
+    xyz, centre = randn(1, 2, 3, n), randn(2, 2, 3, m)
+    index = torch.randint(0, n, (2, m, s), generator=g)
+    index[0, 0] = -1
+    index = index.cuda()
+    inputs = [(xyz, False), (centre, False), (index, False)]
+    if features:
+        inputs.append((randn(3, 2, features, n), tracked))
+
+    def fused(mod, xyz, centre, index, f=None):
+        return mod.forward_grouped_max(f, xyz, centre, index)
+
+    def reference(mod, xyz, centre, index, f=None):
+        return mod(group_points_with_xyz(f, xyz, centre, index)).max(dim=3)[0]
+
+    check(mlp, fused, reference, inputs, monkeypatch)
+
+
+def test_gradient_of_a_gradient(cuda):
+    mlp = make(mlp1d_bn_relu, 6, (8, 5), True, cuda)
+    results = []
+    for module in (mlp, stock(mlp, torch.float32)):
+        x = randn(4, 2, 6, 20).requires_grad_()
+        out = module(x)
+        (first,) = torch.autograd.grad(out.square().sum(), x, create_graph=True)
+        results.append((first.detach(), *torch.autograd.grad(first.square().sum(),
+                                                             [x, *module.parameters()])))
+    for a, b in zip(*results):
+        assert float((a - b).norm()) <= 1e-4 * float(b.norm()) + 1e-6
+
+
+def test_what_is_not_plain_runs_layer_by_layer(cuda):
+    mlp = make(mlp1d_bn_relu, 6, (8, 5), True, cuda)
+    x = randn(5, 2, 6, 20)
+    seen = []
+    handle = mlp[0].bn.register_forward_hook(lambda *a: seen.append(1))
+    mlp(x)
+    assert seen == [1]
+    handle.remove()
+    mlp[1].bn.eval()  # a frozen layer among training ones
+    assert torch.allclose(mlp(x), stock_forward(mlp, x), atol=1e-5)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        mlp(x)
+    nan = x.clone()
+    nan[0, 0, 0] = float("nan")
+    mlp.eval()
+    assert torch.equal(mlp(nan).isnan(), nn.Sequential.forward(mlp, nan).isnan())
+
+
+def stock_forward(mlp, x):
+    return nn.Sequential.forward(mlp, x)

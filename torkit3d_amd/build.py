@@ -8,6 +8,7 @@ import os
 import shutil
 import subprocess
 import sys
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 REPO = os.path.dirname(HERE)
@@ -69,8 +70,6 @@ def sources():
 def build(verbose=False, jobs=None):
     """Compile every kernel source for gfx950 (one hipcc process per source file, run side
     by side) and link ``libtk3d.so`` in-tree."""
-    from concurrent.futures import ThreadPoolExecutor
-
     objdir = os.path.join(HERE, "build")
     os.makedirs(objdir, exist_ok=True)
     compile_flags = [f for f in HIPCC_FLAGS if f != "-shared"] + optional_flags()
@@ -102,7 +101,7 @@ def build(verbose=False, jobs=None):
 
 
 def build_native(verbose=False):
-    """Compile the Python extension with the operators' host path (``csrc/native.cpp``) against
+    """Compile the Python extension with the operators' host path (``csrc/native*.cpp``) against
     the installed torch and ``libtk3d.so``, which it finds beside itself."""
     import sysconfig
 
@@ -110,26 +109,40 @@ def build_native(verbose=False):
     from torch.utils import cpp_extension
 
     torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
-    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared",
-           "-fvisibility=hidden", "-Wall", "-Wno-deprecated-declarations",
-           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-DTORCH_EXTENSION_NAME=_host",
-           "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI),
-           "-I", os.path.join(REPO, "include"), "-I", sysconfig.get_paths()["include"]]
+    flags = ["-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-Wall",
+             "-Wno-deprecated-declarations", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+             "-DTORCH_EXTENSION_NAME=_host",
+             "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI),
+             "-I", os.path.join(REPO, "include"), "-I", sysconfig.get_paths()["include"]]
     rocm = os.path.dirname(os.path.dirname(hipcc_path()))
     for path in cpp_extension.include_paths() + [os.path.join(rocm, "include"),
                                                  "/opt/rocm/include"]:
-        cmd += ["-isystem", path]
-    cmd += [os.path.join(CSRC, "native.cpp"), "-o", NATIVE_PATH + ".tmp", "-L", HERE,
-            "-l:" + os.path.basename(LIB_PATH),
-            "-L", torch_lib, "-ltorch_python", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10",
-            "-lc10_hip", "-Wl,-rpath,$ORIGIN"]
-    if verbose:
-        print(" ".join(cmd))
-    res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
-    if res.returncode != 0:
-        raise RuntimeError("building _host.so failed:\n" + res.stdout)
-    if verbose and res.stdout.strip():
-        print(res.stdout)
+        flags += ["-isystem", path]
+    objdir = os.path.join(HERE, "build_host")
+    os.makedirs(objdir, exist_ok=True)
+    cxx = os.environ.get("CXX", "g++")
+
+    def run(cmd):
+        if verbose:
+            print(" ".join(cmd))
+        res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+        if res.returncode != 0:
+            raise RuntimeError("building _host.so failed:\n" + res.stdout)
+        if verbose and res.stdout.strip():
+            print(res.stdout)
+
+    def compile_one(src):
+        obj = os.path.join(objdir, os.path.basename(src)[:-4] + ".o")
+        run([cxx] + flags + ["-c", src, "-o", obj])
+        return obj
+
+    srcs = sorted(glob.glob(os.path.join(CSRC, "native*.cpp")))
+    with ThreadPoolExecutor(max_workers=len(srcs)) as pool:
+        objects = list(pool.map(compile_one, srcs))
+    run([cxx, "-shared", "-o", NATIVE_PATH + ".tmp"] + objects
+        + ["-L", HERE, "-l:" + os.path.basename(LIB_PATH), "-L", torch_lib, "-ltorch_python",
+           "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN"])
+    shutil.rmtree(objdir, ignore_errors=True)
     os.replace(NATIVE_PATH + ".tmp", NATIVE_PATH)
     return NATIVE_PATH
 

@@ -1,0 +1,1475 @@
+// Shared MLPs: 1x1 convolution, batch norm and ReLU per layer on [B, C, P] tensors, forward and
+// backward, with the grouping in front of the first layer and the maximum over neighbours behind
+// the last one where a layer has them (include/tk3d_mlp.h says what each entry point computes).
+//
+// What bounds it: an activation is read and written once per layer and direction, everything
+// else is what can be fused into those passes. A layer's product reads the PREVIOUS layer's
+// product and normalises it on the way into the matrix cores, adds up the statistics of its own
+// result on the way out, and a last layer under a maximum writes the maximum only. Narrow layers
+// (up to 64 channels) are bound by HBM, wide ones by the fp32 matrix rate (157 TFLOP/s), which is
+// why the products are fp32 v_mfma_f32_32x32x2 and nothing is rounded to a shorter type.
+#include "tk3d_common.h"
+#include "tk3d_mlp.h"
+
+namespace {
+
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// ReLU that keeps NaN, as torch's does.
+__device__ __forceinline__ float relu(float z) { return __builtin_elementwise_maximum(z, 0.0f); }
+// Whether the gradient passes a ReLU whose input was z (torch: where the output is > 0 or NaN).
+__device__ __forceinline__ bool passes(float z) { return !(z <= 0.0f); }
+
+__device__ __forceinline__ f32x2 scale_shift(const tk3d_mlp_norm &n, int c)
+{
+    const float scale = n.gamma[c] * (1.0f / __builtin_sqrtf(n.var[c] + n.eps));
+    return f32x2{scale, __builtin_fmaf(-n.mean[c], scale, n.beta[c])};
+}
+
+// ---- the product ---------------------------------------------------------------------------------
+//
+// out[c][p] = sum over k of w(k, c) * in(k, p) for one batch element at a time.
+//
+// A wave owns 32 * PT positions and 32 * CT output channels: rows of the matrix instruction are
+// positions, columns channels, so a lane of the result holds 16 * PT positions of one channel in
+// registers, and statistics, maxima and 16-byte stores need no exchange between lanes. Tile t of
+// the PT holds positions PT * i + t: a lane then reads PT consecutive positions of an input row
+// with one load, and its results are runs of 4 * PT consecutive positions. Input rows come
+// straight from memory into the lanes that feed them to the matrix cores (a wave's positions are
+// its own, LDS would not be shared by anybody); the weights, which all waves share, are staged in
+// LDS in the order in which lanes read them (16 bytes, four steps of the product). A workgroup
+// keeps its weights and loops over positions; the rows of the next eight input channels, also
+// those of the next positions, are requested before the present eight are multiplied.
+
+enum Input {      // in(k, p)
+    IN_RAW,       // x
+    IN_RAW2,      // x of two tensors, one after the other
+    IN_ACT,       // relu(norm(x))
+    IN_GRAD,      // a e + b y + d: gradient before the norm from the gradient behind it (e)
+    IN_GRAD_OUT,  // the same where e = g masked by the ReLU still has to be formed from g and y
+    IN_POOL,      // sparse gradient of a maximum, then relu(norm(x)) (see pooled layers below)
+};
+enum Output {
+    OUT_STATS,      // store, and sums of the stored values and their squares per channel
+    OUT_PLAIN,      // store, in two tensors if asked for
+    OUT_POINTS,     // store as [B, P, C]
+    OUT_EVAL,       // store relu(norm(out))
+    OUT_POOL,       // store the extreme over each group and where it is, with the sums
+    OUT_POOL_EVAL,  // store relu(norm(extreme over each group))
+    OUT_MASK,       // store out masked by the ReLU in front of it, with the sums of its gradient
+};
+
+constexpr int kBlock = 256;
+constexpr int kWaves = kBlock / TK_WAVE;
+
+template <int PT> struct VecOf;
+template <> struct VecOf<1> { typedef float type; };
+template <> struct VecOf<2> { typedef f32x2 type; };
+template <> struct VecOf<4> { typedef f32x4 type; };
+
+template <int PT>
+__device__ __forceinline__ void load_run(float (&dst)[PT], const float *base, unsigned offset)
+{
+    const typename VecOf<PT>::type v =
+        *reinterpret_cast<const typename VecOf<PT>::type *>(reinterpret_cast<const char *>(base) + offset);
+    if constexpr (PT == 1)
+        dst[0] = v;
+    else
+#pragma unroll
+        for (int t = 0; t < PT; ++t)
+            dst[t] = v[t];
+}
+
+constexpr bool reads_y(int in) { return in == IN_GRAD || in == IN_GRAD_OUT; }
+
+template <int IN, int PT> struct Rows {  // eight input channels of a wave's positions
+    float x[4][PT];
+    float y[reads_y(IN) ? 4 : 1][PT];
+    int2 sel[IN == IN_POOL ? 4 : 1];
+};
+
+struct GemmArgs {
+    tk3d_mlp_product p;
+    int tiles;       // wave tiles per batch element
+    int total;       // wave tiles in all
+    int kg0, kg;     // groups of eight input channels: of the first source, of all
+    int chunk;       // groups whose weights are in LDS at once
+    int slots;       // partial sums per channel (gridDim.x)
+    int coef_bytes;
+};
+
+template <int IN, int OUT, int PT, int CT>
+__global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
+{
+    extern __shared__ char lds[];
+    const tk3d_mlp_product &p = a.p;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int half = lane >> 5, col = lane & 31;
+    const int cbase = blockIdx.y * (32 * CT);
+    const int P = p.P;
+
+    // LDS: normalisation of the input channels, then the weights.
+    f32x4 *grad_coef = reinterpret_cast<f32x4 *>(lds);              // [K] (a, b, d, -)
+    f32x2 *act_coef = reinterpret_cast<f32x2 *>(lds);               // [K] (scale, shift)
+    if constexpr (IN == IN_GRAD_OUT)
+        act_coef = reinterpret_cast<f32x2 *>(lds + (size_t)a.kg * 8 * sizeof(f32x4));
+    float *weights = reinterpret_cast<float *>(lds + a.coef_bytes);  // [CT][chunk][64][4]
+
+    if constexpr (IN == IN_ACT || IN == IN_POOL || IN == IN_GRAD_OUT) {
+        const int K = IN == IN_POOL ? p.src[1].K : p.src[0].K;
+        for (int k = tid; k < ((K + 7) & ~7); k += kBlock)
+            act_coef[k] = k < K ? scale_shift(p.in_norm, k) : f32x2{0.0f, 0.0f};
+    }
+    if constexpr (reads_y(IN)) {
+        const f32x4 *coef = reinterpret_cast<const f32x4 *>(p.src[0].coef);
+        for (int k = tid; k < a.kg * 8; k += kBlock)
+            grad_coef[k] = k < p.src[0].K ? coef[k] : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+
+    // Weights of channel groups [first, first + count): element (ct, g, lane, s) belongs to
+    // input channel 8 g + 2 s + (lane >> 5) and output channel 32 ct + (lane & 31).
+    const auto stage = [&](int first, int count) {
+        for (int i = tid; i < CT * count * 256; i += kBlock) {
+            // (consecutive threads walk the direction in which the weights lie in memory)
+            int k8, c;
+            const int g = i >> 8;  // (ct, group), 256 elements each
+            const int e = i & 255;
+            const int ct = g / count, grp = first + g - ct * count;
+            const bool second = grp >= a.kg0;
+            const tk3d_mlp_source &s = p.src[second ? 1 : 0];
+            if (s.wk == 1) {
+                k8 = e & 7;
+                c = e >> 3;
+            } else {
+                c = e & 31;
+                k8 = e >> 5;
+            }
+            const int k = (grp - (second ? a.kg0 : 0)) * 8 + k8, cc = cbase + ct * 32 + c;
+            const float v = k < s.K && cc < p.C
+                                ? s.w[(int64_t)k * s.wk + (int64_t)cc * s.wc] : 0.0f;
+            weights[((ct * a.chunk + (grp - first)) * 64 + (k8 & 1) * 32 + c) * 4 + (k8 >> 1)] = v;
+        }
+    };
+
+    // Rows of channel group g for the positions of a wave tile.
+    const auto load = [&](Rows<IN, PT> &r, int tile, int g) {
+        const int b = tile / a.tiles;
+        int pos = (tile - b * a.tiles) * (32 * PT) + PT * col;
+        pos = pos > P - PT ? P - PT : pos;  // (results of the surplus are dropped)
+        const bool second = (IN == IN_RAW2 || IN == IN_POOL) && g >= a.kg0;
+        const tk3d_mlp_source &s = p.src[second ? 1 : 0];
+        const int k0 = (g - (second ? a.kg0 : 0)) * 8 + half;
+        if (IN == IN_POOL && !second) {
+            const int m = pos / p.group;
+            const int2 *sel = reinterpret_cast<const int2 *>(s.sel) + (int64_t)b * s.K * p.M;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int k = k0 + 2 * q < s.K ? k0 + 2 * q : s.K - 1;
+                r.sel[IN == IN_POOL ? q : 0] = sel[(unsigned)k * (unsigned)p.M + (unsigned)m];
+            }
+            return;
+        }
+        const float *x = s.x + (int64_t)b * s.batch_stride;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int k = k0 + 2 * q < s.K ? k0 + 2 * q : s.K - 1;
+            const unsigned offset = ((unsigned)k * (unsigned)P + (unsigned)pos) * 4u;
+            load_run<PT>(r.x[q], x, offset);
+            if constexpr (reads_y(IN))
+                load_run<PT>(r.y[q], s.y + (int64_t)b * s.batch_stride, offset);
+        }
+    };
+
+    tk_f32x16 acc[PT][CT];
+    const auto clear = [&] {
+#pragma unroll
+        for (int t = 0; t < PT; ++t)
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    acc[t][ct][r] = 0.0f;
+    };
+
+    const auto multiply = [&](const Rows<IN, PT> &r, int tile, int g, int first) {
+        const bool second = (IN == IN_RAW2 || IN == IN_POOL) && g >= a.kg0;
+        const int K = p.src[second ? 1 : 0].K, gs = g - (second ? a.kg0 : 0);
+        const int k0 = gs * 8 + half;
+        float v[4][PT];
+        if (IN == IN_POOL && !second) {
+            const int b = tile / a.tiles;
+            int pos = (tile - b * a.tiles) * (32 * PT) + PT * col;
+            pos = pos > P - PT ? P - PT : pos;
+            const int kk = pos - pos / p.group * p.group;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int2 sel = r.sel[IN == IN_POOL ? q : 0];
+#pragma unroll
+                for (int t = 0; t < PT; ++t)
+                    v[q][t] = sel.y == kk + t ? __int_as_float(sel.x) : 0.0f;
+            }
+        } else {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                if constexpr (reads_y(IN)) {
+                    const f32x4 c = grad_coef[k0 + 2 * q];
+                    f32x2 ss{0.0f, 0.0f};
+                    if constexpr (IN == IN_GRAD_OUT)
+                        ss = act_coef[k0 + 2 * q];
+#pragma unroll
+                    for (int t = 0; t < PT; ++t) {
+                        float e = r.x[q][t];
+                        const float y = r.y[reads_y(IN) ? q : 0][t];
+                        if constexpr (IN == IN_GRAD_OUT)
+                            e = passes(__builtin_fmaf(y, ss.x, ss.y)) ? e : 0.0f;
+                        v[q][t] = __builtin_fmaf(c.x, e, __builtin_fmaf(c.y, y, c.z));
+                    }
+                } else if constexpr (IN == IN_ACT || IN == IN_POOL) {
+                    const f32x2 c = act_coef[k0 + 2 * q];
+#pragma unroll
+                    for (int t = 0; t < PT; ++t)
+                        v[q][t] = relu(__builtin_fmaf(r.x[q][t], c.x, c.y));
+                } else {
+#pragma unroll
+                    for (int t = 0; t < PT; ++t)
+                        v[q][t] = r.x[q][t];
+                }
+            }
+        }
+        if (gs * 8 + 8 > K) {  // channels past the last one (their weights are zero) must not be inf
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int t = 0; t < PT; ++t)
+                    v[q][t] = k0 + 2 * q < K ? v[q][t] : 0.0f;
+        }
+        f32x4 w[CT];
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct)
+            w[ct] = *reinterpret_cast<const f32x4 *>(
+                weights + ((ct * a.chunk + (g - first)) * 64 + lane) * 4);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                for (int t = 0; t < PT; ++t)
+                    acc[t][ct] = __builtin_amdgcn_mfma_f32_32x32x2f32(v[q][t], w[ct][q], acc[t][ct],
+                                                                      0, 0, 0);
+    };
+
+    // Per-lane constants and sums of the output channels (lane = channel).
+    constexpr bool kSums = OUT == OUT_STATS || OUT == OUT_POOL || OUT == OUT_MASK;
+    int chan[CT];
+    float shift[CT], sum1[CT], sum2[CT];
+    f32x2 out_coef[CT];
+    float sign[CT], bias[CT];
+    int count = 0;
+    bool fresh = true;
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+        chan[ct] = cbase + ct * 32 + col;
+        const int c = chan[ct] < p.C ? chan[ct] : p.C - 1;
+        sum1[ct] = sum2[ct] = shift[ct] = 0.0f;
+        if constexpr (OUT == OUT_EVAL || OUT == OUT_POOL_EVAL || OUT == OUT_MASK)
+            out_coef[ct] = scale_shift(p.out_norm, c);
+        if constexpr (OUT == OUT_POOL || OUT == OUT_POOL_EVAL) {
+            const float g = p.out_norm.gamma[c];
+            sign[ct] = g > 0.0f ? 1.0f : g < 0.0f ? -1.0f : 0.0f;
+        }
+        if constexpr (OUT == OUT_MASK) {
+            shift[ct] = p.out_norm.mean[c];
+            bias[ct] = p.bias ? p.bias[c] : 0.0f;
+        }
+        if constexpr (OUT == OUT_PLAIN)
+            bias[ct] = p.bias ? p.bias[c] : 0.0f;
+    }
+
+    const auto finish = [&](int tile) {
+        const int b = tile / a.tiles;
+        const int base = (tile - b * a.tiles) * (32 * PT);
+        const bool full = base + 32 * PT <= P;
+        const bool vec = (P & 3) == 0;
+        constexpr int RUN = 4 * PT;
+        if constexpr (OUT == OUT_STATS || OUT == OUT_POOL) {
+            if (fresh) {  // the sums are taken around a value of the channel itself
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct)
+                    shift[ct] = acc[0][ct][0];
+                fresh = false;
+            }
+        }
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) {
+            const int c = chan[ct];
+            const bool mine = c < p.C;
+            float *row = nullptr;
+            if constexpr (OUT == OUT_STATS || OUT == OUT_PLAIN || OUT == OUT_EVAL || OUT == OUT_MASK) {
+                const bool first = c < p.C0;
+                float *out = first ? p.out : p.out2;
+                const int rows = first ? p.C0 : p.C - p.C0, r = first ? c : c - p.C0;
+                row = mine && out ? out + ((int64_t)b * rows + r) * P : nullptr;
+            }
+            float best = 0.0f, first_y = 0.0f;
+            int where = -1;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int pos = base + PT * (8 * q + 4 * half);
+                float v[RUN];
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int t = 0; t < PT; ++t)
+                        v[i * PT + t] = acc[t][ct][4 * q + i];
+                if constexpr (OUT == OUT_MASK || OUT == OUT_PLAIN) {
+#pragma unroll
+                    for (int i = 0; i < RUN; ++i)
+                        v[i] += bias[ct];
+                }
+                float before[OUT == OUT_MASK ? RUN : 1];
+                if constexpr (OUT == OUT_MASK) {
+                    const float *yrow = p.yprev + ((int64_t)b * p.C + (mine ? c : p.C - 1)) * P;
+                    if (vec) {
+#pragma unroll
+                        for (int i = 0; i < PT; ++i) {
+                            const int at = pos + 4 * i > P - 4 ? P - 4 : pos + 4 * i;
+                            const f32x4 w = *reinterpret_cast<const f32x4 *>(yrow + at);
+#pragma unroll
+                            for (int j = 0; j < 4; ++j)
+                                before[(OUT == OUT_MASK) ? 4 * i + j : 0] = w[j];
+                        }
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < RUN; ++i)
+                            before[OUT == OUT_MASK ? i : 0] = yrow[pos + i > P - 1 ? P - 1 : pos + i];
+                    }
+#pragma unroll
+                    for (int i = 0; i < RUN; ++i) {
+                        const float y = before[OUT == OUT_MASK ? i : 0];
+                        v[i] = passes(__builtin_fmaf(y, out_coef[ct].x, out_coef[ct].y)) ? v[i] : 0.0f;
+                    }
+                }
+                if constexpr (kSums) {
+                    if (full) {
+#pragma unroll
+                        for (int i = 0; i < RUN; ++i) {
+                            if constexpr (OUT == OUT_MASK) {
+                                sum1[ct] += v[i];
+                                sum2[ct] = __builtin_fmaf(v[i], before[OUT == OUT_MASK ? i : 0] - shift[ct], sum2[ct]);
+                            } else {
+                                const float d = v[i] - shift[ct];
+                                sum1[ct] += d;
+                                sum2[ct] = __builtin_fmaf(d, d, sum2[ct]);
+                            }
+                        }
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < RUN; ++i) {
+                            if (pos + i < P) {
+                                if constexpr (OUT == OUT_MASK) {
+                                    sum1[ct] += v[i];
+                                    sum2[ct] = __builtin_fmaf(v[i], before[OUT == OUT_MASK ? i : 0] - shift[ct], sum2[ct]);
+                                } else {
+                                    const float d = v[i] - shift[ct];
+                                    sum1[ct] += d;
+                                    sum2[ct] = __builtin_fmaf(d, d, sum2[ct]);
+                                }
+                            }
+                        }
+                    }
+                }
+                if constexpr (OUT == OUT_EVAL) {
+#pragma unroll
+                    for (int i = 0; i < RUN; ++i)
+                        v[i] = relu(__builtin_fmaf(v[i], out_coef[ct].x, out_coef[ct].y));
+                }
+                if constexpr (OUT == OUT_STATS || OUT == OUT_PLAIN || OUT == OUT_EVAL || OUT == OUT_MASK) {
+                    if (row) {
+                        if (vec) {
+#pragma unroll
+                            for (int i = 0; i < PT; ++i)
+                                if (full || pos + 4 * i < P)
+                                    *reinterpret_cast<f32x4 *>(row + pos + 4 * i) =
+                                        f32x4{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
+                        } else {
+#pragma unroll
+                            for (int i = 0; i < RUN; ++i)
+                                if (pos + i < P)
+                                    row[pos + i] = v[i];
+                        }
+                    }
+                } else if constexpr (OUT == OUT_POINTS) {
+#pragma unroll
+                    for (int i = 0; i < RUN; ++i)
+                        if (mine && pos + i < P)
+                            p.out[((int64_t)b * P + pos + i) * p.C + c] = v[i];
+                } else {
+                    // A group is both halves of one q or of several; the positions of a run and
+                    // the q come in ascending order, so the first of equal values stays.
+#pragma unroll
+                    for (int i = 0; i < RUN; ++i) {
+                        const float s = v[i] * sign[ct];
+                        if constexpr (OUT == OUT_POOL) {
+                            const bool up = where < 0 || s > best;
+                            if (i == 0)
+                                first_y = where < 0 ? v[0] : first_y;
+                            best = up ? s : best;
+                            where = up ? pos + i : where;
+                        } else {
+                            best = where < 0 ? s : __builtin_elementwise_maximum(best, s);
+                            where = 0;
+                        }
+                    }
+                    const int qs = p.group / (2 * RUN);
+                    if (((q + 1) & (qs - 1)) == 0) {
+                        const float other = __shfl_xor(best, 32);
+                        if constexpr (OUT == OUT_POOL) {
+                            const int at = __shfl_xor(where, 32);
+                            const bool up = other > best || (other == best && at < where);
+                            best = up ? other : best;
+                            where = up ? at : where;
+                        } else {
+                            best = __builtin_elementwise_maximum(best, other);
+                        }
+                        const int m = pos / p.group;
+                        if (mine && half == 0 && pos < P) {
+                            const int64_t at = ((int64_t)b * p.C + c) * p.M + m;
+                            if constexpr (OUT == OUT_POOL) {
+                                // (a zero gamma makes all values equal: the first one's place)
+                                p.out[at] = sign[ct] == 0.0f ? first_y : best * sign[ct];
+                                p.arg[at] = (unsigned char)(where - m * p.group);
+                            } else {
+                                p.out[at] = relu(sign[ct] == 0.0f
+                                    ? __builtin_fmaf(best, 0.0f, out_coef[ct].y)
+                                    : __builtin_fmaf(best * sign[ct], out_coef[ct].x, out_coef[ct].y));
+                            }
+                        }
+                        where = -1;
+                    }
+                }
+            }
+        }
+        if constexpr (kSums) {
+            if (full) {
+                count += 16 * PT;
+            } else {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int left = P - (base + PT * (8 * q + 4 * half));
+                    count += left <= 0 ? 0 : left < RUN ? left : RUN;
+                }
+            }
+        }
+    };
+
+    const int stride = gridDim.x * kWaves;
+    const int mine0 = blockIdx.x * kWaves + wave;
+    if (a.kg <= a.chunk) {
+        stage(0, a.kg);
+        __syncthreads();
+        if (mine0 < a.total) {
+            Rows<IN, PT> now, next;
+            load(now, mine0, 0);
+            for (int tile = mine0; tile < a.total; tile += stride) {
+                clear();
+                int g = 0;
+                for (; g + 1 < a.kg; ++g) {
+                    load(next, tile, g + 1);
+                    multiply(now, tile, g, 0);
+                    now = next;
+                }
+                if (tile + stride < a.total)
+                    load(next, tile + stride, 0);
+                multiply(now, tile, g, 0);
+                now = next;
+                finish(tile);
+            }
+        }
+    } else {
+        for (int base = blockIdx.x * kWaves; base < a.total; base += stride) {
+            const int tile = base + wave;
+            const bool active = tile < a.total;
+            clear();
+            for (int first = 0; first < a.kg; first += a.chunk) {
+                const int n = a.kg - first < a.chunk ? a.kg - first : a.chunk;
+                Rows<IN, PT> now, next;
+                if (active)
+                    load(now, tile, first);
+                __syncthreads();
+                stage(first, n);
+                __syncthreads();
+                if (active) {
+                    for (int g = first; g < first + n; ++g) {
+                        if (g + 1 < first + n)
+                            load(next, tile, g + 1);
+                        multiply(now, tile, g, first);
+                        now = next;
+                    }
+                }
+            }
+            if (active)
+                finish(tile);
+        }
+    }
+
+    if constexpr (kSums) {  // (sum, sum of squares) or (sum e, sum e (y - mean)) of this workgroup
+        __syncthreads();
+        double2 *part = reinterpret_cast<double2 *>(lds);  // [kWaves][32 CT]
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) {
+            double s1 = sum1[ct], s2 = sum2[ct];
+            if constexpr (OUT != OUT_MASK) {
+                const double sh = count ? (double)shift[ct] : 0.0, n = count;
+                s2 = s2 + 2.0 * sh * s1 + n * sh * sh;
+                s1 = s1 + n * sh;
+            }
+            s1 += __shfl_xor(s1, 32);
+            s2 += __shfl_xor(s2, 32);
+            if (half == 0)
+                part[wave * (32 * CT) + ct * 32 + col] = double2{s1, s2};
+        }
+        __syncthreads();
+        if (tid < 32 * CT && cbase + tid < p.C) {
+            double2 s = part[tid];
+            for (int w = 1; w < kWaves; ++w) {
+                s.x += part[w * (32 * CT) + tid].x;
+                s.y += part[w * (32 * CT) + tid].y;
+            }
+            reinterpret_cast<double2 *>(p.partial)[(int64_t)(cbase + tid) * a.slots + blockIdx.x] = s;
+        }
+    }
+}
+
+// ---- the weight gradient ---------------------------------------------------------------------------
+//
+// Rows times columns over positions. A lane reads runs of eight positions of one row and of one
+// column, which are eight steps of the product for it (lanes 0-31 take positions 0-7 and 8-15 of
+// a unit of 32, the other half 16-31); nothing goes through LDS until the four waves of a
+// workgroup, which take different positions, add up their results at the end.
+
+struct OuterArgs {
+    tk3d_mlp_outer p;
+    int units, total;  // units of 32 positions: per batch element, in all
+};
+
+template <int ROW, int COL, int TA, int TB>
+__global__ void __launch_bounds__(kBlock, 2) mlp_outer_kernel(OuterArgs a)
+{
+    extern __shared__ float sums[];
+    const tk3d_mlp_outer &p = a.p;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int half = lane >> 5, l32 = lane & 31;
+    const int rbase = blockIdx.y * (32 * TA), cbase = blockIdx.z * (32 * TB);
+    const int R = p.row.K, C = p.col.K, P = p.P;
+    const bool vec = (P & 3) == 0;
+    constexpr bool kGrad = ROW == TK3D_MLP_ROW_GRAD || ROW == TK3D_MLP_ROW_GRAD_OUT;
+
+    int r[TA], c[TB];
+    f32x4 coef[TA];
+    f32x2 row_act[TA], col_act[TB];
+    float total[TA];
+#pragma unroll
+    for (int t = 0; t < TA; ++t) {
+        r[t] = rbase + 32 * t + l32;
+        r[t] = r[t] < R ? r[t] : R - 1;
+        total[t] = 0.0f;
+        if constexpr (kGrad)
+            coef[t] = reinterpret_cast<const f32x4 *>(p.row.coef)[r[t]];
+        if constexpr (ROW == TK3D_MLP_ROW_GRAD_OUT || ROW == TK3D_MLP_ROW_ACT)
+            row_act[t] = scale_shift(p.row_norm, r[t]);
+    }
+#pragma unroll
+    for (int t = 0; t < TB; ++t) {
+        c[t] = cbase + 32 * t + l32;
+        c[t] = c[t] < C ? c[t] : C - 1;
+        if constexpr (COL == TK3D_MLP_COL_ACT)
+            col_act[t] = scale_shift(p.col_norm, c[t]);
+    }
+
+    struct Part {
+        float x[TA][8], y[kGrad ? TA : 1][8], c[TB][8];
+        int2 sel[TA];
+    };
+    const auto run8 = [&](float (&dst)[8], const float *row, int pos) {
+        if (vec) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const int at = pos + 4 * j > P - 4 ? P - 4 : pos + 4 * j;
+                const f32x4 v = *reinterpret_cast<const f32x4 *>(row + at);
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    dst[4 * j + i] = v[i];
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                dst[i] = row[pos + i > P - 1 ? P - 1 : pos + i];
+        }
+    };
+    const auto load = [&](Part &q, int unit, int sub) {
+        const int b = unit / a.units;
+        const int pos = (unit - b * a.units) * 32 + half * 16 + sub * 8;
+#pragma unroll
+        for (int t = 0; t < TA; ++t) {
+            if constexpr (ROW == TK3D_MLP_ROW_POOL) {
+                const int m = (pos > P - 8 ? P - 8 : pos) / p.group;
+                q.sel[t] = reinterpret_cast<const int2 *>(p.row.sel)[((int64_t)b * R + r[t]) * p.M + m];
+            } else {
+                const int64_t row = (int64_t)b * p.row.batch_stride + (int64_t)r[t] * P;
+                run8(q.x[t], p.row.x + row, pos);
+                if constexpr (kGrad)
+                    run8(q.y[kGrad ? t : 0], p.row.y + row, pos);
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < TB; ++t)
+            run8(q.c[t], p.col.x + (int64_t)b * p.col.batch_stride + (int64_t)c[t] * P, pos);
+    };
+
+    tk_f32x16 acc[TA][TB];
+#pragma unroll
+    for (int i = 0; i < TA; ++i)
+#pragma unroll
+        for (int j = 0; j < TB; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e)
+                acc[i][j][e] = 0.0f;
+
+    const auto multiply = [&](const Part &q, int unit, int sub) {
+        const int b = unit / a.units;
+        const int pos = (unit - b * a.units) * 32 + half * 16 + sub * 8;
+        float x[TA][8], y[TB][8];
+#pragma unroll
+        for (int t = 0; t < TA; ++t)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                float v;
+                if constexpr (ROW == TK3D_MLP_ROW_POOL) {
+                    const int kk = pos - pos / p.group * p.group;
+                    v = q.sel[t].y == kk + i ? __int_as_float(q.sel[t].x) : 0.0f;
+                } else if constexpr (kGrad) {
+                    float e = q.x[t][i];
+                    const float yy = q.y[kGrad ? t : 0][i];
+                    if constexpr (ROW == TK3D_MLP_ROW_GRAD_OUT)
+                        e = passes(__builtin_fmaf(yy, row_act[t].x, row_act[t].y)) ? e : 0.0f;
+                    v = __builtin_fmaf(coef[t].x, e, __builtin_fmaf(coef[t].y, yy, coef[t].z));
+                } else if constexpr (ROW == TK3D_MLP_ROW_ACT) {
+                    v = relu(__builtin_fmaf(q.x[t][i], row_act[t].x, row_act[t].y));
+                } else {
+                    v = q.x[t][i];
+                }
+                x[t][i] = pos + i < P ? v : 0.0f;
+                if constexpr (ROW == TK3D_MLP_ROW_ACT)
+                    total[t] += x[t][i];
+            }
+#pragma unroll
+        for (int t = 0; t < TB; ++t)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                float v = q.c[t][i];
+                if constexpr (COL == TK3D_MLP_COL_ACT)
+                    v = relu(__builtin_fmaf(v, col_act[t].x, col_act[t].y));
+                y[t][i] = v;
+            }
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+#pragma unroll
+            for (int u = 0; u < TA; ++u)
+#pragma unroll
+                for (int w = 0; w < TB; ++w)
+                    acc[u][w] = __builtin_amdgcn_mfma_f32_32x32x2f32(x[u][i], y[w][i], acc[u][w], 0, 0, 0);
+    };
+
+    const int stride = gridDim.x * kWaves;
+    int unit = blockIdx.x * kWaves + wave;
+    if (unit < a.total) {
+        Part now, next;
+        load(now, unit, 0);
+        for (; unit < a.total; unit += stride) {
+            load(next, unit, 1);
+            multiply(now, unit, 0);
+            if (unit + stride < a.total)
+                load(now, unit + stride, 0);
+            multiply(next, unit, 1);
+        }
+    }
+
+    constexpr int TILE = 16 * TK_WAVE;
+#pragma unroll
+    for (int i = 0; i < TA; ++i)
+#pragma unroll
+        for (int j = 0; j < TB; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e)
+                sums[((wave * TA + i) * TB + j) * TILE + e * TK_WAVE + lane] = acc[i][j][e];
+    __syncthreads();
+    for (int i = tid; i < TA * TB * TILE; i += kBlock) {
+        float s = 0.0f;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w)
+            s += sums[w * TA * TB * TILE + i];
+        const int tile = i / TILE, e = (i % TILE) / TK_WAVE, l = i % TK_WAVE;
+        const int row = rbase + (tile / TB) * 32 + 8 * (e >> 2) + 4 * (l >> 5) + (e & 3);
+        const int col = cbase + (tile % TB) * 32 + (l & 31);
+        if (row < R && col < C)
+            p.partial[((int64_t)blockIdx.x * R + row) * C + col] = s;
+    }
+    if constexpr (ROW == TK3D_MLP_ROW_ACT) {
+        if (p.rowsum && blockIdx.z == 0) {
+            __syncthreads();
+#pragma unroll
+            for (int t = 0; t < TA; ++t) {
+                const float s = total[t] + __shfl_xor(total[t], 32);
+                if (half == 0)
+                    sums[wave * (32 * TA) + t * 32 + l32] = s;
+            }
+            __syncthreads();
+            if (tid < 32 * TA && rbase + tid < R) {
+                float s = 0.0f;
+                for (int w = 0; w < kWaves; ++w)
+                    s += sums[w * (32 * TA) + tid];
+                p.rowsum[(int64_t)blockIdx.x * R + rbase + tid] = s;
+            }
+        }
+    }
+}
+
+constexpr int kMaxSums = 8;
+struct SumArgs {
+    tk3d_mlp_sum s[kMaxSums];
+};
+
+__global__ void __launch_bounds__(kBlock) mlp_sum_kernel(SumArgs a)
+{
+    const tk3d_mlp_sum &s = a.s[blockIdx.y];
+    const int n = s.R * s.C;
+    for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
+        double sum = 0.0;
+        for (int k = 0; k < s.splits; ++k)
+            sum += (double)s.partial[(int64_t)k * n + i];
+        const int r = i / s.C;
+        s.out[(int64_t)r * s.ld + (i - r * s.C)] = (float)sum;
+    }
+}
+
+// ---- statistics and coefficients ---------------------------------------------------------------------
+
+// Sum of (x, y) over the block; the result is valid in every thread.
+__device__ __forceinline__ double2 block_sum(double2 v, double2 *lds)
+{
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        v.x += __shfl_xor(v.x, off);
+        v.y += __shfl_xor(v.y, off);
+    }
+    const int waves = blockDim.x >> 6;
+    if ((threadIdx.x & 63) == 0)
+        lds[threadIdx.x >> 6] = v;
+    __syncthreads();
+    double2 s = lds[0];
+    for (int w = 1; w < waves; ++w) {
+        s.x += lds[w].x;
+        s.y += lds[w].y;
+    }
+    return s;
+}
+
+__device__ __forceinline__ double2 slot_sum(const void *partial, int slots, int c, double2 *lds)
+{
+    const double2 *row = reinterpret_cast<const double2 *>(partial) + (int64_t)c * slots;
+    double2 v{0.0, 0.0};
+    for (int i = threadIdx.x; i < slots; i += blockDim.x) {
+        v.x += row[i].x;
+        v.y += row[i].y;
+    }
+    return block_sum(v, lds);
+}
+
+__global__ void __launch_bounds__(kBlock)
+    mlp_statistics_kernel(const void *partial, int slots, double n, float momentum, float *mean,
+                          float *var, float *running_mean, float *running_var, int64_t *batches)
+{
+    __shared__ double2 lds[kWaves];
+    const int c = blockIdx.x;
+    const double2 s = slot_sum(partial, slots, c, lds);
+    if (threadIdx.x == 0) {
+        const double m = s.x / n;
+        double v = s.y / n - m * m;
+        v = v < 0.0 ? 0.0 : v;  // (NaN stays)
+        mean[c] = (float)m;
+        var[c] = (float)v;
+        if (running_mean) {
+            running_mean[c] = (float)((1.0 - (double)momentum) * running_mean[c] + (double)momentum * m);
+            running_var[c] = (float)((1.0 - (double)momentum) * running_var[c] + (double)momentum * (v * n / (n - 1.0)));
+        }
+        if (batches && c == 0)
+            *batches += 1;
+    }
+}
+
+struct Coefficients {
+    f32x4 abd;
+    float dgamma, dbeta;
+};
+
+__device__ __forceinline__ Coefficients grad_coefficients(double2 s, double n, const tk3d_mlp_norm &norm,
+                                                          int c, int frozen)
+{
+    const double is = 1.0 / __builtin_sqrt((double)norm.var[c] + (double)norm.eps);
+    const double gamma = norm.gamma[c], mean = norm.mean[c];
+    const double b = frozen ? 0.0 : -gamma * is * is * is * s.y / n;
+    const double d = frozen ? 0.0 : -gamma * is * s.x / n - b * mean;
+    return {f32x4{(float)(gamma * is), (float)b, (float)d, 0.0f}, (float)(s.y * is), (float)s.x};
+}
+
+__global__ void __launch_bounds__(kBlock)
+    mlp_grad_coefficients_kernel(const void *partial, int slots, double n, tk3d_mlp_norm norm,
+                                 int frozen, float *coef, float *dgamma, float *dbeta)
+{
+    __shared__ double2 lds[kWaves];
+    const int c = blockIdx.x;
+    const double2 s = slot_sum(partial, slots, c, lds);
+    if (threadIdx.x == 0) {
+        const Coefficients k = grad_coefficients(s, n, norm, c, frozen);
+        reinterpret_cast<f32x4 *>(coef)[c] = k.abd;
+        dgamma[c] = k.dgamma;
+        dbeta[c] = k.dbeta;
+    }
+}
+
+__global__ void __launch_bounds__(kBlock)
+    mlp_mask_sums_kernel(const float *g, const float *y, int B, int C, int P, tk3d_mlp_norm norm,
+                         double2 *partial, int slots)
+{
+    __shared__ double2 lds[kWaves];
+    const int c = blockIdx.y;
+    const f32x2 ss = scale_shift(norm, c);
+    const float mean = norm.mean[c];
+    float s1 = 0.0f, s2 = 0.0f;
+    const auto add = [&](float gv, float yv) {
+        const float e = passes(__builtin_fmaf(yv, ss.x, ss.y)) ? gv : 0.0f;
+        s1 += e;
+        s2 = __builtin_fmaf(e, yv - mean, s2);
+    };
+    for (int b = 0; b < B; ++b) {
+        const int64_t row = ((int64_t)b * C + c) * P;
+        if ((P & 3) == 0) {
+            for (int i = (blockIdx.x * kBlock + threadIdx.x) * 4; i < P; i += gridDim.x * kBlock * 4) {
+                const f32x4 gv = *reinterpret_cast<const f32x4 *>(g + row + i);
+                const f32x4 yv = *reinterpret_cast<const f32x4 *>(y + row + i);
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    add(gv[j], yv[j]);
+            }
+        } else {
+            for (int i = blockIdx.x * kBlock + threadIdx.x; i < P; i += gridDim.x * kBlock)
+                add(g[row + i], y[row + i]);
+        }
+    }
+    const double2 s = block_sum(double2{s1, s2}, lds);
+    if (threadIdx.x == 0)
+        partial[(int64_t)c * slots + blockIdx.x] = s;
+}
+
+// f(value, channel constants) over rows of P values; blockIdx.y = row, channel = row % C.
+__global__ void __launch_bounds__(kBlock)
+    mlp_activate_kernel(const float *y, int C, int P, tk3d_mlp_norm norm, float *z)
+{
+    const int64_t row = (int64_t)blockIdx.y * P;
+    const f32x2 ss = scale_shift(norm, blockIdx.y % C);
+    if ((P & 3) == 0) {
+        for (int i = (blockIdx.x * kBlock + threadIdx.x) * 4; i < P; i += gridDim.x * kBlock * 4) {
+            f32x4 v = *reinterpret_cast<const f32x4 *>(y + row + i);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                v[j] = relu(__builtin_fmaf(v[j], ss.x, ss.y));
+            *reinterpret_cast<f32x4 *>(z + row + i) = v;
+        }
+    } else {
+        for (int i = blockIdx.x * kBlock + threadIdx.x; i < P; i += gridDim.x * kBlock)
+            z[row + i] = relu(__builtin_fmaf(y[row + i], ss.x, ss.y));
+    }
+}
+
+__global__ void __launch_bounds__(kBlock)
+    mlp_grad_apply_kernel(float *e, const float *y, const float *coef, int C, int P)
+{
+    const int64_t row = (int64_t)blockIdx.y * P;
+    const f32x4 k = reinterpret_cast<const f32x4 *>(coef)[blockIdx.y % C];
+    const auto f = [&](float ev, float yv) {
+        return __builtin_fmaf(k.x, ev, __builtin_fmaf(k.y, yv, k.z));
+    };
+    if ((P & 3) == 0) {
+        for (int i = (blockIdx.x * kBlock + threadIdx.x) * 4; i < P; i += gridDim.x * kBlock * 4) {
+            f32x4 v = *reinterpret_cast<const f32x4 *>(e + row + i);
+            const f32x4 w = *reinterpret_cast<const f32x4 *>(y + row + i);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                v[j] = f(v[j], w[j]);
+            *reinterpret_cast<f32x4 *>(e + row + i) = v;
+        }
+    } else {
+        for (int i = blockIdx.x * kBlock + threadIdx.x; i < P; i += gridDim.x * kBlock)
+            e[row + i] = f(e[row + i], y[row + i]);
+    }
+}
+
+// ---- pooled layers, backward ---------------------------------------------------------------------------
+
+// One workgroup per channel: the sums, then the coefficients, then the sparse gradient.
+__global__ void __launch_bounds__(1024)
+    mlp_pool_grad_kernel(const float *g, const float *extreme, const unsigned char *arg, int B, int C,
+                         int M, double n, tk3d_mlp_norm norm, int frozen, int2 *sel, float *coef,
+                         float *dgamma, float *dbeta)
+{
+    __shared__ double2 lds[16];
+    const int c = blockIdx.x;
+    const f32x2 ss = scale_shift(norm, c);
+    const float mean = norm.mean[c];
+    const int count = B * M;
+    const auto at = [&](int i) {
+        const int b = i / M;
+        return ((int64_t)b * C + c) * M + (i - b * M);
+    };
+    double2 v{0.0, 0.0};
+    for (int i = threadIdx.x; i < count; i += blockDim.x) {
+        const int64_t j = at(i);
+        const float y = extreme[j];
+        const float e = passes(__builtin_fmaf(y, ss.x, ss.y)) ? g[j] : 0.0f;
+        v.x += e;
+        v.y += (double)e * (double)(y - mean);
+    }
+    const Coefficients k = grad_coefficients(block_sum(v, lds), n, norm, c, frozen);
+    if (threadIdx.x == 0) {
+        reinterpret_cast<f32x4 *>(coef)[c] = k.abd;
+        dgamma[c] = k.dgamma;
+        dbeta[c] = k.dbeta;
+    }
+    for (int i = threadIdx.x; i < count; i += blockDim.x) {
+        const int64_t j = at(i);
+        const float e = passes(__builtin_fmaf(extreme[j], ss.x, ss.y)) ? g[j] : 0.0f;
+        sel[j] = int2{__float_as_int(k.abd.x * e), (int)arg[j]};
+    }
+}
+
+constexpr int kT = 16;
+
+// gram[k][c] = sum_o W[o][k] b[o] W[o][c]; the first row of blocks also adds up bias[c].
+__global__ void __launch_bounds__(kT *kT)
+    mlp_pool_gram_kernel(const float *w, const float *coef, int O, int I, float *gram, float *bias)
+{
+    __shared__ float wk[kT][kT + 1], wc[kT][kT + 1];
+    __shared__ float dd[kT];
+    const int x = threadIdx.x % kT, y = threadIdx.x / kT;
+    const int k = blockIdx.y * kT, c = blockIdx.x * kT;
+    float sum = 0.0f, off = 0.0f;
+    for (int o = 0; o < O; o += kT) {
+        const bool in = o + y < O;
+        wk[y][x] = in && k + x < I ? w[(int64_t)(o + y) * I + k + x] * coef[(o + y) * 4 + 1] : 0.0f;
+        wc[y][x] = in && c + x < I ? w[(int64_t)(o + y) * I + c + x] : 0.0f;
+        if (x == 0)
+            dd[y] = in ? coef[(o + y) * 4 + 2] : 0.0f;
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kT; ++i) {
+            sum = __builtin_fmaf(wk[i][y], wc[i][x], sum);
+            off = __builtin_fmaf(dd[i], wc[i][x], off);
+        }
+        __syncthreads();
+    }
+    if (k + y < I && c + x < I)
+        gram[(int64_t)(k + y) * I + c + x] = sum;
+    if (blockIdx.y == 0 && y == 0 && c + x < I)
+        bias[c + x] = off;
+}
+
+// dw[o][i] += b[o] (W xx)[o][i] + d[o] xsum[i]
+__global__ void __launch_bounds__(kT *kT)
+    mlp_pool_weight_grad_kernel(const float *w, const float *coef, const float *xx, const float *xsum,
+                                int O, int I, float *dw)
+{
+    __shared__ float wt[kT][kT + 1], xt[kT][kT + 1];
+    const int x = threadIdx.x % kT, y = threadIdx.x / kT;
+    const int o = blockIdx.y * kT + y, i = blockIdx.x * kT + x;
+    float sum = 0.0f;
+    for (int k = 0; k < I; k += kT) {
+        wt[y][x] = o < O && k + x < I ? w[(int64_t)o * I + k + x] : 0.0f;
+        xt[y][x] = k + y < I && i < I ? xx[(int64_t)(k + y) * I + i] : 0.0f;
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < kT; ++j)
+            sum = __builtin_fmaf(wt[y][j], xt[j][x], sum);
+        __syncthreads();
+    }
+    if (o < O && i < I) {
+        float &out = dw[(int64_t)o * I + i];
+        out = __builtin_fmaf(coef[o * 4 + 1], sum, __builtin_fmaf(coef[o * 4 + 2], xsum[i], out));
+    }
+}
+
+// ---- the first layer behind a grouping -------------------------------------------------------------------
+//
+// The layer is linear, so its product with the features is taken once per point (u, stored with a
+// point's channels side by side) and not once per neighbour; what a neighbour adds is its centred
+// coordinates. A lane is a grouped position: it gathers 128 bytes of its point's row and writes
+// 32 channels, each a run over the wave.
+
+constexpr int kGroupChannels = 32;
+
+template <bool FEATURES>
+__global__ void __launch_bounds__(kBlock, 2)
+    mlp_group_kernel(const float *__restrict__ u, const float *__restrict__ xyz,
+                     const float *__restrict__ centre, const int64_t *__restrict__ index,
+                     const float *__restrict__ wx, int ldw, int C, int N, int M, int S, int tiles,
+                     int total, float *__restrict__ out, float *__restrict__ rel,
+                     double2 *__restrict__ partial, int slots)
+{
+    __shared__ f32x4 weights[kGroupChannels];
+    __shared__ double2 sums[kWaves][kGroupChannels];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int cbase = blockIdx.y * kGroupChannels;
+    const int P = M * S;
+    const bool vec = (C & 3) == 0;
+    if (tid < kGroupChannels) {
+        f32x4 w{0.0f, 0.0f, 0.0f, 0.0f};
+        if (cbase + tid < C)
+            for (int j = 0; j < 3; ++j)
+                w[j] = wx[(int64_t)(cbase + tid) * ldw + j];
+        weights[tid] = w;
+    }
+    __syncthreads();
+
+    float shift[kGroupChannels], s1[kGroupChannels], s2[kGroupChannels];
+#pragma unroll
+    for (int i = 0; i < kGroupChannels; ++i)
+        shift[i] = s1[i] = s2[i] = 0.0f;
+    double n = 0.0;
+    bool fresh = true;
+    for (int tile = blockIdx.x; tile < total; tile += gridDim.x) {
+        const int b = tile / tiles;
+        const int pos = (tile - b * tiles) * kBlock + tid;
+        const bool in = pos < P;
+        const int p = in ? pos : P - 1;
+        const int m = p / S;
+        const int64_t j64 = index[(int64_t)b * P + p];
+        const bool hit = j64 >= 0 && j64 < N;
+        const int j = hit ? (int)j64 : 0;
+        float r[3];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            const float x = xyz[((int64_t)b * 3 + d) * N + j];
+            r[d] = (hit ? x : 0.0f) - centre[((int64_t)b * 3 + d) * M + m];
+            if (rel && blockIdx.y == 0 && in)
+                rel[((int64_t)b * 3 + d) * P + p] = r[d];
+        }
+        float v[kGroupChannels];
+        const float *row = FEATURES ? u + ((int64_t)b * N + j) * C + cbase : nullptr;
+#pragma unroll
+        for (int i = 0; i < kGroupChannels; i += 4) {
+            f32x4 f{0.0f, 0.0f, 0.0f, 0.0f};
+            if constexpr (FEATURES) {
+                if (vec && cbase + i < C) {
+                    f = *reinterpret_cast<const f32x4 *>(row + i);
+                } else if (!vec) {
+#pragma unroll
+                    for (int d = 0; d < 4; ++d)
+                        f[d] = cbase + i + d < C ? row[i + d] : 0.0f;
+                }
+            }
+#pragma unroll
+            for (int d = 0; d < 4; ++d)
+                v[i + d] = hit ? f[d] : 0.0f;
+        }
+#pragma unroll
+        for (int i = 0; i < kGroupChannels; ++i) {
+            const f32x4 w = weights[i];
+            v[i] = __builtin_fmaf(w.x, r[0], __builtin_fmaf(w.y, r[1], __builtin_fmaf(w.z, r[2], v[i])));
+            if (in && cbase + i < C)
+                out[((int64_t)b * C + cbase + i) * P + pos] = v[i];
+        }
+        if (fresh) {
+#pragma unroll
+            for (int i = 0; i < kGroupChannels; ++i)
+                shift[i] = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v[i])));
+            fresh = false;
+        }
+        if (in) {
+            n += 1.0;
+#pragma unroll
+            for (int i = 0; i < kGroupChannels; ++i) {
+                const float d = v[i] - shift[i];
+                s1[i] += d;
+                s2[i] = __builtin_fmaf(d, d, s2[i]);
+            }
+        }
+    }
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1)
+        n += __shfl_xor(n, off);
+#pragma unroll
+    for (int i = 0; i < kGroupChannels; ++i) {
+        float a = s1[i], q = s2[i];
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            a += __shfl_xor(a, off);
+            q += __shfl_xor(q, off);
+        }
+        if (lane == 0) {
+            const double sh = n > 0.0 ? (double)shift[i] : 0.0;
+            sums[wave][i] = double2{a + n * sh, q + 2.0 * sh * a + n * sh * sh};
+        }
+    }
+    __syncthreads();
+    if (tid < kGroupChannels && cbase + tid < C) {
+        double2 s = sums[0][tid];
+        for (int w = 1; w < kWaves; ++w) {
+            s.x += sums[w][tid].x;
+            s.y += sums[w][tid].y;
+        }
+        partial[(int64_t)(cbase + tid) * slots + blockIdx.x] = s;
+    }
+}
+
+// ---- launches ------------------------------------------------------------------------------------------
+
+constexpr int kWeightBytes = 64 << 10;  // weights in LDS: two workgroups to a CU
+
+struct Shape {
+    int pt, ct;
+};
+
+// The largest wave tile that still gives every SIMD of the chip a wave; 16-byte rows need lengths
+// that are multiples of four, a group of 64 positions needs a tile that holds it.
+Shape pick_shape(int out, const tk3d_mlp_product &p)
+{
+    const int simds = 4 * tk_cu_count();
+    const auto waves = [&](int pt, int ct) {
+        return (int64_t)p.B * ((p.P + 32 * pt - 1) / (32 * pt)) * ((p.C + 32 * ct - 1) / (32 * ct));
+    };
+    const bool pooled = out == TK3D_MLP_OUT_POOL || out == TK3D_MLP_OUT_POOL_EVAL;
+    if (p.P % 4 != 0)
+        return {1, 1};
+    if (p.C <= 32 && waves(4, 1) >= simds)
+        return {4, 1};
+    if (p.C > 32 && waves(4, 2) >= simds)
+        return {4, 2};
+    if (waves(2, 2) >= simds || (pooled && p.group > 32))
+        return {2, 2};
+    return {1, 1};
+}
+
+int fill(const tk3d_mlp_product &p, int in, int out, Shape s, GemmArgs &g)
+{
+    g.p = p;
+    g.tiles = (p.P + 32 * s.pt - 1) / (32 * s.pt);
+    g.total = p.B * g.tiles;
+    const bool two = in == TK3D_MLP_IN_RAW2 || in == TK3D_MLP_IN_POOL;
+    g.kg0 = (p.src[0].K + 7) / 8;
+    g.kg = g.kg0 + (two ? (p.src[1].K + 7) / 8 : 0);
+    const int group_bytes = s.ct * 1024;
+    g.chunk = g.kg * group_bytes <= kWeightBytes ? g.kg : kWeightBytes / 2 / group_bytes;
+    g.coef_bytes = in == TK3D_MLP_IN_RAW || in == TK3D_MLP_IN_RAW2 ? 0
+                   : in == TK3D_MLP_IN_GRAD ? g.kg * 8 * 16
+                   : in == TK3D_MLP_IN_GRAD_OUT ? g.kg * 8 * 24 : g.kg * 8 * 8;
+    const int cblocks = (p.C + 32 * s.ct - 1) / (32 * s.ct);
+    int wgs = (g.total + kWaves - 1) / kWaves;
+    int most = (2 * tk_cu_count() + cblocks - 1) / cblocks;
+    // (a multiple of the XCDs, so that the channel blocks of a position share an L2)
+    most = (most + 7) & ~7;
+    g.slots = wgs < most ? wgs : most;
+    return cblocks;
+}
+
+template <int IN, int OUT, int PT, int CT>
+int launch_product(const GemmArgs &g, int cblocks, hipStream_t stream)
+{
+    int bytes = g.coef_bytes + g.chunk * CT * 1024;
+    const int sum_bytes = kWaves * 32 * CT * 16;
+    bytes = bytes > sum_bytes ? bytes : sum_bytes;
+    if (bytes > 150 << 10)
+        return TK3D_ERR_UNSUPPORTED;
+    const int rc = tk_allow_dynamic_lds<mlp_product_kernel<IN, OUT, PT, CT>>(150 << 10);
+    if (rc != TK3D_OK)
+        return rc;
+    mlp_product_kernel<IN, OUT, PT, CT><<<dim3(g.slots, cblocks), kBlock, bytes, stream>>>(g);
+    return tk_launch_status();
+}
+
+template <int IN, int OUT>
+int launch_shape(const GemmArgs &g, Shape s, int cblocks, hipStream_t stream)
+{
+    if (s.pt == 4 && s.ct == 2)
+        return launch_product<IN, OUT, 4, 2>(g, cblocks, stream);
+    if (s.pt == 4)
+        return launch_product<IN, OUT, 4, 1>(g, cblocks, stream);
+    if (s.pt == 2)
+        return launch_product<IN, OUT, 2, 2>(g, cblocks, stream);
+    return launch_product<IN, OUT, 1, 1>(g, cblocks, stream);
+}
+
+template <int ROW, int COL, int TA, int TB>
+int launch_outer(const OuterArgs &a, int splits, hipStream_t stream)
+{
+    const int bytes = kWaves * TA * TB * 16 * TK_WAVE * 4;
+    const int rc = tk_allow_dynamic_lds<mlp_outer_kernel<ROW, COL, TA, TB>>(bytes);
+    if (rc != TK3D_OK)
+        return rc;
+    const dim3 grid(splits, (a.p.row.K + 32 * TA - 1) / (32 * TA), (a.p.col.K + 32 * TB - 1) / (32 * TB));
+    mlp_outer_kernel<ROW, COL, TA, TB><<<grid, kBlock, bytes, stream>>>(a);
+    return tk_launch_status();
+}
+
+template <int ROW, int COL>
+int launch_outer_shape(const OuterArgs &a, int splits, hipStream_t stream)
+{
+    const bool ra = a.p.row.K > 32, cb = a.p.col.K > 32;
+    if (ra && cb)
+        return launch_outer<ROW, COL, 2, 2>(a, splits, stream);
+    if (ra)
+        return launch_outer<ROW, COL, 2, 1>(a, splits, stream);
+    if (cb)
+        return launch_outer<ROW, COL, 1, 2>(a, splits, stream);
+    return launch_outer<ROW, COL, 1, 1>(a, splits, stream);
+}
+
+// Workgroups along a row of P values, and the most rows (whole batch elements) of one launch.
+int row_blocks(int P)
+{
+    const int x = (P + kBlock * 4 * 4 - 1) / (kBlock * 4 * 4);
+    return x < 1 ? 1 : x > 64 ? 64 : x;
+}
+int64_t rows_at_once(int C) { return C < 65535 ? 65535 / C * C : C; }
+
+// A row's byte offsets are 32-bit in the kernels.
+bool indexable(int64_t rows, int64_t P) { return tk_fits(1 << 29, rows + 8, P); }
+
+}  // namespace
+
+extern "C" {
+
+int tk3d_mlp_product_slots(int in, int out, const tk3d_mlp_product *p)
+{
+    GemmArgs g;
+    fill(*p, in, out, pick_shape(out, *p), g);
+    return g.slots;
+}
+
+int tk3d_mlp_product_f32(int in, int out, const tk3d_mlp_product *p, void *stream_)
+{
+    if (!p)
+        return TK3D_ERR_NULL_POINTER;
+    const bool two = in == TK3D_MLP_IN_RAW2 || in == TK3D_MLP_IN_POOL;
+    if (p->B < 0 || p->C <= 0 || p->P < 0 || p->src[0].K <= 0 || (two && p->src[1].K <= 0))
+        return TK3D_ERR_BAD_SIZE;
+    if (p->B == 0 || p->P == 0)
+        return TK3D_OK;
+    const int widest = two && p->src[1].K > p->src[0].K ? p->src[1].K : p->src[0].K;
+    if (!indexable(widest, p->P) || !indexable(p->C, p->P) || p->C > 65535 * 32)
+        return TK3D_ERR_UNSUPPORTED;
+    const bool grouped = in == TK3D_MLP_IN_POOL || out == TK3D_MLP_OUT_POOL || out == TK3D_MLP_OUT_POOL_EVAL;
+    if (grouped && ((p->group != 32 && p->group != 64) || p->M * p->group != p->P))
+        return TK3D_ERR_UNSUPPORTED;
+    const Shape s = pick_shape(out, *p);
+    GemmArgs g;
+    const int cblocks = fill(*p, in, out, s, g);
+    const hipStream_t stream = (hipStream_t)stream_;
+#define TK_CASE(IN, OUT)                                                                                 if (in == TK3D_MLP_##IN && out == TK3D_MLP_##OUT)                                                        return launch_shape<IN, OUT>(g, s, cblocks, stream);
+    TK_CASE(IN_RAW, OUT_STATS)
+    TK_CASE(IN_RAW, OUT_EVAL)
+    TK_CASE(IN_RAW, OUT_PLAIN)
+    TK_CASE(IN_RAW, OUT_POINTS)
+    TK_CASE(IN_RAW, OUT_POOL_EVAL)
+    TK_CASE(IN_RAW2, OUT_STATS)
+    TK_CASE(IN_RAW2, OUT_EVAL)
+    TK_CASE(IN_ACT, OUT_STATS)
+    TK_CASE(IN_ACT, OUT_EVAL)
+    TK_CASE(IN_ACT, OUT_POOL)
+    TK_CASE(IN_ACT, OUT_POOL_EVAL)
+    TK_CASE(IN_GRAD, OUT_MASK)
+    TK_CASE(IN_GRAD, OUT_PLAIN)
+    TK_CASE(IN_GRAD_OUT, OUT_MASK)
+    TK_CASE(IN_GRAD_OUT, OUT_PLAIN)
+    TK_CASE(IN_POOL, OUT_MASK)
+#undef TK_CASE
+    return TK3D_ERR_UNSUPPORTED;
+}
+
+int tk3d_mlp_outer_splits(const tk3d_mlp_outer *p)
+{
+    const int ta = p->row.K > 32 ? 2 : 1, tb = p->col.K > 32 ? 2 : 1;
+    const int blocks = ((p->row.K + 32 * ta - 1) / (32 * ta)) * ((p->col.K + 32 * tb - 1) / (32 * tb));
+    const int64_t units = (int64_t)p->B * ((p->P + 31) / 32);
+    // two workgroups to a CU, and at least two units to a wave
+    int64_t splits = (2 * tk_cu_count() + blocks - 1) / blocks;
+    const int64_t most = (units + 2 * kWaves - 1) / (2 * kWaves);
+    splits = splits > most ? most : splits;
+    return splits < 1 ? 1 : (int)splits;
+}
+
+int tk3d_mlp_outer_f32(int row, int col, const tk3d_mlp_outer *p, void *stream_)
+{
+    if (!p)
+        return TK3D_ERR_NULL_POINTER;
+    if (p->B <= 0 || p->P <= 0 || p->row.K <= 0 || p->col.K <= 0)
+        return TK3D_ERR_BAD_SIZE;
+    if (!indexable(p->row.K, p->P) || !indexable(p->col.K, p->P))
+        return TK3D_ERR_UNSUPPORTED;
+    if (row == TK3D_MLP_ROW_POOL && (p->group % 32 != 0 || p->group * p->M != p->P))
+        return TK3D_ERR_UNSUPPORTED;
+    OuterArgs a;
+    a.p = *p;
+    a.units = (p->P + 31) / 32;
+    a.total = p->B * a.units;
+    const int splits = tk3d_mlp_outer_splits(p);
+    const hipStream_t stream = (hipStream_t)stream_;
+#define TK_CASE(ROW, COL)                                                                                if (row == ROW && col == COL)                                                                            return launch_outer_shape<ROW, COL>(a, splits, stream);
+    TK_CASE(TK3D_MLP_ROW_RAW, TK3D_MLP_COL_RAW)
+    TK_CASE(TK3D_MLP_ROW_GRAD, TK3D_MLP_COL_RAW)
+    TK_CASE(TK3D_MLP_ROW_GRAD, TK3D_MLP_COL_ACT)
+    TK_CASE(TK3D_MLP_ROW_GRAD_OUT, TK3D_MLP_COL_RAW)
+    TK_CASE(TK3D_MLP_ROW_GRAD_OUT, TK3D_MLP_COL_ACT)
+    TK_CASE(TK3D_MLP_ROW_POOL, TK3D_MLP_COL_ACT)
+    TK_CASE(TK3D_MLP_ROW_ACT, TK3D_MLP_COL_ACT)
+#undef TK_CASE
+    return TK3D_ERR_UNSUPPORTED;
+}
+
+int tk3d_mlp_sum_f32(const tk3d_mlp_sum *sums, int n, void *stream)
+{
+    for (int i = 0; i < n; i += kMaxSums) {
+        SumArgs a;
+        int most = 0;
+        const int m = n - i < kMaxSums ? n - i : kMaxSums;
+        for (int j = 0; j < m; ++j) {
+            a.s[j] = sums[i + j];
+            const int size = a.s[j].R * a.s[j].C;
+            most = size > most ? size : most;
+        }
+        int blocks = (most + kBlock - 1) / kBlock;
+        blocks = blocks < 1 ? 1 : blocks > 1024 ? 1024 : blocks;
+        mlp_sum_kernel<<<dim3(blocks, m), kBlock, 0, (hipStream_t)stream>>>(a);
+    }
+    return tk_launch_status();
+}
+
+int tk3d_mlp_statistics_f32(const void *partial, int slots, int64_t n, int C, float momentum,
+                            float *mean, float *var, float *running_mean, float *running_var,
+                            int64_t *batches, void *stream)
+{
+    mlp_statistics_kernel<<<C, kBlock, 0, (hipStream_t)stream>>>(partial, slots, (double)n, momentum,
+                                                               mean, var, running_mean, running_var, batches);
+    return tk_launch_status();
+}
+
+int tk3d_mlp_grad_coefficients_f32(const void *partial, int slots, int64_t n, int C,
+                                   const tk3d_mlp_norm *norm, int frozen, float *coef,
+                                   float *dgamma, float *dbeta, void *stream)
+{
+    mlp_grad_coefficients_kernel<<<C, kBlock, 0, (hipStream_t)stream>>>(partial, slots, (double)n, *norm,
+                                                                      frozen, coef, dgamma, dbeta);
+    return tk_launch_status();
+}
+
+int tk3d_mlp_mask_slots(int B, int C, int P)
+{
+    int slots = (2048 + C - 1) / C;
+    const int most = (P + kBlock * 4 - 1) / (kBlock * 4);
+    slots = slots > most ? most : slots;
+    return slots < 1 ? 1 : slots;
+}
+
+int tk3d_mlp_mask_sums_f32(const float *g, const float *y, int B, int C, int P,
+                           const tk3d_mlp_norm *norm, void *partial, void *stream)
+{
+    const int slots = tk3d_mlp_mask_slots(B, C, P);
+    mlp_mask_sums_kernel<<<dim3(slots, C), kBlock, 0, (hipStream_t)stream>>>(
+        g, y, B, C, P, *norm, reinterpret_cast<double2 *>(partial), slots);
+    return tk_launch_status();
+}
+
+int tk3d_mlp_activate_f32(const float *y, int64_t rows, int C, int P, const tk3d_mlp_norm *norm,
+                          float *z, void *stream)
+{
+    const int64_t step = rows_at_once(C);
+    for (int64_t r = 0; r < rows; r += step)
+        mlp_activate_kernel<<<dim3(row_blocks(P), (unsigned)(rows - r < step ? rows - r : step)), kBlock, 0,
+                              (hipStream_t)stream>>>(y + r * P, C, P, *norm, z + r * P);
+    return tk_launch_status();
+}
+
+int tk3d_mlp_grad_apply_f32(float *e, const float *y, const float *coef, int B, int C, int P,
+                            void *stream)
+{
+    const int64_t rows = (int64_t)B * C, step = rows_at_once(C);
+    for (int64_t r = 0; r < rows; r += step)
+        mlp_grad_apply_kernel<<<dim3(row_blocks(P), (unsigned)(rows - r < step ? rows - r : step)), kBlock, 0,
+                                (hipStream_t)stream>>>(e + r * P, y + r * P, coef, C, P);
+    return tk_launch_status();
+}
+
+int tk3d_mlp_pool_grad_f32(const float *g, const float *extreme, const unsigned char *arg, int B,
+                           int C, int M, int64_t positions, const tk3d_mlp_norm *norm, int frozen,
+                           void *sel, float *coef, float *dgamma, float *dbeta, void *stream)
+{
+    mlp_pool_grad_kernel<<<C, 1024, 0, (hipStream_t)stream>>>(
+        g, extreme, arg, B, C, M, (double)positions, *norm, frozen, reinterpret_cast<int2 *>(sel), coef,
+        dgamma, dbeta);
+    return tk_launch_status();
+}
+
+int tk3d_mlp_pool_gram_f32(const float *w, const float *coef, int O, int I, float *gram, float *bias,
+                           void *stream)
+{
+    const int n = (I + kT - 1) / kT;
+    mlp_pool_gram_kernel<<<dim3(n, n), kT * kT, 0, (hipStream_t)stream>>>(w, coef, O, I, gram, bias);
+    return tk_launch_status();
+}
+
+int tk3d_mlp_pool_weight_grad_f32(const float *sparse, int sparse_splits, const float *xx,
+                                  const float *xsum, int xx_splits, const float *w,
+                                  const float *coef, int O, int I, float *scratch, float *dw,
+                                  void *stream)
+{
+    const tk3d_mlp_sum sums[3] = {{sparse, dw, sparse_splits, O, I, I},
+                                  {xx, scratch, xx_splits, I, I, I},
+                                  {xsum, scratch + (int64_t)I * I, xx_splits, 1, I, I}};
+    const int rc = tk3d_mlp_sum_f32(sums, 3, stream);
+    if (rc != TK3D_OK)
+        return rc;
+    mlp_pool_weight_grad_kernel<<<dim3((I + kT - 1) / kT, (O + kT - 1) / kT), kT * kT, 0, (hipStream_t)stream>>>(
+        w, coef, scratch, scratch + (int64_t)I * I, O, I, dw);
+    return tk_launch_status();
+}
+
+int tk3d_mlp_group_slots(int B, int C, int M, int S)
+{
+    const int chunks = (C + kGroupChannels - 1) / kGroupChannels;
+    const int64_t total = (int64_t)B * (((int64_t)M * S + kBlock - 1) / kBlock);
+    int64_t most = (4 * tk_cu_count() + chunks - 1) / chunks;
+    most = (most + 7) & ~7;
+    return (int)(total < most ? total : most);
+}
+
+int tk3d_mlp_group_f32(const float *u, const float *xyz, const float *centre, const int64_t *index,
+                       const float *wx, int ldw, int B, int C, int N, int M, int S, float *y,
+                       float *rel, void *partial, void *stream)
+{
+    if (B <= 0 || C <= 0 || N <= 0 || M <= 0 || S <= 0 || !tk_fits(TK_MAX_I32, M, S))
+        return TK3D_ERR_BAD_SIZE;
+    const int slots = tk3d_mlp_group_slots(B, C, M, S);
+    const int tiles = (M * S + kBlock - 1) / kBlock;
+    if (!tk_fits(TK_MAX_I32, B, tiles))
+        return TK3D_ERR_UNSUPPORTED;
+    const dim3 grid(slots, (C + kGroupChannels - 1) / kGroupChannels);
+    double2 *part = reinterpret_cast<double2 *>(partial);
+    if (u)
+        mlp_group_kernel<true><<<grid, kBlock, 0, (hipStream_t)stream>>>(
+            u, xyz, centre, index, wx, ldw, C, N, M, S, tiles, B * tiles, y, rel, part, slots);
+    else
+        mlp_group_kernel<false><<<grid, kBlock, 0, (hipStream_t)stream>>>(
+            u, xyz, centre, index, wx, ldw, C, N, M, S, tiles, B * tiles, y, rel, part, slots);
+    return tk_launch_status();
+}
+
+}  // extern "C"

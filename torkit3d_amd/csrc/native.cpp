@@ -2,35 +2,21 @@
 // into the C ABI (include/tk3d.h), as a Python extension module (torkit3d_amd/_host.so).
 // A small call is host work only: through ctypes and Python's autograd.Function a chamfer
 // forward + backward on 2 x 1024 points took 100 to 160 us around 27 us of kernels.
-#include <algorithm>
-#include <optional>
-#include <stdexcept>
-#include <string>
-#include <tuple>
-#include <vector>
-
-#include <ATen/ATen.h>
-#include <c10/core/DeviceGuard.h>
-#include <c10/core/GradMode.h>
-#include <c10/hip/HIPStream.h>
 #include <pybind11/pybind11.h>
 #include <pybind11/stl.h>
-#include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/pybind.h>
 
-#include "tk3d.h"
+#include "native.h"
 
 namespace py = pybind11;
-using at::Tensor;
+using namespace tk3d;
 using torch::autograd::AutogradContext;
 using torch::autograd::variable_list;
 
 namespace {
 
 // ---- checks (messages as the reference's TORCH_CHECKs give them; RuntimeError in Python) ----
-
-[[noreturn]] void fail(const std::string &message) { throw std::runtime_error(message); }
 
 void check(bool ok, const std::string &message)
 {
@@ -90,13 +76,6 @@ bool is_f32(const Tensor &t)
     return false;
 }
 
-void done(int code, const char *what)
-{
-    if (code != TK3D_OK)
-        fail(std::string(what) + " failed: " + tk3d_error_string(code) + " (code " +
-             std::to_string(code) + ")");
-}
-
 // ---- device pointers, outputs, stream ---------------------------------------------------------
 
 struct Ptr {  // becomes whatever pointer the entry point takes
@@ -120,14 +99,6 @@ Tensor scratch(const Tensor &t, size_t bytes)
 {
     return bytes ? at::empty({(int64_t)bytes}, t.options().dtype(at::kByte)) : Tensor();
 }
-
-void *stream_of(const Tensor &t)
-{
-    return c10::hip::getCurrentHIPStream(t.device().index()).stream();
-}
-
-// Makes the tensor's GPU the current one (kernels, allocations and streams follow it).
-using OnDeviceOf = c10::OptionalDeviceGuard;
 
 #define TK3D_CALL(is32, name, ...)                                                             \
     done((is32) ? name##_f32(__VA_ARGS__) : name##_f64(__VA_ARGS__), #name)
@@ -663,5 +634,16 @@ PYBIND11_MODULE(_host, m)
         const Tensor x = tensor_arg("input", feature), i = tensor_arg("index", index),
                      w = tensor_arg("weight", weight);
         return unlocked([&] { return interpolate(x, i, w); });
+    });
+    m.def("mlp", [](py::handle x, py::handle x2, py::handle xyz, py::handle centre,
+                    py::handle index, std::vector<Tensor> params, std::vector<Tensor> buffers,
+                    std::vector<double> eps, std::vector<double> momentum, bool training,
+                    int64_t pool) {
+        const Tensor t[] = {optional_arg("x", x), optional_arg("x2", x2), optional_arg("xyz", xyz),
+                            optional_arg("centre", centre), optional_arg("index", index)};
+        return unlocked([&] {
+            return mlp(t[0], t[1], t[2], t[3], t[4], std::move(params), std::move(buffers),
+                       std::move(eps), std::move(momentum), training, pool);
+        });
     });
 }

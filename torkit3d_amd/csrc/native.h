@@ -1,0 +1,44 @@
+// What the parts of the extension module share (native.cpp, native_mlp.cpp).
+#pragma once
+
+#include <algorithm>
+#include <optional>
+#include <stdexcept>
+#include <string>
+#include <tuple>
+#include <vector>
+
+#include <ATen/ATen.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/core/GradMode.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/custom_function.h>
+
+#include "tk3d.h"
+
+namespace tk3d {
+
+using at::Tensor;
+
+[[noreturn]] inline void fail(const std::string &message) { throw std::runtime_error(message); }
+
+inline void done(int code, const char *what)
+{
+    if (code != TK3D_OK)
+        fail(std::string(what) + " failed: " + tk3d_error_string(code) + " (code " +
+             std::to_string(code) + ")");
+}
+
+inline void *stream_of(const Tensor &t)
+{
+    return c10::hip::getCurrentHIPStream(t.device().index()).stream();
+}
+
+// Makes the tensor's GPU the current one (kernels, allocations and streams follow it).
+using OnDeviceOf = c10::OptionalDeviceGuard;
+
+Tensor mlp(Tensor x, Tensor x2, const Tensor &xyz, const Tensor &centre, const Tensor &index,
+           std::vector<Tensor> params, std::vector<Tensor> buffers, std::vector<double> eps,
+           std::vector<double> momentum, bool training, int64_t pool);
+
+}  // namespace tk3d

@@ -1,0 +1,681 @@
+// Host path of the shared MLPs (include/tk3d_mlp.h): which products, sums and small kernels a
+// chain of "1x1 convolution, batch norm, ReLU" layers is made of, forward and backward.
+#include "native.h"
+#include "tk3d_mlp.h"
+
+#include <torch/csrc/autograd/autograd.h>
+
+namespace tk3d {
+namespace {
+
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+float *f32(const Tensor &t) { return t.defined() ? t.data_ptr<float>() : nullptr; }
+
+// What a chain is applied to and how.
+struct Call {
+    // dense input: x [B, C, P] and, if defined, x2 [B, C2, P] behind its channels
+    Tensor x, x2;
+    // grouped input: features [B, C, N] (x above, may be undefined), xyz [B, 3, N],
+    // centre [B, 3, M], index [B, M, S]
+    Tensor xyz, centre, index;
+    int64_t pool = 0;  // maximum over groups of this many consecutive positions, 0: none
+    bool training = false;
+    std::vector<double> eps, momentum;
+    std::vector<Tensor> params;   // weight, gamma, beta of every layer
+    std::vector<Tensor> buffers;  // running mean, running variance, batch count of every layer
+
+    bool grouped() const { return xyz.defined(); }
+    int64_t layers() const { return (int64_t)params.size() / 3; }
+    const Tensor &weight(int64_t l) const { return params[3 * l]; }
+    int64_t out_channels(int64_t l) const { return params[3 * l].size(0); }
+    int64_t in_channels(int64_t l) const { return params[3 * l].size(1); }
+    int64_t batch() const { return grouped() ? xyz.size(0) : x.size(0); }
+    int64_t positions() const { return grouped() ? index.size(1) * index.size(2) : x.size(2); }
+    Tensor like() const { return grouped() ? xyz : x; }
+};
+
+// What the backward needs besides the call: the product of every layer (of a pooled last layer
+// the extremes, and their places), and the statistics it was normalised with.
+struct Kept {
+    std::vector<Tensor> y, mean, var;
+    Tensor arg;
+};
+
+tk3d_mlp_norm norm_of(const Call &c, const Kept &k, int64_t l)
+{
+    return {f32(k.mean[l]), f32(k.var[l]), f32(c.params[3 * l + 1]), f32(c.params[3 * l + 2]),
+            (float)c.eps[l]};
+}
+
+tk3d_mlp_source source(const Tensor &x, const float *w, int64_t wk, int64_t wc)
+{
+    tk3d_mlp_source s{};
+    s.x = f32(x);
+    s.w = w;
+    s.batch_stride = x.size(1) * x.size(2);
+    s.K = (int32_t)x.size(1);
+    s.wk = (int32_t)wk;
+    s.wc = (int32_t)wc;
+    return s;
+}
+
+tk3d_mlp_product product(int64_t B, int64_t C, int64_t P)
+{
+    tk3d_mlp_product p{};
+    p.B = (int32_t)B;
+    p.C = p.C0 = (int32_t)C;
+    p.P = (int32_t)P;
+    p.group = 1;
+    p.M = (int32_t)P;
+    return p;
+}
+
+// Partial sums [C][slots] of (double, double).
+Tensor partial_sums(const Tensor &like, int64_t C, int slots)
+{
+    return at::empty({C, slots, 2}, like.options().dtype(at::kDouble));
+}
+
+// Runs a product with partial sums; returns them and their number per channel.
+std::pair<Tensor, int> summed_product(int in, int out, tk3d_mlp_product &p, const Tensor &like,
+                                      void *stream)
+{
+    const int slots = tk3d_mlp_product_slots(in, out, &p);
+    const Tensor partial = partial_sums(like, p.C, slots);
+    p.partial = partial.data_ptr();
+    done(tk3d_mlp_product_f32(in, out, &p, stream), "tk3d_mlp_product_f32");
+    return {partial, slots};
+}
+
+void run_product(int in, int out, tk3d_mlp_product &p, void *stream)
+{
+    done(tk3d_mlp_product_f32(in, out, &p, stream), "tk3d_mlp_product_f32");
+}
+
+// Evaluation without gradients: every layer leaves its activations.
+Tensor evaluate(const Call &c)
+{
+    const int64_t B = c.batch(), P = c.positions(), L = c.layers();
+    const Tensor like = c.like();
+    void *stream = stream_of(like);
+    Kept k;
+    for (int64_t l = 0; l < L; ++l) {
+        k.mean.push_back(c.buffers[3 * l]);
+        k.var.push_back(c.buffers[3 * l + 1]);
+    }
+    Tensor h;
+    for (int64_t l = 0; l < L; ++l) {
+        const int64_t C = c.out_channels(l), K = c.in_channels(l);
+        const float *w = f32(c.weight(l));
+        tk3d_mlp_product p = product(B, C, P);
+        p.out_norm = norm_of(c, k, l);
+        if (l == 0 && c.grouped()) {
+            const int64_t M = c.index.size(1), S = c.index.size(2), N = c.xyz.size(2);
+            Tensor u;
+            if (c.x.defined()) {
+                u = at::empty({B, N, C}, like.options());
+                tk3d_mlp_product q = product(B, C, N);
+                q.src[0] = source(c.x, w, 1, K);
+                q.out = f32(u);
+                run_product(TK3D_MLP_IN_RAW, TK3D_MLP_OUT_POINTS, q, stream);
+            }
+            h = at::empty({B, C, P}, like.options());
+            const Tensor partial =
+                partial_sums(like, C, tk3d_mlp_group_slots((int)B, (int)C, (int)M, (int)S));
+            done(tk3d_mlp_group_f32(f32(u), f32(c.xyz), f32(c.centre),
+                                    c.index.data_ptr<int64_t>(), w + (K - 3), (int)K, (int)B, (int)C,
+                                    (int)N, (int)M, (int)S, f32(h), nullptr, partial.data_ptr(),
+                                    stream),
+                 "tk3d_mlp_group_f32");
+            continue;
+        }
+        int in = TK3D_MLP_IN_RAW, out = TK3D_MLP_OUT_EVAL;
+        if (l == 0) {
+            p.src[0] = source(c.x, w, 1, K);
+            if (c.x2.defined()) {
+                in = TK3D_MLP_IN_RAW2;
+                p.src[1] = source(c.x2, w + c.x.size(1), 1, K);
+            }
+        } else {
+            p.src[0] = source(h, w, 1, K);
+            if (l == 1 && c.grouped()) {
+                in = TK3D_MLP_IN_ACT;
+                p.in_norm = norm_of(c, k, 0);
+            }
+        }
+        Tensor next;
+        if (c.pool && l == L - 1) {
+            out = TK3D_MLP_OUT_POOL_EVAL;
+            p.group = (int32_t)c.pool;
+            p.M = (int32_t)(P / c.pool);
+            next = at::empty({B, C, p.M}, like.options());
+        } else {
+            next = at::empty({B, C, P}, like.options());
+        }
+        p.out = f32(next);
+        run_product(in, out, p, stream);
+        h = next;
+    }
+    return h;
+}
+
+// Forward that keeps what the backward needs (and, in training, takes batch statistics).
+Tensor forward(const Call &c, Kept &k)
+{
+    const int64_t B = c.batch(), P = c.positions(), L = c.layers();
+    const Tensor like = c.like();
+    void *stream = stream_of(like);
+    for (int64_t l = 0; l < L; ++l) {
+        const int64_t C = c.out_channels(l), K = c.in_channels(l);
+        const float *w = f32(c.weight(l));
+        tk3d_mlp_product p = product(B, C, P);
+        const bool pooled = c.pool && l == L - 1;
+        std::pair<Tensor, int> sums;
+        Tensor y;
+        if (l == 0 && c.grouped()) {
+            const int64_t M = c.index.size(1), S = c.index.size(2), N = c.xyz.size(2);
+            Tensor u;
+            if (c.x.defined()) {
+                u = at::empty({B, N, C}, like.options());
+                tk3d_mlp_product q = product(B, C, N);
+                q.src[0] = source(c.x, w, 1, K);
+                q.out = f32(u);
+                run_product(TK3D_MLP_IN_RAW, TK3D_MLP_OUT_POINTS, q, stream);
+            }
+            y = at::empty({B, C, P}, like.options());
+            sums.second = tk3d_mlp_group_slots((int)B, (int)C, (int)M, (int)S);
+            sums.first = partial_sums(like, C, sums.second);
+            done(tk3d_mlp_group_f32(f32(u), f32(c.xyz), f32(c.centre),
+                                    c.index.data_ptr<int64_t>(), w + (K - 3), (int)K, (int)B, (int)C,
+                                    (int)N, (int)M, (int)S, f32(y), nullptr,
+                                    sums.first.data_ptr(), stream),
+                 "tk3d_mlp_group_f32");
+        } else {
+            int in = TK3D_MLP_IN_ACT, out = TK3D_MLP_OUT_STATS;
+            if (l == 0) {
+                in = TK3D_MLP_IN_RAW;
+                p.src[0] = source(c.x, w, 1, K);
+                if (c.x2.defined()) {
+                    in = TK3D_MLP_IN_RAW2;
+                    p.src[1] = source(c.x2, w + c.x.size(1), 1, K);
+                }
+            } else {
+                p.src[0] = source(k.y[l - 1], w, 1, K);
+                p.in_norm = norm_of(c, k, l - 1);
+            }
+            if (pooled) {
+                out = TK3D_MLP_OUT_POOL;
+                p.group = (int32_t)c.pool;
+                p.M = (int32_t)(P / c.pool);
+                p.out_norm.gamma = f32(c.params[3 * l + 1]);
+                k.arg = at::empty({B, C, p.M}, like.options().dtype(at::kByte));
+                p.arg = k.arg.data_ptr<uint8_t>();
+            }
+            y = at::empty({B, C, pooled ? P / c.pool : P}, like.options());
+            p.out = f32(y);
+            sums = summed_product(in, out, p, like, stream);
+        }
+        k.y.push_back(y);
+        if (c.training) {
+            const Tensor stats = at::empty({2, C}, like.options());
+            k.mean.push_back(stats.select(0, 0));
+            k.var.push_back(stats.select(0, 1));
+            const Tensor &count = c.buffers[3 * l + 2];
+            done(tk3d_mlp_statistics_f32(sums.first.data_ptr(), sums.second, B * P, (int)C,
+                                         (float)c.momentum[l], f32(k.mean[l]), f32(k.var[l]),
+                                         f32(c.buffers[3 * l]), f32(c.buffers[3 * l + 1]),
+                                         count.defined() ? count.data_ptr<int64_t>() : nullptr,
+                                         stream),
+                 "tk3d_mlp_statistics_f32");
+        } else {
+            k.mean.push_back(c.buffers[3 * l]);
+            k.var.push_back(c.buffers[3 * l + 1]);
+        }
+    }
+    const Tensor &last = k.y[L - 1];
+    const Tensor z = at::empty(last.sizes(), like.options());
+    const tk3d_mlp_norm norm = norm_of(c, k, L - 1);
+    done(tk3d_mlp_activate_f32(f32(last), B * last.size(1), (int)last.size(1), (int)last.size(2),
+                               &norm, f32(z), stream),
+         "tk3d_mlp_activate_f32");
+    return z;
+}
+
+struct Grads {
+    Tensor x, x2;
+    std::vector<Tensor> params;
+};
+
+// A weight gradient in partial sums, and where their sum goes.
+struct Pending {
+    std::vector<tk3d_mlp_sum> sums;
+    std::vector<Tensor> alive;
+};
+
+void outer(int row, int col, tk3d_mlp_outer &o, const Tensor &like, float *out, int64_t ld,
+           Pending &pending, void *stream)
+{
+    const int splits = tk3d_mlp_outer_splits(&o);
+    const Tensor partial = at::empty({splits, o.row.K, o.col.K}, like.options());
+    o.partial = f32(partial);
+    done(tk3d_mlp_outer_f32(row, col, &o, stream), "tk3d_mlp_outer_f32");
+    pending.sums.push_back({f32(partial), out, splits, o.row.K, o.col.K, (int32_t)ld});
+    pending.alive.push_back(partial);
+}
+
+Grads backward(const Call &c, const Kept &k, const Tensor &g, bool want_x, bool want_x2)
+{
+    const int64_t B = c.batch(), P = c.positions(), L = c.layers();
+    const Tensor like = c.like();
+    void *stream = stream_of(like);
+    const int frozen = c.training ? 0 : 1;
+    Grads out;
+    out.params.resize(3 * L);
+    for (int64_t l = 0; l < L; ++l) {
+        out.params[3 * l] = at::empty(c.weight(l).sizes(), like.options());
+        const Tensor affine = at::empty({2, c.out_channels(l)}, like.options());
+        out.params[3 * l + 1] = affine.select(0, 0);
+        out.params[3 * l + 2] = affine.select(0, 1);
+    }
+    Pending pending;
+    std::vector<Tensor> coef(L);
+    for (int64_t l = 0; l < L; ++l)
+        coef[l] = at::empty({c.out_channels(l), 4}, like.options());
+    const auto coefficients = [&](int64_t l, const void *partial, int slots) {
+        const tk3d_mlp_norm norm = norm_of(c, k, l);
+        done(tk3d_mlp_grad_coefficients_f32(partial, slots, B * P, (int)c.out_channels(l), &norm,
+                                            frozen, f32(coef[l]), f32(out.params[3 * l + 1]),
+                                            f32(out.params[3 * l + 2]), stream),
+             "tk3d_mlp_grad_coefficients_f32");
+    };
+
+    int64_t l = L - 1;
+    Tensor e = g;
+    bool masked = false;  // whether e already is the gradient behind the norm
+    if (c.pool) {
+        const int64_t O = c.out_channels(l), I = c.in_channels(l), M = P / c.pool;
+        const tk3d_mlp_norm norm = norm_of(c, k, l), inner = norm_of(c, k, l - 1);
+        const Tensor sel = at::empty({B, O, M, 2}, like.options());
+        done(tk3d_mlp_pool_grad_f32(f32(g), f32(k.y[l]), k.arg.data_ptr<uint8_t>(), (int)B, (int)O,
+                                    (int)M, B * P, &norm, frozen, sel.data_ptr(), f32(coef[l]),
+                                    f32(out.params[3 * l + 1]), f32(out.params[3 * l + 2]), stream),
+             "tk3d_mlp_pool_grad_f32");
+        const Tensor gram = at::empty({I + 1, I}, like.options());
+        const float *w = f32(c.weight(l));
+        done(tk3d_mlp_pool_gram_f32(w, f32(coef[l]), (int)O, (int)I, f32(gram), f32(gram) + I * I,
+                                    stream),
+             "tk3d_mlp_pool_gram_f32");
+        tk3d_mlp_product p = product(B, I, P);
+        p.group = (int32_t)c.pool;
+        p.M = (int32_t)M;
+        p.src[0].sel = sel.data_ptr();
+        p.src[0].K = (int32_t)O;
+        p.src[0].w = w;
+        p.src[0].wk = (int32_t)I;
+        p.src[0].wc = 1;
+        p.src[1] = source(k.y[l - 1], f32(gram), I, 1);
+        p.in_norm = p.out_norm = inner;
+        p.yprev = f32(k.y[l - 1]);
+        p.bias = f32(gram) + I * I;
+        e = at::empty({B, I, P}, like.options());
+        p.out = f32(e);
+        const auto sums = summed_product(TK3D_MLP_IN_POOL, TK3D_MLP_OUT_MASK, p, like, stream);
+
+        tk3d_mlp_outer o{};
+        o.B = (int32_t)B;
+        o.P = (int32_t)P;
+        o.group = p.group;
+        o.M = p.M;
+        o.col = source(k.y[l - 1], nullptr, 0, 0);
+        o.col_norm = o.row_norm = inner;
+        o.row.K = (int32_t)O;
+        o.row.sel = sel.data_ptr();
+        const int sparse_splits = tk3d_mlp_outer_splits(&o);
+        const Tensor sparse = at::empty({sparse_splits, O, I}, like.options());
+        o.partial = f32(sparse);
+        done(tk3d_mlp_outer_f32(TK3D_MLP_ROW_POOL, TK3D_MLP_COL_ACT, &o, stream), "tk3d_mlp_outer_f32");
+        o.row = o.col;
+        const int splits = tk3d_mlp_outer_splits(&o);
+        const Tensor xx = at::empty({splits, I, I}, like.options());
+        const Tensor xsum = at::empty({splits, I}, like.options());
+        o.partial = f32(xx);
+        o.rowsum = f32(xsum);
+        done(tk3d_mlp_outer_f32(TK3D_MLP_ROW_ACT, TK3D_MLP_COL_ACT, &o, stream), "tk3d_mlp_outer_f32");
+        const Tensor scratch = at::empty({I + 1, I}, like.options());
+        done(tk3d_mlp_pool_weight_grad_f32(f32(sparse), sparse_splits, f32(xx), f32(xsum), splits, w,
+                                           f32(coef[l]), (int)O, (int)I, f32(scratch),
+                                           f32(out.params[3 * l]), stream),
+             "tk3d_mlp_pool_weight_grad_f32");
+        coefficients(l - 1, sums.first.data_ptr(), sums.second);
+        masked = true;
+        --l;
+    } else {
+        const tk3d_mlp_norm norm = norm_of(c, k, l);
+        const int C = (int)c.out_channels(l);
+        const int slots = tk3d_mlp_mask_slots((int)B, C, (int)P);
+        const Tensor partial = partial_sums(like, C, slots);
+        done(tk3d_mlp_mask_sums_f32(f32(g), f32(k.y[l]), (int)B, C, (int)P, &norm,
+                                    partial.data_ptr(), stream),
+             "tk3d_mlp_mask_sums_f32");
+        coefficients(l, partial.data_ptr(), slots);
+    }
+
+    for (; l >= 0; --l) {
+        const int64_t O = c.out_channels(l), I = c.in_channels(l);
+        const float *w = f32(c.weight(l));
+        float *dw = f32(out.params[3 * l]);
+        tk3d_mlp_outer o{};
+        o.B = (int32_t)B;
+        o.P = (int32_t)P;
+        o.row = source(e, nullptr, 0, 0);
+        o.row.y = f32(k.y[l]);
+        o.row.coef = f32(coef[l]);
+        o.row_norm = norm_of(c, k, l);
+        const int row = masked ? TK3D_MLP_ROW_GRAD : TK3D_MLP_ROW_GRAD_OUT;
+        const int in = masked ? TK3D_MLP_IN_GRAD : TK3D_MLP_IN_GRAD_OUT;
+        const auto gradient_product = [&](int64_t channels) {
+            tk3d_mlp_product p = product(B, channels, P);
+            p.src[0] = source(e, w, I, 1);
+            p.src[0].y = f32(k.y[l]);
+            p.src[0].coef = f32(coef[l]);
+            p.in_norm = norm_of(c, k, l);
+            return p;
+        };
+        if (l > 0) {
+            o.col = source(k.y[l - 1], nullptr, 0, 0);
+            o.col_norm = norm_of(c, k, l - 1);
+            outer(row, TK3D_MLP_COL_ACT, o, like, dw, I, pending, stream);
+            tk3d_mlp_product p = gradient_product(I);
+            p.out_norm = o.col_norm;
+            p.yprev = f32(k.y[l - 1]);
+            const Tensor before = at::empty({B, I, P}, like.options());
+            p.out = f32(before);
+            const auto sums = summed_product(in, TK3D_MLP_OUT_MASK, p, like, stream);
+            coefficients(l - 1, sums.first.data_ptr(), sums.second);
+            e = before;
+            masked = true;
+            continue;
+        }
+        if (!c.grouped()) {
+            const int64_t C1 = c.x.size(1);
+            o.col = source(c.x, nullptr, 0, 0);
+            outer(row, TK3D_MLP_COL_RAW, o, like, dw, I, pending, stream);
+            if (c.x2.defined()) {
+                o.col = source(c.x2, nullptr, 0, 0);
+                outer(row, TK3D_MLP_COL_RAW, o, like, dw + C1, I, pending, stream);
+            }
+            if (want_x || want_x2) {
+                tk3d_mlp_product p = gradient_product(I);
+                p.C0 = (int32_t)C1;
+                if (want_x)
+                    out.x = at::empty(c.x.sizes(), like.options());
+                if (want_x2)
+                    out.x2 = at::empty(c.x2.sizes(), like.options());
+                p.out = f32(out.x);
+                p.out2 = f32(out.x2);
+                run_product(in, TK3D_MLP_OUT_PLAIN, p, stream);
+            }
+            continue;
+        }
+        const int64_t M = c.index.size(1), S = c.index.size(2), N = c.xyz.size(2), F = I - 3;
+        const int64_t *index = c.index.data_ptr<int64_t>();
+        if (!want_x && F <= 29) {
+            // The grouped input itself, in one tile of columns: it is small, and nothing else of
+            // this layer's gradient is needed.
+            const Tensor grouped = at::empty({B, I, P}, like.options());
+            done(tk3d_group_points_concat_forward_f32(f32(c.x), f32(c.xyz), f32(c.centre), index, B,
+                                                      F, N, M, S, f32(grouped), stream),
+                 "tk3d_group_points_concat_forward_f32");
+            o.col = source(grouped, nullptr, 0, 0);
+            outer(row, TK3D_MLP_COL_RAW, o, like, dw, I, pending, stream);
+            continue;
+        }
+        // dy, summed per point; the rest is per point.
+        const Tensor rel = at::empty({B, 3, P}, like.options());
+        done(tk3d_group_points_concat_forward_f32(nullptr, f32(c.xyz), f32(c.centre), index, B, 0, N,
+                                                  M, S, f32(rel), stream),
+             "tk3d_group_points_concat_forward_f32");
+        done(tk3d_mlp_grad_apply_f32(f32(e), f32(k.y[0]), f32(coef[0]), (int)B, (int)O, (int)P,
+                                     stream),
+             "tk3d_mlp_grad_apply_f32");
+        o.col = source(rel, nullptr, 0, 0);
+        outer(TK3D_MLP_ROW_RAW, TK3D_MLP_COL_RAW, o, like, dw + F, I, pending, stream);
+        const Tensor du = at::empty({B, O, N}, like.options());
+        done(tk3d_group_points_backward_f32(f32(e), index, B, O, N, M, S, f32(du), stream),
+             "tk3d_group_points_backward_f32");
+        tk3d_mlp_outer q{};
+        q.B = (int32_t)B;
+        q.P = (int32_t)N;
+        q.row = source(du, nullptr, 0, 0);
+        q.col = source(c.x, nullptr, 0, 0);
+        outer(TK3D_MLP_ROW_RAW, TK3D_MLP_COL_RAW, q, like, dw, I, pending, stream);
+        if (want_x) {
+            out.x = at::empty(c.x.sizes(), like.options());
+            tk3d_mlp_product p = product(B, F, N);
+            p.src[0] = source(du, w, I, 1);
+            p.out = f32(out.x);
+            run_product(TK3D_MLP_IN_RAW, TK3D_MLP_OUT_PLAIN, p, stream);
+        }
+    }
+    done(tk3d_mlp_sum_f32(pending.sums.data(), (int)pending.sums.size(), stream), "tk3d_mlp_sum_f32");
+    return out;
+}
+
+// The same chain in stock operators: for gradients of gradients.
+Tensor in_stock_operators(const Call &c)
+{
+    Tensor h;
+    if (c.grouped()) {
+        const int64_t B = c.batch(), M = c.index.size(1), S = c.index.size(2);
+        const Tensor valid = (c.index.ge(0) & c.index.lt(c.xyz.size(2))).view({B, 1, M * S});
+        const Tensor flat = c.index.view({B, 1, M * S}).clamp(0, c.xyz.size(2) - 1);
+        const auto gather = [&](const Tensor &t) {
+            return at::where(valid, at::gather(t, 2, flat.expand({B, t.size(1), M * S})),
+                             at::zeros({}, t.options()));
+        };
+        h = gather(c.xyz) - c.centre.unsqueeze(3).expand({B, 3, M, S}).reshape({B, 3, M * S});
+        if (c.x.defined())
+            h = at::cat({gather(c.x), h}, 1);
+    } else {
+        h = c.x2.defined() ? at::cat({c.x, c.x2}, 1) : c.x;
+    }
+    for (int64_t l = 0; l < c.layers(); ++l) {
+        h = at::conv1d(h, c.weight(l).view({c.out_channels(l), c.in_channels(l), 1}));
+        const Tensor none;
+        h = at::batch_norm(h, c.params[3 * l + 1], c.params[3 * l + 2],
+                           c.training ? none : c.buffers[3 * l],
+                           c.training ? none : c.buffers[3 * l + 1], c.training, 0.0, c.eps[l], false);
+        h = at::relu(h);
+    }
+    if (c.pool)
+        h = std::get<0>(at::max(h.view({h.size(0), h.size(1), h.size(2) / c.pool, c.pool}), 3));
+    return h;
+}
+
+struct Node : torch::autograd::Function<Node> {
+    // Saved: x, x2, xyz, centre, index, arg, then of every layer weight, gamma, beta, y, mean, var.
+    static Tensor forward(AutogradContext *ctx, const std::optional<Tensor> &x,
+                          const std::optional<Tensor> &x2, at::TensorList params, const Call &call)
+    {
+        Kept k;
+        const Tensor z = tk3d::forward(call, k);
+        variable_list saved = {call.x, call.x2, call.xyz, call.centre, call.index, k.arg};
+        for (int64_t l = 0; l < call.layers(); ++l) {
+            for (int64_t i = 0; i < 3; ++i)
+                saved.push_back(call.params[3 * l + i]);
+            saved.push_back(k.y[l]);
+            saved.push_back(k.mean[l]);
+            saved.push_back(k.var[l]);
+        }
+        ctx->save_for_backward(std::move(saved));
+        ctx->saved_data["pool"] = call.pool;
+        ctx->saved_data["training"] = call.training;
+        ctx->saved_data["eps"] = call.eps;
+        ctx->saved_data["x"] = x.has_value();
+        ctx->saved_data["x2"] = x2.has_value();
+        ctx->saved_data["want_x"] = call.x.defined() && call.x.requires_grad();
+        ctx->saved_data["want_x2"] = call.x2.defined() && call.x2.requires_grad();
+        return z;
+    }
+
+    static variable_list backward(AutogradContext *ctx, variable_list grads)
+    {
+        const variable_list s = ctx->get_saved_variables();
+        Call c;
+        Kept k;
+        c.x = s[0];
+        c.x2 = s[1];
+        c.xyz = s[2];
+        c.centre = s[3];
+        c.index = s[4];
+        k.arg = s[5];
+        c.pool = ctx->saved_data["pool"].toInt();
+        c.training = ctx->saved_data["training"].toBool();
+        c.eps = ctx->saved_data["eps"].toDoubleVector();
+        const int64_t L = ((int64_t)s.size() - 6) / 6;
+        for (int64_t l = 0; l < L; ++l) {
+            const Tensor *t = &s[6 + 6 * l];
+            for (int i = 0; i < 3; ++i)
+                c.params.push_back(t[i]);
+            k.y.push_back(t[3]);
+            k.mean.push_back(t[4]);
+            k.var.push_back(t[5]);
+            c.buffers.push_back(t[4]);
+            c.buffers.push_back(t[5]);
+            c.buffers.push_back(Tensor());
+        }
+        const bool want_x = ctx->saved_data["want_x"].toBool();
+        const bool want_x2 = ctx->saved_data["want_x2"].toBool();
+        // One gradient per tensor that apply() was given.
+        variable_list result;
+        const bool has_x = ctx->saved_data["x"].toBool(), has_x2 = ctx->saved_data["x2"].toBool();
+        if (c10::GradMode::is_enabled()) {  // a gradient of this gradient will be asked for
+            const Tensor z = in_stock_operators(c);
+            variable_list inputs;
+            if (want_x)
+                inputs.push_back(c.x);
+            if (want_x2)
+                inputs.push_back(c.x2);
+            for (const Tensor &t : c.params)
+                if (t.requires_grad())
+                    inputs.push_back(t);
+            const variable_list d =
+                torch::autograd::grad({z}, inputs, {grads[0]}, std::nullopt, true, true);
+            size_t i = 0;
+            result.push_back(want_x ? d[i++] : Tensor());
+            result.push_back(want_x2 ? d[i++] : Tensor());
+            for (const Tensor &t : c.params)
+                result.push_back(t.requires_grad() ? d[i++] : Tensor());
+        } else {
+            OnDeviceOf guard(c.like().device());
+            const Grads d = tk3d::backward(c, k, grads[0].contiguous(), want_x, want_x2);
+            result.push_back(d.x);
+            result.push_back(d.x2);
+            for (int64_t l = 0; l < L; ++l)
+                for (int i = 0; i < 3; ++i)
+                    result.push_back(d.params[3 * l + i]);
+        }
+        result.push_back(Tensor());  // (the call itself)
+        (void)has_x;
+        (void)has_x2;
+        return result;
+    }
+};
+
+bool usable(const Tensor &t) { return t.is_cuda() && t.scalar_type() == at::kFloat; }
+
+}  // namespace
+
+// x [B,C,P] (or [B,C,M,S]); a chain applied to it. Declines (undefined result) what the kernels
+// do not take: the caller then runs the stock modules.
+Tensor mlp(Tensor x, Tensor x2, const Tensor &xyz, const Tensor &centre, const Tensor &index,
+           std::vector<Tensor> params, std::vector<Tensor> buffers, std::vector<double> eps,
+           std::vector<double> momentum, bool training, int64_t pool)
+{
+    Call c;
+    const int64_t L = (int64_t)params.size() / 3;
+    // (Pooled forms: groups of 32 or 64, which fill whole tiles of every shape; other groups take
+    // the dense chain and a maximum behind it.)
+    if (L == 0 || (pool && (L < 2 || (pool != 32 && pool != 64))))
+        return Tensor();
+    const bool grouped = xyz.defined();
+    std::vector<int64_t> shape;
+    if (grouped) {
+        if (L < 2 || !pool || !usable(xyz) || !usable(centre) || !index.is_cuda() || xyz.dim() != 3 ||
+            centre.dim() != 3 || index.dim() != 3 || index.scalar_type() != at::kLong ||
+            index.size(2) != pool || centre.size(2) != index.size(1) || xyz.size(1) != 3 ||
+            centre.size(1) != 3 || index.size(0) != xyz.size(0) || centre.size(0) != xyz.size(0))
+            return Tensor();
+        c.xyz = xyz.contiguous();
+        c.centre = centre.contiguous();
+        c.index = index.contiguous();
+        if (x.defined() && (x.dim() != 3 || x.size(2) != xyz.size(2) || x.size(0) != xyz.size(0)))
+            return Tensor();
+    } else {
+        if (!x.defined() || x.dim() < 3 || x.dim() > 4 || (pool && x.size(-1) != pool))
+            return Tensor();
+        if (x2.defined() && (x.dim() != 3 || x2.dim() != 3 || x2.size(0) != x.size(0) ||
+                             x2.size(2) != x.size(2)))
+            return Tensor();
+        shape = x.sizes().vec();
+    }
+    const bool has_x = x.defined(), has_x2 = x2.defined();
+    if ((has_x && !usable(x)) || (has_x2 && !usable(x2)))
+        return Tensor();
+    int64_t channels = (has_x ? x.size(1) : 0) + (has_x2 ? x2.size(1) : 0) + (grouped ? 3 : 0);
+    bool tracked = (has_x && x.requires_grad()) || (has_x2 && x2.requires_grad());
+    for (int64_t l = 0; l < L; ++l) {
+        for (int i = 0; i < 3; ++i) {
+            if (!usable(params[3 * l + i]) || !params[3 * l + i].is_contiguous())
+                return Tensor();
+            tracked = tracked || params[3 * l + i].requires_grad();
+        }
+        if (!usable(buffers[3 * l]) || !usable(buffers[3 * l + 1]) ||
+            !buffers[3 * l].is_contiguous() || !buffers[3 * l + 1].is_contiguous())
+            return Tensor();
+        if (params[3 * l].size(1) != channels)
+            return Tensor();
+        channels = params[3 * l].size(0);
+    }
+    if (has_x)
+        c.x = x.dim() == 4 ? x.flatten(2).contiguous() : x.contiguous();
+    if (has_x2)
+        c.x2 = x2.contiguous();
+    c.pool = pool;
+    c.training = training;
+    c.params = std::move(params);
+    c.buffers = std::move(buffers);
+    c.eps = std::move(eps);
+    c.momentum = std::move(momentum);
+    const int64_t B = c.batch(), P = c.positions();
+    int64_t widest = has_x ? c.x.size(1) : 0;
+    if (has_x2)
+        widest = std::max(widest, c.x2.size(1));
+    for (int64_t l = 0; l < L; ++l)
+        widest = std::max(widest, c.out_channels(l));
+    const int64_t longest = grouped ? std::max(P, c.xyz.size(2)) : P;
+    // (one value per channel has no variance: stock batch norm raises the error)
+    if (B == 0 || P == 0 || longest == 0 || B * P < 2 || widest > 4096 ||
+        (widest + 8) * longest > (1 << 29) || B * longest > (1 << 30))
+        return Tensor();
+    OnDeviceOf guard(c.like().device());
+    Tensor z;
+    if (c10::GradMode::is_enabled() && tracked) {
+        const auto given = [](const Tensor &t) {
+            return t.defined() ? std::optional<Tensor>(t) : std::nullopt;
+        };
+        z = Node::apply(given(c.x), given(c.x2), at::TensorList(c.params), c);
+    } else if (training) {
+        Kept k;
+        z = forward(c, k);
+    } else {
+        z = evaluate(c);
+    }
+    if (!grouped && x.dim() == 4 && !pool)
+        z = z.view({shape[0], z.size(1), shape[2], shape[3]});
+    return z;
+}
+
+}  // namespace tk3d

@@ -2,8 +2,10 @@
 (torkit3d/layers/pointnet2.py), built on the fused ops of this package.
 
 Differences from the reference, none of which change the result:
-  * ``SetAbstraction`` groups features and centred coordinates into one tensor with
-    one op instead of two gathers, a subtraction and ``torch.cat``;
+  * ``SetAbstraction`` hands the ungrouped features, the coordinates and the neighbour index
+    to its MLP, whose first layer gathers (elsewhere features and centred coordinates are
+    grouped into one tensor with one op instead of two gathers, a subtraction and
+    ``torch.cat``), and the maximum over the neighbours is taken by the last layer;
   * ``BallQuery`` and ``FeatureInterpolator`` hand their [B, 3, N] clouds to kernels
     that read that layout, instead of copying them to [B, N, 3];
   * ``FeatureInterpolator`` gets index and weight from one kernel. The reference
@@ -38,15 +40,16 @@ class SetAbstraction(nn.Module):
         with torch.no_grad():
             nbr_index = self.query_neighbor(out_xyz, in_xyz)  # [B, N2, K]
         if self.use_xyz:
+            out_feature = self.mlp.forward_grouped_max(in_feature, in_xyz, out_xyz, nbr_index)
+            if out_feature is not None:
+                return out_feature
             nbr_feature = group_points_with_xyz(in_feature, in_xyz, out_xyz, nbr_index)
         elif in_feature is not None:
             nbr_feature = group_points(in_feature, nbr_index)
         else:
             nbr_feature = in_xyz.new_empty(
                 [in_xyz.size(0), 0, nbr_index.size(1), nbr_index.size(2)])
-        out_feature = self.mlp(nbr_feature)
-        out_feature, _ = torch.max(out_feature, dim=3)
-        return out_feature
+        return self.mlp.forward_max(nbr_feature)
 
     def extra_repr(self):
         return "use_xyz={}".format(self.use_xyz)
@@ -105,5 +108,5 @@ class FeaturePropagation(nn.Module):
     def forward(self, in_xyz, in_feature, out_xyz, out_feature=None):
         interp_feature = self.interpolator(out_xyz, in_xyz, in_feature)
         if out_feature is not None:
-            interp_feature = torch.cat([interp_feature, out_feature], dim=1)
+            return self.mlp.forward_cat(interp_feature, out_feature)
         return self.mlp(interp_feature)

@@ -1,13 +1,17 @@
 """The ``torkit3d.nn`` helpers the layers and models are built from: shared MLPs as
 1x1 convolutions or linear layers with batch norm and ReLU
 (torkit3d/nn/modules/conv.py, torkit3d/nn/modules/linear.py, torkit3d/nn/modules/mlp.py)
-and ``batch_index_select`` (torkit3d/nn/functional.py:34-69). Stock torch modules;
-sub-module names match the reference so that its checkpoints load.
+and ``batch_index_select`` (torkit3d/nn/functional.py:34-69). Modules and sub-module names
+are the reference's, so that its checkpoints load; the shared MLPs run on fused kernels where
+these take them (``SharedMLP``).
 """
 import torch
 from torch import nn
+from torch.nn.modules.module import _has_any_global_hook
 
-__all__ = ["Conv1dBNReLU", "Conv2dBNReLU", "LinearBNReLU", "mlp_bn_relu", "mlp1d_bn_relu",
+from .. import _native
+
+__all__ = ["Conv1dBNReLU", "Conv2dBNReLU", "LinearBNReLU", "SharedMLP", "mlp_bn_relu", "mlp1d_bn_relu",
            "mlp2d_bn_relu", "batch_index_select"]
 
 
@@ -36,11 +40,13 @@ class _ConvBNReLU(nn.Module):
 class Conv1dBNReLU(_ConvBNReLU):
     conv_type = nn.Conv1d
     bn_type = nn.BatchNorm1d
+    ones, no_padding = (1,), (0,)
 
 
 class Conv2dBNReLU(_ConvBNReLU):
     conv_type = nn.Conv2d
     bn_type = nn.BatchNorm2d
+    ones, no_padding = (1, 1), (0, 0)
 
 
 class LinearBNReLU(nn.Module):
@@ -64,12 +70,81 @@ class LinearBNReLU(nn.Module):
         return x
 
 
+class SharedMLP(nn.Sequential):
+    """The layers of ``mlp1d_bn_relu`` / ``mlp2d_bn_relu`` (an ``nn.Sequential`` to its
+    checkpoints and to anything that walks its modules), run as one chain of fused kernels
+    (csrc/mlp.hip) on float32 GPU tensors: the product of a layer normalises its input as it
+    reads it and sums up the statistics of its output. Whatever is not plain - hooks, other
+    modules in place of the blocks', frozen layers among training ones, autocast - runs layer
+    by layer in stock torch."""
+
+    def forward(self, x):
+        out = self._chain(x)
+        return super().forward(x) if out is None else out
+
+    def forward_cat(self, x, x2):
+        """``self(torch.cat([x, x2], dim=1))`` without the concatenation."""
+        out = self._chain(x, x2)
+        return self(torch.cat([x, x2], dim=1)) if out is None else out
+
+    def forward_max(self, x):
+        """``self(x).max(dim=3)[0]`` for x [B, C, M, S]."""
+        out = self._chain(x, pool=x.size(-1))
+        return torch.max(self(x), dim=3)[0] if out is None else out
+
+    def forward_grouped_max(self, feature, xyz, centre, index):
+        """``self(group_points_with_xyz(feature, xyz, centre, index)).max(dim=3)[0]``, or None
+        where the fused chain does not take it."""
+        if torch.is_grad_enabled() and (xyz.requires_grad or centre.requires_grad):
+            return None
+        return self._chain(feature, None, xyz, centre, index, pool=index.size(2))
+
+    def _chain(self, x, x2=None, xyz=None, centre=None, index=None, pool=0):
+        like = xyz if x is None else x
+        if (not like.is_cuda or like.dtype != torch.float32 or torch.is_autocast_enabled()
+                or torch.compiler.is_compiling() or torch.jit.is_tracing()
+                or _has_any_global_hook() or type(self) is not SharedMLP
+                or self._forward_hooks or self._forward_pre_hooks
+                or self._backward_hooks or self._backward_pre_hooks):
+            return None
+        params, buffers, eps, momentum = [], [], [], []
+        training = None
+        for block in self._modules.values():
+            if type(block) not in (Conv1dBNReLU, Conv2dBNReLU) or not _plain(block):
+                return None
+            conv, bn, relu = (block._modules.get(name) for name in ("conv", "bn", "relu"))
+            if (type(conv) not in (nn.Conv1d, nn.Conv2d) or not _plain(conv)
+                    or type(bn) not in (nn.BatchNorm1d, nn.BatchNorm2d) or not _plain(bn)
+                    or type(relu) is not nn.ReLU or not _plain(relu)
+                    or conv.groups != 1 or conv.padding != block.no_padding
+                    or conv.kernel_size != block.ones or conv.stride != block.ones
+                    or conv._parameters["bias"] is not None or bn.momentum is None):
+                return None
+            if training is None:
+                training = bn.training
+            weight, gamma, beta = conv._parameters["weight"], *bn._parameters.values()
+            mean, var, count = bn._buffers.values()
+            if training != bn.training or gamma is None or beta is None or mean is None:
+                return None
+            params += (weight, gamma, beta)
+            buffers += (mean, var, count)
+            eps.append(bn.eps)
+            momentum.append(bn.momentum)
+        return _native.mlp(x, x2, xyz, centre, index, params, buffers, eps, momentum,
+                           bool(training), pool)
+
+
+def _plain(module):
+    return not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks
+                or module._backward_pre_hooks)
+
+
 def _mlp(block, in_channels, out_channels_list):
     layers = []
     for out_channels in out_channels_list:
         layers.append(block(in_channels, out_channels, 1, relu=True))
         in_channels = out_channels
-    return nn.Sequential(*layers)
+    return SharedMLP(*layers)
 
 
 def mlp_bn_relu(in_channels, out_channels_list):
