@@ -83,10 +83,16 @@ __device__ __forceinline__ void load_run(float (&dst)[PT], const float *base, un
 
 constexpr bool reads_y(int in) { return in == IN_GRAD || in == IN_GRAD_OUT; }
 
-template <int IN, int PT> struct Rows {  // eight input channels of a wave's positions
-    float x[4][PT];
-    float y[reads_y(IN) ? 4 : 1][PT];
-    int2 sel[IN == IN_POOL ? 4 : 1];
+// Channel groups that are requested at once: 16 bytes per lane and channel pair of the wide tiles
+// cover a trip to memory with one group, the narrow ones need four (1024 positions, 768 -> 256
+// channels: 68 us with one group of eight channels at a time).
+template <int PT> constexpr int kDepth = PT == 4 ? 1 : PT == 2 ? 2 : 4;
+
+template <int IN, int PT> struct Rows {  // groups of eight input channels of a wave's positions
+    static constexpr int D = kDepth<PT>;
+    float x[D][4][PT];
+    float y[reads_y(IN) ? D : 1][4][PT];
+    int2 sel[IN == IN_POOL ? D : 1][4];
 };
 
 struct GemmArgs {
@@ -130,33 +136,35 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
     // Weights of channel groups [first, first + count): element (ct, g, lane, s) belongs to
     // input channel 8 g + 2 s + (lane >> 5) and output channel 32 ct + (lane & 31).
     const auto stage = [&](int first, int count) {
-        for (int i = tid; i < CT * count * 256; i += kBlock) {
-            // (consecutive threads walk the direction in which the weights lie in memory)
-            int k8, c;
-            const int g = i >> 8;  // (ct, group), 256 elements each
-            const int e = i & 255;
-            const int ct = g / count, grp = first + g - ct * count;
-            const bool second = grp >= a.kg0;
-            const tk3d_mlp_source &s = p.src[second ? 1 : 0];
-            if (s.wk == 1) {
-                k8 = e & 7;
-                c = e >> 3;
-            } else {
-                c = e & 31;
-                k8 = e >> 5;
+        // (a group of a channel tile is 256 weights, one per thread; consecutive threads walk the
+        // direction in which the weights lie in memory; eight requests before the first wait)
+        constexpr int AT_ONCE = 8;
+        for (int j = 0; j < CT * count; j += AT_ONCE) {
+            float v[AT_ONCE];
+            int at[AT_ONCE];
+#pragma unroll
+            for (int i = 0; i < AT_ONCE; ++i) {
+                const int ct = CT > 1 && j + i >= count ? 1 : 0;
+                const int local = j + i - ct * count, grp = first + local;
+                const bool second = grp >= a.kg0;
+                const tk3d_mlp_source &s = p.src[second ? 1 : 0];
+                const int k8 = s.wk == 1 ? tid & 7 : tid >> 5;
+                const int c = s.wk == 1 ? tid >> 3 : tid & 31;
+                const int k = (grp - (second ? a.kg0 : 0)) * 8 + k8, cc = cbase + ct * 32 + c;
+                v[i] = j + i < CT * count && k < s.K && cc < p.C
+                           ? s.w[(int64_t)k * s.wk + (int64_t)cc * s.wc] : 0.0f;
+                at[i] = ((ct * a.chunk + local) * 64 + (k8 & 1) * 32 + c) * 4 + (k8 >> 1);
             }
-            const int k = (grp - (second ? a.kg0 : 0)) * 8 + k8, cc = cbase + ct * 32 + c;
-            const float v = k < s.K && cc < p.C
-                                ? s.w[(int64_t)k * s.wk + (int64_t)cc * s.wc] : 0.0f;
-            weights[((ct * a.chunk + (grp - first)) * 64 + (k8 & 1) * 32 + c) * 4 + (k8 >> 1)] = v;
+#pragma unroll
+            for (int i = 0; i < AT_ONCE; ++i)
+                if (j + i < CT * count)
+                    weights[at[i]] = v[i];
         }
     };
 
-    // Rows of channel group g for the positions of a wave tile.
-    const auto load = [&](Rows<IN, PT> &r, int tile, int g) {
-        const int b = tile / a.tiles;
-        int pos = (tile - b * a.tiles) * (32 * PT) + PT * col;
-        pos = pos > P - PT ? P - PT : pos;  // (results of the surplus are dropped)
+    // Rows of the channel groups of a step for the positions of a wave tile.
+    constexpr int D = kDepth<PT>;
+    const auto load_group = [&](Rows<IN, PT> &r, int d, int b, int pos, int g) {
         const bool second = (IN == IN_RAW2 || IN == IN_POOL) && g >= a.kg0;
         const tk3d_mlp_source &s = p.src[second ? 1 : 0];
         const int k0 = (g - (second ? a.kg0 : 0)) * 8 + half;
@@ -166,7 +174,7 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const int k = k0 + 2 * q < s.K ? k0 + 2 * q : s.K - 1;
-                r.sel[IN == IN_POOL ? q : 0] = sel[(unsigned)k * (unsigned)p.M + (unsigned)m];
+                r.sel[IN == IN_POOL ? d : 0][q] = sel[(unsigned)k * (unsigned)p.M + (unsigned)m];
             }
             return;
         }
@@ -175,10 +183,19 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
         for (int q = 0; q < 4; ++q) {
             const int k = k0 + 2 * q < s.K ? k0 + 2 * q : s.K - 1;
             const unsigned offset = ((unsigned)k * (unsigned)P + (unsigned)pos) * 4u;
-            load_run<PT>(r.x[q], x, offset);
+            load_run<PT>(r.x[d][q], x, offset);
             if constexpr (reads_y(IN))
-                load_run<PT>(r.y[q], s.y + (int64_t)b * s.batch_stride, offset);
+                load_run<PT>(r.y[d][q], s.y + (int64_t)b * s.batch_stride, offset);
         }
+    };
+    const auto load = [&](Rows<IN, PT> &r, int tile, int step) {
+        const int b = tile / a.tiles;
+        int pos = (tile - b * a.tiles) * (32 * PT) + PT * col;
+        pos = pos > P - PT ? P - PT : pos;  // (results of the surplus are dropped)
+#pragma unroll
+        for (int d = 0; d < D; ++d)
+            if (D == 1 || step * D + d < a.kg)
+                load_group(r, d, b, pos, step * D + d);
     };
 
     tk_f32x16 acc[PT][CT];
@@ -192,7 +209,7 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
                     acc[t][ct][r] = 0.0f;
     };
 
-    const auto multiply = [&](const Rows<IN, PT> &r, int tile, int g, int first) {
+    const auto multiply_group = [&](const Rows<IN, PT> &r, int d, int tile, int g, int first) {
         const bool second = (IN == IN_RAW2 || IN == IN_POOL) && g >= a.kg0;
         const int K = p.src[second ? 1 : 0].K, gs = g - (second ? a.kg0 : 0);
         const int k0 = gs * 8 + half;
@@ -204,7 +221,7 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
             const int kk = pos - pos / p.group * p.group;
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                const int2 sel = r.sel[IN == IN_POOL ? q : 0];
+                const int2 sel = r.sel[IN == IN_POOL ? d : 0][q];
 #pragma unroll
                 for (int t = 0; t < PT; ++t)
                     v[q][t] = sel.y == kk + t ? __int_as_float(sel.x) : 0.0f;
@@ -219,8 +236,8 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
                         ss = act_coef[k0 + 2 * q];
 #pragma unroll
                     for (int t = 0; t < PT; ++t) {
-                        float e = r.x[q][t];
-                        const float y = r.y[reads_y(IN) ? q : 0][t];
+                        float e = r.x[d][q][t];
+                        const float y = r.y[reads_y(IN) ? d : 0][q][t];
                         if constexpr (IN == IN_GRAD_OUT)
                             e = passes(__builtin_fmaf(y, ss.x, ss.y)) ? e : 0.0f;
                         v[q][t] = __builtin_fmaf(c.x, e, __builtin_fmaf(c.y, y, c.z));
@@ -229,11 +246,11 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
                     const f32x2 c = act_coef[k0 + 2 * q];
 #pragma unroll
                     for (int t = 0; t < PT; ++t)
-                        v[q][t] = relu(__builtin_fmaf(r.x[q][t], c.x, c.y));
+                        v[q][t] = relu(__builtin_fmaf(r.x[d][q][t], c.x, c.y));
                 } else {
 #pragma unroll
                     for (int t = 0; t < PT; ++t)
-                        v[q][t] = r.x[q][t];
+                        v[q][t] = r.x[d][q][t];
                 }
             }
         }
@@ -257,6 +274,12 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
                 for (int t = 0; t < PT; ++t)
                     acc[t][ct] = __builtin_amdgcn_mfma_f32_32x32x2f32(v[q][t], w[ct][q], acc[t][ct],
                                                                       0, 0, 0);
+    };
+    const auto multiply = [&](const Rows<IN, PT> &r, int tile, int step, int first) {
+#pragma unroll
+        for (int d = 0; d < D; ++d)
+            if (D == 1 || step * D + d < a.kg)
+                multiply_group(r, d, tile, step * D + d, first);
     };
 
     // Per-lane constants and sums of the output channels (lane = channel).
@@ -470,18 +493,19 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
         __syncthreads();
         if (mine0 < a.total) {
             Rows<IN, PT> now, next;
+            const int steps = (a.kg + D - 1) / D;
             load(now, mine0, 0);
             for (int tile = mine0; tile < a.total; tile += stride) {
                 clear();
-                int g = 0;
-                for (; g + 1 < a.kg; ++g) {
-                    load(next, tile, g + 1);
-                    multiply(now, tile, g, 0);
+                int step = 0;
+                for (; step + 1 < steps; ++step) {
+                    load(next, tile, step + 1);
+                    multiply(now, tile, step, 0);
                     now = next;
                 }
                 if (tile + stride < a.total)
                     load(next, tile + stride, 0);
-                multiply(now, tile, g, 0);
+                multiply(now, tile, step, 0);
                 now = next;
                 finish(tile);
             }
@@ -495,15 +519,15 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
                 const int n = a.kg - first < a.chunk ? a.kg - first : a.chunk;
                 Rows<IN, PT> now, next;
                 if (active)
-                    load(now, tile, first);
+                    load(now, tile, first / D);
                 __syncthreads();
                 stage(first, n);
                 __syncthreads();
                 if (active) {
-                    for (int g = first; g < first + n; ++g) {
-                        if (g + 1 < first + n)
-                            load(next, tile, g + 1);
-                        multiply(now, tile, g, first);
+                    for (int step = first / D; step * D < first + n; ++step) {
+                        if ((step + 1) * D < first + n)
+                            load(next, tile, step + 1);
+                        multiply(now, tile, step, first);
                         now = next;
                     }
                 }
@@ -740,16 +764,31 @@ struct SumArgs {
     tk3d_mlp_sum s[kMaxSums];
 };
 
+// Sixteen outputs to a workgroup, sixteen threads to an output: the partial sums are up to 512 of
+// few values (one thread per output took 123 us on 512 sums of 32 x 32).
 __global__ void __launch_bounds__(kBlock) mlp_sum_kernel(SumArgs a)
 {
     const tk3d_mlp_sum &s = a.s[blockIdx.y];
+    __shared__ double lds[kWaves][16];
     const int n = s.R * s.C;
-    for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
+    const int at = threadIdx.x & 15, lane = threadIdx.x >> 4;
+    for (int first = blockIdx.x * 16; first < n; first += gridDim.x * 16) {
+        const int i = first + at < n ? first + at : n - 1;
         double sum = 0.0;
-        for (int k = 0; k < s.splits; ++k)
+#pragma unroll 4
+        for (int k = lane; k < s.splits; k += 16)
             sum += (double)s.partial[(int64_t)k * n + i];
-        const int r = i / s.C;
-        s.out[(int64_t)r * s.ld + (i - r * s.C)] = (float)sum;
+        sum += __shfl_xor(sum, 16);
+        sum += __shfl_xor(sum, 32);
+        if ((threadIdx.x & 63) < 16)
+            lds[threadIdx.x >> 6][at] = sum;
+        __syncthreads();
+        if (threadIdx.x < 16 && first + at < n) {
+            sum = lds[0][at] + lds[1][at] + lds[2][at] + lds[3][at];
+            const int r = i / s.C;
+            s.out[(int64_t)r * s.ld + (i - r * s.C)] = (float)sum;
+        }
+        __syncthreads();
     }
 }
 
@@ -1012,13 +1051,14 @@ __global__ void __launch_bounds__(kT *kT)
 //
 // The layer is linear, so its product with the features is taken once per point (u, stored with a
 // point's channels side by side) and not once per neighbour; what a neighbour adds is its centred
-// coordinates. A lane is a grouped position: it gathers 128 bytes of its point's row and writes
-// 32 channels, each a run over the wave.
+// coordinates. A lane is a grouped position: it gathers 64 bytes of its point's row and writes
+// 16 channels, each a run over the wave. (With 32 channels a lane two waves fit on a SIMD, and the
+// chain index -> point -> row is latency: 54 us on 8 x 65536 positions of 32 channels.)
 
-constexpr int kGroupChannels = 32;
+constexpr int kGroupChannels = 16;
 
 template <bool FEATURES>
-__global__ void __launch_bounds__(kBlock, 2)
+__global__ void __launch_bounds__(kBlock, 4)
     mlp_group_kernel(const float *__restrict__ u, const float *__restrict__ xyz,
                      const float *__restrict__ centre, const int64_t *__restrict__ index,
                      const float *__restrict__ wx, int ldw, int C, int N, int M, int S, int tiles,
@@ -1346,8 +1386,8 @@ int tk3d_mlp_sum_f32(const tk3d_mlp_sum *sums, int n, void *stream)
             const int size = a.s[j].R * a.s[j].C;
             most = size > most ? size : most;
         }
-        int blocks = (most + kBlock - 1) / kBlock;
-        blocks = blocks < 1 ? 1 : blocks > 1024 ? 1024 : blocks;
+        int blocks = (most + 15) / 16;
+        blocks = blocks < 1 ? 1 : blocks > 2048 ? 2048 : blocks;
         mlp_sum_kernel<<<dim3(blocks, m), kBlock, 0, (hipStream_t)stream>>>(a);
     }
     return tk_launch_status();
@@ -1446,7 +1486,7 @@ int tk3d_mlp_group_slots(int B, int C, int M, int S)
 {
     const int chunks = (C + kGroupChannels - 1) / kGroupChannels;
     const int64_t total = (int64_t)B * (((int64_t)M * S + kBlock - 1) / kBlock);
-    int64_t most = (4 * tk_cu_count() + chunks - 1) / chunks;
+    int64_t most = (8 * tk_cu_count() + chunks - 1) / chunks;
     most = (most + 7) & ~7;
     return (int)(total < most ? total : most);
 }

@@ -50,6 +50,6 @@ def descend(levels, num_samples, points, feature):
     sampled = farthest_points_xyz(points, num_samples[0])
     xyz, features = [points], [feature]
     for level, count in zip(levels, num_samples):
-        xyz.append(sampled[..., :count])
+        xyz.append(sampled[..., :count].contiguous())
         features.append(level(xyz[-2], xyz[-1], features[-1]))
     return xyz, features
