@@ -102,10 +102,12 @@ typedef struct {
 int tk3d_mlp_outer_splits(const tk3d_mlp_outer *p);
 int tk3d_mlp_outer_f32(int row, int col, const tk3d_mlp_outer *p, void *stream);
 
-/* out[r * ld + c] = sum of the partial sums [splits][R][C]; n of them in one launch. */
+/* out[r * ld + c] = sum over the splits of partial[r][c] - minus[r][c] (minus NULL or like
+ * partial), rows of C, `stride` elements from one split to the next; n of them in one launch. */
 typedef struct {
-    const float *partial;
+    const float *partial, *minus;
     float *out;
+    int64_t stride;
     int32_t splits, R, C, ld;
 } tk3d_mlp_sum;
 int tk3d_mlp_sum_f32(const tk3d_mlp_sum *sums, int n, void *stream);
@@ -158,6 +160,26 @@ int tk3d_mlp_group_slots(int B, int C, int M, int S);
 int tk3d_mlp_group_f32(const float *u, const float *xyz, const float *centre, const int64_t *index,
                        const float *wx, int ldw, int B, int C, int N, int M, int S, float *y,
                        float *rel, void *partial, void *stream);
+
+/* EdgeConv (torkit3d/ops/edge_conv.py) with one layer, on a graph of a cloud with itself, pooled
+ * over the K neighbours: y(i, k) = W1 (x_j - x_i) + W2 x_i = u_j + v_i, j = index[b, i, k] (x_j = 0
+ * for an index outside [0,N)), where w = [W1 W2], u = W1 x and v = (W2 - W1) x; uv [B, N, 2 O] is
+ * the product of x with the [2 O][C] matrix that tk3d_mlp_edge_weights_f32 makes of w. Forward:
+ * extreme and arg [B, O, N] as in pooled layers (arg may be NULL), sum [B, N, O] of the u of a
+ * point's neighbours (or NULL), partial sums. Backward: lists is the inverse of the graph
+ * (int32 [B][N + 1 + N K]), sel a buffer of B N O 8-byte elements, duv [B, 2 O, N] the gradients
+ * of u and v. tk3d_mlp_edge_supported: the sizes these take (N <= 32768, K <= 255). */
+int tk3d_mlp_edge_supported(int64_t B, int64_t N, int64_t K, int64_t O);
+int tk3d_mlp_edge_weights_f32(const float *w, int O, int C, float *out, void *stream);
+int tk3d_mlp_edge_slots(int B, int N);
+int tk3d_mlp_edge_forward_f32(const float *uv, const int64_t *index, const float *gamma, int B, int N,
+                              int K, int O, float *extreme, unsigned char *arg, float *sum,
+                              void *partial, void *stream);
+int tk3d_mlp_edge_lists(const int64_t *index, int B, int N, int K, int32_t *lists, void *stream);
+int tk3d_mlp_edge_backward_f32(const float *g, const float *extreme, const unsigned char *arg,
+                               const float *uv, const float *sum, const int32_t *lists, int B, int N,
+                               int K, int O, const tk3d_mlp_norm *norm, const float *coef, void *sel,
+                               float *duv, void *stream);
 
 #ifdef __cplusplus
 }

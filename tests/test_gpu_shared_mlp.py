@@ -162,3 +162,66 @@ def test_what_is_not_plain_runs_layer_by_layer(cuda):
 
 def stock_forward(mlp, x):
     return nn.Sequential.forward(mlp, x)
+
+
+# EdgeConv on a graph of a cloud with itself: points around the workgroup's 32, channels around
+# its 64, neighbours around the eight rows requested at once; an index outside; lists given or not.
+@pytest.mark.parametrize("training", [True, False])
+@pytest.mark.parametrize("b,c,n,k,o,lists", [
+    (1, 3, 5, 2, 5, False), (2, 3, 33, 7, 64, False), (3, 64, 100, 20, 65, True),
+    (2, 70, 31, 9, 130, True), (8, 64, 2048, 20, 64, True), (1, 6, 5000, 40, 128, False),
+])
+def test_edge_conv(cuda, b, c, n, k, o, lists, training):
+    from torkit3d_amd.ops.edge_conv import EdgeConvBlock, edge_lists, get_edge_feature_builtin
+
+    torch.manual_seed(1)
+    block = EdgeConvBlock(c, [o])
+    block.convs = make(mlp2d_bn_relu, 2 * c, [o], training, cuda)
+    index = torch.randint(0, n, (b, n, k), generator=torch.Generator().manual_seed(n)).to(cuda)
+    x = randn(7, b, c, n)
+    results = []
+    for dtype in (None, torch.float32, torch.float64):
+        leaf = x.clone().to(dtype or torch.float32).requires_grad_()
+        if dtype is None:
+            module = block.convs
+            extra = {"lists": edge_lists(index, n)} if lists else {}
+            out = block(leaf, leaf, index, **extra)
+            assert "EdgeNode" in out.grad_fn.name(), "the fused kernels did not run"
+        else:
+            module = saved if dtype == torch.float32 else saved64
+            out = module(get_edge_feature_builtin(leaf, leaf, index)).max(dim=3)[0]
+        grad = torch.sin(torch.arange(out.numel(), device=cuda, dtype=torch.float64) * 1.7)
+        grads = torch.autograd.grad(out, [leaf, *module.parameters()],
+                                    grad.view_as(out).to(out.dtype))
+        results.append([out.detach(), *grads, *[t.clone() for t in module.buffers()]])
+        if dtype is None:
+            # (statistics as they were before this pass)
+            fresh = make(mlp2d_bn_relu, 2 * c, [o], training, cuda)
+            saved, saved64 = stock(fresh, torch.float32), stock(fresh, torch.float64)
+    for i, (a, s, e) in enumerate(zip(*results)):
+        assert a.shape == e.shape
+        if not e.is_floating_point():
+            assert torch.equal(a, e)
+            continue
+        norm = float(e.norm()) + 1e-30
+        mine, theirs = float((a.double() - e).norm()) / norm, float((s.double() - e).norm()) / norm
+        assert mine <= 4 * theirs + 2e-6, (i, tuple(e.shape), mine, theirs)
+
+
+def test_edge_conv_with_indices_outside(cuda):
+    """A neighbour outside the cloud reads as zeros, as ``group_points`` reads it."""
+    from torkit3d_amd.ops.edge_conv import EdgeConvBlock, get_edge_feature_custom
+
+    block = EdgeConvBlock(4, [8])
+    block.convs = make(mlp2d_bn_relu, 8, [8], True, cuda)
+    index = torch.randint(0, 50, (2, 50, 6), generator=torch.Generator().manual_seed(0)).to(cuda)
+    index[0, :, 2], index[1, 3, :] = -1, 50
+    x, y = randn(8, 2, 4, 50).requires_grad_(), randn(8, 2, 4, 50).requires_grad_()
+    out = block(x, x, index)
+    ref = stock(make(mlp2d_bn_relu, 8, [8], True, cuda), torch.float32)(
+        get_edge_feature_custom(y, y, index)).max(dim=3)[0]
+    torch.testing.assert_close(out, ref, rtol=1e-5, atol=1e-5)
+    weight = randn(9, *out.shape)
+    (out * weight).sum().backward()
+    (ref * weight).sum().backward()
+    torch.testing.assert_close(x.grad, y.grad, rtol=1e-4, atol=1e-4)

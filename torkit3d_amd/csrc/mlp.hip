@@ -8,24 +8,9 @@
 // result on the way out, and a last layer under a maximum writes the maximum only. Narrow layers
 // (up to 64 channels) are bound by HBM, wide ones by the fp32 matrix rate (157 TFLOP/s), which is
 // why the products are fp32 v_mfma_f32_32x32x2 and nothing is rounded to a shorter type.
-#include "tk3d_common.h"
-#include "tk3d_mlp.h"
+#include "mlp_common.h"
 
 namespace {
-
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-// ReLU that keeps NaN, as torch's does.
-__device__ __forceinline__ float relu(float z) { return __builtin_elementwise_maximum(z, 0.0f); }
-// Whether the gradient passes a ReLU whose input was z (torch: where the output is > 0 or NaN).
-__device__ __forceinline__ bool passes(float z) { return !(z <= 0.0f); }
-
-__device__ __forceinline__ f32x2 scale_shift(const tk3d_mlp_norm &n, int c)
-{
-    const float scale = n.gamma[c] * (1.0f / __builtin_sqrtf(n.var[c] + n.eps));
-    return f32x2{scale, __builtin_fmaf(-n.mean[c], scale, n.beta[c])};
-}
 
 // ---- the product ---------------------------------------------------------------------------------
 //
@@ -59,9 +44,6 @@ enum Output {
     OUT_POOL_EVAL,  // store relu(norm(extreme over each group))
     OUT_MASK,       // store out masked by the ReLU in front of it, with the sums of its gradient
 };
-
-constexpr int kBlock = 256;
-constexpr int kWaves = kBlock / TK_WAVE;
 
 template <int PT> struct VecOf;
 template <> struct VecOf<1> { typedef float type; };
@@ -298,8 +280,7 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
         if constexpr (OUT == OUT_EVAL || OUT == OUT_POOL_EVAL || OUT == OUT_MASK)
             out_coef[ct] = scale_shift(p.out_norm, c);
         if constexpr (OUT == OUT_POOL || OUT == OUT_POOL_EVAL) {
-            const float g = p.out_norm.gamma[c];
-            sign[ct] = g > 0.0f ? 1.0f : g < 0.0f ? -1.0f : 0.0f;
+            sign[ct] = sign_of(p.out_norm.gamma[c]);
         }
         if constexpr (OUT == OUT_MASK) {
             shift[ct] = p.out_norm.mean[c];
@@ -777,7 +758,8 @@ __global__ void __launch_bounds__(kBlock) mlp_sum_kernel(SumArgs a)
         double sum = 0.0;
 #pragma unroll 4
         for (int k = lane; k < s.splits; k += 16)
-            sum += (double)s.partial[(int64_t)k * n + i];
+            sum += (double)s.partial[k * s.stride + i] -
+                   (s.minus ? (double)s.minus[k * s.stride + i] : 0.0);
         sum += __shfl_xor(sum, 16);
         sum += __shfl_xor(sum, 32);
         if ((threadIdx.x & 63) < 16)
@@ -1471,9 +1453,10 @@ int tk3d_mlp_pool_weight_grad_f32(const float *sparse, int sparse_splits, const 
                                   const float *coef, int O, int I, float *scratch, float *dw,
                                   void *stream)
 {
-    const tk3d_mlp_sum sums[3] = {{sparse, dw, sparse_splits, O, I, I},
-                                  {xx, scratch, xx_splits, I, I, I},
-                                  {xsum, scratch + (int64_t)I * I, xx_splits, 1, I, I}};
+    const tk3d_mlp_sum sums[3] = {
+        {sparse, nullptr, dw, (int64_t)O * I, sparse_splits, O, I, I},
+        {xx, nullptr, scratch, (int64_t)I * I, xx_splits, I, I, I},
+        {xsum, nullptr, scratch + (int64_t)I * I, I, xx_splits, 1, I, I}};
     const int rc = tk3d_mlp_sum_f32(sums, 3, stream);
     if (rc != TK3D_OK)
         return rc;

@@ -646,4 +646,17 @@ PYBIND11_MODULE(_host, m)
                        std::move(eps), std::move(momentum), training, pool);
         });
     });
+    m.def("edge_lists", [](py::handle index, int64_t n) {
+        const Tensor i = tensor_arg("index", index);
+        return unlocked([&] { return edge_lists(i, n); });
+    });
+    m.def("edge_conv", [](py::handle x, py::handle index, py::handle lists,
+                          std::vector<Tensor> params, std::vector<Tensor> buffers, double eps,
+                          double momentum, bool training) {
+        const Tensor t[] = {tensor_arg("x", x), tensor_arg("index", index),
+                            optional_arg("lists", lists)};
+        return unlocked([&] {
+            return edge_conv(t[0], t[1], t[2], params, buffers, eps, momentum, training);
+        });
+    });
 }

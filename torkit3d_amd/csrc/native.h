@@ -41,4 +41,9 @@ Tensor mlp(Tensor x, Tensor x2, const Tensor &xyz, const Tensor &centre, const T
            std::vector<Tensor> params, std::vector<Tensor> buffers, std::vector<double> eps,
            std::vector<double> momentum, bool training, int64_t pool);
 
+Tensor edge_lists(const Tensor &index, int64_t n);
+Tensor edge_conv(const Tensor &x, const Tensor &index, const Tensor &lists,
+                 const std::vector<Tensor> &params, const std::vector<Tensor> &buffers, double eps,
+                 double momentum, bool training);
+
 }  // namespace tk3d

@@ -261,7 +261,8 @@ void outer(int row, int col, tk3d_mlp_outer &o, const Tensor &like, float *out, 
     const Tensor partial = at::empty({splits, o.row.K, o.col.K}, like.options());
     o.partial = f32(partial);
     done(tk3d_mlp_outer_f32(row, col, &o, stream), "tk3d_mlp_outer_f32");
-    pending.sums.push_back({f32(partial), out, splits, o.row.K, o.col.K, (int32_t)ld});
+    pending.sums.push_back({f32(partial), nullptr, out, (int64_t)o.row.K * o.col.K, splits, o.row.K,
+                            o.col.K, (int32_t)ld});
     pending.alive.push_back(partial);
 }
 
@@ -584,6 +585,197 @@ struct Node : torch::autograd::Function<Node> {
     }
 };
 
+// ---- EdgeConv with one layer ---------------------------------------------------------------------
+
+struct EdgeCall {
+    Tensor x, index;   // [B, C, N], [B, N, K]
+    Tensor lists;      // the inverse of the graph, where the caller has it
+    Tensor weight, gamma, beta, running_mean, running_var, batches;
+    double eps = 0.0, momentum = 0.0;
+    bool training = false;
+
+    int64_t batch() const { return x.size(0); }
+    int64_t points() const { return x.size(2); }
+    int64_t neighbours() const { return index.size(2); }
+    int64_t out_channels() const { return weight.size(0); }
+};
+
+struct EdgeKept {
+    Tensor matrix, uv, extreme, arg, sum, mean, var;
+};
+
+tk3d_mlp_norm norm_of(const EdgeCall &c, const EdgeKept &k)
+{
+    return {f32(k.mean), f32(k.var), f32(c.gamma), f32(c.beta), (float)c.eps};
+}
+
+Tensor edge_forward(const EdgeCall &c, EdgeKept &k, bool keep)
+{
+    const int64_t B = c.batch(), N = c.points(), K = c.neighbours(), O = c.out_channels();
+    const int64_t C = c.x.size(1);
+    const auto options = c.x.options();
+    void *stream = stream_of(c.x);
+    k.matrix = at::empty({2 * O, C}, options);
+    done(tk3d_mlp_edge_weights_f32(f32(c.weight), (int)O, (int)C, f32(k.matrix), stream),
+         "tk3d_mlp_edge_weights_f32");
+    k.uv = at::empty({B, N, 2 * O}, options);
+    tk3d_mlp_product p = product(B, 2 * O, N);
+    p.src[0] = source(c.x, f32(k.matrix), 1, C);
+    p.out = f32(k.uv);
+    run_product(TK3D_MLP_IN_RAW, TK3D_MLP_OUT_POINTS, p, stream);
+    k.extreme = at::empty({B, O, N}, options);
+    if (keep) {
+        k.arg = at::empty({B, O, N}, options.dtype(at::kByte));
+        k.sum = at::empty({B, N, O}, options);
+    }
+    const int slots = tk3d_mlp_edge_slots((int)B, (int)N);
+    const Tensor partial = partial_sums(c.x, O, slots);
+    done(tk3d_mlp_edge_forward_f32(f32(k.uv), c.index.data_ptr<int64_t>(), f32(c.gamma), (int)B,
+                                   (int)N, (int)K, (int)O, f32(k.extreme),
+                                   keep ? k.arg.data_ptr<uint8_t>() : nullptr, f32(k.sum),
+                                   partial.data_ptr(), stream),
+         "tk3d_mlp_edge_forward_f32");
+    if (c.training) {
+        const Tensor stats = at::empty({2, O}, options);
+        k.mean = stats.select(0, 0);
+        k.var = stats.select(0, 1);
+        done(tk3d_mlp_statistics_f32(partial.data_ptr(), slots, B * N * K, (int)O, (float)c.momentum,
+                                     f32(k.mean), f32(k.var), f32(c.running_mean),
+                                     f32(c.running_var),
+                                     c.batches.defined() ? c.batches.data_ptr<int64_t>() : nullptr,
+                                     stream),
+             "tk3d_mlp_statistics_f32");
+    } else {
+        k.mean = c.running_mean;
+        k.var = c.running_var;
+    }
+    const Tensor z = at::empty({B, O, N}, options);
+    const tk3d_mlp_norm norm = norm_of(c, k);
+    done(tk3d_mlp_activate_f32(f32(k.extreme), B * O, (int)O, (int)N, &norm, f32(z), stream),
+         "tk3d_mlp_activate_f32");
+    return z;
+}
+
+variable_list edge_backward(const EdgeCall &c, const EdgeKept &k, const Tensor &g, bool want_x)
+{
+    const int64_t B = c.batch(), N = c.points(), K = c.neighbours(), O = c.out_channels();
+    const int64_t C = c.x.size(1);
+    const auto options = c.x.options();
+    void *stream = stream_of(c.x);
+    const tk3d_mlp_norm norm = norm_of(c, k);
+    const Tensor affine = at::empty({2, O}, options), coef = at::empty({O, 4}, options);
+    const int slots = tk3d_mlp_mask_slots((int)B, (int)O, (int)N);
+    const Tensor partial = partial_sums(c.x, O, slots);
+    done(tk3d_mlp_mask_sums_f32(f32(g), f32(k.extreme), (int)B, (int)O, (int)N, &norm,
+                                partial.data_ptr(), stream),
+         "tk3d_mlp_mask_sums_f32");
+    done(tk3d_mlp_grad_coefficients_f32(partial.data_ptr(), slots, B * N * K, (int)O, &norm,
+                                        c.training ? 0 : 1, f32(coef), f32(affine), f32(affine) + O,
+                                        stream),
+         "tk3d_mlp_grad_coefficients_f32");
+    const Tensor sel = at::empty({B, N, O, 2}, options), duv = at::empty({B, 2 * O, N}, options);
+    done(tk3d_mlp_edge_backward_f32(f32(g), f32(k.extreme), k.arg.data_ptr<uint8_t>(), f32(k.uv),
+                                    f32(k.sum), c.lists.data_ptr<int32_t>(), (int)B, (int)N, (int)K,
+                                    (int)O, &norm, f32(coef), sel.data_ptr(), f32(duv), stream),
+         "tk3d_mlp_edge_backward_f32");
+    // dW1 = du x^T - dv x^T, dW2 = dv x^T
+    tk3d_mlp_outer o{};
+    o.B = (int32_t)B;
+    o.P = (int32_t)N;
+    o.row = source(duv, nullptr, 0, 0);
+    o.col = source(c.x, nullptr, 0, 0);
+    const int splits = tk3d_mlp_outer_splits(&o);
+    const Tensor parts = at::empty({splits, 2 * O, C}, options);
+    o.partial = f32(parts);
+    done(tk3d_mlp_outer_f32(TK3D_MLP_ROW_RAW, TK3D_MLP_COL_RAW, &o, stream), "tk3d_mlp_outer_f32");
+    const Tensor dw = at::empty(c.weight.sizes(), options);
+    const float *of_u = f32(parts), *of_v = of_u + O * C;
+    const tk3d_mlp_sum sums[2] = {
+        {of_u, of_v, f32(dw), 2 * O * C, splits, (int32_t)O, (int32_t)C, (int32_t)(2 * C)},
+        {of_v, nullptr, f32(dw) + C, 2 * O * C, splits, (int32_t)O, (int32_t)C, (int32_t)(2 * C)}};
+    done(tk3d_mlp_sum_f32(sums, 2, stream), "tk3d_mlp_sum_f32");
+    Tensor dx;
+    if (want_x) {
+        dx = at::empty(c.x.sizes(), options);
+        tk3d_mlp_product p = product(B, C, N);
+        p.src[0] = source(duv, f32(k.matrix), C, 1);
+        p.out = f32(dx);
+        run_product(TK3D_MLP_IN_RAW, TK3D_MLP_OUT_PLAIN, p, stream);
+    }
+    return {dx, dw, affine.select(0, 0), affine.select(0, 1)};
+}
+
+Tensor edge_in_stock_operators(const EdgeCall &c)
+{
+    const int64_t B = c.batch(), N = c.points(), K = c.neighbours(), C = c.x.size(1);
+    const Tensor valid = (c.index.ge(0) & c.index.lt(N)).view({B, 1, N * K});
+    const Tensor flat = c.index.view({B, 1, N * K}).clamp(0, N - 1).expand({B, C, N * K});
+    const Tensor query = c.x.unsqueeze(3).expand({B, C, N, K}).reshape({B, C, N * K});
+    const Tensor near = at::where(valid, at::gather(c.x, 2, flat), at::zeros({}, c.x.options()));
+    Tensor h = at::conv1d(at::cat({near - query, query}, 1),
+                          c.weight.view({c.out_channels(), 2 * C, 1}));
+    const Tensor none;
+    h = at::batch_norm(h, c.gamma, c.beta, c.training ? none : c.running_mean,
+                       c.training ? none : c.running_var, c.training, 0.0, c.eps, false);
+    return std::get<0>(at::max(at::relu(h).view({B, c.out_channels(), N, K}), 3));
+}
+
+struct EdgeNode : torch::autograd::Function<EdgeNode> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &x, const Tensor &weight,
+                          const Tensor &gamma, const Tensor &beta, const EdgeCall &call)
+    {
+        EdgeKept k;
+        const Tensor z = edge_forward(call, k, true);
+        ctx->save_for_backward({call.x, call.index, call.lists, call.weight, call.gamma, call.beta,
+                                k.matrix, k.uv, k.extreme, k.arg, k.sum, k.mean, k.var});
+        ctx->saved_data["training"] = call.training;
+        ctx->saved_data["eps"] = call.eps;
+        ctx->saved_data["want_x"] = x.requires_grad();
+        return z;
+    }
+
+    static variable_list backward(AutogradContext *ctx, variable_list grads)
+    {
+        const variable_list s = ctx->get_saved_variables();
+        EdgeCall c;
+        EdgeKept k;
+        c.x = s[0];
+        c.index = s[1];
+        c.lists = s[2];
+        c.weight = s[3];
+        c.gamma = s[4];
+        c.beta = s[5];
+        k.matrix = s[6];
+        k.uv = s[7];
+        k.extreme = s[8];
+        k.arg = s[9];
+        k.sum = s[10];
+        k.mean = c.running_mean = s[11];
+        k.var = c.running_var = s[12];
+        c.training = ctx->saved_data["training"].toBool();
+        c.eps = ctx->saved_data["eps"].toDouble();
+        const bool want_x = ctx->saved_data["want_x"].toBool();
+        variable_list d;
+        if (c10::GradMode::is_enabled()) {
+            const Tensor z = edge_in_stock_operators(c);
+            variable_list inputs;
+            for (const Tensor &t : {c.x, c.weight, c.gamma, c.beta})
+                if (t.requires_grad())
+                    inputs.push_back(t);
+            const variable_list found =
+                torch::autograd::grad({z}, inputs, {grads[0]}, std::nullopt, true, true);
+            size_t i = 0;
+            for (const Tensor &t : {c.x, c.weight, c.gamma, c.beta})
+                d.push_back(t.requires_grad() ? found[i++] : Tensor());
+        } else {
+            OnDeviceOf guard(c.x.device());
+            d = edge_backward(c, k, grads[0].contiguous(), want_x);
+        }
+        d.push_back(Tensor());
+        return d;
+    }
+};
+
 bool usable(const Tensor &t) { return t.is_cuda() && t.scalar_type() == at::kFloat; }
 
 }  // namespace
@@ -676,6 +868,66 @@ Tensor mlp(Tensor x, Tensor x2, const Tensor &xyz, const Tensor &centre, const T
     if (!grouped && x.dim() == 4 && !pool)
         z = z.view({shape[0], z.size(1), shape[2], shape[3]});
     return z;
+}
+
+// The inverse of a graph [B, N, K] over N points, for edge_conv(); undefined where the kernels do
+// not take its size.
+Tensor edge_lists(const Tensor &index_, int64_t n)
+{
+    if (!index_.is_cuda() || index_.dim() != 3 || index_.scalar_type() != at::kLong ||
+        index_.size(1) != n || !tk3d_mlp_edge_supported(index_.size(0), n, index_.size(2), 1))
+        return Tensor();
+    const Tensor index = index_.contiguous();
+    const int64_t B = index.size(0), K = index.size(2);
+    OnDeviceOf guard(index.device());
+    const Tensor lists = at::empty({B, n + 1 + n * K}, index.options().dtype(at::kInt));
+    done(tk3d_mlp_edge_lists(index.data_ptr<int64_t>(), (int)B, (int)n, (int)K,
+                             lists.data_ptr<int32_t>(), stream_of(index)),
+         "tk3d_mlp_edge_lists");
+    return lists;
+}
+
+// EdgeConv with one layer on the graph of x with itself; undefined where the caller has to run it
+// layer by layer.
+Tensor edge_conv(const Tensor &x, const Tensor &index, const Tensor &lists,
+                 const std::vector<Tensor> &params, const std::vector<Tensor> &buffers, double eps,
+                 double momentum, bool training)
+{
+    if (!usable(x) || x.dim() != 3 || !index.is_cuda() || index.dim() != 3 ||
+        index.scalar_type() != at::kLong || index.size(0) != x.size(0) ||
+        index.size(1) != x.size(2) || params.size() != 3)
+        return Tensor();
+    for (const Tensor &t : params)
+        if (!usable(t) || !t.is_contiguous())
+            return Tensor();
+    for (int i = 0; i < 2; ++i)
+        if (!usable(buffers[i]) || !buffers[i].is_contiguous())
+            return Tensor();
+    const int64_t B = x.size(0), C = x.size(1), N = x.size(2), K = index.size(2);
+    const int64_t O = params[0].size(0);
+    if (params[0].size(1) != 2 * C || !tk3d_mlp_edge_supported(B, N, K, O) || B * N * K < 2 ||
+        C > 4096 || (std::max(C, 2 * O) + 8) * N > (1 << 29))
+        return Tensor();
+    EdgeCall c;
+    c.x = x.contiguous();
+    c.index = index.contiguous();
+    c.weight = params[0];
+    c.gamma = params[1];
+    c.beta = params[2];
+    c.running_mean = buffers[0];
+    c.running_var = buffers[1];
+    c.batches = buffers[2];
+    c.eps = eps;
+    c.momentum = momentum;
+    c.training = training;
+    OnDeviceOf guard(x.device());
+    if (c10::GradMode::is_enabled() && (x.requires_grad() || c.weight.requires_grad() ||
+                                        c.gamma.requires_grad() || c.beta.requires_grad())) {
+        c.lists = lists.defined() ? lists : edge_lists(c.index, N);
+        return EdgeNode::apply(c.x, c.weight, c.gamma, c.beta, c);
+    }
+    EdgeKept k;
+    return edge_forward(c, k, false);
 }
 
 }  // namespace tk3d

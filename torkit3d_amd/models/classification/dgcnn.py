@@ -4,7 +4,7 @@ from torch import nn
 
 from ...nn import mlp1d_bn_relu, mlp_bn_relu
 from ...ops import native
-from ...ops.edge_conv import EdgeConvBlock
+from ...ops.edge_conv import EdgeConvBlock, edge_lists
 from ...ops.knn_points import knn_points
 from .._common import zero_biases
 
@@ -58,12 +58,18 @@ class DGCNN(nn.Module):
         every block after the first rebuilds it on its input features."""
         x = points if points_feature is None else torch.cat([points, points_feature], dim=1)
         outputs = []
+        graph = None
         for edge_conv in self.edge_convs:
             if knn_ind is None:
-                knn_ind = neighbour_index(points, self.k)
+                knn_ind, graph = neighbour_index(points, self.k), None
             elif self.feature_knn:
-                knn_ind = neighbour_index(x, self.k)
-            x = edge_conv(x, x, knn_ind)
+                knn_ind, graph = neighbour_index(x, self.k), None
+            if graph is None:
+                graph = {}
+                if x.is_cuda and x.dtype == torch.float32 and torch.is_grad_enabled():
+                    lists = edge_lists(knn_ind, x.size(2))  # one inverse for all blocks
+                    graph = {} if lists is None else {"lists": lists}
+            x = edge_conv(x, x, knn_ind, **graph)
             outputs.append(x)
         x = self.mlp_local(torch.cat(outputs, dim=1))
         pooled, max_indices = torch.max(x, 2)

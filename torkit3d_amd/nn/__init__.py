@@ -99,8 +99,24 @@ class SharedMLP(nn.Sequential):
             return None
         return self._chain(feature, None, xyz, centre, index, pool=index.size(2))
 
+    def forward_edges_max(self, x, index, lists=None):
+        """A single layer on the edge features of x's graph with itself, then the maximum over
+        the neighbours: x [B, C, N], index [B, N, K] -> [B, C', N]; ``lists`` is
+        ``edge_lists(index, N)``. None where the fused kernels do not take it."""
+        plan = self._plan(x) if len(self) == 1 else None
+        if plan is None:
+            return None
+        params, buffers, (eps,), (momentum,), training = plan
+        return _native.edge_conv(x, index, lists, params, buffers, eps, momentum, training)
+
     def _chain(self, x, x2=None, xyz=None, centre=None, index=None, pool=0):
-        like = xyz if x is None else x
+        plan = self._plan(xyz if x is None else x)
+        if plan is None:
+            return None
+        return _native.mlp(x, x2, xyz, centre, index, *plan, pool)
+
+    def _plan(self, like):
+        """(parameters, buffers, eps, momentum, training) of plain layers, or None."""
         if (not like.is_cuda or like.dtype != torch.float32 or torch.is_autocast_enabled()
                 or torch.compiler.is_compiling() or torch.jit.is_tracing()
                 or _has_any_global_hook() or type(self) is not SharedMLP
@@ -130,8 +146,7 @@ class SharedMLP(nn.Sequential):
             buffers += (mean, var, count)
             eps.append(bn.eps)
             momentum.append(bn.momentum)
-        return _native.mlp(x, x2, xyz, centre, index, params, buffers, eps, momentum,
-                           bool(training), pool)
+        return params, buffers, eps, momentum, bool(training)
 
 
 def _plain(module):

@@ -2,6 +2,7 @@
 import torch
 import torch.utils.checkpoint
 
+from .. import _native
 from ..nn import mlp2d_bn_relu
 from .group_points import group_points
 
@@ -42,6 +43,12 @@ def get_edge_feature_custom(query_feature, key_feature, key_ind, include_query=T
 get_edge_feature = get_edge_feature_custom
 
 
+def edge_lists(key_ind, num_points):
+    """The inverse of a graph [B, N, K] of a cloud with itself, as the backward of the blocks
+    needs it, or None where they do not."""
+    return _native.edge_lists(key_ind, num_points)
+
+
 class EdgeConvBlock(torch.nn.Module):
     """EdgeConv block (torkit3d/ops/edge_conv.py:8-45).
 
@@ -58,13 +65,18 @@ class EdgeConvBlock(torch.nn.Module):
         self.checkpoint = checkpoint
         self.convs = mlp2d_bn_relu(in_channels * 2, conv_channels)
 
-    def forward(self, query_feature, key_feature, key_ind):
-        """query_feature [B,C,N1], key_feature [B,C,N2], key_ind [B,N1,K] -> [B,C',N1]."""
+    def forward(self, query_feature, key_feature, key_ind, lists=None):
+        """query_feature [B,C,N1], key_feature [B,C,N2], key_ind [B,N1,K] -> [B,C',N1].
+
+        ``lists`` (not in the reference) is the inverse of the graph (``edge_lists``), for
+        callers that run several blocks on one graph; without it every block works it out."""
+        if query_feature is key_feature and not self.checkpoint:
+            output = self.convs.forward_edges_max(query_feature, key_ind, lists)
+            if output is not None:
+                return output
         edge_feature = get_edge_feature(query_feature, key_feature, key_ind)
         if self.checkpoint and edge_feature.requires_grad:
             edge_feature = torch.utils.checkpoint.checkpoint(self.convs, edge_feature,
                                                              use_reentrant=False)
-        else:
-            edge_feature = self.convs(edge_feature)
-        output, _ = edge_feature.max(dim=3)
-        return output
+            return edge_feature.max(dim=3)[0]
+        return self.convs.forward_max(edge_feature)
