@@ -150,6 +150,17 @@ int tk3d_knn_distance_bcn_f64(const double *query, const double *key, int64_t B,
                               int64_t N1, int64_t N2, int64_t k, int version,
                               double *distance, int64_t *index, void *stream);
 
+/* KNN with what knn_points does behind the op in Python (torkit3d/ops/knn_points.py:46-51) in the
+ * same call: with `sorted` a row comes in ascending distance (equal distances in slot order, NaNs
+ * last) instead of in slot order, with `root` the distances are square roots. channels_first as in
+ * tk3d_three_nn_*. k <= 64; TK3D_ERR_UNSUPPORTED (nothing launched) beyond. */
+int tk3d_knn_distance_ordered_f32(const float *query, const float *key, int channels_first,
+                                  int64_t B, int64_t N1, int64_t N2, int64_t k, int sorted, int root,
+                                  float *distance, int64_t *index, void *stream);
+int tk3d_knn_distance_ordered_f64(const double *query, const double *key, int channels_first,
+                                  int64_t B, int64_t N1, int64_t N2, int64_t k, int sorted, int root,
+                                  double *distance, int64_t *index, void *stream);
+
 /* 3 nearest neighbours and their interpolation weights in one launch. Fuses what
  * FeatureInterpolator.forward does in Python (torkit3d/layers/pointnet2.py:125-130):
  * knn_points(query, key, 3), then 1/clamp(d2, min=eps), a sum and a division as

@@ -119,3 +119,19 @@ def chamfer_scores(keys, queries):
                                                     stream_of(keys))
     assert code == 0, _lib.error_string(code)
     return scores
+
+
+def knn_wave(query, key, k, channels_first=False):
+    """[distance, index] through the wave-per-query KNN kernel whatever the launch size."""
+    from torkit3d_amd import _lib
+
+    axis = 2 if channels_first else 1
+    b, n1, n2 = query.shape[0], query.shape[axis], key.shape[axis]
+    out = [torch.empty((b, n1, k), device=query.device),
+           torch.empty((b, n1, k), dtype=torch.int64, device=query.device)]
+    code = _fn("tk3d_debug_knn_wave_f32")(
+        _lib.ptr(query), _lib.ptr(key), ctypes.c_int(1 if channels_first else 0), _lib.i64(b),
+        _lib.i64(n1), _lib.i64(n2), _lib.i64(k), *[_lib.ptr(t) for t in out],
+        _lib.stream_of(query))
+    assert code == 0, _lib.error_string(code)
+    return out

@@ -1,0 +1,92 @@
+"""The wave-per-query KNN kernel (launches of few queries, k <= 64) and the rows put in order on
+the way out, against the oracle's literal MinK: slot for slot, bit for bit."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from debug_abi import knn_wave
+from torkit3d_amd.ops.interpolate_feature import three_nn_interpolation
+from torkit3d_amd.ops.knn_points import knn_points
+
+pytestmark = pytest.mark.gpu
+
+
+def cloud(kind, seed, b, n):
+    g = np.random.default_rng(seed)
+    p = g.random((b, n, 3), dtype=np.float32)
+    if kind == "lattice":  # equal distances everywhere
+        p = np.floor(p * 4).astype(np.float32)
+    elif kind == "far to near":  # every key is inserted
+        order = np.argsort(-((p - 0.5) ** 2).sum(-1), axis=1)
+        p = np.take_along_axis(p, order[:, :, None], 1)
+    elif kind == "broken":
+        p[:, g.integers(0, n, max(1, n // 5)), 0] = np.nan
+        p[:, g.integers(0, n, max(1, n // 7)), 1] = np.inf
+        p[0, 0, 2] = np.nan  # MinK starts with a NaN maximum on this cloud
+    return p
+
+
+def same(got, want):
+    assert np.array_equal(got[0].cpu().numpy(), want[0], equal_nan=True)
+    assert np.array_equal(got[1].cpu().numpy(), want[1])
+
+
+# k around the 16, 32 and 64 lanes of the maximum, keys around the chunks of 64 and 256.
+@pytest.mark.parametrize("channels_first", [False, True])
+@pytest.mark.parametrize("kind", ["uniform", "lattice", "far to near", "broken"])
+@pytest.mark.parametrize("n2,k", [(1, 1), (2, 2), (16, 16), (63, 17), (64, 64), (65, 33), (255, 32),
+                                  (256, 3), (257, 15), (300, 64), (1000, 20), (2049, 63)])
+def test_slots(cuda, kind, n2, k, channels_first):
+    q, c = cloud("uniform", 1, 2, 37), cloud(kind, n2 + k, 2, n2)
+    a, b = torch.from_numpy(q).to(cuda), torch.from_numpy(c).to(cuda)
+    if channels_first:
+        a, b = a.transpose(1, 2).contiguous(), b.transpose(1, 2).contiguous()
+    want = oracle.knn(q, c, k)
+    same(knn_wave(a, b, k, channels_first), want)
+    same(knn_points(a, b, k, transpose=channels_first), want)
+
+
+def in_order(want, root):
+    """A stable sort of the slots, NaNs last (numpy sorts NaNs last)."""
+    order = np.argsort(want[0], axis=2, kind="stable")
+    d = np.take_along_axis(want[0], order, 2)
+    return (np.sqrt(d) if root else d), np.take_along_axis(want[1], order, 2)
+
+
+# few queries: in the wave kernel; many, or float64: a kernel over the rows (8, 16, 32, 64 lanes)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("kind", ["uniform", "lattice", "broken"])
+@pytest.mark.parametrize("n1,k", [(5, 1), (37, 7), (37, 16), (33, 24), (40, 64), (19001, 8),
+                                  (19000, 20), (37001, 33)])
+def test_rows_in_order(cuda, kind, n1, k, dtype):
+    few = 40 if n1 > 1000 else n1
+    q = np.tile(cloud("uniform", 2, 1, few), (1, n1 // few + 1, 1))[:, :n1]
+    c = cloud(kind, k, 1, 300)
+    if dtype == torch.float64:
+        q, c = q.astype(np.float64), c.astype(np.float64)
+    want = oracle.knn(q, c, k)
+    a, b = torch.from_numpy(q).to(cuda), torch.from_numpy(c).to(cuda)
+    same(knn_points(a, b, k, sorted=True), in_order(want, False))
+    same(knn_points(a, b, k, sorted=True, sqrt_distance=True), in_order(want, True))
+    with np.errstate(invalid="ignore"):
+        same(knn_points(a, b, k, sqrt_distance=True), (np.sqrt(want[0]), want[1]))
+
+
+@pytest.mark.parametrize("kind", ["uniform", "lattice"])
+@pytest.mark.parametrize("n2", [3, 64, 700])
+def test_three_nn_weights(cuda, kind, n2):
+    q, c = cloud("uniform", 3, 2, 50), cloud(kind, n2, 2, n2)
+    d, i, w = three_nn_interpolation(torch.from_numpy(q).to(cuda), torch.from_numpy(c).to(cuda))
+    want = oracle.knn(q, c, 3)
+    same((d, i), want)
+    # one division and one sum of three: the same float32 operations in the same order
+    assert np.allclose(w.cpu().numpy(), oracle.three_nn_weights(want[0]), rtol=1e-6, atol=0)
+
+
+@pytest.mark.parametrize("k,n2", [(3, 200), (8, 300), (12, 400), (24, 300), (48, 200)])
+def test_launches_of_many_queries_keep_their_kernels(cuda, k, n2):
+    """Beyond the wave kernel's launches: a lane per query, short clouds."""
+    q, c = cloud("uniform", 5, 2, 20000), cloud("lattice", 6, 2, n2)
+    same(knn_points(torch.from_numpy(q).to(cuda), torch.from_numpy(c).to(cuda), k),
+         oracle.knn(q, c, k))

@@ -1510,714 +1510,6 @@ __global__ __launch_bounds__(64) void knn_tree_kernel(
     }
 }
 
-// fp32, 17 <= k <= 32 on launches of a chip's worth of queries: the sweep of the pre-filtered kernel
-// on the matrix cores (see knn_filter_kernel_f32, MATRIX) feeding the LDS tournament tree
-// of knn_tree_kernel. A lane owns one query; a wave's 64 queries are two blocks of 32
-// (block h = the lanes of half h), so a chunk of 32 keys is two matrix instructions, the
-// lane collects the 16 sign bits of its rows in both blocks, keeps those of its own block
-// and hands the other 16 to lane ^ 32. The mask is a superset of the keys below the
-// query's maximum (slack 64 u R + 48 u M as above); every candidate is re-evaluated with
-// the canonical arithmetic and inserted under MinK's strict test in ascending key order
-// by the rounds of the tree kernel, so the slots go through exactly MinK's states. A key
-// cloud outside the range of the fp16 pieces (or non-finite) makes the workgroup compute
-// its masks with the exact distances instead, as the tree kernel does; a query outside it
-// takes every key as a candidate.
-template <int KMAX, bool IDX16, int NW>
-__global__ __launch_bounds__(64 * NW) void knn_tree_matrix_kernel_f32(
-    const float *__restrict__ query, const float *__restrict__ key,
-    float *__restrict__ distance, int64_t *__restrict__ index, int blocks_per_batch, int n1,
-    int n2, int k)
-{
-    using Lay = KnnTreeLayout<KMAX, IDX16>;
-    using Idx = typename Lay::Idx;
-    constexpr int CHUNK = 32;
-    constexpr int NT = 64;
-    constexpr int BLOCK = 64 * NW;
-    constexpr int STAGE = 256;
-    constexpr int PER = (STAGE + BLOCK - 1) / BLOCK;
-    constexpr int HALF = KMAX / 2;
-    constexpr int LEVELS = KMAX == 8 ? 3 : KMAX == 16 ? 4 : KMAX == 32 ? 5 : 6;
-    static_assert((1 << LEVELS) == KMAX, "KMAX must be a power of two from 8 to 64");
-    constexpr int TERM_BYTES = 2 * STAGE * 32;  // two stage buffers of key terms
-    extern __shared__ __align__(16) unsigned char knn_tm_lds[];
-    __shared__ float sred[NW][8];
-    uint4 *const sterm = reinterpret_cast<uint4 *>(knn_tm_lds);
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int half = lane >> 5;
-    unsigned char *const mine = knn_tm_lds + TERM_BYTES + wave * Lay::BYTES;
-    float *const leaf = reinterpret_cast<float *>(mine) + lane;
-    Idx *const kidx = reinterpret_cast<Idx *>(mine + Lay::LEAF_BYTES) + lane;
-    float *const ival = reinterpret_cast<float *>(mine + Lay::LEAF_BYTES + Lay::KIDX_BYTES) + lane;
-    unsigned char *const iarg =
-        mine + Lay::LEAF_BYTES + Lay::KIDX_BYTES + Lay::IVAL_BYTES + lane;
-
-    const int b = blockIdx.x / blocks_per_batch;
-    const int qi = (blockIdx.x - b * blocks_per_batch) * BLOCK + tid;
-    const bool active = qi < n1;
-    const float *__restrict__ K = key + (int64_t)b * n2 * 3;
-    const float INF = __builtin_huge_valf();
-    float qx = 0, qy = 0, qz = 0;
-    if (active) {
-        const float *q = query + ((int64_t)b * n1 + qi) * 3;
-        qx = q[0];
-        qy = q[1];
-        qz = q[2];
-    }
-
-    // ---- bounding box of the key cloud -> centre; largest centred norm -> scale ----
-    float lo[3] = {INF, INF, INF}, hi[3] = {-INF, -INF, -INF};
-    for (int j = tid; j < n2; j += BLOCK) {
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            const float v = K[(int64_t)j * 3 + a];
-            lo[a] = __builtin_fminf(lo[a], v);
-            hi[a] = __builtin_fmaxf(hi[a], v);
-        }
-    }
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            lo[a] = __builtin_fminf(lo[a], __shfl_xor(lo[a], o));
-            hi[a] = __builtin_fmaxf(hi[a], __shfl_xor(hi[a], o));
-        }
-    }
-    if (lane == 0) {
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            sred[wave][a] = lo[a];
-            sred[wave][3 + a] = hi[a];
-        }
-    }
-    __syncthreads();
-    float cc[3];
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        float l = INF, h = -INF;
-#pragma unroll
-        for (int w = 0; w < NW; ++w) {
-            l = __builtin_fminf(l, sred[w][a]);
-            h = __builtin_fmaxf(h, sred[w][3 + a]);
-        }
-        cc[a] = 0.5f * l + 0.5f * h;
-    }
-    const float c0 = cc[0], c1 = cc[1], c2 = cc[2];
-    float kmax2 = 0.0f;
-    for (int j = tid; j < n2; j += BLOCK) {
-        const float x = K[(int64_t)j * 3 + 0] - c0, y = K[(int64_t)j * 3 + 1] - c1,
-                    z = K[(int64_t)j * 3 + 2] - c2;
-        kmax2 = __builtin_fmaxf(kmax2, __builtin_fmaf(z, z, __builtin_fmaf(y, y, x * x)));
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1)
-        kmax2 = __builtin_fmaxf(kmax2, __shfl_xor(kmax2, o));
-    if (lane == 0)
-        sred[wave][6] = kmax2;
-    __syncthreads();
-    kmax2 = 0.0f;
-#pragma unroll
-    for (int w = 0; w < NW; ++w)
-        kmax2 = __builtin_fmaxf(kmax2, sred[w][6]);
-    // (a NaN or infinite key coordinate is skipped by the reductions above or makes the
-    // centre non-finite; either way such keys never compare below a maximum and the exact
-    // masks below handle the cloud)
-    const float ext = __builtin_sqrtf(kmax2);
-    const int ebits = (int)((__builtin_bit_cast(unsigned, ext) >> 23) & 0xffu) - 127;
-    const bool matrix = (c0 - c0 == 0.0f) && (c1 - c1 == 0.0f) && (c2 - c2 == 0.0f) &&
-                        (kmax2 < 1e30f) && (ext == 0.0f || (ebits >= -40 && ebits <= 40));  // uniform
-    const float scale =
-        (!matrix || ext == 0.0f) ? 1.0f : __builtin_bit_cast(float, (unsigned)(127 - ebits) << 23);
-    const float scale2 = scale * scale;
-    const float kmax = ext * scale * 1.000001f;
-
-    // ---- the query in rescaled units; its terms for both blocks of the wave ----
-    const float px = (qx - c0) * scale, py = (qy - c1) * scale, pz = (qz - c2) * scale;
-    const float qn = __builtin_fmaf(pz, pz, __builtin_fmaf(py, py, px * px));
-    const float qnorm = __builtin_sqrtf(qn) * 1.000001f;
-    const bool usable = matrix && qnorm <= 200.0f;  // false for NaN
-    const float rr = kmax + qnorm;
-    const float slack_r = rr * rr * 3.8146973e-06f + 1e-37f * scale2;  // 64 u R
-    uint4 qterm[2];
-    {
-        const float ax = usable ? -2.0f * px : 0.0f, ay = usable ? -2.0f * py : 0.0f,
-                    az = usable ? -2.0f * pz : 0.0f;
-        const float ox = __shfl_xor(ax, 32), oy = __shfl_xor(ay, 32), oz = __shfl_xor(az, 32);
-#pragma unroll
-        for (int hb = 0; hb < 2; ++hb) {  // block hb: the queries of the lanes of half hb
-            const bool own = half == hb;
-            const float X = own ? ax : ox, Y = own ? ay : oy, Z = own ? az : oz;
-            const unsigned sx = tk_f16_split2(X), sy = tk_f16_split2(Y), sz = tk_f16_split2(Z);
-            const unsigned xh = sx & 0xffffu, yh = sy & 0xffffu, zh = sz & 0xffffu;
-            qterm[hb] = half == 0 ? make_uint4(sx, xh | (yh << 16), (sy >> 16) | (yh << 16), 0u)
-                                  : make_uint4(sz, zh | 0x3c000000u, 0x00003c00u, 0u);
-        }
-    }
-
-    auto leaf_parent = [&](int n, float &v, int &a) {
-        const int s = 2 * n - KMAX;
-        const float lv = leaf[s * NT], rv = leaf[(s + 1) * NT];
-        const bool right = rv > lv;
-        v = right ? rv : lv;
-        a = right ? s + 1 : s;
-    };
-
-    // Fill phase: keys 0..k-1 go to slots 0..k-1 (mink.cuh:63-72); unused slots hold -inf.
-    bool frozen = false;
-    for (int s = 0; s < KMAX; ++s) {
-        float d = -INF;
-        if (s < k) {
-            d = tk_dist2<float>(K[s * 3 + 0], K[s * 3 + 1], K[s * 3 + 2], qx, qy, qz);
-            if (d != d) {
-                frozen |= s == 0;
-                d = -INF;  // marks the slot: no real distance is -inf
-            }
-        }
-        leaf[s * NT] = d;
-        kidx[s * NT] = (Idx)s;
-    }
-    for (int n = HALF - 1; n >= 1; --n) {
-        float lv, rv;
-        int la, ra;
-        if (2 * n >= HALF) {
-            leaf_parent(2 * n, lv, la);
-            leaf_parent(2 * n + 1, rv, ra);
-        } else {
-            lv = ival[2 * n * NT];
-            rv = ival[(2 * n + 1) * NT];
-            la = iarg[2 * n * NT];
-            ra = iarg[(2 * n + 1) * NT];
-        }
-        const bool right = rv > lv;
-        ival[n * NT] = right ? rv : lv;
-        iarg[n * NT] = (unsigned char)(right ? ra : la);
-    }
-    float max_key = frozen ? -INF : ival[NT];
-    int max_idx = iarg[NT];
-
-    // ---- key terms, staged STAGE keys at a time in two buffers ----
-    const int nstages = (n2 + STAGE - 1) / STAGE;
-    float pre[PER][3];
-    auto fetch = [&](int st) {
-#pragma unroll
-        for (int r = 0; r < PER; ++r) {
-            const int j = r * BLOCK + tid;
-            const int kj = st * STAGE + j;
-            pre[r][0] = pre[r][1] = pre[r][2] = INF;  // past the end
-            if (j < STAGE && kj < n2) {
-                pre[r][0] = K[(int64_t)kj * 3 + 0];
-                pre[r][1] = K[(int64_t)kj * 3 + 1];
-                pre[r][2] = K[(int64_t)kj * 3 + 2];
-            }
-        }
-    };
-    auto stash = [&](int st, int buf) {
-#pragma unroll
-        for (int r = 0; r < PER; ++r) {
-            const int j = r * BLOCK + tid;  // key within the stage
-            if (j >= STAGE)
-                continue;
-            const bool exists = st * STAGE + j < n2;
-            const float x = exists ? (pre[r][0] - c0) * scale : 0.0f;
-            const float y = exists ? (pre[r][1] - c1) * scale : 0.0f;
-            const float z = exists ? (pre[r][2] - c2) * scale : 0.0f;
-            const float n = __builtin_fmaf(z, z, __builtin_fmaf(y, y, x * x));
-            const unsigned sx = tk_f16_split2(x), sy = tk_f16_split2(y), sz = tk_f16_split2(z);
-            const unsigned xh = sx & 0xffffu, yh = sy & 0xffffu, zh = sz & 0xffffu;
-            const unsigned sn = tk_f16_split2(n);
-            const unsigned n0 = exists ? (sn & 0xffffu) : 0x7c00u, n1p = exists ? (sn >> 16) : 0u;
-            // row of the tile: lane half h of the result holds rows 8 a + 4 h + c
-            const int row = ((j & 12) << 1) | ((j & 16) >> 2) | (j & 3);
-            uint4 *t = sterm + buf * (STAGE * 2) + (j >> 5) * 64 + row;
-            t[0] = make_uint4(xh * 0x10001u, (sx >> 16) | (yh << 16), yh | (sy & 0xffff0000u),
-                              0x3c003c00u);
-            t[32] = make_uint4(zh * 0x10001u, (sz >> 16) | (n0 << 16), n1p, 0x3c003c00u);
-        }
-    };
-    if (matrix) {  // uniform
-        __syncthreads();
-        fetch(0);
-        stash(0, 0);
-        __syncthreads();
-    }
-    for (int st = 0; st < nstages; ++st) {
-        const int stage0 = st * STAGE;
-        if (matrix && st + 1 < nstages)
-            fetch(st + 1);
-        const int left = n2 - stage0;
-        const int cnt = left < STAGE ? left : STAGE;
-        for (int c0k = 0; c0k < cnt; c0k += CHUNK) {
-            const int first = stage0 + c0k;  // key index of bit 31
-            unsigned mask = 0u;
-            if (matrix) {
-                const float m = max_key * scale2;
-                const float thr = (m - qn) + __builtin_fmaf(m, 2.8610229e-06f, slack_r);
-                const unsigned tp = tk_f16_split2(-thr);
-                qterm[0].w = half == 0 ? tp : 0u;
-                qterm[1].w = half == 1 ? tp : 0u;
-                const tk_f16x8 ka = __builtin_bit_cast(
-                    tk_f16x8, sterm[(st & 1) * (STAGE * 2) + (c0k >> 5) * 64 + lane]);
-                const tk_f32x16 zero = {};
-                unsigned m16[2];
-#pragma unroll
-                for (int g = 0; g < 2; ++g) {
-                    const tk_f32x16 acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-                        ka, __builtin_bit_cast(tk_f16x8, qterm[g]), zero, 0, 0, 0);
-                    unsigned mm = 0u;
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        const float t = acc[r];
-                        mm = __builtin_amdgcn_alignbit(mm, __builtin_bit_cast(unsigned, t), 31);
-                    }
-                    m16[g] = mm;
-                }
-                const unsigned own = half == 0 ? m16[0] : m16[1];
-                const unsigned recv = __shfl_xor(half == 0 ? m16[1] : m16[0], 32);
-                mask = half == 0 ? ((own << 16) | recv) : ((recv << 16) | own);
-                mask = usable ? mask : 0xffffffffu;
-            } else {
-                const int maxbits = __builtin_bit_cast(int, max_key);
-                for (int i = 0; i < CHUNK; ++i) {
-                    const int j = first + i < n2 ? first + i : n2 - 1;  // clamped, masked below
-                    const float d = tk_dist2<float>(K[(int64_t)j * 3 + 0], K[(int64_t)j * 3 + 1],
-                                                    K[(int64_t)j * 3 + 2], qx, qy, qz);
-                    const unsigned diff = (unsigned)(__builtin_bit_cast(int, d) - maxbits);
-                    mask = __builtin_amdgcn_alignbit(mask, diff, 31);
-                }
-            }
-            // Keys that do not exist, or that the fill phase took, are no candidates.
-            int vlo = k - first;
-            vlo = vlo < 0 ? 0 : (vlo > CHUNK ? CHUNK : vlo);
-            int vhi = n2 - first;
-            vhi = vhi > CHUNK ? CHUNK : vhi;
-            unsigned valid = (vlo >= CHUNK) ? 0u : (0xffffffffu >> vlo);
-            valid &= (vhi >= CHUNK) ? 0xffffffffu : ~(0xffffffffu >> vhi);
-            mask = active ? (mask & valid) : 0u;
-
-            // ---- insertion rounds, the next candidate's key in flight during the current ----
-            const float *__restrict__ ck = K + (int64_t)first * 3;
-            bool has = mask != 0u;
-            int i = has ? __builtin_clz(mask) : 0;
-            float ex = ck[3 * i + 0], ey = ck[3 * i + 1], ez = ck[3 * i + 2];
-            while (__builtin_amdgcn_ballot_w64(has)) {  // wave-uniform
-                mask &= ~(0x80000000u >> i);  // no-op for a lane without a candidate
-                const bool has_next = mask != 0u;
-                const int i_next = has_next ? __builtin_clz(mask) : 0;
-                const float nx = ck[3 * i_next + 0], ny = ck[3 * i_next + 1],
-                            nz = ck[3 * i_next + 2];
-                const float d = tk_dist2<float>(ex, ey, ez, qx, qy, qz);
-                if (has && d < max_key) {
-                    const int p = max_idx;
-                    leaf[p * NT] = d;
-                    kidx[p * NT] = (Idx)(first + i);
-                    // the other side of every match on the path, fetched together
-                    float sv[LEVELS];
-                    int sa[LEVELS];
-                    sv[0] = leaf[(p ^ 1) * NT];
-                    sa[0] = p ^ 1;
-                    leaf_parent(((KMAX + p) >> 1) ^ 1, sv[1], sa[1]);
-#pragma unroll
-                    for (int l = 2; l < LEVELS; ++l) {
-                        const int sib = ((KMAX + p) >> l) ^ 1;
-                        sv[l] = ival[sib * NT];
-                        sa[l] = iarg[sib * NT];
-                    }
-                    float v = d;
-                    int a = p;
-#pragma unroll
-                    for (int l = 0; l < LEVELS; ++l) {
-                        const int node = (KMAX + p) >> l;
-                        // the other side wins from the right only when strictly greater
-                        const bool take = (node & 1) ? !(v > sv[l]) : (sv[l] > v);
-                        v = take ? sv[l] : v;
-                        a = take ? sa[l] : a;
-                        // parents of leaves are not stored; the root lives in max_key / max_idx
-                        if (l >= 1 && l + 1 < LEVELS) {
-                            ival[(node >> 1) * NT] = v;
-                            iarg[(node >> 1) * NT] = (unsigned char)a;
-                        }
-                    }
-                    max_key = v;
-                    max_idx = v != d ? a : p;
-                }
-                has = has_next;
-                i = i_next;
-                ex = nx;
-                ey = ny;
-                ez = nz;
-            }
-        }
-        if (matrix) {
-            if (st + 1 < nstages) {
-                __syncthreads();  // every wave is done with the buffer of the previous stage
-                stash(st + 1, (st + 1) & 1);
-            }
-            __syncthreads();
-        }
-    }
-
-    if (active) {
-        float *od = distance + ((int64_t)b * n1 + qi) * k;
-        int64_t *oi = index + ((int64_t)b * n1 + qi) * k;
-        for (int s = 0; s < k; ++s) {
-            float d = leaf[s * NT];
-            if (d == -INF)  // a NaN of the fill phase, still in its slot
-                d = tk_dist2<float>(K[s * 3 + 0], K[s * 3 + 1], K[s * 3 + 2], qx, qy, qz);
-            od[s] = d;
-            oi[s] = (int64_t)kidx[s * NT];
-        }
-    }
-}
-
-// The tree kernel for launches with few queries. One wave per 64 queries leaves most of
-// the chip idle when B * N1 is small, and the keys cannot simply be divided among waves:
-// the slot order MinK leaves behind depends on every insertion in key order. But a key
-// that the k best of a *slice* of the keys would not take is not taken by the whole
-// sequence either (the slice's k-th best so far is no better than the whole sequence's).
-// So S waves serve the same 64 queries: wave 0 runs MinK on the first slice as usual;
-// every other wave runs a MinK of its own on its slice, starting from k empty slots, and
-// logs the keys it inserts (a superset of what the whole sequence would insert from that
-// slice); then wave 0 replays the logs slice by slice, in key order, against its own
-// structure with the usual strict test. A log that overflows makes wave 0 sweep that
-// slice in full instead. The result is MinK's, slot for slot. A log entry is the key's
-// position within its slice in 16 bits, so a slice has at most 65536 keys; longer clouds
-// are taken in groups of S slices, wave 0 replaying each group before the next is swept.
-template <int KMAX, bool IDX16, int S, int CAP> struct KnnSplitLayout {
-    using Tree = KnnTreeLayout<KMAX, IDX16>;
-    using Idx = typename Tree::Idx;
-    using LogIdx = unsigned short;  // a logged key, counted from the start of its slice
-    static constexpr int LOG_BYTES = (int)sizeof(LogIdx) * CAP * 64;
-    static constexpr int LOGS_AT = S * Tree::BYTES;          // S trees, then S - 1 logs
-    static constexpr int BYTES = LOGS_AT + (S - 1) * LOG_BYTES;  // (wave 0 keeps none)
-};
-
-template <int KMAX, bool IDX16, int S, int CAP>
-__global__ __launch_bounds__(64 * S) void knn_tree_split_kernel_f32(
-    const float *__restrict__ query, const float *__restrict__ key,
-    float *__restrict__ distance, int64_t *__restrict__ index, int blocks_per_batch, int n1,
-    int n2, int k, int slice_len)
-{
-    using Lay = KnnTreeLayout<KMAX, IDX16>;
-    using Split = KnnSplitLayout<KMAX, IDX16, S, CAP>;
-    using Idx = typename Lay::Idx;
-    using LogIdx = typename Split::LogIdx;
-    constexpr int CHUNK = 32;
-    constexpr int NT = 64;
-    constexpr int HALF = KMAX / 2;
-    constexpr int LEVELS = KMAX == 8 ? 3 : KMAX == 16 ? 4 : KMAX == 32 ? 5 : KMAX == 64 ? 6
-                           : KMAX == 128 ? 7 : 8;
-    static_assert((1 << LEVELS) == KMAX, "KMAX must be a power of two from 8 to 256");
-    extern __shared__ __align__(16) unsigned char knn_split_lds[];
-    __shared__ int s_count[S][NT];
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    unsigned char *const mine = knn_split_lds + wave * Lay::BYTES;
-    float *const leaf = reinterpret_cast<float *>(mine) + lane;
-    Idx *const kidx = reinterpret_cast<Idx *>(mine + Lay::LEAF_BYTES) + lane;
-    float *const ival = reinterpret_cast<float *>(mine + Lay::LEAF_BYTES + Lay::KIDX_BYTES) + lane;
-    unsigned char *const iarg =
-        mine + Lay::LEAF_BYTES + Lay::KIDX_BYTES + Lay::IVAL_BYTES + lane;
-    auto log_of = [&](int w) {  // w >= 1
-        return reinterpret_cast<LogIdx *>(knn_split_lds + Split::LOGS_AT +
-                                          (w - 1) * Split::LOG_BYTES) + lane;
-    };
-    LogIdx *const log = log_of(wave > 0 ? wave : 1);  // wave 0 never writes one
-
-    const int b = blockIdx.x / blocks_per_batch;
-    const int qi = (blockIdx.x - b * blocks_per_batch) * NT + lane;
-    const bool active = qi < n1;
-    const float *__restrict__ K = key + (int64_t)b * n2 * 3;
-    float qx = 0, qy = 0, qz = 0;
-    if (active) {
-        const float *q = query + ((int64_t)b * n1 + qi) * 3;
-        qx = q[0];
-        qy = q[1];
-        qz = q[2];
-    }
-
-    auto leaf_parent = [&](int n, float &v, int &a) {
-        const int s = 2 * n - KMAX;
-        const float lv = leaf[s * NT], rv = leaf[(s + 1) * NT];
-        const bool right = rv > lv;
-        v = right ? rv : lv;
-        a = right ? s + 1 : s;
-    };
-
-    // Slots: wave 0 fills them with keys 0..k-1 (mink.cuh:63-72; unused slots hold -inf);
-    // the other waves start from k empty slots (+inf), which any real distance displaces.
-    bool frozen = false;
-    float max_key = 0.0f;
-    int max_idx = 0;
-    auto start_slots = [&]() {
-    for (int s = 0; s < KMAX; ++s) {
-        float d = -__builtin_huge_valf();
-        if (s < k) {
-            if (wave == 0) {
-                d = tk_dist2<float>(K[s * 3 + 0], K[s * 3 + 1], K[s * 3 + 2], qx, qy, qz);
-                if (d != d) {
-                    frozen |= s == 0;
-                    d = -__builtin_huge_valf();
-                }
-            } else {
-                d = __builtin_huge_valf();
-            }
-        }
-        leaf[s * NT] = d;
-        kidx[s * NT] = (Idx)s;
-    }
-    for (int n = HALF - 1; n >= 1; --n) {
-        float lv, rv;
-        int la, ra;
-        if (2 * n >= HALF) {
-            leaf_parent(2 * n, lv, la);
-            leaf_parent(2 * n + 1, rv, ra);
-        } else {
-            lv = ival[2 * n * NT];
-            rv = ival[(2 * n + 1) * NT];
-            la = iarg[2 * n * NT];
-            ra = iarg[(2 * n + 1) * NT];
-        }
-        const bool right = rv > lv;
-        ival[n * NT] = right ? rv : lv;
-        iarg[n * NT] = (unsigned char)(right ? ra : la);
-    }
-    max_key = frozen ? -__builtin_huge_valf() : ival[NT];
-    max_idx = iarg[NT];
-    };
-    start_slots();
-    int logged = 0;  // entries this lane wrote to its log (may exceed CAP: overflow)
-
-    // MinK's insertion of key j at distance d < max_key (see knn_tree_kernel).
-    auto insert = [&](float d, int j) {
-        const int p = max_idx;
-        leaf[p * NT] = d;
-        kidx[p * NT] = (Idx)j;
-        float sv[LEVELS];
-        int sa[LEVELS];
-        sv[0] = leaf[(p ^ 1) * NT];
-        sa[0] = p ^ 1;
-        leaf_parent(((KMAX + p) >> 1) ^ 1, sv[1], sa[1]);
-#pragma unroll
-        for (int l = 2; l < LEVELS; ++l) {
-            const int sib = ((KMAX + p) >> l) ^ 1;
-            sv[l] = ival[sib * NT];
-            sa[l] = iarg[sib * NT];
-        }
-        float v = d;
-        int a = p;
-#pragma unroll
-        for (int l = 0; l < LEVELS; ++l) {
-            const int node = (KMAX + p) >> l;
-            const bool take = (node & 1) ? !(v > sv[l]) : (sv[l] > v);
-            v = take ? sv[l] : v;
-            a = take ? sa[l] : a;
-            if (l >= 1 && l + 1 < LEVELS) {
-                ival[(node >> 1) * NT] = v;
-                iarg[(node >> 1) * NT] = (unsigned char)a;
-            }
-        }
-        max_key = v;
-        max_idx = v != d ? a : p;
-    };
-
-    // Sweep of the keys [k_begin, k_end) in chunks of 32, inserting (and, for the waves
-    // other than 0, logging) as the tree kernel does. `skip_below`: keys the fill took.
-    int log_base = 0;  // first key of the slice this wave is sweeping
-    auto sweep = [&](int k_begin, int k_end, int skip_below, bool write_log) {
-        // With one wave per SIMD nothing hides the latency of the key loads, so they run
-        // ahead: lane l holds key `held + l` (two chunks per load, the next 64 keys
-        // requested before the current ones are used) and a chunk takes its keys out of
-        // those registers lane by lane.
-        float hx = 0, hy = 0, hz = 0, nx2 = 0, ny2 = 0, nz2 = 0;
-        auto request = [&](int base) {
-            int j = base + lane;
-            j = j < k_end ? j : k_end - 1;
-            j = j < 0 ? 0 : j;
-            nx2 = K[(int64_t)j * 3 + 0];
-            ny2 = K[(int64_t)j * 3 + 1];
-            nz2 = K[(int64_t)j * 3 + 2];
-        };
-        if (k_begin < k_end)
-            request(k_begin);
-        for (int first = k_begin; first < k_end; first += CHUNK) {
-            const int within = (first - k_begin) & 63;  // 0 or 32: uniform
-            if (within == 0) {
-                hx = nx2;
-                hy = ny2;
-                hz = nz2;
-                if (first + 64 < k_end)
-                    request(first + 64);
-            }
-            const int maxbits = __builtin_bit_cast(int, max_key);
-            unsigned mask = 0u;
-            if (first + CHUNK <= k_end) {
-#pragma unroll
-                for (int i = 0; i < CHUNK; ++i) {
-                    const float kx = __builtin_bit_cast(
-                        float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, hx), within + i));
-                    const float ky = __builtin_bit_cast(
-                        float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, hy), within + i));
-                    const float kz = __builtin_bit_cast(
-                        float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, hz), within + i));
-                    const float d = tk_dist2<float>(kx, ky, kz, qx, qy, qz);
-                    const unsigned diff = (unsigned)(__builtin_bit_cast(int, d) - maxbits);
-                    mask = __builtin_amdgcn_alignbit(mask, diff, 31);
-                }
-            } else {
-                for (int i = 0; i < CHUNK; ++i) {
-                    const int j = first + i < k_end ? first + i : k_end - 1;  // masked below
-                    const float d = tk_dist2<float>(K[(int64_t)j * 3 + 0], K[(int64_t)j * 3 + 1],
-                                                    K[(int64_t)j * 3 + 2], qx, qy, qz);
-                    const unsigned diff = (unsigned)(__builtin_bit_cast(int, d) - maxbits);
-                    mask = __builtin_amdgcn_alignbit(mask, diff, 31);
-                }
-            }
-            int lo = skip_below - first;
-            lo = lo < 0 ? 0 : (lo > CHUNK ? CHUNK : lo);
-            int hi = k_end - first;
-            hi = hi > CHUNK ? CHUNK : hi;
-            unsigned valid = (lo >= CHUNK) ? 0u : (0xffffffffu >> lo);
-            valid &= (hi >= CHUNK) ? 0xffffffffu : ~(0xffffffffu >> hi);
-            mask &= valid;
-            const float *__restrict__ ck = K + (int64_t)first * 3;
-            bool has = mask != 0u;
-            int i = has ? __builtin_clz(mask) : 0;
-            float ex = ck[3 * i + 0], ey = ck[3 * i + 1], ez = ck[3 * i + 2];
-            while (__builtin_amdgcn_ballot_w64(has)) {  // wave-uniform
-                mask &= ~(0x80000000u >> i);
-                const bool has_next = mask != 0u;
-                const int i_next = has_next ? __builtin_clz(mask) : 0;
-                const float nx = ck[3 * i_next + 0], ny = ck[3 * i_next + 1],
-                            nz = ck[3 * i_next + 2];
-                const float d = tk_dist2<float>(ex, ey, ez, qx, qy, qz);
-                if (has && d < max_key) {
-                    insert(d, first + i);
-                    if (write_log) {
-                        if (logged < CAP)
-                            log[logged * NT] = (LogIdx)(first + i - log_base);
-                        ++logged;
-                    }
-                }
-                has = has_next;
-                i = i_next;
-                ex = nx;
-                ey = ny;
-                ez = nz;
-            }
-        }
-    };
-
-    // The keys are taken in groups of S slices (one group unless the cloud is longer than
-    // S slices of 65536 keys): wave 0 carries its slots from group to group, the others
-    // start every group from empty slots.
-    for (int g0 = 0; g0 < n2; g0 += S * slice_len) {  // uniform over the workgroup
-        const int k_begin = g0 + wave * slice_len;
-        const int k_end = (k_begin + slice_len < n2) ? k_begin + slice_len : n2;
-        log_base = k_begin;
-        if (wave == 0) {
-            sweep(k_begin, k_end, g0 == 0 ? k : 0, false);
-        } else {
-            if (g0 > 0)
-                start_slots();
-            logged = 0;
-            if (k_begin < n2)
-                sweep(k_begin, k_end, 0, true);
-        }
-        s_count[wave][lane] = logged;
-        __syncthreads();
-        if (wave == 0) {
-            // ---- wave 0 replays the other slices of the group in key order ----
-            for (int w = 1; w < S; ++w) {
-                const int w_begin = g0 + w * slice_len;
-                if (w_begin >= n2)
-                    break;
-                const int w_end = (w_begin + slice_len < n2) ? w_begin + slice_len : n2;
-                const int count = s_count[w][lane];
-                if (__builtin_amdgcn_ballot_w64(count > CAP)) {  // uniform: a log overflowed
-                    sweep(w_begin, w_end, 0, false);
-                    continue;
-                }
-                const LogIdx *__restrict__ wl = log_of(w);
-                int r = 0;
-                bool has = r < count;
-                int j = w_begin + (has ? (int)wl[0] : 0);
-                float ex = K[(int64_t)j * 3 + 0], ey = K[(int64_t)j * 3 + 1],
-                      ez = K[(int64_t)j * 3 + 2];
-                while (__builtin_amdgcn_ballot_w64(has)) {  // wave-uniform
-                    const bool has_next = r + 1 < count;
-                    const int j_next = w_begin + (has_next ? (int)wl[(r + 1) * NT] : 0);
-                    const float nx = K[(int64_t)j_next * 3 + 0], ny = K[(int64_t)j_next * 3 + 1],
-                                nz = K[(int64_t)j_next * 3 + 2];
-                    const float d = tk_dist2<float>(ex, ey, ez, qx, qy, qz);
-                    if (has && d < max_key)
-                        insert(d, j);
-                    ++r;
-                    has = has_next;
-                    j = j_next;
-                    ex = nx;
-                    ey = ny;
-                    ez = nz;
-                }
-            }
-        }
-        if (g0 + S * slice_len < n2)  // uniform
-            __syncthreads();  // the logs are free for the next group
-    }
-    if (wave != 0)
-        return;
-
-    if (active) {
-        float *od = distance + ((int64_t)b * n1 + qi) * k;
-        int64_t *oi = index + ((int64_t)b * n1 + qi) * k;
-        for (int s = 0; s < k; ++s) {
-            float d = leaf[s * NT];
-            if (d == -__builtin_huge_valf())  // a NaN of the fill phase, still in its slot
-                d = tk_dist2<float>(K[s * 3 + 0], K[s * 3 + 1], K[s * 3 + 2], qx, qy, qz);
-            od[s] = d;
-            oi[s] = (int64_t)kidx[s * NT];
-        }
-    }
-}
-
-// Launch with S waves per 64 queries when the plain launch would leave most SIMDs
-// without a wave; returns TK3D_ERR_UNSUPPORTED when it does not apply.
-template <int KMAX, int S, int CAP>
-int knn_tree_split_launch(const float *query, const float *key, float *distance,
-                          int64_t *index, int64_t B, int n1, int n2, int k, hipStream_t s)
-{
-    // a log holds 16-bit positions within its slice: slices of at most 65536 keys, in as
-    // many groups of S slices as that takes
-    const int groups = (int)(((int64_t)n2 + (int64_t)S * 65536 - 1) / ((int64_t)S * 65536));
-    int slice_len = (int)(((int64_t)n2 + (int64_t)S * groups - 1) / ((int64_t)S * groups));
-    slice_len = (slice_len + 31) / 32 * 32;
-    const int64_t bpb = ((int64_t)n1 + 63) / 64;
-    // Worth it when sweeping dominates the insertions (timed on an MI355X): from 2048 keys
-    // for k <= 8, 4096 for k <= 16, 8192 for k <= 32, and only while every workgroup has a
-    // CU to itself.
-    constexpr int MIN_KEYS = KMAX <= 8 ? 2048 : KMAX <= 16 ? 4096 : 8192;
-    if (n2 < MIN_KEYS || slice_len < k || B * bpb > 256)
-        return TK3D_ERR_UNSUPPORTED;
-    auto launch = [&](auto wide) {
-        // key indices of the slots in LDS: 16 bits up to 65536 keys, else 32 bits and
-        // slightly shorter logs (a slice whose log overflows is swept again by wave 0)
-        constexpr bool IDX16 = !decltype(wide)::value;
-        constexpr int LOG = IDX16 ? CAP : CAP - 16 * S;
-        using Split = KnnSplitLayout<KMAX, IDX16, S, LOG>;
-        static_assert(Split::BYTES + 64 * S * 4 <= 160 * 1024, "LDS of one CU");
-        constexpr auto kernel = knn_tree_split_kernel_f32<KMAX, IDX16, S, LOG>;
-        const int allowed = tk_allow_dynamic_lds<kernel>(Split::BYTES);
-        if (allowed != TK3D_OK)
-            return allowed;
-        hipLaunchKernelGGL(kernel, dim3((unsigned)(B * bpb)), dim3(64 * S), Split::BYTES, s,
-                           query, key, distance, index, (int)bpb, n1, n2, k, slice_len);
-        return tk_launch_status();
-    };
-    if (n2 <= 65536)
-        return launch(std::false_type{});
-    return launch(std::true_type{});
-}
-
 template <int KMAX, bool IDX16, typename T = float, bool SOA = false>
 int knn_tree_launch_as(const T *query, const T *key, T *distance, int64_t *index,
                        int64_t B, int n1, int n2, int k, hipStream_t s)
@@ -2246,28 +1538,177 @@ int knn_tree_launch(const T *query, const T *key, T *distance, int64_t *index,
     return knn_tree_launch_as<KMAX, false, T, SOA>(query, key, distance, index, B, n1, n2, k, s);
 }
 
-// The tree kernel with the matrix-core sweep: pays where the launch fills the chip and the
-// key cloud amortises the prologue (two passes over the keys per workgroup).
-// Timed against the plain tree kernel on an MI355X for k = 17..32: 1.1-1.5 times faster
-// for 32768 to 65536 queries against 4096 keys or more, slower with more queries (fewer
-// waves fit beside the staged terms, and a workgroup's waves wait for each other at every
-// stage) and no faster on shorter key clouds; for k <= 16 the register kernel above wins.
-template <int KMAX, int NW>
-int knn_tree_matrix_launch(const float *query, const float *key, float *distance,
-                           int64_t *index, int64_t B, int n1, int n2, int k, hipStream_t s)
+// ---- a wave per query ---------------------------------------------------------------------------
+//
+// With a lane per query a launch needs 65536 queries to give every SIMD a wave, and an insertion
+// is a chain of dependent LDS or register steps for the whole wave. Here a wave has ONE query and
+// up to 64 slots, a slot per lane: 64 keys are measured at once, and those below the maximum are
+// inserted one after the other in key order, which are MinK's insertions in MinK's order. The
+// kernel is bound by what an insertion issues, about k (1 + ln(N2 / k)) times per query in random
+// key order: two selects and a maximum over the lanes that hold slots (4, 5 or 6 steps). (A list
+// of the lanes in descending order, which needs no maximum, moves three values per insertion and
+// was 1.1 to 1.3 times slower.)
+// Distances are kept as bit patterns, which order as integers; a NaN is -1 in a slot, where no
+// maximum picks it, and above every maximum as a candidate, where no comparison takes it.
+
+// Maximum over the first KMAX lanes.
+template <int KMAX> __device__ __forceinline__ int knn_wave_max(int v)
 {
-    if (n2 > 65536 || n2 < 4096 || B * n1 < 32768 || B * n1 >= 131072)
+    const int none = -2147483647 - 1;
+#define TK_MAX_STEP(CTRL)                                                                      \
+    {                                                                                          \
+        const int o = __builtin_amdgcn_update_dpp(none, v, CTRL, 0xf, 0xf, false);             \
+        v = o > v ? o : v;                                                                     \
+    }
+    TK_MAX_STEP(0x111)  // row_shr:1
+    TK_MAX_STEP(0x112)
+    TK_MAX_STEP(0x114)
+    TK_MAX_STEP(0x118)
+    if constexpr (KMAX > 16)
+        TK_MAX_STEP(0x142)  // row_bcast:15
+    if constexpr (KMAX > 32)
+        TK_MAX_STEP(0x143)  // row_bcast:31
+#undef TK_MAX_STEP
+    return __builtin_amdgcn_readlane(v, KMAX - 1);
+}
+
+constexpr int KNN_WAVE_CHUNKS = 4;  // 64 keys each, requested together
+
+template <int KMAX, bool SOA, bool WEIGHTS>
+__global__ __launch_bounds__(KNN_BLOCK) void knn_wave_kernel_f32(
+    const float *__restrict__ query, const float *__restrict__ key, float *__restrict__ distance,
+    int64_t *__restrict__ index, float *__restrict__ weight, float eps, int64_t queries, int n1,
+    int n2, int k, int sorted, int root)
+{
+    const int lane = threadIdx.x & 63;
+    const int64_t row = (int64_t)blockIdx.x * (KNN_BLOCK / 64) +
+                        __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (row >= queries)
+        return;
+    const int b = (int)(row / n1), qi = (int)(row - (int64_t)b * n1);
+    const float *__restrict__ Q = query + (int64_t)b * n1 * 3;
+    const float *__restrict__ K = key + (int64_t)b * n2 * 3;
+    const float qx = knn_coord<SOA>(Q, n1, qi, 0), qy = knn_coord<SOA>(Q, n1, qi, 1),
+                qz = knn_coord<SOA>(Q, n1, qi, 2);
+
+    float px[KNN_WAVE_CHUNKS], py[KNN_WAVE_CHUNKS], pz[KNN_WAVE_CHUNKS];
+    const auto load = [&](int base) {
+#pragma unroll
+        for (int c = 0; c < KNN_WAVE_CHUNKS; ++c) {
+            int j = base + 64 * c + lane;
+            j = j < n2 ? j : n2 - 1;
+            if constexpr (SOA) {
+                px[c] = K[j];
+                py[c] = K[n2 + j];
+                pz[c] = K[2 * n2 + j];
+            } else {
+                const TkPoint3<float> p = tk_load3<float>(K + (int64_t)j * 3);
+                px[c] = p.x;
+                py[c] = p.y;
+                pz[c] = p.z;
+            }
+        }
+    };
+    load(0);
+
+    // The first k keys fill the slots (mink.cuh:63-72); with a NaN in slot 0 MinK's maximum is a
+    // NaN, which nothing is below.
+    const float filled = tk_dist2<float>(px[0], py[0], pz[0], qx, qy, qz);
+    const bool nan = filled != filled;
+    int value = lane < k && !nan ? __float_as_int(filled) : -1, where = lane;
+    int best, most = knn_wave_max<KMAX>(value);  // the slot of the maximum, the maximum
+    best = (int)__builtin_ctzll(__ballot(value == most));
+    const bool frozen = __builtin_amdgcn_readfirstlane((int)nan) != 0;
+    unsigned top = frozen || most < 0 ? 0u : (unsigned)most;  // what a key has to be below
+
+    for (int base = 0; base < n2; base += 64 * KNN_WAVE_CHUNKS) {
+        unsigned d[KNN_WAVE_CHUNKS];
+#pragma unroll
+        for (int c = 0; c < KNN_WAVE_CHUNKS; ++c) {
+            const int j = base + 64 * c + lane;
+            const unsigned bits =
+                __float_as_uint(tk_dist2<float>(px[c], py[c], pz[c], qx, qy, qz));
+            d[c] = j >= k && j < n2 ? bits : 0xffffffffu;
+        }
+        if (base + 64 * KNN_WAVE_CHUNKS < n2)
+            load(base + 64 * KNN_WAVE_CHUNKS);
+#pragma unroll
+        for (int c = 0; c < KNN_WAVE_CHUNKS; ++c) {
+            unsigned long long mask = __ballot(d[c] < top);
+            while (mask) {
+                const int l = (int)__builtin_ctzll(mask);
+                const int x = __builtin_amdgcn_readlane((int)d[c], l);
+                value = lane == best ? x : value;
+                where = lane == best ? base + 64 * c + l : where;
+                // the slot just written is the maximum unless another holds more: then the first
+                // of those that hold the most (mink.cuh:74-87)
+                most = knn_wave_max<KMAX>(value);
+                if (most > x)
+                    best = (int)__builtin_ctzll(__ballot(value == most));
+                top = (unsigned)most;
+                mask = __ballot(d[c] < top) & (~1ull << l);
+            }
+        }
+    }
+
+    // An entry goes to its slot, or to its place in ascending order (equal distances in slot
+    // order, NaNs last, as a stable sort of the slots leaves them).
+    float out = value < 0 ? filled : __int_as_float(value);  // (a NaN never leaves its slot)
+    int place = lane;
+    if (sorted) {
+        const unsigned mine = (unsigned)value;  // (NaN: the largest)
+        place = 0;
+        for (int l = 0; l < k; ++l) {
+            const unsigned other = (unsigned)__builtin_amdgcn_readlane(value, l);
+            place += other < mine || (other == mine && l < lane) ? 1 : 0;
+        }
+    }
+    if (root)
+        out = __builtin_sqrtf(out);
+    if (lane < k) {
+        distance[row * k + place] = out;
+        index[row * k + place] = where;
+    }
+    if constexpr (WEIGHTS) {  // k == 3
+        float d3[3];
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+            d3[i] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(out), i));
+        float w[3];
+        knn_three_weights<float>(d3, eps, w);
+        if (lane < 3)
+            weight[row * 3 + lane] = lane == 0 ? w[0] : lane == 1 ? w[1] : w[2];
+    }
+}
+
+// Where a wave per query wins (timed against every other kernel here on 260 shapes, 256 to 131072
+// queries, 64 to 16384 keys, k = 1 to 64; the ratio goes with the number of queries): 1.1 to 19
+// times faster up to 16384 queries, even at about 20000 (32768 with more than 32 neighbours,
+// which the lane-per-query kernels keep in LDS).
+inline bool knn_wave_pays(int64_t queries, int k)
+{
+    return k <= 64 && queries <= (k <= 32 ? 18432 : 36864);
+}
+
+template <bool SOA, bool WEIGHTS>
+int knn_wave_launch(const float *query, const float *key, float *distance, int64_t *index,
+                    float *weight, float eps, int64_t B, int n1, int n2, int k, int sorted,
+                    int root, hipStream_t s)
+{
+    const int64_t queries = B * n1, blocks = (queries + KNN_BLOCK / 64 - 1) / (KNN_BLOCK / 64);
+    if (k > 64 || blocks > TK_MAX_I32)
         return TK3D_ERR_UNSUPPORTED;
-    constexpr int LDS_BYTES = 2 * 256 * 32 + NW * KnnTreeLayout<KMAX, true>::BYTES;
-    constexpr auto kernel = knn_tree_matrix_kernel_f32<KMAX, true, NW>;
-    const int allowed = tk_allow_dynamic_lds<kernel>(LDS_BYTES);
-    if (allowed != TK3D_OK)
-        return allowed;
-    const int64_t bpb = ((int64_t)n1 + 64 * NW - 1) / (64 * NW);
-    if (B * bpb > TK_MAX_I32)
-        return TK3D_ERR_UNSUPPORTED;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)(B * bpb)), dim3(64 * NW), LDS_BYTES, s, query, key,
-                       distance, index, (int)bpb, n1, n2, k);
+#define TK_WAVE_LAUNCH(KMAX)                                                                      \
+    hipLaunchKernelGGL((knn_wave_kernel_f32<KMAX, SOA, WEIGHTS>), dim3((unsigned)blocks),         \
+                       dim3(KNN_BLOCK), 0, s, query, key, distance, index, weight, eps, queries,  \
+                       n1, n2, k, sorted, root)
+    if (k <= 16)
+        TK_WAVE_LAUNCH(16);
+    else if (k <= 32)
+        TK_WAVE_LAUNCH(32);
+    else
+        TK_WAVE_LAUNCH(64);
+#undef TK_WAVE_LAUNCH
     return tk_launch_status();
 }
 
@@ -2435,6 +1876,61 @@ int knn_filter_launch(const float *query, const float *key, float *distance, int
                                                          B, n1, n2, k, s);
 }
 
+// Rows of k <= 64 results in place: ascending distance (equal ones in slot order, NaNs last, as a
+// stable sort leaves them) if `sorted`, then square roots if `root`. W lanes to a row.
+template <typename T, int W>
+__global__ __launch_bounds__(KNN_BLOCK) void knn_rows_kernel(T *distance, int64_t *index, int64_t rows,
+                                                             int k, int sorted, int root)
+{
+    const int lane = threadIdx.x & 63, at = lane & (W - 1), first = lane - at;
+    const int64_t row = ((int64_t)blockIdx.x * KNN_BLOCK + threadIdx.x) / W;
+    const bool mine = row < rows && at < k;
+    T d = 0;
+    int64_t i = 0;
+    if (mine) {
+        d = distance[row * k + at];
+        i = index[row * k + at];
+    }
+    int place = at;
+    if (sorted) {
+        place = 0;
+        for (int l = 0; l < k; ++l) {
+            const T other = __shfl(d, first + l);
+            const bool less = other < d || (d != d && other == other);
+            const bool same = other == d || (d != d && other != other);
+            place += less || (same && l < at) ? 1 : 0;
+        }
+    }
+    if (root)
+        d = sizeof(T) == 4 ? (T)__builtin_sqrtf((float)d) : (T)__builtin_sqrt((double)d);
+    if (mine) {
+        distance[row * k + place] = d;
+        index[row * k + place] = i;
+    }
+}
+
+template <typename T>
+int knn_rows(T *distance, int64_t *index, int64_t rows, int k, int sorted, int root, hipStream_t s)
+{
+    const int width = k <= 8 ? 8 : k <= 16 ? 16 : k <= 32 ? 32 : 64;
+    const int64_t blocks = (rows * width + KNN_BLOCK - 1) / KNN_BLOCK;
+    if (k > 64 || blocks > TK_MAX_I32)
+        return TK3D_ERR_UNSUPPORTED;
+#define TK_ROWS(W)                                                                             \
+    hipLaunchKernelGGL((knn_rows_kernel<T, W>), dim3((unsigned)blocks), dim3(KNN_BLOCK), 0, s, \
+                       distance, index, rows, k, sorted, root)
+    if (width == 8)
+        TK_ROWS(8);
+    else if (width == 16)
+        TK_ROWS(16);
+    else if (width == 32)
+        TK_ROWS(32);
+    else
+        TK_ROWS(64);
+#undef TK_ROWS
+    return tk_launch_status();
+}
+
 template <typename T>
 int knn(const T *query, const T *key, int64_t B, int64_t N1, int64_t N2, int64_t k,
         int version, T *distance, int64_t *index, void *stream)
@@ -2457,6 +1953,11 @@ int knn(const T *query, const T *key, int64_t B, int64_t N1, int64_t N2, int64_t
         return TK3D_ERR_UNSUPPORTED;
     hipStream_t s = (hipStream_t)stream;
     const int n1 = (int)N1, n2 = (int)N2, kk = (int)k;
+    if constexpr (sizeof(T) == 4) {
+        if (knn_wave_pays(B * N1, kk))
+            return knn_wave_launch<false, false>(query, key, distance, index, nullptr, 0.0f, B, n1,
+                                                 n2, kk, 0, 0, s);
+    }
     if (k <= 4) {
         // the pre-filtered kernel wherever it pays (512 keys or more), else the batched kernel
         if constexpr (sizeof(T) == 4) {
@@ -2480,31 +1981,6 @@ int knn(const T *query, const T *key, int64_t B, int64_t N1, int64_t N2, int64_t
                                                           0.0f, B, n1, n2, kk, s)
                     : knn_filter_launch<32, false, false>(query, key, distance, index, nullptr,
                                                           0.0f, B, n1, n2, kk, s);
-            if (rc != TK3D_ERR_UNSUPPORTED)
-                return rc;
-        }
-        if (k <= 16) {
-            // few queries: four waves share the keys of every 64 queries (1.2-3.3 times
-            // faster from 2048 / 4096 keys on)
-            const int rc = k <= 8 ? knn_tree_split_launch<8, 4, 352>(query, key, distance, index,
-                                                                     B, n1, n2, kk, s)
-                                  : knn_tree_split_launch<16, 4, 320>(query, key, distance,
-                                                                      index, B, n1, n2, kk, s);
-            if (rc != TK3D_ERR_UNSUPPORTED)
-                return rc;
-        }
-        if (k > 16 && k <= 32) {
-            // k = 17..32 logs more insertions: two waves per 64 queries, the second wave's
-            // log gets all the spare LDS (1.15-1.5 times faster from 8192 keys on)
-            const int rc = knn_tree_split_launch<32, 2, 896>(query, key, distance, index, B, n1,
-                                                             n2, kk, s);
-            if (rc != TK3D_ERR_UNSUPPORTED)
-                return rc;
-        }
-        if (k > 16 && k <= 32) {
-            // a chip's worth of queries on long key clouds: matrix-core sweep into the tree
-            const int rc = knn_tree_matrix_launch<32, 2>(query, key, distance, index, B, n1, n2,
-                                                         kk, s);
             if (rc != TK3D_ERR_UNSUPPORTED)
                 return rc;
         }
@@ -2578,6 +2054,9 @@ int knn_bcn(const T *query, const T *key, int64_t B, int64_t N1, int64_t N2, int
         return TK3D_ERR_NULL_POINTER;
     hipStream_t s = (hipStream_t)stream;
     if constexpr (sizeof(T) == 4) {
+        if (knn_wave_pays(B * N1, kk))
+            return knn_wave_launch<true, false>(query, key, distance, index, nullptr, 0.0f, B, n1, n2,
+                                                kk, 0, 0, s);
         if (k > 4 && !knn_filter_takes(B, n1, n2, kk)) {
             // k = 17..64, or a launch the pre-filtered sweep does not pay for: the LDS tree,
             // reading the coordinate planes
@@ -2623,6 +2102,29 @@ int knn_bcn(const T *query, const T *key, int64_t B, int64_t N1, int64_t N2, int
     }
 }
 
+// KNN with the rows put in order and the square roots taken on the way out, k <= 64.
+template <typename T>
+int knn_ordered(const T *query, const T *key, bool channels_first, int64_t B, int64_t N1, int64_t N2,
+                int64_t k, int sorted, int root, T *distance, int64_t *index, void *stream)
+{
+    if (k > 64)
+        return TK3D_ERR_UNSUPPORTED;
+    if constexpr (sizeof(T) == 4) {
+        if (B > 0 && N1 > 0 && k > 0 && k <= N2 && query && key && distance && index &&
+            N1 <= TK_MAX_I32 / 4 && N2 <= TK_MAX_I32 / 4 && tk_fits(TK_MAX_ELEMS, B, N2, 3) &&
+            knn_wave_pays(B * N1, (int)k)) {
+            const auto launch = channels_first ? knn_wave_launch<true, false> : knn_wave_launch<false, false>;
+            return launch(query, key, distance, index, nullptr, 0.0f, B, (int)N1, (int)N2, (int)k,
+                          sorted, root, (hipStream_t)stream);
+        }
+    }
+    const int rc = channels_first ? knn_bcn<T>(query, key, B, N1, N2, k, 1, distance, index, stream)
+                                  : knn<T>(query, key, B, N1, N2, k, 1, distance, index, stream);
+    if (rc != TK3D_OK || B * N1 == 0 || !(sorted || root))
+        return rc;
+    return knn_rows<T>(distance, index, B * N1, (int)k, sorted, root, (hipStream_t)stream);
+}
+
 // 3 nearest neighbours with the interpolation weights formed in the same kernel.
 template <typename T>
 int three_nn(const T *query, const T *key, bool channels_first, int64_t B, int64_t N1,
@@ -2644,6 +2146,11 @@ int three_nn(const T *query, const T *key, bool channels_first, int64_t B, int64
         return TK3D_ERR_UNSUPPORTED;
     hipStream_t s = (hipStream_t)stream;
     if constexpr (sizeof(T) == 4) {
+        if (knn_wave_pays(B * N1, 3)) {
+            const auto launch = channels_first ? knn_wave_launch<true, true> : knn_wave_launch<false, true>;
+            return launch(query, key, distance, index, weight, (float)eps, B, (int)N1, (int)N2, 3, 0, 0,
+                          s);
+        }
         const int rf = channels_first
                            ? knn_filter_launch<4, true, true>(query, key, distance, index, weight,
                                                               (float)eps, B, (int)N1, (int)N2, 3, s)
@@ -2708,6 +2215,42 @@ int tk3d_knn_distance_f64(const double *query, const double *key, int64_t B, int
                           int64_t *index, void *stream)
 {
     return knn<double>(query, key, B, N1, N2, k, version, distance, index, stream);
+}
+
+int tk3d_knn_distance_ordered_f32(const float *query, const float *key, int channels_first,
+                                  int64_t B, int64_t N1, int64_t N2, int64_t k, int sorted, int root,
+                                  float *distance, int64_t *index, void *stream)
+{
+    return knn_ordered<float>(query, key, channels_first != 0, B, N1, N2, k, sorted, root, distance,
+                              index, stream);
+}
+
+int tk3d_knn_distance_ordered_f64(const double *query, const double *key, int channels_first,
+                                  int64_t B, int64_t N1, int64_t N2, int64_t k, int sorted, int root,
+                                  double *distance, int64_t *index, void *stream)
+{
+    return knn_ordered<double>(query, key, channels_first != 0, B, N1, N2, k, sorted, root, distance,
+                               index, stream);
+}
+
+int tk3d_debug_knn_wave_f32(const float *query, const float *key, int channels_first, int64_t B,
+                            int64_t N1, int64_t N2, int64_t k, float *distance, int64_t *index,
+                            void *stream)
+{
+    if (B < 0 || N1 < 0 || N2 < 0)
+        return TK3D_ERR_BAD_SIZE;
+    if (k <= 0 || k > N2)
+        return TK3D_ERR_BAD_K;
+    if (N1 > TK_MAX_I32 / 4 || N2 > TK_MAX_I32 / 4 || !tk_fits(TK_MAX_ELEMS, B, N1, k) ||
+        !tk_fits(TK_MAX_ELEMS, B, N2, 3))
+        return TK3D_ERR_UNSUPPORTED;
+    if (B * N1 == 0)
+        return TK3D_OK;
+    if (!query || !key || !distance || !index)
+        return TK3D_ERR_NULL_POINTER;
+    hipStream_t s = (hipStream_t)stream;
+    const auto launch = channels_first ? knn_wave_launch<true, false> : knn_wave_launch<false, false>;
+    return launch(query, key, distance, index, nullptr, 0.0f, B, (int)N1, (int)N2, (int)k, 0, 0, s);
 }
 
 int tk3d_debug_knn_filter_f32(const float *query, const float *key, int64_t B, int64_t N1,

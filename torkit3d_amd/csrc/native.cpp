@@ -159,9 +159,10 @@ Tensor ball_query(const Tensor &query, const Tensor &key, double radius, int64_t
     return index;
 }
 
-// Empty when the library has no kernel for this k on [B,3,N] clouds (k > 64).
+// Empty when the library has no kernel for this k on [B,3,N] clouds, or none that puts the rows in
+// order or takes roots (k > 64).
 std::vector<Tensor> knn(const Tensor &query, const Tensor &key, int64_t k, int64_t version,
-                        bool channels_first)
+                        bool channels_first, bool sorted = false, bool root = false)
 {
     const Cloud q = cloud_dims("query", query, channels_first);
     const Cloud c = cloud_dims("key", key, channels_first);
@@ -171,12 +172,15 @@ std::vector<Tensor> knn(const Tensor &query, const Tensor &key, int64_t k, int64
     check_same("query", query, "key", key);
     check(version == 0 || version == 1, "Invalid version");
     check(k >= 0, "k must be non-negative.");
-    if (channels_first && k > 64)
+    if ((channels_first || sorted || root) && k > 64)
         return {};
     OnDeviceOf guard(query.device());
     const Tensor distance = like(query, {q.b, q.n, k});
     const Tensor index = index_like(query, {q.b, q.n, k});
-    if (k > 0 && channels_first) {
+    if (k > 0 && (sorted || root)) {
+        TK3D_CALL(is_f32(query), tk3d_knn_distance_ordered, ptr(query), ptr(key), channels_first, q.b,
+                  q.n, c.n, k, sorted, root, ptr(distance), ptr(index), stream_of(query));
+    } else if (k > 0 && channels_first) {
         const int code =
             is_f32(query)
                 ? tk3d_knn_distance_bcn_f32(ptr(query), ptr(key), q.b, q.n, c.n, k, (int)version,
@@ -564,11 +568,15 @@ PYBIND11_MODULE(_host, m)
         const Tensor q = tensor_arg("query", query), c = tensor_arg("key", key);
         return unlocked([&] { return ball_query(q, c, radius, k, channels_first); });
     });
-    m.def("knn", [](py::handle query, py::handle key, int64_t k, int64_t version,
-                    bool channels_first) {
-        const Tensor q = tensor_arg("query", query), c = tensor_arg("key", key);
-        return unlocked([&] { return knn(q, c, k, version, channels_first); });
-    });
+    m.def(
+        "knn",
+        [](py::handle query, py::handle key, int64_t k, int64_t version, bool channels_first,
+           bool sorted, bool root) {
+            const Tensor q = tensor_arg("query", query), c = tensor_arg("key", key);
+            return unlocked([&] { return knn(q, c, k, version, channels_first, sorted, root); });
+        },
+        py::arg("query"), py::arg("key"), py::arg("k"), py::arg("version"),
+        py::arg("channels_first"), py::arg("sorted") = false, py::arg("root") = false);
     m.def("three_nn", [](py::handle query, py::handle key, bool channels_first, double eps) {
         const Tensor q = tensor_arg("query", query), c = tensor_arg("key", key);
         return unlocked([&] { return three_nn(q, c, channels_first, eps); });

@@ -65,6 +65,11 @@ int tk3d_debug_mfma_dot16_f16(const uint16_t *key_terms, const uint16_t *query_t
 int tk3d_debug_chamfer_scores_f32(const float *keys, const float *queries, int64_t T,
                                   float *scores, void *stream);
 
+/* The wave-per-query KNN kernel (k <= 64) whatever the launch size. */
+int tk3d_debug_knn_wave_f32(const float *query, const float *key, int channels_first, int64_t B,
+                            int64_t N1, int64_t N2, int64_t k, float *distance, int64_t *index,
+                            void *stream);
+
 /* tk3d_knn_distance_f32 through the pre-filtered kernel (knn_filter_kernel_f32, scores on
  * the matrix cores) whatever the launch size; k <= 16 and at least 256 keys. */
 int tk3d_debug_knn_filter_f32(const float *query, const float *key, int64_t B, int64_t N1,
