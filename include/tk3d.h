@@ -104,11 +104,45 @@ int tk3d_chamfer_distance_forward_bcn_f64(const double *xyz1, const double *xyz2
                                           double *dist1, int64_t *idx1, double *dist2,
                                           int64_t *idx2, void *stream);
 
+/* chamfer_distance_forward on a copy of both clouds as [B, rows, 3] with rows the next multiple of
+ * four, which the sweeps read faster than ragged lengths and short [B,3,N] clouds. `workspace`:
+ * 16-byte aligned device memory of at least the size that
+ * tk3d_chamfer_distance_forward_rows_bytes returns, which is 0 for shapes that are as fast
+ * without (pass on to the calls above). Results are bit-identical to theirs. */
+size_t tk3d_chamfer_distance_forward_rows_bytes(int64_t B, int64_t N1, int64_t N2, int channels_first);
+int tk3d_chamfer_distance_forward_rows_f32(const float *xyz1, const float *xyz2, int channels_first,
+                                           int64_t B, int64_t N1, int64_t N2, float *dist1,
+                                           int64_t *idx1, float *dist2, int64_t *idx2,
+                                           void *workspace, size_t workspace_bytes, void *stream);
+
+/* The copy alone (points past a cloud's last are NaN), both clouds in one launch. */
+int tk3d_chamfer_rows_f32(const float *xyz1, const float *xyz2, int channels_first, int64_t B,
+                          int64_t N1, int64_t N2, int64_t rows1, int64_t rows2, float *out1,
+                          float *out2, void *stream);
+int tk3d_chamfer_rows_f64(const double *xyz1, const double *xyz2, int channels_first, int64_t B,
+                          int64_t N1, int64_t N2, int64_t rows1, int64_t rows2, double *out1,
+                          double *out2, void *stream);
+
+/* What chamfer_distance(sqrt=True) does around the op in Python (torkit3d/ops/chamfer_distance.py:
+ * 6-7,57-58) for both directions in one launch: root = sqrt(max(dist, eps)), and backwards
+ * out = grad / (2 root) where dist >= eps, else 0. */
+int tk3d_chamfer_roots_f32(const float *dist1, const float *dist2, int64_t n1, int64_t n2, double eps,
+                           float *root1, float *root2, void *stream);
+int tk3d_chamfer_root_grads_f32(const float *grad1, const float *grad2, const float *dist1,
+                                const float *dist2, const float *root1, const float *root2, int64_t n1,
+                                int64_t n2, double eps, float *out1, float *out2, void *stream);
+int tk3d_chamfer_roots_f64(const double *dist1, const double *dist2, int64_t n1, int64_t n2, double eps,
+                           double *root1, double *root2, void *stream);
+int tk3d_chamfer_root_grads_f64(const double *grad1, const double *grad2, const double *dist1,
+                                const double *dist2, const double *root1, const double *root2, int64_t n1,
+                                int64_t n2, double eps, double *out1, double *out2, void *stream);
+
 /* Replaces chamfer_distance_backward_cuda
  * (chamfer_distance.h:10-16, chamfer_distance_kernel.cu:200-274).
  * grad_xyz1[b,i] = 2*gd1[b,i]*(x1[b,i]-x2[b,idx1[b,i]])
  *                  - sum over {j: idx2[b,j]==i} 2*gd2[b,j]*(x2[b,j]-x1[b,i]),
- * and symmetrically for grad_xyz2. Index entries outside [0,N) contribute nothing. */
+ * and symmetrically for grad_xyz2. Index entries outside [0,N) contribute nothing. In fp32 one of
+ * grad_xyz1 and grad_xyz2 may be NULL (not wanted; clouds of up to 2^27 points). */
 int tk3d_chamfer_distance_backward_f32(const float *grad_dist1,
                                        const float *grad_dist2, const float *xyz1,
                                        const float *xyz2, const int64_t *idx1,

@@ -1,0 +1,73 @@
+"""What surrounds the chamfer op: the copy to padded rows, one gradient alone, square roots."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from torkit3d_amd.ops.chamfer_distance import chamfer_distance, nn_distance, safe_sqrt
+
+pytestmark = pytest.mark.gpu
+
+
+def clouds(b, n1, n2, dtype=torch.float32):
+    g = torch.Generator().manual_seed(n1 + n2)
+    return [torch.rand(b, n, 3, generator=g, dtype=dtype) for n in (n1, n2)]
+
+
+# lengths on either side of a multiple of four, of the shortest cloud that is copied, and of the
+# matrix kernel's shortest
+@pytest.mark.parametrize("transpose", [False, True])
+@pytest.mark.parametrize("b,n1,n2", [(2, 255, 256), (3, 256, 257), (2, 259, 1000), (2, 1021, 1023),
+                                     (2, 1024, 1025), (3, 1027, 300), (8, 2500, 3001), (2, 4099, 1)])
+def test_copied_clouds(cuda, b, n1, n2, transpose):
+    x, y = clouds(b, n1, n2)
+    a, c = [(t.transpose(1, 2) if transpose else t).contiguous().to(cuda) for t in (x, y)]
+    for got, want in zip(nn_distance(a, c, transpose=transpose),
+                         oracle.chamfer_forward(x.numpy(), y.numpy())):
+        assert np.array_equal(got.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("transpose", [False, True])
+@pytest.mark.parametrize("which", [(True, False), (False, True), (True, True)])
+def test_gradients_that_are_wanted(cuda, which, transpose, dtype):
+    x, y = [(t.transpose(1, 2) if transpose else t).contiguous().to(cuda)
+            for t in clouds(2, 700, 5001, dtype)]
+    g1, g2 = torch.randn(2, 700, device=cuda, dtype=dtype), torch.randn(2, 5001, device=cuda, dtype=dtype)
+    both = [t.clone().requires_grad_() for t in (x, y)]
+    some = [t.clone().requires_grad_(w) for t, w in zip((x, y), which)]
+    for leaves in (both, some):
+        torch.autograd.backward(chamfer_distance(*leaves, transpose=transpose), (g1, g2))
+    for a, c, w in zip(both, some, which):
+        if not w:
+            assert c.grad is None
+        elif dtype == torch.float32:
+            assert torch.equal(a.grad, c.grad)
+        else:  # (float64 sums through atomics)
+            torch.testing.assert_close(a.grad, c.grad, rtol=1e-12, atol=1e-12)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("transpose", [False, True])
+def test_square_roots(cuda, transpose, dtype):
+    x, y = [(t.transpose(1, 2) if transpose else t).contiguous().to(cuda)
+            for t in clouds(2, 300, 513, dtype)]
+    eps = 1e-4  # above some of the squared distances, below others
+    leaves = [[t.clone().requires_grad_() for t in (x, y)] for _ in range(2)]
+    fused = chamfer_distance(*leaves[0], transpose=transpose, sqrt=True, eps=eps)
+    plain = [safe_sqrt(d, eps) for d in chamfer_distance(*leaves[1], transpose=transpose)]
+    low = sum(int((d * d <= eps * 1.0001).sum()) for d in plain)
+    assert 0 < low < 2 * (300 + 513)
+    grads = [torch.randn(2, n, device=cuda, dtype=dtype) for n in (300, 513)]
+    for f, p in zip(fused, plain):
+        assert torch.equal(f, p)
+    torch.autograd.backward(fused, grads)
+    torch.autograd.backward(plain, grads)
+    for a, c in zip(*leaves):
+        if dtype == torch.float32:
+            assert torch.equal(a.grad, c.grad)
+        else:
+            torch.testing.assert_close(a.grad, c.grad, rtol=1e-12, atol=1e-12)
+    with torch.no_grad():
+        for f, p in zip(chamfer_distance(x, y, transpose=transpose, sqrt=True, eps=eps), plain):
+            assert torch.equal(f, p)

@@ -37,6 +37,7 @@ template <typename T> struct ChamferDir {
     int blocks_per_batch;  // query blocks x key slices
     int slices;            // key slices a query's sweep is split into (1: no split)
     int slice_len;         // keys per slice, a multiple of the tile length
+    int qrows, krows;      // points from one batch element to the next in query and key
 };
 
 template <typename T> struct ChamferFwdArgs {
@@ -152,8 +153,8 @@ __device__ __forceinline__ void chamfer_exact_sweep(const ChamferDir<T> &d, int 
     const int nq = d.nq;
     const int k0 = slice * d.slice_len;  // this workgroup sweeps keys [k0, k0 + nk)
     const int nk = (d.nk - k0 < d.slice_len) ? d.nk - k0 : d.slice_len;
-    const T *__restrict__ Q = d.query + (int64_t)b * nq * 3;
-    const T *__restrict__ K = chamfer_key_base<SOA, T>(d.key, b, d.nk, k0);
+    const T *__restrict__ Q = d.query + (int64_t)b * d.qrows * 3;
+    const T *__restrict__ K = chamfer_key_base<SOA, T>(d.key, b, d.krows, k0);
 
     T qx[QPL], qy[QPL], qz[QPL], best[QPL];
     int btile[QPL];
@@ -392,8 +393,8 @@ __global__ __launch_bounds__(BLOCK) void chamfer_forward_filter_kernel(ChamferFw
     // This workgroup sweeps keys [k0, k0 + nk); to the filter that slice is the key cloud.
     const int k0 = slice * d.slice_len;
     const int nk = (d.nk - k0 < d.slice_len) ? d.nk - k0 : d.slice_len;
-    const float *__restrict__ Q = d.query + (int64_t)b * nq * 3;
-    const float *__restrict__ K = d.key + ((int64_t)b * d.nk + k0) * 3;
+    const float *__restrict__ Q = d.query + (int64_t)b * d.qrows * 3;
+    const float *__restrict__ K = d.key + ((int64_t)b * d.krows + k0) * 3;
     const float INF = __builtin_huge_valf();
 
     // ---- bounding box of the key cloud -> centre ----
@@ -836,8 +837,8 @@ __device__ __forceinline__ void chamfer_mfma_block(const ChamferDir<float> &d, c
     const int nq = d.nq;
     const int k0 = slice * d.slice_len;
     const int nk = (d.nk - k0 < d.slice_len) ? d.nk - k0 : d.slice_len;
-    const float *__restrict__ Q = d.query + (int64_t)b * nq * 3;
-    const float *__restrict__ K = chamfer_key_base<SOA, float>(d.key, b, d.nk, k0);
+    const float *__restrict__ Q = d.query + (int64_t)b * d.qrows * 3;
+    const float *__restrict__ K = chamfer_key_base<SOA, float>(d.key, b, d.krows, k0);
     const float INF = __builtin_huge_valf();
 
     // ---- centre and scale from a strided sample of the key cloud ----
@@ -1738,7 +1739,8 @@ inline int64_t chamfer_slices(int64_t nk, int64_t want, int tile, int64_t &len)
 template <typename T, int QB, int TILE>
 int chamfer_fill_args(ChamferFwdArgs<T> &a, const T *xyz1, const T *xyz2, int64_t B, int64_t N1,
                       int64_t N2, T *dist1, int64_t *idx1, T *dist2, int64_t *idx2,
-                      int want_slices, int64_t &nblocks, int want_slices_dir1 = -1)
+                      int want_slices, int64_t &nblocks, int want_slices_dir1 = -1,
+                      int64_t rows1 = 0, int64_t rows2 = 0)
 {
     // (one count for both directions unless the second is given)
     const int want[2] = {want_slices, want_slices_dir1 < 0 ? want_slices : want_slices_dir1};
@@ -1746,13 +1748,15 @@ int chamfer_fill_args(ChamferFwdArgs<T> &a, const T *xyz1, const T *xyz2, int64_
     T *dist[2] = {dist1, dist2};
     int64_t *idx[2] = {idx1, idx2};
     const int64_t nq[2] = {N1, N2}, nk[2] = {N2, N1};
+    const int64_t rows[2] = {rows1 ? rows1 : N1, rows2 ? rows2 : N2};
     int64_t nb[2];
     for (int w = 0; w < 2; ++w) {
         int64_t len;
         const int64_t slices = chamfer_slices(nk[w], sizeof(T) == 4 ? want[w] : 1, TILE, len);
         const int64_t qblocks = (nq[w] + QB - 1) / QB;
         a.dir[w] = {q[w], k[w], dist[w], idx[w], (int)nq[w], (int)nk[w],
-                    (int)(qblocks * slices), (int)slices, (int)(len > 0 ? len : 1)};
+                    (int)(qblocks * slices), (int)slices, (int)(len > 0 ? len : 1),
+                    (int)rows[w], (int)rows[1 - w]};
         nb[w] = B * qblocks * slices;
     }
     nblocks = nb[0] + nb[1];
@@ -1795,12 +1799,14 @@ int chamfer_forward_run(Kernel kernel, int block, const ChamferFwdArgs<T> &a, in
 template <typename T, int QPL, int BLOCK = 256, int TILE = 32, int STAGE = 1024, bool SOA = false>
 int chamfer_forward_launch(const T *xyz1, const T *xyz2, int64_t B, int64_t N1,
                            int64_t N2, T *dist1, int64_t *idx1, T *dist2,
-                           int64_t *idx2, hipStream_t stream, int slices = 1)
+                           int64_t *idx2, hipStream_t stream, int slices = 1, int64_t rows1 = 0,
+                           int64_t rows2 = 0)
 {
     ChamferFwdArgs<T> a;
     int64_t nblocks;
     const int rc = chamfer_fill_args<T, QPL * BLOCK, TILE>(a, xyz1, xyz2, B, N1, N2, dist1, idx1,
-                                                           dist2, idx2, slices, nblocks);
+                                                           dist2, idx2, slices, nblocks, -1, rows1,
+                                                           rows2);
     if (rc != TK3D_OK)
         return rc;
     return chamfer_forward_run<T>(chamfer_forward_kernel<T, QPL, BLOCK, TILE, STAGE, SOA>, BLOCK, a,
@@ -1810,12 +1816,13 @@ int chamfer_forward_launch(const T *xyz1, const T *xyz2, int64_t B, int64_t N1,
 template <int QPL, int BLOCK = 256, int TILE = 64, int STAGE = 1024>
 int chamfer_forward_filter_launch(const float *xyz1, const float *xyz2, int64_t B, int64_t N1,
                                   int64_t N2, float *dist1, int64_t *idx1, float *dist2,
-                                  int64_t *idx2, hipStream_t stream, int slices = 1)
+                                  int64_t *idx2, hipStream_t stream, int slices = 1,
+                                  int64_t rows1 = 0, int64_t rows2 = 0)
 {
     ChamferFwdArgs<float> a;
     int64_t nblocks;
     const int rc = chamfer_fill_args<float, QPL * BLOCK, TILE>(
-        a, xyz1, xyz2, B, N1, N2, dist1, idx1, dist2, idx2, slices, nblocks);
+        a, xyz1, xyz2, B, N1, N2, dist1, idx1, dist2, idx2, slices, nblocks, -1, rows1, rows2);
     if (rc != TK3D_OK)
         return rc;
     return chamfer_forward_run<float>(chamfer_forward_filter_kernel<QPL, BLOCK, TILE, STAGE>,
@@ -1847,12 +1854,13 @@ int chamfer_forward_mfma_flagged_launch(const float *xyz1, const float *xyz2, in
 template <int NQB, bool SOA = false, int BLOCK = 256, int STAGE = 512>
 int chamfer_forward_mfma_launch(const float *xyz1, const float *xyz2, int64_t B, int64_t N1,
                                 int64_t N2, float *dist1, int64_t *idx1, float *dist2,
-                                int64_t *idx2, hipStream_t stream, int slices0 = 1, int slices1 = 1)
+                                int64_t *idx2, hipStream_t stream, int slices0 = 1, int slices1 = 1,
+                                int64_t rows1 = 0, int64_t rows2 = 0)
 {
     ChamferFwdArgs<float> a;
     int64_t nblocks;
     const int rc = chamfer_fill_args<float, (BLOCK / TK_WAVE) * NQB * 32, 128>(
-        a, xyz1, xyz2, B, N1, N2, dist1, idx1, dist2, idx2, slices0, nblocks, slices1);
+        a, xyz1, xyz2, B, N1, N2, dist1, idx1, dist2, idx2, slices0, nblocks, slices1, rows1, rows2);
     if (rc != TK3D_OK)
         return rc;
     return chamfer_forward_run<float>(chamfer_forward_mfma_kernel<NQB, BLOCK, STAGE, SOA>, BLOCK, a,
@@ -1893,9 +1901,11 @@ inline double chamfer_sweep_cost(int64_t B, int64_t N1, int64_t N2, int qpl, int
     return (want_slices > 1 ? 20.0 : 12.0) + cycles / 2100.0;
 }
 
+// rows1, rows2: points from one batch element to the next where that is more than N1, N2.
 template <typename T, bool SOA = false>
 int chamfer_forward(const T *xyz1, const T *xyz2, int64_t B, int64_t N1, int64_t N2,
-                    T *dist1, int64_t *idx1, T *dist2, int64_t *idx2, void *stream)
+                    T *dist1, int64_t *idx1, T *dist2, int64_t *idx2, void *stream,
+                    int64_t rows1 = 0, int64_t rows2 = 0)
 {
     if (B < 0 || N1 < 0 || N2 < 0)
         return TK3D_ERR_BAD_SIZE;
@@ -1959,10 +1969,12 @@ int chamfer_forward(const T *xyz1, const T *xyz2, int64_t B, int64_t N1, int64_t
             // pre-filter also takes the launches of under 96 workgroups)
             if ((SOA || blocks >= 96) && (blocks <= 384 || (blocks <= 640 && nkmax <= 4096)))
                 return chamfer_forward_mfma_launch<2, SOA>(xyz1, xyz2, B, N1, N2, dist1, idx1,
-                                                           dist2, idx2, s, want[0], want[1]);
+                                                           dist2, idx2, s, want[0], want[1],
+                                                           rows1, rows2);
             if (blocks >= 96)
                 return chamfer_forward_mfma_launch<4, SOA>(xyz1, xyz2, B, N1, N2, dist1, idx1,
-                                                           dist2, idx2, s, want[0], want[1]);
+                                                           dist2, idx2, s, want[0], want[1],
+                                                           rows1, rows2);
         }
         if (!SOA && nkmin >= 512) {
             // Launch shapes: 4 queries per lane in 512-lane workgroups is the fastest
@@ -1979,16 +1991,16 @@ int chamfer_forward(const T *xyz1, const T *xyz2, int64_t B, int64_t N1, int64_t
             }
             if (best_slices == 0)
                 return chamfer_forward_filter_launch<4, 512, 64, 512>(
-                    xyz1, xyz2, B, N1, N2, dist1, idx1, dist2, idx2, s);
+                    xyz1, xyz2, B, N1, N2, dist1, idx1, dist2, idx2, s, 1, rows1, rows2);
             return chamfer_forward_filter_launch<2, 256, 64, 512>(
-                xyz1, xyz2, B, N1, N2, dist1, idx1, dist2, idx2, s, best_slices);
+                xyz1, xyz2, B, N1, N2, dist1, idx1, dist2, idx2, s, best_slices, rows1, rows2);
         }
     }
     if (sizeof(T) == 8 || work < (int64_t)256 * 1024)
         return chamfer_forward_launch<T, 2, 256, 32, 1024, SOA>(xyz1, xyz2, B, N1, N2, dist1, idx1,
-                                                                dist2, idx2, s);
+                                                                dist2, idx2, s, 1, rows1, rows2);
     return chamfer_forward_launch<T, 4, 512, 64, 1024, SOA>(xyz1, xyz2, B, N1, N2, dist1, idx1,
-                                                            dist2, idx2, s);
+                                                            dist2, idx2, s, 1, rows1, rows2);
 }
 
 // ---- fp32 forward on clouds sorted along a space-filling curve ---------------------
@@ -3717,9 +3729,10 @@ int chamfer_backward(const T *gd1, const T *gd2, const T *xyz1, const T *xyz2,
         !tk_fits(TK_MAX_ELEMS, B, N2, 3))
         return TK3D_ERR_UNSUPPORTED;
     const int64_t t1 = B * N1, t2 = B * N2;
-    if (t1 > 0 && (!gd1 || !xyz1 || !idx1 || !gx1))
+    // (fp32: either gradient alone may be asked for)
+    if (t1 > 0 && (!gd1 || !xyz1 || !idx1 || (!gx1 && (sizeof(T) == 8 || !gx2))))
         return TK3D_ERR_NULL_POINTER;
-    if (t2 > 0 && (!gd2 || !xyz2 || !idx2 || !gx2))
+    if (t2 > 0 && (!gd2 || !xyz2 || !idx2 || (!gx2 && (sizeof(T) == 8 || !gx1))))
         return TK3D_ERR_NULL_POINTER;
     if (t1 + t2 == 0)
         return TK3D_OK;
@@ -3728,7 +3741,9 @@ int chamfer_backward(const T *gd1, const T *gd2, const T *xyz1, const T *xyz2,
         // Every range scans all senders of its batch, so ranges are as long as LDS
         // allows: 4096 points x 3 x (8 bytes of accumulator + 4 of the point) = 144 KiB.
         constexpr int R = 4096, NT = 1024;
-        const int64_t r1 = (N1 + R - 1) / R, r2 = (N2 + R - 1) / R;
+        const int64_t r1 = gx1 ? (N1 + R - 1) / R : 0, r2 = gx2 ? (N2 + R - 1) / R : 0;
+        if (B * (r1 + r2) == 0)
+            return TK3D_OK;
         // (the kernel addresses a cloud with 32-bit byte offsets: 12 bytes a point)
         if (B * (r1 + r2) <= TK_MAX_I32 && N1 <= (1 << 27) && N2 <= (1 << 27)) {
             constexpr auto kernel = chamfer_backward_fixed_kernel<R, NT>;
@@ -3742,6 +3757,8 @@ int chamfer_backward(const T *gd1, const T *gd2, const T *xyz1, const T *xyz2,
             return tk_launch_status();
         }
     }
+    if ((t1 > 0 && !gx1) || (t2 > 0 && !gx2))
+        return TK3D_ERR_UNSUPPORTED;  // (longer clouds than the kernel above takes: both or none)
     int64_t blocks = (t1 + t2 + 255) / 256;
     if (blocks > 65536)
         blocks = 65536;
@@ -3752,6 +3769,93 @@ int chamfer_backward(const T *gd1, const T *gd2, const T *xyz1, const T *xyz2,
                        dim3(256), 0, s, gd1, gd2, xyz1, xyz2, idx1, idx2, t1, t2, (int)N1,
                        (int)N2, gx1, gx2);
     return tk_launch_status();
+}
+
+// ---- what surrounds the op -------------------------------------------------------------------
+
+// Both clouds as [B, rows, 3], from either layout; points past a cloud's last are NaN.
+template <typename T, bool SOA>
+__global__ __launch_bounds__(256) void chamfer_rows_kernel(const T *__restrict__ xyz1,
+                                                           const T *__restrict__ xyz2, int n1, int n2,
+                                                           int rows1, int rows2, int64_t total1,
+                                                           int64_t total, T *__restrict__ out1,
+                                                           T *__restrict__ out2)
+{
+    int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= total)
+        return;
+    const bool second = i >= total1;
+    i -= second ? total1 : 0;
+    const int rows = second ? rows2 : rows1, n = second ? n2 : n1;
+    const int64_t b = i / rows;
+    const int j = (int)(i - b * rows);
+    const T *base = (second ? xyz2 : xyz1) + b * n * 3;
+    T *out = (second ? out2 : out1) + i * 3;
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+        out[a] = j < n ? chamfer_coord<SOA, T>(base, n, j, a) : (T)__builtin_nanf("");
+}
+
+template <typename T>
+int chamfer_rows(const T *xyz1, const T *xyz2, bool soa, int64_t B, int64_t N1, int64_t N2,
+                 int64_t rows1, int64_t rows2, T *out1, T *out2, hipStream_t s)
+{
+    const int64_t t1 = B * rows1, total = t1 + B * rows2, blocks = (total + 255) / 256;
+    if (blocks > TK_MAX_I32)
+        return TK3D_ERR_UNSUPPORTED;
+    if (blocks == 0)
+        return TK3D_OK;
+    if (soa)
+        hipLaunchKernelGGL((chamfer_rows_kernel<T, true>), dim3((unsigned)blocks), dim3(256), 0, s, xyz1,
+                           xyz2, (int)N1, (int)N2, (int)rows1, (int)rows2, t1, total, out1, out2);
+    else
+        hipLaunchKernelGGL((chamfer_rows_kernel<T, false>), dim3((unsigned)blocks), dim3(256), 0, s, xyz1,
+                           xyz2, (int)N1, (int)N2, (int)rows1, (int)rows2, t1, total, out1, out2);
+    return tk_launch_status();
+}
+
+// Where a copy to [B, rows, 3] with rows a multiple of four pays: the matrix kernel re-evaluates its
+// candidates in 48-byte runs of four keys only if every batch element starts on 16 bytes (B=8,
+// 2500 x 3001 points: 51 us with one 12-byte load per key, 79 us with three 4-byte loads on [3,N],
+// 35 us on the copy, which takes 3), and on [3,N] clouds too short for the matrix kernel the vector
+// pre-filter, which reads [N,3] only, beats the exact sweep (8 x 1000 x 1000: 54 -> 22 us).
+inline bool chamfer_copy_pays(int64_t B, int64_t N1, int64_t N2, bool soa)
+{
+    const int64_t most = N1 > N2 ? N1 : N2, least = N1 > N2 ? N2 : N1;
+    if (B <= 0 || least <= 0 || N1 > TK_MAX_I32 / 8 || N2 > TK_MAX_I32 / 8)
+        return false;
+    if (most >= 1024)
+        return (N1 & 3) != 0 || (N2 & 3) != 0;
+    return soa && least >= 256;
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void chamfer_roots_kernel(const T *__restrict__ d1,
+                                                            const T *__restrict__ d2, int64_t n1,
+                                                            int64_t n, T eps, T *__restrict__ r1,
+                                                            T *__restrict__ r2)
+{
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n)
+        return;
+    const T d = i < n1 ? d1[i] : d2[i - n1];
+    const T c = d < eps ? eps : d;  // a NaN stays a NaN, as in clamp
+    (i < n1 ? r1[i] : r2[i - n1]) = sizeof(T) == 4 ? (T)__builtin_sqrtf((float)c) : (T)__builtin_sqrt((double)c);
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void chamfer_root_grads_kernel(
+    const T *__restrict__ g1, const T *__restrict__ g2, const T *__restrict__ d1,
+    const T *__restrict__ d2, const T *__restrict__ r1, const T *__restrict__ r2, int64_t n1, int64_t n,
+    T eps, T *__restrict__ o1, T *__restrict__ o2)
+{
+    int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n)
+        return;
+    const bool second = i >= n1;
+    i -= second ? n1 : 0;
+    const T g = (second ? g2 : g1)[i] / ((second ? r2 : r1)[i] * 2);
+    (second ? o2 : o1)[i] = (second ? d2 : d1)[i] >= eps ? g : (T)0;
 }
 
 // ---- entry points for the tests and the benchmark (tk3d_debug.h) ----------------------
@@ -3984,6 +4088,131 @@ int tk3d_debug_chamfer_scores_f32(const float *keys, const float *queries, int64
     hipLaunchKernelGGL(debug_chamfer_scores_kernel, dim3((unsigned)T), dim3(64), 0,
                        (hipStream_t)stream, keys, queries, scores);
     return tk_launch_status();
+}
+
+int tk3d_chamfer_rows_f32(const float *xyz1, const float *xyz2, int channels_first, int64_t B, int64_t N1,
+                          int64_t N2, int64_t rows1, int64_t rows2, float *out1, float *out2, void *stream)
+{
+    if (B < 0 || N1 < 0 || N2 < 0 || rows1 < N1 || rows2 < N2)
+        return TK3D_ERR_BAD_SIZE;
+    if (rows1 > TK_MAX_I32 || rows2 > TK_MAX_I32 || !tk_fits(TK_MAX_ELEMS, B, rows1, 3) ||
+        !tk_fits(TK_MAX_ELEMS, B, rows2, 3))
+        return TK3D_ERR_UNSUPPORTED;
+    if ((B * N1 > 0 && (!xyz1 || !out1)) || (B * N2 > 0 && (!xyz2 || !out2)))
+        return TK3D_ERR_NULL_POINTER;
+    return chamfer_rows<float>(xyz1, xyz2, channels_first != 0, B, N1, N2, rows1, rows2, out1, out2,
+                           (hipStream_t)stream);
+}
+
+int tk3d_chamfer_roots_f32(const float *dist1, const float *dist2, int64_t n1, int64_t n2, double eps,
+                           float *root1, float *root2, void *stream)
+{
+    if (n1 < 0 || n2 < 0)
+        return TK3D_ERR_BAD_SIZE;
+    const int64_t blocks = (n1 + n2 + 255) / 256;
+    if (blocks > TK_MAX_I32)
+        return TK3D_ERR_UNSUPPORTED;
+    if (blocks == 0)
+        return TK3D_OK;
+    hipLaunchKernelGGL((chamfer_roots_kernel<float>), dim3((unsigned)blocks), dim3(256), 0,
+                       (hipStream_t)stream, dist1, dist2, n1, n1 + n2, (float)eps, root1, root2);
+    return tk_launch_status();
+}
+
+int tk3d_chamfer_root_grads_f32(const float *grad1, const float *grad2, const float *dist1,
+                                const float *dist2, const float *root1, const float *root2, int64_t n1,
+                                int64_t n2, double eps, float *out1, float *out2, void *stream)
+{
+    if (n1 < 0 || n2 < 0)
+        return TK3D_ERR_BAD_SIZE;
+    const int64_t blocks = (n1 + n2 + 255) / 256;
+    if (blocks > TK_MAX_I32)
+        return TK3D_ERR_UNSUPPORTED;
+    if (blocks == 0)
+        return TK3D_OK;
+    hipLaunchKernelGGL((chamfer_root_grads_kernel<float>), dim3((unsigned)blocks), dim3(256), 0,
+                       (hipStream_t)stream, grad1, grad2, dist1, dist2, root1, root2, n1, n1 + n2,
+                       (float)eps, out1, out2);
+    return tk_launch_status();
+}
+
+int tk3d_chamfer_rows_f64(const double *xyz1, const double *xyz2, int channels_first, int64_t B, int64_t N1,
+                          int64_t N2, int64_t rows1, int64_t rows2, double *out1, double *out2, void *stream)
+{
+    if (B < 0 || N1 < 0 || N2 < 0 || rows1 < N1 || rows2 < N2)
+        return TK3D_ERR_BAD_SIZE;
+    if (rows1 > TK_MAX_I32 || rows2 > TK_MAX_I32 || !tk_fits(TK_MAX_ELEMS, B, rows1, 3) ||
+        !tk_fits(TK_MAX_ELEMS, B, rows2, 3))
+        return TK3D_ERR_UNSUPPORTED;
+    if ((B * N1 > 0 && (!xyz1 || !out1)) || (B * N2 > 0 && (!xyz2 || !out2)))
+        return TK3D_ERR_NULL_POINTER;
+    return chamfer_rows<double>(xyz1, xyz2, channels_first != 0, B, N1, N2, rows1, rows2, out1, out2,
+                           (hipStream_t)stream);
+}
+
+int tk3d_chamfer_roots_f64(const double *dist1, const double *dist2, int64_t n1, int64_t n2, double eps,
+                           double *root1, double *root2, void *stream)
+{
+    if (n1 < 0 || n2 < 0)
+        return TK3D_ERR_BAD_SIZE;
+    const int64_t blocks = (n1 + n2 + 255) / 256;
+    if (blocks > TK_MAX_I32)
+        return TK3D_ERR_UNSUPPORTED;
+    if (blocks == 0)
+        return TK3D_OK;
+    hipLaunchKernelGGL((chamfer_roots_kernel<double>), dim3((unsigned)blocks), dim3(256), 0,
+                       (hipStream_t)stream, dist1, dist2, n1, n1 + n2, (double)eps, root1, root2);
+    return tk_launch_status();
+}
+
+int tk3d_chamfer_root_grads_f64(const double *grad1, const double *grad2, const double *dist1,
+                                const double *dist2, const double *root1, const double *root2, int64_t n1,
+                                int64_t n2, double eps, double *out1, double *out2, void *stream)
+{
+    if (n1 < 0 || n2 < 0)
+        return TK3D_ERR_BAD_SIZE;
+    const int64_t blocks = (n1 + n2 + 255) / 256;
+    if (blocks > TK_MAX_I32)
+        return TK3D_ERR_UNSUPPORTED;
+    if (blocks == 0)
+        return TK3D_OK;
+    hipLaunchKernelGGL((chamfer_root_grads_kernel<double>), dim3((unsigned)blocks), dim3(256), 0,
+                       (hipStream_t)stream, grad1, grad2, dist1, dist2, root1, root2, n1, n1 + n2,
+                       (double)eps, out1, out2);
+    return tk_launch_status();
+}
+
+size_t tk3d_chamfer_distance_forward_rows_bytes(int64_t B, int64_t N1, int64_t N2, int channels_first)
+{
+    if (!chamfer_copy_pays(B, N1, N2, channels_first != 0))
+        return 0;
+    return (size_t)B * (size_t)(((N1 + 3) & ~3) + ((N2 + 3) & ~3)) * 3 * sizeof(float);
+}
+
+int tk3d_chamfer_distance_forward_rows_f32(const float *xyz1, const float *xyz2, int channels_first,
+                                           int64_t B, int64_t N1, int64_t N2, float *dist1,
+                                           int64_t *idx1, float *dist2, int64_t *idx2,
+                                           void *workspace, size_t workspace_bytes, void *stream)
+{
+    const int64_t rows1 = (N1 + 3) & ~3, rows2 = (N2 + 3) & ~3;
+    if (B <= 0 || N1 <= 0 || N2 <= 0 || workspace == nullptr ||
+        (reinterpret_cast<uintptr_t>(workspace) & 15) != 0 ||
+        !tk_fits(TK_MAX_ELEMS, B, rows1 + rows2, 3) ||
+        workspace_bytes < (size_t)B * (size_t)(rows1 + rows2) * 3 * sizeof(float))
+        return channels_first
+                   ? chamfer_forward<float, true>(xyz1, xyz2, B, N1, N2, dist1, idx1, dist2, idx2, stream)
+                   : chamfer_forward<float>(xyz1, xyz2, B, N1, N2, dist1, idx1, dist2, idx2, stream);
+    if (!xyz1 || !xyz2 || !dist1 || !idx1 || !dist2 || !idx2)
+        return TK3D_ERR_NULL_POINTER;
+    if (rows1 > TK_MAX_I32 / 4 || rows2 > TK_MAX_I32 / 4)
+        return TK3D_ERR_UNSUPPORTED;
+    float *copy1 = static_cast<float *>(workspace), *copy2 = copy1 + B * rows1 * 3;
+    const int rc = chamfer_rows<float>(xyz1, xyz2, channels_first != 0, B, N1, N2, rows1, rows2, copy1,
+                                       copy2, (hipStream_t)stream);
+    if (rc != TK3D_OK)
+        return rc;
+    return chamfer_forward<float>(copy1, copy2, B, N1, N2, dist1, idx1, dist2, idx2, stream, rows1,
+                                  rows2);
 }
 
 }  // extern "C"

@@ -231,12 +231,20 @@ std::vector<Tensor> chamfer_forward(const Tensor &xyz1, const Tensor &xyz2, bool
         const bool sortable = !channels_first || std::max(a.n, c.n) <= 16384;
         const size_t bytes =
             sortable ? tk3d_chamfer_distance_forward_workspace_bytes(a.b, a.n, c.n, 0) : 0;
-        const Tensor ws = scratch(xyz1, bytes);
+        const size_t copy_bytes =
+            bytes ? 0 : tk3d_chamfer_distance_forward_rows_bytes(a.b, a.n, c.n, channels_first);
+        const Tensor ws = scratch(xyz1, bytes ? bytes : copy_bytes);
         const auto call = channels_first ? tk3d_chamfer_distance_forward_bcn_f32
                                          : tk3d_chamfer_distance_forward_ws_f32;
-        done(call(ptr(xyz1), ptr(xyz2), a.b, a.n, c.n, ptr(dist1), ptr(idx1), ptr(dist2),
-                  ptr(idx2), ptr(ws), bytes, stream),
-             "tk3d_chamfer_distance_forward_f32");
+        if (copy_bytes)
+            done(tk3d_chamfer_distance_forward_rows_f32(
+                     ptr(xyz1), ptr(xyz2), channels_first, a.b, a.n, c.n, ptr(dist1), ptr(idx1),
+                     ptr(dist2), ptr(idx2), ptr(ws), copy_bytes, stream),
+                 "tk3d_chamfer_distance_forward_rows_f32");
+        else
+            done(call(ptr(xyz1), ptr(xyz2), a.b, a.n, c.n, ptr(dist1), ptr(idx1), ptr(dist2),
+                      ptr(idx2), ptr(ws), bytes, stream),
+                 "tk3d_chamfer_distance_forward_f32");
     } else {
         const auto call = channels_first ? tk3d_chamfer_distance_forward_bcn_f64
                                          : tk3d_chamfer_distance_forward_f64;
@@ -248,7 +256,8 @@ std::vector<Tensor> chamfer_forward(const Tensor &xyz1, const Tensor &xyz2, bool
 }
 
 std::vector<Tensor> chamfer_backward(const Tensor &grad1, const Tensor &grad2, const Tensor &xyz1,
-                                     const Tensor &xyz2, const Tensor &idx1, const Tensor &idx2)
+                                     const Tensor &xyz2, const Tensor &idx1, const Tensor &idx2,
+                                     bool want1 = true, bool want2 = true)
 {
     check_contiguous_cuda("grad_dist1", grad1);
     check_contiguous_cuda("grad_dist2", grad2);
@@ -277,7 +286,13 @@ std::vector<Tensor> chamfer_backward(const Tensor &grad1, const Tensor &grad2, c
     check_same("grad_dist2", grad2, "xyz2", xyz2);
     check_same("xyz1", xyz1, "xyz2", xyz2);
     OnDeviceOf guard(xyz1.device());
-    const Tensor grad_xyz1 = like(xyz1, {b, n1, 3}), grad_xyz2 = like(xyz1, {b, n2, 3});
+    if (!is_f32(xyz1) || std::max(n1, n2) > (1 << 27))
+        want1 = want2 = true;  // (one gradient alone: the fp32 kernel)
+    Tensor grad_xyz1, grad_xyz2;
+    if (want1)
+        grad_xyz1 = like(xyz1, {b, n1, 3});
+    if (want2)
+        grad_xyz2 = like(xyz1, {b, n2, 3});
     TK3D_CALL(is_f32(xyz1), tk3d_chamfer_distance_backward, ptr(grad1), ptr(grad2), ptr(xyz1),
               ptr(xyz2), ptr(idx1), ptr(idx2), b, n1, n2, ptr(grad_xyz1), ptr(grad_xyz2),
               stream_of(xyz1));
@@ -418,41 +433,81 @@ Tensor interpolate_backward(const Tensor &grad, const Tensor &index, const Tenso
 
 bool tracked(const Tensor &t) { return t.defined() && t.requires_grad(); }
 
+// sqrt(max(d, eps)) of both directions.
+std::vector<Tensor> roots(const Tensor &d1, const Tensor &d2, double eps)
+{
+    OnDeviceOf guard(d1.device());
+    const Tensor r1 = like(d1, d1.sizes()), r2 = like(d2, d2.sizes());
+    TK3D_CALL(is_f32(d1), tk3d_chamfer_roots, ptr(d1), ptr(d2), d1.numel(), d2.numel(), eps, ptr(r1),
+              ptr(r2), stream_of(d1));
+    return {r1, r2};
+}
+
 struct ChamferNode : torch::autograd::Function<ChamferNode> {
     static variable_list forward(AutogradContext *ctx, const Tensor &xyz1, const Tensor &xyz2,
-                                 bool channels_first)
+                                 bool channels_first, bool root, double eps)
     {
-        const std::vector<Tensor> out =
-            chamfer_forward(xyz1.contiguous(), xyz2.contiguous(), channels_first);
-        ctx->save_for_backward({xyz1.contiguous(), xyz2.contiguous(), out[1], out[3]});
+        const Tensor a = xyz1.contiguous(), c = xyz2.contiguous();
+        const std::vector<Tensor> out = chamfer_forward(a, c, channels_first);
         ctx->saved_data["channels_first"] = channels_first;
-        return {out[0], out[2]};
+        ctx->saved_data["want"] = (xyz1.requires_grad() ? 1 : 0) + (xyz2.requires_grad() ? 2 : 0);
+        if (!root) {
+            ctx->save_for_backward({a, c, out[1], out[3]});
+            return {out[0], out[2]};
+        }
+        const std::vector<Tensor> r = roots(out[0], out[2], eps);
+        ctx->saved_data["eps"] = eps;
+        ctx->save_for_backward({a, c, out[1], out[3], out[0], out[2], r[0], r[1]});
+        return r;
     }
     static variable_list backward(AutogradContext *ctx, variable_list grads)
     {
         const variable_list saved = ctx->get_saved_variables();
-        if (!ctx->saved_data["channels_first"].toBool()) {
-            const std::vector<Tensor> g =
-                chamfer_backward(grads[0].contiguous(), grads[1].contiguous(), saved[0], saved[1],
-                                 saved[2], saved[3]);
-            return {g[0], g[1], Tensor()};
+        const int64_t want = ctx->saved_data["want"].toInt();
+        const bool channels_first = ctx->saved_data["channels_first"].toBool();
+        Tensor g1 = grads[0].contiguous(), g2 = grads[1].contiguous();
+        Tensor a = saved[0], c = saved[1];
+        OnDeviceOf guard(a.device());
+        if (saved.size() > 4) {
+            const Tensor o1 = like(g1, g1.sizes()), o2 = like(g2, g2.sizes());
+            TK3D_CALL(is_f32(g1), tk3d_chamfer_root_grads, ptr(g1), ptr(g2), ptr(saved[4]),
+                      ptr(saved[5]), ptr(saved[6]), ptr(saved[7]), g1.numel(), g2.numel(),
+                      ctx->saved_data["eps"].toDouble(), ptr(o1), ptr(o2), stream_of(g1));
+            g1 = o1;
+            g2 = o2;
         }
-        // (the backward kernel works on [B,N,3])
-        const std::vector<Tensor> g = chamfer_backward(
-            grads[0].contiguous(), grads[1].contiguous(), saved[0].transpose(1, 2).contiguous(),
-            saved[1].transpose(1, 2).contiguous(), saved[2], saved[3]);
-        return {g[0].transpose(1, 2), g[1].transpose(1, 2), Tensor()};
+        if (channels_first) {  // (the backward kernel works on [B,N,3])
+            const int64_t b = a.size(0), n1 = a.size(2), n2 = c.size(2);
+            const Tensor a3 = like(a, {b, n1, 3}), c3 = like(c, {b, n2, 3});
+            TK3D_CALL(is_f32(a), tk3d_chamfer_rows, ptr(a), ptr(c), 1, b, n1, n2, n1, n2, ptr(a3),
+                      ptr(c3), stream_of(a));
+            a = a3;
+            c = c3;
+        }
+        std::vector<Tensor> g = chamfer_backward(g1, g2, a, c, saved[2], saved[3], (want & 1) != 0,
+                                                 (want & 2) != 0);
+        for (int i = 0; i < 2; ++i) {
+            if (!(want & (1 << i)))
+                g[i] = Tensor();
+            else if (channels_first)
+                g[i] = g[i].transpose(1, 2);
+        }
+        return {g[0], g[1], Tensor(), Tensor(), Tensor()};
     }
 };
 
-std::tuple<Tensor, Tensor> chamfer(const Tensor &xyz1, const Tensor &xyz2, bool channels_first)
+std::tuple<Tensor, Tensor> chamfer(const Tensor &xyz1, const Tensor &xyz2, bool channels_first,
+                                   bool root, double eps)
 {
     if (c10::GradMode::is_enabled() && (tracked(xyz1) || tracked(xyz2))) {
-        const variable_list out = ChamferNode::apply(xyz1, xyz2, channels_first);
+        const variable_list out = ChamferNode::apply(xyz1, xyz2, channels_first, root, eps);
         return {out[0], out[1]};
     }
-    const std::vector<Tensor> out =
-        chamfer_forward(xyz1.contiguous(), xyz2.contiguous(), channels_first);
+    std::vector<Tensor> out = chamfer_forward(xyz1.contiguous(), xyz2.contiguous(), channels_first);
+    if (root) {
+        const std::vector<Tensor> r = roots(out[0], out[2], eps);
+        return {r[0], r[1]};
+    }
     return {out[0], out[2]};
 }
 
@@ -624,9 +679,10 @@ PYBIND11_MODULE(_host, m)
     });
 
     // differentiable forms
-    m.def("chamfer", [](py::handle xyz1, py::handle xyz2, bool channels_first) {
+    m.def("chamfer", [](py::handle xyz1, py::handle xyz2, bool channels_first, bool root,
+                        double eps) {
         const Tensor a = tensor_arg("xyz1", xyz1), c = tensor_arg("xyz2", xyz2);
-        return unlocked([&] { return chamfer(a, c, channels_first); });
+        return unlocked([&] { return chamfer(a, c, channels_first, root, eps); });
     });
     m.def("group_points", [](py::handle points, py::handle index) {
         const Tensor x = tensor_arg("input", points), i = tensor_arg("index", index);
