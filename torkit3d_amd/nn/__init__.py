@@ -78,6 +78,8 @@ class SharedMLP(nn.Sequential):
     modules in place of the blocks', frozen layers among training ones, autocast - runs layer
     by layer in stock torch."""
 
+    fused_training = True  # whether training mode takes the fused kernels too
+
     def forward(self, x):
         out = self._chain(x)
         return super().forward(x) if out is None else out
@@ -138,6 +140,8 @@ class SharedMLP(nn.Sequential):
                 return None
             if training is None:
                 training = bn.training
+                if training and not self.fused_training:
+                    return None
             weight, gamma, beta = conv._parameters["weight"], *bn._parameters.values()
             mean, var, count = bn._buffers.values()
             if training != bn.training or gamma is None or beta is None or mean is None:
