@@ -1,0 +1,154 @@
+"""What may be done to a ``SharedMLP`` besides calling it: whatever an ``nn.Sequential`` of the same
+blocks takes (scripting, symbolic tracing, function transforms, forward-mode gradients, foreign
+modules in its place, replicas without parameters) it takes too, with the result of the stock
+layers; and what those refuse stays refused."""
+import copy
+
+import pytest
+import torch
+from torch import nn
+from torch.autograd import forward_ad
+from torch.func import functional_call, grad, jvp, vmap
+
+import torkit3d_amd.nn
+from torkit3d_amd.layers.pointnet2 import FeaturePropagation
+from torkit3d_amd.nn import forward_cat, forward_max, mlp1d_bn_relu, mlp2d_bn_relu
+
+DEVICES = ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)]
+
+
+def pair(device, build=mlp1d_bn_relu, widths=(6, 8, 40)):
+    """A chain in evaluation mode and the same layers as an nn.Sequential."""
+    torch.manual_seed(0)
+    mlp = build(widths[0], widths[1:]).to(device).eval()
+    for m in mlp.modules():
+        if isinstance(m, (nn.BatchNorm1d, nn.BatchNorm2d)):
+            nn.init.uniform_(m.running_var, 0.5, 2.0)
+    return mlp, nn.Sequential(*copy.deepcopy(mlp).children()).eval()
+
+
+def close(a, b):
+    # (two orders of float32 sums over up to 8 terms through two layers)
+    torch.testing.assert_close(a, b, rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("device", DEVICES)
+def test_scripted_and_traced(device):
+    mlp, stock = pair(device)
+    x = torch.rand(2, 6, 33, device=device)
+    with torch.no_grad():
+        want = stock(x)
+        close(torch.jit.script(mlp)(x), want)
+        close(torch.jit.trace(mlp, x)(x), want)
+        close(torch.fx.symbolic_trace(mlp)(x), want)
+        close(mlp(input=x), want)
+
+
+@pytest.mark.parametrize("device", DEVICES)
+def test_function_transforms(device):
+    mlp, stock = pair(device)
+    x, t = torch.rand(3, 6, 33, device=device), torch.rand(3, 6, 33, device=device)
+    for m in (mlp, stock):
+        m.requires_grad_(False)
+    close(vmap(lambda v: mlp(v[None])[0])(x), vmap(lambda v: stock(v[None])[0])(x))
+    for a, b in zip(jvp(mlp, (x,), (t,)), jvp(stock, (x,), (t,))):
+        close(a, b)
+
+    def grads(m):
+        params, buffers = dict(m.named_parameters()), dict(m.named_buffers())
+        return grad(lambda p: functional_call(m, (p, buffers), (x,)).square().sum())(params)
+
+    for a, b in zip(grads(mlp).values(), grads(stock).values()):
+        close(a, b)
+    # the function under the transform does not depend on what is transformed
+    close(vmap(lambda v: stock(x).sum() * v)(t[0, 0]), vmap(lambda v: mlp(x).sum() * v)(t[0, 0]))
+    with forward_ad.dual_level(), torch.no_grad():
+        dual = forward_ad.make_dual(x, t)
+        close(forward_ad.unpack_dual(mlp(dual)).tangent, forward_ad.unpack_dual(stock(dual)).tangent)
+
+
+def test_foreign_modules_in_place_of_a_chain():
+    mlp, stock = pair("cpu", mlp2d_bn_relu)
+    x = torch.rand(2, 6, 5, 7)
+    close(forward_max(stock, x), forward_max(mlp, x))
+    layer = FeaturePropagation(6, (8, 40)).eval()
+    x2 = torch.rand(2, 4, 9)
+    want = layer.mlp(torch.cat([x2[:, :2], x2], dim=1))
+    layer.mlp = nn.Sequential(*layer.mlp.children())
+    close(forward_cat(layer.mlp, x2[:, :2], x2), want)
+
+
+def test_replica_without_parameters_is_left_to_stock(monkeypatch):
+    # (what nn.DataParallel makes of a module: tensors as plain attributes)
+    mlp, _ = pair("cpu")
+
+    def replica_of(module):
+        replica = module._replicate_for_data_parallel()
+        replica._modules = {name: replica_of(child) for name, child in module.named_children()}
+        for name, value in module.named_parameters(recurse=False):
+            setattr(replica, name, value.detach().clone())
+        return replica
+
+    class OnGpu:  # what the plan looks at
+        is_cuda, dtype = True, torch.float32
+
+    monkeypatch.setattr(torkit3d_amd.nn, "_TENSORS", (OnGpu,))
+    assert mlp._plan(OnGpu()) is not None and replica_of(mlp)._plan(OnGpu()) is None
+    monkeypatch.setattr(torkit3d_amd.nn, "_TENSORS", ())
+    assert mlp._plan(OnGpu()) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("at", [0, 31, 40])
+def test_nan_reaches_the_maximum(at):
+    """One NaN among the neighbours: in the group it is in, as torch's maximum has it."""
+    mlp, stock = pair("cuda", mlp2d_bn_relu)
+    x = torch.rand(1, 6, 3, 64, device="cuda")
+    x[0, 2, 1, at] = float("nan")
+    want = torch.max(stock(x), dim=3)[0]
+    for grads in (False, True):
+        with torch.set_grad_enabled(grads):
+            got = mlp.forward_max(x)
+        assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.isnan(got[0, :, 1]).all()
+        close(torch.nan_to_num(got), torch.nan_to_num(want))
+
+
+@pytest.mark.gpu
+def test_nan_reaches_the_maximum_over_edges():
+    from torkit3d_amd.ops.edge_conv import EdgeConvBlock
+
+    torch.manual_seed(0)
+    block = EdgeConvBlock(3, (16,)).cuda().eval()
+    x = torch.rand(1, 3, 40, device="cuda")
+    x[0, 1, 7] = float("nan")
+    index = torch.randint(0, 40, (1, 40, 9), device="cuda")
+    got = block(x, x, index)
+    want = block(x, x.clone(), index)  # (two clouds: the general path)
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+
+
+@pytest.mark.gpu
+def test_running_statistics_count_as_written():
+    """A pass in training mode changes what a pass in evaluation mode has saved: its backward is
+    refused, as with stock batch norm."""
+    mlp, _ = pair("cuda")
+    x = torch.rand(2, 6, 33, device="cuda", requires_grad=True)
+    out = mlp(x)
+    with torch.no_grad():
+        mlp.train()(x)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        out.sum().backward()
+
+
+@pytest.mark.gpu
+def test_forward_mode_is_refused_by_operators():
+    from torkit3d_amd.ops.chamfer_distance import chamfer_distance
+    from torkit3d_amd.ops.group_points import group_points
+
+    x = torch.rand(1, 16, 3, device="cuda")
+    with forward_ad.dual_level():
+        dual = forward_ad.make_dual(x, torch.ones_like(x))
+        with pytest.raises(Exception):
+            chamfer_distance(dual, x)
+        with pytest.raises(Exception):
+            group_points(dual, torch.zeros(1, 2, 2, dtype=torch.long, device="cuda"))

@@ -71,7 +71,8 @@ __global__ void __launch_bounds__(kBlock)
                     s2 = __builtin_fmaf(d, d, s2);
                     total_u += r[k];
                     const float s = y * sign;
-                    const bool up = k0 + k == 0 || s > best;
+                    // (the first NaN stays, as in torch's maximum)
+                    const bool up = k0 + k == 0 || (!(s <= best) && best == best);
                     best = up ? s : best;
                     chosen = up ? y : chosen;
                     where = up ? k0 + k : where;

@@ -415,7 +415,8 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
                     for (int i = 0; i < RUN; ++i) {
                         const float s = v[i] * sign[ct];
                         if constexpr (OUT == OUT_POOL) {
-                            const bool up = where < 0 || s > best;
+                            // (the first NaN stays, as in torch's maximum)
+                            const bool up = where < 0 || (!(s <= best) && best == best);
                             if (i == 0)
                                 first_y = where < 0 ? v[0] : first_y;
                             best = up ? s : best;
@@ -430,7 +431,9 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
                         const float other = __shfl_xor(best, 32);
                         if constexpr (OUT == OUT_POOL) {
                             const int at = __shfl_xor(where, 32);
-                            const bool up = other > best || (other == best && at < where);
+                            const bool up = other != other
+                                ? best == best || at < where
+                                : other > best || (other == best && at < where);
                             best = up ? other : best;
                             where = up ? at : where;
                         } else {
@@ -441,7 +444,7 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
                             const int64_t at = ((int64_t)b * p.C + c) * p.M + m;
                             if constexpr (OUT == OUT_POOL) {
                                 // (a zero gamma makes all values equal: the first one's place)
-                                p.out[at] = sign[ct] == 0.0f ? first_y : best * sign[ct];
+                                p.out[at] = sign[ct] == 0.0f && best == best ? first_y : best * sign[ct];
                                 p.arg[at] = (unsigned char)(where - m * p.group);
                             } else {
                                 p.out[at] = relu(sign[ct] == 0.0f

@@ -431,7 +431,13 @@ Tensor interpolate_backward(const Tensor &grad, const Tensor &index, const Tenso
 
 // ---- autograd nodes ------------------------------------------------------------------------------
 
-bool tracked(const Tensor &t) { return t.defined() && t.requires_grad(); }
+// Whether a node has to be made: for gradients, and for a forward-mode tangent, which the nodes
+// refuse (without one it would be dropped in silence).
+template <typename... T> bool tracked(const T &...t)
+{
+    return (c10::GradMode::is_enabled() && ((t.defined() && t.requires_grad()) || ...)) ||
+           ((t.defined() && t._fw_grad(0).defined()) || ...);
+}
 
 // sqrt(max(d, eps)) of both directions.
 std::vector<Tensor> roots(const Tensor &d1, const Tensor &d2, double eps)
@@ -499,7 +505,7 @@ struct ChamferNode : torch::autograd::Function<ChamferNode> {
 std::tuple<Tensor, Tensor> chamfer(const Tensor &xyz1, const Tensor &xyz2, bool channels_first,
                                    bool root, double eps)
 {
-    if (c10::GradMode::is_enabled() && (tracked(xyz1) || tracked(xyz2))) {
+    if (tracked(xyz1, xyz2)) {
         const variable_list out = ChamferNode::apply(xyz1, xyz2, channels_first, root, eps);
         return {out[0], out[1]};
     }
@@ -529,7 +535,7 @@ struct GroupNode : torch::autograd::Function<GroupNode> {
 
 Tensor group_points(const Tensor &points, const Tensor &index)
 {
-    if (c10::GradMode::is_enabled() && tracked(points))
+    if (tracked(points))
         return GroupNode::apply(points, index);
     return group_forward(points, index);
 }
@@ -564,7 +570,7 @@ struct GroupConcatNode : torch::autograd::Function<GroupConcatNode> {
 Tensor group_points_with_xyz(const Tensor &feature, const Tensor &xyz, const Tensor &centre,
                              const Tensor &index)
 {
-    if (c10::GradMode::is_enabled() && (tracked(feature) || tracked(xyz) || tracked(centre)))
+    if (tracked(feature, xyz, centre))
         return GroupConcatNode::apply(
             feature.defined() ? std::optional<Tensor>(feature) : std::nullopt, xyz, centre, index);
     return group_concat_forward(feature.defined() ? feature.contiguous() : feature,
@@ -590,7 +596,7 @@ struct InterpolateNode : torch::autograd::Function<InterpolateNode> {
 
 Tensor interpolate(const Tensor &feature, const Tensor &index, const Tensor &weight)
 {
-    if (c10::GradMode::is_enabled() && (tracked(feature) || tracked(weight)))
+    if (tracked(feature, weight))
         return InterpolateNode::apply(feature, index, weight);
     return interpolate_forward(feature.contiguous(), index.contiguous(), weight.contiguous());
 }

@@ -37,6 +37,12 @@ inline void *stream_of(const Tensor &t)
 // Makes the tensor's GPU the current one (kernels, allocations and streams follow it).
 using OnDeviceOf = c10::OptionalDeviceGuard;
 
+// Whether the tensor is what its pointer and sizes say: no subclass that dispatches in Python, no
+// wrapper of a function transform, no pending conjugation, and no forward-mode tangent.
+bool plain(const Tensor &t);
+// A function transform (torch.func) or a dispatch mode is active: it has to see the operators.
+bool watched();
+
 Tensor mlp(Tensor x, Tensor x2, const Tensor &xyz, const Tensor &centre, const Tensor &index,
            std::vector<Tensor> params, std::vector<Tensor> buffers, std::vector<double> eps,
            std::vector<double> momentum, bool training, int64_t pool);

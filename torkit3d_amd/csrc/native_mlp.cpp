@@ -3,15 +3,53 @@
 #include "native.h"
 #include "tk3d_mlp.h"
 
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <torch/csrc/autograd/autograd.h>
 
 namespace tk3d {
+
+bool plain(const Tensor &t)
+{
+    using c10::DispatchKey;
+    constexpr c10::DispatchKeySet odd({DispatchKey::Python, DispatchKey::PythonTLSSnapshot,
+                                       DispatchKey::FuncTorchBatched,
+                                       DispatchKey::FuncTorchGradWrapper, DispatchKey::Functionalize,
+                                       DispatchKey::Conjugate, DispatchKey::Negative,
+                                       DispatchKey::ZeroTensor});
+    return !t.key_set().has_any(odd) && !t._fw_grad(0).defined();
+}
+
+bool watched()
+{
+    return c10::impl::tls_is_dispatch_key_included(
+               c10::DispatchKey::FuncTorchDynamicLayerFrontMode) ||
+           c10::impl::TorchDispatchModeTLS::any_modes_set();
+}
+
 namespace {
 
 using torch::autograd::AutogradContext;
 using torch::autograd::variable_list;
 
 float *f32(const Tensor &t) { return t.defined() ? t.data_ptr<float>() : nullptr; }
+
+// The statistics kernels write the running statistics: whoever saved them has to see that.
+void written(const Tensor &mean, const Tensor &var, const Tensor &count)
+{
+    for (const Tensor *t : {&mean, &var, &count})
+        if (t->defined())
+            t->unsafeGetTensorImpl()->bump_version();
+}
+
+// Saved tensors come back through hooks, which may lay them out anew.
+variable_list dense(variable_list saved)
+{
+    for (Tensor &t : saved)
+        if (t.defined())
+            t = t.contiguous();
+    return saved;
+}
 
 // What a chain is applied to and how.
 struct Call {
@@ -229,6 +267,7 @@ Tensor forward(const Call &c, Kept &k)
                                          count.defined() ? count.data_ptr<int64_t>() : nullptr,
                                          stream),
                  "tk3d_mlp_statistics_f32");
+            written(c.buffers[3 * l], c.buffers[3 * l + 1], count);
         } else {
             k.mean.push_back(c.buffers[3 * l]);
             k.var.push_back(c.buffers[3 * l + 1]);
@@ -523,7 +562,7 @@ struct Node : torch::autograd::Function<Node> {
 
     static variable_list backward(AutogradContext *ctx, variable_list grads)
     {
-        const variable_list s = ctx->get_saved_variables();
+        const variable_list s = dense(ctx->get_saved_variables());
         Call c;
         Kept k;
         c.x = s[0];
@@ -645,6 +684,7 @@ Tensor edge_forward(const EdgeCall &c, EdgeKept &k, bool keep)
                                      c.batches.defined() ? c.batches.data_ptr<int64_t>() : nullptr,
                                      stream),
              "tk3d_mlp_statistics_f32");
+        written(c.running_mean, c.running_var, c.batches);
     } else {
         k.mean = c.running_mean;
         k.var = c.running_var;
@@ -736,7 +776,7 @@ struct EdgeNode : torch::autograd::Function<EdgeNode> {
 
     static variable_list backward(AutogradContext *ctx, variable_list grads)
     {
-        const variable_list s = ctx->get_saved_variables();
+        const variable_list s = dense(ctx->get_saved_variables());
         EdgeCall c;
         EdgeKept k;
         c.x = s[0];
@@ -776,7 +816,30 @@ struct EdgeNode : torch::autograd::Function<EdgeNode> {
     }
 };
 
-bool usable(const Tensor &t) { return t.is_cuda() && t.scalar_type() == at::kFloat; }
+bool usable(const Tensor &t, const Tensor &like)
+{
+    return t.is_cuda() && t.scalar_type() == at::kFloat && t.layout() == at::kStrided &&
+           t.device() == like.device() && plain(t);
+}
+
+bool usable_index(const Tensor &t, const Tensor &like)
+{
+    return t.scalar_type() == at::kLong && t.layout() == at::kStrided && t.device() == like.device() &&
+           plain(t);
+}
+
+// Weight, gamma and beta, running mean, running variance and batch count of one layer.
+bool usable_layer(const Tensor *params, const Tensor *buffers, const Tensor &like)
+{
+    const int64_t C = params[0].dim() > 1 ? params[0].size(0) : -1;
+    for (int i = 0; i < 3; ++i)
+        if (!usable(params[i], like) || !params[i].is_contiguous() || (i && params[i].numel() != C))
+            return false;
+    for (int i = 0; i < 2; ++i)
+        if (!usable(buffers[i], like) || !buffers[i].is_contiguous() || buffers[i].numel() != C)
+            return false;
+    return !buffers[2].defined() || (usable_index(buffers[2], like) && buffers[2].numel() == 1);
+}
 
 }  // namespace
 
@@ -790,14 +853,13 @@ Tensor mlp(Tensor x, Tensor x2, const Tensor &xyz, const Tensor &centre, const T
     const int64_t L = (int64_t)params.size() / 3;
     // (Pooled forms: groups of 32 or 64, which fill whole tiles of every shape; other groups take
     // the dense chain and a maximum behind it.)
-    if (L == 0 || (pool && (L < 2 || (pool != 32 && pool != 64))))
+    if (L == 0 || (pool && (L < 2 || (pool != 32 && pool != 64))) || watched())
         return Tensor();
     const bool grouped = xyz.defined();
     std::vector<int64_t> shape;
     if (grouped) {
-        if (L < 2 || !pool || !usable(xyz) || !usable(centre) || !index.is_cuda() || xyz.dim() != 3 ||
-            centre.dim() != 3 || index.dim() != 3 || index.scalar_type() != at::kLong ||
-            index.size(2) != pool || centre.size(2) != index.size(1) || xyz.size(1) != 3 ||
+        if (L < 2 || !pool || !usable(xyz, xyz) || !usable(centre, xyz) || !usable_index(index, xyz) ||
+            xyz.dim() != 3 || centre.dim() != 3 || index.dim() != 3 || index.size(2) != pool || centre.size(2) != index.size(1) || xyz.size(1) != 3 ||
             centre.size(1) != 3 || index.size(0) != xyz.size(0) || centre.size(0) != xyz.size(0))
             return Tensor();
         c.xyz = xyz.contiguous();
@@ -814,19 +876,16 @@ Tensor mlp(Tensor x, Tensor x2, const Tensor &xyz, const Tensor &centre, const T
         shape = x.sizes().vec();
     }
     const bool has_x = x.defined(), has_x2 = x2.defined();
-    if ((has_x && !usable(x)) || (has_x2 && !usable(x2)))
+    const Tensor &first = grouped ? xyz : x;
+    if ((has_x && !usable(x, first)) || (has_x2 && !usable(x2, first)))
         return Tensor();
     int64_t channels = (has_x ? x.size(1) : 0) + (has_x2 ? x2.size(1) : 0) + (grouped ? 3 : 0);
     bool tracked = (has_x && x.requires_grad()) || (has_x2 && x2.requires_grad());
     for (int64_t l = 0; l < L; ++l) {
-        for (int i = 0; i < 3; ++i) {
-            if (!usable(params[3 * l + i]) || !params[3 * l + i].is_contiguous())
-                return Tensor();
-            tracked = tracked || params[3 * l + i].requires_grad();
-        }
-        if (!usable(buffers[3 * l]) || !usable(buffers[3 * l + 1]) ||
-            !buffers[3 * l].is_contiguous() || !buffers[3 * l + 1].is_contiguous())
+        if (!usable_layer(&params[3 * l], &buffers[3 * l], first))
             return Tensor();
+        for (int i = 0; i < 3; ++i)
+            tracked = tracked || params[3 * l + i].requires_grad();
         if (params[3 * l].size(1) != channels)
             return Tensor();
         channels = params[3 * l].size(0);
@@ -874,7 +933,7 @@ Tensor mlp(Tensor x, Tensor x2, const Tensor &xyz, const Tensor &centre, const T
 // not take its size.
 Tensor edge_lists(const Tensor &index_, int64_t n)
 {
-    if (!index_.is_cuda() || index_.dim() != 3 || index_.scalar_type() != at::kLong ||
+    if (!index_.is_cuda() || !usable_index(index_, index_) || index_.dim() != 3 || watched() ||
         index_.size(1) != n || !tk3d_mlp_edge_supported(index_.size(0), n, index_.size(2), 1))
         return Tensor();
     const Tensor index = index_.contiguous();
@@ -893,16 +952,10 @@ Tensor edge_conv(const Tensor &x, const Tensor &index, const Tensor &lists,
                  const std::vector<Tensor> &params, const std::vector<Tensor> &buffers, double eps,
                  double momentum, bool training)
 {
-    if (!usable(x) || x.dim() != 3 || !index.is_cuda() || index.dim() != 3 ||
-        index.scalar_type() != at::kLong || index.size(0) != x.size(0) ||
-        index.size(1) != x.size(2) || params.size() != 3)
+    if (!usable(x, x) || x.dim() != 3 || !usable_index(index, x) || index.dim() != 3 ||
+        index.size(0) != x.size(0) || index.size(1) != x.size(2) || params.size() != 3 || watched() ||
+        !usable_layer(params.data(), buffers.data(), x))
         return Tensor();
-    for (const Tensor &t : params)
-        if (!usable(t) || !t.is_contiguous())
-            return Tensor();
-    for (int i = 0; i < 2; ++i)
-        if (!usable(buffers[i]) || !buffers[i].is_contiguous())
-            return Tensor();
     const int64_t B = x.size(0), C = x.size(1), N = x.size(2), K = index.size(2);
     const int64_t O = params[0].size(0);
     if (params[0].size(1) != 2 * C || !tk3d_mlp_edge_supported(B, N, K, O) || B * N * K < 2 ||

@@ -15,7 +15,8 @@ Differences from the reference, none of which change the result:
 import torch
 from torch import nn
 
-from ..nn import mlp1d_bn_relu, mlp2d_bn_relu
+from ..nn import (forward_cat, forward_grouped_max, forward_max, mlp1d_bn_relu,
+                  mlp2d_bn_relu)
 from ..ops.ball_query import ball_query
 from ..ops.group_points import group_points, group_points_with_xyz
 from ..ops.interpolate_feature import interpolate_feature, three_nn_interpolation
@@ -40,7 +41,7 @@ class SetAbstraction(nn.Module):
         with torch.no_grad():
             nbr_index = self.query_neighbor(out_xyz, in_xyz)  # [B, N2, K]
         if self.use_xyz:
-            out_feature = self.mlp.forward_grouped_max(in_feature, in_xyz, out_xyz, nbr_index)
+            out_feature = forward_grouped_max(self.mlp, in_feature, in_xyz, out_xyz, nbr_index)
             if out_feature is not None:
                 return out_feature
             nbr_feature = group_points_with_xyz(in_feature, in_xyz, out_xyz, nbr_index)
@@ -49,7 +50,7 @@ class SetAbstraction(nn.Module):
         else:
             nbr_feature = in_xyz.new_empty(
                 [in_xyz.size(0), 0, nbr_index.size(1), nbr_index.size(2)])
-        return self.mlp.forward_max(nbr_feature)
+        return forward_max(self.mlp, nbr_feature)
 
     def extra_repr(self):
         return "use_xyz={}".format(self.use_xyz)
@@ -108,5 +109,5 @@ class FeaturePropagation(nn.Module):
     def forward(self, in_xyz, in_feature, out_xyz, out_feature=None):
         interp_feature = self.interpolator(out_xyz, in_xyz, in_feature)
         if out_feature is not None:
-            return self.mlp.forward_cat(interp_feature, out_feature)
+            return forward_cat(self.mlp, interp_feature, out_feature)
         return self.mlp(interp_feature)

@@ -80,9 +80,14 @@ class SharedMLP(nn.Sequential):
 
     fused_training = True  # whether training mode takes the fused kernels too
 
-    def forward(self, x):
-        out = self._chain(x)
-        return super().forward(x) if out is None else out
+    def forward(self, input):
+        if not torch.jit.is_scripting():
+            out = self._chain(input)
+            if out is not None:
+                return out
+        for module in self:
+            input = module(input)
+        return input
 
     def forward_cat(self, x, x2):
         """``self(torch.cat([x, x2], dim=1))`` without the concatenation."""
@@ -119,11 +124,10 @@ class SharedMLP(nn.Sequential):
 
     def _plan(self, like):
         """(parameters, buffers, eps, momentum, training) of plain layers, or None."""
-        if (not like.is_cuda or like.dtype != torch.float32 or torch.is_autocast_enabled()
+        if (type(like) not in _TENSORS  # (a tracer's proxy, a subclass)
+                or not like.is_cuda or like.dtype != torch.float32 or torch.is_autocast_enabled()
                 or torch.compiler.is_compiling() or torch.jit.is_tracing()
-                or _has_any_global_hook() or type(self) is not SharedMLP
-                or self._forward_hooks or self._forward_pre_hooks
-                or self._backward_hooks or self._backward_pre_hooks):
+                or _has_any_global_hook() or type(self) is not SharedMLP or not _plain(self)):
             return None
         params, buffers, eps, momentum = [], [], [], []
         training = None
@@ -136,15 +140,19 @@ class SharedMLP(nn.Sequential):
                     or type(relu) is not nn.ReLU or not _plain(relu)
                     or conv.groups != 1 or conv.padding != block.no_padding
                     or conv.kernel_size != block.ones or conv.stride != block.ones
-                    or conv._parameters["bias"] is not None or bn.momentum is None):
+                    or conv._parameters.get("bias") is not None or bn.momentum is None):
                 return None
             if training is None:
                 training = bn.training
                 if training and not self.fused_training:
                     return None
-            weight, gamma, beta = conv._parameters["weight"], *bn._parameters.values()
-            mean, var, count = bn._buffers.values()
-            if training != bn.training or gamma is None or beta is None or mean is None:
+            # (a replica of DataParallel holds its tensors as attributes: get() finds none)
+            weight = conv._parameters.get("weight")
+            gamma, beta = (bn._parameters.get(name) for name in ("weight", "bias"))
+            mean, var, count = (bn._buffers.get(name) for name in
+                                ("running_mean", "running_var", "num_batches_tracked"))
+            if (training != bn.training or weight is None or gamma is None or beta is None
+                    or mean is None or var is None):
                 return None
             params += (weight, gamma, beta)
             buffers += (mean, var, count)
@@ -153,9 +161,39 @@ class SharedMLP(nn.Sequential):
         return params, buffers, eps, momentum, bool(training)
 
 
+_TENSORS = (torch.Tensor, nn.Parameter)
+
+
 def _plain(module):
     return not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks
-                or module._backward_pre_hooks)
+                or module._backward_pre_hooks or "forward" in module.__dict__)
+
+
+# The forms of a shared MLP that layers call. A layer's MLP may also be a plain nn.Sequential: put
+# there by hand, or from a model that was pickled as a whole before SharedMLP was there.
+
+def forward_cat(mlp, x, x2):
+    if isinstance(mlp, SharedMLP):
+        return mlp.forward_cat(x, x2)
+    return mlp(torch.cat([x, x2], dim=1))
+
+
+def forward_max(mlp, x):
+    if isinstance(mlp, SharedMLP):
+        return mlp.forward_max(x)
+    return torch.max(mlp(x), dim=3)[0]
+
+
+def forward_grouped_max(mlp, feature, xyz, centre, index):
+    if isinstance(mlp, SharedMLP):
+        return mlp.forward_grouped_max(feature, xyz, centre, index)
+    return None
+
+
+def forward_edges_max(mlp, x, index, lists=None):
+    if isinstance(mlp, SharedMLP):
+        return mlp.forward_edges_max(x, index, lists)
+    return None
 
 
 def _mlp(block, in_channels, out_channels_list):

@@ -3,7 +3,7 @@ import torch
 import torch.utils.checkpoint
 
 from .. import _native
-from ..nn import mlp2d_bn_relu
+from ..nn import forward_edges_max, forward_max, mlp2d_bn_relu
 from .group_points import group_points
 
 
@@ -71,7 +71,7 @@ class EdgeConvBlock(torch.nn.Module):
         ``lists`` (not in the reference) is the inverse of the graph (``edge_lists``), for
         callers that run several blocks on one graph; without it every block works it out."""
         if query_feature is key_feature and not self.checkpoint:
-            output = self.convs.forward_edges_max(query_feature, key_ind, lists)
+            output = forward_edges_max(self.convs, query_feature, key_ind, lists)
             if output is not None:
                 return output
         edge_feature = get_edge_feature(query_feature, key_feature, key_ind)
@@ -79,4 +79,4 @@ class EdgeConvBlock(torch.nn.Module):
             edge_feature = torch.utils.checkpoint.checkpoint(self.convs, edge_feature,
                                                              use_reentrant=False)
             return edge_feature.max(dim=3)[0]
-        return self.convs.forward_max(edge_feature)
+        return forward_max(self.convs, edge_feature)
