@@ -33,7 +33,7 @@ extern "C" {
 
 typedef struct {
     const float *mean, *var, *gamma, *beta; /* [C] each */
-    float eps;
+    float eps; /* negative: var holds 1 / sqrt(variance + eps) itself */
 } tk3d_mlp_norm;
 
 typedef struct {
@@ -54,11 +54,10 @@ enum {
     TK3D_MLP_IN_GRAD = 3,     /* a x + b y + d */
     TK3D_MLP_IN_GRAD_OUT = 4, /* the same with x masked by relu(in_norm(y)) first */
     TK3D_MLP_IN_POOL = 5,     /* the sparse src[0].sel, then relu(in_norm(src[1].x)) */
-    TK3D_MLP_OUT_STATS = 0,     /* out, and partial sums of it and of its square */
     TK3D_MLP_OUT_PLAIN = 1,     /* out + bias, channels from C0 on in out2; either may be NULL */
     TK3D_MLP_OUT_POINTS = 2,    /* out as [B, P, C] */
     TK3D_MLP_OUT_EVAL = 3,      /* relu(out_norm(out)) */
-    TK3D_MLP_OUT_POOL = 4,      /* extreme over groups (out [B,C,M]), place (arg), partial sums */
+    TK3D_MLP_OUT_POOL = 4,      /* extreme over groups (out [B,C,M]) and place (arg) */
     TK3D_MLP_OUT_POOL_EVAL = 5, /* relu(out_norm(extreme over groups)) */
     TK3D_MLP_OUT_MASK = 6       /* e = (out + bias) where relu(out_norm(yprev)) passes, and partial
                                    sums of e and e (yprev - mean) */
@@ -71,7 +70,7 @@ typedef struct {
     const float *yprev; /* [B, C, P] */
     const float *bias;  /* [C] or NULL */
     unsigned char *arg; /* [B, C, M] */
-    void *partial;      /* doubles [C][slots][2]; tk3d_mlp_product_slots gives slots */
+    void *partial;      /* OUT_MASK: doubles [C][slots][2]; tk3d_mlp_product_slots gives slots */
     int32_t B, C, C0, P;
     int32_t group, M;   /* pooled forms: P == group * M, group 32 or 64 */
 } tk3d_mlp_product;
@@ -112,12 +111,10 @@ typedef struct {
 } tk3d_mlp_sum;
 int tk3d_mlp_sum_f32(const tk3d_mlp_sum *sums, int n, void *stream);
 
-/* Batch statistics of `n` values per channel from the partial sums: mean and (biased) variance,
- * running statistics updated with `momentum` (unbiased variance) and *batches incremented where
- * given (NULL otherwise). */
-int tk3d_mlp_statistics_f32(const void *partial, int slots, int64_t n, int C, float momentum,
-                            float *mean, float *var, float *running_mean, float *running_var,
-                            int64_t *batches, void *stream);
+/* A normalised layer's ReLU and maximum over groups of `size` <= 255 consecutive values: out =
+ * relu(max z), arg the place of the maximum and extreme the y at that place, [groups] each. */
+int tk3d_mlp_pool_max_f32(const float *z, const float *y, int64_t groups, int size, float *out,
+                          float *extreme, unsigned char *arg, void *stream);
 
 /* (a, b, d) per channel from the partial sums of (e, e (y - mean)), and dgamma, dbeta.
  * frozen: the statistics are constants (evaluation mode), b = d = 0. */
@@ -154,27 +151,27 @@ int tk3d_mlp_pool_weight_grad_f32(const float *sparse, int sparse_splits, const 
 
 /* First layer behind a grouping: y[b,c,m,s] = u[b,j,c] + sum_a wx[c][a] (xyz[b,a,j] -
  * centre[b,a,m]), j = index[b,m,s] (an index outside [0,N) reads as zeros). u [B,N,C] (the product
- * of the features with their weights, or NULL), wx rows ldw apart. rel (NULL or [B,3,M*S]) gets
- * the centred coordinates. Partial sums as TK3D_MLP_OUT_STATS. */
-int tk3d_mlp_group_slots(int B, int C, int M, int S);
+ * of the features with their weights, or NULL), wx rows ldw apart. */
 int tk3d_mlp_group_f32(const float *u, const float *xyz, const float *centre, const int64_t *index,
                        const float *wx, int ldw, int B, int C, int N, int M, int S, float *y,
-                       float *rel, void *partial, void *stream);
+                       void *stream);
 
 /* EdgeConv (torkit3d/ops/edge_conv.py) with one layer, on a graph of a cloud with itself, pooled
  * over the K neighbours: y(i, k) = W1 (x_j - x_i) + W2 x_i = u_j + v_i, j = index[b, i, k] (x_j = 0
  * for an index outside [0,N)), where w = [W1 W2], u = W1 x and v = (W2 - W1) x; uv [B, N, 2 O] is
  * the product of x with the [2 O][C] matrix that tk3d_mlp_edge_weights_f32 makes of w. Forward:
- * extreme and arg [B, O, N] as in pooled layers (arg may be NULL), sum [B, N, O] of the u of a
- * point's neighbours (or NULL), partial sums. Backward: lists is the inverse of the graph
+ * extreme and arg [B, O, N] as in pooled layers (either may be NULL), sum [B, N, O] of the u of a
+ * point's neighbours (or NULL). tk3d_mlp_edge_features_f32 makes the edge features themselves,
+ * [B, 2 C, N, K]. Backward: lists is the inverse of the graph
  * (int32 [B][N + 1 + N K]), sel a buffer of B N O 8-byte elements, duv [B, 2 O, N] the gradients
  * of u and v. tk3d_mlp_edge_supported: the sizes these take (N <= 32768, K <= 255). */
 int tk3d_mlp_edge_supported(int64_t B, int64_t N, int64_t K, int64_t O);
 int tk3d_mlp_edge_weights_f32(const float *w, int O, int C, float *out, void *stream);
-int tk3d_mlp_edge_slots(int B, int N);
+int tk3d_mlp_edge_features_f32(const float *x, const int64_t *index, int B, int C, int N, int K,
+                               float *out, void *stream);
 int tk3d_mlp_edge_forward_f32(const float *uv, const int64_t *index, const float *gamma, int B, int N,
                               int K, int O, float *extreme, unsigned char *arg, float *sum,
-                              void *partial, void *stream);
+                              void *stream);
 int tk3d_mlp_edge_lists(const int64_t *index, int B, int N, int K, int32_t *lists, void *stream);
 int tk3d_mlp_edge_backward_f32(const float *g, const float *extreme, const unsigned char *arg,
                                const float *uv, const float *sum, const int32_t *lists, int B, int N,

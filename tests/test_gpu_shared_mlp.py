@@ -129,6 +129,38 @@ def test_grouped(cuda, monkeypatch, features, tracked, n, m, s, training):
     check(mlp, fused, reference, inputs, monkeypatch)
 
 
+# In training mode the activations and statistics are the stock modules' own, bit by bit, and so are
+# the signs the backward takes: gradients differ by sums in another order alone, 1.5e-6 over 40
+# steps of whole networks (four times that is the bound), where a single sign gave 1e-2.
+@pytest.mark.parametrize("b,p,widths,pool", [(3, 1000, (6, 64, 33), 0), (2, 512, (67, 64, 128), 32),
+                                             (1, 130, (20, 128, 40), 64), (2, 4096, (9, 32, 32), 0)])
+def test_training_is_that_of_the_stock_modules(cuda, b, p, widths, pool):
+    mlp = make(mlp2d_bn_relu if pool else mlp1d_bn_relu, widths[0], widths[1:], True, cuda)
+    plain = stock(mlp, torch.float32)
+    x = randn(p, b, widths[0], p, *([pool] if pool else []))
+    results = []
+    for module in (mlp, plain):
+        leaf = x.clone().requires_grad_()
+        if pool:
+            out = mlp.forward_max(leaf) if module is mlp else module(leaf).max(dim=3)[0]
+        else:
+            out = module(leaf)
+        grads = torch.autograd.grad(out, [leaf, *module.parameters()], torch.sin(out.detach() * 50))
+        results.append((out.detach(), [t.clone() for t in module.buffers()], grads))
+    assert torch.equal(results[0][0], results[1][0])
+    assert all(torch.equal(a, c) for a, c in zip(results[0][1], results[1][1]))
+    for a, c in zip(results[0][2], results[1][2]):
+        assert float((a - c).norm()) <= 6e-6 * float(c.norm())
+
+
+@pytest.mark.parametrize("p", [514, 1030])
+def test_rows_on_which_the_library_differs_run_in_stock(cuda, p):
+    mlp = make(mlp1d_bn_relu, 6, (8, 5), True, cuda)
+    out = mlp(randn(1, 2, 6, p).requires_grad_())
+    assert "Relu" in out.grad_fn.name()
+    assert "Node" in mlp(randn(1, 2, 6, p + 2).requires_grad_()).grad_fn.name()
+
+
 def test_gradient_of_a_gradient(cuda):
     mlp = make(mlp1d_bn_relu, 6, (8, 5), True, cuda)
     results = []

@@ -30,17 +30,14 @@ __global__ void __launch_bounds__(kBlock)
     edge_forward_kernel(const float *__restrict__ uv, const int64_t *__restrict__ index,
                         const float *__restrict__ gamma, int B, int N, int K, int O, int total,
                         float *__restrict__ extreme, unsigned char *__restrict__ arg,
-                        float *__restrict__ sum, double2 *__restrict__ partial, int slots)
+                        float *__restrict__ sum)
 {
     __shared__ float values[kChannels][kPoints + 1];
     __shared__ unsigned char places[kChannels][kPoints];
-    __shared__ double2 sums[kWaves][kChannels];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int cbase = blockIdx.y * kChannels;
     const int c = cbase + lane < O ? cbase + lane : O - 1;
     const float sign = sign_of(gamma[c]);
-    float shift = 0.0f, s1 = 0.0f, s2 = 0.0f;
-    double n = 0.0;
     for (int tile = blockIdx.x; tile < total; tile += gridDim.x) {
         const int b = tile % B, first = tile / B * kPoints;
         const float *u = uv + (int64_t)b * N * 2 * O + c;
@@ -64,11 +61,6 @@ __global__ void __launch_bounds__(kBlock)
                     if (k0 + k >= K)
                         break;
                     const float y = r[k] + v;
-                    if (n == 0.0 && k0 + k == 0)
-                        shift = y;
-                    const float d = y - shift;
-                    s1 += d;
-                    s2 = __builtin_fmaf(d, d, s2);
                     total_u += r[k];
                     const float s = y * sign;
                     // (the first NaN stays, as in torch's maximum)
@@ -78,12 +70,13 @@ __global__ void __launch_bounds__(kBlock)
                     where = up ? k0 + k : where;
                 }
             }
-            n += K;
             values[lane][local] = chosen;
             places[lane][local] = (unsigned char)where;
             if (sum && cbase + lane < O)
                 sum[((int64_t)b * N + i) * O + c] = total_u;
         }
+        if (!extreme)
+            continue;
         __syncthreads();
         for (int e = tid; e < kChannels * kPoints; e += kBlock) {
             const int ch = e / kPoints, p = e % kPoints;
@@ -96,16 +89,46 @@ __global__ void __launch_bounds__(kBlock)
         }
         __syncthreads();
     }
-    const double sh = n > 0.0 ? (double)shift : 0.0;
-    sums[wave][lane] = double2{s1 + n * sh, s2 + 2.0 * sh * s1 + n * sh * sh};
-    __syncthreads();
-    if (tid < kChannels && cbase + tid < O) {
-        double2 s = sums[0][tid];
-        for (int w = 1; w < kWaves; ++w) {
-            s.x += sums[w][tid].x;
-            s.y += sums[w][tid].y;
+}
+
+// The edge features themselves, [x_j - x_i, x_i] as [B, 2 C, N, K] (x_j = 0 for an index outside):
+// written once, where group, difference and concatenation were three passes over them and more.
+// A thread has four consecutive edges (one where their number is odd) of kEdgeChannels channels.
+constexpr int kEdgeChannels = 8;
+
+template <int RUN>
+__global__ void __launch_bounds__(kBlock)
+    edge_features_kernel(const float *__restrict__ x, const int64_t *__restrict__ index, int C, int N,
+                         int K, float *__restrict__ out)
+{
+    const int b = blockIdx.z, edges = N * K;
+    const int cbase = blockIdx.y * kEdgeChannels;
+    const int e = (blockIdx.x * kBlock + threadIdx.x) * RUN;
+    if (e >= edges)
+        return;
+    int i[RUN], j[RUN];
+#pragma unroll
+    for (int r = 0; r < RUN; ++r) {
+        const int64_t at = index[(int64_t)b * edges + e + r];
+        i[r] = (e + r) / K;
+        j[r] = at >= 0 && at < N ? (int)at : -1;
+    }
+    float *diff = out + (int64_t)b * 2 * C * edges + e, *own = diff + (int64_t)C * edges;
+    const float *row = x + (int64_t)b * C * N;
+    for (int c = cbase; c < C && c < cbase + kEdgeChannels; ++c) {
+        float d[RUN], q[RUN];
+#pragma unroll
+        for (int r = 0; r < RUN; ++r) {
+            q[r] = row[(int64_t)c * N + i[r]];
+            d[r] = (j[r] >= 0 ? row[(int64_t)c * N + j[r]] : 0.0f) - q[r];
         }
-        partial[(int64_t)(cbase + tid) * slots + blockIdx.x] = s;
+        if constexpr (RUN == 4) {
+            *reinterpret_cast<f32x4 *>(diff + (int64_t)c * edges) = f32x4{d[0], d[1], d[2], d[3]};
+            *reinterpret_cast<f32x4 *>(own + (int64_t)c * edges) = f32x4{q[0], q[1], q[2], q[3]};
+        } else {
+            diff[(int64_t)c * edges] = d[0];
+            own[(int64_t)c * edges] = q[0];
+        }
     }
 }
 
@@ -176,8 +199,8 @@ __global__ void __launch_bounds__(kBlock)
         const int ch = e / kPoints, p = e % kPoints, c = cbase + ch;
         if (c < O && first + p < N) {
             const int64_t at = ((int64_t)b * O + c) * N + first + p;
-            const f32x2 ss = scale_shift(norm, c);
-            const float ev = passes(__builtin_fmaf(extreme[at], ss.x, ss.y)) ? g[at] : 0.0f;
+            const f32x4 ss = constants_of(norm, c);
+            const float ev = passes(normalised(extreme[at], ss)) ? g[at] : 0.0f;
             tile[p][ch] = int2{__float_as_int(coef[c * 4] * ev), (int)arg[at]};
         }
     }
@@ -267,23 +290,31 @@ int tk3d_mlp_edge_weights_f32(const float *w, int O, int C, float *out, void *st
     return tk_launch_status();
 }
 
-int tk3d_mlp_edge_slots(int B, int N)
+int tk3d_mlp_edge_features_f32(const float *x, const int64_t *index, int B, int C, int N, int K,
+                               float *out, void *stream)
 {
-    const int64_t tiles = (int64_t)B * ((N + kPoints - 1) / kPoints);
-    const int64_t most = 4 * tk_cu_count() / B * B;  // (whole rounds of the batch)
-    return (int)(tiles < most || most == 0 ? tiles : most);
+    if (!tk3d_mlp_edge_supported(B, N, K, 1) || C <= 0 || C > 4096)
+        return TK3D_ERR_UNSUPPORTED;
+    const int edges = N * K, run = edges % 4 == 0 ? 4 : 1;
+    const dim3 grid((edges / run + kBlock - 1) / kBlock, (C + kEdgeChannels - 1) / kEdgeChannels, B);
+    if (run == 4)
+        edge_features_kernel<4><<<grid, kBlock, 0, (hipStream_t)stream>>>(x, index, C, N, K, out);
+    else
+        edge_features_kernel<1><<<grid, kBlock, 0, (hipStream_t)stream>>>(x, index, C, N, K, out);
+    return tk_launch_status();
 }
 
 int tk3d_mlp_edge_forward_f32(const float *uv, const int64_t *index, const float *gamma, int B, int N,
                               int K, int O, float *extreme, unsigned char *arg, float *sum,
-                              void *partial, void *stream)
+                              void *stream)
 {
     if (!tk3d_mlp_edge_supported(B, N, K, O))
         return TK3D_ERR_UNSUPPORTED;
-    const int slots = tk3d_mlp_edge_slots(B, N);
-    edge_forward_kernel<<<dim3(slots, (O + kChannels - 1) / kChannels), kBlock, 0, (hipStream_t)stream>>>(
-        uv, index, gamma, B, N, K, O, B * ((N + kPoints - 1) / kPoints), extreme, arg, sum,
-        reinterpret_cast<double2 *>(partial), slots);
+    const int tiles = B * ((N + kPoints - 1) / kPoints);
+    const int most = 4 * tk_cu_count() / B * B;  // (whole rounds of the batch)
+    const int blocks = tiles < most || most == 0 ? tiles : most;
+    edge_forward_kernel<<<dim3(blocks, (O + kChannels - 1) / kChannels), kBlock, 0, (hipStream_t)stream>>>(
+        uv, index, gamma, B, N, K, O, tiles, extreme, arg, sum);
     return tk_launch_status();
 }
 

@@ -4,8 +4,8 @@
 //
 // What bounds it: an activation is read and written once per layer and direction, everything
 // else is what can be fused into those passes. A layer's product reads the PREVIOUS layer's
-// product and normalises it on the way into the matrix cores, adds up the statistics of its own
-// result on the way out, and a last layer under a maximum writes the maximum only. Narrow layers
+// product and normalises it on the way into the matrix cores, a gradient is masked and its sums are
+// taken on the way out, and a last layer under a maximum writes the maximum only. Narrow layers
 // (up to 64 channels) are bound by HBM, wide ones by the fp32 matrix rate (157 TFLOP/s), which is
 // why the products are fp32 v_mfma_f32_32x32x2 and nothing is rounded to a shorter type.
 #include "mlp_common.h"
@@ -36,11 +36,10 @@ enum Input {      // in(k, p)
     IN_POOL,      // sparse gradient of a maximum, then relu(norm(x)) (see pooled layers below)
 };
 enum Output {
-    OUT_STATS,      // store, and sums of the stored values and their squares per channel
     OUT_PLAIN,      // store, in two tensors if asked for
     OUT_POINTS,     // store as [B, P, C]
     OUT_EVAL,       // store relu(norm(out))
-    OUT_POOL,       // store the extreme over each group and where it is, with the sums
+    OUT_POOL,       // store the extreme over each group and where it is
     OUT_POOL_EVAL,  // store relu(norm(extreme over each group))
     OUT_MASK,       // store out masked by the ReLU in front of it, with the sums of its gradient
 };
@@ -99,15 +98,15 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
 
     // LDS: normalisation of the input channels, then the weights.
     f32x4 *grad_coef = reinterpret_cast<f32x4 *>(lds);              // [K] (a, b, d, -)
-    f32x2 *act_coef = reinterpret_cast<f32x2 *>(lds);               // [K] (scale, shift)
+    f32x4 *act_coef = reinterpret_cast<f32x4 *>(lds);               // [K] of the norm
     if constexpr (IN == IN_GRAD_OUT)
-        act_coef = reinterpret_cast<f32x2 *>(lds + (size_t)a.kg * 8 * sizeof(f32x4));
+        act_coef = grad_coef + (size_t)a.kg * 8;
     float *weights = reinterpret_cast<float *>(lds + a.coef_bytes);  // [CT][chunk][64][4]
 
     if constexpr (IN == IN_ACT || IN == IN_POOL || IN == IN_GRAD_OUT) {
         const int K = IN == IN_POOL ? p.src[1].K : p.src[0].K;
         for (int k = tid; k < ((K + 7) & ~7); k += kBlock)
-            act_coef[k] = k < K ? scale_shift(p.in_norm, k) : f32x2{0.0f, 0.0f};
+            act_coef[k] = k < K ? constants_of(p.in_norm, k) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     }
     if constexpr (reads_y(IN)) {
         const f32x4 *coef = reinterpret_cast<const f32x4 *>(p.src[0].coef);
@@ -213,7 +212,7 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
             for (int q = 0; q < 4; ++q) {
                 if constexpr (reads_y(IN)) {
                     const f32x4 c = grad_coef[k0 + 2 * q];
-                    f32x2 ss{0.0f, 0.0f};
+                    f32x4 ss{0.0f, 0.0f, 0.0f, 0.0f};
                     if constexpr (IN == IN_GRAD_OUT)
                         ss = act_coef[k0 + 2 * q];
 #pragma unroll
@@ -221,14 +220,14 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
                         float e = r.x[d][q][t];
                         const float y = r.y[reads_y(IN) ? d : 0][q][t];
                         if constexpr (IN == IN_GRAD_OUT)
-                            e = passes(__builtin_fmaf(y, ss.x, ss.y)) ? e : 0.0f;
+                            e = passes(normalised(y, ss)) ? e : 0.0f;
                         v[q][t] = __builtin_fmaf(c.x, e, __builtin_fmaf(c.y, y, c.z));
                     }
                 } else if constexpr (IN == IN_ACT || IN == IN_POOL) {
-                    const f32x2 c = act_coef[k0 + 2 * q];
+                    const f32x4 c = act_coef[k0 + 2 * q];
 #pragma unroll
                     for (int t = 0; t < PT; ++t)
-                        v[q][t] = relu(__builtin_fmaf(r.x[d][q][t], c.x, c.y));
+                        v[q][t] = relu(normalised(r.x[d][q][t], c));
                 } else {
 #pragma unroll
                     for (int t = 0; t < PT; ++t)
@@ -265,20 +264,17 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
     };
 
     // Per-lane constants and sums of the output channels (lane = channel).
-    constexpr bool kSums = OUT == OUT_STATS || OUT == OUT_POOL || OUT == OUT_MASK;
     int chan[CT];
     float shift[CT], sum1[CT], sum2[CT];
-    f32x2 out_coef[CT];
+    f32x4 out_coef[CT];
     float sign[CT], bias[CT];
-    int count = 0;
-    bool fresh = true;
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct) {
         chan[ct] = cbase + ct * 32 + col;
         const int c = chan[ct] < p.C ? chan[ct] : p.C - 1;
         sum1[ct] = sum2[ct] = shift[ct] = 0.0f;
         if constexpr (OUT == OUT_EVAL || OUT == OUT_POOL_EVAL || OUT == OUT_MASK)
-            out_coef[ct] = scale_shift(p.out_norm, c);
+            out_coef[ct] = constants_of(p.out_norm, c);
         if constexpr (OUT == OUT_POOL || OUT == OUT_POOL_EVAL) {
             sign[ct] = sign_of(p.out_norm.gamma[c]);
         }
@@ -296,20 +292,12 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
         const bool full = base + 32 * PT <= P;
         const bool vec = (P & 3) == 0;
         constexpr int RUN = 4 * PT;
-        if constexpr (OUT == OUT_STATS || OUT == OUT_POOL) {
-            if (fresh) {  // the sums are taken around a value of the channel itself
-#pragma unroll
-                for (int ct = 0; ct < CT; ++ct)
-                    shift[ct] = acc[0][ct][0];
-                fresh = false;
-            }
-        }
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) {
             const int c = chan[ct];
             const bool mine = c < p.C;
             float *row = nullptr;
-            if constexpr (OUT == OUT_STATS || OUT == OUT_PLAIN || OUT == OUT_EVAL || OUT == OUT_MASK) {
+            if constexpr (OUT == OUT_PLAIN || OUT == OUT_EVAL || OUT == OUT_MASK) {
                 const bool first = c < p.C0;
                 float *out = first ? p.out : p.out2;
                 const int rows = first ? p.C0 : p.C - p.C0, r = first ? c : c - p.C0;
@@ -351,44 +339,24 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
 #pragma unroll
                     for (int i = 0; i < RUN; ++i) {
                         const float y = before[OUT == OUT_MASK ? i : 0];
-                        v[i] = passes(__builtin_fmaf(y, out_coef[ct].x, out_coef[ct].y)) ? v[i] : 0.0f;
+                        v[i] = passes(normalised(y, out_coef[ct])) ? v[i] : 0.0f;
                     }
                 }
-                if constexpr (kSums) {
-                    if (full) {
+                if constexpr (OUT == OUT_MASK) {
 #pragma unroll
-                        for (int i = 0; i < RUN; ++i) {
-                            if constexpr (OUT == OUT_MASK) {
-                                sum1[ct] += v[i];
-                                sum2[ct] = __builtin_fmaf(v[i], before[OUT == OUT_MASK ? i : 0] - shift[ct], sum2[ct]);
-                            } else {
-                                const float d = v[i] - shift[ct];
-                                sum1[ct] += d;
-                                sum2[ct] = __builtin_fmaf(d, d, sum2[ct]);
-                            }
-                        }
-                    } else {
-#pragma unroll
-                        for (int i = 0; i < RUN; ++i) {
-                            if (pos + i < P) {
-                                if constexpr (OUT == OUT_MASK) {
-                                    sum1[ct] += v[i];
-                                    sum2[ct] = __builtin_fmaf(v[i], before[OUT == OUT_MASK ? i : 0] - shift[ct], sum2[ct]);
-                                } else {
-                                    const float d = v[i] - shift[ct];
-                                    sum1[ct] += d;
-                                    sum2[ct] = __builtin_fmaf(d, d, sum2[ct]);
-                                }
-                            }
+                    for (int i = 0; i < RUN; ++i) {
+                        if (full || pos + i < P) {
+                            sum1[ct] += v[i];
+                            sum2[ct] = __builtin_fmaf(v[i], before[OUT == OUT_MASK ? i : 0] - shift[ct], sum2[ct]);
                         }
                     }
                 }
                 if constexpr (OUT == OUT_EVAL) {
 #pragma unroll
                     for (int i = 0; i < RUN; ++i)
-                        v[i] = relu(__builtin_fmaf(v[i], out_coef[ct].x, out_coef[ct].y));
+                        v[i] = relu(normalised(v[i], out_coef[ct]));
                 }
-                if constexpr (OUT == OUT_STATS || OUT == OUT_PLAIN || OUT == OUT_EVAL || OUT == OUT_MASK) {
+                if constexpr (OUT == OUT_PLAIN || OUT == OUT_EVAL || OUT == OUT_MASK) {
                     if (row) {
                         if (vec) {
 #pragma unroll
@@ -447,24 +415,11 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
                                 p.out[at] = sign[ct] == 0.0f && best == best ? first_y : best * sign[ct];
                                 p.arg[at] = (unsigned char)(where - m * p.group);
                             } else {
-                                p.out[at] = relu(sign[ct] == 0.0f
-                                    ? __builtin_fmaf(best, 0.0f, out_coef[ct].y)
-                                    : __builtin_fmaf(best * sign[ct], out_coef[ct].x, out_coef[ct].y));
+                                p.out[at] = relu(normalised(sign[ct] == 0.0f ? best : best * sign[ct], out_coef[ct]));
                             }
                         }
                         where = -1;
                     }
-                }
-            }
-        }
-        if constexpr (kSums) {
-            if (full) {
-                count += 16 * PT;
-            } else {
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int left = P - (base + PT * (8 * q + 4 * half));
-                    count += left <= 0 ? 0 : left < RUN ? left : RUN;
                 }
             }
         }
@@ -521,17 +476,12 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
         }
     }
 
-    if constexpr (kSums) {  // (sum, sum of squares) or (sum e, sum e (y - mean)) of this workgroup
+    if constexpr (OUT == OUT_MASK) {  // (sum e, sum e (y - mean)) of this workgroup
         __syncthreads();
         double2 *part = reinterpret_cast<double2 *>(lds);  // [kWaves][32 CT]
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) {
             double s1 = sum1[ct], s2 = sum2[ct];
-            if constexpr (OUT != OUT_MASK) {
-                const double sh = count ? (double)shift[ct] : 0.0, n = count;
-                s2 = s2 + 2.0 * sh * s1 + n * sh * sh;
-                s1 = s1 + n * sh;
-            }
             s1 += __shfl_xor(s1, 32);
             s2 += __shfl_xor(s2, 32);
             if (half == 0)
@@ -575,7 +525,7 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_outer_kernel(OuterArgs a)
 
     int r[TA], c[TB];
     f32x4 coef[TA];
-    f32x2 row_act[TA], col_act[TB];
+    f32x4 row_act[TA], col_act[TB];
     float total[TA];
 #pragma unroll
     for (int t = 0; t < TA; ++t) {
@@ -585,14 +535,14 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_outer_kernel(OuterArgs a)
         if constexpr (kGrad)
             coef[t] = reinterpret_cast<const f32x4 *>(p.row.coef)[r[t]];
         if constexpr (ROW == TK3D_MLP_ROW_GRAD_OUT || ROW == TK3D_MLP_ROW_ACT)
-            row_act[t] = scale_shift(p.row_norm, r[t]);
+            row_act[t] = constants_of(p.row_norm, r[t]);
     }
 #pragma unroll
     for (int t = 0; t < TB; ++t) {
         c[t] = cbase + 32 * t + l32;
         c[t] = c[t] < C ? c[t] : C - 1;
         if constexpr (COL == TK3D_MLP_COL_ACT)
-            col_act[t] = scale_shift(p.col_norm, c[t]);
+            col_act[t] = constants_of(p.col_norm, c[t]);
     }
 
     struct Part {
@@ -660,10 +610,10 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_outer_kernel(OuterArgs a)
                     float e = q.x[t][i];
                     const float yy = q.y[kGrad ? t : 0][i];
                     if constexpr (ROW == TK3D_MLP_ROW_GRAD_OUT)
-                        e = passes(__builtin_fmaf(yy, row_act[t].x, row_act[t].y)) ? e : 0.0f;
+                        e = passes(normalised(yy, row_act[t])) ? e : 0.0f;
                     v = __builtin_fmaf(coef[t].x, e, __builtin_fmaf(coef[t].y, yy, coef[t].z));
                 } else if constexpr (ROW == TK3D_MLP_ROW_ACT) {
-                    v = relu(__builtin_fmaf(q.x[t][i], row_act[t].x, row_act[t].y));
+                    v = relu(normalised(q.x[t][i], row_act[t]));
                 } else {
                     v = q.x[t][i];
                 }
@@ -677,7 +627,7 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_outer_kernel(OuterArgs a)
             for (int i = 0; i < 8; ++i) {
                 float v = q.c[t][i];
                 if constexpr (COL == TK3D_MLP_COL_ACT)
-                    v = relu(__builtin_fmaf(v, col_act[t].x, col_act[t].y));
+                    v = relu(normalised(v, col_act[t]));
                 y[t][i] = v;
             }
 #pragma unroll
@@ -810,28 +760,6 @@ __device__ __forceinline__ double2 slot_sum(const void *partial, int slots, int 
     return block_sum(v, lds);
 }
 
-__global__ void __launch_bounds__(kBlock)
-    mlp_statistics_kernel(const void *partial, int slots, double n, float momentum, float *mean,
-                          float *var, float *running_mean, float *running_var, int64_t *batches)
-{
-    __shared__ double2 lds[kWaves];
-    const int c = blockIdx.x;
-    const double2 s = slot_sum(partial, slots, c, lds);
-    if (threadIdx.x == 0) {
-        const double m = s.x / n;
-        double v = s.y / n - m * m;
-        v = v < 0.0 ? 0.0 : v;  // (NaN stays)
-        mean[c] = (float)m;
-        var[c] = (float)v;
-        if (running_mean) {
-            running_mean[c] = (float)((1.0 - (double)momentum) * running_mean[c] + (double)momentum * m);
-            running_var[c] = (float)((1.0 - (double)momentum) * running_var[c] + (double)momentum * (v * n / (n - 1.0)));
-        }
-        if (batches && c == 0)
-            *batches += 1;
-    }
-}
-
 struct Coefficients {
     f32x4 abd;
     float dgamma, dbeta;
@@ -840,7 +768,8 @@ struct Coefficients {
 __device__ __forceinline__ Coefficients grad_coefficients(double2 s, double n, const tk3d_mlp_norm &norm,
                                                           int c, int frozen)
 {
-    const double is = 1.0 / __builtin_sqrt((double)norm.var[c] + (double)norm.eps);
+    const double is = norm.eps < 0.0f ? (double)norm.var[c]
+                                      : 1.0 / __builtin_sqrt((double)norm.var[c] + (double)norm.eps);
     const double gamma = norm.gamma[c], mean = norm.mean[c];
     const double b = frozen ? 0.0 : -gamma * is * is * is * s.y / n;
     const double d = frozen ? 0.0 : -gamma * is * s.x / n - b * mean;
@@ -868,11 +797,11 @@ __global__ void __launch_bounds__(kBlock)
 {
     __shared__ double2 lds[kWaves];
     const int c = blockIdx.y;
-    const f32x2 ss = scale_shift(norm, c);
+    const f32x4 ss = constants_of(norm, c);
     const float mean = norm.mean[c];
     float s1 = 0.0f, s2 = 0.0f;
     const auto add = [&](float gv, float yv) {
-        const float e = passes(__builtin_fmaf(yv, ss.x, ss.y)) ? gv : 0.0f;
+        const float e = passes(normalised(yv, ss)) ? gv : 0.0f;
         s1 += e;
         s2 = __builtin_fmaf(e, yv - mean, s2);
     };
@@ -901,18 +830,18 @@ __global__ void __launch_bounds__(kBlock)
     mlp_activate_kernel(const float *y, int C, int P, tk3d_mlp_norm norm, float *z)
 {
     const int64_t row = (int64_t)blockIdx.y * P;
-    const f32x2 ss = scale_shift(norm, blockIdx.y % C);
+    const f32x4 ss = constants_of(norm, blockIdx.y % C);
     if ((P & 3) == 0) {
         for (int i = (blockIdx.x * kBlock + threadIdx.x) * 4; i < P; i += gridDim.x * kBlock * 4) {
             f32x4 v = *reinterpret_cast<const f32x4 *>(y + row + i);
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-                v[j] = relu(__builtin_fmaf(v[j], ss.x, ss.y));
+                v[j] = relu(normalised(v[j], ss));
             *reinterpret_cast<f32x4 *>(z + row + i) = v;
         }
     } else {
         for (int i = blockIdx.x * kBlock + threadIdx.x; i < P; i += gridDim.x * kBlock)
-            z[row + i] = relu(__builtin_fmaf(y[row + i], ss.x, ss.y));
+            z[row + i] = relu(normalised(y[row + i], ss));
     }
 }
 
@@ -949,7 +878,7 @@ __global__ void __launch_bounds__(1024)
 {
     __shared__ double2 lds[16];
     const int c = blockIdx.x;
-    const f32x2 ss = scale_shift(norm, c);
+    const f32x4 ss = constants_of(norm, c);
     const float mean = norm.mean[c];
     const int count = B * M;
     const auto at = [&](int i) {
@@ -960,7 +889,7 @@ __global__ void __launch_bounds__(1024)
     for (int i = threadIdx.x; i < count; i += blockDim.x) {
         const int64_t j = at(i);
         const float y = extreme[j];
-        const float e = passes(__builtin_fmaf(y, ss.x, ss.y)) ? g[j] : 0.0f;
+        const float e = passes(normalised(y, ss)) ? g[j] : 0.0f;
         v.x += e;
         v.y += (double)e * (double)(y - mean);
     }
@@ -972,7 +901,7 @@ __global__ void __launch_bounds__(1024)
     }
     for (int i = threadIdx.x; i < count; i += blockDim.x) {
         const int64_t j = at(i);
-        const float e = passes(__builtin_fmaf(extreme[j], ss.x, ss.y)) ? g[j] : 0.0f;
+        const float e = passes(normalised(extreme[j], ss)) ? g[j] : 0.0f;
         sel[j] = int2{__float_as_int(k.abd.x * e), (int)arg[j]};
     }
 }
@@ -1047,12 +976,10 @@ __global__ void __launch_bounds__(kBlock, 4)
     mlp_group_kernel(const float *__restrict__ u, const float *__restrict__ xyz,
                      const float *__restrict__ centre, const int64_t *__restrict__ index,
                      const float *__restrict__ wx, int ldw, int C, int N, int M, int S, int tiles,
-                     int total, float *__restrict__ out, float *__restrict__ rel,
-                     double2 *__restrict__ partial, int slots)
+                     int total, float *__restrict__ out)
 {
     __shared__ f32x4 weights[kGroupChannels];
-    __shared__ double2 sums[kWaves][kGroupChannels];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x;
     const int cbase = blockIdx.y * kGroupChannels;
     const int P = M * S;
     const bool vec = (C & 3) == 0;
@@ -1065,12 +992,6 @@ __global__ void __launch_bounds__(kBlock, 4)
     }
     __syncthreads();
 
-    float shift[kGroupChannels], s1[kGroupChannels], s2[kGroupChannels];
-#pragma unroll
-    for (int i = 0; i < kGroupChannels; ++i)
-        shift[i] = s1[i] = s2[i] = 0.0f;
-    double n = 0.0;
-    bool fresh = true;
     for (int tile = blockIdx.x; tile < total; tile += gridDim.x) {
         const int b = tile / tiles;
         const int pos = (tile - b * tiles) * kBlock + tid;
@@ -1085,8 +1006,6 @@ __global__ void __launch_bounds__(kBlock, 4)
         for (int d = 0; d < 3; ++d) {
             const float x = xyz[((int64_t)b * 3 + d) * N + j];
             r[d] = (hit ? x : 0.0f) - centre[((int64_t)b * 3 + d) * M + m];
-            if (rel && blockIdx.y == 0 && in)
-                rel[((int64_t)b * 3 + d) * P + p] = r[d];
         }
         float v[kGroupChannels];
         const float *row = FEATURES ? u + ((int64_t)b * N + j) * C + cbase : nullptr;
@@ -1113,46 +1032,70 @@ __global__ void __launch_bounds__(kBlock, 4)
             if (in && cbase + i < C)
                 out[((int64_t)b * C + cbase + i) * P + pos] = v[i];
         }
-        if (fresh) {
+    }
+}
+
+// ---- the maximum over neighbours of a normalised layer ----------------------------------------------------
+//
+// One pass over z (and one value of y a group) in place of a ReLU over z and a maximum over that.
+// A group of 32 or 64 is a run of 8 or 16 lanes with four values each; of any other size, a lane's.
+
+// (best, where) or (s, at), the first of the largest; NaN above all.
+__device__ __forceinline__ void take_larger(float &best, int &where, float s, int at)
+{
+    const bool up = s != s ? best == best || at < where : s > best || (s == best && at < where);
+    best = up ? s : best;
+    where = up ? at : where;
+}
+
+template <int S>  // 0: `size`
+__global__ void __launch_bounds__(kBlock)
+    mlp_pool_max_kernel(const float *__restrict__ z, const float *__restrict__ y, int64_t groups,
+                        int size, float *__restrict__ out, float *__restrict__ extreme,
+                        unsigned char *__restrict__ arg)
+{
+    constexpr int LANES = S ? S / 4 : 1;
+    const int64_t stride = (int64_t)gridDim.x * kBlock / LANES;
+    const int l = threadIdx.x % LANES;
+    for (int64_t g = ((int64_t)blockIdx.x * kBlock + threadIdx.x) / LANES; g < groups; g += stride) {
+        float best;
+        int where;
+        if constexpr (S != 0) {
+            const f32x4 v = *reinterpret_cast<const f32x4 *>(z + g * S + 4 * l);
+            best = v[0];
+            where = 4 * l;
 #pragma unroll
-            for (int i = 0; i < kGroupChannels; ++i)
-                shift[i] = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v[i])));
-            fresh = false;
-        }
-        if (in) {
-            n += 1.0;
+            for (int i = 1; i < 4; ++i)
+                take_larger(best, where, v[i], 4 * l + i);
 #pragma unroll
-            for (int i = 0; i < kGroupChannels; ++i) {
-                const float d = v[i] - shift[i];
-                s1[i] += d;
-                s2[i] = __builtin_fmaf(d, d, s2[i]);
+            for (int off = 1; off < LANES; off <<= 1) {
+                const float other = __shfl_xor(best, off);
+                const int at = __shfl_xor(where, off);
+                take_larger(best, where, other, at);
             }
-        }
-    }
+        } else {
+            const float *row = z + g * size;
+            best = row[0];
+            where = 0;
+            int i = 1;
+            if ((size & 3) == 0) {
+                i = 0;
+                for (; i < size; i += 4) {
+                    const f32x4 v = *reinterpret_cast<const f32x4 *>(row + i);
 #pragma unroll
-    for (int off = 1; off < 64; off <<= 1)
-        n += __shfl_xor(n, off);
-#pragma unroll
-    for (int i = 0; i < kGroupChannels; ++i) {
-        float a = s1[i], q = s2[i];
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            a += __shfl_xor(a, off);
-            q += __shfl_xor(q, off);
+                    for (int j = 0; j < 4; ++j)
+                        if (i + j > 0)
+                            take_larger(best, where, v[j], i + j);
+                }
+            }
+            for (; i < size; ++i)
+                take_larger(best, where, row[i], i);
         }
-        if (lane == 0) {
-            const double sh = n > 0.0 ? (double)shift[i] : 0.0;
-            sums[wave][i] = double2{a + n * sh, q + 2.0 * sh * a + n * sh * sh};
+        if (l == 0) {
+            out[g] = relu(best);
+            extreme[g] = y[g * (S ? S : size) + where];
+            arg[g] = (unsigned char)where;
         }
-    }
-    __syncthreads();
-    if (tid < kGroupChannels && cbase + tid < C) {
-        double2 s = sums[0][tid];
-        for (int w = 1; w < kWaves; ++w) {
-            s.x += sums[w][tid].x;
-            s.y += sums[w][tid].y;
-        }
-        partial[(int64_t)(cbase + tid) * slots + blockIdx.x] = s;
     }
 }
 
@@ -1195,8 +1138,7 @@ int fill(const tk3d_mlp_product &p, int in, int out, Shape s, GemmArgs &g)
     const int group_bytes = s.ct * 1024;
     g.chunk = g.kg * group_bytes <= kWeightBytes ? g.kg : kWeightBytes / 2 / group_bytes;
     g.coef_bytes = in == TK3D_MLP_IN_RAW || in == TK3D_MLP_IN_RAW2 ? 0
-                   : in == TK3D_MLP_IN_GRAD ? g.kg * 8 * 16
-                   : in == TK3D_MLP_IN_GRAD_OUT ? g.kg * 8 * 24 : g.kg * 8 * 8;
+                   : in == TK3D_MLP_IN_GRAD_OUT ? g.kg * 8 * 32 : g.kg * 8 * 16;
     const int cblocks = (p.C + 32 * s.ct - 1) / (32 * s.ct);
     int wgs = (g.total + kWaves - 1) / kWaves;
     int most = (2 * tk_cu_count() + cblocks - 1) / cblocks;
@@ -1300,14 +1242,13 @@ int tk3d_mlp_product_f32(int in, int out, const tk3d_mlp_product *p, void *strea
     const int cblocks = fill(*p, in, out, s, g);
     const hipStream_t stream = (hipStream_t)stream_;
 #define TK_CASE(IN, OUT)                                                                                 if (in == TK3D_MLP_##IN && out == TK3D_MLP_##OUT)                                                        return launch_shape<IN, OUT>(g, s, cblocks, stream);
-    TK_CASE(IN_RAW, OUT_STATS)
     TK_CASE(IN_RAW, OUT_EVAL)
     TK_CASE(IN_RAW, OUT_PLAIN)
     TK_CASE(IN_RAW, OUT_POINTS)
     TK_CASE(IN_RAW, OUT_POOL_EVAL)
-    TK_CASE(IN_RAW2, OUT_STATS)
+    TK_CASE(IN_RAW2, OUT_PLAIN)
     TK_CASE(IN_RAW2, OUT_EVAL)
-    TK_CASE(IN_ACT, OUT_STATS)
+    TK_CASE(IN_ACT, OUT_PLAIN)
     TK_CASE(IN_ACT, OUT_EVAL)
     TK_CASE(IN_ACT, OUT_POOL)
     TK_CASE(IN_ACT, OUT_POOL_EVAL)
@@ -1378,12 +1319,23 @@ int tk3d_mlp_sum_f32(const tk3d_mlp_sum *sums, int n, void *stream)
     return tk_launch_status();
 }
 
-int tk3d_mlp_statistics_f32(const void *partial, int slots, int64_t n, int C, float momentum,
-                            float *mean, float *var, float *running_mean, float *running_var,
-                            int64_t *batches, void *stream)
+int tk3d_mlp_pool_max_f32(const float *z, const float *y, int64_t groups, int size, float *out,
+                          float *extreme, unsigned char *arg, void *stream_)
 {
-    mlp_statistics_kernel<<<C, kBlock, 0, (hipStream_t)stream>>>(partial, slots, (double)n, momentum,
-                                                               mean, var, running_mean, running_var, batches);
+    if (groups < 0 || size <= 0 || size > 255)
+        return TK3D_ERR_BAD_SIZE;
+    if (groups == 0)
+        return TK3D_OK;
+    const int lanes = size == 32 ? 8 : size == 64 ? 16 : 1;
+    const int64_t blocks = (groups * lanes + kBlock - 1) / kBlock, most = 16 * tk_cu_count();
+    const unsigned grid = (unsigned)(blocks < most ? blocks : most);
+    const hipStream_t stream = (hipStream_t)stream_;
+    if (size == 32)
+        mlp_pool_max_kernel<32><<<grid, kBlock, 0, stream>>>(z, y, groups, size, out, extreme, arg);
+    else if (size == 64)
+        mlp_pool_max_kernel<64><<<grid, kBlock, 0, stream>>>(z, y, groups, size, out, extreme, arg);
+    else
+        mlp_pool_max_kernel<0><<<grid, kBlock, 0, stream>>>(z, y, groups, size, out, extreme, arg);
     return tk_launch_status();
 }
 
@@ -1468,33 +1420,24 @@ int tk3d_mlp_pool_weight_grad_f32(const float *sparse, int sparse_splits, const 
     return tk_launch_status();
 }
 
-int tk3d_mlp_group_slots(int B, int C, int M, int S)
-{
-    const int chunks = (C + kGroupChannels - 1) / kGroupChannels;
-    const int64_t total = (int64_t)B * (((int64_t)M * S + kBlock - 1) / kBlock);
-    int64_t most = (8 * tk_cu_count() + chunks - 1) / chunks;
-    most = (most + 7) & ~7;
-    return (int)(total < most ? total : most);
-}
-
 int tk3d_mlp_group_f32(const float *u, const float *xyz, const float *centre, const int64_t *index,
                        const float *wx, int ldw, int B, int C, int N, int M, int S, float *y,
-                       float *rel, void *partial, void *stream)
+                       void *stream)
 {
     if (B <= 0 || C <= 0 || N <= 0 || M <= 0 || S <= 0 || !tk_fits(TK_MAX_I32, M, S))
         return TK3D_ERR_BAD_SIZE;
-    const int slots = tk3d_mlp_group_slots(B, C, M, S);
     const int tiles = (M * S + kBlock - 1) / kBlock;
     if (!tk_fits(TK_MAX_I32, B, tiles))
         return TK3D_ERR_UNSUPPORTED;
-    const dim3 grid(slots, (C + kGroupChannels - 1) / kGroupChannels);
-    double2 *part = reinterpret_cast<double2 *>(partial);
+    const int chunks = (C + kGroupChannels - 1) / kGroupChannels;
+    const int most = ((8 * tk_cu_count() + chunks - 1) / chunks + 7) & ~7;
+    const dim3 grid(B * tiles < most ? B * tiles : most, chunks);
     if (u)
         mlp_group_kernel<true><<<grid, kBlock, 0, (hipStream_t)stream>>>(
-            u, xyz, centre, index, wx, ldw, C, N, M, S, tiles, B * tiles, y, rel, part, slots);
+            u, xyz, centre, index, wx, ldw, C, N, M, S, tiles, B * tiles, y);
     else
         mlp_group_kernel<false><<<grid, kBlock, 0, (hipStream_t)stream>>>(
-            u, xyz, centre, index, wx, ldw, C, N, M, S, tiles, B * tiles, y, rel, part, slots);
+            u, xyz, centre, index, wx, ldw, C, N, M, S, tiles, B * tiles, y);
     return tk_launch_status();
 }
 

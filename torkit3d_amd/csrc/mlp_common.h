@@ -17,10 +17,19 @@ __device__ __forceinline__ float relu(float z) { return __builtin_elementwise_ma
 // Whether the gradient passes a ReLU whose input was z (torch: where the output is > 0 or NaN).
 __device__ __forceinline__ bool passes(float z) { return !(z <= 0.0f); }
 
-__device__ __forceinline__ f32x2 scale_shift(const tk3d_mlp_norm &n, int c)
+// A channel's batch norm: (mean, 1 / sqrt(variance + eps), gamma, beta).
+__device__ __forceinline__ f32x4 constants_of(const tk3d_mlp_norm &n, int c)
 {
-    const float scale = n.gamma[c] * (1.0f / __builtin_sqrtf(n.var[c] + n.eps));
-    return f32x2{scale, __builtin_fmaf(-n.mean[c], scale, n.beta[c])};
+    return f32x4{n.mean[c], n.eps < 0.0f ? n.var[c] : 1.0f / __builtin_sqrtf(n.var[c] + n.eps),
+                 n.gamma[c], n.beta[c]};
+}
+
+// In this order of operations the library's batch norm gives the same bits (12 shapes, 10^8 values),
+// so that in training the ReLU's signs are those of the forward pass. A scale and a shift worked
+// out beforehand would save two operations a value, but round differently.
+__device__ __forceinline__ float normalised(float y, f32x4 k)
+{
+    return __builtin_fmaf(k.z, (y - k.x) * k.y, k.w);
 }
 
 // The sign by which a maximum over relu(norm(y)) becomes one over y.

@@ -34,13 +34,12 @@ using torch::autograd::variable_list;
 
 float *f32(const Tensor &t) { return t.defined() ? t.data_ptr<float>() : nullptr; }
 
-// The statistics kernels write the running statistics: whoever saved them has to see that.
-void written(const Tensor &mean, const Tensor &var, const Tensor &count)
-{
-    for (const Tensor *t : {&mean, &var, &count})
-        if (t->defined())
-            t->unsafeGetTensorImpl()->bump_version();
-}
+// Whether the gradients of a training step are those of the stock modules, for rows of P values. On
+// rows whose length is no multiple of four the library's batch norm backward loses values where
+// they are longer than 1024, in large batches longer than 512: dgamma and dbeta of [2, 64, 1025] and
+// of [40, 64, 515] are 1e-1 off from float64, 1e-7 at [2, 64, 1023] and [40, 64, 511]. The kernels
+// here are not, but a step on such clouds goes on giving what it gave.
+bool same_gradients(int64_t P) { return P <= 512 || P % 4 == 0; }
 
 // Saved tensors come back through hooks, which may lay them out anew.
 variable_list dense(variable_list saved)
@@ -59,6 +58,7 @@ struct Call {
     // centre [B, 3, M], index [B, M, S]
     Tensor xyz, centre, index;
     int64_t pool = 0;  // maximum over groups of this many consecutive positions, 0: none
+    int64_t rows = 0;  // of a dense input given as [B, C, rows, P / rows]
     bool training = false;
     std::vector<double> eps, momentum;
     std::vector<Tensor> params;   // weight, gamma, beta of every layer
@@ -75,7 +75,8 @@ struct Call {
 };
 
 // What the backward needs besides the call: the product of every layer (of a pooled last layer
-// the extremes, and their places), and the statistics it was normalised with.
+// the extremes, and their places), and the statistics it was normalised with (training: `var` is
+// 1 / sqrt(variance + eps), as batch norm saves it).
 struct Kept {
     std::vector<Tensor> y, mean, var;
     Tensor arg;
@@ -84,7 +85,7 @@ struct Kept {
 tk3d_mlp_norm norm_of(const Call &c, const Kept &k, int64_t l)
 {
     return {f32(k.mean[l]), f32(k.var[l]), f32(c.params[3 * l + 1]), f32(c.params[3 * l + 2]),
-            (float)c.eps[l]};
+            c.training ? -1.0f : (float)c.eps[l]};
 }
 
 tk3d_mlp_source source(const Tensor &x, const float *w, int64_t wk, int64_t wc)
@@ -132,6 +133,26 @@ void run_product(int in, int out, tk3d_mlp_product &p, void *stream)
     done(tk3d_mlp_product_f32(in, out, &p, stream), "tk3d_mlp_product_f32");
 }
 
+// The product of the first layer behind a grouping, without the grouped tensor.
+void first_grouped(const Call &c, const Tensor &y)
+{
+    const int64_t B = c.batch(), C = c.out_channels(0), K = c.in_channels(0);
+    const int64_t M = c.index.size(1), S = c.index.size(2), N = c.xyz.size(2);
+    const float *w = f32(c.weight(0));
+    void *stream = stream_of(c.xyz);
+    Tensor u;
+    if (c.x.defined()) {
+        u = at::empty({B, N, C}, c.xyz.options());
+        tk3d_mlp_product q = product(B, C, N);
+        q.src[0] = source(c.x, w, 1, K);
+        q.out = f32(u);
+        run_product(TK3D_MLP_IN_RAW, TK3D_MLP_OUT_POINTS, q, stream);
+    }
+    done(tk3d_mlp_group_f32(f32(u), f32(c.xyz), f32(c.centre), c.index.data_ptr<int64_t>(), w + (K - 3),
+                            (int)K, (int)B, (int)C, (int)N, (int)M, (int)S, f32(y), stream),
+         "tk3d_mlp_group_f32");
+}
+
 // Evaluation without gradients: every layer leaves its activations.
 Tensor evaluate(const Call &c)
 {
@@ -150,23 +171,8 @@ Tensor evaluate(const Call &c)
         tk3d_mlp_product p = product(B, C, P);
         p.out_norm = norm_of(c, k, l);
         if (l == 0 && c.grouped()) {
-            const int64_t M = c.index.size(1), S = c.index.size(2), N = c.xyz.size(2);
-            Tensor u;
-            if (c.x.defined()) {
-                u = at::empty({B, N, C}, like.options());
-                tk3d_mlp_product q = product(B, C, N);
-                q.src[0] = source(c.x, w, 1, K);
-                q.out = f32(u);
-                run_product(TK3D_MLP_IN_RAW, TK3D_MLP_OUT_POINTS, q, stream);
-            }
             h = at::empty({B, C, P}, like.options());
-            const Tensor partial =
-                partial_sums(like, C, tk3d_mlp_group_slots((int)B, (int)C, (int)M, (int)S));
-            done(tk3d_mlp_group_f32(f32(u), f32(c.xyz), f32(c.centre),
-                                    c.index.data_ptr<int64_t>(), w + (K - 3), (int)K, (int)B, (int)C,
-                                    (int)N, (int)M, (int)S, f32(h), nullptr, partial.data_ptr(),
-                                    stream),
-                 "tk3d_mlp_group_f32");
+            first_grouped(c, h);
             continue;
         }
         int in = TK3D_MLP_IN_RAW, out = TK3D_MLP_OUT_EVAL;
@@ -199,7 +205,79 @@ Tensor evaluate(const Call &c)
     return h;
 }
 
-// Forward that keeps what the backward needs (and, in training, takes batch statistics).
+// A layer of stock operators in training mode: the product, and its batch norm with the statistics
+// of this batch (and the running ones updated).
+struct Normalised {
+    Tensor y, z, mean, inv_std;
+};
+
+Normalised stock_layer(const Tensor &h, const Tensor &weight, const Tensor &gamma, const Tensor &beta,
+                       const Tensor &running_mean, const Tensor &running_var, const Tensor &batches,
+                       double momentum, double eps)
+{
+    Normalised n;
+    n.y = h.dim() == 4 ? at::conv2d(h, weight) : at::conv1d(h, weight);
+    if (batches.defined())
+        Tensor(batches).add_(1);
+    std::tie(n.z, n.mean, n.inv_std, std::ignore, std::ignore) =
+        at::_batch_norm_impl_index(n.y, gamma, beta, running_mean, running_var, true, momentum, eps,
+                                   at::globalContext().userEnabledCuDNN());
+    return n;
+}
+
+// ReLU and the maximum over the last dimension of z, with the y at the place of the maximum.
+Tensor pool_max(const Normalised &n, Tensor &extreme, Tensor &arg)
+{
+    const Tensor z = n.z.contiguous(), y = n.y.contiguous();
+    const int64_t B = z.size(0), C = z.size(1), M = z.size(2);
+    const Tensor out = at::empty({B, C, M}, z.options());
+    extreme = at::empty({B, C, M}, z.options());
+    arg = at::empty({B, C, M}, z.options().dtype(at::kByte));
+    done(tk3d_mlp_pool_max_f32(f32(z), f32(y), B * C * M, (int)z.size(3), f32(out), f32(extreme),
+                               arg.data_ptr<uint8_t>(), stream_of(z)),
+         "tk3d_mlp_pool_max_f32");
+    return out;
+}
+
+// Training: the activations of the stock modules, bit by bit. The gradient of a training step
+// follows the signs and places that last-bit differences decide: with products and statistics of
+// its own, however exact, one step in six of a PointNet++ or DGCNN had single gradients off by more
+// than half their root mean square from the stock modules' (which are as far from float64). Fused
+// are the grouping, the maximum behind the last layer, what is kept (the products alone, no
+// activations, no edge of a pooled layer), and the whole backward.
+Tensor forward_training(const Call &c, Kept &k)
+{
+    const int64_t B = c.batch(), L = c.layers();
+    Tensor h = c.x2.defined() ? at::cat({c.x, c.x2}, 1) : c.x;
+    if (c.grouped()) {
+        const int64_t M = c.index.size(1), S = c.index.size(2), N = c.xyz.size(2);
+        const int64_t F = c.in_channels(0) - 3;
+        h = at::empty({B, F + 3, M, S}, c.xyz.options());
+        done(tk3d_group_points_concat_forward_f32(f32(c.x), f32(c.xyz), f32(c.centre),
+                                                  c.index.data_ptr<int64_t>(), B, F, N, M, S, f32(h),
+                                                  stream_of(h)),
+             "tk3d_group_points_concat_forward_f32");
+    } else if (c.params[0].dim() == 4) {
+        h = h.view({B, h.size(1), c.rows, -1});
+    }
+    for (int64_t l = 0; l < L; ++l) {
+        const Tensor *w = &c.params[3 * l], *s = &c.buffers[3 * l];
+        const Normalised n = stock_layer(h, w[0], w[1], w[2], s[0], s[1], s[2], c.momentum[l], c.eps[l]);
+        k.mean.push_back(n.mean);
+        k.var.push_back(n.inv_std);
+        if (c.pool && l == L - 1) {
+            Tensor extreme;
+            h = pool_max(n, extreme, k.arg);
+            k.y.push_back(extreme);
+        } else {
+            h = Tensor(n.z).relu_();
+            k.y.push_back(n.y.flatten(2).contiguous());
+        }
+    }
+    return h;
+}
+
+// Forward in evaluation mode that keeps what the backward needs.
 Tensor forward(const Call &c, Kept &k)
 {
     const int64_t B = c.batch(), P = c.positions(), L = c.layers();
@@ -210,28 +288,11 @@ Tensor forward(const Call &c, Kept &k)
         const float *w = f32(c.weight(l));
         tk3d_mlp_product p = product(B, C, P);
         const bool pooled = c.pool && l == L - 1;
-        std::pair<Tensor, int> sums;
-        Tensor y;
+        const Tensor y = at::empty({B, C, pooled ? P / c.pool : P}, like.options());
         if (l == 0 && c.grouped()) {
-            const int64_t M = c.index.size(1), S = c.index.size(2), N = c.xyz.size(2);
-            Tensor u;
-            if (c.x.defined()) {
-                u = at::empty({B, N, C}, like.options());
-                tk3d_mlp_product q = product(B, C, N);
-                q.src[0] = source(c.x, w, 1, K);
-                q.out = f32(u);
-                run_product(TK3D_MLP_IN_RAW, TK3D_MLP_OUT_POINTS, q, stream);
-            }
-            y = at::empty({B, C, P}, like.options());
-            sums.second = tk3d_mlp_group_slots((int)B, (int)C, (int)M, (int)S);
-            sums.first = partial_sums(like, C, sums.second);
-            done(tk3d_mlp_group_f32(f32(u), f32(c.xyz), f32(c.centre),
-                                    c.index.data_ptr<int64_t>(), w + (K - 3), (int)K, (int)B, (int)C,
-                                    (int)N, (int)M, (int)S, f32(y), nullptr,
-                                    sums.first.data_ptr(), stream),
-                 "tk3d_mlp_group_f32");
+            first_grouped(c, y);
         } else {
-            int in = TK3D_MLP_IN_ACT, out = TK3D_MLP_OUT_STATS;
+            int in = TK3D_MLP_IN_ACT, out = TK3D_MLP_OUT_PLAIN;
             if (l == 0) {
                 in = TK3D_MLP_IN_RAW;
                 p.src[0] = source(c.x, w, 1, K);
@@ -251,27 +312,12 @@ Tensor forward(const Call &c, Kept &k)
                 k.arg = at::empty({B, C, p.M}, like.options().dtype(at::kByte));
                 p.arg = k.arg.data_ptr<uint8_t>();
             }
-            y = at::empty({B, C, pooled ? P / c.pool : P}, like.options());
             p.out = f32(y);
-            sums = summed_product(in, out, p, like, stream);
+            run_product(in, out, p, stream);
         }
         k.y.push_back(y);
-        if (c.training) {
-            const Tensor stats = at::empty({2, C}, like.options());
-            k.mean.push_back(stats.select(0, 0));
-            k.var.push_back(stats.select(0, 1));
-            const Tensor &count = c.buffers[3 * l + 2];
-            done(tk3d_mlp_statistics_f32(sums.first.data_ptr(), sums.second, B * P, (int)C,
-                                         (float)c.momentum[l], f32(k.mean[l]), f32(k.var[l]),
-                                         f32(c.buffers[3 * l]), f32(c.buffers[3 * l + 1]),
-                                         count.defined() ? count.data_ptr<int64_t>() : nullptr,
-                                         stream),
-                 "tk3d_mlp_statistics_f32");
-            written(c.buffers[3 * l], c.buffers[3 * l + 1], count);
-        } else {
-            k.mean.push_back(c.buffers[3 * l]);
-            k.var.push_back(c.buffers[3 * l + 1]);
-        }
+        k.mean.push_back(c.buffers[3 * l]);
+        k.var.push_back(c.buffers[3 * l + 1]);
     }
     const Tensor &last = k.y[L - 1];
     const Tensor z = at::empty(last.sizes(), like.options());
@@ -540,7 +586,7 @@ struct Node : torch::autograd::Function<Node> {
                           const std::optional<Tensor> &x2, at::TensorList params, const Call &call)
     {
         Kept k;
-        const Tensor z = tk3d::forward(call, k);
+        const Tensor z = call.training ? forward_training(call, k) : tk3d::forward(call, k);
         variable_list saved = {call.x, call.x2, call.xyz, call.centre, call.index, k.arg};
         for (int64_t l = 0; l < call.layers(); ++l) {
             for (int64_t i = 0; i < 3; ++i)
@@ -602,7 +648,8 @@ struct Node : torch::autograd::Function<Node> {
                 if (t.requires_grad())
                     inputs.push_back(t);
             const variable_list d =
-                torch::autograd::grad({z}, inputs, {grads[0]}, std::nullopt, true, true);
+                torch::autograd::grad({z}, inputs, {grads[0].reshape(z.sizes())}, std::nullopt, true,
+                                      true);
             size_t i = 0;
             result.push_back(want_x ? d[i++] : Tensor());
             result.push_back(want_x2 ? d[i++] : Tensor());
@@ -645,7 +692,7 @@ struct EdgeKept {
 
 tk3d_mlp_norm norm_of(const EdgeCall &c, const EdgeKept &k)
 {
-    return {f32(k.mean), f32(k.var), f32(c.gamma), f32(c.beta), (float)c.eps};
+    return {f32(k.mean), f32(k.var), f32(c.gamma), f32(c.beta), c.training ? -1.0f : (float)c.eps};
 }
 
 Tensor edge_forward(const EdgeCall &c, EdgeKept &k, bool keep)
@@ -662,32 +709,30 @@ Tensor edge_forward(const EdgeCall &c, EdgeKept &k, bool keep)
     p.src[0] = source(c.x, f32(k.matrix), 1, C);
     p.out = f32(k.uv);
     run_product(TK3D_MLP_IN_RAW, TK3D_MLP_OUT_POINTS, p, stream);
-    k.extreme = at::empty({B, O, N}, options);
-    if (keep) {
-        k.arg = at::empty({B, O, N}, options.dtype(at::kByte));
+    if (keep)
         k.sum = at::empty({B, N, O}, options);
-    }
-    const int slots = tk3d_mlp_edge_slots((int)B, (int)N);
-    const Tensor partial = partial_sums(c.x, O, slots);
-    done(tk3d_mlp_edge_forward_f32(f32(k.uv), c.index.data_ptr<int64_t>(), f32(c.gamma), (int)B,
-                                   (int)N, (int)K, (int)O, f32(k.extreme),
-                                   keep ? k.arg.data_ptr<uint8_t>() : nullptr, f32(k.sum),
-                                   partial.data_ptr(), stream),
-         "tk3d_mlp_edge_forward_f32");
-    if (c.training) {
-        const Tensor stats = at::empty({2, O}, options);
-        k.mean = stats.select(0, 0);
-        k.var = stats.select(0, 1);
-        done(tk3d_mlp_statistics_f32(partial.data_ptr(), slots, B * N * K, (int)O, (float)c.momentum,
-                                     f32(k.mean), f32(k.var), f32(c.running_mean),
-                                     f32(c.running_var),
-                                     c.batches.defined() ? c.batches.data_ptr<int64_t>() : nullptr,
-                                     stream),
-             "tk3d_mlp_statistics_f32");
-        written(c.running_mean, c.running_var, c.batches);
-    } else {
+    if (!c.training) {
+        k.extreme = at::empty({B, O, N}, options);
+        if (keep)
+            k.arg = at::empty({B, O, N}, options.dtype(at::kByte));
         k.mean = c.running_mean;
         k.var = c.running_var;
+    }
+    done(tk3d_mlp_edge_forward_f32(f32(k.uv), c.index.data_ptr<int64_t>(), f32(c.gamma), (int)B,
+                                   (int)N, (int)K, (int)O, f32(k.extreme),
+                                   k.arg.defined() ? k.arg.data_ptr<uint8_t>() : nullptr, f32(k.sum),
+                                   stream),
+         "tk3d_mlp_edge_forward_f32");
+    if (c.training) {  // (bit by bit what the stock modules give, see forward_training)
+        const Tensor edges = at::empty({B, 2 * C, N, K}, options);
+        done(tk3d_mlp_edge_features_f32(f32(c.x), c.index.data_ptr<int64_t>(), (int)B, (int)C, (int)N,
+                                        (int)K, f32(edges), stream),
+             "tk3d_mlp_edge_features_f32");
+        const Normalised n = stock_layer(edges, c.weight, c.gamma, c.beta, c.running_mean,
+                                         c.running_var, c.batches, c.momentum, c.eps);
+        k.mean = n.mean;
+        k.var = n.inv_std;
+        return pool_max(n, k.extreme, k.arg);
     }
     const Tensor z = at::empty({B, O, N}, options);
     const tk3d_mlp_norm norm = norm_of(c, k);
@@ -890,6 +935,9 @@ Tensor mlp(Tensor x, Tensor x2, const Tensor &xyz, const Tensor &centre, const T
             return Tensor();
         channels = params[3 * l].size(0);
     }
+    if (params[0].dim() != (grouped ? 4 : x.dim()))
+        return Tensor();  // (a Conv1d on [B, C, M, S] and the like: stock torch has the error)
+    c.rows = !grouped && x.dim() == 4 ? x.size(2) : 0;
     if (has_x)
         c.x = x.dim() == 4 ? x.flatten(2).contiguous() : x.contiguous();
     if (has_x2)
@@ -901,6 +949,9 @@ Tensor mlp(Tensor x, Tensor x2, const Tensor &xyz, const Tensor &centre, const T
     c.eps = std::move(eps);
     c.momentum = std::move(momentum);
     const int64_t B = c.batch(), P = c.positions();
+    // (training mode without gradients updates running statistics: the stock modules do)
+    if (training && (!(c10::GradMode::is_enabled() && tracked) || !same_gradients(P)))
+        return Tensor();
     int64_t widest = has_x ? c.x.size(1) : 0;
     if (has_x2)
         widest = std::max(widest, c.x2.size(1));
@@ -908,7 +959,7 @@ Tensor mlp(Tensor x, Tensor x2, const Tensor &xyz, const Tensor &centre, const T
         widest = std::max(widest, c.out_channels(l));
     const int64_t longest = grouped ? std::max(P, c.xyz.size(2)) : P;
     // (one value per channel has no variance: stock batch norm raises the error)
-    if (B == 0 || P == 0 || longest == 0 || B * P < 2 || widest > 4096 ||
+    if (B == 0 || P == 0 || longest == 0 || B * P < 2 || widest > 2048 ||
         (widest + 8) * longest > (1 << 29) || B * longest > (1 << 30))
         return Tensor();
     OnDeviceOf guard(c.like().device());
@@ -918,14 +969,11 @@ Tensor mlp(Tensor x, Tensor x2, const Tensor &xyz, const Tensor &centre, const T
             return t.defined() ? std::optional<Tensor>(t) : std::nullopt;
         };
         z = Node::apply(given(c.x), given(c.x2), at::TensorList(c.params), c);
-    } else if (training) {
-        Kept k;
-        z = forward(c, k);
     } else {
         z = evaluate(c);
     }
     if (!grouped && x.dim() == 4 && !pool)
-        z = z.view({shape[0], z.size(1), shape[2], shape[3]});
+        z = z.reshape({shape[0], z.size(1), shape[2], shape[3]});
     return z;
 }
 
@@ -954,12 +1002,12 @@ Tensor edge_conv(const Tensor &x, const Tensor &index, const Tensor &lists,
 {
     if (!usable(x, x) || x.dim() != 3 || !usable_index(index, x) || index.dim() != 3 ||
         index.size(0) != x.size(0) || index.size(1) != x.size(2) || params.size() != 3 || watched() ||
-        !usable_layer(params.data(), buffers.data(), x))
+        params[0].dim() != 4 || !usable_layer(params.data(), buffers.data(), x))
         return Tensor();
     const int64_t B = x.size(0), C = x.size(1), N = x.size(2), K = index.size(2);
     const int64_t O = params[0].size(0);
     if (params[0].size(1) != 2 * C || !tk3d_mlp_edge_supported(B, N, K, O) || B * N * K < 2 ||
-        C > 4096 || (std::max(C, 2 * O) + 8) * N > (1 << 29))
+        C > 4096 || (std::max(C, 2 * O) + 8) * N > (1 << 29) || (training && !same_gradients(N * K)))
         return Tensor();
     EdgeCall c;
     c.x = x.contiguous();
@@ -979,6 +1027,8 @@ Tensor edge_conv(const Tensor &x, const Tensor &index, const Tensor &lists,
         c.lists = lists.defined() ? lists : edge_lists(c.index, N);
         return EdgeNode::apply(c.x, c.weight, c.gamma, c.beta, c);
     }
+    if (training)
+        return Tensor();  // (as for mlp())
     EdgeKept k;
     return edge_forward(c, k, false);
 }

@@ -19,10 +19,6 @@ class PointNet(nn.Module):
         self.in_channels = in_channels
         self.out_channels = (tuple(local_channels) + tuple(global_channels))[-1]
         self.mlp_local = mlp1d_bn_relu(in_channels, local_channels)
-        # Clouds of one distribution have nearly equal pooled features, and the head's batch norm
-        # over a few of them turns last-bit differences of the local statistics into percents of
-        # the gradients. Training keeps the stock modules, so that it reproduces earlier runs.
-        self.mlp_local.fused_training = False
         self.mlp_global = mlp_bn_relu(local_channels[-1], global_channels)
         self.reset_parameters()
 

@@ -73,12 +73,11 @@ class LinearBNReLU(nn.Module):
 class SharedMLP(nn.Sequential):
     """The layers of ``mlp1d_bn_relu`` / ``mlp2d_bn_relu`` (an ``nn.Sequential`` to its
     checkpoints and to anything that walks its modules), run as one chain of fused kernels
-    (csrc/mlp.hip) on float32 GPU tensors: the product of a layer normalises its input as it
-    reads it and sums up the statistics of its output. Whatever is not plain - hooks, other
-    modules in place of the blocks', frozen layers among training ones, autocast - runs layer
-    by layer in stock torch."""
-
-    fused_training = True  # whether training mode takes the fused kernels too
+    (csrc/mlp.hip) on float32 GPU tensors: in evaluation mode the products with their norms and
+    maxima, in training mode the backward and what it needs of the forward (the activations stay
+    those of the stock modules, bit by bit). Whatever is not plain - hooks, other modules in place
+    of the blocks', frozen layers among training ones, autocast - runs layer by layer in stock
+    torch."""
 
     def forward(self, input):
         if not torch.jit.is_scripting():
@@ -144,8 +143,6 @@ class SharedMLP(nn.Sequential):
                 return None
             if training is None:
                 training = bn.training
-                if training and not self.fused_training:
-                    return None
             # (a replica of DataParallel holds its tensors as attributes: get() finds none)
             weight = conv._parameters.get("weight")
             gamma, beta = (bn._parameters.get(name) for name in ("weight", "bias"))
