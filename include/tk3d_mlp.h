@@ -14,9 +14,8 @@
  *     dy = a e + b y + d  with (a, b, d) per channel (tk3d_mlp_grad_coefficients_f32).
  *
  * Pooled layers. Where only the maximum of z over groups of `group` consecutive positions is
- * wanted, y itself is never stored: the product keeps the extreme of y over each group (the
- * largest for gamma >= 0, else the smallest) and its place. In the backward e has one nonzero per
- * group and channel, and with y = W x
+ * wanted, the place of the maximum and the y there are all of the layer that is kept. In the
+ * backward e has one nonzero per group and channel, and with y = W x
  *     W^T dy = W^T (a e) + (W^T diag(b) W) x + W^T d
  *     dW     = (a e) x^T + diag(b) W (x x^T) + d (sum x)^T
  * so the dense part needs only the input x.
@@ -40,7 +39,6 @@ typedef struct {
     const float *x;        /* [B, K, P]; batch_stride elements from one batch element to the next */
     const float *y;        /* same shape, for the gradient inputs */
     const float *coef;     /* [K][4]: (a, b, d, -), for the gradient inputs */
-    const void *sel;       /* [B, K, M] of (float a e, int32 place in the group), sparse input */
     const float *w;        /* weight of input channel k and output channel c: w[k * wk + c * wc] */
     int64_t batch_stride;
     int32_t K, wk, wc;
@@ -53,13 +51,11 @@ enum {
     TK3D_MLP_IN_ACT = 2,      /* relu(in_norm(x)) */
     TK3D_MLP_IN_GRAD = 3,     /* a x + b y + d */
     TK3D_MLP_IN_GRAD_OUT = 4, /* the same with x masked by relu(in_norm(y)) first */
-    TK3D_MLP_IN_POOL = 5,     /* the sparse src[0].sel, then relu(in_norm(src[1].x)) */
     TK3D_MLP_OUT_PLAIN = 1,     /* out + bias, channels from C0 on in out2; either may be NULL */
     TK3D_MLP_OUT_POINTS = 2,    /* out as [B, P, C] */
     TK3D_MLP_OUT_EVAL = 3,      /* relu(out_norm(out)) */
-    TK3D_MLP_OUT_POOL = 4,      /* extreme over groups (out [B,C,M]) and place (arg) */
     TK3D_MLP_OUT_POOL_EVAL = 5, /* relu(out_norm(extreme over groups)) */
-    TK3D_MLP_OUT_MASK = 6       /* e = (out + bias) where relu(out_norm(yprev)) passes, and partial
+    TK3D_MLP_OUT_MASK = 6       /* e = (out + bias, IN_ACT: + add) where relu(out_norm(yprev)) passes, and partial
                                    sums of e and e (yprev - mean) */
 };
 
@@ -69,7 +65,7 @@ typedef struct {
     float *out, *out2;
     const float *yprev; /* [B, C, P] */
     const float *bias;  /* [C] or NULL */
-    unsigned char *arg; /* [B, C, M] */
+    const float *add;   /* [B, C, P], may be out itself; IN_ACT to OUT_MASK alone (P % 32 == 0) */
     void *partial;      /* OUT_MASK: doubles [C][slots][2]; tk3d_mlp_product_slots gives slots */
     int32_t B, C, C0, P;
     int32_t group, M;   /* pooled forms: P == group * M, group 32 or 64 */
@@ -81,13 +77,12 @@ int tk3d_mlp_product_f32(int in, int out, const tk3d_mlp_product *p, void *strea
 
 /* Weight gradient: out[r][c] = sum over (b, p) of row(r, p) * colv(c, p), r < R, c < C, in
  * `splits` partial sums [splits][R][C]. Rows: raw x, gradient (a x + b y + d, masked or not),
- * sparse, or activations; columns: raw x or activations. rowsum (NULL or [splits][R]) gets the
+ * or activations; columns: raw x or activations. rowsum (NULL or [splits][R]) gets the
  * sums of the rows themselves. */
 enum {
     TK3D_MLP_ROW_RAW = 0,
     TK3D_MLP_ROW_GRAD = 1,
     TK3D_MLP_ROW_GRAD_OUT = 2,
-    TK3D_MLP_ROW_POOL = 3,
     TK3D_MLP_ROW_ACT = 4,
     TK3D_MLP_COL_RAW = 0,
     TK3D_MLP_COL_ACT = 1
@@ -96,7 +91,7 @@ typedef struct {
     tk3d_mlp_source row, col; /* K = R and C; weights unused */
     tk3d_mlp_norm row_norm, col_norm;
     float *partial, *rowsum;
-    int32_t B, P, group, M;
+    int32_t B, P;
 } tk3d_mlp_outer;
 int tk3d_mlp_outer_splits(const tk3d_mlp_outer *p);
 int tk3d_mlp_outer_f32(int row, int col, const tk3d_mlp_outer *p, void *stream);
@@ -117,10 +112,10 @@ int tk3d_mlp_pool_max_f32(const float *z, const float *y, int64_t groups, int si
                           float *extreme, unsigned char *arg, void *stream);
 
 /* (a, b, d) per channel from the partial sums of (e, e (y - mean)), and dgamma, dbeta.
- * frozen: the statistics are constants (evaluation mode), b = d = 0. */
+ */
 int tk3d_mlp_grad_coefficients_f32(const void *partial, int slots, int64_t n, int C,
-                                   const tk3d_mlp_norm *norm, int frozen, float *coef,
-                                   float *dgamma, float *dbeta, void *stream);
+                                   const tk3d_mlp_norm *norm, float *coef, float *dgamma,
+                                   float *dbeta, void *stream);
 
 /* Partial sums of (e, e (y - mean)) with e = g masked by relu(norm(y)); g, y [B, C, P].
  * slots of tk3d_mlp_mask_slots. */
@@ -136,10 +131,18 @@ int tk3d_mlp_grad_apply_f32(float *e, const float *y, const float *coef, int B, 
                             void *stream);
 
 /* Backward of a pooled layer, before the products: from g [B,C,M], the extremes and their places
- * the coefficients, dgamma, dbeta and sel (see tk3d_mlp_source); positions = B * group * M. */
+ * the coefficients, dgamma, dbeta and sel, [B, C, M] of (float a e, int32 place in the group);
+ * positions = B * group * M. */
 int tk3d_mlp_pool_grad_f32(const float *g, const float *extreme, const unsigned char *arg, int B,
-                           int C, int M, int64_t positions, const tk3d_mlp_norm *norm, int frozen,
+                           int C, int M, int64_t positions, const tk3d_mlp_norm *norm,
                            void *sel, float *coef, float *dgamma, float *dbeta, void *stream);
+/* The sparse half of W^T dy, [B, I, M * group] (groups of 32 or 64; W [O][I]), and that of dW in
+ * partial sums [splits][O][I] (y [B, I, M * group], norm of y). */
+int tk3d_mlp_pool_scatter_f32(const void *sel, const float *w, int B, int O, int I, int M, int group,
+                              float *out, void *stream);
+int tk3d_mlp_pool_outer_splits(int B, int O, int I, int M);
+int tk3d_mlp_pool_outer_f32(const void *sel, const float *y, const tk3d_mlp_norm *norm, int B, int O,
+                            int I, int M, int group, float *partial, void *stream);
 /* gram[k][c] = sum_o W[o][k] b[o] W[o][c] and bias[c] = sum_o W[o][c] d[o]; W [O][I]. */
 int tk3d_mlp_pool_gram_f32(const float *w, const float *coef, int O, int I, float *gram, float *bias,
                            void *stream);
@@ -160,8 +163,8 @@ int tk3d_mlp_group_f32(const float *u, const float *xyz, const float *centre, co
  * over the K neighbours: y(i, k) = W1 (x_j - x_i) + W2 x_i = u_j + v_i, j = index[b, i, k] (x_j = 0
  * for an index outside [0,N)), where w = [W1 W2], u = W1 x and v = (W2 - W1) x; uv [B, N, 2 O] is
  * the product of x with the [2 O][C] matrix that tk3d_mlp_edge_weights_f32 makes of w. Forward:
- * extreme and arg [B, O, N] as in pooled layers (either may be NULL), sum [B, N, O] of the u of a
- * point's neighbours (or NULL). tk3d_mlp_edge_features_f32 makes the edge features themselves,
+ * the extreme of y [B, O, N] (or NULL) and the sum [B, N, O] of the u of a point's neighbours (or
+ * NULL). tk3d_mlp_edge_features_f32 makes the edge features themselves,
  * [B, 2 C, N, K]. Backward: lists is the inverse of the graph
  * (int32 [B][N + 1 + N K]), sel a buffer of B N O 8-byte elements, duv [B, 2 O, N] the gradients
  * of u and v. tk3d_mlp_edge_supported: the sizes these take (N <= 32768, K <= 255). */
@@ -170,8 +173,7 @@ int tk3d_mlp_edge_weights_f32(const float *w, int O, int C, float *out, void *st
 int tk3d_mlp_edge_features_f32(const float *x, const int64_t *index, int B, int C, int N, int K,
                                float *out, void *stream);
 int tk3d_mlp_edge_forward_f32(const float *uv, const int64_t *index, const float *gamma, int B, int N,
-                              int K, int O, float *extreme, unsigned char *arg, float *sum,
-                              void *stream);
+                              int K, int O, float *extreme, float *sum, void *stream);
 int tk3d_mlp_edge_lists(const int64_t *index, int B, int N, int K, int32_t *lists, void *stream);
 int tk3d_mlp_edge_backward_f32(const float *g, const float *extreme, const unsigned char *arg,
                                const float *uv, const float *sum, const int32_t *lists, int B, int N,

@@ -29,11 +29,9 @@ __global__ void __launch_bounds__(kBlock) edge_weights_kernel(const float *w, in
 __global__ void __launch_bounds__(kBlock)
     edge_forward_kernel(const float *__restrict__ uv, const int64_t *__restrict__ index,
                         const float *__restrict__ gamma, int B, int N, int K, int O, int total,
-                        float *__restrict__ extreme, unsigned char *__restrict__ arg,
-                        float *__restrict__ sum)
+                        float *__restrict__ extreme, float *__restrict__ sum)
 {
     __shared__ float values[kChannels][kPoints + 1];
-    __shared__ unsigned char places[kChannels][kPoints];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int cbase = blockIdx.y * kChannels;
     const int c = cbase + lane < O ? cbase + lane : O - 1;
@@ -48,7 +46,6 @@ __global__ void __launch_bounds__(kBlock)
             const int64_t *row = index + ((int64_t)b * N + i) * K;
             const float v = u[(int64_t)i * 2 * O + O];
             float best = 0.0f, chosen = 0.0f, total_u = 0.0f;
-            int where = 0;
             for (int k0 = 0; k0 < K; k0 += kAtOnce) {
                 float r[kAtOnce];
 #pragma unroll
@@ -67,11 +64,9 @@ __global__ void __launch_bounds__(kBlock)
                     const bool up = k0 + k == 0 || (!(s <= best) && best == best);
                     best = up ? s : best;
                     chosen = up ? y : chosen;
-                    where = up ? k0 + k : where;
                 }
             }
             values[lane][local] = chosen;
-            places[lane][local] = (unsigned char)where;
             if (sum && cbase + lane < O)
                 sum[((int64_t)b * N + i) * O + c] = total_u;
         }
@@ -83,8 +78,6 @@ __global__ void __launch_bounds__(kBlock)
             if (cbase + ch < O && first + p < N) {
                 const int64_t at = ((int64_t)b * O + cbase + ch) * N + first + p;
                 extreme[at] = values[ch][p];
-                if (arg)
-                    arg[at] = places[ch][p];
             }
         }
         __syncthreads();
@@ -305,8 +298,7 @@ int tk3d_mlp_edge_features_f32(const float *x, const int64_t *index, int B, int 
 }
 
 int tk3d_mlp_edge_forward_f32(const float *uv, const int64_t *index, const float *gamma, int B, int N,
-                              int K, int O, float *extreme, unsigned char *arg, float *sum,
-                              void *stream)
+                              int K, int O, float *extreme, float *sum, void *stream)
 {
     if (!tk3d_mlp_edge_supported(B, N, K, O))
         return TK3D_ERR_UNSUPPORTED;
@@ -314,7 +306,7 @@ int tk3d_mlp_edge_forward_f32(const float *uv, const int64_t *index, const float
     const int most = 4 * tk_cu_count() / B * B;  // (whole rounds of the batch)
     const int blocks = tiles < most || most == 0 ? tiles : most;
     edge_forward_kernel<<<dim3(blocks, (O + kChannels - 1) / kChannels), kBlock, 0, (hipStream_t)stream>>>(
-        uv, index, gamma, B, N, K, O, tiles, extreme, arg, sum);
+        uv, index, gamma, B, N, K, O, tiles, extreme, sum);
     return tk_launch_status();
 }
 

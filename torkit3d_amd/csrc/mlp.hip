@@ -33,13 +33,11 @@ enum Input {      // in(k, p)
     IN_ACT,       // relu(norm(x))
     IN_GRAD,      // a e + b y + d: gradient before the norm from the gradient behind it (e)
     IN_GRAD_OUT,  // the same where e = g masked by the ReLU still has to be formed from g and y
-    IN_POOL,      // sparse gradient of a maximum, then relu(norm(x)) (see pooled layers below)
 };
 enum Output {
     OUT_PLAIN,      // store, in two tensors if asked for
     OUT_POINTS,     // store as [B, P, C]
     OUT_EVAL,       // store relu(norm(out))
-    OUT_POOL,       // store the extreme over each group and where it is
     OUT_POOL_EVAL,  // store relu(norm(extreme over each group))
     OUT_MASK,       // store out masked by the ReLU in front of it, with the sums of its gradient
 };
@@ -73,7 +71,6 @@ template <int IN, int PT> struct Rows {  // groups of eight input channels of a 
     static constexpr int D = kDepth<PT>;
     float x[D][4][PT];
     float y[reads_y(IN) ? D : 1][4][PT];
-    int2 sel[IN == IN_POOL ? D : 1][4];
 };
 
 struct GemmArgs {
@@ -103,8 +100,8 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
         act_coef = grad_coef + (size_t)a.kg * 8;
     float *weights = reinterpret_cast<float *>(lds + a.coef_bytes);  // [CT][chunk][64][4]
 
-    if constexpr (IN == IN_ACT || IN == IN_POOL || IN == IN_GRAD_OUT) {
-        const int K = IN == IN_POOL ? p.src[1].K : p.src[0].K;
+    if constexpr (IN == IN_ACT || IN == IN_GRAD_OUT) {
+        const int K = p.src[0].K;
         for (int k = tid; k < ((K + 7) & ~7); k += kBlock)
             act_coef[k] = k < K ? constants_of(p.in_norm, k) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     }
@@ -146,19 +143,9 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
     // Rows of the channel groups of a step for the positions of a wave tile.
     constexpr int D = kDepth<PT>;
     const auto load_group = [&](Rows<IN, PT> &r, int d, int b, int pos, int g) {
-        const bool second = (IN == IN_RAW2 || IN == IN_POOL) && g >= a.kg0;
+        const bool second = IN == IN_RAW2 && g >= a.kg0;
         const tk3d_mlp_source &s = p.src[second ? 1 : 0];
         const int k0 = (g - (second ? a.kg0 : 0)) * 8 + half;
-        if (IN == IN_POOL && !second) {
-            const int m = pos / p.group;
-            const int2 *sel = reinterpret_cast<const int2 *>(s.sel) + (int64_t)b * s.K * p.M;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int k = k0 + 2 * q < s.K ? k0 + 2 * q : s.K - 1;
-                r.sel[IN == IN_POOL ? d : 0][q] = sel[(unsigned)k * (unsigned)p.M + (unsigned)m];
-            }
-            return;
-        }
         const float *x = s.x + (int64_t)b * s.batch_stride;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
@@ -191,48 +178,34 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
     };
 
     const auto multiply_group = [&](const Rows<IN, PT> &r, int d, int tile, int g, int first) {
-        const bool second = (IN == IN_RAW2 || IN == IN_POOL) && g >= a.kg0;
+        const bool second = IN == IN_RAW2 && g >= a.kg0;
         const int K = p.src[second ? 1 : 0].K, gs = g - (second ? a.kg0 : 0);
         const int k0 = gs * 8 + half;
         float v[4][PT];
-        if (IN == IN_POOL && !second) {
-            const int b = tile / a.tiles;
-            int pos = (tile - b * a.tiles) * (32 * PT) + PT * col;
-            pos = pos > P - PT ? P - PT : pos;
-            const int kk = pos - pos / p.group * p.group;
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int2 sel = r.sel[IN == IN_POOL ? d : 0][q];
+        for (int q = 0; q < 4; ++q) {
+            if constexpr (reads_y(IN)) {
+                const f32x4 c = grad_coef[k0 + 2 * q];
+                f32x4 ss{0.0f, 0.0f, 0.0f, 0.0f};
+                if constexpr (IN == IN_GRAD_OUT)
+                    ss = act_coef[k0 + 2 * q];
+#pragma unroll
+                for (int t = 0; t < PT; ++t) {
+                    float e = r.x[d][q][t];
+                    const float y = r.y[reads_y(IN) ? d : 0][q][t];
+                    if constexpr (IN == IN_GRAD_OUT)
+                        e = passes(normalised(y, ss)) ? e : 0.0f;
+                    v[q][t] = __builtin_fmaf(c.x, e, __builtin_fmaf(c.y, y, c.z));
+                }
+            } else if constexpr (IN == IN_ACT) {
+                const f32x4 c = act_coef[k0 + 2 * q];
 #pragma unroll
                 for (int t = 0; t < PT; ++t)
-                    v[q][t] = sel.y == kk + t ? __int_as_float(sel.x) : 0.0f;
-            }
-        } else {
+                    v[q][t] = relu(normalised(r.x[d][q][t], c));
+            } else {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                if constexpr (reads_y(IN)) {
-                    const f32x4 c = grad_coef[k0 + 2 * q];
-                    f32x4 ss{0.0f, 0.0f, 0.0f, 0.0f};
-                    if constexpr (IN == IN_GRAD_OUT)
-                        ss = act_coef[k0 + 2 * q];
-#pragma unroll
-                    for (int t = 0; t < PT; ++t) {
-                        float e = r.x[d][q][t];
-                        const float y = r.y[reads_y(IN) ? d : 0][q][t];
-                        if constexpr (IN == IN_GRAD_OUT)
-                            e = passes(normalised(y, ss)) ? e : 0.0f;
-                        v[q][t] = __builtin_fmaf(c.x, e, __builtin_fmaf(c.y, y, c.z));
-                    }
-                } else if constexpr (IN == IN_ACT || IN == IN_POOL) {
-                    const f32x4 c = act_coef[k0 + 2 * q];
-#pragma unroll
-                    for (int t = 0; t < PT; ++t)
-                        v[q][t] = relu(normalised(r.x[d][q][t], c));
-                } else {
-#pragma unroll
-                    for (int t = 0; t < PT; ++t)
-                        v[q][t] = r.x[d][q][t];
-                }
+                for (int t = 0; t < PT; ++t)
+                    v[q][t] = r.x[d][q][t];
             }
         }
         if (gs * 8 + 8 > K) {  // channels past the last one (their weights are zero) must not be inf
@@ -275,9 +248,8 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
         sum1[ct] = sum2[ct] = shift[ct] = 0.0f;
         if constexpr (OUT == OUT_EVAL || OUT == OUT_POOL_EVAL || OUT == OUT_MASK)
             out_coef[ct] = constants_of(p.out_norm, c);
-        if constexpr (OUT == OUT_POOL || OUT == OUT_POOL_EVAL) {
+        if constexpr (OUT == OUT_POOL_EVAL)
             sign[ct] = sign_of(p.out_norm.gamma[c]);
-        }
         if constexpr (OUT == OUT_MASK) {
             shift[ct] = p.out_norm.mean[c];
             bias[ct] = p.bias ? p.bias[c] : 0.0f;
@@ -303,8 +275,8 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
                 const int rows = first ? p.C0 : p.C - p.C0, r = first ? c : c - p.C0;
                 row = mine && out ? out + ((int64_t)b * rows + r) * P : nullptr;
             }
-            float best = 0.0f, first_y = 0.0f;
-            int where = -1;
+            float best = 0.0f;
+            bool fresh = true;
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const int pos = base + PT * (8 * q + 4 * half);
@@ -335,6 +307,17 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
 #pragma unroll
                         for (int i = 0; i < RUN; ++i)
                             before[OUT == OUT_MASK ? i : 0] = yrow[pos + i > P - 1 ? P - 1 : pos + i];
+                    }
+                    if constexpr (IN == IN_ACT) {  // (P is a multiple of 32 here)
+                        const float *arow = p.add + ((int64_t)b * p.C + (mine ? c : p.C - 1)) * P;
+#pragma unroll
+                        for (int i = 0; i < PT; ++i) {
+                            const int at = pos + 4 * i > P - 4 ? P - 4 : pos + 4 * i;
+                            const f32x4 w = *reinterpret_cast<const f32x4 *>(arow + at);
+#pragma unroll
+                            for (int j = 0; j < 4; ++j)
+                                v[4 * i + j] += w[j];
+                        }
                     }
 #pragma unroll
                     for (int i = 0; i < RUN; ++i) {
@@ -377,48 +360,21 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
                         if (mine && pos + i < P)
                             p.out[((int64_t)b * P + pos + i) * p.C + c] = v[i];
                 } else {
-                    // A group is both halves of one q or of several; the positions of a run and
-                    // the q come in ascending order, so the first of equal values stays.
+                    // A group is both halves of one q or of several.
 #pragma unroll
                     for (int i = 0; i < RUN; ++i) {
                         const float s = v[i] * sign[ct];
-                        if constexpr (OUT == OUT_POOL) {
-                            // (the first NaN stays, as in torch's maximum)
-                            const bool up = where < 0 || (!(s <= best) && best == best);
-                            if (i == 0)
-                                first_y = where < 0 ? v[0] : first_y;
-                            best = up ? s : best;
-                            where = up ? pos + i : where;
-                        } else {
-                            best = where < 0 ? s : __builtin_elementwise_maximum(best, s);
-                            where = 0;
-                        }
+                        best = fresh ? s : __builtin_elementwise_maximum(best, s);
+                        fresh = false;
                     }
                     const int qs = p.group / (2 * RUN);
                     if (((q + 1) & (qs - 1)) == 0) {
-                        const float other = __shfl_xor(best, 32);
-                        if constexpr (OUT == OUT_POOL) {
-                            const int at = __shfl_xor(where, 32);
-                            const bool up = other != other
-                                ? best == best || at < where
-                                : other > best || (other == best && at < where);
-                            best = up ? other : best;
-                            where = up ? at : where;
-                        } else {
-                            best = __builtin_elementwise_maximum(best, other);
-                        }
+                        best = __builtin_elementwise_maximum(best, __shfl_xor(best, 32));
                         const int m = pos / p.group;
-                        if (mine && half == 0 && pos < P) {
-                            const int64_t at = ((int64_t)b * p.C + c) * p.M + m;
-                            if constexpr (OUT == OUT_POOL) {
-                                // (a zero gamma makes all values equal: the first one's place)
-                                p.out[at] = sign[ct] == 0.0f && best == best ? first_y : best * sign[ct];
-                                p.arg[at] = (unsigned char)(where - m * p.group);
-                            } else {
-                                p.out[at] = relu(normalised(sign[ct] == 0.0f ? best : best * sign[ct], out_coef[ct]));
-                            }
-                        }
-                        where = -1;
+                        if (mine && half == 0 && pos < P)
+                            p.out[((int64_t)b * p.C + c) * p.M + m] = relu(
+                                normalised(sign[ct] == 0.0f ? best : best * sign[ct], out_coef[ct]));
+                        fresh = true;
                     }
                 }
             }
@@ -547,7 +503,6 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_outer_kernel(OuterArgs a)
 
     struct Part {
         float x[TA][8], y[kGrad ? TA : 1][8], c[TB][8];
-        int2 sel[TA];
     };
     const auto run8 = [&](float (&dst)[8], const float *row, int pos) {
         if (vec) {
@@ -570,15 +525,10 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_outer_kernel(OuterArgs a)
         const int pos = (unit - b * a.units) * 32 + half * 16 + sub * 8;
 #pragma unroll
         for (int t = 0; t < TA; ++t) {
-            if constexpr (ROW == TK3D_MLP_ROW_POOL) {
-                const int m = (pos > P - 8 ? P - 8 : pos) / p.group;
-                q.sel[t] = reinterpret_cast<const int2 *>(p.row.sel)[((int64_t)b * R + r[t]) * p.M + m];
-            } else {
-                const int64_t row = (int64_t)b * p.row.batch_stride + (int64_t)r[t] * P;
-                run8(q.x[t], p.row.x + row, pos);
-                if constexpr (kGrad)
-                    run8(q.y[kGrad ? t : 0], p.row.y + row, pos);
-            }
+            const int64_t row = (int64_t)b * p.row.batch_stride + (int64_t)r[t] * P;
+            run8(q.x[t], p.row.x + row, pos);
+            if constexpr (kGrad)
+                run8(q.y[kGrad ? t : 0], p.row.y + row, pos);
         }
 #pragma unroll
         for (int t = 0; t < TB; ++t)
@@ -603,10 +553,7 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_outer_kernel(OuterArgs a)
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 float v;
-                if constexpr (ROW == TK3D_MLP_ROW_POOL) {
-                    const int kk = pos - pos / p.group * p.group;
-                    v = q.sel[t].y == kk + i ? __int_as_float(q.sel[t].x) : 0.0f;
-                } else if constexpr (kGrad) {
+                if constexpr (kGrad) {
                     float e = q.x[t][i];
                     const float yy = q.y[kGrad ? t : 0][i];
                     if constexpr (ROW == TK3D_MLP_ROW_GRAD_OUT)
@@ -766,25 +713,25 @@ struct Coefficients {
 };
 
 __device__ __forceinline__ Coefficients grad_coefficients(double2 s, double n, const tk3d_mlp_norm &norm,
-                                                          int c, int frozen)
+                                                          int c)
 {
     const double is = norm.eps < 0.0f ? (double)norm.var[c]
                                       : 1.0 / __builtin_sqrt((double)norm.var[c] + (double)norm.eps);
     const double gamma = norm.gamma[c], mean = norm.mean[c];
-    const double b = frozen ? 0.0 : -gamma * is * is * is * s.y / n;
-    const double d = frozen ? 0.0 : -gamma * is * s.x / n - b * mean;
+    const double b = -gamma * is * is * is * s.y / n;
+    const double d = -gamma * is * s.x / n - b * mean;
     return {f32x4{(float)(gamma * is), (float)b, (float)d, 0.0f}, (float)(s.y * is), (float)s.x};
 }
 
 __global__ void __launch_bounds__(kBlock)
     mlp_grad_coefficients_kernel(const void *partial, int slots, double n, tk3d_mlp_norm norm,
-                                 int frozen, float *coef, float *dgamma, float *dbeta)
+                                 float *coef, float *dgamma, float *dbeta)
 {
     __shared__ double2 lds[kWaves];
     const int c = blockIdx.x;
     const double2 s = slot_sum(partial, slots, c, lds);
     if (threadIdx.x == 0) {
-        const Coefficients k = grad_coefficients(s, n, norm, c, frozen);
+        const Coefficients k = grad_coefficients(s, n, norm, c);
         reinterpret_cast<f32x4 *>(coef)[c] = k.abd;
         dgamma[c] = k.dgamma;
         dbeta[c] = k.dbeta;
@@ -873,7 +820,7 @@ __global__ void __launch_bounds__(kBlock)
 // One workgroup per channel: the sums, then the coefficients, then the sparse gradient.
 __global__ void __launch_bounds__(1024)
     mlp_pool_grad_kernel(const float *g, const float *extreme, const unsigned char *arg, int B, int C,
-                         int M, double n, tk3d_mlp_norm norm, int frozen, int2 *sel, float *coef,
+                         int M, double n, tk3d_mlp_norm norm, int2 *sel, float *coef,
                          float *dgamma, float *dbeta)
 {
     __shared__ double2 lds[16];
@@ -893,7 +840,7 @@ __global__ void __launch_bounds__(1024)
         v.x += e;
         v.y += (double)e * (double)(y - mean);
     }
-    const Coefficients k = grad_coefficients(block_sum(v, lds), n, norm, c, frozen);
+    const Coefficients k = grad_coefficients(block_sum(v, lds), n, norm, c);
     if (threadIdx.x == 0) {
         reinterpret_cast<f32x4 *>(coef)[c] = k.abd;
         dgamma[c] = k.dgamma;
@@ -903,6 +850,157 @@ __global__ void __launch_bounds__(1024)
         const int64_t j = at(i);
         const float e = passes(normalised(extreme[j], ss)) ? g[j] : 0.0f;
         sel[j] = int2{__float_as_int(k.abd.x * e), (int)arg[j]};
+    }
+}
+
+// The sparse halves. In a group of S positions a channel o has one value a e, at one place, so that
+// W^T (a e) and (a e) x^T take O x I operations a group. As products over all positions (matrix cores,
+// zeros among the rows) they took S times as many: on 16 x 512 groups of 32, O = 128, I = 64, both
+// halves of W^T dy in one product 174 us, (a e) x^T 78 us; now 46 and 72 (the product), and 31 us. A
+// wave has a group, lanes are input channels, the places are scalars, and the group's tile of S x 64
+// lies in LDS (rows of 65: read by channels and by positions).
+
+constexpr int kRow = 65;
+
+__device__ __forceinline__ float scalar_of(float v, int lane)
+{
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+
+struct SparseArgs {
+    const int2 *sel;       // [B, O, M]
+    const float *w;        // [O][I] (scatter)
+    const float *y;        // [B, I, P] (outer)
+    tk3d_mlp_norm norm;    // of y
+    float *out;            // [B, I, P] (scatter), partial sums [splits][O][I] (outer)
+    int O, I, M, run;      // a wave takes `run` consecutive groups at once
+    int units, total;      // runs: per batch element, in all
+};
+
+// out[b, i, (m, place)] = sum over o of w[o][i] a e; zero at the other places. A
+// lane adds to a column of its own, in the order of o: 12 to 16 waves a CU cover the trips to LDS (as LDS
+// atomics, without the trips, the additions took 341 us for 42 on 16 x 512 groups of 32).
+template <int S>
+__global__ void __launch_bounds__(kBlock) mlp_pool_scatter_kernel(SparseArgs a)
+{
+    extern __shared__ float tiles[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    float *tile = tiles + wave * (S * kRow);
+    const int i0 = blockIdx.y * 64, c = i0 + lane < a.I ? i0 + lane : a.I - 1;
+    const int p = lane & (S - 1), first = lane / S;  // of the loop over positions
+    for (int unit = blockIdx.x * kWaves + wave; unit < a.total; unit += gridDim.x * kWaves) {
+        const int b = unit / a.units, from = (unit - b * a.units) * a.run;
+        const int to = from + a.run < a.M ? from + a.run : a.M;
+        for (int m = from; m < to; ++m) {
+#pragma unroll 8
+            for (int q = 0; q < S; ++q)
+                tile[q * kRow + lane] = 0.0f;
+            for (int o0 = 0; o0 < a.O; o0 += 64) {
+                const int o = o0 + lane < a.O ? o0 + lane : a.O - 1;
+                const int2 s = a.sel[((int64_t)b * a.O + o) * a.M + m];
+                const float e = o0 + lane < a.O ? __int_as_float(s.x) : 0.0f;
+                const int n = a.O - o0 < 64 ? a.O - o0 : 64;
+                for (int k = 0; k < n; k += 8) {
+                    float w[8];
+#pragma unroll
+                    for (int j = 0; j < 8; ++j)
+                        w[j] = a.w[(int64_t)(o0 + (k + j < n ? k + j : n - 1)) * a.I + c];
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) {  // (lanes from n on: zeros at a place of the tile)
+                        float &at = tiles[wave * (S * kRow) + __builtin_amdgcn_readlane(s.y, k + j) * kRow + lane];
+                        at = __builtin_fmaf(scalar_of(e, k + j), w[j], at);
+                    }
+                }
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            const int64_t P = (int64_t)a.M * S;
+            float *out = a.out + ((int64_t)b * a.I + i0) * P + (int64_t)m * S + p;
+#pragma unroll 8
+            for (int i = first; i < 64; i += 64 / S)
+                if (i0 + i < a.I)
+                    out[i * P] = tile[p * kRow + i];
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
+}
+
+// partial[split][o][i] = sum over groups of a e relu(norm(y[i, (m, place)])): 64 rows and 64 columns
+// a workgroup, rows in registers.
+template <int S>
+__global__ void __launch_bounds__(kBlock) mlp_pool_outer_kernel(SparseArgs a)
+{
+    extern __shared__ float tiles[];
+    __shared__ f32x4 constants[64];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    float *tile = tiles + wave * (S * kRow);
+    const int o0 = blockIdx.y * 64, i0 = blockIdx.z * 64;
+    const int o = o0 + lane < a.O ? o0 + lane : a.O - 1;
+    const int p = lane & (S - 1), first = lane / S;
+    if (tid < 64)
+        constants[tid] = constants_of(a.norm, i0 + tid < a.I ? i0 + tid : a.I - 1);
+    __syncthreads();
+    float acc[64];
+#pragma unroll
+    for (int k = 0; k < 64; ++k)
+        acc[k] = 0.0f;
+    // The values of the next group are requested before the present one's rows are added up.
+    const int64_t P = (int64_t)a.M * S;
+    float v[S];
+    int2 sel{0, 0};
+    const auto load = [&](int b, int m) {
+        sel = a.sel[((int64_t)b * a.O + o) * a.M + m];
+        const float *y = a.y + (int64_t)b * a.I * P + (int64_t)m * S + p;
+#pragma unroll
+        for (int q = 0; q < S; ++q) {
+            const int i = i0 + first + q * (64 / S);
+            v[q] = y[(i < a.I ? i : a.I - 1) * P];
+        }
+    };
+    int unit = blockIdx.x * kWaves + wave, b = unit / a.units, m = (unit - b * a.units) * a.run;
+    bool more = unit < a.total;
+    if (more)
+        load(b, m);
+    while (more) {
+#pragma unroll
+        for (int q = 0; q < S; ++q) {
+            const int i = first + q * (64 / S);
+            tile[p * kRow + i] = relu(normalised(v[q], constants[i]));
+        }
+        const float e = o0 + lane < a.O ? __int_as_float(sel.x) : 0.0f;
+        const int place = sel.y;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        const int to = (unit - b * a.units + 1) * a.run;
+        if (++m >= (to < a.M ? to : a.M)) {
+            unit += gridDim.x * kWaves;
+            b = unit / a.units;
+            m = (unit - b * a.units) * a.run;
+            more = unit < a.total;
+        }
+        if (more)
+            load(b, m);
+#pragma unroll
+        for (int k = 0; k < 64; ++k)
+            acc[k] = __builtin_fmaf(scalar_of(e, k),
+                                    tile[__builtin_amdgcn_readlane(place, k) * kRow + lane], acc[k]);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+    // (one wave after the other: 16 KB, within the tiles of four waves)
+    for (int w = 0; w < kWaves; ++w) {
+        __syncthreads();
+        if (w == wave)
+#pragma unroll
+            for (int k = 0; k < 64; ++k)
+                tiles[k * 64 + lane] = w ? tiles[k * 64 + lane] + acc[k] : acc[k];
+    }
+    __syncthreads();
+    for (int e = tid; e < 64 * 64; e += kBlock) {
+        const int k = e >> 6, i = e & 63;
+        if (o0 + k < a.O && i0 + i < a.I)
+            a.out[((int64_t)blockIdx.x * a.O + o0 + k) * a.I + i0 + i] = tiles[e];
     }
 }
 
@@ -1101,6 +1199,15 @@ __global__ void __launch_bounds__(kBlock)
 
 // ---- launches ------------------------------------------------------------------------------------------
 
+// Runs of four groups read whole sectors of sel ([B, O, M]), as long as every SIMD keeps a wave.
+void fill_sparse(SparseArgs &a, int B)
+{
+    a.run = (int64_t)B * a.M >= 16 * tk_cu_count() ? 4 : 1;
+    a.units = (a.M + a.run - 1) / a.run;
+    a.total = B * a.units;
+}
+int sparse_bytes(int group) { return kWaves * group * kRow * 4; }
+
 constexpr int kWeightBytes = 64 << 10;  // weights in LDS: two workgroups to a CU
 
 struct Shape {
@@ -1108,20 +1215,23 @@ struct Shape {
 };
 
 // The largest wave tile that still gives every SIMD of the chip a wave; 16-byte rows need lengths
-// that are multiples of four, a group of 64 positions needs a tile that holds it.
+// that are multiples of four, a group of 64 positions needs a tile that holds it. A masked gradient
+// reads as much on the way out as on the way in, and waits for it with nothing of its own to do: half
+// the positions a wave leave room for twice the waves (64 -> 64 channels, 16 x 16384 positions:
+// 4 x 2 tiles 116 us, 2 x 2 tiles 72 us; at 32 channels and less there is nothing between).
 Shape pick_shape(int out, const tk3d_mlp_product &p)
 {
     const int simds = 4 * tk_cu_count();
     const auto waves = [&](int pt, int ct) {
         return (int64_t)p.B * ((p.P + 32 * pt - 1) / (32 * pt)) * ((p.C + 32 * ct - 1) / (32 * ct));
     };
-    const bool pooled = out == TK3D_MLP_OUT_POOL || out == TK3D_MLP_OUT_POOL_EVAL;
+    const bool pooled = out == TK3D_MLP_OUT_POOL_EVAL;
     if (p.P % 4 != 0)
         return {1, 1};
     if (p.C <= 32 && waves(4, 1) >= simds)
         return {4, 1};
     if (p.C > 32 && waves(4, 2) >= simds)
-        return {4, 2};
+        return out == TK3D_MLP_OUT_MASK ? Shape{2, 2} : Shape{4, 2};
     if (waves(2, 2) >= simds || (pooled && p.group > 32))
         return {2, 2};
     return {1, 1};
@@ -1132,7 +1242,7 @@ int fill(const tk3d_mlp_product &p, int in, int out, Shape s, GemmArgs &g)
     g.p = p;
     g.tiles = (p.P + 32 * s.pt - 1) / (32 * s.pt);
     g.total = p.B * g.tiles;
-    const bool two = in == TK3D_MLP_IN_RAW2 || in == TK3D_MLP_IN_POOL;
+    const bool two = in == TK3D_MLP_IN_RAW2;
     g.kg0 = (p.src[0].K + 7) / 8;
     g.kg = g.kg0 + (two ? (p.src[1].K + 7) / 8 : 0);
     const int group_bytes = s.ct * 1024;
@@ -1166,8 +1276,9 @@ int launch_product(const GemmArgs &g, int cblocks, hipStream_t stream)
 template <int IN, int OUT>
 int launch_shape(const GemmArgs &g, Shape s, int cblocks, hipStream_t stream)
 {
-    if (s.pt == 4 && s.ct == 2)
-        return launch_product<IN, OUT, 4, 2>(g, cblocks, stream);
+    if constexpr (OUT != OUT_MASK)
+        if (s.pt == 4 && s.ct == 2)
+            return launch_product<IN, OUT, 4, 2>(g, cblocks, stream);
     if (s.pt == 4)
         return launch_product<IN, OUT, 4, 1>(g, cblocks, stream);
     if (s.pt == 2)
@@ -1226,7 +1337,7 @@ int tk3d_mlp_product_f32(int in, int out, const tk3d_mlp_product *p, void *strea
 {
     if (!p)
         return TK3D_ERR_NULL_POINTER;
-    const bool two = in == TK3D_MLP_IN_RAW2 || in == TK3D_MLP_IN_POOL;
+    const bool two = in == TK3D_MLP_IN_RAW2;
     if (p->B < 0 || p->C <= 0 || p->P < 0 || p->src[0].K <= 0 || (two && p->src[1].K <= 0))
         return TK3D_ERR_BAD_SIZE;
     if (p->B == 0 || p->P == 0)
@@ -1234,9 +1345,10 @@ int tk3d_mlp_product_f32(int in, int out, const tk3d_mlp_product *p, void *strea
     const int widest = two && p->src[1].K > p->src[0].K ? p->src[1].K : p->src[0].K;
     if (!indexable(widest, p->P) || !indexable(p->C, p->P) || p->C > 65535 * 32)
         return TK3D_ERR_UNSUPPORTED;
-    const bool grouped = in == TK3D_MLP_IN_POOL || out == TK3D_MLP_OUT_POOL || out == TK3D_MLP_OUT_POOL_EVAL;
-    if (grouped && ((p->group != 32 && p->group != 64) || p->M * p->group != p->P))
+    if (out == TK3D_MLP_OUT_POOL_EVAL && ((p->group != 32 && p->group != 64) || p->M * p->group != p->P))
         return TK3D_ERR_UNSUPPORTED;
+    if (in == TK3D_MLP_IN_ACT && out == TK3D_MLP_OUT_MASK && (!p->add || p->P % 32 != 0))
+        return TK3D_ERR_BAD_SIZE;
     const Shape s = pick_shape(out, *p);
     GemmArgs g;
     const int cblocks = fill(*p, in, out, s, g);
@@ -1246,17 +1358,14 @@ int tk3d_mlp_product_f32(int in, int out, const tk3d_mlp_product *p, void *strea
     TK_CASE(IN_RAW, OUT_PLAIN)
     TK_CASE(IN_RAW, OUT_POINTS)
     TK_CASE(IN_RAW, OUT_POOL_EVAL)
-    TK_CASE(IN_RAW2, OUT_PLAIN)
     TK_CASE(IN_RAW2, OUT_EVAL)
-    TK_CASE(IN_ACT, OUT_PLAIN)
     TK_CASE(IN_ACT, OUT_EVAL)
-    TK_CASE(IN_ACT, OUT_POOL)
     TK_CASE(IN_ACT, OUT_POOL_EVAL)
     TK_CASE(IN_GRAD, OUT_MASK)
     TK_CASE(IN_GRAD, OUT_PLAIN)
     TK_CASE(IN_GRAD_OUT, OUT_MASK)
     TK_CASE(IN_GRAD_OUT, OUT_PLAIN)
-    TK_CASE(IN_POOL, OUT_MASK)
+    TK_CASE(IN_ACT, OUT_MASK)
 #undef TK_CASE
     return TK3D_ERR_UNSUPPORTED;
 }
@@ -1281,8 +1390,6 @@ int tk3d_mlp_outer_f32(int row, int col, const tk3d_mlp_outer *p, void *stream_)
         return TK3D_ERR_BAD_SIZE;
     if (!indexable(p->row.K, p->P) || !indexable(p->col.K, p->P))
         return TK3D_ERR_UNSUPPORTED;
-    if (row == TK3D_MLP_ROW_POOL && (p->group % 32 != 0 || p->group * p->M != p->P))
-        return TK3D_ERR_UNSUPPORTED;
     OuterArgs a;
     a.p = *p;
     a.units = (p->P + 31) / 32;
@@ -1295,7 +1402,6 @@ int tk3d_mlp_outer_f32(int row, int col, const tk3d_mlp_outer *p, void *stream_)
     TK_CASE(TK3D_MLP_ROW_GRAD, TK3D_MLP_COL_ACT)
     TK_CASE(TK3D_MLP_ROW_GRAD_OUT, TK3D_MLP_COL_RAW)
     TK_CASE(TK3D_MLP_ROW_GRAD_OUT, TK3D_MLP_COL_ACT)
-    TK_CASE(TK3D_MLP_ROW_POOL, TK3D_MLP_COL_ACT)
     TK_CASE(TK3D_MLP_ROW_ACT, TK3D_MLP_COL_ACT)
 #undef TK_CASE
     return TK3D_ERR_UNSUPPORTED;
@@ -1340,11 +1446,11 @@ int tk3d_mlp_pool_max_f32(const float *z, const float *y, int64_t groups, int si
 }
 
 int tk3d_mlp_grad_coefficients_f32(const void *partial, int slots, int64_t n, int C,
-                                   const tk3d_mlp_norm *norm, int frozen, float *coef,
-                                   float *dgamma, float *dbeta, void *stream)
+                                   const tk3d_mlp_norm *norm, float *coef, float *dgamma,
+                                   float *dbeta, void *stream)
 {
     mlp_grad_coefficients_kernel<<<C, kBlock, 0, (hipStream_t)stream>>>(partial, slots, (double)n, *norm,
-                                                                      frozen, coef, dgamma, dbeta);
+                                                                      coef, dgamma, dbeta);
     return tk_launch_status();
 }
 
@@ -1386,12 +1492,79 @@ int tk3d_mlp_grad_apply_f32(float *e, const float *y, const float *coef, int B, 
 }
 
 int tk3d_mlp_pool_grad_f32(const float *g, const float *extreme, const unsigned char *arg, int B,
-                           int C, int M, int64_t positions, const tk3d_mlp_norm *norm, int frozen,
+                           int C, int M, int64_t positions, const tk3d_mlp_norm *norm,
                            void *sel, float *coef, float *dgamma, float *dbeta, void *stream)
 {
     mlp_pool_grad_kernel<<<C, 1024, 0, (hipStream_t)stream>>>(
-        g, extreme, arg, B, C, M, (double)positions, *norm, frozen, reinterpret_cast<int2 *>(sel), coef,
+        g, extreme, arg, B, C, M, (double)positions, *norm, reinterpret_cast<int2 *>(sel), coef,
         dgamma, dbeta);
+    return tk_launch_status();
+}
+
+int tk3d_mlp_pool_scatter_f32(const void *sel, const float *w, int B, int O, int I, int M, int group,
+                              float *out, void *stream_)
+{
+    if (B <= 0 || O <= 0 || I <= 0 || M <= 0)
+        return TK3D_ERR_BAD_SIZE;
+    if ((group != 32 && group != 64) || !tk_fits(TK_MAX_I32, B, M) || I > 65535 * 64)
+        return TK3D_ERR_UNSUPPORTED;
+    SparseArgs a{};
+    a.sel = reinterpret_cast<const int2 *>(sel);
+    a.w = w;
+    a.out = out;
+    a.O = O;
+    a.I = I;
+    a.M = M;
+    fill_sparse(a, B);
+    const int rc = group == 32 ? tk_allow_dynamic_lds<mlp_pool_scatter_kernel<32>>(sparse_bytes(32))
+                               : tk_allow_dynamic_lds<mlp_pool_scatter_kernel<64>>(sparse_bytes(64));
+    if (rc != TK3D_OK)
+        return rc;
+    const int wgs = (a.total + kWaves - 1) / kWaves, most = 4 * tk_cu_count();
+    const dim3 grid(wgs < most ? wgs : most, (I + 63) / 64);
+    if (group == 32)
+        mlp_pool_scatter_kernel<32><<<grid, kBlock, sparse_bytes(32), (hipStream_t)stream_>>>(a);
+    else
+        mlp_pool_scatter_kernel<64><<<grid, kBlock, sparse_bytes(64), (hipStream_t)stream_>>>(a);
+    return tk_launch_status();
+}
+
+// Two workgroups to a CU, and no more than there are runs for.
+int tk3d_mlp_pool_outer_splits(int B, int O, int I, int M)
+{
+    SparseArgs a{};
+    a.M = M;
+    fill_sparse(a, B);
+    const int blocks = ((O + 63) / 64) * ((I + 63) / 64), wgs = (a.total + kWaves - 1) / kWaves;
+    const int most = (2 * tk_cu_count() + blocks - 1) / blocks;
+    return wgs < most ? wgs : most;
+}
+
+int tk3d_mlp_pool_outer_f32(const void *sel, const float *y, const tk3d_mlp_norm *norm, int B, int O,
+                            int I, int M, int group, float *partial, void *stream_)
+{
+    if (B <= 0 || O <= 0 || I <= 0 || M <= 0)
+        return TK3D_ERR_BAD_SIZE;
+    if ((group != 32 && group != 64) || !tk_fits(TK_MAX_I32, B, M) || I > 65535 * 64 || O > 65535 * 64)
+        return TK3D_ERR_UNSUPPORTED;
+    SparseArgs a{};
+    a.sel = reinterpret_cast<const int2 *>(sel);
+    a.y = y;
+    a.norm = *norm;
+    a.out = partial;
+    a.O = O;
+    a.I = I;
+    a.M = M;
+    fill_sparse(a, B);
+    const int rc = group == 32 ? tk_allow_dynamic_lds<mlp_pool_outer_kernel<32>>(sparse_bytes(32))
+                               : tk_allow_dynamic_lds<mlp_pool_outer_kernel<64>>(sparse_bytes(64));
+    if (rc != TK3D_OK)
+        return rc;
+    const dim3 grid(tk3d_mlp_pool_outer_splits(B, O, I, M), (O + 63) / 64, (I + 63) / 64);
+    if (group == 32)
+        mlp_pool_outer_kernel<32><<<grid, kBlock, sparse_bytes(32), (hipStream_t)stream_>>>(a);
+    else
+        mlp_pool_outer_kernel<64><<<grid, kBlock, sparse_bytes(64), (hipStream_t)stream_>>>(a);
     return tk_launch_status();
 }
 

@@ -212,13 +212,11 @@ struct Normalised {
 };
 
 Normalised stock_layer(const Tensor &h, const Tensor &weight, const Tensor &gamma, const Tensor &beta,
-                       const Tensor &running_mean, const Tensor &running_var, const Tensor &batches,
-                       double momentum, double eps)
+                       const Tensor &running_mean, const Tensor &running_var, double momentum,
+                       double eps)
 {
     Normalised n;
     n.y = h.dim() == 4 ? at::conv2d(h, weight) : at::conv1d(h, weight);
-    if (batches.defined())
-        Tensor(batches).add_(1);
     std::tie(n.z, n.mean, n.inv_std, std::ignore, std::ignore) =
         at::_batch_norm_impl_index(n.y, gamma, beta, running_mean, running_var, true, momentum, eps,
                                    at::globalContext().userEnabledCuDNN());
@@ -260,9 +258,10 @@ Tensor forward_training(const Call &c, Kept &k)
     } else if (c.params[0].dim() == 4) {
         h = h.view({B, h.size(1), c.rows, -1});
     }
+    std::vector<Tensor> counts;  // (one launch for all layers)
     for (int64_t l = 0; l < L; ++l) {
         const Tensor *w = &c.params[3 * l], *s = &c.buffers[3 * l];
-        const Normalised n = stock_layer(h, w[0], w[1], w[2], s[0], s[1], s[2], c.momentum[l], c.eps[l]);
+        const Normalised n = stock_layer(h, w[0], w[1], w[2], s[0], s[1], c.momentum[l], c.eps[l]);
         k.mean.push_back(n.mean);
         k.var.push_back(n.inv_std);
         if (c.pool && l == L - 1) {
@@ -273,59 +272,12 @@ Tensor forward_training(const Call &c, Kept &k)
             h = Tensor(n.z).relu_();
             k.y.push_back(n.y.flatten(2).contiguous());
         }
+        if (s[2].defined())
+            counts.push_back(s[2]);
     }
+    if (!counts.empty())
+        at::_foreach_add_(counts, 1);
     return h;
-}
-
-// Forward in evaluation mode that keeps what the backward needs.
-Tensor forward(const Call &c, Kept &k)
-{
-    const int64_t B = c.batch(), P = c.positions(), L = c.layers();
-    const Tensor like = c.like();
-    void *stream = stream_of(like);
-    for (int64_t l = 0; l < L; ++l) {
-        const int64_t C = c.out_channels(l), K = c.in_channels(l);
-        const float *w = f32(c.weight(l));
-        tk3d_mlp_product p = product(B, C, P);
-        const bool pooled = c.pool && l == L - 1;
-        const Tensor y = at::empty({B, C, pooled ? P / c.pool : P}, like.options());
-        if (l == 0 && c.grouped()) {
-            first_grouped(c, y);
-        } else {
-            int in = TK3D_MLP_IN_ACT, out = TK3D_MLP_OUT_PLAIN;
-            if (l == 0) {
-                in = TK3D_MLP_IN_RAW;
-                p.src[0] = source(c.x, w, 1, K);
-                if (c.x2.defined()) {
-                    in = TK3D_MLP_IN_RAW2;
-                    p.src[1] = source(c.x2, w + c.x.size(1), 1, K);
-                }
-            } else {
-                p.src[0] = source(k.y[l - 1], w, 1, K);
-                p.in_norm = norm_of(c, k, l - 1);
-            }
-            if (pooled) {
-                out = TK3D_MLP_OUT_POOL;
-                p.group = (int32_t)c.pool;
-                p.M = (int32_t)(P / c.pool);
-                p.out_norm.gamma = f32(c.params[3 * l + 1]);
-                k.arg = at::empty({B, C, p.M}, like.options().dtype(at::kByte));
-                p.arg = k.arg.data_ptr<uint8_t>();
-            }
-            p.out = f32(y);
-            run_product(in, out, p, stream);
-        }
-        k.y.push_back(y);
-        k.mean.push_back(c.buffers[3 * l]);
-        k.var.push_back(c.buffers[3 * l + 1]);
-    }
-    const Tensor &last = k.y[L - 1];
-    const Tensor z = at::empty(last.sizes(), like.options());
-    const tk3d_mlp_norm norm = norm_of(c, k, L - 1);
-    done(tk3d_mlp_activate_f32(f32(last), B * last.size(1), (int)last.size(1), (int)last.size(2),
-                               &norm, f32(z), stream),
-         "tk3d_mlp_activate_f32");
-    return z;
 }
 
 struct Grads {
@@ -356,7 +308,6 @@ Grads backward(const Call &c, const Kept &k, const Tensor &g, bool want_x, bool 
     const int64_t B = c.batch(), P = c.positions(), L = c.layers();
     const Tensor like = c.like();
     void *stream = stream_of(like);
-    const int frozen = c.training ? 0 : 1;
     Grads out;
     out.params.resize(3 * L);
     for (int64_t l = 0; l < L; ++l) {
@@ -372,7 +323,7 @@ Grads backward(const Call &c, const Kept &k, const Tensor &g, bool want_x, bool 
     const auto coefficients = [&](int64_t l, const void *partial, int slots) {
         const tk3d_mlp_norm norm = norm_of(c, k, l);
         done(tk3d_mlp_grad_coefficients_f32(partial, slots, B * P, (int)c.out_channels(l), &norm,
-                                            frozen, f32(coef[l]), f32(out.params[3 * l + 1]),
+                                            f32(coef[l]), f32(out.params[3 * l + 1]),
                                             f32(out.params[3 * l + 2]), stream),
              "tk3d_mlp_grad_coefficients_f32");
     };
@@ -385,7 +336,7 @@ Grads backward(const Call &c, const Kept &k, const Tensor &g, bool want_x, bool 
         const tk3d_mlp_norm norm = norm_of(c, k, l), inner = norm_of(c, k, l - 1);
         const Tensor sel = at::empty({B, O, M, 2}, like.options());
         done(tk3d_mlp_pool_grad_f32(f32(g), f32(k.y[l]), k.arg.data_ptr<uint8_t>(), (int)B, (int)O,
-                                    (int)M, B * P, &norm, frozen, sel.data_ptr(), f32(coef[l]),
+                                    (int)M, B * P, &norm, sel.data_ptr(), f32(coef[l]),
                                     f32(out.params[3 * l + 1]), f32(out.params[3 * l + 2]), stream),
              "tk3d_mlp_pool_grad_f32");
         const Tensor gram = at::empty({I + 1, I}, like.options());
@@ -393,35 +344,28 @@ Grads backward(const Call &c, const Kept &k, const Tensor &g, bool want_x, bool 
         done(tk3d_mlp_pool_gram_f32(w, f32(coef[l]), (int)O, (int)I, f32(gram), f32(gram) + I * I,
                                     stream),
              "tk3d_mlp_pool_gram_f32");
+        e = at::empty({B, I, P}, like.options());
+        done(tk3d_mlp_pool_scatter_f32(sel.data_ptr(), w, (int)B, (int)O, (int)I, (int)M, (int)c.pool,
+                                       f32(e), stream),
+             "tk3d_mlp_pool_scatter_f32");
         tk3d_mlp_product p = product(B, I, P);
-        p.group = (int32_t)c.pool;
-        p.M = (int32_t)M;
-        p.src[0].sel = sel.data_ptr();
-        p.src[0].K = (int32_t)O;
-        p.src[0].w = w;
-        p.src[0].wk = (int32_t)I;
-        p.src[0].wc = 1;
-        p.src[1] = source(k.y[l - 1], f32(gram), I, 1);
+        p.src[0] = source(k.y[l - 1], f32(gram), I, 1);
         p.in_norm = p.out_norm = inner;
         p.yprev = f32(k.y[l - 1]);
         p.bias = f32(gram) + I * I;
-        e = at::empty({B, I, P}, like.options());
-        p.out = f32(e);
-        const auto sums = summed_product(TK3D_MLP_IN_POOL, TK3D_MLP_OUT_MASK, p, like, stream);
+        p.add = p.out = f32(e);
+        const auto sums = summed_product(TK3D_MLP_IN_ACT, TK3D_MLP_OUT_MASK, p, like, stream);
 
+        const int sparse_splits = tk3d_mlp_pool_outer_splits((int)B, (int)O, (int)I, (int)M);
+        const Tensor sparse = at::empty({sparse_splits, O, I}, like.options());
+        done(tk3d_mlp_pool_outer_f32(sel.data_ptr(), f32(k.y[l - 1]), &inner, (int)B, (int)O, (int)I,
+                                     (int)M, (int)c.pool, f32(sparse), stream),
+             "tk3d_mlp_pool_outer_f32");
         tk3d_mlp_outer o{};
         o.B = (int32_t)B;
         o.P = (int32_t)P;
-        o.group = p.group;
-        o.M = p.M;
         o.col = source(k.y[l - 1], nullptr, 0, 0);
         o.col_norm = o.row_norm = inner;
-        o.row.K = (int32_t)O;
-        o.row.sel = sel.data_ptr();
-        const int sparse_splits = tk3d_mlp_outer_splits(&o);
-        const Tensor sparse = at::empty({sparse_splits, O, I}, like.options());
-        o.partial = f32(sparse);
-        done(tk3d_mlp_outer_f32(TK3D_MLP_ROW_POOL, TK3D_MLP_COL_ACT, &o, stream), "tk3d_mlp_outer_f32");
         o.row = o.col;
         const int splits = tk3d_mlp_outer_splits(&o);
         const Tensor xx = at::empty({splits, I, I}, like.options());
@@ -586,7 +530,7 @@ struct Node : torch::autograd::Function<Node> {
                           const std::optional<Tensor> &x2, at::TensorList params, const Call &call)
     {
         Kept k;
-        const Tensor z = call.training ? forward_training(call, k) : tk3d::forward(call, k);
+        const Tensor z = forward_training(call, k);
         variable_list saved = {call.x, call.x2, call.xyz, call.centre, call.index, k.arg};
         for (int64_t l = 0; l < call.layers(); ++l) {
             for (int64_t i = 0; i < 3; ++i)
@@ -695,7 +639,7 @@ tk3d_mlp_norm norm_of(const EdgeCall &c, const EdgeKept &k)
     return {f32(k.mean), f32(k.var), f32(c.gamma), f32(c.beta), c.training ? -1.0f : (float)c.eps};
 }
 
-Tensor edge_forward(const EdgeCall &c, EdgeKept &k, bool keep)
+Tensor edge_forward(const EdgeCall &c, EdgeKept &k)
 {
     const int64_t B = c.batch(), N = c.points(), K = c.neighbours(), O = c.out_channels();
     const int64_t C = c.x.size(1);
@@ -709,19 +653,15 @@ Tensor edge_forward(const EdgeCall &c, EdgeKept &k, bool keep)
     p.src[0] = source(c.x, f32(k.matrix), 1, C);
     p.out = f32(k.uv);
     run_product(TK3D_MLP_IN_RAW, TK3D_MLP_OUT_POINTS, p, stream);
-    if (keep)
+    if (c.training)
         k.sum = at::empty({B, N, O}, options);
     if (!c.training) {
         k.extreme = at::empty({B, O, N}, options);
-        if (keep)
-            k.arg = at::empty({B, O, N}, options.dtype(at::kByte));
         k.mean = c.running_mean;
         k.var = c.running_var;
     }
     done(tk3d_mlp_edge_forward_f32(f32(k.uv), c.index.data_ptr<int64_t>(), f32(c.gamma), (int)B,
-                                   (int)N, (int)K, (int)O, f32(k.extreme),
-                                   k.arg.defined() ? k.arg.data_ptr<uint8_t>() : nullptr, f32(k.sum),
-                                   stream),
+                                   (int)N, (int)K, (int)O, f32(k.extreme), f32(k.sum), stream),
          "tk3d_mlp_edge_forward_f32");
     if (c.training) {  // (bit by bit what the stock modules give, see forward_training)
         const Tensor edges = at::empty({B, 2 * C, N, K}, options);
@@ -729,7 +669,9 @@ Tensor edge_forward(const EdgeCall &c, EdgeKept &k, bool keep)
                                         (int)K, f32(edges), stream),
              "tk3d_mlp_edge_features_f32");
         const Normalised n = stock_layer(edges, c.weight, c.gamma, c.beta, c.running_mean,
-                                         c.running_var, c.batches, c.momentum, c.eps);
+                                         c.running_var, c.momentum, c.eps);
+        if (c.batches.defined())
+            Tensor(c.batches).add_(1);
         k.mean = n.mean;
         k.var = n.inv_std;
         return pool_max(n, k.extreme, k.arg);
@@ -755,8 +697,7 @@ variable_list edge_backward(const EdgeCall &c, const EdgeKept &k, const Tensor &
                                 partial.data_ptr(), stream),
          "tk3d_mlp_mask_sums_f32");
     done(tk3d_mlp_grad_coefficients_f32(partial.data_ptr(), slots, B * N * K, (int)O, &norm,
-                                        c.training ? 0 : 1, f32(coef), f32(affine), f32(affine) + O,
-                                        stream),
+                                        f32(coef), f32(affine), f32(affine) + O, stream),
          "tk3d_mlp_grad_coefficients_f32");
     const Tensor sel = at::empty({B, N, O, 2}, options), duv = at::empty({B, 2 * O, N}, options);
     done(tk3d_mlp_edge_backward_f32(f32(g), f32(k.extreme), k.arg.data_ptr<uint8_t>(), f32(k.uv),
@@ -810,7 +751,7 @@ struct EdgeNode : torch::autograd::Function<EdgeNode> {
                           const Tensor &gamma, const Tensor &beta, const EdgeCall &call)
     {
         EdgeKept k;
-        const Tensor z = edge_forward(call, k, true);
+        const Tensor z = edge_forward(call, k);
         ctx->save_for_backward({call.x, call.index, call.lists, call.weight, call.gamma, call.beta,
                                 k.matrix, k.uv, k.extreme, k.arg, k.sum, k.mean, k.var});
         ctx->saved_data["training"] = call.training;
@@ -949,8 +890,10 @@ Tensor mlp(Tensor x, Tensor x2, const Tensor &xyz, const Tensor &centre, const T
     c.eps = std::move(eps);
     c.momentum = std::move(momentum);
     const int64_t B = c.batch(), P = c.positions();
-    // (training mode without gradients updates running statistics: the stock modules do)
-    if (training && (!(c10::GradMode::is_enabled() && tracked) || !same_gradients(P)))
+    // The stock modules run training mode without gradients, and evaluation mode with them: there,
+    // too, signs and places decide the gradients, and nothing of the forward would be left to fuse.
+    const bool grads = c10::GradMode::is_enabled() && tracked;
+    if (training != grads || (training && !same_gradients(P)))
         return Tensor();
     int64_t widest = has_x ? c.x.size(1) : 0;
     if (has_x2)
@@ -964,7 +907,7 @@ Tensor mlp(Tensor x, Tensor x2, const Tensor &xyz, const Tensor &centre, const T
         return Tensor();
     OnDeviceOf guard(c.like().device());
     Tensor z;
-    if (c10::GradMode::is_enabled() && tracked) {
+    if (training) {
         const auto given = [](const Tensor &t) {
             return t.defined() ? std::optional<Tensor>(t) : std::nullopt;
         };
@@ -1022,15 +965,16 @@ Tensor edge_conv(const Tensor &x, const Tensor &index, const Tensor &lists,
     c.momentum = momentum;
     c.training = training;
     OnDeviceOf guard(x.device());
-    if (c10::GradMode::is_enabled() && (x.requires_grad() || c.weight.requires_grad() ||
-                                        c.gamma.requires_grad() || c.beta.requires_grad())) {
+    const bool grads = c10::GradMode::is_enabled() && (x.requires_grad() || c.weight.requires_grad() ||
+                                                       c.gamma.requires_grad() || c.beta.requires_grad());
+    if (training != grads)
+        return Tensor();  // (as for mlp())
+    if (grads) {
         c.lists = lists.defined() ? lists : edge_lists(c.index, N);
         return EdgeNode::apply(c.x, c.weight, c.gamma, c.beta, c);
     }
-    if (training)
-        return Tensor();  // (as for mlp())
     EdgeKept k;
-    return edge_forward(c, k, false);
+    return edge_forward(c, k);
 }
 
 }  // namespace tk3d

@@ -66,7 +66,8 @@ class DGCNN(nn.Module):
                 knn_ind, graph = neighbour_index(x, self.k), None
             if graph is None:
                 graph = {}
-                if x.is_cuda and x.dtype == torch.float32 and torch.is_grad_enabled():
+                if (x.is_cuda and x.dtype == torch.float32 and self.training
+                        and torch.is_grad_enabled()):
                     lists = edge_lists(knn_ind, x.size(2))  # one inverse for all blocks
                     graph = {} if lists is None else {"lists": lists}
             x = edge_conv(x, x, knn_ind, **graph)
