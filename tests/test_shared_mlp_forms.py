@@ -78,6 +78,10 @@ def test_foreign_modules_in_place_of_a_chain():
     close(forward_cat(layer.mlp, x2[:, :2], x2), want)
 
 
+class OnGpu:  # what the plan of a chain looks at
+    is_cuda, dtype = True, torch.float32
+
+
 def test_replica_without_parameters_is_left_to_stock(monkeypatch):
     # (what nn.DataParallel makes of a module: tensors as plain attributes)
     mlp, _ = pair("cpu")
@@ -89,13 +93,42 @@ def test_replica_without_parameters_is_left_to_stock(monkeypatch):
             setattr(replica, name, value.detach().clone())
         return replica
 
-    class OnGpu:  # what the plan looks at
-        is_cuda, dtype = True, torch.float32
-
     monkeypatch.setattr(torkit3d_amd.nn, "_TENSORS", (OnGpu,))
     assert mlp._plan(OnGpu()) is not None and replica_of(mlp)._plan(OnGpu()) is None
     monkeypatch.setattr(torkit3d_amd.nn, "_TENSORS", ())
     assert mlp._plan(OnGpu()) is None
+
+
+def test_batch_norm_that_does_not_track_is_left_to_stock(monkeypatch):
+    """Training mode with the flag off although the buffers are there (the pass of a teacher or an
+    adversary): the chain, which updates them, is not for that; evaluation uses them all the same."""
+    mlp, _ = pair("cpu")
+    monkeypatch.setattr(torkit3d_amd.nn, "_TENSORS", (OnGpu,))
+    assert mlp.train()._plan(OnGpu()) is not None
+    mlp[1].bn.track_running_stats = False
+    assert mlp._plan(OnGpu()) is None and mlp.eval()._plan(OnGpu()) is not None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", ["dense", "pooled", "edges"])
+def test_batch_norm_that_does_not_track_keeps_its_buffers(form):
+    from torkit3d_amd.ops.edge_conv import EdgeConvBlock
+
+    torch.manual_seed(0)
+    index = torch.randint(0, 20, (2, 20, 5), device="cuda")
+    x = torch.rand(2, 6, *{"dense": (24,), "pooled": (3, 32), "edges": (20,)}[form], device="cuda")
+    if form == "edges":
+        module = EdgeConvBlock(6, (8,)).cuda().train()
+        call = lambda: module(x, x, index)  # noqa: E731
+    else:
+        module = pair("cuda", mlp1d_bn_relu if form == "dense" else mlp2d_bn_relu)[0].train()
+        call = lambda: module(x) if form == "dense" else module.forward_max(x)  # noqa: E731
+    for m in module.modules():
+        if isinstance(m, (nn.BatchNorm1d, nn.BatchNorm2d)):
+            m.track_running_stats = False
+    before = [b.clone() for b in module.buffers()]
+    call().sum().backward()
+    assert all(torch.equal(a, b) for a, b in zip(before, module.buffers()))
 
 
 @pytest.mark.gpu

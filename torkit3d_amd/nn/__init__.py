@@ -139,7 +139,9 @@ class SharedMLP(nn.Sequential):
                     or type(relu) is not nn.ReLU or not _plain(relu)
                     or conv.groups != 1 or conv.padding != block.no_padding
                     or conv.kernel_size != block.ones or conv.stride != block.ones
-                    or conv._parameters.get("bias") is not None or bn.momentum is None):
+                    or conv._parameters.get("bias") is not None or bn.momentum is None
+                    # (the flag may be off although the buffers are there: training leaves them)
+                    or (bn.training and not bn.track_running_stats)):
                 return None
             if training is None:
                 training = bn.training
