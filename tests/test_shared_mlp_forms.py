@@ -158,17 +158,3 @@ def test_nan_reaches_the_maximum_over_edges():
     got = block(x, x, index)
     want = block(x, x.clone(), index)  # (two clouds: the general path)
     assert torch.equal(torch.isnan(got), torch.isnan(want))
-
-
-@pytest.mark.gpu
-def test_forward_mode_is_refused_by_operators():
-    from torkit3d_amd.ops.chamfer_distance import chamfer_distance
-    from torkit3d_amd.ops.group_points import group_points
-
-    x = torch.rand(1, 16, 3, device="cuda")
-    with forward_ad.dual_level():
-        dual = forward_ad.make_dual(x, torch.ones_like(x))
-        with pytest.raises(Exception):
-            chamfer_distance(dual, x)
-        with pytest.raises(Exception):
-            group_points(dual, torch.zeros(1, 2, 2, dtype=torch.long, device="cuda"))

@@ -431,12 +431,9 @@ Tensor interpolate_backward(const Tensor &grad, const Tensor &index, const Tenso
 
 // ---- autograd nodes ------------------------------------------------------------------------------
 
-// Whether a node has to be made: for gradients, and for a forward-mode tangent, which the nodes
-// refuse (without one it would be dropped in silence).
 template <typename... T> bool tracked(const T &...t)
 {
-    return (c10::GradMode::is_enabled() && ((t.defined() && t.requires_grad()) || ...)) ||
-           ((t.defined() && t._fw_grad(0).defined()) || ...);
+    return c10::GradMode::is_enabled() && ((t.defined() && t.requires_grad()) || ...);
 }
 
 // sqrt(max(d, eps)) of both directions.
@@ -682,6 +679,19 @@ PYBIND11_MODULE(_host, m)
         const Tensor g = tensor_arg("grad_output", grad), i = tensor_arg("index", index),
                      w = tensor_arg("weight", weight);
         return unlocked([&] { return interpolate_backward(g, i, w, n1); });
+    });
+
+    // Whether a call on these arguments may go straight to the functions here. Where a tracer, a
+    // function transform or a dispatch mode is active, or a tensor carries a forward-mode tangent,
+    // these would leave nothing to see: a trace would hold memory that nobody fills, a tangent would
+    // be lost. The caller then takes its torch.autograd.Function, which such things know.
+    m.def("direct", [](py::args args) {
+        if (watched())
+            return false;
+        for (const py::handle h : args)
+            if (THPVariable_Check(h.ptr()) && !plain(THPVariable_Unpack(h.ptr())))
+                return false;
+        return true;
     });
 
     // differentiable forms

@@ -40,7 +40,7 @@ using OnDeviceOf = c10::OptionalDeviceGuard;
 // Whether the tensor is what its pointer and sizes say: no subclass that dispatches in Python, no
 // wrapper of a function transform, no pending conjugation, and no forward-mode tangent.
 bool plain(const Tensor &t);
-// A function transform (torch.func) or a dispatch mode is active: it has to see the operators.
+// A function transform (torch.func), a dispatch mode or a tracer is active: it has to see the operators.
 bool watched();
 
 Tensor mlp(Tensor x, Tensor x2, const Tensor &xyz, const Tensor &centre, const Tensor &index,

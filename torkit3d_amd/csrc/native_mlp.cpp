@@ -3,6 +3,7 @@
 #include "native.h"
 #include "tk3d_mlp.h"
 
+#include <ATen/TracerMode.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <torch/csrc/autograd/autograd.h>
@@ -24,7 +25,7 @@ bool watched()
 {
     return c10::impl::tls_is_dispatch_key_included(
                c10::DispatchKey::FuncTorchDynamicLayerFrontMode) ||
-           c10::impl::TorchDispatchModeTLS::any_modes_set();
+           c10::impl::TorchDispatchModeTLS::any_modes_set() || at::tracer::impl::is_dispatch_enabled();
 }
 
 namespace {

@@ -25,6 +25,8 @@ class GroupPointsFunction(torch.autograd.Function):
 def group_points(points, index):
     """points [B, C, N1], index [B, N2, K] -> [B, C, N2, K] with
     out[b, c, m, s] = points[b, c, index[b, m, s]]."""
+    if not _native.direct(points, index):
+        return GroupPointsFunction.apply(points, index)
     return _native.group_points(points, index)
 
 
@@ -38,6 +40,11 @@ def group_points_with_xyz(feature, xyz, centre, index):
         feature: [B, C, N1] or None; xyz: [B, 3, N1]; centre: [B, 3, N2];
         index: [B, N2, K] int64.
     """
+    if not _native.direct(feature, xyz, centre, index):
+        grouped = GroupPointsFunction.apply(xyz, index) - centre.unsqueeze(-1)
+        if feature is None:
+            return grouped
+        return torch.cat([GroupPointsFunction.apply(feature, index), grouped], dim=1)
     return _native.group_points_with_xyz(feature, xyz, centre, index)
 
 gather_points = group_points  # the spelling common elsewhere

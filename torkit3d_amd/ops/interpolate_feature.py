@@ -26,6 +26,8 @@ class InterpolateFeature(torch.autograd.Function):
 def interpolate_feature(feature, index, weight):
     """feature [B, C, N1], index [B, N2, K], weight [B, N2, K] -> [B, C, N2] with
     out[b, c, n] = sum_i feature[b, c, index[b, n, i]] * weight[b, n, i]."""
+    if not _native.direct(feature, index, weight):
+        return InterpolateFeature.apply(feature, index, weight)
     return _native.interpolate(feature, index, weight)
 
 
