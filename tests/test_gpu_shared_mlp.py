@@ -245,6 +245,32 @@ def test_edge_conv(cuda, b, c, n, k, o, lists, training):
         assert mine <= 4 * theirs + 2e-6, (i, tuple(e.shape), mine, theirs)
 
 
+def test_edge_conv_lists_are_checked(cuda):
+    """What is not the inverse of a graph of this size is refused, and whatever such a tensor holds,
+    the backward stays inside it and inside the cloud."""
+    from torkit3d_amd.ops.edge_conv import EdgeConvBlock, edge_lists
+
+    block = EdgeConvBlock(4, [8]).to(cuda).train()
+    b, n, k = 2, 50, 6
+    index = torch.randint(0, n, (b, n, k), generator=torch.Generator().manual_seed(0)).to(cuda)
+    x = randn(8, b, 4, n).requires_grad_()
+    lists = edge_lists(index, n)
+    shorter = edge_lists(index[:, :40, :].clamp(max=39).contiguous(), 40)
+    for wrong in (shorter, edge_lists(index[:, :, :5].contiguous(), n), lists[:1], lists.long(),
+                  lists.cpu(), lists.view(-1), lists.t().contiguous().t()):
+        with pytest.raises(RuntimeError, match="lists"):
+            block(x, x, index, lists=wrong)
+    block(x, x, index, lists=lists).sum().backward()
+    low, high = torch.iinfo(torch.int32).min, torch.iinfo(torch.int32).max
+    noise = torch.randint(low, high, tuple(lists.shape), dtype=torch.int32,
+                          generator=torch.Generator().manual_seed(1)).to(cuda)
+    noise[1, : n + 1] = torch.arange(n + 1, dtype=torch.int32, device=cuda) * k
+    for any_lists in (noise, torch.full_like(lists, low), torch.full_like(lists, high)):
+        x.grad = None
+        block(x, x, index, lists=any_lists).sum().backward()
+        assert torch.isfinite(x.grad).all()
+
+
 def test_edge_conv_with_indices_outside(cuda):
     """A neighbour outside the cloud reads as zeros, as ``group_points`` reads it."""
     from torkit3d_amd.ops.edge_conv import EdgeConvBlock, get_edge_feature_custom

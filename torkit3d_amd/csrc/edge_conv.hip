@@ -227,7 +227,8 @@ __global__ void __launch_bounds__(kBlock)
         const int local = wave * (kPoints / kWaves) + q, j = first + local;
         if (j >= N)
             break;
-        const int from = start[j], to = start[j + 1];
+        // (the lists come from the caller: whatever they hold, nothing outside is read)
+        const int from = min(max(start[j], 0), N * K), to = min(max(start[j + 1], from), N * K);
         double acc = 0.0;
         for (int e0 = from; e0 < to; e0 += kAtOnce) {
             float v[kAtOnce];
@@ -236,7 +237,7 @@ __global__ void __launch_bounds__(kBlock)
 #pragma unroll
             for (int i = 0; i < kAtOnce; ++i) {
                 const int entry = entries[e0 + i < to ? e0 + i : to - 1];
-                const int64_t at = entry >> 8;
+                const int64_t at = min((unsigned)entry >> 8, (unsigned)N - 1u);
                 k[i] = entry & 255;
                 v[i] = u[at * 2 * O + O];
                 s[i] = selected[at * O];

@@ -950,6 +950,12 @@ Tensor edge_conv(const Tensor &x, const Tensor &index, const Tensor &lists,
         return Tensor();
     const int64_t B = x.size(0), C = x.size(1), N = x.size(2), K = index.size(2);
     const int64_t O = params[0].size(0);
+    if (lists.defined() &&
+        (lists.scalar_type() != at::kInt || lists.device() != x.device() || !plain(lists) ||
+         lists.dim() != 2 || lists.size(0) != B || lists.size(1) != N + 1 + N * K ||
+         !lists.is_contiguous()))
+        fail("lists must be edge_lists(key_ind, N): contiguous int32 [B, N + 1 + N K] on the GPU of "
+             "the features.");
     if (params[0].size(1) != 2 * C || !tk3d_mlp_edge_supported(B, N, K, O) || B * N * K < 2 ||
         C > 4096 || (std::max(C, 2 * O) + 8) * N > (1 << 29) || (training && !same_gradients(N * K)))
         return Tensor();

@@ -69,7 +69,9 @@ class EdgeConvBlock(torch.nn.Module):
         """query_feature [B,C,N1], key_feature [B,C,N2], key_ind [B,N1,K] -> [B,C',N1].
 
         ``lists`` (not in the reference) is the inverse of the graph (``edge_lists``), for
-        callers that run several blocks on one graph; without it every block works it out."""
+        callers that run several blocks on one graph; without it every block works it out. Its
+        type, shape and device are checked; that it belongs to ``key_ind`` is up to the caller
+        (lists of another graph of the same size give that graph's gradients)."""
         if query_feature is key_feature and not self.checkpoint:
             output = forward_edges_max(self.convs, query_feature, key_ind, lists)
             if output is not None:
