@@ -16,9 +16,13 @@
  * Pooled layers. Where only the maximum of z over groups of `group` consecutive positions is
  * wanted, the place of the maximum and the y there are all of the layer that is kept. In the
  * backward e has one nonzero per group and channel, and with y = W x
- *     W^T dy = W^T (a e) + (W^T diag(b) W) x + W^T d
- *     dW     = (a e) x^T + diag(b) W (x x^T) + d (sum x)^T
- * so the dense part needs only the input x.
+ *     W^T dy = W^T (a e) + (W^T diag(b) W) x' + W^T d'
+ *     dW     = (a e) x'^T + diag(b) W (x' x'^T) + d' (sum x')^T
+ * so the dense part needs only the input x. In it x' = x - m and d' = d + b (W m) for any m (a
+ * channel's dy add up to zero over the batch, so that sum dy m^T is nothing). Here m = relu(beta) of
+ * the norm in front, of which the mean of x is never further than |gamma| / 2: with m = 0 the terms
+ * of dW cancel where activations sit far from zero (mean / deviation of 8: 2.1 times the error of
+ * the sum over positions).
  */
 #ifndef TK3D_MLP_H
 #define TK3D_MLP_H
@@ -51,11 +55,12 @@ enum {
     TK3D_MLP_IN_ACT = 2,      /* relu(in_norm(x)) */
     TK3D_MLP_IN_GRAD = 3,     /* a x + b y + d */
     TK3D_MLP_IN_GRAD_OUT = 4, /* the same with x masked by relu(in_norm(y)) first */
+    TK3D_MLP_IN_CENTRED = 5,  /* relu(in_norm(x)) - relu(beta of in_norm) */
     TK3D_MLP_OUT_PLAIN = 1,     /* out + bias, channels from C0 on in out2; either may be NULL */
     TK3D_MLP_OUT_POINTS = 2,    /* out as [B, P, C] */
     TK3D_MLP_OUT_EVAL = 3,      /* relu(out_norm(out)) */
     TK3D_MLP_OUT_POOL_EVAL = 5, /* relu(out_norm(extreme over groups)) */
-    TK3D_MLP_OUT_MASK = 6       /* e = (out + bias, IN_ACT: + add) where relu(out_norm(yprev)) passes, and partial
+    TK3D_MLP_OUT_MASK = 6       /* e = (out + bias, IN_CENTRED: + add) where relu(out_norm(yprev)) passes, and partial
                                    sums of e and e (yprev - mean) */
 };
 
@@ -65,7 +70,7 @@ typedef struct {
     float *out, *out2;
     const float *yprev; /* [B, C, P] */
     const float *bias;  /* [C] or NULL */
-    const float *add;   /* [B, C, P], may be out itself; IN_ACT to OUT_MASK alone (P % 32 == 0) */
+    const float *add;   /* [B, C, P], may be out itself; IN_CENTRED to OUT_MASK alone (P % 32 == 0) */
     void *partial;      /* OUT_MASK: doubles [C][slots][2]; tk3d_mlp_product_slots gives slots */
     int32_t B, C, C0, P;
     int32_t group, M;   /* pooled forms: P == group * M, group 32 or 64 */
@@ -77,15 +82,16 @@ int tk3d_mlp_product_f32(int in, int out, const tk3d_mlp_product *p, void *strea
 
 /* Weight gradient: out[r][c] = sum over (b, p) of row(r, p) * colv(c, p), r < R, c < C, in
  * `splits` partial sums [splits][R][C]. Rows: raw x, gradient (a x + b y + d, masked or not),
- * or activations; columns: raw x or activations. rowsum (NULL or [splits][R]) gets the
+ * or activations less relu(beta); columns: raw x, activations, or these less relu(beta). rowsum (NULL or [splits][R]) gets the
  * sums of the rows themselves. */
 enum {
     TK3D_MLP_ROW_RAW = 0,
     TK3D_MLP_ROW_GRAD = 1,
     TK3D_MLP_ROW_GRAD_OUT = 2,
-    TK3D_MLP_ROW_ACT = 4,
+    TK3D_MLP_ROW_CENTRED = 4,
     TK3D_MLP_COL_RAW = 0,
-    TK3D_MLP_COL_ACT = 1
+    TK3D_MLP_COL_ACT = 1,
+    TK3D_MLP_COL_CENTRED = 2
 };
 typedef struct {
     tk3d_mlp_source row, col; /* K = R and C; weights unused */
@@ -131,11 +137,12 @@ int tk3d_mlp_grad_apply_f32(float *e, const float *y, const float *coef, int B, 
                             void *stream);
 
 /* Backward of a pooled layer, before the products: from g [B,C,M], the extremes and their places
- * the coefficients, dgamma, dbeta and sel, [B, C, M] of (float a e, int32 place in the group);
- * positions = B * group * M. */
+ * the coefficients (a, b, d'), dgamma, dbeta and sel, [B, C, M] of (float a e, int32 place in the
+ * group); positions = B * group * M, w [C][I], inner the norm in front of the layer. */
 int tk3d_mlp_pool_grad_f32(const float *g, const float *extreme, const unsigned char *arg, int B,
-                           int C, int M, int64_t positions, const tk3d_mlp_norm *norm,
-                           void *sel, float *coef, float *dgamma, float *dbeta, void *stream);
+                           int C, int M, int64_t positions, const tk3d_mlp_norm *norm, const float *w,
+                           int I, const tk3d_mlp_norm *inner, void *sel, float *coef, float *dgamma,
+                           float *dbeta, void *stream);
 /* The sparse half of W^T dy, [B, I, M * group] (groups of 32 or 64; W [O][I]), and that of dW in
  * partial sums [splits][O][I] (y [B, I, M * group], norm of y). */
 int tk3d_mlp_pool_scatter_f32(const void *sel, const float *w, int B, int O, int I, int M, int group,
@@ -143,10 +150,10 @@ int tk3d_mlp_pool_scatter_f32(const void *sel, const float *w, int B, int O, int
 int tk3d_mlp_pool_outer_splits(int B, int O, int I, int M);
 int tk3d_mlp_pool_outer_f32(const void *sel, const float *y, const tk3d_mlp_norm *norm, int B, int O,
                             int I, int M, int group, float *partial, void *stream);
-/* gram[k][c] = sum_o W[o][k] b[o] W[o][c] and bias[c] = sum_o W[o][c] d[o]; W [O][I]. */
+/* gram[k][c] = sum_o W[o][k] b[o] W[o][c] and bias[c] = sum_o W[o][c] d'[o]; W [O][I]. */
 int tk3d_mlp_pool_gram_f32(const float *w, const float *coef, int O, int I, float *gram, float *bias,
                            void *stream);
-/* dW[o][i] = sparse[o][i] + b[o] (W xx)[o][i] + d[o] xsum[i]; sparse, xx, xsum as partial sums. */
+/* dW[o][i] = sparse[o][i] + b[o] (W xx)[o][i] + d'[o] xsum[i]; sparse, xx, xsum as partial sums. */
 int tk3d_mlp_pool_weight_grad_f32(const float *sparse, int sparse_splits, const float *xx,
                                   const float *xsum, int xx_splits, const float *w,
                                   const float *coef, int O, int I, float *scratch, float *dw,

@@ -157,6 +157,46 @@ def test_training_is_that_of_the_stock_modules(cuda, b, p, widths, pool):
         assert float((a - c).norm()) <= 6e-6 * float(c.norm())
 
 
+def pinned(single, exact, x, x64):
+    """The maxima over neighbours of the float64 chain `exact`, with the signs and places of the
+    float32 chain `single` (the same layers): what differs in its gradients is arithmetic alone."""
+    for a, b in zip(single, exact):
+        with torch.no_grad():
+            z = a.bn(a.conv(x))
+            x = torch.relu(z)
+        x64 = b.bn(b.conv(x64)) * (z > 0)
+    return x64.gather(3, z.max(dim=3, keepdim=True)[1]).squeeze(3)
+
+
+# Activations in front of a pooled layer at up to `far` deviations from zero. The weight gradient is
+# made of second moments there: about zero they give 2.1 times the stock modules' error at 3 and
+# at 8, about the activations' mean 0.6 times. (The error of one draw is good to a tenth: a quarter is
+# left for it.)
+@pytest.mark.parametrize("far", [0, 3, 8])
+@pytest.mark.parametrize("b,m,s,widths", [(8, 128, 64, (131, 128, 256)), (3, 70, 32, (9, 40, 33)),
+                                          (2, 512, 32, (6, 64, 64, 128))])
+def test_pooled_layer_far_from_zero(cuda, b, m, s, widths, far):
+    mlp = make(mlp2d_bn_relu, widths[0], widths[1:], True, cuda)
+    with torch.no_grad():
+        for block in mlp:
+            block.bn.weight.abs_().add_(0.5)
+            block.bn.bias.add_(far * block.bn.weight)
+    single, again, exact = stock(mlp, torch.float32), stock(mlp, torch.float32), stock(mlp, torch.float64)
+    x, g = randn(m, b, widths[0], m, s), randn(3, b, widths[-1], m)
+    grads = []
+    for module, dtype in ((mlp, torch.float32), (single, torch.float32), (exact, torch.float64)):
+        leaf = x.to(dtype).requires_grad_()
+        if module is exact:
+            out = pinned(again, exact, x, leaf)
+        else:
+            out = mlp.forward_max(leaf) if module is mlp else module(leaf).max(dim=3)[0]
+        wanted = [leaf, *[p for block in module for p in (block.conv.weight, block.bn.weight)]]
+        grads.append(torch.autograd.grad(out, wanted, g.to(dtype)))
+    for mine, theirs, e in zip(*grads):
+        errors = [float((t.double() - e).norm() / e.norm()) for t in (mine, theirs)]
+        assert errors[0] <= 1.25 * errors[1] + 2e-7, (tuple(e.shape), errors)
+
+
 @pytest.mark.parametrize("p", [514, 1030])
 def test_rows_on_which_the_library_differs_run_in_stock(cuda, p):
     mlp = make(mlp1d_bn_relu, 6, (8, 5), True, cuda)

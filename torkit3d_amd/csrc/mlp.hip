@@ -33,6 +33,7 @@ enum Input {      // in(k, p)
     IN_ACT,       // relu(norm(x))
     IN_GRAD,      // a e + b y + d: gradient before the norm from the gradient behind it (e)
     IN_GRAD_OUT,  // the same where e = g masked by the ReLU still has to be formed from g and y
+    IN_CENTRED,   // relu(norm(x)) less the channel's centre
 };
 enum Output {
     OUT_PLAIN,      // store, in two tensors if asked for
@@ -100,7 +101,7 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
         act_coef = grad_coef + (size_t)a.kg * 8;
     float *weights = reinterpret_cast<float *>(lds + a.coef_bytes);  // [CT][chunk][64][4]
 
-    if constexpr (IN == IN_ACT || IN == IN_GRAD_OUT) {
+    if constexpr (IN == IN_ACT || IN == IN_CENTRED || IN == IN_GRAD_OUT) {
         const int K = p.src[0].K;
         for (int k = tid; k < ((K + 7) & ~7); k += kBlock)
             act_coef[k] = k < K ? constants_of(p.in_norm, k) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -197,11 +198,15 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
                         e = passes(normalised(y, ss)) ? e : 0.0f;
                     v[q][t] = __builtin_fmaf(c.x, e, __builtin_fmaf(c.y, y, c.z));
                 }
-            } else if constexpr (IN == IN_ACT) {
+            } else if constexpr (IN == IN_ACT || IN == IN_CENTRED) {
                 const f32x4 c = act_coef[k0 + 2 * q];
+                const float centre = IN == IN_CENTRED ? centre_of(c) : 0.0f;
 #pragma unroll
-                for (int t = 0; t < PT; ++t)
+                for (int t = 0; t < PT; ++t) {
                     v[q][t] = relu(normalised(r.x[d][q][t], c));
+                    if constexpr (IN == IN_CENTRED)
+                        v[q][t] -= centre;
+                }
             } else {
 #pragma unroll
                 for (int t = 0; t < PT; ++t)
@@ -308,7 +313,7 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
                         for (int i = 0; i < RUN; ++i)
                             before[OUT == OUT_MASK ? i : 0] = yrow[pos + i > P - 1 ? P - 1 : pos + i];
                     }
-                    if constexpr (IN == IN_ACT) {  // (P is a multiple of 32 here)
+                    if constexpr (IN == IN_CENTRED) {  // (P is a multiple of 32 here)
                         const float *arow = p.add + ((int64_t)b * p.C + (mine ? c : p.C - 1)) * P;
 #pragma unroll
                         for (int i = 0; i < PT; ++i) {
@@ -490,14 +495,14 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_outer_kernel(OuterArgs a)
         total[t] = 0.0f;
         if constexpr (kGrad)
             coef[t] = reinterpret_cast<const f32x4 *>(p.row.coef)[r[t]];
-        if constexpr (ROW == TK3D_MLP_ROW_GRAD_OUT || ROW == TK3D_MLP_ROW_ACT)
+        if constexpr (ROW == TK3D_MLP_ROW_GRAD_OUT || ROW == TK3D_MLP_ROW_CENTRED)
             row_act[t] = constants_of(p.row_norm, r[t]);
     }
 #pragma unroll
     for (int t = 0; t < TB; ++t) {
         c[t] = cbase + 32 * t + l32;
         c[t] = c[t] < C ? c[t] : C - 1;
-        if constexpr (COL == TK3D_MLP_COL_ACT)
+        if constexpr (COL != TK3D_MLP_COL_RAW)
             col_act[t] = constants_of(p.col_norm, c[t]);
     }
 
@@ -559,13 +564,13 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_outer_kernel(OuterArgs a)
                     if constexpr (ROW == TK3D_MLP_ROW_GRAD_OUT)
                         e = passes(normalised(yy, row_act[t])) ? e : 0.0f;
                     v = __builtin_fmaf(coef[t].x, e, __builtin_fmaf(coef[t].y, yy, coef[t].z));
-                } else if constexpr (ROW == TK3D_MLP_ROW_ACT) {
-                    v = relu(normalised(q.x[t][i], row_act[t]));
+                } else if constexpr (ROW == TK3D_MLP_ROW_CENTRED) {
+                    v = relu(normalised(q.x[t][i], row_act[t])) - centre_of(row_act[t]);
                 } else {
                     v = q.x[t][i];
                 }
                 x[t][i] = pos + i < P ? v : 0.0f;
-                if constexpr (ROW == TK3D_MLP_ROW_ACT)
+                if constexpr (ROW == TK3D_MLP_ROW_CENTRED)
                     total[t] += x[t][i];
             }
 #pragma unroll
@@ -573,8 +578,10 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_outer_kernel(OuterArgs a)
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 float v = q.c[t][i];
-                if constexpr (COL == TK3D_MLP_COL_ACT)
+                if constexpr (COL != TK3D_MLP_COL_RAW)
                     v = relu(normalised(v, col_act[t]));
+                if constexpr (COL == TK3D_MLP_COL_CENTRED)
+                    v -= centre_of(col_act[t]);
                 y[t][i] = v;
             }
 #pragma unroll
@@ -620,7 +627,7 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_outer_kernel(OuterArgs a)
         if (row < R && col < C)
             p.partial[((int64_t)blockIdx.x * R + row) * C + col] = s;
     }
-    if constexpr (ROW == TK3D_MLP_ROW_ACT) {
+    if constexpr (ROW == TK3D_MLP_ROW_CENTRED) {
         if (p.rowsum && blockIdx.z == 0) {
             __syncthreads();
 #pragma unroll
@@ -712,14 +719,15 @@ struct Coefficients {
     float dgamma, dbeta;
 };
 
+// (`origin`: the y from which the b y of the caller is counted)
 __device__ __forceinline__ Coefficients grad_coefficients(double2 s, double n, const tk3d_mlp_norm &norm,
-                                                          int c)
+                                                          int c, double origin = 0.0)
 {
     const double is = norm.eps < 0.0f ? (double)norm.var[c]
                                       : 1.0 / __builtin_sqrt((double)norm.var[c] + (double)norm.eps);
     const double gamma = norm.gamma[c], mean = norm.mean[c];
     const double b = -gamma * is * is * is * s.y / n;
-    const double d = -gamma * is * s.x / n - b * mean;
+    const double d = -gamma * is * s.x / n - b * (mean - origin);
     return {f32x4{(float)(gamma * is), (float)b, (float)d, 0.0f}, (float)(s.y * is), (float)s.x};
 }
 
@@ -820,10 +828,10 @@ __global__ void __launch_bounds__(kBlock)
 // One workgroup per channel: the sums, then the coefficients, then the sparse gradient.
 __global__ void __launch_bounds__(1024)
     mlp_pool_grad_kernel(const float *g, const float *extreme, const unsigned char *arg, int B, int C,
-                         int M, double n, tk3d_mlp_norm norm, int2 *sel, float *coef,
-                         float *dgamma, float *dbeta)
+                         int M, double n, tk3d_mlp_norm norm, const float *w, int I,
+                         tk3d_mlp_norm inner, int2 *sel, float *coef, float *dgamma, float *dbeta)
 {
-    __shared__ double2 lds[16];
+    __shared__ double2 lds[16], lds2[16];
     const int c = blockIdx.x;
     const f32x4 ss = constants_of(norm, c);
     const float mean = norm.mean[c];
@@ -840,7 +848,11 @@ __global__ void __launch_bounds__(1024)
         v.x += e;
         v.y += (double)e * (double)(y - mean);
     }
-    const Coefficients k = grad_coefficients(block_sum(v, lds), n, norm, c);
+    double2 wm{0.0, 0.0};
+    for (int i = threadIdx.x; i < I; i += blockDim.x)
+        wm.x += (double)w[(int64_t)c * I + i] * (double)centre_of(constants_of(inner, i));
+    wm = block_sum(wm, lds2);
+    const Coefficients k = grad_coefficients(block_sum(v, lds), n, norm, c, wm.x);
     if (threadIdx.x == 0) {
         reinterpret_cast<f32x4 *>(coef)[c] = k.abd;
         dgamma[c] = k.dgamma;
@@ -926,8 +938,8 @@ __global__ void __launch_bounds__(kBlock) mlp_pool_scatter_kernel(SparseArgs a)
     }
 }
 
-// partial[split][o][i] = sum over groups of a e relu(norm(y[i, (m, place)])): 64 rows and 64 columns
-// a workgroup, rows in registers.
+// partial[split][o][i] = sum over groups of a e (relu(norm(y[i, (m, place)])) less the centre of i): 64
+// rows and 64 columns a workgroup, rows in registers.
 template <int S>
 __global__ void __launch_bounds__(kBlock) mlp_pool_outer_kernel(SparseArgs a)
 {
@@ -966,7 +978,7 @@ __global__ void __launch_bounds__(kBlock) mlp_pool_outer_kernel(SparseArgs a)
 #pragma unroll
         for (int q = 0; q < S; ++q) {
             const int i = first + q * (64 / S);
-            tile[p * kRow + i] = relu(normalised(v[q], constants[i]));
+            tile[p * kRow + i] = relu(normalised(v[q], constants[i])) - centre_of(constants[i]);
         }
         const float e = o0 + lane < a.O ? __int_as_float(sel.x) : 0.0f;
         const int place = sel.y;
@@ -1347,7 +1359,7 @@ int tk3d_mlp_product_f32(int in, int out, const tk3d_mlp_product *p, void *strea
         return TK3D_ERR_UNSUPPORTED;
     if (out == TK3D_MLP_OUT_POOL_EVAL && ((p->group != 32 && p->group != 64) || p->M * p->group != p->P))
         return TK3D_ERR_UNSUPPORTED;
-    if (in == TK3D_MLP_IN_ACT && out == TK3D_MLP_OUT_MASK && (!p->add || p->P % 32 != 0))
+    if (in == TK3D_MLP_IN_CENTRED && out == TK3D_MLP_OUT_MASK && (!p->add || p->P % 32 != 0))
         return TK3D_ERR_BAD_SIZE;
     const Shape s = pick_shape(out, *p);
     GemmArgs g;
@@ -1365,7 +1377,7 @@ int tk3d_mlp_product_f32(int in, int out, const tk3d_mlp_product *p, void *strea
     TK_CASE(IN_GRAD, OUT_PLAIN)
     TK_CASE(IN_GRAD_OUT, OUT_MASK)
     TK_CASE(IN_GRAD_OUT, OUT_PLAIN)
-    TK_CASE(IN_ACT, OUT_MASK)
+    TK_CASE(IN_CENTRED, OUT_MASK)
 #undef TK_CASE
     return TK3D_ERR_UNSUPPORTED;
 }
@@ -1402,7 +1414,7 @@ int tk3d_mlp_outer_f32(int row, int col, const tk3d_mlp_outer *p, void *stream_)
     TK_CASE(TK3D_MLP_ROW_GRAD, TK3D_MLP_COL_ACT)
     TK_CASE(TK3D_MLP_ROW_GRAD_OUT, TK3D_MLP_COL_RAW)
     TK_CASE(TK3D_MLP_ROW_GRAD_OUT, TK3D_MLP_COL_ACT)
-    TK_CASE(TK3D_MLP_ROW_ACT, TK3D_MLP_COL_ACT)
+    TK_CASE(TK3D_MLP_ROW_CENTRED, TK3D_MLP_COL_CENTRED)
 #undef TK_CASE
     return TK3D_ERR_UNSUPPORTED;
 }
@@ -1492,12 +1504,13 @@ int tk3d_mlp_grad_apply_f32(float *e, const float *y, const float *coef, int B, 
 }
 
 int tk3d_mlp_pool_grad_f32(const float *g, const float *extreme, const unsigned char *arg, int B,
-                           int C, int M, int64_t positions, const tk3d_mlp_norm *norm,
-                           void *sel, float *coef, float *dgamma, float *dbeta, void *stream)
+                           int C, int M, int64_t positions, const tk3d_mlp_norm *norm, const float *w,
+                           int I, const tk3d_mlp_norm *inner, void *sel, float *coef, float *dgamma,
+                           float *dbeta, void *stream)
 {
     mlp_pool_grad_kernel<<<C, 1024, 0, (hipStream_t)stream>>>(
-        g, extreme, arg, B, C, M, (double)positions, *norm, reinterpret_cast<int2 *>(sel), coef,
-        dgamma, dbeta);
+        g, extreme, arg, B, C, M, (double)positions, *norm, w, I, *inner,
+        reinterpret_cast<int2 *>(sel), coef, dgamma, dbeta);
     return tk_launch_status();
 }
 

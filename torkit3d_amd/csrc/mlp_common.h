@@ -32,6 +32,10 @@ __device__ __forceinline__ float normalised(float y, f32x4 k)
     return __builtin_fmaf(k.z, (y - k.x) * k.y, k.w);
 }
 
+// What a pooled layer's backward takes from the activations of a channel in front of it (near their
+// mean, include/tk3d_mlp.h).
+__device__ __forceinline__ float centre_of(f32x4 k) { return relu(k.w); }
+
 // The sign by which a maximum over relu(norm(y)) becomes one over y.
 __device__ __forceinline__ float sign_of(float gamma)
 {

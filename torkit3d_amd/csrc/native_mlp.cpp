@@ -336,12 +336,13 @@ Grads backward(const Call &c, const Kept &k, const Tensor &g, bool want_x, bool 
         const int64_t O = c.out_channels(l), I = c.in_channels(l), M = P / c.pool;
         const tk3d_mlp_norm norm = norm_of(c, k, l), inner = norm_of(c, k, l - 1);
         const Tensor sel = at::empty({B, O, M, 2}, like.options());
+        const float *w = f32(c.weight(l));
         done(tk3d_mlp_pool_grad_f32(f32(g), f32(k.y[l]), k.arg.data_ptr<uint8_t>(), (int)B, (int)O,
-                                    (int)M, B * P, &norm, sel.data_ptr(), f32(coef[l]),
-                                    f32(out.params[3 * l + 1]), f32(out.params[3 * l + 2]), stream),
+                                    (int)M, B * P, &norm, w, (int)I, &inner, sel.data_ptr(),
+                                    f32(coef[l]), f32(out.params[3 * l + 1]),
+                                    f32(out.params[3 * l + 2]), stream),
              "tk3d_mlp_pool_grad_f32");
         const Tensor gram = at::empty({I + 1, I}, like.options());
-        const float *w = f32(c.weight(l));
         done(tk3d_mlp_pool_gram_f32(w, f32(coef[l]), (int)O, (int)I, f32(gram), f32(gram) + I * I,
                                     stream),
              "tk3d_mlp_pool_gram_f32");
@@ -355,7 +356,7 @@ Grads backward(const Call &c, const Kept &k, const Tensor &g, bool want_x, bool 
         p.yprev = f32(k.y[l - 1]);
         p.bias = f32(gram) + I * I;
         p.add = p.out = f32(e);
-        const auto sums = summed_product(TK3D_MLP_IN_ACT, TK3D_MLP_OUT_MASK, p, like, stream);
+        const auto sums = summed_product(TK3D_MLP_IN_CENTRED, TK3D_MLP_OUT_MASK, p, like, stream);
 
         const int sparse_splits = tk3d_mlp_pool_outer_splits((int)B, (int)O, (int)I, (int)M);
         const Tensor sparse = at::empty({sparse_splits, O, I}, like.options());
@@ -373,7 +374,8 @@ Grads backward(const Call &c, const Kept &k, const Tensor &g, bool want_x, bool 
         const Tensor xsum = at::empty({splits, I}, like.options());
         o.partial = f32(xx);
         o.rowsum = f32(xsum);
-        done(tk3d_mlp_outer_f32(TK3D_MLP_ROW_ACT, TK3D_MLP_COL_ACT, &o, stream), "tk3d_mlp_outer_f32");
+        done(tk3d_mlp_outer_f32(TK3D_MLP_ROW_CENTRED, TK3D_MLP_COL_CENTRED, &o, stream),
+             "tk3d_mlp_outer_f32");
         const Tensor scratch = at::empty({I + 1, I}, like.options());
         done(tk3d_mlp_pool_weight_grad_f32(f32(sparse), sparse_splits, f32(xx), f32(xsum), splits, w,
                                            f32(coef[l]), (int)O, (int)I, f32(scratch),
