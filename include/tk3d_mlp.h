@@ -11,7 +11,8 @@
  * entry points hand y from layer to layer: the norm and the ReLU are applied where y is read.
  * Backward, with g the gradient of z, e = g where z > 0 (or NaN) else 0:
  *     dbeta = sum e,   dgamma = sum e (y - mean) / sqrt(var + eps),
- *     dy = a e + b y + d  with (a, b, d) per channel (tk3d_mlp_grad_coefficients_f32).
+ *     dy = a e + b y + d = a e + b (y - mean) + d0  with (a, b, d, d0) per channel
+ * (tk3d_mlp_grad_coefficients_f32).
  *
  * Pooled layers. Where only the maximum of z over groups of `group` consecutive positions is
  * wanted, the place of the maximum and the y there are all of the layer that is kept. In the
@@ -42,7 +43,7 @@ typedef struct {
 typedef struct {
     const float *x;        /* [B, K, P]; batch_stride elements from one batch element to the next */
     const float *y;        /* same shape, for the gradient inputs */
-    const float *coef;     /* [K][4]: (a, b, d, -), for the gradient inputs */
+    const float *coef;     /* [K][4]: (a, b, d, d0), for the gradient inputs */
     const float *w;        /* weight of input channel k and output channel c: w[k * wk + c * wc] */
     int64_t batch_stride;
     int32_t K, wk, wc;
@@ -117,7 +118,7 @@ int tk3d_mlp_sum_f32(const tk3d_mlp_sum *sums, int n, void *stream);
 int tk3d_mlp_pool_max_f32(const float *z, const float *y, int64_t groups, int size, float *out,
                           float *extreme, unsigned char *arg, void *stream);
 
-/* (a, b, d) per channel from the partial sums of (e, e (y - mean)), and dgamma, dbeta.
+/* (a, b, d, d0) per channel from the partial sums of (e, e (y - mean)), and dgamma, dbeta.
  */
 int tk3d_mlp_grad_coefficients_f32(const void *partial, int slots, int64_t n, int C,
                                    const tk3d_mlp_norm *norm, float *coef, float *dgamma,
@@ -167,25 +168,26 @@ int tk3d_mlp_group_f32(const float *u, const float *xyz, const float *centre, co
                        void *stream);
 
 /* EdgeConv (torkit3d/ops/edge_conv.py) with one layer, on a graph of a cloud with itself, pooled
- * over the K neighbours: y(i, k) = W1 (x_j - x_i) + W2 x_i = u_j + v_i, j = index[b, i, k] (x_j = 0
- * for an index outside [0,N)), where w = [W1 W2], u = W1 x and v = (W2 - W1) x; uv [B, N, 2 O] is
- * the product of x with the [2 O][C] matrix that tk3d_mlp_edge_weights_f32 makes of w. Forward:
- * the extreme of y [B, O, N] (or NULL) and the sum [B, N, O] of the u of a point's neighbours (or
- * NULL). tk3d_mlp_edge_features_f32 makes the edge features themselves,
- * [B, 2 C, N, K]. Backward: lists is the inverse of the graph
- * (int32 [B][N + 1 + N K]), sel a buffer of B N O 8-byte elements, duv [B, 2 O, N] the gradients
- * of u and v. tk3d_mlp_edge_supported: the sizes these take (N <= 32768, K <= 255). */
+ * over the K neighbours: y(i, k) = W1 (x_j - x_i) + W2 x_i, j = index[b, i, k] (x_j = 0 for an index
+ * outside [0,N)), where w [O][2 C] = [W1 W2] and x [B, C, N].
+ * tk3d_mlp_edge_forward_f32: the extreme of y [B, O, N]; uv is a buffer [B, N, 2 O] where
+ * tk3d_mlp_edge_terms_wanted(C), else it may be NULL. tk3d_mlp_edge_features_f32 makes the edge
+ * features themselves, [B, 2 C, N, K]. Backward: lists is the inverse of the graph (int32
+ * [B][N + 1 + N K], tk3d_mlp_edge_lists), extreme and arg [B, O, N] the y at the maxima and their
+ * places, coef as tk3d_mlp_grad_coefficients_f32 leaves it; dx [B, C, N] may be NULL, dw is like w.
+ * tk3d_mlp_edge_supported: the sizes these take (N <= 32768, K <= 255). */
 int tk3d_mlp_edge_supported(int64_t B, int64_t N, int64_t K, int64_t O);
-int tk3d_mlp_edge_weights_f32(const float *w, int O, int C, float *out, void *stream);
 int tk3d_mlp_edge_features_f32(const float *x, const int64_t *index, int B, int C, int N, int K,
                                float *out, void *stream);
-int tk3d_mlp_edge_forward_f32(const float *uv, const int64_t *index, const float *gamma, int B, int N,
-                              int K, int O, float *extreme, float *sum, void *stream);
+int tk3d_mlp_edge_terms_wanted(int C);
+int tk3d_mlp_edge_forward_f32(const float *x, const int64_t *index, const float *w, const float *gamma,
+                              int B, int N, int K, int C, int O, float *uv, float *extreme, void *stream);
 int tk3d_mlp_edge_lists(const int64_t *index, int B, int N, int K, int32_t *lists, void *stream);
+int64_t tk3d_mlp_edge_backward_bytes(int B, int N, int O, int C);
 int tk3d_mlp_edge_backward_f32(const float *g, const float *extreme, const unsigned char *arg,
-                               const float *uv, const float *sum, const int32_t *lists, int B, int N,
-                               int K, int O, const tk3d_mlp_norm *norm, const float *coef, void *sel,
-                               float *duv, void *stream);
+                               const float *x, const int64_t *index, const int32_t *lists, const float *w,
+                               int B, int N, int K, int C, int O, const tk3d_mlp_norm *norm,
+                               const float *coef, void *workspace, float *dx, float *dw, void *stream);
 
 #ifdef __cplusplus
 }

@@ -1,84 +1,120 @@
-// EdgeConv with one layer, pooled over the neighbours (include/tk3d_mlp.h): the layer is linear in
-// the edge feature [x_j - x_i, x_i], so y(i, j) = u_j + v_i with u = W1 x and v = (W2 - W1) x, two
-// products per POINT instead of one per edge, and nothing of the size of the edges is ever stored:
-// the forward gathers the u of a point's neighbours and keeps the extreme, its place, the sum and
-// the statistics; the backward gathers, through the inverse of the graph, what the edges into a
-// point contribute. Bound by the L2: a row of 64 channels (256 bytes) per edge and direction.
+// EdgeConv with one layer, pooled over the neighbours (include/tk3d_mlp.h). The layer is linear in the
+// edge feature [x_j - x_i, x_i], so what runs over the edges are gathers of rows per point, and the
+// products are per point: nothing of the size of the edges is stored but what the stock modules leave
+// in training. Bound by the L2 (a row of 64 channels, 256 bytes, per edge and direction) and, in the
+// products, by the rate of the fp64 matrix instructions (79 TFLOP/s).
+//
+// Why fp64: y taken apart into a term of j and one of i loses what the difference of near
+// neighbours keeps. With fp32 products u + v of [W1 x]_j and [(W2 - W1) x]_i is 1.6 to 2.3 times as far
+// from float64 as the product with the edge feature, and dW1 = du x^T - dv x^T up to 2.7 times; with
+// fp64 products, rounded once, u + v 0.2 to 0.4 times (C = 64; below kDirect channels evaluation takes
+// the differences themselves, 0.7 times), dW1 0.2 to 0.3 and dx 0.4 to 0.6 times on clouds about the
+// origin. Far from it both forms are as exact as the statistics that the library saved.
 #include "mlp_common.h"
 
 namespace {
 
 constexpr int kPoints = 32;    // points of a workgroup
 constexpr int kChannels = 64;  // channels of a workgroup: a lane is a channel
+constexpr int kGather = 16;    // points of a workgroup that gathers in the backward: waves to hide trips
 constexpr int kAtOnce = 8;     // rows requested before the first is used
+constexpr int kDirect = 16;    // channels from which u + v is the more exact form in evaluation
 
-// out [2 O][C]: W1, then W2 - W1, from w [O][2 C].
-__global__ void __launch_bounds__(kBlock) edge_weights_kernel(const float *w, int O, int C, float *out)
-{
-    const int n = O * C;
-    for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
-        const int o = i / C, c = i - o * C;
-        const float w1 = w[(int64_t)o * 2 * C + c], w2 = w[(int64_t)o * 2 * C + C + c];
-        out[i] = w1;
-        out[n + i] = w2 - w1;
+// The maximum over neighbours as one over signed y.
+struct Best {
+    float value, chosen;
+    __device__ __forceinline__ void take(float y, float sign, bool first)
+    {
+        const float s = y * sign;
+        // (the first NaN stays, as in torch's maximum)
+        const bool up = first || (!(s <= value) && value == value);
+        value = up ? s : value;
+        chosen = up ? y : chosen;
     }
-}
+};
 
-// A workgroup takes 32 points, a wave eight of them, a lane one of 64 channels. Consecutive
+// The extreme of y over the neighbours: CIN 0: y = u_j + v_i with uv in `source`; else from the cloud
+// x [B, C, N] in `source` itself, C <= CIN: the differences in fp32 as in an edge feature, the rest
+// of y, which is the same for all neighbours, in fp64, so that y is rounded once.
+// A workgroup takes 32 points, a wave eight of them, a lane one of 64 output channels. Consecutive
 // workgroups take different batch elements, so that an XCD's L2 holds the rows of few.
+template <int CIN>
 __global__ void __launch_bounds__(kBlock)
-    edge_forward_kernel(const float *__restrict__ uv, const int64_t *__restrict__ index,
-                        const float *__restrict__ gamma, int B, int N, int K, int O, int total,
-                        float *__restrict__ extreme, float *__restrict__ sum)
+    edge_forward_kernel(const float *__restrict__ source, const int64_t *__restrict__ index,
+                        const float *__restrict__ w, const float *__restrict__ gamma, int B, int N,
+                        int K, int C, int O, int total, float *__restrict__ extreme)
 {
     __shared__ float values[kChannels][kPoints + 1];
+    constexpr int AT_ONCE = CIN > 4 ? 2 : kAtOnce;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int cbase = blockIdx.y * kChannels;
     const int c = cbase + lane < O ? cbase + lane : O - 1;
     const float sign = sign_of(gamma[c]);
+    float w1[CIN ? CIN : 1];
+    if constexpr (CIN != 0)
+#pragma unroll
+        for (int a = 0; a < CIN; ++a)
+            w1[a] = a < C ? w[(int64_t)c * 2 * C + a] : 0.0f;
     for (int tile = blockIdx.x; tile < total; tile += gridDim.x) {
         const int b = tile % B, first = tile / B * kPoints;
-        const float *u = uv + (int64_t)b * N * 2 * O + c;
+        const float *u = source + (int64_t)b * N * 2 * O + c;
+        const float *x = source + (int64_t)b * C * N;
         for (int q = 0; q < kPoints / kWaves; ++q) {
             const int local = wave * (kPoints / kWaves) + q, i = first + local;
             if (i >= N)
                 break;
             const int64_t *row = index + ((int64_t)b * N + i) * K;
-            const float v = u[(int64_t)i * 2 * O + O];
-            float best = 0.0f, chosen = 0.0f, total_u = 0.0f;
-            for (int k0 = 0; k0 < K; k0 += kAtOnce) {
-                float r[kAtOnce];
+            Best best{0.0f, 0.0f};
+            if constexpr (CIN == 0) {
+                const float v = u[(int64_t)i * 2 * O + O];
+                for (int k0 = 0; k0 < K; k0 += AT_ONCE) {
+                    float r[AT_ONCE];
 #pragma unroll
-                for (int k = 0; k < kAtOnce; ++k) {
-                    const int64_t j = row[k0 + k < K ? k0 + k : K - 1];
-                    r[k] = j >= 0 && j < N ? u[j * 2 * O] : 0.0f;
+                    for (int k = 0; k < AT_ONCE; ++k) {
+                        const int64_t j = row[k0 + k < K ? k0 + k : K - 1];
+                        r[k] = j >= 0 && j < N ? u[j * 2 * O] : 0.0f;
+                    }
+#pragma unroll
+                    for (int k = 0; k < AT_ONCE; ++k)
+                        if (k0 + k < K)
+                            best.take(r[k] + v, sign, k0 + k == 0);
                 }
+            } else {
+                float xi[CIN];
+                double v = 0.0;
 #pragma unroll
-                for (int k = 0; k < kAtOnce; ++k) {
-                    if (k0 + k >= K)
-                        break;
-                    const float y = r[k] + v;
-                    total_u += r[k];
-                    const float s = y * sign;
-                    // (the first NaN stays, as in torch's maximum)
-                    const bool up = k0 + k == 0 || (!(s <= best) && best == best);
-                    best = up ? s : best;
-                    chosen = up ? y : chosen;
+                for (int a = 0; a < CIN; ++a) {
+                    xi[a] = a < C ? x[(int64_t)a * N + i] : 0.0f;
+                    v = __builtin_fma(a < C ? (double)w[(int64_t)c * 2 * C + C + a] : 0.0, (double)xi[a], v);
+                }
+                for (int k0 = 0; k0 < K; k0 += AT_ONCE) {
+                    float r[AT_ONCE][CIN];
+#pragma unroll
+                    for (int k = 0; k < AT_ONCE; ++k) {
+                        const int64_t j = row[k0 + k < K ? k0 + k : K - 1];
+                        const bool in = j >= 0 && j < N;
+#pragma unroll
+                        for (int a = 0; a < CIN; ++a)
+                            r[k][a] = in && a < C ? x[(int64_t)a * N + j] : 0.0f;
+                    }
+#pragma unroll
+                    for (int k = 0; k < AT_ONCE; ++k) {
+                        float s = 0.0f;
+#pragma unroll
+                        for (int a = 0; a < CIN; ++a)
+                            s = __builtin_fmaf(w1[a], r[k][a] - xi[a], s);
+                        if (k0 + k < K)
+                            best.take((float)(v + (double)s), sign, k0 + k == 0);
+                    }
                 }
             }
-            values[lane][local] = chosen;
-            if (sum && cbase + lane < O)
-                sum[((int64_t)b * N + i) * O + c] = total_u;
+            values[lane][local] = best.chosen;
         }
-        if (!extreme)
-            continue;
         __syncthreads();
         for (int e = tid; e < kChannels * kPoints; e += kBlock) {
             const int ch = e / kPoints, p = e % kPoints;
-            if (cbase + ch < O && first + p < N) {
-                const int64_t at = ((int64_t)b * O + cbase + ch) * N + first + p;
-                extreme[at] = values[ch][p];
-            }
+            if (cbase + ch < O && first + p < N)
+                extreme[((int64_t)b * O + cbase + ch) * N + first + p] = values[ch][p];
         }
         __syncthreads();
     }
@@ -180,6 +216,21 @@ __global__ void __launch_bounds__(1024)
     }
 }
 
+// The edges into point j, as positions of the entries. (The lists come from the caller: whatever they
+// hold, nothing outside is read.)
+struct Run {
+    int from, to;
+};
+__device__ __forceinline__ Run edges_into(const int *start, int j, int N, int K)
+{
+    const int from = min(max(start[j], 0), N * K);
+    return {from, min(max(start[j + 1], from), N * K)};
+}
+__device__ __forceinline__ int point_of(int entry, int N)
+{
+    return min((unsigned)entry >> 8, (unsigned)N - 1u);
+}
+
 // The sparse gradient, [B, N, O] of (a e, place), from g, extreme and arg [B, O, N].
 __global__ void __launch_bounds__(kBlock)
     edge_select_kernel(const float *g, const float *extreme, const unsigned char *arg, int N, int O,
@@ -205,66 +256,433 @@ __global__ void __launch_bounds__(kBlock)
     }
 }
 
-// dy(i, k) = (a e)_i [k is the place] + b y + d, summed over the edges into a point (du) and out of
-// it (dv); out [B, 2 O, N]: du, then dv.
+// What the sparse gradient adds to du and dv: out [B, 2 O, N], the a e of the edges into a point whose
+// place they are, then a point's own.
 __global__ void __launch_bounds__(kBlock)
-    edge_backward_kernel(const float *__restrict__ uv, const int2 *__restrict__ sel,
-                         const float *__restrict__ sum, const int *__restrict__ lists,
-                         const float *__restrict__ coef, int B, int N, int K, int O,
-                         float *__restrict__ out)
+    edge_sparse_kernel(const int2 *__restrict__ sel, const int *__restrict__ lists, int B, int N, int K,
+                       int O, float *__restrict__ out)
 {
-    __shared__ float du[kChannels][kPoints + 1], dv[kChannels][kPoints + 1];
+    __shared__ float du[kChannels][kGather + 1], dv[kChannels][kGather + 1];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int cbase = blockIdx.y * kChannels;
     const int c = cbase + lane < O ? cbase + lane : O - 1;
-    const int b = blockIdx.x % B, first = blockIdx.x / B * kPoints;
-    const float kb = coef[c * 4 + 1], kd = coef[c * 4 + 2];
-    const float *u = uv + (int64_t)b * N * 2 * O + c;
+    const int b = blockIdx.x % B, first = blockIdx.x / B * kGather;
     const int2 *selected = sel + (int64_t)b * N * O + c;
     const int *start = lists + (int64_t)b * (N + 1 + (int64_t)N * K);
     const int *entries = start + N + 1;
-    for (int q = 0; q < kPoints / kWaves; ++q) {
-        const int local = wave * (kPoints / kWaves) + q, j = first + local;
+    for (int q = 0; q < kGather / kWaves; ++q) {
+        const int local = wave * (kGather / kWaves) + q, j = first + local;
         if (j >= N)
             break;
-        // (the lists come from the caller: whatever they hold, nothing outside is read)
-        const int from = min(max(start[j], 0), N * K), to = min(max(start[j + 1], from), N * K);
+        const Run run = edges_into(start, j, N, K);
         double acc = 0.0;
-        for (int e0 = from; e0 < to; e0 += kAtOnce) {
-            float v[kAtOnce];
+        for (int e0 = run.from; e0 < run.to; e0 += kAtOnce) {
             int2 s[kAtOnce];
             int k[kAtOnce];
 #pragma unroll
             for (int i = 0; i < kAtOnce; ++i) {
-                const int entry = entries[e0 + i < to ? e0 + i : to - 1];
-                const int64_t at = min((unsigned)entry >> 8, (unsigned)N - 1u);
+                const int entry = entries[e0 + i < run.to ? e0 + i : run.to - 1];
                 k[i] = entry & 255;
-                v[i] = u[at * 2 * O + O];
-                s[i] = selected[at * O];
+                s[i] = selected[(int64_t)point_of(entry, N) * O];
             }
 #pragma unroll
-            for (int i = 0; i < kAtOnce; ++i) {
-                if (e0 + i >= to)
-                    break;
-                acc += (double)__builtin_fmaf(kb, v[i], s[i].y == k[i] ? __int_as_float(s[i].x) : 0.0f);
-            }
+            for (int i = 0; i < kAtOnce; ++i)
+                if (e0 + i < run.to && s[i].y == k[i])
+                    acc += (double)__int_as_float(s[i].x);
         }
-        const float deg = (float)(to - from), all = (float)K;
-        const float uj = u[(int64_t)j * 2 * O], vj = u[(int64_t)j * 2 * O + O];
-        du[lane][local] = (float)(acc + (double)deg * ((double)kb * (double)uj + (double)kd));
-        const float s = sum[((int64_t)b * N + j) * O + c];
-        dv[lane][local] = __int_as_float(selected[(int64_t)j * O].x) +
-                          __builtin_fmaf(kb, __builtin_fmaf(all, vj, s), all * kd);
+        du[lane][local] = (float)acc;
+        dv[lane][local] = __int_as_float(selected[(int64_t)j * O].x);
     }
     __syncthreads();
-    for (int e = tid; e < kChannels * kPoints; e += kBlock) {
-        const int ch = e / kPoints, p = e % kPoints;
+    for (int e = tid; e < kChannels * kGather; e += kBlock) {
+        const int ch = e / kGather, p = e % kGather;
         if (cbase + ch < O && first + p < N) {
             float *row = out + ((int64_t)b * 2 * O + cbase + ch) * N + first + p;
             row[0] = du[ch][p];
             row[(int64_t)O * N] = dv[ch][p];
         }
     }
+}
+
+// x [B, C, N] as rows of points [B, N, C].
+__global__ void __launch_bounds__(kBlock) edge_rows_kernel(const float *x, int C, int N, float *rows)
+{
+    __shared__ float tile[kPoints][kChannels + 1];
+    const int tid = threadIdx.x, first = blockIdx.x * kPoints, cbase = blockIdx.y * kChannels;
+    const int64_t b = blockIdx.z;
+    for (int e = tid; e < kChannels * kPoints; e += kBlock) {
+        const int ch = e / kPoints, p = e % kPoints;
+        if (cbase + ch < C && first + p < N)
+            tile[p][ch] = x[(b * C + cbase + ch) * N + first + p];
+    }
+    __syncthreads();
+    for (int e = tid; e < kChannels * kPoints; e += kBlock) {
+        const int p = e / kChannels, ch = e % kChannels;
+        if (cbase + ch < C && first + p < N)
+            rows[(b * N + first + p) * C + cbase + ch] = tile[p][ch];
+    }
+}
+
+// The sums of the differences to the neighbours, out [B, 2 C, N]: s = sum of x_i - x_j over the edges
+// i -> j into a point, then t = sum of x_j - x_i over the edges out of it (x_j = 0 outside the cloud).
+// W of them lie side by side in a wave: channels of one point.
+template <int W>
+__global__ void __launch_bounds__(kBlock)
+    edge_neighbours_kernel(const float *__restrict__ rows, const int64_t *__restrict__ index,
+                           const int *__restrict__ lists, int B, int N, int K, int C,
+                           float *__restrict__ out)
+{
+    __shared__ float into[W][kGather + 1], from[W][kGather + 1];
+    constexpr int AT_ONCE = kBlock / W;  // points
+    const int tid = threadIdx.x, lane = tid % W;
+    const int sub = W == 64 ? __builtin_amdgcn_readfirstlane(tid / W) : tid / W;
+    const int cbase = blockIdx.y * W;
+    const int c = cbase + lane < C ? cbase + lane : C - 1;
+    const int b = blockIdx.x % B, first = blockIdx.x / B * kGather;
+    const float *x = rows + (int64_t)b * N * C + c;
+    const int *start = lists + (int64_t)b * (N + 1 + (int64_t)N * K);
+    const int *entries = start + N + 1;
+    for (int local = sub; local < kGather && first + local < N; local += AT_ONCE) {
+        const int p = first + local;
+        const float own = x[(int64_t)p * C];
+        const Run run = edges_into(start, p, N, K);
+        double s = 0.0, t = 0.0;
+        for (int e0 = run.from; e0 < run.to; e0 += kAtOnce) {
+            float v[kAtOnce];
+#pragma unroll
+            for (int i = 0; i < kAtOnce; ++i)
+                v[i] = x[(int64_t)point_of(entries[e0 + i < run.to ? e0 + i : run.to - 1], N) * C];
+#pragma unroll
+            for (int i = 0; i < kAtOnce; ++i)
+                s += e0 + i < run.to ? (double)(v[i] - own) : 0.0;
+        }
+        const int64_t *neighbours = index + ((int64_t)b * N + p) * K;
+        for (int k0 = 0; k0 < K; k0 += kAtOnce) {
+            float v[kAtOnce];
+#pragma unroll
+            for (int i = 0; i < kAtOnce; ++i) {
+                const int64_t j = neighbours[k0 + i < K ? k0 + i : K - 1];
+                v[i] = j >= 0 && j < N ? x[j * C] : 0.0f;
+            }
+#pragma unroll
+            for (int i = 0; i < kAtOnce; ++i)
+                t += k0 + i < K ? (double)(v[i] - own) : 0.0;
+        }
+        into[lane][local] = (float)s;
+        from[lane][local] = (float)t;
+    }
+    __syncthreads();
+    for (int e = tid; e < W * kGather; e += kBlock) {
+        const int ch = e / kGather, p = e % kGather;
+        if (cbase + ch < C && first + p < N) {
+            float *row = out + ((int64_t)b * 2 * C + cbase + ch) * N + first + p;
+            row[0] = into[ch][p];
+            row[(int64_t)C * N] = from[ch][p];
+        }
+    }
+}
+
+// ---- the products, in fp64 -------------------------------------------------------------------------
+//
+// result(m, n) = sum over k of a(m, k) b(k, n) for what an Op makes of its tensors: 64 x 64 results a
+// workgroup, 32 x 32 a wave (2 x 2 tiles of the 16 x 16 x 4 instruction), sixteen k at a time in LDS,
+// the next sixteen requested before these are multiplied. Rows of LDS are 82 doubles: writes along k
+// then meet few banks twice. An Op loads what an element is made of (m, n and k clamped to the last)
+// and makes it of that in a second function, called when the element goes to LDS: the loads are in
+// flight during a whole step. (8 x 2048 points, mean over DGCNN's four blocks: gradients 27 us, weights
+// 15, input 16; 44, 29 and 24 where the loading function made the element, and so waited for it.)
+
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+constexpr int kTile = 64, kDepth = 16, kPitch = kTile + 18;
+
+struct Raw {
+    float p, q;
+};
+struct Rest {  // of a result: times * sum + plus
+    double times, plus;
+};
+
+template <typename Op> __global__ void __launch_bounds__(kBlock) edge_product_kernel(Op op)
+{
+    __shared__ double at[kDepth][kPitch], bt[kDepth][kPitch];
+    constexpr int EACH = kTile * kDepth / kBlock;  // elements of either tile a thread loads
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int m0 = blockIdx.y * kTile, n0 = blockIdx.x * kTile, z = blockIdx.z;
+    const int from = op.from(z), to = op.to(z);
+    // (consecutive threads walk the direction in which the tensor lies in memory)
+    const auto place = [&](bool along_k, int i, int &k, int &x) {
+        k = along_k ? tid % kDepth : tid / kTile + kBlock / kTile * i;
+        x = along_k ? tid / kDepth + kBlock / kDepth * i : tid % kTile;
+    };
+    int am[EACH], bn[EACH];
+    double column[EACH];  // what b() wants to know of its n
+#pragma unroll
+    for (int i = 0; i < EACH; ++i) {
+        int k, x;
+        place(Op::kAlongKA, i, k, x);
+        am[i] = min(m0 + x, op.rows - 1);
+        place(Op::kAlongKB, i, k, x);
+        bn[i] = min(n0 + x, op.cols - 1);
+        column[i] = op.column(bn[i], z, m0);
+    }
+    Raw ar[EACH], br[EACH];
+    const auto load = [&](int k0) {
+        const int b = op.batch(z, k0);
+#pragma unroll
+        for (int i = 0; i < EACH; ++i) {
+            int k, x;
+            place(Op::kAlongKA, i, k, x);
+            ar[i] = op.load_a(am[i], op.clamped(min(k0 + k, to - 1), b), b);
+            place(Op::kAlongKB, i, k, x);
+            br[i] = op.load_b(bn[i], op.clamped(min(k0 + k, to - 1), b), b, m0);
+        }
+    };
+    f64x4 acc[2][2] = {};
+    const int row = (wave >> 1) * 32, col = (wave & 1) * 32;
+    load(from);
+    for (int k0 = from; k0 < to; k0 += kDepth) {
+        const int b = op.batch(z, k0);
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < EACH; ++i) {
+            int k, x;
+            place(Op::kAlongKA, i, k, x);
+            const double av = op.a(ar[i], am[i], k0 + k);
+            at[k][x] = k0 + k < to && op.inside(k0 + k, b) ? av : 0.0;
+            place(Op::kAlongKB, i, k, x);
+            const double bv = op.b(br[i], bn[i], k0 + k, column[i]);
+            bt[k][x] = k0 + k < to && op.inside(k0 + k, b) ? bv : 0.0;
+        }
+        __syncthreads();
+        if (k0 + kDepth < to)
+            load(k0 + kDepth);
+#pragma unroll
+        for (int k = 0; k < kDepth; k += 4) {
+            double a[2], b[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                a[i] = at[k + (lane >> 4)][row + 16 * i + (lane & 15)];
+                b[i] = bt[k + (lane >> 4)][col + 16 * i + (lane & 15)];
+            }
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b[j], acc[i][j], 0, 0, 0);
+        }
+    }
+    // (everything that the results are put together with is requested before the first store)
+    Rest rest[2][2][4];
+    const auto each = [&](auto f) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    f(m0 + row + 16 * i + 4 * v + (lane >> 4), n0 + col + 16 * j + (lane & 15),
+                      rest[i][j][v], acc[i][j][v]);
+    };
+    each([&](int m, int n, Rest &r, double) {
+        r = op.rest(min(m, op.rows - 1), min(n, op.cols - 1), z);
+    });
+    each([&](int m, int n, const Rest &r, double sum) {
+        if (m < op.rows && n < op.cols)
+            op.store(m, n, z, __builtin_fma(r.times, sum, r.plus));
+    });
+}
+
+// What most Ops have nothing to say about. (The functions a() and b() ignore what they do not need.)
+struct PlainOp {
+    __device__ int batch(int z, int) const { return z; }
+    __device__ int from(int) const { return 0; }
+    __device__ int clamped(int k, int) const { return k; }
+    __device__ bool inside(int, int) const { return true; }
+    __device__ double column(int, int, int) const { return 0.0; }
+    __device__ Rest rest(int, int, int) const { return {1.0, 0.0}; }
+};
+
+// uv [B, N, 2 O]: a point a row, u = W1 x then v = (W2 - W1) x. m = points, n = u and v, k = channels.
+struct EdgeTermsOp : PlainOp {
+    static constexpr bool kAlongKA = false, kAlongKB = true;
+    const float *x, *w;
+    float *uv;
+    int C, O, rows, cols;  // rows = N, cols = 2 O
+    __device__ int to(int) const { return C; }
+    __device__ Raw load_a(int p, int c, int b) const
+    {
+        return {(x + (int64_t)b * C * rows)[(unsigned)(c * rows + p)], 0.0f};
+    }
+    __device__ double a(Raw r, int, int) const { return r.p; }
+    __device__ Raw load_b(int n, int c, int, int) const
+    {
+        const unsigned at = (n < O ? n : n - O) * 2 * C + c;
+        return {w[at], w[at + C]};
+    }
+    __device__ double b(Raw r, int n, int, double) const { return n < O ? r.p : (double)r.q - (double)r.p; }
+    __device__ void store(int p, int n, int b, double v) const
+    {
+        uv[((int64_t)b * rows + p) * cols + n] = (float)v;
+    }
+};
+
+// duv [B, 2 O, N] in place, from the sparse parts: the sum of dy = a e + b (y - mean) + d0 over the
+// edges into a point (du) and out of it (dv). y is linear in the edge feature:
+//     into j:   sum of y = (W2 - W1) s_j + W2 (deg x_j)
+//     out of i: sum of y = W1 t_i + W2 (K x_i)
+// m = du then dv, `half` each (a multiple of the tile: a block is all du or all dv), n = points, k =
+// the channels of s or t, then those of x.
+struct EdgeGradOp : PlainOp {
+    static constexpr bool kAlongKA = true, kAlongKB = false;
+    const float *x, *st, *w, *coef, *mean;  // st [B, 2 C, N]: s, then t
+    const int *lists;
+    float *duv;
+    int C, O, K, half, rows, cols;  // rows = 2 half, cols = N
+    __device__ int to(int) const { return 2 * C; }
+    __device__ int edges(int p, int b, bool out) const
+    {
+        if (out)
+            return K;
+        const Run run = edges_into(lists + (int64_t)b * (cols + 1 + (int64_t)cols * K), p, cols, K);
+        return run.to - run.from;
+    }
+    __device__ int channel(int m) const { return min(m >= half ? m - half : m, O - 1); }
+    __device__ Raw load_a(int m, int k, int) const
+    {
+        const unsigned row = channel(m) * 2 * C;  // (W1, W2 side by side)
+        return {w[row + k], w[row + min(k + C, 2 * C - 1)]};
+    }
+    __device__ double a(Raw r, int m, int k) const
+    {
+        return m >= half || k >= C ? r.p : (double)r.q - (double)r.p;
+    }
+    __device__ double column(int p, int b, int m0) const { return edges(p, b, m0 >= half); }
+    __device__ Raw load_b(int p, int k, int b, int m0) const
+    {
+        const float *own = x + (int64_t)b * C * cols;
+        const float *sums = st + ((int64_t)b * 2 + (m0 >= half)) * C * cols;
+        return {(k < C ? sums : own)[(unsigned)((k < C ? k : k - C) * cols + p)], 0.0f};
+    }
+    __device__ double b(Raw r, int, int k, double count) const { return k < C ? r.p : count * (double)r.p; }
+    __device__ float *result(int m, int p, int b) const
+    {
+        return duv + ((int64_t)b * 2 * O + (m >= half ? O : 0) + channel(m)) * cols + p;
+    }
+    __device__ Rest rest(int m, int p, int b) const
+    {
+        const f32x4 k = reinterpret_cast<const f32x4 *>(coef)[channel(m)];
+        const double n = edges(p, b, m >= half);
+        return {k.y, (double)*result(m, p, b) + n * ((double)k.w - (double)k.y * (double)mean[channel(m)])};
+    }
+    __device__ void store(int m, int p, int b, double v) const
+    {
+        if ((m >= half ? m - half : m) < O)
+            *result(m, p, b) = (float)v;
+    }
+};
+
+// dx [B, C, N] = W1^T du + (W2 - W1)^T dv. m = channels, n = points, k = du then dv.
+struct EdgeInputOp : PlainOp {
+    static constexpr bool kAlongKA = false, kAlongKB = false;
+    const float *duv, *w;
+    float *dx;
+    int O, rows, cols;  // rows = C, cols = N
+    __device__ int to(int) const { return 2 * O; }
+    __device__ Raw load_a(int c, int k, int) const
+    {
+        const unsigned at = (k < O ? k : k - O) * 2 * rows + c;
+        return {w[at], w[at + rows]};
+    }
+    __device__ double a(Raw r, int, int k) const { return k < O ? r.p : (double)r.q - (double)r.p; }
+    __device__ Raw load_b(int p, int k, int b, int) const
+    {
+        return {(duv + (int64_t)b * 2 * O * cols)[(unsigned)(k * cols + p)], 0.0f};
+    }
+    __device__ double b(Raw r, int, int, double) const { return r.p; }
+    __device__ void store(int c, int p, int b, double v) const
+    {
+        dx[((int64_t)b * rows + c) * cols + p] = (float)v;
+    }
+};
+
+// dW1 = (du - dv) x^T and dW2 = dv x^T, partial[z][2 half][C]. The dv of a channel add up to zero, so
+// dW2 may count x from its first point: their rounding then does not meet how far x is from zero. (The
+// du do so only where no neighbour is outside the cloud.) m = rows of dW1 then of dW2, n = channels, k =
+// the points of all batch elements, each filled up to `padded`, a multiple of the depth.
+struct EdgeWeightOp : PlainOp {
+    static constexpr bool kAlongKA = true, kAlongKB = true;
+    const float *x, *duv;
+    double *partial;
+    int N, O, half, padded, run, total, rows, cols;  // rows = 2 half, cols = C
+    __device__ int batch(int, int k0) const { return k0 / padded; }
+    __device__ int from(int z) const { return z * run; }
+    __device__ int to(int z) const { return total - z * run < run ? total : (z + 1) * run; }
+    __device__ int clamped(int k, int b) const { return min(k - b * padded, N - 1); }
+    __device__ bool inside(int k, int b) const { return k - b * padded < N; }
+    __device__ Raw load_a(int m, int p, int b) const
+    {
+        const float *du = duv + (int64_t)b * 2 * O * N, *dv = du + (int64_t)O * N;
+        const unsigned at = min(m >= half ? m - half : m, O - 1) * N + p;
+        return {du[at], dv[at]};
+    }
+    __device__ double a(Raw r, int m, int) const { return m >= half ? r.q : (double)r.p - (double)r.q; }
+    __device__ double column(int c, int, int m0) const { return m0 >= half ? x[(int64_t)c * N] : 0.0f; }
+    __device__ Raw load_b(int c, int p, int b, int) const
+    {
+        return {(x + (int64_t)b * cols * N)[(unsigned)(c * N + p)], 0.0f};
+    }
+    __device__ double b(Raw r, int, int, double origin) const { return (double)r.p - origin; }
+    __device__ void store(int m, int c, int z, double v) const
+    {
+        partial[((int64_t)z * rows + m) * cols + c] = v;
+    }
+};
+
+// dw [O][2 C] from the partial sums: sixteen outputs to a workgroup, sixteen threads to an output.
+__global__ void __launch_bounds__(kBlock)
+    edge_weight_sum_kernel(const double *partial, int parts, int half, int O, int C, float *dw)
+{
+    __shared__ double lds[kWaves][16];
+    const int at = threadIdx.x & 15, lane = threadIdx.x >> 4, i = blockIdx.x * 16 + at;
+    const int m = i / C, c = i - m * C, o = m < half ? m : m - half;
+    const bool mine = m < 2 * half && o < O;
+    double sum = 0.0;
+    if (mine)
+        for (int z = lane; z < parts; z += 16)
+            sum += partial[((int64_t)z * 2 * half + m) * C + c];
+    sum += __shfl_xor(sum, 16);
+    sum += __shfl_xor(sum, 32);
+    if ((threadIdx.x & 63) < 16)
+        lds[threadIdx.x >> 6][at] = sum;
+    __syncthreads();
+    if (threadIdx.x < 16 && mine)
+        dw[(int64_t)o * 2 * C + (m < half ? 0 : C) + c] =
+            (float)(lds[0][at] + lds[1][at] + lds[2][at] + lds[3][at]);
+}
+
+int tiles_of(int n) { return (n + kTile - 1) / kTile; }
+
+// The points of the weight gradient: padded per batch element, in all, and of one workgroup - four
+// workgroups to a CU, and no less than 128 points.
+struct WeightRuns {
+    int padded, total, run, parts;
+};
+WeightRuns weight_runs(int B, int N, int O, int C)
+{
+    WeightRuns r;
+    r.padded = (N + kDepth - 1) / kDepth * kDepth;
+    r.total = B * r.padded;
+    const int blocks = 2 * tiles_of(O) * tiles_of(C), want = (4 * tk_cu_count() + blocks - 1) / blocks;
+    r.run = ((r.total + want - 1) / want + kDepth - 1) / kDepth * kDepth;
+    r.run = r.run < 128 ? 128 : r.run;
+    r.parts = (r.total + r.run - 1) / r.run;
+    return r;
+}
+
+template <typename Op> int launch_product(const Op &op, int batches, hipStream_t stream)
+{
+    edge_product_kernel<Op><<<dim3(tiles_of(op.cols), tiles_of(op.rows), batches), kBlock, 0, stream>>>(op);
+    return tk_launch_status();
 }
 
 }  // namespace
@@ -274,14 +692,7 @@ extern "C" {
 int tk3d_mlp_edge_supported(int64_t B, int64_t N, int64_t K, int64_t O)
 {
     return B > 0 && B <= 65535 && N > 0 && N <= 32768 && K > 0 && K <= 255 && O > 0 && O <= 4096 &&
-           tk_fits(TK_MAX_I32, B, (N + kPoints - 1) / kPoints) && tk_fits(TK_MAX_I32 / 2, N, K);
-}
-
-int tk3d_mlp_edge_weights_f32(const float *w, int O, int C, float *out, void *stream)
-{
-    const int blocks = (O * C + kBlock - 1) / kBlock;
-    edge_weights_kernel<<<blocks < 256 ? blocks : 256, kBlock, 0, (hipStream_t)stream>>>(w, O, C, out);
-    return tk_launch_status();
+           tk_fits(TK_MAX_I32 / 2, B, N + kPoints) && tk_fits(TK_MAX_I32 / 2, N, K);
 }
 
 int tk3d_mlp_edge_features_f32(const float *x, const int64_t *index, int B, int C, int N, int K,
@@ -298,16 +709,31 @@ int tk3d_mlp_edge_features_f32(const float *x, const int64_t *index, int B, int 
     return tk_launch_status();
 }
 
-int tk3d_mlp_edge_forward_f32(const float *uv, const int64_t *index, const float *gamma, int B, int N,
-                              int K, int O, float *extreme, float *sum, void *stream)
+int tk3d_mlp_edge_terms_wanted(int C) { return C >= kDirect; }
+
+int tk3d_mlp_edge_forward_f32(const float *x, const int64_t *index, const float *w, const float *gamma,
+                              int B, int N, int K, int C, int O, float *uv, float *extreme, void *stream_)
 {
-    if (!tk3d_mlp_edge_supported(B, N, K, O))
+    if (!tk3d_mlp_edge_supported(B, N, K, O) || C <= 0 || C > 4096)
         return TK3D_ERR_UNSUPPORTED;
+    if (tk3d_mlp_edge_terms_wanted(C) && !uv)
+        return TK3D_ERR_NULL_POINTER;
+    const hipStream_t stream = (hipStream_t)stream_;
     const int tiles = B * ((N + kPoints - 1) / kPoints);
     const int most = 4 * tk_cu_count() / B * B;  // (whole rounds of the batch)
-    const int blocks = tiles < most || most == 0 ? tiles : most;
-    edge_forward_kernel<<<dim3(blocks, (O + kChannels - 1) / kChannels), kBlock, 0, (hipStream_t)stream>>>(
-        uv, index, gamma, B, N, K, O, tiles, extreme, sum);
+    const dim3 grid(tiles < most || most == 0 ? tiles : most, (O + kChannels - 1) / kChannels);
+    if (C >= kDirect) {
+        const EdgeTermsOp op{{}, x, w, uv, C, O, N, 2 * O};
+        const int rc = launch_product(op, B, stream);
+        if (rc != TK3D_OK)
+            return rc;
+        edge_forward_kernel<0><<<grid, kBlock, 0, stream>>>(uv, index, w, gamma, B, N, K, C, O, tiles, extreme);
+    } else if (C <= 4) {
+        edge_forward_kernel<4><<<grid, kBlock, 0, stream>>>(x, index, w, gamma, B, N, K, C, O, tiles, extreme);
+    } else {
+        edge_forward_kernel<kDirect><<<grid, kBlock, 0, stream>>>(x, index, w, gamma, B, N, K, C, O, tiles,
+                                                                  extreme);
+    }
     return tk_launch_status();
 }
 
@@ -322,18 +748,55 @@ int tk3d_mlp_edge_lists(const int64_t *index, int B, int N, int K, int32_t *list
     return tk_launch_status();
 }
 
-int tk3d_mlp_edge_backward_f32(const float *g, const float *extreme, const unsigned char *arg,
-                               const float *uv, const float *sum, const int32_t *lists, int B, int N,
-                               int K, int O, const tk3d_mlp_norm *norm, const float *coef, void *sel,
-                               float *duv, void *stream)
+int64_t tk3d_mlp_edge_backward_bytes(int B, int N, int O, int C)
 {
-    if (!tk3d_mlp_edge_supported(B, N, K, O))
+    const int64_t partial = (int64_t)weight_runs(B, N, O, C).parts * 2 * tiles_of(O) * kTile * C * 8;
+    const int64_t points = (int64_t)B * N * 4;
+    return partial + points * (2 * O + 2 * O + 3 * (int64_t)C);
+}
+
+int tk3d_mlp_edge_backward_f32(const float *g, const float *extreme, const unsigned char *arg,
+                               const float *x, const int64_t *index, const int32_t *lists, const float *w,
+                               int B, int N, int K, int C, int O, const tk3d_mlp_norm *norm,
+                               const float *coef, void *workspace, float *dx, float *dw, void *stream_)
+{
+    if (!tk3d_mlp_edge_supported(B, N, K, O) || C <= 0 || C > 4096)
         return TK3D_ERR_UNSUPPORTED;
+    const hipStream_t stream = (hipStream_t)stream_;
+    const WeightRuns r = weight_runs(B, N, O, C);
+    const int half = tiles_of(O) * kTile;
+    // the workspace: partial sums, sel [B, N, O] of 8 bytes, duv [B, 2 O, N], rows [B, N, C], st [B, 2 C, N]
+    double *partial = reinterpret_cast<double *>(workspace);
+    int2 *sel = reinterpret_cast<int2 *>(partial + (int64_t)r.parts * 2 * half * C);
+    float *duv = reinterpret_cast<float *>(sel + (int64_t)B * N * O);
+    float *rows = duv + (int64_t)B * N * 2 * O, *st = rows + (int64_t)B * N * C;
     const int tiles = (N + kPoints - 1) / kPoints, blocks = (O + kChannels - 1) / kChannels;
-    edge_select_kernel<<<dim3(tiles, blocks, B), kBlock, 0, (hipStream_t)stream>>>(
-        g, extreme, arg, N, O, *norm, coef, reinterpret_cast<int2 *>(sel));
-    edge_backward_kernel<<<dim3(tiles * B, blocks), kBlock, 0, (hipStream_t)stream>>>(
-        uv, reinterpret_cast<const int2 *>(sel), sum, lists, coef, B, N, K, O, duv);
+    const int gathers = (N + kGather - 1) / kGather * B;
+    edge_select_kernel<<<dim3(tiles, blocks, B), kBlock, 0, stream>>>(g, extreme, arg, N, O, *norm, coef,
+                                                                    sel);
+    edge_sparse_kernel<<<dim3(gathers, blocks), kBlock, 0, stream>>>(sel, lists, B, N, K, O, duv);
+    edge_rows_kernel<<<dim3(tiles, (C + kChannels - 1) / kChannels, B), kBlock, 0, stream>>>(x, C, N, rows);
+    if (C <= 4)
+        edge_neighbours_kernel<4><<<dim3(gathers, 1), kBlock, 0, stream>>>(rows, index, lists, B, N, K, C, st);
+    else if (C <= 16)
+        edge_neighbours_kernel<16><<<dim3(gathers, 1), kBlock, 0, stream>>>(rows, index, lists, B, N, K, C,
+                                                                             st);
+    else
+        edge_neighbours_kernel<64><<<dim3(gathers, (C + 63) / 64), kBlock, 0, stream>>>(rows, index, lists,
+                                                                                        B, N, K, C, st);
+    const EdgeGradOp grad{{}, x, st, w, coef, norm->mean, lists, duv, C, O, K, half, 2 * half, N};
+    int rc = launch_product(grad, B, stream);
+    if (rc == TK3D_OK && dx) {
+        const EdgeInputOp input{{}, duv, w, dx, O, C, N};
+        rc = launch_product(input, B, stream);
+    }
+    if (rc != TK3D_OK)
+        return rc;
+    const EdgeWeightOp weight{{}, x, duv, partial, N, O, half, r.padded, r.run, r.total, 2 * half, C};
+    rc = launch_product(weight, r.parts, stream);
+    if (rc != TK3D_OK)
+        return rc;
+    edge_weight_sum_kernel<<<(2 * half * C + 15) / 16, kBlock, 0, stream>>>(partial, r.parts, half, O, C, dw);
     return tk_launch_status();
 }
 

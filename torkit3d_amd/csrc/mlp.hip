@@ -727,8 +727,8 @@ __device__ __forceinline__ Coefficients grad_coefficients(double2 s, double n, c
                                       : 1.0 / __builtin_sqrt((double)norm.var[c] + (double)norm.eps);
     const double gamma = norm.gamma[c], mean = norm.mean[c];
     const double b = -gamma * is * is * is * s.y / n;
-    const double d = -gamma * is * s.x / n - b * (mean - origin);
-    return {f32x4{(float)(gamma * is), (float)b, (float)d, 0.0f}, (float)(s.y * is), (float)s.x};
+    const double d0 = -gamma * is * s.x / n, d = d0 - b * (mean - origin);
+    return {f32x4{(float)(gamma * is), (float)b, (float)d, (float)d0}, (float)(s.y * is), (float)s.x};
 }
 
 __global__ void __launch_bounds__(kBlock)

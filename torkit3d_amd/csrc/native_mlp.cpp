@@ -634,7 +634,7 @@ struct EdgeCall {
 };
 
 struct EdgeKept {
-    Tensor matrix, uv, extreme, arg, sum, mean, var;
+    Tensor extreme, arg, mean, var;
 };
 
 tk3d_mlp_norm norm_of(const EdgeCall &c, const EdgeKept &k)
@@ -648,24 +648,6 @@ Tensor edge_forward(const EdgeCall &c, EdgeKept &k)
     const int64_t C = c.x.size(1);
     const auto options = c.x.options();
     void *stream = stream_of(c.x);
-    k.matrix = at::empty({2 * O, C}, options);
-    done(tk3d_mlp_edge_weights_f32(f32(c.weight), (int)O, (int)C, f32(k.matrix), stream),
-         "tk3d_mlp_edge_weights_f32");
-    k.uv = at::empty({B, N, 2 * O}, options);
-    tk3d_mlp_product p = product(B, 2 * O, N);
-    p.src[0] = source(c.x, f32(k.matrix), 1, C);
-    p.out = f32(k.uv);
-    run_product(TK3D_MLP_IN_RAW, TK3D_MLP_OUT_POINTS, p, stream);
-    if (c.training)
-        k.sum = at::empty({B, N, O}, options);
-    if (!c.training) {
-        k.extreme = at::empty({B, O, N}, options);
-        k.mean = c.running_mean;
-        k.var = c.running_var;
-    }
-    done(tk3d_mlp_edge_forward_f32(f32(k.uv), c.index.data_ptr<int64_t>(), f32(c.gamma), (int)B,
-                                   (int)N, (int)K, (int)O, f32(k.extreme), f32(k.sum), stream),
-         "tk3d_mlp_edge_forward_f32");
     if (c.training) {  // (bit by bit what the stock modules give, see forward_training)
         const Tensor edges = at::empty({B, 2 * C, N, K}, options);
         done(tk3d_mlp_edge_features_f32(f32(c.x), c.index.data_ptr<int64_t>(), (int)B, (int)C, (int)N,
@@ -679,6 +661,16 @@ Tensor edge_forward(const EdgeCall &c, EdgeKept &k)
         k.var = n.inv_std;
         return pool_max(n, k.extreme, k.arg);
     }
+    k.extreme = at::empty({B, O, N}, options);
+    k.mean = c.running_mean;
+    k.var = c.running_var;
+    Tensor uv;
+    if (tk3d_mlp_edge_terms_wanted((int)C))
+        uv = at::empty({B, N, 2 * O}, options);
+    done(tk3d_mlp_edge_forward_f32(f32(c.x), c.index.data_ptr<int64_t>(), f32(c.weight), f32(c.gamma),
+                                   (int)B, (int)N, (int)K, (int)C, (int)O, f32(uv), f32(k.extreme),
+                                   stream),
+         "tk3d_mlp_edge_forward_f32");
     const Tensor z = at::empty({B, O, N}, options);
     const tk3d_mlp_norm norm = norm_of(c, k);
     done(tk3d_mlp_activate_f32(f32(k.extreme), B * O, (int)O, (int)N, &norm, f32(z), stream),
@@ -702,35 +694,17 @@ variable_list edge_backward(const EdgeCall &c, const EdgeKept &k, const Tensor &
     done(tk3d_mlp_grad_coefficients_f32(partial.data_ptr(), slots, B * N * K, (int)O, &norm,
                                         f32(coef), f32(affine), f32(affine) + O, stream),
          "tk3d_mlp_grad_coefficients_f32");
-    const Tensor sel = at::empty({B, N, O, 2}, options), duv = at::empty({B, 2 * O, N}, options);
-    done(tk3d_mlp_edge_backward_f32(f32(g), f32(k.extreme), k.arg.data_ptr<uint8_t>(), f32(k.uv),
-                                    f32(k.sum), c.lists.data_ptr<int32_t>(), (int)B, (int)N, (int)K,
-                                    (int)O, &norm, f32(coef), sel.data_ptr(), f32(duv), stream),
-         "tk3d_mlp_edge_backward_f32");
-    // dW1 = du x^T - dv x^T, dW2 = dv x^T
-    tk3d_mlp_outer o{};
-    o.B = (int32_t)B;
-    o.P = (int32_t)N;
-    o.row = source(duv, nullptr, 0, 0);
-    o.col = source(c.x, nullptr, 0, 0);
-    const int splits = tk3d_mlp_outer_splits(&o);
-    const Tensor parts = at::empty({splits, 2 * O, C}, options);
-    o.partial = f32(parts);
-    done(tk3d_mlp_outer_f32(TK3D_MLP_ROW_RAW, TK3D_MLP_COL_RAW, &o, stream), "tk3d_mlp_outer_f32");
     const Tensor dw = at::empty(c.weight.sizes(), options);
-    const float *of_u = f32(parts), *of_v = of_u + O * C;
-    const tk3d_mlp_sum sums[2] = {
-        {of_u, of_v, f32(dw), 2 * O * C, splits, (int32_t)O, (int32_t)C, (int32_t)(2 * C)},
-        {of_v, nullptr, f32(dw) + C, 2 * O * C, splits, (int32_t)O, (int32_t)C, (int32_t)(2 * C)}};
-    done(tk3d_mlp_sum_f32(sums, 2, stream), "tk3d_mlp_sum_f32");
     Tensor dx;
-    if (want_x) {
+    if (want_x)
         dx = at::empty(c.x.sizes(), options);
-        tk3d_mlp_product p = product(B, C, N);
-        p.src[0] = source(duv, f32(k.matrix), C, 1);
-        p.out = f32(dx);
-        run_product(TK3D_MLP_IN_RAW, TK3D_MLP_OUT_PLAIN, p, stream);
-    }
+    const Tensor workspace =
+        at::empty({tk3d_mlp_edge_backward_bytes((int)B, (int)N, (int)O, (int)C)}, options.dtype(at::kByte));
+    done(tk3d_mlp_edge_backward_f32(f32(g), f32(k.extreme), k.arg.data_ptr<uint8_t>(), f32(c.x),
+                                    c.index.data_ptr<int64_t>(), c.lists.data_ptr<int32_t>(),
+                                    f32(c.weight), (int)B, (int)N, (int)K, (int)C, (int)O, &norm,
+                                    f32(coef), workspace.data_ptr(), f32(dx), f32(dw), stream),
+         "tk3d_mlp_edge_backward_f32");
     return {dx, dw, affine.select(0, 0), affine.select(0, 1)};
 }
 
@@ -756,7 +730,7 @@ struct EdgeNode : torch::autograd::Function<EdgeNode> {
         EdgeKept k;
         const Tensor z = edge_forward(call, k);
         ctx->save_for_backward({call.x, call.index, call.lists, call.weight, call.gamma, call.beta,
-                                k.matrix, k.uv, k.extreme, k.arg, k.sum, k.mean, k.var});
+                                k.extreme, k.arg, k.mean, k.var});
         ctx->saved_data["training"] = call.training;
         ctx->saved_data["eps"] = call.eps;
         ctx->saved_data["want_x"] = x.requires_grad();
@@ -774,13 +748,10 @@ struct EdgeNode : torch::autograd::Function<EdgeNode> {
         c.weight = s[3];
         c.gamma = s[4];
         c.beta = s[5];
-        k.matrix = s[6];
-        k.uv = s[7];
-        k.extreme = s[8];
-        k.arg = s[9];
-        k.sum = s[10];
-        k.mean = c.running_mean = s[11];
-        k.var = c.running_var = s[12];
+        k.extreme = s[6];
+        k.arg = s[7];
+        k.mean = c.running_mean = s[8];
+        k.var = c.running_var = s[9];
         c.training = ctx->saved_data["training"].toBool();
         c.eps = ctx->saved_data["eps"].toDouble();
         const bool want_x = ctx->saved_data["want_x"].toBool();
