@@ -61,6 +61,12 @@ __device__ __forceinline__ void load_run(float (&dst)[PT], const float *base, un
             dst[t] = v[t];
 }
 
+// Evaluation adds up sixteen channels at a time and these sums on top of each other, in tiles of 32 x
+// 32, which have the registers, in four chains over every fourth group of channels: in one chain over
+// all channels the error grows with their number (768 -> 256 channels: 3.5e-7 of the result, 1.9 times
+// that of the library's product, which runs in up to four chains; 64 -> 128: 1.4 times).
+constexpr bool short_chains(int out) { return out == OUT_EVAL || out == OUT_POOL_EVAL || out == OUT_POINTS; }
+
 constexpr bool reads_y(int in) { return in == IN_GRAD || in == IN_GRAD_OUT; }
 
 // Channel groups that are requested at once: 16 bytes per lane and channel pair of the wide tiles
@@ -167,15 +173,32 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
                 load_group(r, d, b, pos, step * D + d);
     };
 
-    tk_f32x16 acc[PT][CT];
+    constexpr bool SHORT = short_chains(OUT) && PT * CT > 1;
+    constexpr int CHAINS = short_chains(OUT) && PT * CT == 1 ? kDepth<1> : 1;
+    tk_f32x16 acc[PT][CT * CHAINS], total[SHORT ? PT : 1][SHORT ? CT : 1];
     const auto clear = [&] {
 #pragma unroll
         for (int t = 0; t < PT; ++t)
 #pragma unroll
-            for (int ct = 0; ct < CT; ++ct)
+            for (int ct = 0; ct < CT * CHAINS; ++ct)
 #pragma unroll
-                for (int r = 0; r < 16; ++r)
+                for (int r = 0; r < 16; ++r) {
                     acc[t][ct][r] = 0.0f;
+                    if constexpr (SHORT)
+                        total[t][ct][r] = 0.0f;
+                }
+    };
+    const auto end_chain = [&] {
+        if constexpr (SHORT)
+#pragma unroll
+            for (int t = 0; t < PT; ++t)
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        total[t][ct][r] += acc[t][ct][r];
+                        acc[t][ct][r] = 0.0f;
+                    }
     };
 
     const auto multiply_group = [&](const Rows<IN, PT> &r, int d, int tile, int g, int first) {
@@ -230,15 +253,19 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
 #pragma unroll
             for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
-                for (int t = 0; t < PT; ++t)
-                    acc[t][ct] = __builtin_amdgcn_mfma_f32_32x32x2f32(v[q][t], w[ct][q], acc[t][ct],
-                                                                      0, 0, 0);
+                for (int t = 0; t < PT; ++t) {
+                    tk_f32x16 &sum = acc[t][CHAINS > 1 ? d : ct];
+                    sum = __builtin_amdgcn_mfma_f32_32x32x2f32(v[q][t], w[ct][q], sum, 0, 0, 0);
+                }
     };
     const auto multiply = [&](const Rows<IN, PT> &r, int tile, int step, int first) {
 #pragma unroll
         for (int d = 0; d < D; ++d)
-            if (D == 1 || step * D + d < a.kg)
+            if (D == 1 || step * D + d < a.kg) {
                 multiply_group(r, d, tile, step * D + d, first);
+                if (d % 2 == 1 || D == 1)
+                    end_chain();
+            }
     };
 
     // Per-lane constants and sums of the output channels (lane = channel).
@@ -264,6 +291,13 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
     }
 
     const auto finish = [&](int tile) {
+        if (D > 1)
+            end_chain();  // (of an odd number of groups)
+        if constexpr (CHAINS > 1)
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                acc[0][0][r] = (acc[0][0][r] + acc[0][1][r]) + (acc[0][2][r] + acc[0][3][r]);
+        static_assert(CHAINS == 1 || CHAINS == 4, "one chain per group of a step");
         const int b = tile / a.tiles;
         const int base = (tile - b * a.tiles) * (32 * PT);
         const bool full = base + 32 * PT <= P;
@@ -290,7 +324,7 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
                 for (int i = 0; i < 4; ++i)
 #pragma unroll
                     for (int t = 0; t < PT; ++t)
-                        v[i * PT + t] = acc[t][ct][4 * q + i];
+                        v[i * PT + t] = SHORT ? total[SHORT ? t : 0][SHORT ? ct : 0][4 * q + i] : acc[t][ct][4 * q + i];
                 if constexpr (OUT == OUT_MASK || OUT == OUT_PLAIN) {
 #pragma unroll
                     for (int i = 0; i < RUN; ++i)
@@ -1230,7 +1264,12 @@ struct Shape {
 // that are multiples of four, a group of 64 positions needs a tile that holds it. A masked gradient
 // reads as much on the way out as on the way in, and waits for it with nothing of its own to do: half
 // the positions a wave leave room for twice the waves (64 -> 64 channels, 16 x 16384 positions:
-// 4 x 2 tiles 116 us, 2 x 2 tiles 72 us; at 32 channels and less there is nothing between).
+// 4 x 2 tiles 116 us, 2 x 2 tiles 72 us; at 32 channels and less there is nothing between). In
+// evaluation the sums of the short chains take as many registers as the chains themselves: 2 x 2 too.
+bool short_chains_of(int out)
+{
+    return out == TK3D_MLP_OUT_EVAL || out == TK3D_MLP_OUT_POOL_EVAL || out == TK3D_MLP_OUT_POINTS;
+}
 Shape pick_shape(int out, const tk3d_mlp_product &p)
 {
     const int simds = 4 * tk_cu_count();
@@ -1243,7 +1282,7 @@ Shape pick_shape(int out, const tk3d_mlp_product &p)
     if (p.C <= 32 && waves(4, 1) >= simds)
         return {4, 1};
     if (p.C > 32 && waves(4, 2) >= simds)
-        return out == TK3D_MLP_OUT_MASK ? Shape{2, 2} : Shape{4, 2};
+        return out == TK3D_MLP_OUT_MASK || short_chains_of(out) ? Shape{2, 2} : Shape{4, 2};
     if (waves(2, 2) >= simds || (pooled && p.group > 32))
         return {2, 2};
     return {1, 1};
@@ -1288,7 +1327,7 @@ int launch_product(const GemmArgs &g, int cblocks, hipStream_t stream)
 template <int IN, int OUT>
 int launch_shape(const GemmArgs &g, Shape s, int cblocks, hipStream_t stream)
 {
-    if constexpr (OUT != OUT_MASK)
+    if constexpr (OUT == OUT_PLAIN)
         if (s.pt == 4 && s.ct == 2)
             return launch_product<IN, OUT, 4, 2>(g, cblocks, stream);
     if (s.pt == 4)
