@@ -107,7 +107,7 @@ int tk3d_chamfer_distance_forward_bcn_f64(const double *xyz1, const double *xyz2
 /* chamfer_distance_forward on a copy of both clouds as [B, rows, 3] with rows the next multiple of
  * four, which the sweeps read faster than ragged lengths and short [B,3,N] clouds. `workspace`:
  * 16-byte aligned device memory of at least the size that
- * tk3d_chamfer_distance_forward_rows_bytes returns, which is 0 for shapes that are as fast
+ * tk3d_chamfer_distance_forward_rows_bytes returns, which is 0 for shapes that are as fast or faster
  * without (pass on to the calls above). Results are bit-identical to theirs. */
 size_t tk3d_chamfer_distance_forward_rows_bytes(int64_t B, int64_t N1, int64_t N2, int channels_first);
 int tk3d_chamfer_distance_forward_rows_f32(const float *xyz1, const float *xyz2, int channels_first,

@@ -161,3 +161,26 @@ def test_chamfer_workspace_size_and_argument_checks(lib):
               ctypes.c_size_t(0), NULL) == -2
     assert fn(NULL, NULL, i64(0), i64(8), i64(8), NULL, NULL, NULL, NULL, NULL,
               ctypes.c_size_t(0), NULL) == 0
+
+
+# Calls that lost to the copy (or took it for nothing), then calls that win by it, as timed.
+@pytest.mark.parametrize("b,n1,n2,channels_first,copied", [
+    (1, 1025, 1025, 0, False),    # the only batch element starts on 16 bytes as it is
+    (2, 1025, 1025, 0, False),    # few workgroups: the vector pre-filter
+    (128, 1000, 999, 0, False),
+    (4, 2049, 400, 0, False),     # few workgroups, a short cloud: the exact sweep
+    (32, 489, 1130, 0, False),    # the matrix kernel, but the last 128 keys are nearly full
+    (4, 5001, 300, 1, False), (1, 2049, 400, 1, False), (8, 126, 1144, 1, False),
+    (16, 1024, 2048, 0, False), (16, 1024, 2048, 1, False),
+    (16, 1025, 1025, 0, True), (8, 4099, 4097, 0, True), (4, 7569, 1552, 0, True),
+    (24, 1550, 8803, 0, True),
+    (1, 1025, 1025, 1, True), (8, 2500, 3001, 1, True), (8, 5001, 300, 1, True),
+    (8, 1000, 1000, 1, True), (1, 257, 300, 1, True),
+])
+def test_chamfer_clouds_are_copied_where_it_pays(lib, b, n1, n2, channels_first, copied):
+    fn = lib.tk3d_chamfer_distance_forward_rows_bytes
+    fn.restype = ctypes.c_size_t
+    for sizes in ((n1, n2), (n2, n1)):
+        padded = sum((n + 3) // 4 * 4 for n in sizes)
+        want = b * padded * 12 if copied else 0
+        assert fn(i64(b), i64(sizes[0]), i64(sizes[1]), ctypes.c_int(channels_first)) == want

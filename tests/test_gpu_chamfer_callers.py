@@ -18,7 +18,8 @@ def clouds(b, n1, n2, dtype=torch.float32):
 # matrix kernel's shortest
 @pytest.mark.parametrize("transpose", [False, True])
 @pytest.mark.parametrize("b,n1,n2", [(2, 255, 256), (3, 256, 257), (2, 259, 1000), (2, 1021, 1023),
-                                     (2, 1024, 1025), (3, 1027, 300), (8, 2500, 3001), (2, 4099, 1)])
+                                     (2, 1024, 1025), (3, 1027, 300), (8, 2500, 3001), (2, 4099, 1),
+                                     (1, 1025, 1025), (16, 1025, 1027), (32, 489, 1130), (8, 5001, 300)])
 def test_copied_clouds(cuda, b, n1, n2, transpose):
     x, y = clouds(b, n1, n2)
     a, c = [(t.transpose(1, 2) if transpose else t).contiguous().to(cuda) for t in (x, y)]

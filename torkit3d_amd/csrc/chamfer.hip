@@ -1901,6 +1901,44 @@ inline double chamfer_sweep_cost(int64_t B, int64_t N1, int64_t N2, int qpl, int
     return (want_slices > 1 ? 20.0 : 12.0) + cycles / 2100.0;
 }
 
+// Matrix-core pre-filter, 512 queries per workgroup: the fastest sweep from about a
+// hundred workgroups on key clouds of 1024 points or more (1.3-2.2x over the
+// vector pre-filter). A workgroup sweeps its direction's whole key cloud unless
+// that leaves fewer than 256 workgroups or - clouds of very different lengths -
+// a few workgroups with most of the work: a direction's key cloud is then cut
+// into slices no longer than 1/256 of all the sweeping (and no shorter than 1024
+// keys), each direction on its own (B=1, 200000 x 2048: 1.99 -> 0.07 ms).
+// Returns the number of workgroups, and the slices of either direction.
+inline int64_t chamfer_matrix_blocks(int64_t B, int64_t N1, int64_t N2, int (&want)[2])
+{
+    const int64_t qb[2] = {B * ((N1 + 511) / 512), B * ((N2 + 511) / 512)};
+    const int64_t nk[2] = {N2, N1};
+    const double sweep = (double)qb[0] * (double)nk[0] + (double)qb[1] * (double)nk[1];
+    double longest = sweep / 256.0;
+    longest = longest < 1024.0 ? 1024.0 : longest;
+    double len[2];
+    for (int w = 0; w < 2; ++w) {
+        const double parts = (double)nk[w] / longest;
+        want[w] = parts <= 1.0 ? 1 : parts >= 256.0 ? 256 : (int)(parts + 0.999);
+        len[w] = (double)nk[w] / want[w];
+    }
+    // ... and no workgroup sweeps more than twice what the other direction's do
+    // (the long ones would run on alone at the end)
+    const double shorter = len[0] < len[1] ? len[0] : len[1];
+    const double cap = 2.0 * shorter < 1024.0 ? 1024.0 : 2.0 * shorter;
+    int64_t blocks = 0;
+    for (int w = 0; w < 2; ++w) {
+        if (len[w] > cap) {
+            const double parts = (double)nk[w] / cap;
+            want[w] = parts >= 256.0 ? 256 : (int)(parts + 0.999);
+        }
+        int64_t slice_len;
+        blocks += qb[w] * chamfer_slices(nk[w], want[w], 128, slice_len);
+    }
+    return blocks;
+}
+constexpr int64_t CHAMFER_MATRIX_BLOCKS = 96;  // fewer: the vector pre-filter ([N,3] clouds)
+
 // rows1, rows2: points from one batch element to the next where that is more than N1, N2.
 template <typename T, bool SOA = false>
 int chamfer_forward(const T *xyz1, const T *xyz2, int64_t B, int64_t N1, int64_t N2,
@@ -1924,39 +1962,9 @@ int chamfer_forward(const T *xyz1, const T *xyz2, int64_t B, int64_t N1, int64_t
         // The pre-filter pays off once the key clouds are a few hundred points long
         // (its prologue passes over the keys twice per workgroup).
         const int64_t nkmin = N1 < N2 ? N1 : N2;
-        // Matrix-core pre-filter, 512 queries per workgroup: the fastest sweep from about a
-        // hundred workgroups on key clouds of 1024 points or more (1.3-2.2x over the
-        // vector pre-filter). A workgroup sweeps its direction's whole key cloud unless
-        // that leaves fewer than 256 workgroups or - clouds of very different lengths -
-        // a few workgroups with most of the work: a direction's key cloud is then cut
-        // into slices no longer than 1/256 of all the sweeping (and no shorter than 1024
-        // keys), each direction on its own (B=1, 200000 x 2048: 1.99 -> 0.07 ms).
         if (nkmin >= 1 && (N1 > N2 ? N1 : N2) >= 1024) {
-            const int64_t qb[2] = {B * ((N1 + 511) / 512), B * ((N2 + 511) / 512)};
-            const int64_t nk[2] = {N2, N1};
-            const double sweep = (double)qb[0] * (double)nk[0] + (double)qb[1] * (double)nk[1];
-            double longest = sweep / 256.0;
-            longest = longest < 1024.0 ? 1024.0 : longest;
             int want[2];
-            double len[2];
-            for (int w = 0; w < 2; ++w) {
-                const double parts = (double)nk[w] / longest;
-                want[w] = parts <= 1.0 ? 1 : parts >= 256.0 ? 256 : (int)(parts + 0.999);
-                len[w] = (double)nk[w] / want[w];
-            }
-            // ... and no workgroup sweeps more than twice what the other direction's do
-            // (the long ones would run on alone at the end)
-            const double shorter = len[0] < len[1] ? len[0] : len[1];
-            const double cap = 2.0 * shorter < 1024.0 ? 1024.0 : 2.0 * shorter;
-            int64_t blocks = 0;
-            for (int w = 0; w < 2; ++w) {
-                if (len[w] > cap) {
-                    const double parts = (double)nk[w] / cap;
-                    want[w] = parts >= 256.0 ? 256 : (int)(parts + 0.999);
-                }
-                int64_t slice_len;
-                blocks += qb[w] * chamfer_slices(nk[w], want[w], 128, slice_len);
-            }
+            const int64_t blocks = chamfer_matrix_blocks(B, N1, N2, want);
             // Launches of up to one and a half workgroups per CU (two and a half on key
             // clouds of up to 4096 points) run with two query blocks per wave instead of
             // four: twice the workgroups of half the queries, so the chip holds them all at
@@ -1967,11 +1975,11 @@ int chamfer_forward(const T *xyz1, const T *xyz2, int64_t B, int64_t N1, int64_t
             const int64_t nkmax = N1 > N2 ? N1 : N2;
             // ([3,N] clouds: the vector pre-filter below reads [N,3] only, so the matrix
             // pre-filter also takes the launches of under 96 workgroups)
-            if ((SOA || blocks >= 96) && (blocks <= 384 || (blocks <= 640 && nkmax <= 4096)))
+            if ((SOA || blocks >= CHAMFER_MATRIX_BLOCKS) && (blocks <= 384 || (blocks <= 640 && nkmax <= 4096)))
                 return chamfer_forward_mfma_launch<2, SOA>(xyz1, xyz2, B, N1, N2, dist1, idx1,
                                                            dist2, idx2, s, want[0], want[1],
                                                            rows1, rows2);
-            if (blocks >= 96)
+            if (blocks >= CHAMFER_MATRIX_BLOCKS)
                 return chamfer_forward_mfma_launch<4, SOA>(xyz1, xyz2, B, N1, N2, dist1, idx1,
                                                            dist2, idx2, s, want[0], want[1],
                                                            rows1, rows2);
@@ -3814,19 +3822,36 @@ int chamfer_rows(const T *xyz1, const T *xyz2, bool soa, int64_t B, int64_t N1, 
     return tk_launch_status();
 }
 
-// Where a copy to [B, rows, 3] with rows a multiple of four pays: the matrix kernel re-evaluates its
-// candidates in 48-byte runs of four keys only if every batch element starts on 16 bytes (B=8,
-// 2500 x 3001 points: 51 us with one 12-byte load per key, 79 us with three 4-byte loads on [3,N],
-// 35 us on the copy, which takes 3), and on [3,N] clouds too short for the matrix kernel the vector
-// pre-filter, which reads [N,3] only, beats the exact sweep (8 x 1000 x 1000: 54 -> 22 us).
+// Where a copy to [B, rows, 3] with rows a multiple of four pays (its launch takes 3 us), timed with and
+// without on 200 shapes of 1 to 128 batch elements, 126 to 16384 points:
+// - The matrix kernel re-evaluates its candidates in 48-byte runs of four keys only if a batch element
+//   starts on 16 bytes. On ragged [N,3] clouds that is so of the first, so B = 1 gains nothing (3 us
+//   lost); else 15 to 20 us are saved (B=16, 1025 x 1025 points: 38 -> 20 us; B=8, 4099 x 4097: 59 ->
+//   39 us) as long as the last 128 keys of a cloud, which are re-evaluated key by key either way, are
+//   not nearly full (B=32, 489 x 1130, 105 and 106 keys left over: 38 -> 41 us). Launches of many
+//   workgroups gain all the same (B=24, 1550 x 8803: 107 -> 95 us; 5 to 25 % on eleven shapes, nothing
+//   on four, 2 to 10 % lost on one, 16383 x 1027).
+// - The vector pre-filter and the exact sweep load a key at a time: nothing to gain on [N,3] clouds.
+// - [3,N] clouds: ragged ones cost the matrix kernel three 4-byte loads per key (B=8, 2500 x 3001: 76 ->
+//   41 us), and the vector pre-filter, which reads [N,3] only, beats it below 96 workgroups (B=1, 1025 x
+//   1025: 36 -> 21 us) and beats the exact sweep of clouds too short for it (8 x 1000 x 1000: 54 -> 22
+//   us). It takes clouds from 512 points on; below that, with the longer one at 1024 or more, [N,3]
+//   clouds would go through the exact sweep (B=4, 5001 x 300: 40 us as they are, 165 us copied).
 inline bool chamfer_copy_pays(int64_t B, int64_t N1, int64_t N2, bool soa)
 {
     const int64_t most = N1 > N2 ? N1 : N2, least = N1 > N2 ? N2 : N1;
     if (B <= 0 || least <= 0 || N1 > TK_MAX_I32 / 8 || N2 > TK_MAX_I32 / 8)
         return false;
-    if (most >= 1024)
-        return (N1 & 3) != 0 || (N2 & 3) != 0;
-    return soa && least >= 256;
+    if (most < 1024)
+        return soa && least >= 256;
+    if (((N1 | N2) & 3) == 0)
+        return false;
+    int want[2];
+    const int64_t blocks = chamfer_matrix_blocks(B, N1, N2, want);
+    if (soa)
+        return blocks >= CHAMFER_MATRIX_BLOCKS || least >= 512;
+    const int64_t left1 = N1 & 127, left2 = N2 & 127, left = left1 > left2 ? left1 : left2;
+    return B > 1 && blocks >= CHAMFER_MATRIX_BLOCKS && (left <= 80 || blocks > 384);
 }
 
 template <typename T>
