@@ -214,6 +214,56 @@ def test_pooled_layer_far_from_zero(cuda, b, m, s, widths, far):
         assert errors[0] <= 1.25 * errors[1] + 2e-7, (tuple(e.shape), errors)
 
 
+# Short and long rows, few and many of them, one value a row: the library has a kernel for each.
+@pytest.mark.parametrize("b,c,p", [
+    (2, 5, 1), (3, 7, 33), (32, 64, 20), (2, 64, 510), (64, 32, 512), (1, 16, 516), (8, 3, 1000),
+    (16, 64, 1024), (2, 64, 1028), (40, 33, 2048), (8, 64, 4096), (1, 8, 65536), (16, 32, 16384),
+    (8, 64, 40960), (4, 32, 131072),
+])
+def test_the_backward_takes_the_signs_of_the_library(cuda, b, c, p):
+    """The activations as the backward works them out are those of the library's batch norm, bit by
+    bit."""
+    import ctypes
+
+    from torkit3d_amd import _lib
+
+    class Norm(ctypes.Structure):
+        _fields_ = [(n, ctypes.c_void_p) for n in ("mean", "var", "gamma", "beta")] + [("eps", ctypes.c_float)]
+
+    y = randn(p, b, c, p) * 3 + randn(1, c, 1) * 5
+    gamma, beta = randn(2, c), randn(3, c)
+    z, mean, inv_std, _, backend = torch._batch_norm_impl_index(
+        y, gamma, beta, torch.zeros_like(gamma), torch.ones_like(gamma), True, 0.1, 1e-5, True)
+    assert backend == 2  # MIOpen
+    out = torch.empty_like(y)
+    norm = Norm(*(t.data_ptr() for t in (mean, inv_std, gamma, beta)), -1.0)
+    code = _lib.lib().tk3d_mlp_activate_f32(
+        ctypes.c_void_p(y.data_ptr()), ctypes.c_int64(b * c), ctypes.c_int(c), ctypes.c_int(p),
+        ctypes.byref(norm), ctypes.c_void_p(out.data_ptr()),
+        ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert code == 0 and torch.equal(out, torch.relu(z))
+
+
+@pytest.mark.parametrize("form", ["dense", "edges"])
+def test_without_the_library_training_is_left_to_stock(cuda, form):
+    """torch's own batch norm rounds in another order than the backward takes its signs by."""
+    from torkit3d_amd.ops.edge_conv import EdgeConvBlock
+
+    index = torch.randint(0, 40, (2, 40, 5), generator=torch.Generator().manual_seed(0)).to(cuda)
+    block = EdgeConvBlock(6, (8,)).to(cuda).train()
+    mlp = make(mlp1d_bn_relu, 6, (8, 5), True, cuda)
+    x = randn(1, 2, 6, 40).requires_grad_()
+
+    def ran():
+        if form == "dense":
+            return "Node" in mlp(x).grad_fn.name()
+        return block.convs.forward_edges_max(x, index) is not None
+
+    assert ran()
+    with torch.backends.cudnn.flags(enabled=False):
+        assert not ran()
+
+
 @pytest.mark.parametrize("p", [514, 1030])
 def test_rows_on_which_the_library_differs_run_in_stock(cuda, p):
     mlp = make(mlp1d_bn_relu, 6, (8, 5), True, cuda)

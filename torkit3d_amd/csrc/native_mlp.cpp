@@ -4,6 +4,7 @@
 #include "tk3d_mlp.h"
 
 #include <ATen/TracerMode.h>
+#include <ATen/native/Normalization.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <torch/csrc/autograd/autograd.h>
@@ -41,6 +42,18 @@ float *f32(const Tensor &t) { return t.defined() ? t.data_ptr<float>() : nullptr
 // of [40, 64, 515] are 1e-1 off from float64, 1e-7 at [2, 64, 1023] and [40, 64, 511]. The kernels
 // here are not, but a step on such clouds goes on giving what it gave.
 bool same_gradients(int64_t P) { return P <= 512 || P % 4 == 0; }
+
+// Whether training goes through the library's batch norm, whose order of operations the backward
+// repeats where it asks for a sign (normalised() in mlp_common.h). torch has a kernel of its own, which
+// rounds differently, for what MIOpen does not take and where the user has switched it off
+// (torch.backends.cudnn.enabled).
+bool library_norm(const Tensor &like, at::IntArrayRef shape, const Tensor *params, const Tensor *buffers,
+                  double eps)
+{
+    const Tensor y = at::empty({}, like.options()).expand(shape);
+    return at::native::_select_batch_norm_backend(y, params[1], params[2], buffers[0], buffers[1], true,
+                                                  eps) == at::native::BatchNormBackend::Miopen;
+}
 
 // Saved tensors come back through hooks, which may lay them out anew.
 variable_list dense(variable_list saved)
@@ -880,6 +893,13 @@ Tensor mlp(Tensor x, Tensor x2, const Tensor &xyz, const Tensor &centre, const T
         (widest + 8) * longest > (1 << 29) || B * longest > (1 << 30))
         return Tensor();
     OnDeviceOf guard(c.like().device());
+    for (int64_t l = 0; training && l < L; ++l) {
+        const int64_t C = c.out_channels(l), rows = grouped ? index.size(1) : c.rows;
+        const std::vector<int64_t> y =
+            rows ? std::vector<int64_t>{B, C, rows, P / rows} : std::vector<int64_t>{B, C, P};
+        if (!library_norm(c.like(), y, &c.params[3 * l], &c.buffers[3 * l], c.eps[l]))
+            return Tensor();
+    }
     Tensor z;
     if (training) {
         const auto given = [](const Tensor &t) {
@@ -947,8 +967,9 @@ Tensor edge_conv(const Tensor &x, const Tensor &index, const Tensor &lists,
     OnDeviceOf guard(x.device());
     const bool grads = c10::GradMode::is_enabled() && (x.requires_grad() || c.weight.requires_grad() ||
                                                        c.gamma.requires_grad() || c.beta.requires_grad());
-    if (training != grads)
-        return Tensor();  // (as for mlp())
+    if (training != grads ||  // (as for mlp())
+        (training && !library_norm(x, {B, O, N, K}, params.data(), buffers.data(), eps)))
+        return Tensor();
     if (grads) {
         c.lists = lists.defined() ? lists : edge_lists(c.index, N);
         return EdgeNode::apply(c.x, c.weight, c.gamma, c.beta, c);
