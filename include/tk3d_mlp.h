@@ -103,10 +103,10 @@ typedef struct {
 int tk3d_mlp_outer_splits(const tk3d_mlp_outer *p);
 int tk3d_mlp_outer_f32(int row, int col, const tk3d_mlp_outer *p, void *stream);
 
-/* out[r * ld + c] = sum over the splits of partial[r][c] - minus[r][c] (minus NULL or like
- * partial), rows of C, `stride` elements from one split to the next; n of them in one launch. */
+/* out[r * ld + c] = sum over the splits of partial[r][c], rows of C, `stride` elements from one split
+ * to the next; n of them in one launch. */
 typedef struct {
-    const float *partial, *minus;
+    const float *partial;
     float *out;
     int64_t stride;
     int32_t splits, R, C, ld;

@@ -699,8 +699,7 @@ __global__ void __launch_bounds__(kBlock) mlp_sum_kernel(SumArgs a)
         double sum = 0.0;
 #pragma unroll 4
         for (int k = lane; k < s.splits; k += 16)
-            sum += (double)s.partial[k * s.stride + i] -
-                   (s.minus ? (double)s.minus[k * s.stride + i] : 0.0);
+            sum += (double)s.partial[k * s.stride + i];
         sum += __shfl_xor(sum, 16);
         sum += __shfl_xor(sum, 32);
         if ((threadIdx.x & 63) < 16)
@@ -1404,7 +1403,9 @@ int tk3d_mlp_product_f32(int in, int out, const tk3d_mlp_product *p, void *strea
     GemmArgs g;
     const int cblocks = fill(*p, in, out, s, g);
     const hipStream_t stream = (hipStream_t)stream_;
-#define TK_CASE(IN, OUT)                                                                                 if (in == TK3D_MLP_##IN && out == TK3D_MLP_##OUT)                                                        return launch_shape<IN, OUT>(g, s, cblocks, stream);
+#define TK_CASE(IN, OUT)                                                                        \
+    if (in == TK3D_MLP_##IN && out == TK3D_MLP_##OUT)                                           \
+        return launch_shape<IN, OUT>(g, s, cblocks, stream);
     TK_CASE(IN_RAW, OUT_EVAL)
     TK_CASE(IN_RAW, OUT_PLAIN)
     TK_CASE(IN_RAW, OUT_POINTS)
@@ -1447,7 +1448,9 @@ int tk3d_mlp_outer_f32(int row, int col, const tk3d_mlp_outer *p, void *stream_)
     a.total = p->B * a.units;
     const int splits = tk3d_mlp_outer_splits(p);
     const hipStream_t stream = (hipStream_t)stream_;
-#define TK_CASE(ROW, COL)                                                                                if (row == ROW && col == COL)                                                                            return launch_outer_shape<ROW, COL>(a, splits, stream);
+#define TK_CASE(ROW, COL)                                                                       \
+    if (row == ROW && col == COL)                                                               \
+        return launch_outer_shape<ROW, COL>(a, splits, stream);
     TK_CASE(TK3D_MLP_ROW_RAW, TK3D_MLP_COL_RAW)
     TK_CASE(TK3D_MLP_ROW_GRAD, TK3D_MLP_COL_RAW)
     TK_CASE(TK3D_MLP_ROW_GRAD, TK3D_MLP_COL_ACT)
@@ -1634,9 +1637,9 @@ int tk3d_mlp_pool_weight_grad_f32(const float *sparse, int sparse_splits, const 
                                   void *stream)
 {
     const tk3d_mlp_sum sums[3] = {
-        {sparse, nullptr, dw, (int64_t)O * I, sparse_splits, O, I, I},
-        {xx, nullptr, scratch, (int64_t)I * I, xx_splits, I, I, I},
-        {xsum, nullptr, scratch + (int64_t)I * I, I, xx_splits, 1, I, I}};
+        {sparse, dw, (int64_t)O * I, sparse_splits, O, I, I},
+        {xx, scratch, (int64_t)I * I, xx_splits, I, I, I},
+        {xsum, scratch + (int64_t)I * I, I, xx_splits, 1, I, I}};
     const int rc = tk3d_mlp_sum_f32(sums, 3, stream);
     if (rc != TK3D_OK)
         return rc;

@@ -312,7 +312,7 @@ void outer(int row, int col, tk3d_mlp_outer &o, const Tensor &like, float *out, 
     const Tensor partial = at::empty({splits, o.row.K, o.col.K}, like.options());
     o.partial = f32(partial);
     done(tk3d_mlp_outer_f32(row, col, &o, stream), "tk3d_mlp_outer_f32");
-    pending.sums.push_back({f32(partial), nullptr, out, (int64_t)o.row.K * o.col.K, splits, o.row.K,
+    pending.sums.push_back({f32(partial), out, (int64_t)o.row.K * o.col.K, splits, o.row.K,
                             o.col.K, (int32_t)ld});
     pending.alive.push_back(partial);
 }
@@ -509,7 +509,7 @@ Grads backward(const Call &c, const Kept &k, const Tensor &g, bool want_x, bool 
     return out;
 }
 
-// The same chain in stock operators: for gradients of gradients.
+// The same chain in stock operators (training): for gradients of gradients.
 Tensor in_stock_operators(const Call &c)
 {
     Tensor h;
@@ -529,10 +529,8 @@ Tensor in_stock_operators(const Call &c)
     }
     for (int64_t l = 0; l < c.layers(); ++l) {
         h = at::conv1d(h, c.weight(l).view({c.out_channels(l), c.in_channels(l), 1}));
-        const Tensor none;
-        h = at::batch_norm(h, c.params[3 * l + 1], c.params[3 * l + 2],
-                           c.training ? none : c.buffers[3 * l],
-                           c.training ? none : c.buffers[3 * l + 1], c.training, 0.0, c.eps[l], false);
+        h = at::batch_norm(h, c.params[3 * l + 1], c.params[3 * l + 2], Tensor(), Tensor(), true, 0.0,
+                           c.eps[l], false);
         h = at::relu(h);
     }
     if (c.pool)
@@ -540,10 +538,11 @@ Tensor in_stock_operators(const Call &c)
     return h;
 }
 
-struct Node : torch::autograd::Function<Node> {
+struct Node : torch::autograd::Function<Node> {  // (made in training mode alone)
     // Saved: x, x2, xyz, centre, index, arg, then of every layer weight, gamma, beta, y, mean, var.
-    static Tensor forward(AutogradContext *ctx, const std::optional<Tensor> &x,
-                          const std::optional<Tensor> &x2, at::TensorList params, const Call &call)
+    // (The tensors in front of the call are what autograd sees; the call holds them too.)
+    static Tensor forward(AutogradContext *ctx, const std::optional<Tensor> &, const std::optional<Tensor> &,
+                          at::TensorList, const Call &call)
     {
         Kept k;
         const Tensor z = forward_training(call, k);
@@ -557,10 +556,7 @@ struct Node : torch::autograd::Function<Node> {
         }
         ctx->save_for_backward(std::move(saved));
         ctx->saved_data["pool"] = call.pool;
-        ctx->saved_data["training"] = call.training;
         ctx->saved_data["eps"] = call.eps;
-        ctx->saved_data["x"] = x.has_value();
-        ctx->saved_data["x2"] = x2.has_value();
         ctx->saved_data["want_x"] = call.x.defined() && call.x.requires_grad();
         ctx->saved_data["want_x2"] = call.x2.defined() && call.x2.requires_grad();
         return z;
@@ -578,7 +574,7 @@ struct Node : torch::autograd::Function<Node> {
         c.index = s[4];
         k.arg = s[5];
         c.pool = ctx->saved_data["pool"].toInt();
-        c.training = ctx->saved_data["training"].toBool();
+        c.training = true;
         c.eps = ctx->saved_data["eps"].toDoubleVector();
         const int64_t L = ((int64_t)s.size() - 6) / 6;
         for (int64_t l = 0; l < L; ++l) {
@@ -588,15 +584,11 @@ struct Node : torch::autograd::Function<Node> {
             k.y.push_back(t[3]);
             k.mean.push_back(t[4]);
             k.var.push_back(t[5]);
-            c.buffers.push_back(t[4]);
-            c.buffers.push_back(t[5]);
-            c.buffers.push_back(Tensor());
         }
         const bool want_x = ctx->saved_data["want_x"].toBool();
         const bool want_x2 = ctx->saved_data["want_x2"].toBool();
         // One gradient per tensor that apply() was given.
         variable_list result;
-        const bool has_x = ctx->saved_data["x"].toBool(), has_x2 = ctx->saved_data["x2"].toBool();
         if (c10::GradMode::is_enabled()) {  // a gradient of this gradient will be asked for
             const Tensor z = in_stock_operators(c);
             variable_list inputs;
@@ -625,8 +617,6 @@ struct Node : torch::autograd::Function<Node> {
                     result.push_back(d.params[3 * l + i]);
         }
         result.push_back(Tensor());  // (the call itself)
-        (void)has_x;
-        (void)has_x2;
         return result;
     }
 };
@@ -730,21 +720,18 @@ Tensor edge_in_stock_operators(const EdgeCall &c)
     const Tensor near = at::where(valid, at::gather(c.x, 2, flat), at::zeros({}, c.x.options()));
     Tensor h = at::conv1d(at::cat({near - query, query}, 1),
                           c.weight.view({c.out_channels(), 2 * C, 1}));
-    const Tensor none;
-    h = at::batch_norm(h, c.gamma, c.beta, c.training ? none : c.running_mean,
-                       c.training ? none : c.running_var, c.training, 0.0, c.eps, false);
+    h = at::batch_norm(h, c.gamma, c.beta, Tensor(), Tensor(), true, 0.0, c.eps, false);
     return std::get<0>(at::max(at::relu(h).view({B, c.out_channels(), N, K}), 3));
 }
 
-struct EdgeNode : torch::autograd::Function<EdgeNode> {
-    static Tensor forward(AutogradContext *ctx, const Tensor &x, const Tensor &weight,
-                          const Tensor &gamma, const Tensor &beta, const EdgeCall &call)
+struct EdgeNode : torch::autograd::Function<EdgeNode> {  // (made in training mode alone)
+    static Tensor forward(AutogradContext *ctx, const Tensor &x, const Tensor &, const Tensor &,
+                          const Tensor &, const EdgeCall &call)
     {
         EdgeKept k;
         const Tensor z = edge_forward(call, k);
         ctx->save_for_backward({call.x, call.index, call.lists, call.weight, call.gamma, call.beta,
                                 k.extreme, k.arg, k.mean, k.var});
-        ctx->saved_data["training"] = call.training;
         ctx->saved_data["eps"] = call.eps;
         ctx->saved_data["want_x"] = x.requires_grad();
         return z;
@@ -763,9 +750,9 @@ struct EdgeNode : torch::autograd::Function<EdgeNode> {
         c.beta = s[5];
         k.extreme = s[6];
         k.arg = s[7];
-        k.mean = c.running_mean = s[8];
-        k.var = c.running_var = s[9];
-        c.training = ctx->saved_data["training"].toBool();
+        k.mean = s[8];
+        k.var = s[9];
+        c.training = true;
         c.eps = ctx->saved_data["eps"].toDouble();
         const bool want_x = ctx->saved_data["want_x"].toBool();
         variable_list d;
