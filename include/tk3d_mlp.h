@@ -170,18 +170,19 @@ int tk3d_mlp_group_f32(const float *u, const float *xyz, const float *centre, co
 /* EdgeConv (torkit3d/ops/edge_conv.py) with one layer, on a graph of a cloud with itself, pooled
  * over the K neighbours: y(i, k) = W1 (x_j - x_i) + W2 x_i, j = index[b, i, k] (x_j = 0 for an index
  * outside [0,N)), where w [O][2 C] = [W1 W2] and x [B, C, N].
- * tk3d_mlp_edge_forward_f32: the extreme of y [B, O, N]; uv is a buffer [B, N, 2 O] where
- * tk3d_mlp_edge_terms_wanted(C), else it may be NULL. tk3d_mlp_edge_features_f32 makes the edge
+ * tk3d_mlp_edge_forward_f32: the extreme of y [B, O, N]; tk3d_mlp_edge_features_f32: the edge
  * features themselves, [B, 2 C, N, K]. Backward: lists is the inverse of the graph (int32
  * [B][N + 1 + N K], tk3d_mlp_edge_lists), extreme and arg [B, O, N] the y at the maxima and their
  * places, coef as tk3d_mlp_grad_coefficients_f32 leaves it; dx [B, C, N] may be NULL, dw is like w.
+ * Workspaces, aligned to 8 bytes, have the sizes that the _bytes functions return.
  * tk3d_mlp_edge_supported: the sizes these take (N <= 32768, K <= 255). */
 int tk3d_mlp_edge_supported(int64_t B, int64_t N, int64_t K, int64_t O);
 int tk3d_mlp_edge_features_f32(const float *x, const int64_t *index, int B, int C, int N, int K,
                                float *out, void *stream);
-int tk3d_mlp_edge_terms_wanted(int C);
+int64_t tk3d_mlp_edge_forward_bytes(int B, int N, int C, int O);
 int tk3d_mlp_edge_forward_f32(const float *x, const int64_t *index, const float *w, const float *gamma,
-                              int B, int N, int K, int C, int O, float *uv, float *extreme, void *stream);
+                              int B, int N, int K, int C, int O, void *workspace, float *extreme,
+                              void *stream);
 int tk3d_mlp_edge_lists(const int64_t *index, int B, int N, int K, int32_t *lists, void *stream);
 int64_t tk3d_mlp_edge_backward_bytes(int B, int N, int O, int C);
 int tk3d_mlp_edge_backward_f32(const float *g, const float *extreme, const unsigned char *arg,

@@ -7,9 +7,10 @@
 // Why fp64: y taken apart into a term of j and one of i loses what the difference of near
 // neighbours keeps. With fp32 products u + v of [W1 x]_j and [(W2 - W1) x]_i is 1.6 to 2.3 times as far
 // from float64 as the product with the edge feature, and dW1 = du x^T - dv x^T up to 2.7 times; with
-// fp64 products, rounded once, u + v 0.2 to 0.4 times (C = 64; below kDirect channels evaluation takes
-// the differences themselves, 0.7 times), dW1 0.2 to 0.3 and dx 0.4 to 0.6 times on clouds about the
-// origin. Far from it both forms are as exact as the statistics that the library saved.
+// fp64 products, rounded once, u + v 0.2 to 0.4 times (C = 64; at C = 3 it would be 1.2 to 1.5 times, so
+// that below kRounded channels the sum is rounded and not its terms: 0.7 times), dW1 0.2 to 0.3 and dx
+// 0.4 to 0.6 times on clouds about the origin. Far from it both forms are as exact as the statistics
+// that the library saved. (With u and v in fp64 at any C DGCNN's evaluation is 3 to 4 % slower.)
 #include "mlp_common.h"
 
 namespace {
@@ -17,98 +18,52 @@ namespace {
 constexpr int kPoints = 32;    // points of a workgroup
 constexpr int kChannels = 64;  // channels of a workgroup: a lane is a channel
 constexpr int kGather = 16;    // points of a workgroup that gathers in the backward: waves to hide trips
+constexpr int kRounded = 16;   // channels from which u and v may be rounded before they are added
 constexpr int kAtOnce = 8;     // rows requested before the first is used
-constexpr int kDirect = 16;    // channels from which u + v is the more exact form in evaluation
 
-// The maximum over neighbours as one over signed y.
-struct Best {
-    float value, chosen;
-    __device__ __forceinline__ void take(float y, float sign, bool first)
-    {
-        const float s = y * sign;
-        // (the first NaN stays, as in torch's maximum)
-        const bool up = first || (!(s <= value) && value == value);
-        value = up ? s : value;
-        chosen = up ? y : chosen;
-    }
-};
-
-// The extreme of y over the neighbours: CIN 0: y = u_j + v_i with uv in `source`; else from the cloud
-// x [B, C, N] in `source` itself, C <= CIN: the differences in fp32 as in an edge feature, the rest
-// of y, which is the same for all neighbours, in fp64, so that y is rounded once.
+// The extreme of y = u_j + v_i over the neighbours.
 // A workgroup takes 32 points, a wave eight of them, a lane one of 64 output channels. Consecutive
 // workgroups take different batch elements, so that an XCD's L2 holds the rows of few.
-template <int CIN>
+template <typename T>
 __global__ void __launch_bounds__(kBlock)
-    edge_forward_kernel(const float *__restrict__ source, const int64_t *__restrict__ index,
-                        const float *__restrict__ w, const float *__restrict__ gamma, int B, int N,
-                        int K, int C, int O, int total, float *__restrict__ extreme)
+    edge_forward_kernel(const T *__restrict__ uv, const int64_t *__restrict__ index,
+                        const float *__restrict__ gamma, int B, int N, int K, int O, int total,
+                        float *__restrict__ extreme)
 {
     __shared__ float values[kChannels][kPoints + 1];
-    constexpr int AT_ONCE = CIN > 4 ? 2 : kAtOnce;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int cbase = blockIdx.y * kChannels;
     const int c = cbase + lane < O ? cbase + lane : O - 1;
     const float sign = sign_of(gamma[c]);
-    float w1[CIN ? CIN : 1];
-    if constexpr (CIN != 0)
-#pragma unroll
-        for (int a = 0; a < CIN; ++a)
-            w1[a] = a < C ? w[(int64_t)c * 2 * C + a] : 0.0f;
     for (int tile = blockIdx.x; tile < total; tile += gridDim.x) {
         const int b = tile % B, first = tile / B * kPoints;
-        const float *u = source + (int64_t)b * N * 2 * O + c;
-        const float *x = source + (int64_t)b * C * N;
+        const T *u = uv + (int64_t)b * N * 2 * O + c;
         for (int q = 0; q < kPoints / kWaves; ++q) {
             const int local = wave * (kPoints / kWaves) + q, i = first + local;
             if (i >= N)
                 break;
             const int64_t *row = index + ((int64_t)b * N + i) * K;
-            Best best{0.0f, 0.0f};
-            if constexpr (CIN == 0) {
-                const float v = u[(int64_t)i * 2 * O + O];
-                for (int k0 = 0; k0 < K; k0 += AT_ONCE) {
-                    float r[AT_ONCE];
+            const T v = u[(int64_t)i * 2 * O + O];
+            float best = 0.0f, chosen = 0.0f;
+            for (int k0 = 0; k0 < K; k0 += kAtOnce) {
+                T r[kAtOnce];
 #pragma unroll
-                    for (int k = 0; k < AT_ONCE; ++k) {
-                        const int64_t j = row[k0 + k < K ? k0 + k : K - 1];
-                        r[k] = j >= 0 && j < N ? u[j * 2 * O] : 0.0f;
-                    }
-#pragma unroll
-                    for (int k = 0; k < AT_ONCE; ++k)
-                        if (k0 + k < K)
-                            best.take(r[k] + v, sign, k0 + k == 0);
+                for (int k = 0; k < kAtOnce; ++k) {
+                    const int64_t j = row[k0 + k < K ? k0 + k : K - 1];
+                    r[k] = j >= 0 && j < N ? u[j * 2 * O] : (T)0;
                 }
-            } else {
-                float xi[CIN];
-                double v = 0.0;
 #pragma unroll
-                for (int a = 0; a < CIN; ++a) {
-                    xi[a] = a < C ? x[(int64_t)a * N + i] : 0.0f;
-                    v = __builtin_fma(a < C ? (double)w[(int64_t)c * 2 * C + C + a] : 0.0, (double)xi[a], v);
-                }
-                for (int k0 = 0; k0 < K; k0 += AT_ONCE) {
-                    float r[AT_ONCE][CIN];
-#pragma unroll
-                    for (int k = 0; k < AT_ONCE; ++k) {
-                        const int64_t j = row[k0 + k < K ? k0 + k : K - 1];
-                        const bool in = j >= 0 && j < N;
-#pragma unroll
-                        for (int a = 0; a < CIN; ++a)
-                            r[k][a] = in && a < C ? x[(int64_t)a * N + j] : 0.0f;
-                    }
-#pragma unroll
-                    for (int k = 0; k < AT_ONCE; ++k) {
-                        float s = 0.0f;
-#pragma unroll
-                        for (int a = 0; a < CIN; ++a)
-                            s = __builtin_fmaf(w1[a], r[k][a] - xi[a], s);
-                        if (k0 + k < K)
-                            best.take((float)(v + (double)s), sign, k0 + k == 0);
-                    }
+                for (int k = 0; k < kAtOnce; ++k) {
+                    if (k0 + k >= K)
+                        break;
+                    const float y = (float)(r[k] + v), s = y * sign;
+                    // (the first NaN stays, as in torch's maximum)
+                    const bool up = k0 + k == 0 || (!(s <= best) && best == best);
+                    best = up ? s : best;
+                    chosen = up ? y : chosen;
                 }
             }
-            values[lane][local] = best.chosen;
+            values[lane][local] = chosen;
         }
         __syncthreads();
         for (int e = tid; e < kChannels * kPoints; e += kBlock) {
@@ -503,10 +458,10 @@ struct PlainOp {
 };
 
 // uv [B, N, 2 O]: a point a row, u = W1 x then v = (W2 - W1) x. m = points, n = u and v, k = channels.
-struct EdgeTermsOp : PlainOp {
+template <typename T> struct EdgeTermsOp : PlainOp {
     static constexpr bool kAlongKA = false, kAlongKB = true;
     const float *x, *w;
-    float *uv;
+    T *uv;
     int C, O, rows, cols;  // rows = N, cols = 2 O
     __device__ int to(int) const { return C; }
     __device__ Raw load_a(int p, int c, int b) const
@@ -522,7 +477,7 @@ struct EdgeTermsOp : PlainOp {
     __device__ double b(Raw r, int n, int, double) const { return n < O ? r.p : (double)r.q - (double)r.p; }
     __device__ void store(int p, int n, int b, double v) const
     {
-        uv[((int64_t)b * rows + p) * cols + n] = (float)v;
+        uv[((int64_t)b * rows + p) * cols + n] = (T)v;
     }
 };
 
@@ -685,6 +640,21 @@ template <typename Op> int launch_product(const Op &op, int batches, hipStream_t
     return tk_launch_status();
 }
 
+template <typename T>
+int edge_forward(const float *x, const int64_t *index, const float *w, const float *gamma, int B, int N,
+                 int K, int C, int O, T *uv, float *extreme, hipStream_t stream)
+{
+    const EdgeTermsOp<T> op{{}, x, w, uv, C, O, N, 2 * O};
+    const int rc = launch_product(op, B, stream);
+    if (rc != TK3D_OK)
+        return rc;
+    const int tiles = B * ((N + kPoints - 1) / kPoints);
+    const int most = 4 * tk_cu_count() / B * B;  // (whole rounds of the batch)
+    const dim3 grid(tiles < most || most == 0 ? tiles : most, (O + kChannels - 1) / kChannels);
+    edge_forward_kernel<T><<<grid, kBlock, 0, stream>>>(uv, index, gamma, B, N, K, O, tiles, extreme);
+    return tk_launch_status();
+}
+
 }  // namespace
 
 extern "C" {
@@ -709,32 +679,21 @@ int tk3d_mlp_edge_features_f32(const float *x, const int64_t *index, int B, int 
     return tk_launch_status();
 }
 
-int tk3d_mlp_edge_terms_wanted(int C) { return C >= kDirect; }
+int64_t tk3d_mlp_edge_forward_bytes(int B, int N, int C, int O)
+{
+    return (int64_t)B * N * 2 * O * (C < kRounded ? 8 : 4);
+}
 
 int tk3d_mlp_edge_forward_f32(const float *x, const int64_t *index, const float *w, const float *gamma,
-                              int B, int N, int K, int C, int O, float *uv, float *extreme, void *stream_)
+                              int B, int N, int K, int C, int O, void *workspace, float *extreme,
+                              void *stream)
 {
     if (!tk3d_mlp_edge_supported(B, N, K, O) || C <= 0 || C > 4096)
         return TK3D_ERR_UNSUPPORTED;
-    if (tk3d_mlp_edge_terms_wanted(C) && !uv)
-        return TK3D_ERR_NULL_POINTER;
-    const hipStream_t stream = (hipStream_t)stream_;
-    const int tiles = B * ((N + kPoints - 1) / kPoints);
-    const int most = 4 * tk_cu_count() / B * B;  // (whole rounds of the batch)
-    const dim3 grid(tiles < most || most == 0 ? tiles : most, (O + kChannels - 1) / kChannels);
-    if (C >= kDirect) {
-        const EdgeTermsOp op{{}, x, w, uv, C, O, N, 2 * O};
-        const int rc = launch_product(op, B, stream);
-        if (rc != TK3D_OK)
-            return rc;
-        edge_forward_kernel<0><<<grid, kBlock, 0, stream>>>(uv, index, w, gamma, B, N, K, C, O, tiles, extreme);
-    } else if (C <= 4) {
-        edge_forward_kernel<4><<<grid, kBlock, 0, stream>>>(x, index, w, gamma, B, N, K, C, O, tiles, extreme);
-    } else {
-        edge_forward_kernel<kDirect><<<grid, kBlock, 0, stream>>>(x, index, w, gamma, B, N, K, C, O, tiles,
-                                                                  extreme);
-    }
-    return tk_launch_status();
+    return C < kRounded ? edge_forward(x, index, w, gamma, B, N, K, C, O, static_cast<double *>(workspace),
+                                       extreme, (hipStream_t)stream)
+                        : edge_forward(x, index, w, gamma, B, N, K, C, O, static_cast<float *>(workspace),
+                                       extreme, (hipStream_t)stream);
 }
 
 int tk3d_mlp_edge_lists(const int64_t *index, int B, int N, int K, int32_t *lists, void *stream)

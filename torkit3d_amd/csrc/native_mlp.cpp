@@ -667,12 +667,11 @@ Tensor edge_forward(const EdgeCall &c, EdgeKept &k)
     k.extreme = at::empty({B, O, N}, options);
     k.mean = c.running_mean;
     k.var = c.running_var;
-    Tensor uv;
-    if (tk3d_mlp_edge_terms_wanted((int)C))
-        uv = at::empty({B, N, 2 * O}, options);
+    const Tensor workspace =
+        at::empty({tk3d_mlp_edge_forward_bytes((int)B, (int)N, (int)C, (int)O)}, options.dtype(at::kByte));
     done(tk3d_mlp_edge_forward_f32(f32(c.x), c.index.data_ptr<int64_t>(), f32(c.weight), f32(c.gamma),
-                                   (int)B, (int)N, (int)K, (int)C, (int)O, f32(uv), f32(k.extreme),
-                                   stream),
+                                   (int)B, (int)N, (int)K, (int)C, (int)O, workspace.data_ptr(),
+                                   f32(k.extreme), stream),
          "tk3d_mlp_edge_forward_f32");
     const Tensor z = at::empty({B, O, N}, options);
     const tk3d_mlp_norm norm = norm_of(c, k);
