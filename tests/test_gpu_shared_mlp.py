@@ -135,8 +135,8 @@ def test_grouped(cuda, monkeypatch, features, tracked, n, m, s, training):
 
 # Products in evaluation add up in several chains. Roundings of at most u = 2^-24 to numbers that grow as a
 # random walk over n terms make an error of about 0.21 u sqrt(n) of the result (one chain over all K:
-# 1.9 u at 64 channels, 3.4 u at 256, 6.9 u at 1024), in four chains half of it, in chains of sixteen
-# less; the norm adds less than u. (The library runs in one chain or in up to four, depending on the size.)
+# 1.9 u at 64 channels, 3.4 u at 256, 6.9 u at 1024), in four chains half of it, in chains of 16 or
+# 32 less; the norm adds less than u. (The library runs in one chain or in up to four, depending on the size.)
 @pytest.mark.parametrize("b,p", [(1, 128), (1, 129), (8, 2048), (8, 16384)])
 @pytest.mark.parametrize("k,c", [(64, 64), (72, 128), (256, 40), (768, 256), (1024, 64)])
 def test_evaluation_adds_up_in_short_chains(cuda, b, p, k, c):
@@ -308,8 +308,8 @@ def stock_forward(mlp, x):
 
 
 # EdgeConv on a graph of a cloud with itself: points around the workgroup's 16, 32 and 64, channels
-# around its 64 and around the 16 from which evaluation takes products per point, neighbours around the
-# eight rows requested at once; lists given or not.
+# around its 64 and around the 16 of a step, neighbours around the eight rows requested at once; lists
+# given or not.
 @pytest.mark.parametrize("training", [True, False])
 @pytest.mark.parametrize("b,c,n,k,o,lists", [
     (1, 3, 5, 2, 5, False), (2, 3, 33, 7, 64, False), (3, 64, 100, 20, 65, True),
