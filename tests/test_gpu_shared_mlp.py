@@ -150,6 +150,22 @@ def test_evaluation_adds_up_in_short_chains(cuda, b, p, k, c):
     assert error <= 2.0 ** -24 * (1.0 + 0.11 * k ** 0.5), error
 
 
+# The gradient of the input, where the tiles are 32 x 32: four chains over the output channels too. What
+# dy itself brings along (products, statistics and coefficients in float32) is below 2 u.
+@pytest.mark.parametrize("k,c,p", [(64, 256, 128), (96, 512, 100), (32, 1024, 64)])
+def test_input_gradients_add_up_in_short_chains(cuda, k, c, p):
+    mlp = mlp1d_bn_relu(k, [c]).to(cuda).train()
+    single, exact = stock(mlp, torch.float32), stock(mlp, torch.float64)
+    x, g = randn(k, 4, k, p), randn(c, 4, c, p)
+    leaf, leaf64 = x.clone().requires_grad_(), x.double().requires_grad_()
+    (got,) = torch.autograd.grad(mlp(leaf), leaf, g)
+    with torch.no_grad():  # (the signs of the float32 activations)
+        sign = single[0].bn(single[0].conv(x)) > 0
+    (want,) = torch.autograd.grad(exact[0].bn(exact[0].conv(leaf64)) * sign, leaf64, g.double())
+    error = float((got.double() - want).norm() / want.norm())
+    assert error <= 2.0 ** -24 * (2.0 + 0.11 * c ** 0.5), error / 2.0 ** -24
+
+
 # In training mode the activations and statistics are the stock modules' own, bit by bit, and so are
 # the signs the backward takes: gradients differ by sums in another order alone, 1.5e-6 over 40
 # steps of whole networks (four times that is the bound), where a single sign gave 1e-2.

@@ -61,11 +61,11 @@ __device__ __forceinline__ void load_run(float (&dst)[PT], const float *base, un
             dst[t] = v[t];
 }
 
-// Evaluation adds up sixteen channels at a time (32 from 256 channels on: no less exact there, and 142 for
-// 147 us on 320 -> 1024 channels, 16384 positions) and these sums on top of each other, in tiles of 32
-// x 32, which have the registers, in four chains over every fourth group of channels: in one chain over
-// all channels the error grows with their number (768 -> 256 channels: 3.5e-7 of the result, 1.9 times
-// that of the library's product, which runs in up to four chains; 64 -> 128: 1.4 times).
+// In one chain over all channels the error of a product grows with their number (768 -> 256 channels: 3.5e-7
+// of the result, 1.9 times that of the library's product, which runs in up to four chains; 64 -> 128:
+// 1.4 times). Tiles of 32 x 32 have the registers for four chains, over every fourth group of channels;
+// the others add up sixteen channels in evaluation (32 from 256 on: no less exact there, and 142 for 147
+// us on 320 -> 1024 channels, 16384 positions) and these sums on top of each other.
 constexpr bool short_chains(int out) { return out == OUT_EVAL || out == OUT_POOL_EVAL || out == OUT_POINTS; }
 
 constexpr bool reads_y(int in) { return in == IN_GRAD || in == IN_GRAD_OUT; }
@@ -175,7 +175,7 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
     };
 
     constexpr bool SHORT = short_chains(OUT) && PT * CT > 1;
-    constexpr int CHAINS = short_chains(OUT) && PT * CT == 1 ? kDepth<1> : 1;
+    constexpr int CHAINS = PT * CT == 1 ? kDepth<1> : 1;
     tk_f32x16 acc[PT][CT * CHAINS], total[SHORT ? PT : 1][SHORT ? CT : 1];
     const auto clear = [&] {
 #pragma unroll
