@@ -72,6 +72,28 @@ def test_forward_mode_is_refused(cuda, name):
             call(*duals)
 
 
+@pytest.mark.parametrize("name", ["chamfer", "chamfer_roots", "chamfer_rows", "group", "group_with_xyz",
+                                  "interpolate"])
+def test_saved_tensors_come_back_in_another_layout(cuda, name):
+    """What hooks on saved tensors return need not lie in memory as what they were given."""
+
+    def unpack(t):
+        return t.transpose(-1, -2).contiguous().transpose(-1, -2) if t.dim() > 1 else t
+
+    call, clouds = made(name)
+    if name == "interpolate":
+        clouds = (clouds[0], clouds[1].requires_grad_(False))
+    grads = []
+    for hooked in (False, True):
+        leaves = [c.clone().requires_grad_(name != "interpolate" or i == 0) for i, c in enumerate(clouds)]
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack if hooked else lambda t: t):
+            out = call(*leaves)
+        total = sum((o * o).sum() for o in as_list(out))
+        grads.append(torch.autograd.grad(total, [x for x in leaves if x.requires_grad]))
+    for a, b in zip(*grads):
+        torch.testing.assert_close(a, b, rtol=1e-6, atol=1e-6)
+
+
 @pytest.mark.parametrize("name", CASES)
 def test_function_transforms_are_refused(cuda, name):
     call, clouds = made(name)

@@ -12,7 +12,6 @@
 namespace py = pybind11;
 using namespace tk3d;
 using torch::autograd::AutogradContext;
-using torch::autograd::variable_list;
 
 namespace {
 
@@ -465,7 +464,7 @@ struct ChamferNode : torch::autograd::Function<ChamferNode> {
     }
     static variable_list backward(AutogradContext *ctx, variable_list grads)
     {
-        const variable_list saved = ctx->get_saved_variables();
+        const variable_list saved = dense(ctx->get_saved_variables());
         const int64_t want = ctx->saved_data["want"].toInt();
         const bool channels_first = ctx->saved_data["channels_first"].toBool();
         Tensor g1 = grads[0].contiguous(), g2 = grads[1].contiguous();

@@ -19,6 +19,7 @@
 namespace tk3d {
 
 using at::Tensor;
+using torch::autograd::variable_list;
 
 [[noreturn]] inline void fail(const std::string &message) { throw std::runtime_error(message); }
 
@@ -42,6 +43,8 @@ using OnDeviceOf = c10::OptionalDeviceGuard;
 bool plain(const Tensor &t);
 // A function transform (torch.func), a dispatch mode or a tracer is active: it has to see the operators.
 bool watched();
+// Saved tensors come back through hooks, which may lay them out anew.
+variable_list dense(variable_list saved);
 
 Tensor mlp(Tensor x, Tensor x2, const Tensor &xyz, const Tensor &centre, const Tensor &index,
            std::vector<Tensor> params, std::vector<Tensor> buffers, std::vector<double> eps,

@@ -29,10 +29,17 @@ bool watched()
            c10::impl::TorchDispatchModeTLS::any_modes_set() || at::tracer::impl::is_dispatch_enabled();
 }
 
+variable_list dense(variable_list saved)
+{
+    for (Tensor &t : saved)
+        if (t.defined())
+            t = t.contiguous();
+    return saved;
+}
+
 namespace {
 
 using torch::autograd::AutogradContext;
-using torch::autograd::variable_list;
 
 float *f32(const Tensor &t) { return t.defined() ? t.data_ptr<float>() : nullptr; }
 
@@ -53,15 +60,6 @@ bool library_norm(const Tensor &like, at::IntArrayRef shape, const Tensor *param
     const Tensor y = at::empty({}, like.options()).expand(shape);
     return at::native::_select_batch_norm_backend(y, params[1], params[2], buffers[0], buffers[1], true,
                                                   eps) == at::native::BatchNormBackend::Miopen;
-}
-
-// Saved tensors come back through hooks, which may lay them out anew.
-variable_list dense(variable_list saved)
-{
-    for (Tensor &t : saved)
-        if (t.defined())
-            t = t.contiguous();
-    return saved;
 }
 
 // What a chain is applied to and how.
