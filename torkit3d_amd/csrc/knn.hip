@@ -1684,7 +1684,10 @@ __global__ __launch_bounds__(KNN_BLOCK) void knn_wave_kernel_f32(
 // Where a wave per query wins (timed against every other kernel here on 260 shapes, 256 to 131072
 // queries, 64 to 16384 keys, k = 1 to 64; the ratio goes with the number of queries): 1.1 to 19
 // times faster up to 16384 queries, even at about 20000 (32768 with more than 32 neighbours,
-// which the lane-per-query kernels keep in LDS).
+// which the lane-per-query kernels keep in LDS). At the limits themselves, with twelve k from 1 to 64
+// and 64 to 10^6 keys, it never lost: equal at k = 48 and 64 on 256 keys, else 1.1 to 7 times faster,
+// also with keys sorted along an axis or a Morton curve (an insertion costs k (1 + ln(keys / k)) of
+// them on keys in random order; on sorted keys there are more, and the other kernels have them too).
 inline bool knn_wave_pays(int64_t queries, int k)
 {
     return k <= 64 && queries <= (k <= 32 ? 18432 : 36864);
