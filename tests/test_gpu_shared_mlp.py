@@ -206,7 +206,7 @@ def pinned(single, exact, x, x64):
 # at 8, about the activations' mean 0.6 times. (The error of one draw is good to a tenth: a quarter is
 # left for it.)
 @pytest.mark.parametrize("far", [0, 3, 8])
-@pytest.mark.parametrize("b,m,s,widths", [(8, 128, 64, (131, 128, 256)), (3, 70, 32, (9, 40, 33)),
+@pytest.mark.parametrize("b,m,s,widths", [(8, 128, 64, (131, 128, 256)), (4, 513, 32, (9, 40, 33)),
                                           (2, 512, 32, (6, 64, 64, 128))])
 def test_pooled_layer_far_from_zero(cuda, b, m, s, widths, far):
     mlp = make(mlp2d_bn_relu, widths[0], widths[1:], True, cuda)

@@ -78,10 +78,6 @@ def test_foreign_modules_in_place_of_a_chain():
     close(forward_cat(layer.mlp, x2[:, :2], x2), want)
 
 
-class OnGpu:  # what the plan of a chain looks at
-    is_cuda, dtype = True, torch.float32
-
-
 def test_replica_without_parameters_is_left_to_stock(monkeypatch):
     # (what nn.DataParallel makes of a module: tensors as plain attributes)
     mlp, _ = pair("cpu")
@@ -93,6 +89,9 @@ def test_replica_without_parameters_is_left_to_stock(monkeypatch):
             setattr(replica, name, value.detach().clone())
         return replica
 
+    class OnGpu:  # what the plan looks at
+        is_cuda, dtype = True, torch.float32
+
     monkeypatch.setattr(torkit3d_amd.nn, "_TENSORS", (OnGpu,))
     assert mlp._plan(OnGpu()) is not None and replica_of(mlp)._plan(OnGpu()) is None
     monkeypatch.setattr(torkit3d_amd.nn, "_TENSORS", ())
@@ -102,6 +101,9 @@ def test_replica_without_parameters_is_left_to_stock(monkeypatch):
 def test_batch_norm_that_does_not_track_is_left_to_stock(monkeypatch):
     """Training mode with the flag off although the buffers are there (the pass of a teacher or an
     adversary): the chain, which updates them, is not for that; evaluation uses them all the same."""
+    class OnGpu:
+        is_cuda, dtype = True, torch.float32
+
     mlp, _ = pair("cpu")
     monkeypatch.setattr(torkit3d_amd.nn, "_TENSORS", (OnGpu,))
     assert mlp.train()._plan(OnGpu()) is not None
@@ -158,3 +160,17 @@ def test_nan_reaches_the_maximum_over_edges():
     got = block(x, x, index)
     want = block(x, x.clone(), index)  # (two clouds: the general path)
     assert torch.equal(torch.isnan(got), torch.isnan(want))
+
+
+@pytest.mark.gpu
+def test_forward_mode_is_refused_by_operators():
+    from torkit3d_amd.ops.chamfer_distance import chamfer_distance
+    from torkit3d_amd.ops.group_points import group_points
+
+    x = torch.rand(1, 16, 3, device="cuda")
+    with forward_ad.dual_level():
+        dual = forward_ad.make_dual(x, torch.ones_like(x))
+        with pytest.raises(Exception):
+            chamfer_distance(dual, x)
+        with pytest.raises(Exception):
+            group_points(dual, torch.zeros(1, 2, 2, dtype=torch.long, device="cuda"))
