@@ -220,11 +220,10 @@ def test_points_at_infinity(cuda):
     np.testing.assert_array_equal(run(pts, 30, cuda), want)
 
 
-# ---- 4097 to 16384 points, 256 samples or more: the kernel that lays the points out by
-# region (Morton order), skips the blocks a new centre cannot reach and accepts from sixteen
-# candidates per exchange. The lane order is no longer the reference's priority order there,
-# so ties are resolved explicitly. 4097..8192 points run it with 8 points per lane, more with
-# 16. ----
+# ---- 513 to 16384 points, 256 samples or more: the kernel that lays the points out by region
+# (Morton order), skips the blocks a new centre cannot reach and accepts from a candidate per
+# group of lanes. The lane order is no longer the reference's priority order there, so ties are
+# resolved explicitly. ----
 
 def _region_cloud(kind, g, b, n):
     if kind == "uniform":
@@ -291,11 +290,10 @@ def test_region_kernel_shapes_and_layouts(cuda, n, k, transpose):
 @pytest.mark.parametrize("n,k,transpose", [(4096, 1024, False), (3000, 512, True), (2049, 2049, False)])
 def test_clouds_in_sampling_order_between_2049_and_4096_points(cuda, n, k, transpose):
     # A cloud that is itself a farthest point sample in sampling order (the next level of a
-    # PointNet++ encoder): its point 1 is the point farthest from point 0, by which the region
-    # kernel recognises it and leaves it to the multi-step kernel launched behind it. The
-    # answer is the first k indices in order. Then a cloud in random order whose point 1
-    # happens to be the farthest from point 0: it takes the same route and must come out right
-    # as well, and one with a NaN in that place.
+    # PointNet++ encoder): its point 1 is the point farthest from point 0, by which the kernel
+    # suspects it; the suspicion is then checked. The answer is the first k indices in order. Then
+    # a cloud in random order whose point 1 happens to be the farthest from point 0: it is taken
+    # for one at first and must come out right as well, and one with a NaN in that place.
     big = torch.rand(2, 3 * n, 3, generator=gen(n + k))
     first = oracle.sample_farthest_points(big.numpy(), n)
     pts = torch.gather(big, 1, torch.from_numpy(first)[:, :, None].expand(-1, -1, 3)).contiguous()
@@ -332,3 +330,39 @@ def test_shapes_the_reference_author_profiled(cuda, b, n, k):
     # tests/ops/test_sample_farthest_points.py:74-76 (profile runs, no recorded result)
     pts = torch.rand(b, n, 3, generator=gen(8))
     np.testing.assert_array_equal(run(pts, k, cuda), oracle.sample_farthest_points(pts.numpy(), k))
+
+
+# ---- 513 points or more and 256 samples or more: one candidate per group of lanes ----
+
+@pytest.mark.parametrize("n,k", [(513, 256), (1024, 1024), (2048, 256), (2049, 1025), (4096, 257),
+                                 (8192, 1024), (8193, 511), (8193, 512), (16384, 1025)])
+@pytest.mark.parametrize("kind", ["uniform", "lattice", "half_duplicates", "clusters", "order",
+                                  "order_broken_late", "order_broken_by_a_tie", "odd"])
+def test_groups_kernel_edges(cuda, n, k, kind):
+    # the smallest and largest cloud of every launch shape, sample counts around what a claim of
+    # sampling order may cover, a claim that holds, and claims that fail at one late step: two
+    # samples exchanged, or a copy of the last sample that comes before it in the reference's order
+    from torkit3d_amd.ops.sample_farthest_points import sample_farthest_points_gather
+
+    g = gen(n + k)
+    if kind.startswith("order"):
+        big = torch.rand(2, n + n // 2, 3, generator=g)
+        first = torch.from_numpy(oracle.sample_farthest_points(big.numpy(), n))
+        pts = torch.gather(big, 1, first[:, :, None].expand(-1, -1, 3)).contiguous()
+        if kind == "order_broken_late":
+            pts[1, [k - 2, k - 1]] = pts[1, [k - 1, k - 2]].clone()
+        elif kind == "order_broken_by_a_tie" and k < n:
+            pts[1, k:] = pts[1, k - 1]
+    elif kind == "odd":
+        pts = torch.rand(2, n, 3, generator=g)
+        pts[1, n - 1, 2] = float("inf")
+    else:
+        pts = _region_cloud(kind, g, 2, n - n % 2)
+        pts = torch.cat([pts, pts[:, : n % 2]], dim=1)
+    want = oracle.sample_farthest_points(pts.numpy(), k)
+    for transpose in (False, True):
+        dev = (pts.transpose(1, 2) if transpose else pts).contiguous().to(cuda)
+        index, sampled = sample_farthest_points_gather(dev, k, transpose=transpose)
+        np.testing.assert_array_equal(index.cpu().numpy(), want)
+        got = (sampled.transpose(1, 2) if transpose else sampled).cpu().numpy()
+        np.testing.assert_array_equal(got, np.take_along_axis(pts.numpy(), want[:, :, None], 1))

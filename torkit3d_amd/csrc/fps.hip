@@ -193,9 +193,31 @@ template <typename T> __device__ __forceinline__ T fps_first_minimum(bool used, 
     return (used && d0 == d0) ? d0 : (T)-1;
 }
 
-// The whole sampling of one cloud with the plain loop: loads the points into registers
-// and runs fps_one_step_loop. With `only_odd` it does so only for a cloud that holds a NaN
-// or an infinite coordinate, and returns at once for any other.
+// The whole sampling of one cloud with the plain loop.
+template <typename T, int P, int NT, bool SOA>
+__device__ __forceinline__ void fps_plain(const T *__restrict__ pts, int64_t *__restrict__ out,
+                                          const FpsLayout &L)
+{
+    const int tid = threadIdx.x;
+    T x[P], y[P], z[P], md[P];
+    const int npos = L.bs * L.c;
+    const T cx = fps_coord<SOA>(pts, L.n, 0, 0), cy = fps_coord<SOA>(pts, L.n, 0, 1),
+            cz = fps_coord<SOA>(pts, L.n, 0, 2);
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        const int pos = tid * P + p;
+        const int j = pos < npos ? fps_point_of_position(pos, L) : L.n;
+        const bool ok = j < L.n;
+        x[p] = ok ? fps_coord<SOA>(pts, L.n, j, 0) : (T)0;
+        y[p] = ok ? fps_coord<SOA>(pts, L.n, j, 1) : (T)0;
+        z[p] = ok ? fps_coord<SOA>(pts, L.n, j, 2) : (T)0;
+        md[p] = fps_first_minimum<T>(ok, tk_dist2<T>(x[p], y[p], z[p], cx, cy, cz));
+    }
+    fps_one_step_loop<T, P, NT>(out, L, x, y, z, md, cx, cy, cz);
+}
+
+// fps_plain as a kernel. With `only_odd` it does so only for a cloud that holds a NaN or an
+// infinite coordinate, and returns at once for any other.
 //
 // The fp32 kernel below assumes finite coordinates (minima ordered as integers, a selected
 // point's minimum dropping to zero) and is followed by this one with `only_odd`, which
@@ -223,21 +245,7 @@ __global__ __launch_bounds__(NT) void fps_register_kernel(const T *__restrict__ 
         if (!__syncthreads_or(odd ? 1 : 0))  // uniform over the workgroup
             return;
     }
-    T x[P], y[P], z[P], md[P];
-    const int npos = L.bs * L.c;
-    const T cx = fps_coord<SOA>(pts, L.n, 0, 0), cy = fps_coord<SOA>(pts, L.n, 0, 1),
-            cz = fps_coord<SOA>(pts, L.n, 0, 2);
-#pragma unroll
-    for (int p = 0; p < P; ++p) {
-        const int pos = tid * P + p;
-        const int j = pos < npos ? fps_point_of_position(pos, L) : L.n;
-        const bool ok = j < L.n;
-        x[p] = ok ? fps_coord<SOA>(pts, L.n, j, 0) : (T)0;
-        y[p] = ok ? fps_coord<SOA>(pts, L.n, j, 1) : (T)0;
-        z[p] = ok ? fps_coord<SOA>(pts, L.n, j, 2) : (T)0;
-        md[p] = fps_first_minimum<T>(ok, tk_dist2<T>(x[p], y[p], z[p], cx, cy, cz));
-    }
-    fps_one_step_loop<T, P, NT>(out, L, x, y, z, md, cx, cy, cz);
+    fps_plain<T, P, NT, SOA>(pts, out, L);
 }
 
 // ---- fp32 fast path ------------------------------------------------------------
@@ -314,32 +322,6 @@ template <int P, int NODE> struct FpsWalk2 {
     }
 };
 
-// FpsWalk2 for a caller that keeps the point indices elsewhere: reports the leaf reached.
-template <int P, int NODE> struct FpsWalk3 {
-    static __device__ __forceinline__ void go(const int (&t)[2 * P], const float (&x)[P],
-                                              const float (&y)[P], const float (&z)[P], int wl,
-                                              int wmax, FpsPick &out, int &passed)
-    {
-        if constexpr (NODE >= P) {
-            constexpr int p = NODE - P;
-            out.x = read_lane(x[p], wl);
-            out.y = read_lane(y[p], wl);
-            out.z = read_lane(z[p], wl);
-            out.j = p;  // the leaf; the caller turns it into a point index
-        } else {
-            const int left = read_lane(t[2 * NODE], wl);
-            const int right = read_lane(t[2 * NODE + 1], wl);
-            if (left == wmax) {
-                passed = right > passed ? right : passed;
-                FpsWalk3<P, 2 * NODE>::go(t, x, y, z, wl, wmax, out, passed);
-            } else {
-                passed = left > passed ? left : passed;
-                FpsWalk3<P, 2 * NODE + 1>::go(t, x, y, z, wl, wmax, out, passed);
-            }
-        }
-    }
-};
-
 // fp32 kernel that takes up to MAXM selection steps per cross-wave exchange.
 //
 // A step's fixed cost (wave reduction, slot exchange, barrier: about 1000 clocks) is
@@ -361,16 +343,12 @@ template <int P, int NODE> struct FpsWalk3 {
 // instructions is its cost: conditions are single compares whose lane masks are combined
 // in scalar registers, and the accepted candidates never go back to LDS - the coming
 // update reads their coordinates with v_readlane from the lanes that already hold them.
-template <int P, int NT, bool SOA, int MAXM, bool GATED = false>
+template <int P, int NT, bool SOA, int MAXM>
 __global__ __launch_bounds__(NT) void fps_multistep_kernel_f32(const float *__restrict__ points,
                                                                int64_t *__restrict__ index,
                                                                FpsLayout L)
 {
     static_assert((P & (P - 1)) == 0, "P must be a power of two");
-    if constexpr (GATED) {  // only the clouds the region kernel left (see its ORDER_PROBE)
-        if (index[(int64_t)blockIdx.x * L.k + L.k - 1] != -1)  // uniform over the workgroup
-            return;
-    }
     constexpr int NW = NT / TK_WAVE;
     static_assert(NW <= 8, "the cross-wave step relates 8 x 8 candidates");
     constexpr int F32_INF = 0x7f800000;
@@ -522,114 +500,167 @@ __device__ __forceinline__ int fps_position_of_point(int j, const FpsLayout &L)
     return r * L.c + (j >> L.log2_bs);
 }
 
-// fp32 kernel for clouds of 2049 to 16384 points: the multi-step kernel above with the
-// points laid out by region, so that an update only visits the points a new centre can
-// reach, and with sixteen waves, so that an exchange has sixteen candidates to accept from.
-//
-// At 16 or 32 points per lane a step is dominated by the update of the running minima
-// (nine instructions per point and centre), and almost all of that work changes nothing:
-// every running minimum is at most tau, the value of the last exchange's first winner (it
-// was the largest of them all, and minima only shrink), so a centre can lower a point's
-// minimum only if it lies within sqrt(tau) of it - a ball that shrinks as the sampling
-// proceeds. Hence:
-//   * the prologue sorts the points along a Morton curve (a counting sort by cell in LDS)
-//     and cuts the sorted sequence into 64 regions; region R goes to wave R % 16 as block
-//     R / 16 of the lanes' registers (P / 4 points per lane and block), so neighbouring
-//     regions sit in different waves, on different SIMDs;
-//   * every wave keeps the bounding boxes of its four blocks. Before an update, lane
-//     (a, q) evaluates the canonical distance from candidate a to box q - the same rounded
-//     operations as tk_dist2 on the per-axis gaps, each of which is monotone, so the
-//     result is a lower bound of the canonical distance to every point of the box - and a
-//     block is updated only if that bound is below tau. Skipping is therefore exact: a
-//     skipped update would have changed no minimum.
-//
-// Sixteen waves of 16 points per lane instead of eight of 32: an exchange accepts 4.4
-// candidates on uniform clouds where eight waves accepted 3.1, the walk to the winner's leaf
-// is a level shorter and the regions are half the size. The price is what every wave repeats
-// per exchange, now sixteen times on four SIMDs, so that part is kept short: four waves, one
-// per SIMD, rank four candidates each (one ballot per condition) while the others work out
-// how near the candidates come to their boxes, and ranks and verdicts meet in LDS behind a
-// second barrier, as tables that one read and one ballot turn into the mask of certain
-// winners; the wave's runner-up comes from a second plain maximum scan that runs beside the
-// walk instead of a scan that carries pairs.
-//
-// Ties. With this layout the lane order is no longer the reference's priority order
-// (see the top of the file), so equal maxima are resolved explicitly: a wave that holds
-// its maximum more than once picks the point with the lowest reference position (the
-// rare slow path below), the slots carry the point's sorted rank, and candidates with equal
-// values are ranked by their positions. The acceptance rules are those of
-// fps_multistep_kernel_f32.
-template <int P, bool SOA, int MAXM>
-__global__ __launch_bounds__(1024) void fps_region_kernel_f32(const float *__restrict__ points,
-                                                             int64_t *__restrict__ index,
-                                                             FpsLayout L)
+// What one of these kernels leaves as a cloud's first index for the ones behind it.
+constexpr int64_t FPS_ODD = -1;     // a coordinate is not finite: the plain loop has to do it
+constexpr int64_t FPS_CLAIM = -2;   // the cloud looks as if in sampling order: to be checked
+constexpr int64_t FPS_BROKEN = -3;  // it is not
+constexpr int FPS_CLAIM_MAX = 1024;
+
+// The largest and the second-largest running minimum (bits) of some of a lane's points, and
+// the point that holds the largest.
+struct FpsTop {
+    int m, s;
+    float x, y, z;
+    int p;
+};
+
+__device__ __forceinline__ int fps_max(int a, int b) { return a > b ? a : b; }
+__device__ __forceinline__ int fps_min(int a, int b) { return a < b ? a : b; }
+
+// (the left one stays among equals: a tie shows as s == m and is settled elsewhere)
+__device__ __forceinline__ FpsTop fps_merge(const FpsTop &a, const FpsTop &b, bool leaves)
 {
-    constexpr int NT = 1024, NW = 16, NB = 4, PB = P / NB, S = NT * P, RS = TK_WAVE * PB;
-    constexpr int CELLS = 4096;  // 16^3 cells for the sort
-    static_assert(P % NB == 0 && (P & (P - 1)) == 0 && MAXM <= NW && NW * NB == TK_WAVE, "shape");
+    const bool right = b.m > a.m;
+    FpsTop o;
+    o.m = fps_max(a.m, b.m);
+    o.s = fps_min(a.m, b.m);
+    if (!leaves)
+        o.s = fps_max(o.s, fps_max(a.s, b.s));
+    o.x = right ? b.x : a.x;
+    o.y = right ? b.y : a.y;
+    o.z = right ? b.z : a.z;
+    o.p = right ? b.p : a.p;
+    return o;
+}
+
+// fp32 kernel for clouds of 513 to 16384 points: several selection steps per exchange as in the
+// multi-step kernel above, with the points laid out by region, so that an update only visits the
+// points a new centre can reach, and with one candidate from each of 64 (GM = 2: 128) groups of
+// lanes, so that an exchange has many candidates to accept from.
+//
+// Update. Every running minimum is at most tau, the value of the last exchange's first winner (it
+// was the largest of them all, and minima only shrink), so a centre can lower a point's minimum
+// only if it lies within sqrt(tau) of it - a ball that shrinks as the sampling proceeds. The
+// prologue sorts the points along a Morton curve (a counting sort by cell in LDS) and cuts the
+// sequence into 4 NW regions; region R goes to wave R % NW as block R / NW of the lanes' registers
+// (P / 4 points per lane and block), so neighbouring regions sit on different SIMDs. Lane (a, q)
+// evaluates the canonical distance from winner a to the box of block q - the same rounded
+// operations as tk_dist2 on the per-axis gaps, each of which is monotone, so the result is a lower
+// bound of the canonical distance to every point of the box - and a block is updated only if that
+// bound is below tau. Skipping is therefore exact. A wave none of whose blocks is reached leaves
+// its candidates as they are.
+//
+// Candidates. A group is GL = NW / GM neighbouring lanes of a wave (its points are a quarter, an
+// eighth, ... of each of the wave's blocks), because GL lanes agree on their largest and second-
+// largest minimum in log2(GL) DPP steps for all groups of the wave at once, and the lane that holds
+// the largest has its coordinates at hand: no walk, no scalar unit. The kernel before this one had a
+// candidate per wave: 4.4 winners an exchange of sixteen candidates, where 64 groups give 7.5 and
+// 128 groups 8.8 (16384 -> 4096, uniform), and an exchange costs hardly more.
+//
+// Judgement. A candidate above every group's second-largest minimum is listed (at most sixteen are,
+// the upper ones); four waves, one per SIMD and at raised priority, compare four listed candidates
+// each with all of them. Candidates in order of (value, position) are the winners of the following
+// steps up to the first that an earlier one lies nearer to than its value: their updates leave it
+// alone, and everything not listed is below it. They meet in LDS, by order, behind a second barrier.
+//
+// Ties. The lane order is not the reference's priority order (see the top of the file), so equal
+// maxima are resolved explicitly. A group that holds its maximum more than once puts up the point
+// with the lowest reference position and counts as second-largest what the others will be once that
+// one is chosen (copies of a point vanish with it); if the largest minimum of all is still held twice
+// in a group, the candidates in front of the second holder's position are listed. Lattices take
+// several steps per exchange this way: 8 x 4096 -> 1024 on one of 9 x 9 x 9 points 1.61 -> 0.33 ms.
+//
+// What bounds it: one workgroup has one compute unit, and an exchange is a chain of short phases
+// (clocks at 4096 -> 1024, 8 waves, of 4100: update 1230 on average and 1880 in the slowest wave,
+// group maxima 300, judgement 1070, both with the trips through LDS; winners against boxes 600). A
+// lone wave issues an instruction every 6 clocks, two waves on a SIMD one every 4.6 together, so what
+// counts is the number of instructions on the chain. Measured (ms, before: the kernels with a
+// candidate per wave; both with what runs behind them): 8 x 16384 -> 4096 1.87 -> 1.35, 8 x 16384 ->
+// 2048 on a noisy sphere 0.95 -> 0.69, 16 x 8192 -> 2048 0.85 -> 0.58, 16 x 4096 -> 1024 0.39 -> 0.29,
+// 16 x 2048 -> 512 0.185 -> 0.155, 1 x 1024 -> 512 0.140 -> 0.117. Tried: every wave judging by itself
+// without the second barrier (1100 clocks of instructions in every wave instead of 850 in four: 16 x
+// 4096 -> 1024 0.37), blocks of half the size (0.33 for 0.29), no regions for up to 2048 points (8 %
+// faster at 1024 points in random order, three times slower on lattices).
+//
+// A cloud that is itself a farthest point sample, in sampling order from its point 0 (the next level
+// of a PointNet++ encoder), has 0, 1, 2, ... as its answer. Where point 1 is the point farthest from
+// point 0 (a cloud in random order passes once in n) and at most 1024 samples are wanted, this kernel
+// only leaves the claim, which fps_claim_minima_kernel and fps_claim_check_kernel test with the whole
+// chip; the instance with LAST behind them writes the answer, or does the work if the claim was wrong.
+template <int P, int NW, int GM, bool SOA, bool LAST>
+__device__ __forceinline__ void fps_groups(const float *__restrict__ pts, int64_t *__restrict__ out,
+                                           const FpsLayout &L, bool claims)
+{
+    constexpr int NB = 4, NT = NW * TK_WAVE, PB = P / NB, S = NT * P, RS = TK_WAVE * PB;
+    constexpr int GL = NW / GM, GW = TK_WAVE / GL;  // lanes of a group, groups of a wave
+    constexpr int G = NW * GW;                      // 64 GM groups in all
+    constexpr int MAXM = 16;                        // candidates judged at once
+    constexpr int NJ = 4;                           // waves that judge
+    constexpr int CELLS = 4096;                     // 16^3 cells for the sort
+    constexpr bool BOX_IN_LDS = P * NW >= 256;      // (the registers are full)
+    static_assert((P & (P - 1)) == 0 && P % NB == 0 && G == TK_WAVE * GM && NW >= NJ, "shape");
+    static_assert(GL == 2 || GL == 4 || GL == 8 || GL == 16, "groups");
     static_assert(CELLS % NT == 0 && S < (1 << 19), "sort");
     constexpr int F32_INF = 0x7f800000;
     constexpr int F32_NEG1 = (int)0xbf800000;
-    extern __shared__ __align__(16) unsigned char fps_region_lds[];
-    unsigned *const keys = reinterpret_cast<unsigned *>(fps_region_lds);  // [S] points, sorted
+    extern __shared__ __align__(16) unsigned char fps_groups_lds[];
+    unsigned *const keys = reinterpret_cast<unsigned *>(fps_groups_lds);  // [S] points, sorted
     unsigned *const cnt = keys + S;                                       // [CELLS + 1]
-    __shared__ float4 s_cand[2][NW];  // a wave's candidate: x, y, z, running minimum (bits)
-    __shared__ int2 s_aux[2][NW];     // the wave's second-largest minimum, the candidate's rank
-    __shared__ int s_rank[2][NW];     // a candidate's rank among them, + 256: it passed
-    __shared__ int s_byrank[2][NW];   // by rank: the exchange's number << 9, + 256: that one passed
-    __shared__ float s_tau[2];        // the running minimum of the candidate of rank 0
-    __shared__ float s_box[NW][NB][8];  // lo.xyz, hi.xyz of a wave's block
+    __shared__ float4 s_cand[G];         // a group's candidate: x, y, z, running minimum (bits)
+    __shared__ int2 s_aux[G];            // the group's second-largest minimum, the candidate
+    __shared__ int s_next[G];            // position of the next point with the same minimum
+    __shared__ float4 s_list[NJ][MAXM];  // the listed candidates, a copy for every judge
+    __shared__ int s_name[NJ][MAXM];     // which points those are
+    __shared__ float4 s_win[MAXM];       // the same in order
+    __shared__ int2 s_ent[MAXM];         // the exchange's number * 2 + (it is a winner), the point
+    __shared__ float4 s_box[NW][NB][2];  // lo, hi of a wave's block
     __shared__ float s_red[NW][8];
 
     const int tid = threadIdx.x;
     const int lane = tid & (TK_WAVE - 1);
-    const int wave = tid / TK_WAVE;
-    const float *__restrict__ pts = points + (int64_t)blockIdx.x * L.n * 3;
-    int64_t *__restrict__ out = index + (int64_t)blockIdx.x * L.k;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / TK_WAVE);
     const float INF = __builtin_huge_valf();
 
-    // ---- bounding box of the cloud ----
-    // (4 points per lane: also the point farthest from point 0, lowest index first - see
-    // ORDER_PROBE below)
-    constexpr bool ORDER_PROBE = P == 4;
+    float x[P], y[P], z[P];
+    int t[P];  // running minimum of point p (bits)
+    // what a point goes by outside its lane: its sorted rank. Block q, turn u of a lane holds
+    // rank (q * NW + wave) * RS + u * 64 + lane.
+    auto name_of = [&](int in_lane, int p) {
+        return ((p / PB) * NW + wave) * RS + (p % PB) * TK_WAVE + in_lane;
+    };
+    auto point_of = [&](int name) { return (int)keys[name]; };
+    // ---- bounding box of the cloud, whether it is finite, and how far from point 0 it reaches ----
     float lo[3] = {INF, INF, INF}, hi[3] = {-INF, -INF, -INF};
-    float far_d = -1.0f;
-    int far_j = 0;
-    const float p0x = fps_coord<SOA>(pts, L.n, 0, 0), p0y = fps_coord<SOA>(pts, L.n, 0, 1),
-                p0z = fps_coord<SOA>(pts, L.n, 0, 2);
-    for (int j = tid; j < L.n; j += NT) {
-        float v[3];
+    const float p0[3] = {fps_coord<SOA>(pts, L.n, 0, 0), fps_coord<SOA>(pts, L.n, 0, 1),
+                         fps_coord<SOA>(pts, L.n, 0, 2)};
+    float far = 0.0f;
+    bool odd = false;
+    float own[3][P];  // point tid + k * NT (beyond the cloud: its last point), read coalesced
+#pragma unroll
+    for (int k = 0; k < P; ++k) {
+        const int e = fps_min(tid + k * NT, L.n - 1);
+#pragma unroll
+        for (int a = 0; a < 3; ++a)
+            own[a][k] = fps_coord<SOA>(pts, L.n, e, a);
+    }
+#pragma unroll
+    for (int k = 0; k < P; ++k) {
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
-            v[a] = fps_coord<SOA>(pts, L.n, j, a);
-            lo[a] = __builtin_fminf(lo[a], v[a]);
-            hi[a] = __builtin_fmaxf(hi[a], v[a]);
+            lo[a] = __builtin_fminf(lo[a], own[a][k]);
+            hi[a] = __builtin_fmaxf(hi[a], own[a][k]);
+            odd |= !(own[a][k] - own[a][k] == 0.0f);
         }
-        if constexpr (ORDER_PROBE) {
-            const float d = tk_dist2<float>(v[0], v[1], v[2], p0x, p0y, p0z);
-            if (d > far_d) {  // (j ascends within a lane)
-                far_d = d;
-                far_j = j;
-            }
-        }
+        if constexpr (!LAST)
+            far = __builtin_fmaxf(far, tk_dist2<float>(own[0][k], own[1][k], own[2][k], p0[0],
+                                                       p0[1], p0[2]));
     }
+    far = wave_max<float>(far);
+    odd = __builtin_amdgcn_ballot_w64(odd) != 0ull;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            lo[a] = __builtin_fminf(lo[a], __shfl_xor(lo[a], o));
-            hi[a] = __builtin_fmaxf(hi[a], __shfl_xor(hi[a], o));
-        }
-    }
-    if constexpr (ORDER_PROBE) {
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            const float od = __shfl_xor(far_d, o);
-            const int oj = __shfl_xor(far_j, o);
-            const bool take = od > far_d || (od == far_d && oj < far_j);
-            far_d = take ? od : far_d;
-            far_j = take ? oj : far_j;
-        }
+        lo[a] = -wave_max<float>(-lo[a]);
+        hi[a] = wave_max<float>(hi[a]);
     }
     if (lane == 0) {
 #pragma unroll
@@ -637,33 +668,25 @@ __global__ __launch_bounds__(1024) void fps_region_kernel_f32(const float *__res
             s_red[wave][a] = lo[a];
             s_red[wave][3 + a] = hi[a];
         }
-        s_red[wave][6] = far_d;
-        s_red[wave][7] = __builtin_bit_cast(float, far_j);
+        s_red[wave][6] = odd ? -1.0f : far;
     }
+    for (int i = tid; i <= CELLS; i += NT)
+        cnt[i] = 0u;
     __syncthreads();
-    if constexpr (ORDER_PROBE) {
-        // ORDER_PROBE. A cloud whose point 1 is the point farthest from point 0 is, in
-        // practice, itself the output of a farthest point sampling, in sampling order (the
-        // next level of a PointNet++ encoder): every stretch of such a cloud is spread over
-        // all of it, which is what the multi-step kernel's waves want (their candidates get
-        // in each other's way less: B=16, 4096 -> 1024 0.33 ms there against 0.44 on points
-        // in random order) and this kernel, which sorts the points by cell anyway, cannot
-        // use (0.39 either way). Such a cloud is left to the multi-step kernel, which is
-        // launched behind this one and runs only where it finds the mark: -1 as the last
-        // index. (A cloud in random order passes this test once in n.)
-        float d = s_red[0][6];
-        int j = __builtin_bit_cast(int, s_red[0][7]);
+    if constexpr (!LAST) {
+        float reached = 0.0f;
+        bool any_odd = false;
 #pragma unroll
-        for (int w = 1; w < NW; ++w) {
-            const float od = s_red[w][6];
-            const int oj = __builtin_bit_cast(int, s_red[w][7]);
-            const bool take = od > d || (od == d && oj < j);
-            d = take ? od : d;
-            j = take ? oj : j;
+        for (int w = 0; w < NW; ++w) {
+            reached = __builtin_fmaxf(reached, s_red[w][6]);
+            any_odd |= s_red[w][6] < 0.0f;
         }
-        if (j == 1) {  // uniform over the workgroup
-            if (tid == 0)
-                out[L.k - 1] = -1;
+        const float d1 = tk_dist2<float>(fps_coord<SOA>(pts, L.n, 1, 0), fps_coord<SOA>(pts, L.n, 1, 1),
+                                         fps_coord<SOA>(pts, L.n, 1, 2), p0[0], p0[1], p0[2]);
+        if (any_odd || (claims && d1 >= reached)) {  // uniform over the workgroup
+            if (tid == 0) {
+                out[0] = any_odd ? FPS_ODD : FPS_CLAIM;
+            }
             return;
         }
     }
@@ -683,31 +706,21 @@ __global__ __launch_bounds__(1024) void fps_region_kernel_f32(const float *__res
 
     // ---- the points in the order of their cells along a Morton curve; slots beyond the cloud
     // last. A counting sort: any order that keeps neighbours together is a valid layout, so 16
-    // steps per axis are enough and the order within a cell is whatever the atomics give.
-    // (A bitonic sort of (code, point) pairs took 105 passes with a barrier each: two thirds
-    // of a prologue of 0.19 ms.) ----
+    // steps per axis are enough and the order within a cell is whatever the atomics give. ----
     auto spread = [](unsigned v) {  // 4 bits -> every third bit
         v = (v | (v << 4)) & 0x0c3u;
         v = (v | (v << 2)) & 0x249u;
         return v;
     };
-    for (int i = tid; i <= CELLS; i += NT)
-        cnt[i] = 0u;
-    __syncthreads();
     unsigned where[P];  // cell, and the point's turn within it from bit 13
-    float own[P][3];    // point tid + k * NT, as read (coalesced) for its cell
 #pragma unroll
     for (int k = 0; k < P; ++k) {
-        const int e = tid + k * NT;
         unsigned cell = CELLS;
-#pragma unroll
-        for (int a = 0; a < 3; ++a)
-            own[k][a] = e < L.n ? fps_coord<SOA>(pts, L.n, e, a) : 0.0f;
-        if (e < L.n) {
+        if (tid + k * NT < L.n) {
             unsigned c3[3];
 #pragma unroll
             for (int a = 0; a < 3; ++a) {
-                const float f = (own[k][a] - origin[a]) * scale[a];
+                const float f = (own[a][k] - origin[a]) * scale[a];
                 // (a NaN or an out-of-range value lands in cell 0 or 15)
                 c3[a] = (unsigned)(int)__builtin_fminf(__builtin_fmaxf(f, 0.0f), 15.0f);
             }
@@ -732,11 +745,11 @@ __global__ __launch_bounds__(1024) void fps_region_kernel_f32(const float *__res
             incl += lane >= o ? up : 0u;
         }
         if (lane == TK_WAVE - 1)
-            s_red[wave][0] = __builtin_bit_cast(float, incl);
+            s_red[wave][7] = __builtin_bit_cast(float, incl);
         __syncthreads();
         unsigned start = incl - mine;
         for (int w = 0; w < wave; ++w)
-            start += __builtin_bit_cast(unsigned, s_red[w][0]);
+            start += __builtin_bit_cast(unsigned, s_red[w][7]);
 #pragma unroll
         for (int i = 0; i < RUN; ++i) {
             cnt[tid * RUN + i] = start;
@@ -747,47 +760,36 @@ __global__ __launch_bounds__(1024) void fps_region_kernel_f32(const float *__res
     }
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < P; ++k) {
+    for (int k = 0; k < P; ++k)
         where[k] = cnt[where[k] & 0x1fffu] + (where[k] >> 13);  // the point's sorted rank
-        keys[where[k]] = (unsigned)(tid + k * NT);
+    __syncthreads();
+    // ---- this lane's points: block q, turn u <-> sorted rank (q*NW + wave) * RS + u*64 + lane.
+    // The coordinates travel through LDS, x and y first, then z with the list of points, which
+    // stays (fetched from memory by rank they are 48 gathers of 64 cache lines per wave). ----
+    float *const plane0 = reinterpret_cast<float *>(keys), *const plane1 = plane0 + S;
+#pragma unroll
+    for (int k = 0; k < P; ++k) {
+        plane0[where[k]] = own[0][k];
+        plane1[where[k]] = own[1][k];
     }
     __syncthreads();
-
-    // ---- this lane's points: block q, turn u <-> sorted rank (q*8 + wave) * RS + u*64 + lane.
-    // The point indices stay in the sorted list in LDS (16 registers less). ----
-    auto rank_of = [&](int in_lane, int p) {
-        return ((p / PB) * NW + wave) * RS + (p % PB) * TK_WAVE + in_lane;
-    };
-    // The coordinates travel from the lanes that read them to the lanes that own them through
-    // LDS, one coordinate at a time behind the counters (fetched from memory by sorted rank
-    // they were 48 gathers of 64 cache lines per wave: 45 us).
-    float x[P], y[P], z[P];
-    int t[2 * P];  // t[P + p]: running minimum of point p (bits); t[1..P-1]: maxima
-    {
-        float *const plane = reinterpret_cast<float *>(cnt);  // [S]
 #pragma unroll
-        for (int a = 0; a < 3; ++a) {
-#pragma unroll
-            for (int k = 0; k < P; ++k)
-                plane[where[k]] = own[k][a];
-            __syncthreads();
-#pragma unroll
-            for (int p = 0; p < P; ++p) {
-                const float v = plane[rank_of(lane, p)];
-                if (a == 0)
-                    x[p] = v;
-                else if (a == 1)
-                    y[p] = v;
-                else
-                    z[p] = v;
-            }
-            __syncthreads();
-        }
+    for (int p = 0; p < P; ++p) {
+        x[p] = plane0[name_of(lane, p)];
+        y[p] = plane1[name_of(lane, p)];
     }
+    __syncthreads();
 #pragma unroll
-    for (int p = 0; p < P; ++p)
-        t[P + p] = (int)keys[rank_of(lane, p)] < L.n ? F32_INF : F32_NEG1;
-    t[0] = 0;
+    for (int k = 0; k < P; ++k) {
+        keys[where[k]] = (unsigned)(tid + k * NT);
+        plane1[where[k]] = own[2][k];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        z[p] = plane1[name_of(lane, p)];
+        t[p] = (int)keys[name_of(lane, p)] < L.n ? F32_INF : F32_NEG1;
+    }
     // boxes of the wave's blocks (an empty block gets an empty box: never reached)
 #pragma unroll
     for (int q = 0; q < NB; ++q) {
@@ -795,7 +797,7 @@ __global__ __launch_bounds__(1024) void fps_region_kernel_f32(const float *__res
 #pragma unroll
         for (int u = 0; u < PB; ++u) {
             const int p = q * PB + u;
-            const bool ok = t[P + p] == F32_INF;
+            const bool ok = t[p] == F32_INF;
             const float v[3] = {x[p], y[p], z[p]};
 #pragma unroll
             for (int a = 0; a < 3; ++a) {
@@ -805,245 +807,475 @@ __global__ __launch_bounds__(1024) void fps_region_kernel_f32(const float *__res
         }
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) {
-                bl[a] = __builtin_fminf(bl[a], __shfl_xor(bl[a], o));
-                bh[a] = __builtin_fmaxf(bh[a], __shfl_xor(bh[a], o));
-            }
+            bl[a] = -wave_max<float>(-bl[a]);
+            bh[a] = wave_max<float>(bh[a]);
         }
         if (lane == 0) {
-#pragma unroll
-            for (int a = 0; a < 3; ++a) {
-                s_box[wave][q][a] = bl[a];
-                s_box[wave][q][3 + a] = bh[a];
-            }
+            s_box[wave][q][0] = make_float4(bl[0], bl[1], bl[2], 0.0f);
+            s_box[wave][q][1] = make_float4(bh[0], bh[1], bh[2], 0.0f);
         }
     }
-#pragma unroll
-    for (int i = P - 1; i >= 1; --i)  // later only the touched blocks' maxima are redone
-        t[i] = t[2 * i] > t[2 * i + 1] ? t[2 * i] : t[2 * i + 1];
-
-    // From here on a point is named by its rank in the sorted list; the list is consulted
-    // only where a point index is needed (output, ties).
+    if (tid < MAXM)
+        s_ent[tid] = make_int2(-1, 0);
     __syncthreads();  // the boxes are written
-    // After an exchange lane (a, q) = (lane / 4, lane % 4) stands for candidate a and tests it
-    // against the wave's block q, whose box it keeps in registers.
+    // After an exchange lane (a, q) = (lane / 4, lane % 4) stands for candidate a of the list and
+    // tests it against the wave's blocks q, q + 4, ..., whose boxes it keeps in registers.
     const int ca = lane >> 2, cb = lane & 3;
-    float box_lo[3], box_hi[3];
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        box_lo[a] = s_box[wave][cb & (NB - 1)][a];
-        box_hi[a] = s_box[wave][cb & (NB - 1)][3 + a];
+    float4 box_lo, box_hi;
+    if constexpr (!BOX_IN_LDS) {
+        box_lo = s_box[wave][cb][0];
+        box_hi = s_box[wave][cb][1];
     }
-    // The centres of the coming update are the candidates of the lanes in `centres`
-    // (lane 4 a stands for candidate a); bit 4 a + q of `reach` says whether candidate a
-    // can lower a minimum in block q. The first update is point 0 against every block.
-    float ax = fps_coord<SOA>(pts, L.n, 0, 0);
-    float ay = fps_coord<SOA>(pts, L.n, 0, 1);
-    float az = fps_coord<SOA>(pts, L.n, 0, 2);
-    unsigned long long centres = 1ull, reach = (1ull << NB) - 1;
-    // the last point emitted is the candidate of lane ctz(last_mask), whose sorted rank that
-    // lane keeps in last_rank; no mask: point 0
-    unsigned long long last_mask = 0ull;
-    int last_rank = 0;
-    int nc = 1;
+    constexpr unsigned long long QUADS = 0x1111111111111111ull;  // the lanes (a, 0)
+    // The first update is point 0 against every block.
+    float ax = p0[0], ay = p0[1], az = p0[2];
+    unsigned long long reach = 15ull;  // bit 4 a + q: winner a can lower a minimum in block q
+    int last_name = -1;                // the last point emitted; -1: point 0
+    // What the last wave has still to write, lanes (a, 0): the look-up of a point's index would
+    // hold it up behind the barrier that everybody waits at.
+    int pend_at = -1, pend_name = 0;
+    FpsTop top[NB];
+#pragma unroll
+    for (int q = 0; q < NB; ++q)
+        top[q] = FpsTop{F32_NEG1, F32_NEG1, 0.0f, 0.0f, 0.0f, q * PB};
     if (tid == 0)
         out[0] = 0;
 
+    int nc = 1;
     int round = 0;
     for (int it = 1; it < L.k; it += nc, ++round) {
-        // ---- running minima: only the blocks a centre can reach ----
-        unsigned touched = 0u;
-        for (unsigned long long todo = centres; todo != 0ull; todo &= todo - 1) {  // uniform
-            const int l = __builtin_ctzll(todo);
-            const unsigned blocks = (unsigned)(reach >> l) & ((1u << NB) - 1);
-            if (blocks == 0u)
-                continue;
-            const float sx = read_lane(ax, l), sy = read_lane(ay, l), sz = read_lane(az, l);
+        // ---- running minima of the blocks a winner can reach, and those blocks' two largest ----
 #pragma unroll
-            for (int q = 0; q < NB; ++q) {
-                if ((blocks >> q) & 1u) {  // uniform
+        for (int q = 0; q < NB; ++q) {
+            unsigned long long todo = reach & (QUADS << q);
+            if (todo != 0ull) {  // uniform
+                if (__builtin_popcountll(todo) & 1) {  // uniform
+                    const int l = __builtin_ctzll(todo);
+                    const float sx = read_lane(ax, l), sy = read_lane(ay, l), sz = read_lane(az, l);
 #pragma unroll
                     for (int u = 0; u < PB; ++u) {
                         const int p = q * PB + u;
                         const float d = tk_dist2<float>(x[p], y[p], z[p], sx, sy, sz);
-                        const int db = __builtin_bit_cast(int, d);
-                        t[P + p] = t[P + p] < db ? t[P + p] : db;
+                        t[p] = fps_min(t[p], __builtin_bit_cast(int, d));
+                    }
+                    todo &= todo - 1;
+                }
+                while (todo != 0ull) {  // two at a time
+                    const int l = __builtin_ctzll(todo);
+                    const float sx = read_lane(ax, l), sy = read_lane(ay, l), sz = read_lane(az, l);
+                    todo &= todo - 1;
+                    const int h = __builtin_ctzll(todo);
+                    const float hx = read_lane(ax, h), hy = read_lane(ay, h), hz = read_lane(az, h);
+                    todo &= todo - 1;
+#pragma unroll
+                    for (int u = 0; u < PB; ++u) {
+                        const int p = q * PB + u;
+                        const float d = tk_dist2<float>(x[p], y[p], z[p], sx, sy, sz);
+                        const float e = tk_dist2<float>(x[p], y[p], z[p], hx, hy, hz);
+                        t[p] = fps_min(fps_min(t[p], __builtin_bit_cast(int, d)),
+                                       __builtin_bit_cast(int, e));
                     }
                 }
+                FpsTop node[PB];
+#pragma unroll
+                for (int u = 0; u < PB; ++u) {
+                    const int p = q * PB + u;
+                    node[u] = FpsTop{t[p], F32_NEG1, x[p], y[p], z[p], p};
+                }
+#pragma unroll
+                for (int w = PB / 2; w >= 1; w /= 2) {
+#pragma unroll
+                    for (int i = 0; i < w; ++i)
+                        node[i] = fps_merge(node[2 * i], node[2 * i + 1], w == PB / 2);
+                }
+                top[q] = node[0];
             }
-            touched |= blocks;
         }
-        // maxima of the touched blocks (node 4 + q is the root of block q), then the top
+        // (a wave without a touched block has left its groups' candidates already)
+        if (reach != 0ull) {  // uniform
+            FpsTop best[NB];
 #pragma unroll
-        for (int q = 0; q < NB; ++q) {
-            if ((touched >> q) & 1u) {  // uniform
+            for (int q = 0; q < NB; ++q)
+                best[q] = top[q];
 #pragma unroll
-                for (int width = PB / 2; width >= 1; width /= 2) {
-                    const int first = (NB + q) * width;
+            for (int w = NB / 2; w >= 1; w /= 2) {
 #pragma unroll
-                    for (int i = first + width - 1; i >= first; --i)
-                        t[i] = t[2 * i] > t[2 * i + 1] ? t[2 * i] : t[2 * i + 1];
+                for (int i = 0; i < w; ++i)
+                    best[i] = fps_merge(best[2 * i], best[2 * i + 1], PB == 1 && w == NB / 2);
+            }
+            // ---- the group's two largest, in all its lanes ----
+            int gm = best[0].m, gs = best[0].s;
+#define TK3D_GROUP_STEPS(STEP)                                                         \
+            STEP(0xb1) /* quad_perm 1,0,3,2 */                                         \
+            if constexpr (GL >= 4) {                                                   \
+                STEP(0x4e) /* quad_perm 2,3,0,1 */                                     \
+            }                                                                          \
+            if constexpr (GL >= 8) {                                                   \
+                STEP(0x141) /* row_half_mirror */                                      \
+            }                                                                          \
+            if constexpr (GL >= 16) {                                                  \
+                STEP(0x140) /* row_mirror */                                           \
+            }
+#define TK3D_GROUP_TOP(ctrl)                                                           \
+            {                                                                          \
+                const int om = __builtin_amdgcn_update_dpp(gm, gm, ctrl, 0xf, 0xf, true); \
+                const int os = __builtin_amdgcn_update_dpp(gs, gs, ctrl, 0xf, 0xf, true); \
+                gs = fps_max(fps_min(gm, om), fps_max(gs, os));                        \
+                gm = fps_max(gm, om);                                                  \
+            }
+            TK3D_GROUP_STEPS(TK3D_GROUP_TOP)
+#undef TK3D_GROUP_TOP
+            // Only points strictly above zero are candidates (the reference starts its scan from
+            // max_dist = 0 with strict '>'); of a group without one, the lanes that write are many,
+            // and what they write is not looked at.
+            bool holds = best[0].m == gm;
+            int pick = best[0].p;
+            float px = best[0].x, py = best[0].y, pz = best[0].z;
+            if (__builtin_expect(__builtin_amdgcn_ballot_w64(gs == gm && gm > 0) != 0ull, 0)) {  // uniform
+                // A group holds its maximum more than once: the reference takes the point with
+                // the lowest position in its own order.
+                int lane_pos = 0x7fffffff;
+#pragma unroll
+                for (int p = 0; p < P; ++p) {
+                    const int pos = fps_position_of_point(point_of(name_of(lane, p)), L);
+                    const bool take = t[p] == gm && pos < lane_pos;
+                    lane_pos = take ? pos : lane_pos;
+                    pick = take ? p : pick;
+                    px = take ? x[p] : px;
+                    py = take ? y[p] : py;
+                    pz = take ? z[p] : pz;
+                }
+                int group_pos = lane_pos;
+#define TK3D_GROUP_MIN(ctrl)                                                           \
+                group_pos = fps_min(group_pos, __builtin_amdgcn_update_dpp(            \
+                                                   group_pos, group_pos, ctrl, 0xf, 0xf, true));
+                TK3D_GROUP_STEPS(TK3D_GROUP_MIN)
+                holds = lane_pos == group_pos;
+                // The largest of the others counts as it will be once this one is chosen: a
+                // cloud that holds points more than once would accept one winner an exchange
+                // otherwise.
+                if (holds)
+                    s_cand[wave * GW + lane / GL] = make_float4(px, py, pz, 0.0f);
+                __builtin_amdgcn_wave_barrier();
+                const float4 w = s_cand[wave * GW + lane / GL];
+                gs = F32_NEG1;
+#pragma unroll
+                for (int p = 0; p < P; ++p) {
+                    const float d = tk_dist2<float>(x[p], y[p], z[p], w.x, w.y, w.z);
+                    gs = fps_max(gs, fps_min(t[p], __builtin_bit_cast(int, d)));
+                }
+#define TK3D_GROUP_MAX(ctrl)                                                           \
+                gs = fps_max(gs, __builtin_amdgcn_update_dpp(gs, gs, ctrl, 0xf, 0xf, true));
+                TK3D_GROUP_STEPS(TK3D_GROUP_MAX)
+#undef TK3D_GROUP_MAX
+                group_pos = 0x7fffffff;
+                if (__builtin_amdgcn_ballot_w64(gs == gm && gm > 0) != 0ull) {  // uniform
+#pragma unroll
+                    for (int p = 0; p < P; ++p) {
+                        const float d = tk_dist2<float>(x[p], y[p], z[p], w.x, w.y, w.z);
+                        const int pos = fps_position_of_point(point_of(name_of(lane, p)), L);
+                        const bool same = t[p] == gm && __builtin_bit_cast(int, d) >= gm;
+                        group_pos = same ? fps_min(group_pos, pos) : group_pos;
+                    }
+                    TK3D_GROUP_STEPS(TK3D_GROUP_MIN)
+                }
+#undef TK3D_GROUP_MIN
+                if (holds)
+                    s_next[wave * GW + lane / GL] = group_pos;
+            }
+            if (holds) {
+                s_cand[wave * GW + lane / GL] = make_float4(px, py, pz, __builtin_bit_cast(float, gm));
+                s_aux[wave * GW + lane / GL] = make_int2(gs, name_of(lane, pick));
+            }
+        }
+#undef TK3D_GROUP_STEPS
+        __syncthreads();
+        // ---- which of the candidates are certain winners of the coming steps ----
+        if (wave == NW - 1) {  // uniform
+            const int j = point_of(pend_name);
+            if (pend_at >= 0)
+                out[pend_at] = (int64_t)j;
+        }
+        if (wave < NJ) {  // uniform
+            __builtin_amdgcn_s_setprio(3);
+            // lane b holds candidates b (, b + 64)
+            float4 C[GM];
+            int name_of_mine[GM], v[GM], second[GM], limit = 0, vmax = 0;
+#pragma unroll
+            for (int g = 0; g < GM; ++g) {
+                C[g] = s_cand[g * TK_WAVE + lane];
+                const int2 X = s_aux[g * TK_WAVE + lane];
+                asm volatile("" ::"v"(C[g].x), "v"(C[g].y), "v"(C[g].z));  // (loaded once, here)
+                v[g] = __builtin_bit_cast(int, C[g].w);
+                name_of_mine[g] = X.y;
+                second[g] = X.x;
+                limit = fps_max(limit, X.x);
+                vmax = fps_max(vmax, v[g]);
+            }
+            limit = wave_max_i32(limit);
+            bool in_list[GM];
+            int slot[GM], n;
+            auto place = [](unsigned long long m, int from) {
+                return (int)__builtin_amdgcn_mbcnt_hi(
+                    (unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, (unsigned)from));
+            };
+            auto enlist = [&]() {
+                n = 0;
+#pragma unroll
+                for (int g = 0; g < GM; ++g) {
+                    in_list[g] = v[g] > limit;
+                    const unsigned long long m = __builtin_amdgcn_ballot_w64(in_list[g]);
+                    slot[g] = place(m, n);
+                    n += __builtin_popcountll(m);
+                }
+            };
+            enlist();
+            if ((unsigned)(n - 1) >= (unsigned)MAXM) {  // uniform: too many, or none
+                vmax = wave_max_i32(vmax);
+                while (n > MAXM) {  // the upper ones (ends at the latest above vmax)
+                    limit += (vmax - limit + 3) >> 2;
+                    enlist();
+                }
+                if (n == 0 && vmax > 0) {
+                    // The largest minimum is there more than once, also in one group: its
+                    // candidates in front of the first point that no group has put up.
+                    int pos[GM], low = 0x7fffffff, end = 0x7fffffff;
+#pragma unroll
+                    for (int g = 0; g < GM; ++g) {
+                        pos[g] = v[g] == vmax ? fps_position_of_point(point_of(name_of_mine[g]), L)
+                                              : 0x7fffffff;
+                        low = fps_min(low, pos[g]);
+                        if (second[g] == vmax)
+                            end = fps_min(end, s_next[g * TK_WAVE + lane]);
+                    }
+                    low = 0x7fffffff - wave_max_i32(0x7fffffff - low);
+                    end = 0x7fffffff - wave_max_i32(0x7fffffff - end);
+                    do {  // (ends at the latest at one candidate)
+                        n = 0;
+#pragma unroll
+                        for (int g = 0; g < GM; ++g) {
+                            in_list[g] = pos[g] < end;
+                            const unsigned long long m = __builtin_amdgcn_ballot_w64(in_list[g]);
+                            slot[g] = place(m, n);
+                            n += __builtin_popcountll(m);
+                        }
+                        end = low + (int)(((unsigned)end - (unsigned)low + 1u) >> 1);
+                    } while (n > MAXM);
                 }
             }
-        }
-        t[2] = t[4] > t[5] ? t[4] : t[5];
-        t[3] = t[6] > t[7] ? t[6] : t[7];
-        t[1] = t[2] > t[3] ? t[2] : t[3];
-        // Only points strictly above zero are candidates (the reference starts its
-        // scan from max_dist = 0 with strict '>').
-        const int best = t[1] > 0 ? t[1] : 0;
-        // The wave's maximum and the first lane that holds it; the runner-up is the largest of
-        // the other lanes' maxima (a second scan that does not wait for the walk) and of what
-        // the walk through the winner lane's own tree passes by.
-        const int wmax = wave_max_i32(best);
-        int wl = __builtin_ctzll(__builtin_amdgcn_ballot_w64(best == wmax));
-        int second = wave_max_i32(lane == wl ? 0 : best);
-        FpsPick pick;
-        FpsWalk3<P, 1>::go(t, x, y, z, wl, wmax, pick, second);  // and inside lane wl
-        int pick_rank = rank_of(wl, pick.j);
-        if (second == wmax && wmax > 0) {  // uniform
-            // The wave holds its maximum more than once: the reference takes the point with
-            // the lowest position in its own order.
-            int lane_pos = 0x7fffffff, lane_p = 0;
 #pragma unroll
-            for (int p = 0; p < P; ++p) {
-                const int pos = fps_position_of_point((int)(unsigned)keys[rank_of(lane, p)], L);
-                const bool take = t[P + p] == wmax && pos < lane_pos;
-                lane_pos = take ? pos : lane_pos;
-                lane_p = take ? p : lane_p;
-            }
-            int wave_pos = lane_pos;
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) {
-                const int other = __shfl_xor(wave_pos, o);
-                wave_pos = other < wave_pos ? other : wave_pos;
-            }
-            wl = __builtin_ctzll(__builtin_amdgcn_ballot_w64(lane_pos == wave_pos));
-            const int wp = read_lane(lane_p, wl);
-            float sx = x[0], sy = y[0], sz = z[0];
-#pragma unroll
-            for (int p = 1; p < P; ++p) {
-                if (wp == p) {  // uniform
-                    sx = x[p];
-                    sy = y[p];
-                    sz = z[p];
+            for (int g = 0; g < GM; ++g) {
+                if (in_list[g]) {
+                    s_list[wave][slot[g]] = C[g];
+                    s_name[wave][slot[g]] = name_of_mine[g];
                 }
             }
-            pick.x = read_lane(sx, wl);
-            pick.y = read_lane(sy, wl);
-            pick.z = read_lane(sz, wl);
-            pick_rank = rank_of(wl, wp);
+            __builtin_amdgcn_wave_barrier();
+            // lane (c, b) = (lane / 16, lane % 16) compares candidate 4 wave + c of the list
+            // with candidate b
+            const int c = NJ * wave + (lane >> 4), b = lane & 15;
+            const float4 A = s_list[wave][c], B = s_list[wave][b];
+            const int name = s_name[wave][c];
+            const int va = __builtin_bit_cast(int, A.w), vb = __builtin_bit_cast(int, B.w);
+            const unsigned long long there = (unsigned long long)((1u << n) - 1u) * 0x0001000100010001ull;
+            constexpr unsigned long long SELF = 0x0008000400020001ull;
+            unsigned long long before = __builtin_amdgcn_ballot_w64(vb > va) & there;
+            const unsigned long long equal =
+                __builtin_amdgcn_ballot_w64(vb == va && c < n) & there & ~(SELF << (NJ * wave));
+            if (equal != 0ull) {  // uniform
+                const int pa = fps_position_of_point(point_of(c < n ? name : 0), L);
+                const int other = s_name[wave][b];
+                const int pb = fps_position_of_point(point_of(b < n ? other : 0), L);
+                before |= equal & __builtin_amdgcn_ballot_w64(pb < pa);
+            }
+            const float d = tk_dist2<float>(A.x, A.y, A.z, B.x, B.y, B.z);
+            const unsigned long long clash =
+                __builtin_amdgcn_ballot_w64(__builtin_bit_cast(int, d) < va) & before;
+            const int group = lane & 48;
+            const int order = __builtin_popcount((unsigned)(before >> group) & 0xffffu);
+            const bool clear = ((unsigned)(clash >> group) & 0xffffu) == 0u;
+            if (b == 0 && c < n) {
+                s_win[order] = A;
+                s_ent[order] = make_int2(round * 2 + (clear ? 1 : 0), name);
+            }
+            __builtin_amdgcn_s_setprio(0);
         }
-        const int buf = round & 1;
-        if (lane == 0) {
-            s_cand[buf][wave] = make_float4(pick.x, pick.y, pick.z, __builtin_bit_cast(float, wmax));
-            s_aux[buf][wave] = make_int2(second, pick_rank);
+        if constexpr (BOX_IN_LDS) {
+            box_lo = s_box[wave][cb][0];
+            box_hi = s_box[wave][cb][1];
         }
         __syncthreads();
-        // How many of the candidates are certain winners of the coming steps. All 64 lanes are
-        // active, so conditions are combined as lane masks in scalar registers.
-        {
-            // Sixteen candidates, 256 relations between them. Four waves (one per SIMD) rank
-            // four candidates each: lane (c, b) = (lane / 16, lane % 16) compares candidate
-            // 4 wave + c with candidate b, a condition is one ballot whose sixteen-bit groups
-            // belong to the four candidates, and rank and verdict go to LDS, where every wave
-            // reads them after a second barrier. (Every wave ranking its own candidate in
-            // sixteen of its lanes put four copies of the chain on every SIMD; all waves
-            // working through all 256 relations, sixteen.)
-            if (wave < NW / 4) {  // uniform
-                const int mine = 4 * wave + (lane >> 4), other = lane & 15;
-                const float4 W = s_cand[buf][mine];
-                const int2 Wx = s_aux[buf][mine];
-                const float4 Bc = s_cand[buf][other];
-                const int2 Bx = s_aux[buf][other];
-                const int vw = __builtin_bit_cast(int, W.w), vb = __builtin_bit_cast(int, Bc.w);
-                // b comes before the candidate in the reference's order: larger value, then
-                // lower position; positions are looked up only when two candidates really hold
-                // the same value
-                bool before = vb > vw;
-                const bool equal = vb == vw && other != mine && vw > 0;
-                if (__builtin_amdgcn_ballot_w64(equal) != 0ull) {  // uniform
-                    const int pos_w = fps_position_of_point((int)(unsigned)keys[Wx.y], L);
-                    const int pos_b = fps_position_of_point((int)(unsigned)keys[Bx.y], L);
-                    before |= equal && pos_b < pos_w;
-                }
-                const float dwb = tk_dist2<float>(W.x, W.y, W.z, Bc.x, Bc.y, Bc.z);
-                // the candidate survives b's selection: b's update leaves its minimum alone, and
-                // b's wave holds nothing else at or above it
-                const bool fine = !before || (__builtin_bit_cast(int, dwb) >= vw && Bx.x < vw);
-                const unsigned long long m_before = __builtin_amdgcn_ballot_w64(before);
-                const unsigned long long m_fine = __builtin_amdgcn_ballot_w64(fine);
-                const unsigned mb = (unsigned)(m_before >> (lane & 48)) & 0xffffu;
-                const unsigned mf = (unsigned)(m_fine >> (lane & 48)) & 0xffffu;
-                const int verdict = __builtin_popcount(mb) | ((vw > 0 && mf == 0xffffu) ? 256 : 0);
-                if (other == 0) {
-                    // (The table by rank saves every wave the folding of sixteen verdicts into
-                    // one mask, scalar work that sixteen waves repeated. Candidates without a
-                    // point left share a rank: an entry counts only with this exchange's
-                    // number on it.)
-                    s_rank[buf][mine] = verdict;
-                    s_byrank[buf][verdict & 15] = (round << 9) | (verdict & 256);
-                    if ((verdict & 255) == 0)
-                        s_tau[buf] = W.w;
-                }
-            }
-            // Candidate a for lane (a, q) and how near it comes to the box of block q: known
-            // since the first barrier. The twelve waves that have nothing to rank work that
-            // out while they would wait, the four others behind the second barrier.
-            float4 A;
-            int2 Ax;  // its wave's second-largest minimum, its sorted rank
-            float bound;
-            auto approach = [&]() {
-                A = s_cand[buf][ca];
-                Ax = s_aux[buf][ca];
-                const float gx = __builtin_fmaxf(__builtin_fmaxf(box_lo[0] - A.x, A.x - box_hi[0]), 0.0f);
-                const float gy = __builtin_fmaxf(__builtin_fmaxf(box_lo[1] - A.y, A.y - box_hi[1]), 0.0f);
-                const float gz = __builtin_fmaxf(__builtin_fmaxf(box_lo[2] - A.z, A.z - box_hi[2]), 0.0f);
-                bound = __builtin_fmaf(gz, gz, __builtin_fmaf(gy, gy, gx * gx));
-            };
-            if (wave >= NW / 4)  // uniform
-                approach();
-            __syncthreads();
-            if (wave < NW / 4)  // uniform
-                approach();
-            const int verdict = s_rank[buf][ca];
-            ax = A.x;
-            ay = A.y;
-            az = A.z;
-            const int rank = verdict & 255;  // a permutation of the live candidates
-            // lane r (of the first sixteen): did the candidate of rank r pass
-            const int by_rank = s_byrank[buf][lane & 15];
-            const unsigned passed =
-                (unsigned)__builtin_amdgcn_ballot_w64(by_rank == ((round << 9) | 256)) & 0xffffu;
-            const int left = L.k - it;  // steps still wanted
-            int good = __builtin_ctz(~passed | (1u << MAXM));  // ranks 0..good-1 passed
-            good = good < left ? good : left;
-            // tau and the reach of candidate a into block q: as with eight waves
-            const float tau = s_tau[buf];  // (stale without a live candidate: unused then)
-            reach = __builtin_amdgcn_ballot_w64(!(bound >= tau));
-            centres = __builtin_amdgcn_ballot_w64(rank < good) & 0x1111111111111111ull;
-            if (good > 0) {  // uniform
-                if (wave == 0) {  // uniform
-                    if (cb == 0 && rank < good)
-                        out[it + rank] = (int64_t)(unsigned)keys[Ax.y];
-                }
-                // the last point emitted, should the cloud run out of distinct points
-                last_mask = __builtin_amdgcn_ballot_w64(rank == good - 1);
-                last_rank = Ax.y;
-                nc = good;
-            } else {
-                // No point lies away from the chosen set: the previous choice is emitted again.
-                if (tid == 0) {
-                    int64_t j = 0;
-                    if (last_mask != 0ull)
-                        j = (int64_t)(unsigned)keys[read_lane(last_rank, __builtin_ctzll(last_mask))];
-                    out[it] = j;
-                }
-                nc = 1;
-            }
+        const float4 A = s_win[ca];
+        const int2 E = s_ent[ca];
+        ax = A.x;
+        ay = A.y;
+        az = A.z;
+        const unsigned long long missing = ~__builtin_amdgcn_ballot_w64(E.x == round * 2 + 1);
+        int good = missing != 0ull ? __builtin_ctzll(missing) >> 2 : 16;  // winners in a row
+        good = fps_min(good, L.k - it);
+        pend_at = -1;
+        if (good > 0) {  // uniform
+            const float gx = __builtin_fmaxf(__builtin_fmaxf(box_lo.x - A.x, A.x - box_hi.x), 0.0f);
+            const float gy = __builtin_fmaxf(__builtin_fmaxf(box_lo.y - A.y, A.y - box_hi.y), 0.0f);
+            const float gz = __builtin_fmaxf(__builtin_fmaxf(box_lo.z - A.z, A.z - box_hi.z), 0.0f);
+            const float bound = __builtin_fmaf(gz, gz, __builtin_fmaf(gy, gy, gx * gx));
+            const float tau = read_lane(A.w, 0);
+            reach = __builtin_amdgcn_ballot_w64(!(bound >= tau) && ca < good);
+            if (cb == 0 && ca < good)
+                pend_at = it + ca;
+            pend_name = E.y;
+            last_name = read_lane(E.y, 4 * (good - 1));
+            nc = good;
+        } else {
+            // No point lies away from the chosen set, and none will: the previous choice is
+            // emitted from here on.
+            const int64_t j = last_name >= 0 ? (int64_t)point_of(last_name) : (int64_t)0;
+            for (int i = it + tid; i < L.k; i += NT)
+                out[i] = j;
+            break;
         }
     }
+    if (wave == NW - 1 && pend_at >= 0)
+        out[pend_at] = (int64_t)point_of(pend_name);
+}
+
+template <int P, int NW, int GM, bool SOA>
+__global__ __launch_bounds__(NW * 64) void fps_groups_kernel_f32(const float *__restrict__ points,
+                                                                 int64_t *__restrict__ index,
+                                                                 FpsLayout L, bool claims)
+{
+    fps_groups<P, NW, GM, SOA, false>(points + (int64_t)blockIdx.x * L.n * 3,
+                                      index + (int64_t)blockIdx.x * L.k, L, claims);
+}
+
+// Behind the kernel above and the check of its claims: the clouds that it has left, then the
+// coordinates of the picks if wanted ([B,K,3], or [B,3,K] with SOA). One launch for what took two
+// (a second look at every coordinate, the gather): 4.7 us less per call.
+template <int P, int NW, int GM, bool SOA>
+__global__ __launch_bounds__(NW * 64) void fps_last_kernel_f32(const float *__restrict__ points,
+                                                               int64_t *__restrict__ index,
+                                                               float *__restrict__ sampled,
+                                                               FpsLayout L)
+{
+    constexpr int NT = NW * TK_WAVE;
+    const float *__restrict__ pts = points + (int64_t)blockIdx.x * L.n * 3;
+    int64_t *out = index + (int64_t)blockIdx.x * L.k;
+    const int64_t left = out[0];  // uniform over the workgroup
+    if (left < 0) {
+        __syncthreads();  // everybody has read it
+        if (left == FPS_CLAIM) {
+            for (int i = threadIdx.x; i < L.k; i += NT)
+                out[i] = (int64_t)i;
+        } else if (left == FPS_BROKEN) {
+            fps_groups<P, NW, GM, SOA, true>(pts, out, L, false);
+        } else {
+            fps_plain<float, P, NT, SOA>(pts, out, L);
+        }
+        __syncthreads();
+    }
+    if (sampled) {
+        float *__restrict__ so = sampled + (int64_t)blockIdx.x * L.k * 3;
+        for (int i = threadIdx.x; i < L.k; i += NT) {
+            const int64_t j = out[i];
+#pragma unroll
+            for (int a = 0; a < 3; ++a)
+                so[SOA ? (int64_t)a * L.k + i : (int64_t)i * 3 + a] = fps_coord<SOA>(pts, L.n, j, a);
+        }
+    }
+}
+
+// The check of a claim that a cloud's first k points, in this order, are its farthest point sample:
+// step s takes point s exactly if no point has a larger running minimum after the centres 0 .. s - 1,
+// nor an equal one at a lower position. The minimum of point s itself at that time, v_s, is the
+// threshold, worked out by a first kernel into the index row, which nobody else needs yet. Both read
+// the centres at uniform addresses and cut the centres into 16 stretches, a wave each, so that a
+// group of 64 points is done in k / 16 dependent steps, twice in the check (a stretch needs the
+// minimum over those before it). 8 x 4096 -> 1024: 333 us of sampling before, under 30 us with both.
+constexpr int FPS_CLAIM_PARTS = 16;
+
+template <bool SOA>
+__global__ __launch_bounds__(1024) void fps_claim_minima_kernel(const float *__restrict__ points,
+                                                                int64_t *__restrict__ index,
+                                                                FpsLayout L, int chunks)
+{
+    const int b = blockIdx.x / chunks, first = blockIdx.x % chunks * TK_WAVE;
+    const float *__restrict__ pts = points + (int64_t)b * L.n * 3;
+    int64_t *__restrict__ out = index + (int64_t)b * L.k;
+    if (out[0] != FPS_CLAIM)  // uniform over the workgroup
+        return;
+    __shared__ float s_min[FPS_CLAIM_PARTS][TK_WAVE];
+    const int lane = threadIdx.x & (TK_WAVE - 1);
+    const int part = __builtin_amdgcn_readfirstlane(threadIdx.x / TK_WAVE);
+    const int s = first + lane, me = s < L.k ? s : L.k - 1;
+    const float x = fps_coord<SOA>(pts, L.n, me, 0), y = fps_coord<SOA>(pts, L.n, me, 1),
+                z = fps_coord<SOA>(pts, L.n, me, 2);
+    const int end = fps_min(first + TK_WAVE, L.k);  // centres below end can matter
+    const int step = (end + FPS_CLAIM_PARTS - 1) / FPS_CLAIM_PARTS;
+    float m = __builtin_huge_valf();
+#pragma unroll 4
+    for (int i = part * step; i < fps_min((part + 1) * step, end); ++i) {
+        const float d = tk_dist2<float>(x, y, z, fps_coord<SOA>(pts, L.n, i, 0),
+                                        fps_coord<SOA>(pts, L.n, i, 1), fps_coord<SOA>(pts, L.n, i, 2));
+        m = i < s ? __builtin_fminf(m, d) : m;
+    }
+    s_min[part][lane] = m;
+    __syncthreads();
+    if (part == 0 && s > 0 && s < L.k) {
+#pragma unroll
+        for (int w = 1; w < FPS_CLAIM_PARTS; ++w)
+            m = __builtin_fminf(m, s_min[w][lane]);
+        out[s] = (int64_t)__builtin_bit_cast(int, m);
+    }
+}
+
+template <bool SOA>
+__global__ __launch_bounds__(1024) void fps_claim_check_kernel(const float *__restrict__ points,
+                                                               int64_t *__restrict__ index,
+                                                               FpsLayout L, int chunks)
+{
+    const int b = blockIdx.x / chunks, first = blockIdx.x % chunks * TK_WAVE;
+    const float *__restrict__ pts = points + (int64_t)b * L.n * 3;
+    int64_t *__restrict__ out = index + (int64_t)b * L.k;
+    __shared__ float s_min[FPS_CLAIM_PARTS][TK_WAVE];
+    __shared__ int s_open;
+    if (threadIdx.x == 0)
+        s_open = out[0] == FPS_CLAIM;  // (another workgroup may be writing it: read once)
+    __syncthreads();
+    if (!s_open)  // uniform over the workgroup
+        return;
+    const int lane = threadIdx.x & (TK_WAVE - 1);
+    const int part = __builtin_amdgcn_readfirstlane(threadIdx.x / TK_WAVE);
+    const int j = first + lane, me = j < L.n ? j : L.n - 1;
+    const float x = fps_coord<SOA>(pts, L.n, me, 0), y = fps_coord<SOA>(pts, L.n, me, 1),
+                z = fps_coord<SOA>(pts, L.n, me, 2);
+    const int centres = L.k - 1;  // after centre i comes the choice of step i + 1
+    const int step = (centres + FPS_CLAIM_PARTS - 1) / FPS_CLAIM_PARTS;
+    const int from = part * step, to = fps_min(from + step, centres);
+    float m = __builtin_huge_valf();
+#pragma unroll 4
+    for (int i = from; i < to; ++i)
+        m = __builtin_fminf(m, tk_dist2<float>(x, y, z, fps_coord<SOA>(pts, L.n, i, 0),
+                                               fps_coord<SOA>(pts, L.n, i, 1),
+                                               fps_coord<SOA>(pts, L.n, i, 2)));
+    s_min[part][lane] = m;
+    __syncthreads();
+    m = __builtin_huge_valf();
+    for (int w = 0; w < part; ++w)
+        m = __builtin_fminf(m, s_min[w][lane]);
+    bool bad = false;
+#pragma unroll 4
+    for (int i = from; i < to; ++i) {
+        m = __builtin_fminf(m, tk_dist2<float>(x, y, z, fps_coord<SOA>(pts, L.n, i, 0),
+                                               fps_coord<SOA>(pts, L.n, i, 1),
+                                               fps_coord<SOA>(pts, L.n, i, 2)));
+        const float v = __builtin_bit_cast(float, (int)out[i + 1]);
+        if (m >= v && me != i + 1)  // (a point already taken has m = 0: there only if v is)
+            bad |= m > v || !(v > 0.0f) ||
+                   fps_position_of_point(me, L) < fps_position_of_point(i + 1, L);
+        bad |= !(v > 0.0f);
+    }
+    if (bad)
+        out[0] = FPS_BROKEN;  // (the same from whoever writes it)
 }
 
 // Clouds that do not fit in one workgroup's registers: every selection step is one
@@ -1254,46 +1486,74 @@ void fps_launch_f32(const float *points, bool soa, int64_t B, int64_t *index,
     }
 }
 
-// Clouds of 2049 to 16384 points: the region kernel, then the same check for non-finite
-// coordinates as above.
-template <int P>
-int fps_region_launch_f32(const float *points, bool soa, int64_t B, int64_t *index,
-                          const FpsLayout &L, hipStream_t s)
+// The groups kernel, the check of its claims and what is left.
+template <int P, int NW, int GM, bool SOA>
+int fps_groups_launch(const float *points, int64_t B, int64_t *index, float *sampled,
+                      const FpsLayout &L, hipStream_t s)
 {
-    constexpr int MAXM = 8, NT = 1024;
+    constexpr int NT = NW * TK_WAVE;
     // the sorted list, and behind it the sort's counters, then one coordinate of every point
     constexpr int LDS = NT * P * 4 + (NT * P > 4100 ? NT * P : 4100) * 4;
-    if (soa) {
-        constexpr auto kernel = fps_region_kernel_f32<P, true, MAXM>;
-        const int allowed = tk_allow_dynamic_lds<kernel>(LDS);
-        if (allowed != TK3D_OK)
-            return allowed;
-        hipLaunchKernelGGL(kernel, dim3((unsigned)B), dim3(NT), LDS, s, points, index, L);
-        if constexpr (P == 4)  // clouds in sampling order, which the kernel above leaves
-            hipLaunchKernelGGL((fps_multistep_kernel_f32<8, 512, true, 6, true>),
-                               dim3((unsigned)B), dim3(512), 0, s, points, index, L);
-        hipLaunchKernelGGL((fps_register_kernel<float, P, NT, true>), dim3((unsigned)B),
-                           dim3(NT), 0, s, points, index, L, 1);
-    } else {
-        constexpr auto kernel = fps_region_kernel_f32<P, false, MAXM>;
-        const int allowed = tk_allow_dynamic_lds<kernel>(LDS);
-        if (allowed != TK3D_OK)
-            return allowed;
-        hipLaunchKernelGGL(kernel, dim3((unsigned)B), dim3(NT), LDS, s, points, index, L);
-        if constexpr (P == 4)
-            hipLaunchKernelGGL((fps_multistep_kernel_f32<8, 512, false, 6, true>),
-                               dim3((unsigned)B), dim3(512), 0, s, points, index, L);
-        hipLaunchKernelGGL((fps_register_kernel<float, P, NT, false>), dim3((unsigned)B),
-                           dim3(NT), 0, s, points, index, L, 1);
+    constexpr auto kernel = fps_groups_kernel_f32<P, NW, GM, SOA>;
+    constexpr auto last = fps_last_kernel_f32<P, NW, GM, SOA>;
+    int allowed = tk_allow_dynamic_lds<kernel>(LDS);
+    if (allowed == TK3D_OK)
+        allowed = tk_allow_dynamic_lds<last>(LDS);
+    if (allowed != TK3D_OK)
+        return allowed;
+    // a workgroup per 64 points, and a launch holds less than 2^32 lanes
+    const int of_k = (L.k + TK_WAVE - 1) / TK_WAVE, of_n = (L.n + TK_WAVE - 1) / TK_WAVE;
+    const bool claims = L.k <= FPS_CLAIM_MAX && B * of_n < ((int64_t)1 << 22);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)B), dim3(NT), LDS, s, points, index, L, claims);
+    if (claims) {
+        hipLaunchKernelGGL((fps_claim_minima_kernel<SOA>), dim3((unsigned)(B * of_k)), dim3(1024), 0,
+                           s, points, index, L, of_k);
+        hipLaunchKernelGGL((fps_claim_check_kernel<SOA>), dim3((unsigned)(B * of_n)), dim3(1024), 0,
+                           s, points, index, L, of_n);
     }
+    hipLaunchKernelGGL(last, dim3((unsigned)B), dim3(NT), LDS, s, points, index, sampled, L);
     return TK3D_OK;
 }
 
-// fp32: (points per lane, lanes) by cloud size, from timing every shape on an
-// MI355X: two waves per SIMD (512 lanes) hide each other's reduction latency; more
+template <int P, int NW, int GM>
+int fps_groups_launch_f32(const float *points, bool soa, int64_t B, int64_t *index, float *sampled,
+                          const FpsLayout &L, hipStream_t s)
+{
+    return soa ? fps_groups_launch<P, NW, GM, true>(points, B, index, sampled, L, s)
+               : fps_groups_launch<P, NW, GM, false>(points, B, index, sampled, L, s);
+}
+
+// fp32, the groups kernel: whether it takes the call, and its launch if so. It needs 256 samples to
+// be paid for: its prologue sorts the cloud, which costs 5 us at 1024 points and 25 at 16384, and
+// early in a sampling, where a centre reaches every block, an exchange is no faster than the
+// multi-step kernel's. At 256 samples (us, multi-step against this one, with what runs behind
+// them): 16 x 16384 226, 230; 16 x 8192 179, 166; 16 x 4096 134, 134; 16 x 2048 105, 104; from there
+// on it gains with every sample. Up to 512 points the multi-step kernel has four launches less to
+// wait for. 128 groups instead of 64 accept 10-14 % more winners and cost a step of the judgement: with
+// 16 points per lane they lose up to 512 samples (229 against 220 us at 256).
+bool fps_groups_dispatch_f32(const float *points, bool soa, int64_t B, int64_t *index, float *sampled,
+                             const FpsLayout &L, int64_t npos, hipStream_t s, int &rc)
+{
+    if (npos <= 512 || npos > 1024 * 16 || L.k < 256)
+        return false;
+    if (npos <= 512 * 4)
+        rc = fps_groups_launch_f32<4, 8, 1>(points, soa, B, index, sampled, L, s);
+    else if (npos <= 512 * 8)
+        rc = fps_groups_launch_f32<8, 8, 2>(points, soa, B, index, sampled, L, s);
+    else if (npos <= 1024 * 8)
+        rc = fps_groups_launch_f32<8, 16, 2>(points, soa, B, index, sampled, L, s);
+    else if (L.k < 512)
+        rc = fps_groups_launch_f32<16, 16, 1>(points, soa, B, index, sampled, L, s);
+    else
+        rc = fps_groups_launch_f32<16, 16, 2>(points, soa, B, index, sampled, L, s);
+    return true;
+}
+
+// fp32, everything else that fits a workgroup: (points per lane, lanes) by cloud size, from timing
+// every shape on an MI355X: two waves per SIMD (512 lanes) hide each other's reduction latency; more
 // waves only repeat the per-wave reduction.
-int fps_dispatch_f32(const float *points, bool soa, int64_t B, int64_t *index,
-                     const FpsLayout &L, int64_t npos, hipStream_t s)
+void fps_dispatch_f32(const float *points, bool soa, int64_t B, int64_t *index,
+                      const FpsLayout &L, int64_t npos, hipStream_t s)
 {
     if (npos <= 64 * 2)
         fps_launch_f32<2, 64>(points, soa, B, index, L, s);
@@ -1303,26 +1563,12 @@ int fps_dispatch_f32(const float *points, bool soa, int64_t B, int64_t *index,
         fps_launch_f32<2, 512>(points, soa, B, index, L, s);
     else if (npos <= 512 * 4)
         fps_launch_f32<4, 512>(points, soa, B, index, L, s);
-    // From 2049 points on the region kernel with 4 points per lane, once its prologue is paid
-    // for: B=16, 4096 -> 1024 0.44 -> 0.40 ms, 3000 -> 1024 0.47 -> 0.39 ms, 2100 -> 512
-    // 0.26 -> 0.21 ms, 4096 -> 4096 1.65 -> 1.38 ms; 4096 -> 384 is level, -> 256 10 % behind.
-    else if (npos > 512 * 4 && npos <= 512 * 8 && L.k >= (npos <= 512 * 6 ? 256 : 512))
-        return fps_region_launch_f32<4>(points, soa, B, index, L, s);
     else if (npos <= 512 * 8)
         fps_launch_f32<8, 512>(points, soa, B, index, L, s);
-    // Beyond 4096 points the region kernel (sixteen waves; its prologue costs about 30 us) wins
-    // from a few hundred samples on: B=16, 8192 -> 2048 1.20 -> 0.94 ms, B=4, 10000 -> 512
-    // 0.53 -> 0.34 ms, B=8, 16384 -> 512 0.51 -> 0.38 ms; at 4096 points it is level with the
-    // kernel above at 1024 samples and behind it below.
-    else if (npos <= 512 * 16 && L.k >= 256)
-        return fps_region_launch_f32<8>(points, soa, B, index, L, s);
     else if (npos <= 512 * 16)
         fps_launch_f32<16, 512>(points, soa, B, index, L, s);
-    else if (L.k >= 256)
-        return fps_region_launch_f32<16>(points, soa, B, index, L, s);
     else
         fps_launch_f32<32, 512>(points, soa, B, index, L, s);
-    return TK3D_OK;
 }
 
 // Coordinates of the picks: sampled[b, i, :] = points[b, index[b, i], :] in the layout of
@@ -1389,9 +1635,10 @@ int fps(const T *points, bool soa, int64_t B, int64_t N, int64_t K, int64_t *ind
     const int64_t npos = (int64_t)L.bs * L.c;
     if (npos <= fps_register_capacity(sizeof(T))) {
         if constexpr (sizeof(T) == 4) {
-            const int rc = fps_dispatch_f32(points, soa, B, index, L, npos, s);
-            if (rc != TK3D_OK)
-                return rc;
+            int rc;
+            if (fps_groups_dispatch_f32(points, soa, B, index, sampled, L, npos, s, rc))
+                return rc != TK3D_OK ? rc : tk_launch_status();
+            fps_dispatch_f32(points, soa, B, index, L, npos, s);
             return fps_finish<T>(points, soa, B, N, K, index, sampled, s);
         }
         // Fewest points per lane that still covers the cloud: short serial chains.
