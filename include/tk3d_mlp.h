@@ -113,6 +113,27 @@ typedef struct {
 } tk3d_mlp_sum;
 int tk3d_mlp_sum_f32(const tk3d_mlp_sum *sums, int n, void *stream);
 
+/* A batch norm of a training step, statistics in the library's order (csrc/batch_norm.hip): first the
+ * sums, then a pass that normalises with them and leaves mean, 1 / sqrt(variance + eps) and the updated
+ * running statistics. y [B, C, P], 16-byte aligned. */
+typedef struct {
+    void *partial; /* tk3d_mlp_batch_norm_partial_bytes(C), as tk3d_mlp_batch_sums_f32 left it */
+    const float *gamma, *beta;
+    float *running_mean, *running_var, *mean, *inv_std;
+    double eps;
+    float momentum;
+    int32_t B, C, P;
+} tk3d_mlp_batch_norm;
+int tk3d_mlp_batch_norm_supported(int64_t B, int64_t C, int64_t P);
+int64_t tk3d_mlp_batch_norm_partial_bytes(int64_t C);
+int tk3d_mlp_batch_sums_f32(const float *y, int B, int C, int P, void *partial, void *stream);
+/* z = relu(norm(y)) */
+int tk3d_mlp_batch_relu_f32(const float *y, const tk3d_mlp_batch_norm *norm, float *z, void *stream);
+/* out = relu(max norm(y)) over groups of `size` <= 255 consecutive values, arg the place of the maximum
+ * and extreme the y at that place, [B, C, P / size] each */
+int tk3d_mlp_batch_pool_f32(const float *y, const tk3d_mlp_batch_norm *norm, int size, float *out,
+                            float *extreme, unsigned char *arg, void *stream);
+
 /* A normalised layer's ReLU and maximum over groups of `size` <= 255 consecutive values: out =
  * relu(max z), arg the place of the maximum and extreme the y at that place, [groups] each. */
 int tk3d_mlp_pool_max_f32(const float *z, const float *y, int64_t groups, int size, float *out,

@@ -260,6 +260,61 @@ def test_the_backward_takes_the_signs_of_the_library(cuda, b, c, p):
     assert code == 0 and torch.equal(out, torch.relu(z))
 
 
+# Rows around the two orders of summation (4096 values), batches whose last thread chains are shorter
+# than the others, one row, a group that is no power of two; a constant channel (a variance that rounds
+# below zero), one with a NaN and one with an infinity.
+@pytest.mark.parametrize("b,c,m,size", [
+    (2, 5, 257, 4), (3, 4, 33, 32), (1, 64, 64, 64), (7, 33, 100, 20), (5, 6, 1023, 4), (2, 7, 128, 32),
+    (3, 8, 1025, 4), (16, 33, 512, 32), (4, 5, 84, 63), (1, 2048, 64, 32), (512, 3, 128, 32),
+])
+def test_batch_norm_is_the_librarys_bit_by_bit(cuda, b, c, m, size):
+    import ctypes
+
+    from torkit3d_amd import _lib
+
+    class Norm(ctypes.Structure):
+        _fields_ = [(n, ctypes.c_void_p) for n in
+                    ("partial", "gamma", "beta", "running_mean", "running_var", "mean", "inv_std")] + [
+                        ("eps", ctypes.c_double), ("momentum", ctypes.c_float),
+                        ("B", ctypes.c_int32), ("C", ctypes.c_int32), ("P", ctypes.c_int32)]
+
+    def pointers(*tensors):
+        return [ctypes.c_void_p(t.data_ptr()) for t in tensors]
+
+    y = randn(m, b, c, m, size) * (1 + randn(1, c, 1, 1).abs()) + randn(2, c, 1, 1) * 3
+    y[:, 0] = 0.1
+    y[0, 1, 1, 1] = float("nan")
+    y[b - 1, 2 % c, 0, 3] = float("inf")
+    gamma, beta = randn(3, c), randn(4, c)
+    mine, theirs = ([randn(5, c), randn(6, c).abs()] for _ in range(2))
+    z, mean, inv_std, _, backend = torch._batch_norm_impl_index(y, gamma, beta, *theirs, True, 0.3, 1e-3, True)
+    assert backend == 2  # MIOpen
+    lib, p, stream = _lib.lib(), m * size, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    lib.tk3d_mlp_batch_norm_partial_bytes.restype = ctypes.c_int64
+    size_of = [ctypes.c_int64(v) for v in (b, c, p)]
+    assert lib.tk3d_mlp_batch_norm_supported(*size_of) == 1
+    partial = torch.empty(lib.tk3d_mlp_batch_norm_partial_bytes(size_of[1]), dtype=torch.uint8, device=cuda)
+    got = [torch.empty(c, device=cuda) for _ in range(2)]
+    norm = Norm(*(t.data_ptr() for t in (partial, gamma, beta, *mine, *got)), 1e-3, 0.3, b, c, p)
+    assert lib.tk3d_mlp_batch_sums_f32(*pointers(y), b, c, p, *pointers(partial), stream) == 0
+    out = torch.empty_like(y)
+    assert lib.tk3d_mlp_batch_relu_f32(*pointers(y), ctypes.byref(norm), *pointers(out), stream) == 0
+    for a, e in zip((out, *got, *mine), (z.relu(), mean, inv_std, *theirs)):
+        assert torch.equal(a.isnan(), e.isnan()) and torch.equal(a.nan_to_num(7.0), e.nan_to_num(7.0))
+    best, extreme = torch.empty(b, c, m, device=cuda), torch.empty(b, c, m, device=cuda)
+    arg = torch.empty(b, c, m, dtype=torch.uint8, device=cuda)
+    assert lib.tk3d_mlp_batch_pool_f32(*pointers(y), ctypes.byref(norm), size,
+                                       *pointers(best, extreme, arg), stream) == 0
+    top, where = z.max(dim=3)
+    assert torch.equal(best.nan_to_num(7.0), top.relu().nan_to_num(7.0))
+    there = z.gather(3, arg.long()[..., None])[..., 0]
+    assert torch.equal(there.nan_to_num(7.0), top.nan_to_num(7.0))
+    assert torch.equal(extreme.nan_to_num(7.0), y.gather(3, arg.long()[..., None])[..., 0].nan_to_num(7.0))
+    # what it is not made for
+    for shape in ((2, 8, 1024), (2, 8, 1030), (513, 8, 2048), (600, 1, 4096), (2, 2049, 2048)):
+        assert lib.tk3d_mlp_batch_norm_supported(*(ctypes.c_int64(v) for v in shape)) == 0
+
+
 @pytest.mark.parametrize("form", ["dense", "edges"])
 def test_without_the_library_training_is_left_to_stock(cuda, form):
     """torch's own batch norm rounds in another order than the backward takes its signs by."""

@@ -1185,14 +1185,6 @@ __global__ void __launch_bounds__(kBlock, 4)
 // One pass over z (and one value of y a group) in place of a ReLU over z and a maximum over that.
 // A group of 32 or 64 is a run of 8 or 16 lanes with four values each; of any other size, a lane's.
 
-// (best, where) or (s, at), the first of the largest; NaN above all.
-__device__ __forceinline__ void take_larger(float &best, int &where, float s, int at)
-{
-    const bool up = s != s ? best == best || at < where : s > best || (s == best && at < where);
-    best = up ? s : best;
-    where = up ? at : where;
-}
-
 template <int S>  // 0: `size`
 __global__ void __launch_bounds__(kBlock)
     mlp_pool_max_kernel(const float *__restrict__ z, const float *__restrict__ y, int64_t groups,

@@ -42,4 +42,12 @@ __device__ __forceinline__ float sign_of(float gamma)
     return gamma > 0.0f ? 1.0f : gamma < 0.0f ? -1.0f : 0.0f;
 }
 
+// (best, where) or (s, at), the first of the largest; NaN above all.
+__device__ __forceinline__ void take_larger(float &best, int &where, float s, int at)
+{
+    const bool up = s != s ? best == best || at < where : s > best || (s == best && at < where);
+    best = up ? s : best;
+    where = up ? at : where;
+}
+
 }  // namespace

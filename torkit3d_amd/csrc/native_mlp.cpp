@@ -217,10 +217,13 @@ Tensor evaluate(const Call &c)
     return h;
 }
 
-// A layer of stock operators in training mode: the product, and its batch norm with the statistics
-// of this batch (and the running ones updated).
+// A layer of a training step: the library's product, and its batch norm with the statistics of this
+// batch (the running ones updated) behind it.
 struct Normalised {
-    Tensor y, z, mean, inv_std;
+    Tensor y, mean, inv_std;
+    Tensor z;                 // the library's, where it took the batch norm
+    tk3d_mlp_batch_norm norm{};  // else what the pass over y needs
+    Tensor partial;
 };
 
 Normalised stock_layer(const Tensor &h, const Tensor &weight, const Tensor &gamma, const Tensor &beta,
@@ -229,32 +232,62 @@ Normalised stock_layer(const Tensor &h, const Tensor &weight, const Tensor &gamm
 {
     Normalised n;
     n.y = h.dim() == 4 ? at::conv2d(h, weight) : at::conv1d(h, weight);
-    std::tie(n.z, n.mean, n.inv_std, std::ignore, std::ignore) =
-        at::_batch_norm_impl_index(n.y, gamma, beta, running_mean, running_var, true, momentum, eps,
-                                   at::globalContext().userEnabledCuDNN());
+    const int64_t B = n.y.size(0), C = n.y.size(1), P = n.y.numel() / (B * C);
+    if (n.y.is_contiguous() && tk3d_mlp_batch_norm_supported(B, C, P)) {
+        n.mean = at::empty({C}, n.y.options());
+        n.inv_std = at::empty({C}, n.y.options());
+        n.partial = at::empty({tk3d_mlp_batch_norm_partial_bytes(C)}, n.y.options().dtype(at::kByte));
+        n.norm = {n.partial.data_ptr(), f32(gamma), f32(beta), f32(running_mean), f32(running_var),
+                  f32(n.mean), f32(n.inv_std), eps, (float)momentum, (int32_t)B, (int32_t)C, (int32_t)P};
+        done(tk3d_mlp_batch_sums_f32(f32(n.y), (int)B, (int)C, (int)P, n.partial.data_ptr(),
+                                     stream_of(n.y)),
+             "tk3d_mlp_batch_sums_f32");
+    } else {
+        std::tie(n.z, n.mean, n.inv_std, std::ignore, std::ignore) =
+            at::_batch_norm_impl_index(n.y, gamma, beta, running_mean, running_var, true, momentum, eps,
+                                       at::globalContext().userEnabledCuDNN());
+    }
     return n;
 }
 
-// ReLU and the maximum over the last dimension of z, with the y at the place of the maximum.
+// ReLU of the normalised layer.
+Tensor activate(const Normalised &n)
+{
+    if (n.z.defined())
+        return Tensor(n.z).relu_();
+    const Tensor z = at::empty_like(n.y);
+    done(tk3d_mlp_batch_relu_f32(f32(n.y), &n.norm, f32(z), stream_of(z)), "tk3d_mlp_batch_relu_f32");
+    return z;
+}
+
+// ReLU and the maximum over the last dimension, with the y at the place of the maximum.
 Tensor pool_max(const Normalised &n, Tensor &extreme, Tensor &arg)
 {
-    const Tensor z = n.z.contiguous(), y = n.y.contiguous();
-    const int64_t B = z.size(0), C = z.size(1), M = z.size(2);
-    const Tensor out = at::empty({B, C, M}, z.options());
-    extreme = at::empty({B, C, M}, z.options());
-    arg = at::empty({B, C, M}, z.options().dtype(at::kByte));
-    done(tk3d_mlp_pool_max_f32(f32(z), f32(y), B * C * M, (int)z.size(3), f32(out), f32(extreme),
-                               arg.data_ptr<uint8_t>(), stream_of(z)),
-         "tk3d_mlp_pool_max_f32");
+    const Tensor y = n.y.contiguous();
+    const int64_t B = y.size(0), C = y.size(1), M = y.size(2);
+    const Tensor out = at::empty({B, C, M}, y.options());
+    extreme = at::empty({B, C, M}, y.options());
+    arg = at::empty({B, C, M}, y.options().dtype(at::kByte));
+    if (n.z.defined()) {
+        const Tensor z = n.z.contiguous();
+        done(tk3d_mlp_pool_max_f32(f32(z), f32(y), B * C * M, (int)y.size(3), f32(out), f32(extreme),
+                                   arg.data_ptr<uint8_t>(), stream_of(y)),
+             "tk3d_mlp_pool_max_f32");
+    } else {
+        done(tk3d_mlp_batch_pool_f32(f32(y), &n.norm, (int)y.size(3), f32(out), f32(extreme),
+                                     arg.data_ptr<uint8_t>(), stream_of(y)),
+             "tk3d_mlp_batch_pool_f32");
+    }
     return out;
 }
 
 // Training: the activations of the stock modules, bit by bit. The gradient of a training step
 // follows the signs and places that last-bit differences decide: with products and statistics of
 // its own, however exact, one step in six of a PointNet++ or DGCNN had single gradients off by more
-// than half their root mean square from the stock modules' (which are as far from float64). Fused
-// are the grouping, the maximum behind the last layer, what is kept (the products alone, no
-// activations, no edge of a pooled layer), and the whole backward.
+// than half their root mean square from the stock modules' (which are as far from float64). So the
+// products are the library's, and the batch norms' sums come in its order (csrc/batch_norm.hip). Fused
+// are the grouping, the batch norm with the ReLU or the maximum behind it, what is kept (the products
+// alone, no activations, no edge of a pooled layer), and the whole backward.
 Tensor forward_training(const Call &c, Kept &k)
 {
     const int64_t B = c.batch(), L = c.layers();
@@ -281,7 +314,7 @@ Tensor forward_training(const Call &c, Kept &k)
             h = pool_max(n, extreme, k.arg);
             k.y.push_back(extreme);
         } else {
-            h = Tensor(n.z).relu_();
+            h = activate(n);
             k.y.push_back(n.y.flatten(2).contiguous());
         }
         if (s[2].defined())
