@@ -108,7 +108,10 @@ int tk3d_chamfer_distance_forward_bcn_f64(const double *xyz1, const double *xyz2
  * four, which the sweeps read faster than ragged lengths and short [B,3,N] clouds. `workspace`:
  * 16-byte aligned device memory of at least the size that
  * tk3d_chamfer_distance_forward_rows_bytes returns, which is 0 for shapes that are as fast or faster
- * without (pass on to the calls above). Results are bit-identical to theirs. */
+ * without (pass on to the calls above). Results are bit-identical to theirs.
+ * tk3d_chamfer_distance_forward_in_place: 1 where one launch reads the clouds as they lie and is faster
+ * than with a copy; the workspace is then left alone. */
+int tk3d_chamfer_distance_forward_in_place(int64_t B, int64_t N1, int64_t N2, int channels_first);
 size_t tk3d_chamfer_distance_forward_rows_bytes(int64_t B, int64_t N1, int64_t N2, int channels_first);
 int tk3d_chamfer_distance_forward_rows_f32(const float *xyz1, const float *xyz2, int channels_first,
                                            int64_t B, int64_t N1, int64_t N2, float *dist1,
@@ -123,6 +126,14 @@ int tk3d_chamfer_rows_f64(const double *xyz1, const double *xyz2, int channels_f
                           int64_t N1, int64_t N2, int64_t rows1, int64_t rows2, double *out1,
                           double *out2, void *stream);
 
+/* Forward and sqrt(max(dist, eps)) of both directions (tk3d_chamfer_roots_f32 below) in one launch, for
+ * the calls of tk3d_chamfer_distance_forward_in_place; TK3D_ERR_UNSUPPORTED, with nothing launched, for
+ * others. */
+int tk3d_chamfer_distance_forward_roots_f32(const float *xyz1, const float *xyz2, int channels_first,
+                                            int64_t B, int64_t N1, int64_t N2, double eps, float *dist1,
+                                            int64_t *idx1, float *dist2, int64_t *idx2, float *root1,
+                                            float *root2, void *stream);
+
 /* What chamfer_distance(sqrt=True) does around the op in Python (torkit3d/ops/chamfer_distance.py:
  * 6-7,57-58) for both directions in one launch: root = sqrt(max(dist, eps)), and backwards
  * out = grad / (2 root) where dist >= eps, else 0. */
@@ -136,6 +147,14 @@ int tk3d_chamfer_roots_f64(const double *dist1, const double *dist2, int64_t n1,
 int tk3d_chamfer_root_grads_f64(const double *grad1, const double *grad2, const double *dist1,
                                 const double *dist2, const double *root1, const double *root2, int64_t n1,
                                 int64_t n2, double eps, double *out1, double *out2, void *stream);
+
+/* root_grads (grads1 [B,N1], grads2 [B,N2]) and rows (out1 [B,N1,3], out2 [B,N2,3], from [B,3,N]) in one
+ * launch. */
+int tk3d_chamfer_root_grads_rows_f32(const float *grad1, const float *grad2, const float *dist1,
+                                     const float *dist2, const float *root1, const float *root2,
+                                     const float *xyz1, const float *xyz2, int64_t B, int64_t N1,
+                                     int64_t N2, double eps, float *grads1, float *grads2, float *out1,
+                                     float *out2, void *stream);
 
 /* Replaces chamfer_distance_backward_cuda
  * (chamfer_distance.h:10-16, chamfer_distance_kernel.cu:200-274).

@@ -408,6 +408,33 @@ def test_split_sweep_with_slices_that_hold_no_finite_distance(cuda, n1, n2):
     check_forward(a, c, cuda)
 
 
+# ---- the sweep whose waves share the queries -------------------------------------------------
+# One of 64, 128, 192 or 256 queries a workgroup, by what fills the chip; a wave's stretch of keys
+# ends anywhere in a chunk of 64 or holds none at all.
+@pytest.mark.parametrize("b,n1,n2", [(1, 1, 63), (2, 64, 65), (3, 513, 511), (1, 1023, 8 * 64 + 1),      # 64
+                                     (8, 2048, 2048), (5, 1985, 2177), (8, 513, 2049),                # 128
+                                     (8, 2500, 3001), (8, 2497, 3073),                                # 192
+                                     (16, 2048, 2048), (40, 1023, 640), (3, 5001, 300), (300, 50, 700)])
+def test_waves_that_share_queries(cuda, b, n1, n2):
+    from debug_abi import ROUTE_EXACT, chamfer_route
+    from torkit3d_amd.ops.chamfer_distance import chamfer_distance
+
+    g = gen(n1 + 5 * n2)
+    a, c = uniform_cloud(g, b, n1), uniform_cloud(g, b, n2)
+    c[:, n2 // 2:] = c[:, :n2 - n2 // 2].clone()         # every key twice, in different waves' stretches
+    c[0, : n2 // 3] = float("nan")                       # waves without a candidate
+    a[0, n1 // 2] = float("inf")
+    a[b - 1, n1 - 1] = float("nan")
+    out = check_forward(a, c, cuda)
+    check_forward_channels_first(a, c, cuda)
+    for got, want in zip(out, chamfer_route(a.to(cuda), c.to(cuda), ROUTE_EXACT)):
+        assert torch.equal(got, want)
+    for t in (False, True):                              # the roots that the sweep writes itself
+        x, y = [(v.transpose(1, 2) if t else v).contiguous().to(cuda) for v in (a, c)]
+        for got, d in zip(chamfer_distance(x, y, transpose=t, sqrt=True, eps=1e-3), (out[0], out[2])):
+            torch.testing.assert_close(got, torch.sqrt(torch.clamp(d, 1e-3)), rtol=0, atol=0, equal_nan=True)
+
+
 # ---- channel-first clouds, read in place ---------------------------------------------------
 
 def check_forward_channels_first(a, c, cuda):

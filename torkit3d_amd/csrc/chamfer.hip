@@ -19,7 +19,8 @@
 // the minimum bit for bit. This keeps the reference's tie rule (strict '<' over
 // ascending j, chamfer_distance_kernel.cu:73) exactly.
 //
-// Both directions (cloud 1 -> 2 and 2 -> 1) run in one launch.
+// Both directions (cloud 1 -> 2 and 2 -> 1) run in one launch. Launches of a few workgroups of that kind
+// cut the keys between the waves of a workgroup instead (chamfer_forward_team_kernel).
 #include "tk3d_common.h"
 #include "tk3d_debug.h"
 
@@ -1689,6 +1690,147 @@ __global__ __launch_bounds__(NT) void chamfer_backward_fixed_kernel(
     }
 }
 
+struct ChamferRoots {
+    float *root[2];  // sqrt(max(dist, eps)) of either direction, or nullptr
+    float eps;
+};
+template <typename T> __device__ __forceinline__ T chamfer_root(T d, T eps)
+{
+    const T c = d < eps ? eps : d;  // a NaN stays a NaN, as in clamp
+    return sizeof(T) == 4 ? (T)__builtin_sqrtf((float)c) : (T)__builtin_sqrt((double)c);
+}
+
+// Exact sweep of a launch too small for the sweeps above, whose workgroups hold 512 queries and more:
+// the waves of a workgroup share QPL * 64 queries and cut the keys between them, so that 2048 points
+// against 2048 are 32 workgroups of eight waves instead of eight of four. Their minima meet in LDS; the
+// tile that holds a query's minimum is then evaluated once more, by all lanes, for the lowest key index.
+// No slices that meet in global memory, so neither a launch in front that clears nor one behind that
+// unpacks, and any layout and alignment at the same speed: no copy to padded rows.
+//
+// What bounds it: up to a workgroup per CU, the chain of a wave's keys (seven instructions a pair, an
+// LDS broadcast a key, 8 waves on a CU issue one instruction every 5 clocks each), then vector issue:
+// 8.1e12 pairs/s with a full chip, where the matrix pre-filter reaches 27e12 but takes 20 to 40 us of
+// fixed cost. GPU time in us, sweeps above -> this (8 waves of one query a lane, then 16 of two):
+// 300 x 300 19 -> 5; 2 x 1024 x 1024 14 -> 7; 8 x 1024 x 1024 18 -> 7; 4 x 2048 x 2048 25 -> 11.5;
+// 8 x 2048 x 2048 21 -> 13; 4 x 4096 x 4096 26 -> 21; 8 x 4096 x 4096 31 -> 38 (left to them).
+template <int QPL, int NW, bool SOA>
+__global__ __launch_bounds__(NW * 64) void chamfer_forward_team_kernel(ChamferFwdArgs<float> args,
+                                                                       ChamferRoots roots)
+{
+    constexpr int NT = NW * TK_WAVE, QB = QPL * TK_WAVE, TILE = 32, CHUNK = 64;
+    constexpr int LPQ = QPL == 3 ? NT / (4 * TK_WAVE) : NT / QB;  // lanes per query in the epilogue
+    static_assert(LPQ * QB <= NT && (LPQ & (LPQ - 1)) == 0 && TILE % LPQ == 0, "shape");
+    __shared__ __align__(16) float4 s_key[NW][2][CHUNK];
+    __shared__ float s_val[NW][QB];
+    __shared__ int s_tile[NW][QB];
+    const int tid = threadIdx.x, lane = tid & (TK_WAVE - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid / TK_WAVE);
+    int b, qblock, slice;
+    const ChamferDir<float> &d = chamfer_decode_block<float>(args, b, qblock, slice);
+    const int nq = d.nq, nk = d.nk;
+    const float *__restrict__ Q = d.query + (int64_t)b * d.qrows * 3;
+    const float *__restrict__ K = d.key + (int64_t)b * d.krows * 3;
+    const float INF = __builtin_huge_valf(), NAN_ = __builtin_nanf("");
+
+    float qx[QPL], qy[QPL], qz[QPL], best[QPL];
+    int where[QPL];
+#pragma unroll
+    for (int i = 0; i < QPL; ++i) {
+        int qi = qblock * QB + i * TK_WAVE + lane;
+        qi = qi < nq ? qi : nq - 1;
+        const TkPoint3<float> p = chamfer_point<SOA, float>(Q, d.qrows, qi);
+        qx[i] = p.x;
+        qy[i] = p.y;
+        qz[i] = p.z;
+        best[i] = INF;
+        where[i] = -1;
+    }
+    // this wave's stretch of keys, whole chunks
+    const int each = ((nk + NW - 1) / NW + CHUNK - 1) / CHUNK * CHUNK;
+    const int from = wave * each, to = from + each < nk ? from + each : nk;
+    const auto fetch = [&](int c) {
+        const int j = c + lane;
+        const TkPoint3<float> p = chamfer_point<SOA, float>(K, d.krows, j < nk ? j : nk - 1);
+        return j < nk ? make_float4(p.x, p.y, p.z, 0.0f) : make_float4(NAN_, NAN_, NAN_, 0.0f);
+    };
+    float4 next = from < to ? fetch(from) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    int buf = 0;
+    for (int c = from; c < to; c += CHUNK, buf ^= 1) {
+        s_key[wave][buf][lane] = next;
+        __builtin_amdgcn_wave_barrier();
+        if (c + CHUNK < to)
+            next = fetch(c + CHUNK);
+#pragma unroll
+        for (int t = 0; t < CHUNK / TILE; ++t) {
+            const float4 *keys = &s_key[wave][buf][t * TILE];
+            float low[QPL];
+#pragma unroll
+            for (int i = 0; i < QPL; ++i)
+                low[i] = INF;
+#pragma unroll
+            for (int j = 0; j < TILE; j += 2) {
+                const float4 ka = keys[j], kb = keys[j + 1];
+#pragma unroll
+                for (int i = 0; i < QPL; ++i) {
+                    const float da = tk_dist2<float>(qx[i], qy[i], qz[i], ka.x, ka.y, ka.z);
+                    const float db = tk_dist2<float>(qx[i], qy[i], qz[i], kb.x, kb.y, kb.z);
+                    low[i] = __builtin_fminf(__builtin_fminf(low[i], da), db);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < QPL; ++i) {
+                const bool lower = low[i] < best[i];
+                best[i] = lower ? low[i] : best[i];
+                where[i] = lower ? c + t * TILE : where[i];
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < QPL; ++i) {
+        s_val[wave][i * TK_WAVE + lane] = best[i];
+        s_tile[wave][i * TK_WAVE + lane] = where[i];
+    }
+    __syncthreads();
+    // the lowest of the waves' minima, the first tile that has it, and in that the first key
+    const int q = tid / LPQ, part = tid % LPQ, qi = q < QB ? qblock * QB + q : nq;
+    if (q >= QB)  // (whole waves)
+        return;
+    float value = s_val[0][q];
+    int tile = s_tile[0][q];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) {
+        const float v = s_val[w][q];
+        const int t = s_tile[w][q];
+        const bool lower = v < value;  // (waves hold ascending stretches)
+        value = lower ? v : value;
+        tile = lower ? t : tile;
+    }
+    int found = 0x7fffffff;
+    if (qi < nq && tile >= 0) {
+        const TkPoint3<float> p = chamfer_point<SOA, float>(Q, d.qrows, qi);
+#pragma unroll
+        for (int u = TILE / LPQ - 1; u >= 0; --u) {
+            const int j = tile + u * LPQ + part;
+            const TkPoint3<float> k = chamfer_point<SOA, float>(K, d.krows, j < nk ? j : nk - 1);
+            const float dist = tk_dist2<float>(p.x, p.y, p.z, k.x, k.y, k.z);
+            found = j < nk && dist == value ? j : found;
+        }
+    }
+#pragma unroll
+    for (int o = 1; o < LPQ; o <<= 1) {
+        const int other = __shfl_xor(found, o);
+        found = other < found ? other : found;
+    }
+    if (part == 0 && qi < nq) {
+        const int64_t o = (int64_t)b * nq + qi;
+        d.dist[o] = value;
+        d.idx[o] = (int64_t)(tile >= 0 ? found : -1);
+        float *const root = roots.root[&d == &args.dir[1] ? 1 : 0];
+        if (root)
+            root[o] = chamfer_root(value, roots.eps);
+    }
+}
+
 // Split sweeps: the index outputs start as packed (+inf, -1) words ...
 __global__ __launch_bounds__(256) void chamfer_split_init_kernel(ChamferFwdArgs<float> args,
                                                                  int64_t total0, int64_t total1)
@@ -1939,6 +2081,70 @@ inline int64_t chamfer_matrix_blocks(int64_t B, int64_t N1, int64_t N2, int (&wa
 }
 constexpr int64_t CHAMFER_MATRIX_BLOCKS = 96;  // fewer: the vector pre-filter ([N,3] clouds)
 
+// The shape of the team sweep for a call (queries per lane; 0: left to the other sweeps), from its time
+// in microseconds: a CU takes one workgroup after the other (8-wave ones overlap a little), each `key`
+// per key of the longer cloud and `start`. Within 12 % on 37 shapes of 64 to 16384 points in both layouts;
+// above it on launches of many rounds. Where the line lies, other sweeps -> this:
+// - One workgroup per CU: 20 to 26 us at most for the others (1 x 4096 x 4096 23 -> 19, 16 x 2048 x 2048
+//   26 -> 21, 4 x 4096 x 4096 26 -> 22; 1 x 8192 x 8192 26 against 36).
+// - More: 32 x 1024 x 1024 16 -> 14, but 64 x 1024 x 1024 [3,N] 22.3 against 23.8.
+// - Lengths that are no multiple of four (a copy to padded rows before the others): 8 x 2500 x 3001 40 ->
+//   23, 32 x 600 x 2300 50 -> 31; 8 x 4099 x 4097 38 against 52.
+// - A cloud too short for the pre-filters: 3 x 5001 x 300 161 -> 23, 1 x 20000 x 100 608 -> 83, 64 x 300 x
+//   300 19 -> 7.5, 512 x 256 x 256 27 -> 19.
+inline int chamfer_team_shape(int64_t B, int64_t N1, int64_t N2, bool soa)
+{
+    const int64_t most = N1 > N2 ? N1 : N2, least = N1 > N2 ? N2 : N1;
+    if (B <= 0 || least <= 0 || B > 65536 || most > 65536)
+        return 0;
+    const double key[4] = {3.6e-3, 4.0e-3, 5.6e-3, 7.1e-3}, start[4] = {0.3, 1.2, 1.2, 1.2};
+    double best = 1e30;
+    int shape = 0;
+    int64_t rounds = 0;
+    for (int q = 0; q < 4; ++q) {
+        const int64_t qb = 64 * (q + 1);
+        const int64_t r = (B * ((N1 + qb - 1) / qb + (N2 + qb - 1) / qb) + 255) / 256;
+        const double t = 4.5 + (double)r * (key[q] * (double)most + start[q]);
+        if (t < best) {
+            best = t;
+            shape = q + 1;
+            rounds = r;
+        }
+    }
+    const bool ragged = ((N1 | N2) & 3) != 0 && (B > 1 || soa);
+    int want[2];
+    const bool unfiltered = least < 512 && (most < 1024 || (!soa && chamfer_matrix_blocks(B, N1, N2, want) <
+                                                                        CHAMFER_MATRIX_BLOCKS));
+    const double limit = unfiltered ? 22.0 + 0.02 * (double)most : ragged ? 33.0 : rounds == 1 ? 22.5 : 21.0;
+    return best <= limit ? shape : 0;
+}
+
+template <bool SOA>
+int chamfer_team_launch(int shape, const float *xyz1, const float *xyz2, int64_t B, int64_t N1,
+                        int64_t N2, float *dist1, int64_t *idx1, float *dist2, int64_t *idx2,
+                        const ChamferRoots &roots, hipStream_t s, int64_t rows1, int64_t rows2)
+{
+    ChamferFwdArgs<float> a;
+    int64_t nblocks;
+    const auto go = [&](auto q, auto waves) {
+        constexpr int Q = decltype(q)::value, NW = decltype(waves)::value;
+        const int rc = chamfer_fill_args<float, Q * TK_WAVE, 32>(
+            a, xyz1, xyz2, B, N1, N2, dist1, idx1, dist2, idx2, 1, nblocks, -1, rows1, rows2);
+        if (rc != TK3D_OK)
+            return rc;
+        hipLaunchKernelGGL((chamfer_forward_team_kernel<Q, NW, SOA>), dim3((unsigned)nblocks),
+                           dim3(NW * TK_WAVE), 0, s, a, roots);
+        return tk_launch_status();
+    };
+    using std::integral_constant;
+    switch (shape) {
+    case 1: return go(integral_constant<int, 1>(), integral_constant<int, 8>());
+    case 2: return go(integral_constant<int, 2>(), integral_constant<int, 16>());
+    case 3: return go(integral_constant<int, 3>(), integral_constant<int, 16>());
+    default: return go(integral_constant<int, 4>(), integral_constant<int, 16>());
+    }
+}
+
 // rows1, rows2: points from one batch element to the next where that is more than N1, N2.
 template <typename T, bool SOA = false>
 int chamfer_forward(const T *xyz1, const T *xyz2, int64_t B, int64_t N1, int64_t N2,
@@ -1959,6 +2165,9 @@ int chamfer_forward(const T *xyz1, const T *xyz2, int64_t B, int64_t N1, int64_t
     // spreads over the chip.
     const int64_t work = B * (N1 > N2 ? N1 : N2);
     if constexpr (sizeof(T) == 4) {
+        if (const int shape = chamfer_team_shape(B, N1, N2, SOA))
+            return chamfer_team_launch<SOA>(shape, xyz1, xyz2, B, N1, N2, dist1, idx1, dist2, idx2,
+                                            ChamferRoots{}, s, rows1, rows2);
         // The pre-filter pays off once the key clouds are a few hundred points long
         // (its prologue passes over the keys twice per workgroup).
         const int64_t nkmin = N1 < N2 ? N1 : N2;
@@ -3837,6 +4046,7 @@ int chamfer_rows(const T *xyz1, const T *xyz2, bool soa, int64_t B, int64_t N1, 
 //   1025: 36 -> 21 us) and beats the exact sweep of clouds too short for it (8 x 1000 x 1000: 54 -> 22
 //   us). It takes clouds from 512 points on; below that, with the longer one at 1024 or more, [N,3]
 //   clouds would go through the exact sweep (B=4, 5001 x 300: 40 us as they are, 165 us copied).
+// (Timed against those sweeps; the calls that chamfer_team_shape takes read the clouds in place.)
 inline bool chamfer_copy_pays(int64_t B, int64_t N1, int64_t N2, bool soa)
 {
     const int64_t most = N1 > N2 ? N1 : N2, least = N1 > N2 ? N2 : N1;
@@ -3863,9 +4073,13 @@ __global__ __launch_bounds__(256) void chamfer_roots_kernel(const T *__restrict_
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= n)
         return;
-    const T d = i < n1 ? d1[i] : d2[i - n1];
-    const T c = d < eps ? eps : d;  // a NaN stays a NaN, as in clamp
-    (i < n1 ? r1[i] : r2[i - n1]) = sizeof(T) == 4 ? (T)__builtin_sqrtf((float)c) : (T)__builtin_sqrt((double)c);
+    (i < n1 ? r1[i] : r2[i - n1]) = chamfer_root<T>(i < n1 ? d1[i] : d2[i - n1], eps);
+}
+
+template <typename T> __device__ __forceinline__ T chamfer_root_grad(T g, T d, T root, T eps)
+{
+    const T of_root = g / (root * 2);
+    return d >= eps ? of_root : (T)0;
 }
 
 template <typename T>
@@ -3879,8 +4093,33 @@ __global__ __launch_bounds__(256) void chamfer_root_grads_kernel(
         return;
     const bool second = i >= n1;
     i -= second ? n1 : 0;
-    const T g = (second ? g2 : g1)[i] / ((second ? r2 : r1)[i] * 2);
-    (second ? o2 : o1)[i] = (second ? d2 : d1)[i] >= eps ? g : (T)0;
+    (second ? o2 : o1)[i] = chamfer_root_grad<T>((second ? g2 : g1)[i], (second ? d2 : d1)[i],
+                                                 (second ? r2 : r1)[i], eps);
+}
+
+// The same for [B,3,N] clouds together with chamfer_rows_kernel: a lane has a point and its gradient.
+__global__ __launch_bounds__(256) void chamfer_root_grads_rows_kernel(
+    const float *__restrict__ g1, const float *__restrict__ g2, const float *__restrict__ d1,
+    const float *__restrict__ d2, const float *__restrict__ r1, const float *__restrict__ r2,
+    const float *__restrict__ xyz1, const float *__restrict__ xyz2, int n1, int n2, int64_t total1,
+    int64_t total, float eps, float *__restrict__ o1, float *__restrict__ o2, float *__restrict__ out1,
+    float *__restrict__ out2)
+{
+    int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= total)
+        return;
+    const bool second = i >= total1;
+    i -= second ? total1 : 0;
+    (second ? o2 : o1)[i] = chamfer_root_grad<float>((second ? g2 : g1)[i], (second ? d2 : d1)[i],
+                                                     (second ? r2 : r1)[i], eps);
+    const int n = second ? n2 : n1;
+    const int64_t b = i / n;
+    const TkPoint3<float> p =
+        chamfer_point<true, float>((second ? xyz2 : xyz1) + b * n * 3, n, (int)(i - b * n));
+    float *out = (second ? out2 : out1) + i * 3;
+    out[0] = p.x;
+    out[1] = p.y;
+    out[2] = p.z;
 }
 
 // ---- entry points for the tests and the benchmark (tk3d_debug.h) ----------------------
@@ -4207,6 +4446,51 @@ int tk3d_chamfer_root_grads_f64(const double *grad1, const double *grad2, const 
     return tk_launch_status();
 }
 
+int tk3d_chamfer_distance_forward_roots_f32(const float *xyz1, const float *xyz2, int channels_first,
+                                            int64_t B, int64_t N1, int64_t N2, double eps, float *dist1,
+                                            int64_t *idx1, float *dist2, int64_t *idx2, float *root1,
+                                            float *root2, void *stream)
+{
+    const int shape = chamfer_team_shape(B, N1, N2, channels_first != 0);
+    if (!shape || !tk_fits(TK_MAX_ELEMS, B, N1, 3) || !tk_fits(TK_MAX_ELEMS, B, N2, 3))
+        return TK3D_ERR_UNSUPPORTED;
+    if (!xyz1 || !xyz2 || !dist1 || !idx1 || !dist2 || !idx2 || !root1 || !root2)
+        return TK3D_ERR_NULL_POINTER;
+    const ChamferRoots roots{{root1, root2}, (float)eps};
+    return channels_first
+               ? chamfer_team_launch<true>(shape, xyz1, xyz2, B, N1, N2, dist1, idx1, dist2, idx2, roots,
+                                           (hipStream_t)stream, 0, 0)
+               : chamfer_team_launch<false>(shape, xyz1, xyz2, B, N1, N2, dist1, idx1, dist2, idx2, roots,
+                                            (hipStream_t)stream, 0, 0);
+}
+
+int tk3d_chamfer_root_grads_rows_f32(const float *grad1, const float *grad2, const float *dist1,
+                                     const float *dist2, const float *root1, const float *root2,
+                                     const float *xyz1, const float *xyz2, int64_t B, int64_t N1,
+                                     int64_t N2, double eps, float *grads1, float *grads2, float *out1,
+                                     float *out2, void *stream)
+{
+    if (B < 0 || N1 < 0 || N2 < 0)
+        return TK3D_ERR_BAD_SIZE;
+    if (N1 > TK_MAX_I32 || N2 > TK_MAX_I32 || !tk_fits(TK_MAX_ELEMS, B, N1, 3) ||
+        !tk_fits(TK_MAX_ELEMS, B, N2, 3))
+        return TK3D_ERR_UNSUPPORTED;
+    const int64_t t1 = B * N1, total = t1 + B * N2, blocks = (total + 255) / 256;
+    if (blocks > TK_MAX_I32)
+        return TK3D_ERR_UNSUPPORTED;
+    if (blocks == 0)
+        return TK3D_OK;
+    hipLaunchKernelGGL(chamfer_root_grads_rows_kernel, dim3((unsigned)blocks), dim3(256), 0,
+                       (hipStream_t)stream, grad1, grad2, dist1, dist2, root1, root2, xyz1, xyz2, (int)N1,
+                       (int)N2, t1, total, (float)eps, grads1, grads2, out1, out2);
+    return tk_launch_status();
+}
+
+int tk3d_chamfer_distance_forward_in_place(int64_t B, int64_t N1, int64_t N2, int channels_first)
+{
+    return chamfer_team_shape(B, N1, N2, channels_first != 0) != 0;
+}
+
 size_t tk3d_chamfer_distance_forward_rows_bytes(int64_t B, int64_t N1, int64_t N2, int channels_first)
 {
     if (!chamfer_copy_pays(B, N1, N2, channels_first != 0))
@@ -4223,7 +4507,8 @@ int tk3d_chamfer_distance_forward_rows_f32(const float *xyz1, const float *xyz2,
     if (B <= 0 || N1 <= 0 || N2 <= 0 || workspace == nullptr ||
         (reinterpret_cast<uintptr_t>(workspace) & 15) != 0 ||
         !tk_fits(TK_MAX_ELEMS, B, rows1 + rows2, 3) ||
-        workspace_bytes < (size_t)B * (size_t)(rows1 + rows2) * 3 * sizeof(float))
+        workspace_bytes < (size_t)B * (size_t)(rows1 + rows2) * 3 * sizeof(float) ||
+        chamfer_team_shape(B, N1, N2, channels_first != 0))
         return channels_first
                    ? chamfer_forward<float, true>(xyz1, xyz2, B, N1, N2, dist1, idx1, dist2, idx2, stream)
                    : chamfer_forward<float>(xyz1, xyz2, B, N1, N2, dist1, idx1, dist2, idx2, stream);

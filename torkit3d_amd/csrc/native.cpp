@@ -213,7 +213,19 @@ std::tuple<Tensor, Tensor, Tensor> three_nn(const Tensor &query, const Tensor &k
     return {distance, index, weight};
 }
 
-std::vector<Tensor> chamfer_forward(const Tensor &xyz1, const Tensor &xyz2, bool channels_first)
+// sqrt(max(d, eps)) of both directions.
+std::vector<Tensor> roots(const Tensor &d1, const Tensor &d2, double eps)
+{
+    OnDeviceOf guard(d1.device());
+    const Tensor r1 = like(d1, d1.sizes()), r2 = like(d2, d2.sizes());
+    TK3D_CALL(is_f32(d1), tk3d_chamfer_roots, ptr(d1), ptr(d2), d1.numel(), d2.numel(), eps, ptr(r1),
+              ptr(r2), stream_of(d1));
+    return {r1, r2};
+}
+
+// dist1, idx1, dist2, idx2 and, where `root`, sqrt(max(dist, eps)) of both.
+std::vector<Tensor> chamfer_forward(const Tensor &xyz1, const Tensor &xyz2, bool channels_first,
+                                    bool root = false, double eps = 0.0)
 {
     const Cloud a = cloud_dims("xyz1", xyz1, channels_first);
     const Cloud c = cloud_dims("xyz2", xyz2, channels_first);
@@ -223,6 +235,16 @@ std::vector<Tensor> chamfer_forward(const Tensor &xyz1, const Tensor &xyz2, bool
     const Tensor dist1 = like(xyz1, {a.b, a.n}), idx1 = index_like(xyz1, {a.b, a.n});
     const Tensor dist2 = like(xyz1, {a.b, c.n}), idx2 = index_like(xyz1, {a.b, c.n});
     void *stream = stream_of(xyz1);
+    const bool in_place =
+        is_f32(xyz1) && tk3d_chamfer_distance_forward_in_place(a.b, a.n, c.n, channels_first);
+    if (in_place && root) {
+        const Tensor r1 = like(xyz1, {a.b, a.n}), r2 = like(xyz1, {a.b, c.n});
+        done(tk3d_chamfer_distance_forward_roots_f32(ptr(xyz1), ptr(xyz2), channels_first, a.b, a.n, c.n,
+                                                     eps, ptr(dist1), ptr(idx1), ptr(dist2), ptr(idx2),
+                                                     ptr(r1), ptr(r2), stream),
+             "tk3d_chamfer_distance_forward_roots_f32");
+        return {dist1, idx1, dist2, idx2, r1, r2};
+    }
     if (is_f32(xyz1)) {
         // Clouds of a few thousand points and more are sorted along a space-filling curve in a
         // scratch buffer, and only key tiles near a wave's queries are swept. (On [B,3,N]
@@ -231,7 +253,7 @@ std::vector<Tensor> chamfer_forward(const Tensor &xyz1, const Tensor &xyz2, bool
         const size_t bytes =
             sortable ? tk3d_chamfer_distance_forward_workspace_bytes(a.b, a.n, c.n, 0) : 0;
         const size_t copy_bytes =
-            bytes ? 0 : tk3d_chamfer_distance_forward_rows_bytes(a.b, a.n, c.n, channels_first);
+            bytes || in_place ? 0 : tk3d_chamfer_distance_forward_rows_bytes(a.b, a.n, c.n, channels_first);
         const Tensor ws = scratch(xyz1, bytes ? bytes : copy_bytes);
         const auto call = channels_first ? tk3d_chamfer_distance_forward_bcn_f32
                                          : tk3d_chamfer_distance_forward_ws_f32;
@@ -250,6 +272,10 @@ std::vector<Tensor> chamfer_forward(const Tensor &xyz1, const Tensor &xyz2, bool
         done(call(ptr(xyz1), ptr(xyz2), a.b, a.n, c.n, ptr(dist1), ptr(idx1), ptr(dist2),
                   ptr(idx2), stream),
              "tk3d_chamfer_distance_forward_f64");
+    }
+    if (root) {
+        const std::vector<Tensor> r = roots(dist1, dist2, eps);
+        return {dist1, idx1, dist2, idx2, r[0], r[1]};
     }
     return {dist1, idx1, dist2, idx2};
 }
@@ -435,32 +461,21 @@ template <typename... T> bool tracked(const T &...t)
     return c10::GradMode::is_enabled() && ((t.defined() && t.requires_grad()) || ...);
 }
 
-// sqrt(max(d, eps)) of both directions.
-std::vector<Tensor> roots(const Tensor &d1, const Tensor &d2, double eps)
-{
-    OnDeviceOf guard(d1.device());
-    const Tensor r1 = like(d1, d1.sizes()), r2 = like(d2, d2.sizes());
-    TK3D_CALL(is_f32(d1), tk3d_chamfer_roots, ptr(d1), ptr(d2), d1.numel(), d2.numel(), eps, ptr(r1),
-              ptr(r2), stream_of(d1));
-    return {r1, r2};
-}
-
 struct ChamferNode : torch::autograd::Function<ChamferNode> {
     static variable_list forward(AutogradContext *ctx, const Tensor &xyz1, const Tensor &xyz2,
                                  bool channels_first, bool root, double eps)
     {
         const Tensor a = xyz1.contiguous(), c = xyz2.contiguous();
-        const std::vector<Tensor> out = chamfer_forward(a, c, channels_first);
+        const std::vector<Tensor> out = chamfer_forward(a, c, channels_first, root, eps);
         ctx->saved_data["channels_first"] = channels_first;
         ctx->saved_data["want"] = (xyz1.requires_grad() ? 1 : 0) + (xyz2.requires_grad() ? 2 : 0);
         if (!root) {
             ctx->save_for_backward({a, c, out[1], out[3]});
             return {out[0], out[2]};
         }
-        const std::vector<Tensor> r = roots(out[0], out[2], eps);
         ctx->saved_data["eps"] = eps;
-        ctx->save_for_backward({a, c, out[1], out[3], out[0], out[2], r[0], r[1]});
-        return r;
+        ctx->save_for_backward({a, c, out[1], out[3], out[0], out[2], out[4], out[5]});
+        return {out[4], out[5]};
     }
     static variable_list backward(AutogradContext *ctx, variable_list grads)
     {
@@ -470,22 +485,34 @@ struct ChamferNode : torch::autograd::Function<ChamferNode> {
         Tensor g1 = grads[0].contiguous(), g2 = grads[1].contiguous();
         Tensor a = saved[0], c = saved[1];
         OnDeviceOf guard(a.device());
+        // (the backward kernel works on [B,N,3])
+        const int64_t b = a.size(0), n1 = g1.size(1), n2 = g2.size(1);
+        const Tensor a3 = channels_first ? like(a, {b, n1, 3}) : a;
+        const Tensor c3 = channels_first ? like(c, {b, n2, 3}) : c;
+        bool copied = !channels_first;
         if (saved.size() > 4) {
+            const double eps = ctx->saved_data["eps"].toDouble();
             const Tensor o1 = like(g1, g1.sizes()), o2 = like(g2, g2.sizes());
-            TK3D_CALL(is_f32(g1), tk3d_chamfer_root_grads, ptr(g1), ptr(g2), ptr(saved[4]),
-                      ptr(saved[5]), ptr(saved[6]), ptr(saved[7]), g1.numel(), g2.numel(),
-                      ctx->saved_data["eps"].toDouble(), ptr(o1), ptr(o2), stream_of(g1));
+            if (channels_first && is_f32(a)) {
+                done(tk3d_chamfer_root_grads_rows_f32(ptr(g1), ptr(g2), ptr(saved[4]), ptr(saved[5]),
+                                                      ptr(saved[6]), ptr(saved[7]), ptr(a), ptr(c), b, n1,
+                                                      n2, eps, ptr(o1), ptr(o2), ptr(a3), ptr(c3),
+                                                      stream_of(g1)),
+                     "tk3d_chamfer_root_grads_rows_f32");
+                copied = true;
+            } else {
+                TK3D_CALL(is_f32(g1), tk3d_chamfer_root_grads, ptr(g1), ptr(g2), ptr(saved[4]),
+                          ptr(saved[5]), ptr(saved[6]), ptr(saved[7]), g1.numel(), g2.numel(), eps,
+                          ptr(o1), ptr(o2), stream_of(g1));
+            }
             g1 = o1;
             g2 = o2;
         }
-        if (channels_first) {  // (the backward kernel works on [B,N,3])
-            const int64_t b = a.size(0), n1 = a.size(2), n2 = c.size(2);
-            const Tensor a3 = like(a, {b, n1, 3}), c3 = like(c, {b, n2, 3});
+        if (!copied)
             TK3D_CALL(is_f32(a), tk3d_chamfer_rows, ptr(a), ptr(c), 1, b, n1, n2, n1, n2, ptr(a3),
                       ptr(c3), stream_of(a));
-            a = a3;
-            c = c3;
-        }
+        a = a3;
+        c = c3;
         std::vector<Tensor> g = chamfer_backward(g1, g2, a, c, saved[2], saved[3], (want & 1) != 0,
                                                  (want & 2) != 0);
         for (int i = 0; i < 2; ++i) {
@@ -505,12 +532,9 @@ std::tuple<Tensor, Tensor> chamfer(const Tensor &xyz1, const Tensor &xyz2, bool 
         const variable_list out = ChamferNode::apply(xyz1, xyz2, channels_first, root, eps);
         return {out[0], out[1]};
     }
-    std::vector<Tensor> out = chamfer_forward(xyz1.contiguous(), xyz2.contiguous(), channels_first);
-    if (root) {
-        const std::vector<Tensor> r = roots(out[0], out[2], eps);
-        return {r[0], r[1]};
-    }
-    return {out[0], out[2]};
+    const std::vector<Tensor> out =
+        chamfer_forward(xyz1.contiguous(), xyz2.contiguous(), channels_first, root, eps);
+    return root ? std::tuple<Tensor, Tensor>{out[4], out[5]} : std::tuple<Tensor, Tensor>{out[0], out[2]};
 }
 
 struct GroupNode : torch::autograd::Function<GroupNode> {
