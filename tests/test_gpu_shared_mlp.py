@@ -107,6 +107,25 @@ def test_maximum_over_neighbours(cuda, monkeypatch, b, m, s, widths, training):
           [(randn(m, b, widths[0], m, s), True)], monkeypatch)
 
 
+# Products whose waves share a tile: gradients in tiles of 64 x 64 with remainders of both, groups of 32 and
+# of 64 in evaluation (one channel tile and two), channels that leave waves without a group of eight.
+@pytest.mark.parametrize("b,p,widths,pool,training", [
+    (4, 4100, (260, 256, 140), 0, True), (2, 8252, (131, 192, 128), 0, True), (3, 130, (20, 9, 200), 0, True),
+    (1, 32, (16, 64, 128), 64, False), (4, 65, (9, 40, 130), 64, False), (1, 100, (6, 33, 70), 32, False),
+    (1, 260, (200, 128, 64), 32, False), (2, 3, (7, 8, 9), 64, False)])
+def test_products_of_shared_tiles(cuda, monkeypatch, b, p, widths, pool, training):
+    mlp = make(mlp2d_bn_relu if pool else mlp1d_bn_relu, widths[0], widths[1:], training, cuda)
+    x = randn(p, b, widths[0], p, *([pool] if pool else []))
+    fused = (lambda m, x: m.forward_max(x)) if pool else (lambda m, x: m(x))
+    reference = (lambda m, x: m(x).max(dim=3)[0]) if pool else (lambda m, x: m(x))
+    check(mlp, fused, reference, [(x, True)], monkeypatch)
+    if not training:  # infinities and NaN stay where they are
+        x[0, 0, 0], x[-1, -1, -1] = float("inf"), float("nan")
+        with torch.no_grad():
+            got, want = fused(mlp, x), reference(stock(mlp, torch.float32), x)
+        assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+
+
 # Grouped input: with features (gradient wanted or not, few or many), without, indices outside.
 @pytest.mark.parametrize("training", [True, False])
 @pytest.mark.parametrize("features,tracked,n,m,s", [

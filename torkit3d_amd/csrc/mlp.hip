@@ -89,6 +89,221 @@ struct GemmArgs {
     int chunk;       // groups whose weights are in LDS at once
     int slots;       // partial sums per channel (gridDim.x)
     int coef_bytes;
+    int rows4;       // weight rows are 16-byte aligned runs along the input channels
+};
+
+// LDS: normalisation of the input channels.
+template <int IN>
+__device__ __forceinline__ void input_constants(const tk3d_mlp_product &p, int kg, f32x4 *grad_coef,
+                                                f32x4 *act_coef, int tid, int threads)
+{
+    if constexpr (IN == IN_ACT || IN == IN_CENTRED || IN == IN_GRAD_OUT) {
+        const int K = p.src[0].K;
+        for (int k = tid; k < ((K + 7) & ~7); k += threads)
+            act_coef[k] = k < K ? constants_of(p.in_norm, k) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    if constexpr (reads_y(IN)) {
+        const f32x4 *coef = reinterpret_cast<const f32x4 *>(p.src[0].coef);
+        for (int k = tid; k < kg * 8; k += threads)
+            grad_coef[k] = k < p.src[0].K ? coef[k] : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+}
+
+// Rows of a group of eight input channels (a lane's four: 2 q + half) at PT positions.
+template <int IN, int PT>
+__device__ __forceinline__ void load_rows(const tk3d_mlp_product &p, int kg0, int b, int pos, int half, int g,
+                                          float (&x)[4][PT], float (&y)[4][PT])
+{
+    const bool second = IN == IN_RAW2 && g >= kg0;
+    const tk3d_mlp_source &s = p.src[second ? 1 : 0];
+    const int k0 = (g - (second ? kg0 : 0)) * 8 + half;
+    const float *in = s.x + (int64_t)b * s.batch_stride;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int k = k0 + 2 * q < s.K ? k0 + 2 * q : s.K - 1;
+        const unsigned offset = ((unsigned)k * (unsigned)p.P + (unsigned)pos) * 4u;
+        load_run<PT>(x[q], in, offset);
+        if constexpr (reads_y(IN))
+            load_run<PT>(y[q], s.y + (int64_t)b * s.batch_stride, offset);
+    }
+}
+
+// in(k, p) of such a group.
+template <int IN, int PT>
+__device__ __forceinline__ void inputs_of(const tk3d_mlp_product &p, int kg0, int half, int g,
+                                          const float (&x)[4][PT], const float (&yy)[4][PT],
+                                          const f32x4 *grad_coef, const f32x4 *act_coef, float (&v)[4][PT])
+{
+    const bool second = IN == IN_RAW2 && g >= kg0;
+    const int K = p.src[second ? 1 : 0].K, gs = g - (second ? kg0 : 0);
+    const int k0 = gs * 8 + half;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        if constexpr (reads_y(IN)) {
+            const f32x4 c = grad_coef[k0 + 2 * q];
+            f32x4 ss{0.0f, 0.0f, 0.0f, 0.0f};
+            if constexpr (IN == IN_GRAD_OUT)
+                ss = act_coef[k0 + 2 * q];
+#pragma unroll
+            for (int t = 0; t < PT; ++t) {
+                float e = x[q][t];
+                const float y = yy[q][t];
+                if constexpr (IN == IN_GRAD_OUT)
+                    e = passes(normalised(y, ss)) ? e : 0.0f;
+                v[q][t] = __builtin_fmaf(c.x, e, __builtin_fmaf(c.y, y, c.z));
+            }
+        } else if constexpr (IN == IN_ACT || IN == IN_CENTRED) {
+            const f32x4 c = act_coef[k0 + 2 * q];
+            const float centre = IN == IN_CENTRED ? centre_of(c) : 0.0f;
+#pragma unroll
+            for (int t = 0; t < PT; ++t) {
+                v[q][t] = relu(normalised(x[q][t], c));
+                if constexpr (IN == IN_CENTRED)
+                    v[q][t] -= centre;
+            }
+        } else {
+#pragma unroll
+            for (int t = 0; t < PT; ++t)
+                v[q][t] = x[q][t];
+        }
+    }
+    if (gs * 8 + 8 > K) {  // channels past the last one (their weights are zero) must not be inf
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int t = 0; t < PT; ++t)
+                v[q][t] = k0 + 2 * q < K ? v[q][t] : 0.0f;
+    }
+}
+
+// What becomes of the sums: lane's channel of each of CT tiles, runs of 4 * PT positions.
+template <int IN, int OUT, int PT, int CT> struct Results {
+    static constexpr int RUN = 4 * PT;
+    int chan[CT];
+    float shift[CT], sum1[CT], sum2[CT];
+    f32x4 out_coef[CT];
+    float sign[CT], bias[CT];
+
+    __device__ __forceinline__ void prepare(const tk3d_mlp_product &p, int cbase, int col)
+    {
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) {
+            chan[ct] = cbase + ct * 32 + col;
+            const int c = chan[ct] < p.C ? chan[ct] : p.C - 1;
+            sum1[ct] = sum2[ct] = shift[ct] = 0.0f;
+            if constexpr (OUT == OUT_EVAL || OUT == OUT_POOL_EVAL || OUT == OUT_MASK)
+                out_coef[ct] = constants_of(p.out_norm, c);
+            if constexpr (OUT == OUT_POOL_EVAL)
+                sign[ct] = sign_of(p.out_norm.gamma[c]);
+            if constexpr (OUT == OUT_MASK) {
+                shift[ct] = p.out_norm.mean[c];
+                bias[ct] = p.bias ? p.bias[c] : 0.0f;
+            }
+            if constexpr (OUT == OUT_PLAIN)
+                bias[ct] = p.bias ? p.bias[c] : 0.0f;
+        }
+    }
+
+    __device__ __forceinline__ void put(const tk3d_mlp_product &p, int b, int ct, int pos, bool full,
+                                        float (&v)[RUN])
+    {
+        const int P = p.P, c = chan[ct];
+        const bool mine = c < p.C, vec = (P & 3) == 0;
+        float *row = nullptr;
+        if constexpr (OUT == OUT_PLAIN || OUT == OUT_EVAL || OUT == OUT_MASK) {
+            const bool first = c < p.C0;
+            float *out = first ? p.out : p.out2;
+            const int rows = first ? p.C0 : p.C - p.C0, r = first ? c : c - p.C0;
+            row = mine && out ? out + ((int64_t)b * rows + r) * P : nullptr;
+        }
+        if constexpr (OUT == OUT_MASK || OUT == OUT_PLAIN) {
+#pragma unroll
+            for (int i = 0; i < RUN; ++i)
+                v[i] += bias[ct];
+        }
+        if constexpr (OUT == OUT_MASK) {
+            float before[RUN];
+            const float *yrow = p.yprev + ((int64_t)b * p.C + (mine ? c : p.C - 1)) * P;
+            if (vec) {
+#pragma unroll
+                for (int i = 0; i < PT; ++i) {
+                    const int at = pos + 4 * i > P - 4 ? P - 4 : pos + 4 * i;
+                    const f32x4 w = *reinterpret_cast<const f32x4 *>(yrow + at);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        before[4 * i + j] = w[j];
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < RUN; ++i)
+                    before[i] = yrow[pos + i > P - 1 ? P - 1 : pos + i];
+            }
+            if constexpr (IN == IN_CENTRED) {  // (P is a multiple of 32 here)
+                const float *arow = p.add + ((int64_t)b * p.C + (mine ? c : p.C - 1)) * P;
+#pragma unroll
+                for (int i = 0; i < PT; ++i) {
+                    const int at = pos + 4 * i > P - 4 ? P - 4 : pos + 4 * i;
+                    const f32x4 w = *reinterpret_cast<const f32x4 *>(arow + at);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        v[4 * i + j] += w[j];
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < RUN; ++i)
+                v[i] = passes(normalised(before[i], out_coef[ct])) ? v[i] : 0.0f;
+#pragma unroll
+            for (int i = 0; i < RUN; ++i) {
+                if (full || pos + i < P) {
+                    sum1[ct] += v[i];
+                    sum2[ct] = __builtin_fmaf(v[i], before[i] - shift[ct], sum2[ct]);
+                }
+            }
+        }
+        if constexpr (OUT == OUT_EVAL) {
+#pragma unroll
+            for (int i = 0; i < RUN; ++i)
+                v[i] = relu(normalised(v[i], out_coef[ct]));
+        }
+        if constexpr (OUT == OUT_POINTS) {
+#pragma unroll
+            for (int i = 0; i < RUN; ++i)
+                if (mine && pos + i < P)
+                    p.out[((int64_t)b * P + pos + i) * p.C + c] = v[i];
+        } else if (row) {
+            if (vec) {
+#pragma unroll
+                for (int i = 0; i < PT; ++i)
+                    if (full || pos + 4 * i < P)
+                        *reinterpret_cast<f32x4 *>(row + pos + 4 * i) =
+                            f32x4{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
+            } else {
+#pragma unroll
+                for (int i = 0; i < RUN; ++i)
+                    if (pos + i < P)
+                        row[pos + i] = v[i];
+            }
+        }
+    }
+
+    // The extreme of a run, as a maximum, and what becomes of a group's.
+    __device__ __forceinline__ float extreme(int ct, const float (&v)[RUN]) const
+    {
+        float best = v[0] * sign[ct];
+#pragma unroll
+        for (int i = 1; i < RUN; ++i)
+            best = __builtin_elementwise_maximum(best, v[i] * sign[ct]);
+        return best;
+    }
+    __device__ __forceinline__ void put_extreme(const tk3d_mlp_product &p, int b, int ct, int pos, int half,
+                                                float best) const
+    {
+        best = __builtin_elementwise_maximum(best, __shfl_xor(best, 32));
+        const int m = pos / p.group, c = chan[ct];
+        if (c < p.C && half == 0 && pos < p.P)
+            p.out[((int64_t)b * p.C + c) * p.M + m] =
+                relu(normalised(sign[ct] == 0.0f ? best : best * sign[ct], out_coef[ct]));
+    }
 };
 
 template <int IN, int OUT, int PT, int CT>
@@ -101,23 +316,14 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
     const int cbase = blockIdx.y * (32 * CT);
     const int P = p.P;
 
-    // LDS: normalisation of the input channels, then the weights.
+    // LDS: constants of the input channels, then the weights.
     f32x4 *grad_coef = reinterpret_cast<f32x4 *>(lds);              // [K] (a, b, d, -)
     f32x4 *act_coef = reinterpret_cast<f32x4 *>(lds);               // [K] of the norm
     if constexpr (IN == IN_GRAD_OUT)
         act_coef = grad_coef + (size_t)a.kg * 8;
     float *weights = reinterpret_cast<float *>(lds + a.coef_bytes);  // [CT][chunk][64][4]
 
-    if constexpr (IN == IN_ACT || IN == IN_CENTRED || IN == IN_GRAD_OUT) {
-        const int K = p.src[0].K;
-        for (int k = tid; k < ((K + 7) & ~7); k += kBlock)
-            act_coef[k] = k < K ? constants_of(p.in_norm, k) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    }
-    if constexpr (reads_y(IN)) {
-        const f32x4 *coef = reinterpret_cast<const f32x4 *>(p.src[0].coef);
-        for (int k = tid; k < a.kg * 8; k += kBlock)
-            grad_coef[k] = k < p.src[0].K ? coef[k] : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    }
+    input_constants<IN>(p, a.kg, grad_coef, act_coef, tid, kBlock);
 
     // Weights of channel groups [first, first + count): element (ct, g, lane, s) belongs to
     // input channel 8 g + 2 s + (lane >> 5) and output channel 32 ct + (lane & 31).
@@ -150,20 +356,6 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
 
     // Rows of the channel groups of a step for the positions of a wave tile.
     constexpr int D = kDepth<PT>;
-    const auto load_group = [&](Rows<IN, PT> &r, int d, int b, int pos, int g) {
-        const bool second = IN == IN_RAW2 && g >= a.kg0;
-        const tk3d_mlp_source &s = p.src[second ? 1 : 0];
-        const int k0 = (g - (second ? a.kg0 : 0)) * 8 + half;
-        const float *x = s.x + (int64_t)b * s.batch_stride;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int k = k0 + 2 * q < s.K ? k0 + 2 * q : s.K - 1;
-            const unsigned offset = ((unsigned)k * (unsigned)P + (unsigned)pos) * 4u;
-            load_run<PT>(r.x[d][q], x, offset);
-            if constexpr (reads_y(IN))
-                load_run<PT>(r.y[d][q], s.y + (int64_t)b * s.batch_stride, offset);
-        }
-    };
     const auto load = [&](Rows<IN, PT> &r, int tile, int step) {
         const int b = tile / a.tiles;
         int pos = (tile - b * a.tiles) * (32 * PT) + PT * col;
@@ -171,7 +363,7 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
 #pragma unroll
         for (int d = 0; d < D; ++d)
             if (D == 1 || step * D + d < a.kg)
-                load_group(r, d, b, pos, step * D + d);
+                load_rows<IN, PT>(p, a.kg0, b, pos, half, step * D + d, r.x[d], r.y[reads_y(IN) ? d : 0]);
     };
 
     constexpr bool SHORT = short_chains(OUT) && PT * CT > 1;
@@ -203,47 +395,8 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
     };
 
     const auto multiply_group = [&](const Rows<IN, PT> &r, int d, int tile, int g, int first) {
-        const bool second = IN == IN_RAW2 && g >= a.kg0;
-        const int K = p.src[second ? 1 : 0].K, gs = g - (second ? a.kg0 : 0);
-        const int k0 = gs * 8 + half;
         float v[4][PT];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            if constexpr (reads_y(IN)) {
-                const f32x4 c = grad_coef[k0 + 2 * q];
-                f32x4 ss{0.0f, 0.0f, 0.0f, 0.0f};
-                if constexpr (IN == IN_GRAD_OUT)
-                    ss = act_coef[k0 + 2 * q];
-#pragma unroll
-                for (int t = 0; t < PT; ++t) {
-                    float e = r.x[d][q][t];
-                    const float y = r.y[reads_y(IN) ? d : 0][q][t];
-                    if constexpr (IN == IN_GRAD_OUT)
-                        e = passes(normalised(y, ss)) ? e : 0.0f;
-                    v[q][t] = __builtin_fmaf(c.x, e, __builtin_fmaf(c.y, y, c.z));
-                }
-            } else if constexpr (IN == IN_ACT || IN == IN_CENTRED) {
-                const f32x4 c = act_coef[k0 + 2 * q];
-                const float centre = IN == IN_CENTRED ? centre_of(c) : 0.0f;
-#pragma unroll
-                for (int t = 0; t < PT; ++t) {
-                    v[q][t] = relu(normalised(r.x[d][q][t], c));
-                    if constexpr (IN == IN_CENTRED)
-                        v[q][t] -= centre;
-                }
-            } else {
-#pragma unroll
-                for (int t = 0; t < PT; ++t)
-                    v[q][t] = r.x[d][q][t];
-            }
-        }
-        if (gs * 8 + 8 > K) {  // channels past the last one (their weights are zero) must not be inf
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-#pragma unroll
-                for (int t = 0; t < PT; ++t)
-                    v[q][t] = k0 + 2 * q < K ? v[q][t] : 0.0f;
-        }
+        inputs_of<IN, PT>(p, a.kg0, half, g, r.x[d], r.y[reads_y(IN) ? d : 0], grad_coef, act_coef, v);
         f32x4 w[CT];
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct)
@@ -270,27 +423,8 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
             }
     };
 
-    // Per-lane constants and sums of the output channels (lane = channel).
-    int chan[CT];
-    float shift[CT], sum1[CT], sum2[CT];
-    f32x4 out_coef[CT];
-    float sign[CT], bias[CT];
-#pragma unroll
-    for (int ct = 0; ct < CT; ++ct) {
-        chan[ct] = cbase + ct * 32 + col;
-        const int c = chan[ct] < p.C ? chan[ct] : p.C - 1;
-        sum1[ct] = sum2[ct] = shift[ct] = 0.0f;
-        if constexpr (OUT == OUT_EVAL || OUT == OUT_POOL_EVAL || OUT == OUT_MASK)
-            out_coef[ct] = constants_of(p.out_norm, c);
-        if constexpr (OUT == OUT_POOL_EVAL)
-            sign[ct] = sign_of(p.out_norm.gamma[c]);
-        if constexpr (OUT == OUT_MASK) {
-            shift[ct] = p.out_norm.mean[c];
-            bias[ct] = p.bias ? p.bias[c] : 0.0f;
-        }
-        if constexpr (OUT == OUT_PLAIN)
-            bias[ct] = p.bias ? p.bias[c] : 0.0f;
-    }
+    Results<IN, OUT, PT, CT> results;
+    results.prepare(p, cbase, col);
 
     const auto finish = [&](int tile) {
         if (D > 1)
@@ -302,119 +436,30 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
         static_assert(CHAINS == 1 || CHAINS == 4, "one chain per group of a step");
         const int b = tile / a.tiles;
         const int base = (tile - b * a.tiles) * (32 * PT);
-        const bool full = base + 32 * PT <= P;
-        const bool vec = (P & 3) == 0;
         constexpr int RUN = 4 * PT;
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) {
-            const int c = chan[ct];
-            const bool mine = c < p.C;
-            float *row = nullptr;
-            if constexpr (OUT == OUT_PLAIN || OUT == OUT_EVAL || OUT == OUT_MASK) {
-                const bool first = c < p.C0;
-                float *out = first ? p.out : p.out2;
-                const int rows = first ? p.C0 : p.C - p.C0, r = first ? c : c - p.C0;
-                row = mine && out ? out + ((int64_t)b * rows + r) * P : nullptr;
-            }
             float best = 0.0f;
             bool fresh = true;
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                const int pos = base + PT * (8 * q + 4 * half);
                 float v[RUN];
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
 #pragma unroll
                     for (int t = 0; t < PT; ++t)
                         v[i * PT + t] = SHORT ? total[SHORT ? t : 0][SHORT ? ct : 0][4 * q + i] : acc[t][ct][4 * q + i];
-                if constexpr (OUT == OUT_MASK || OUT == OUT_PLAIN) {
-#pragma unroll
-                    for (int i = 0; i < RUN; ++i)
-                        v[i] += bias[ct];
-                }
-                float before[OUT == OUT_MASK ? RUN : 1];
-                if constexpr (OUT == OUT_MASK) {
-                    const float *yrow = p.yprev + ((int64_t)b * p.C + (mine ? c : p.C - 1)) * P;
-                    if (vec) {
-#pragma unroll
-                        for (int i = 0; i < PT; ++i) {
-                            const int at = pos + 4 * i > P - 4 ? P - 4 : pos + 4 * i;
-                            const f32x4 w = *reinterpret_cast<const f32x4 *>(yrow + at);
-#pragma unroll
-                            for (int j = 0; j < 4; ++j)
-                                before[(OUT == OUT_MASK) ? 4 * i + j : 0] = w[j];
-                        }
-                    } else {
-#pragma unroll
-                        for (int i = 0; i < RUN; ++i)
-                            before[OUT == OUT_MASK ? i : 0] = yrow[pos + i > P - 1 ? P - 1 : pos + i];
-                    }
-                    if constexpr (IN == IN_CENTRED) {  // (P is a multiple of 32 here)
-                        const float *arow = p.add + ((int64_t)b * p.C + (mine ? c : p.C - 1)) * P;
-#pragma unroll
-                        for (int i = 0; i < PT; ++i) {
-                            const int at = pos + 4 * i > P - 4 ? P - 4 : pos + 4 * i;
-                            const f32x4 w = *reinterpret_cast<const f32x4 *>(arow + at);
-#pragma unroll
-                            for (int j = 0; j < 4; ++j)
-                                v[4 * i + j] += w[j];
-                        }
-                    }
-#pragma unroll
-                    for (int i = 0; i < RUN; ++i) {
-                        const float y = before[OUT == OUT_MASK ? i : 0];
-                        v[i] = passes(normalised(y, out_coef[ct])) ? v[i] : 0.0f;
-                    }
-                }
-                if constexpr (OUT == OUT_MASK) {
-#pragma unroll
-                    for (int i = 0; i < RUN; ++i) {
-                        if (full || pos + i < P) {
-                            sum1[ct] += v[i];
-                            sum2[ct] = __builtin_fmaf(v[i], before[OUT == OUT_MASK ? i : 0] - shift[ct], sum2[ct]);
-                        }
-                    }
-                }
-                if constexpr (OUT == OUT_EVAL) {
-#pragma unroll
-                    for (int i = 0; i < RUN; ++i)
-                        v[i] = relu(normalised(v[i], out_coef[ct]));
-                }
-                if constexpr (OUT == OUT_PLAIN || OUT == OUT_EVAL || OUT == OUT_MASK) {
-                    if (row) {
-                        if (vec) {
-#pragma unroll
-                            for (int i = 0; i < PT; ++i)
-                                if (full || pos + 4 * i < P)
-                                    *reinterpret_cast<f32x4 *>(row + pos + 4 * i) =
-                                        f32x4{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
-                        } else {
-#pragma unroll
-                            for (int i = 0; i < RUN; ++i)
-                                if (pos + i < P)
-                                    row[pos + i] = v[i];
-                        }
-                    }
-                } else if constexpr (OUT == OUT_POINTS) {
-#pragma unroll
-                    for (int i = 0; i < RUN; ++i)
-                        if (mine && pos + i < P)
-                            p.out[((int64_t)b * P + pos + i) * p.C + c] = v[i];
+                const int pos = base + PT * (8 * q + 4 * half);
+                if constexpr (OUT != OUT_POOL_EVAL) {
+                    results.put(p, b, ct, pos, base + 32 * PT <= P, v);
                 } else {
                     // A group is both halves of one q or of several.
-#pragma unroll
-                    for (int i = 0; i < RUN; ++i) {
-                        const float s = v[i] * sign[ct];
-                        best = fresh ? s : __builtin_elementwise_maximum(best, s);
-                        fresh = false;
-                    }
+                    const float s = results.extreme(ct, v);
+                    best = fresh ? s : __builtin_elementwise_maximum(best, s);
+                    fresh = false;
                     const int qs = p.group / (2 * RUN);
                     if (((q + 1) & (qs - 1)) == 0) {
-                        best = __builtin_elementwise_maximum(best, __shfl_xor(best, 32));
-                        const int m = pos / p.group;
-                        if (mine && half == 0 && pos < P)
-                            p.out[((int64_t)b * p.C + c) * p.M + m] = relu(
-                                normalised(sign[ct] == 0.0f ? best : best * sign[ct], out_coef[ct]));
+                        results.put_extreme(p, b, ct, pos, half, best);
                         fresh = true;
                     }
                 }
@@ -478,7 +523,7 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
         double2 *part = reinterpret_cast<double2 *>(lds);  // [kWaves][32 CT]
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) {
-            double s1 = sum1[ct], s2 = sum2[ct];
+            double s1 = results.sum1[ct], s2 = results.sum2[ct];
             s1 += __shfl_xor(s1, 32);
             s2 += __shfl_xor(s2, 32);
             if (half == 0)
@@ -488,6 +533,216 @@ __global__ void __launch_bounds__(kBlock, 2) mlp_product_kernel(GemmArgs a)
         if (tid < 32 * CT && cbase + tid < p.C) {
             double2 s = part[tid];
             for (int w = 1; w < kWaves; ++w) {
+                s.x += part[w * (32 * CT) + tid].x;
+                s.y += part[w * (32 * CT) + tid].y;
+            }
+            reinterpret_cast<double2 *>(p.partial)[(int64_t)(cbase + tid) * a.slots + blockIdx.x] = s;
+        }
+    }
+}
+
+// The same for products too small to fill the chip with wave tiles of their own, or whose weights don't
+// stay in LDS: the waves of a workgroup share a tile and take every NW-th group of input channels, their
+// sums meet in LDS, and each wave finishes a part of the tile. Nothing is staged: rows and weights come
+// straight into registers, DEPTH groups of them ahead of the one that is multiplied, so a wave waits for
+// memory every DEPTH groups and not at two barriers per chunk of weights (1024 -> 512 channels, 2048
+// positions: 90 -> 44 us, 9 TB/s from L2, which bounds it; 14 us of matrix instructions). The sums of the
+// 32 x 32 tiles are those of the four chains of mlp_product_kernel, bit by bit.
+template <int IN, int OUT, int PT, int CT>
+__global__ void __launch_bounds__(kBlock) mlp_split_kernel(GemmArgs a)
+{
+    extern __shared__ char lds[];
+    constexpr int NW = kWaves;
+    constexpr int DEPTH = PT * CT == 1 ? 4 : 2;
+    const tk3d_mlp_product &p = a.p;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int half = lane >> 5, col = lane & 31;
+    const int cbase = blockIdx.y * (32 * CT);
+    const int tile = blockIdx.x, b = tile / a.tiles, base = (tile - b * a.tiles) * (32 * PT);
+    const int P = p.P;
+    int pos = base + PT * col;
+    pos = pos > P - PT ? P - PT : pos;  // (results of the surplus are dropped)
+
+    f32x4 *grad_coef = reinterpret_cast<f32x4 *>(lds);
+    f32x4 *act_coef = reinterpret_cast<f32x4 *>(lds);
+    if constexpr (IN == IN_GRAD_OUT)
+        act_coef = grad_coef + (size_t)a.kg * 8;
+
+    struct Group {  // input channels 2 q + half of a group: a lane's positions, its channels' weights
+        float x[4][PT], y[4][PT], w[CT][4];
+    };
+    const auto load = [&](Group &r, int g) {
+        const bool second = IN == IN_RAW2 && g >= a.kg0;
+        const tk3d_mlp_source &s = p.src[second ? 1 : 0];
+        const int k0 = (g - (second ? a.kg0 : 0)) * 8;
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) {
+            const int cc = cbase + ct * 32 + col;
+            const float *w = s.w + (int64_t)(cc < p.C ? cc : p.C - 1) * s.wc;
+            if (a.rows4) {  // (half a run of eight, put right by exchange() below)
+                const f32x4 v = *reinterpret_cast<const f32x4 *>(w + k0 + 4 * half);
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    r.w[ct][q] = v[q];
+            } else {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int k = k0 + 2 * q + half;
+                    r.w[ct][q] = w[(int64_t)(k < s.K ? k : s.K - 1) * s.wk];
+                }
+            }
+        }
+        load_rows<IN, PT>(p, a.kg0, b, pos, half, g, r.x, r.y);
+    };
+
+    constexpr bool SHORT = short_chains(OUT) && PT * CT > 1;
+    tk_f32x16 acc[PT][CT], total[SHORT ? PT : 1][SHORT ? CT : 1];
+#pragma unroll
+    for (int t = 0; t < PT; ++t)
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                acc[t][ct][r] = 0.0f;
+                if constexpr (SHORT)
+                    total[t][ct][r] = 0.0f;
+            }
+    const auto multiply = [&](Group &r, int g) {
+        float v[4][PT];
+        inputs_of<IN, PT>(p, a.kg0, half, g, r.x, r.y, grad_coef, act_coef, v);
+        const bool two = IN == IN_RAW2 && g >= a.kg0;
+        const int left = p.src[two ? 1 : 0].K - (g - (two ? a.kg0 : 0)) * 8;
+        if (left < 8)  // (inputs past the last channel are zero)
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    r.w[ct][q] = 2 * q + half < left ? r.w[ct][q] : 0.0f;
+        if (a.rows4) {
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                for (int j = 0; j < 4; j += 2) {
+                    // (k, k + 4) and (k + 1, k + 5) by halves -> (k, k + 1) and (k + 4, k + 5)
+                    const auto e = __builtin_amdgcn_permlane32_swap(__float_as_uint(r.w[ct][j]),
+                                                                    __float_as_uint(r.w[ct][j + 1]), false, false);
+                    r.w[ct][j] = __uint_as_float(e[0]);
+                    r.w[ct][j + 1] = __uint_as_float(e[1]);
+                }
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) {
+                const float second = r.w[ct][1];
+                r.w[ct][1] = r.w[ct][2];
+                r.w[ct][2] = second;
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                for (int t = 0; t < PT; ++t)
+                    acc[t][ct] = __builtin_amdgcn_mfma_f32_32x32x2f32(v[q][t], r.w[ct][q], acc[t][ct], 0, 0, 0);
+        if constexpr (SHORT)
+#pragma unroll
+            for (int t = 0; t < PT; ++t)
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) {
+                        total[t][ct][i] += acc[t][ct][i];
+                        acc[t][ct][i] = 0.0f;
+                    }
+    };
+    Group ring[DEPTH];
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d)
+        if (wave + d * NW < a.kg)
+            load(ring[d], wave + d * NW);
+    Results<IN, OUT, PT, CT> results;
+    results.prepare(p, cbase, col);
+    input_constants<IN>(p, a.kg, grad_coef, act_coef, tid, kBlock);
+    __syncthreads();
+    for (int g0 = wave; g0 < a.kg; g0 += DEPTH * NW) {
+#pragma unroll
+        for (int d = 0; d < DEPTH; ++d) {
+            const int g = g0 + d * NW;
+            if (g < a.kg) {
+                multiply(ring[d], g);
+                if (g + DEPTH * NW < a.kg)
+                    load(ring[d], g + DEPTH * NW);
+            }
+        }
+    }
+
+    // [wave][q][ct][t][lane] runs of four positions; wave q finishes the runs q of all
+    __syncthreads();
+    f32x4 *sums = reinterpret_cast<f32x4 *>(lds);
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+            for (int t = 0; t < PT; ++t) {
+                const tk_f32x16 &v = SHORT ? total[SHORT ? t : 0][SHORT ? ct : 0] : acc[t][ct];
+                sums[((wave * 4 + q) * CT * PT + ct * PT + t) * 64 + lane] =
+                    f32x4{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
+            }
+    __syncthreads();
+    static_assert(NW == 4, "a wave per run of a tile");
+    constexpr int RUN = 4 * PT;
+    float extreme[CT];
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+        float v[RUN];
+#pragma unroll
+        for (int t = 0; t < PT; ++t) {
+            f32x4 part[NW];
+#pragma unroll
+            for (int w = 0; w < NW; ++w)
+                part[w] = sums[((w * 4 + wave) * CT * PT + ct * PT + t) * 64 + lane];
+            const f32x4 sum = (part[0] + part[1]) + (part[2] + part[3]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                v[i * PT + t] = sum[i];
+        }
+        if constexpr (OUT == OUT_POOL_EVAL)
+            extreme[ct] = results.extreme(ct, v);
+        else
+            results.put(p, b, ct, base + PT * (8 * wave + 4 * half), base + 32 * PT <= P, v);
+    }
+    if constexpr (OUT == OUT_POOL_EVAL) {  // (a group is a tile's positions)
+        __syncthreads();
+        float *best = reinterpret_cast<float *>(lds);  // [wave][CT][64]
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct)
+            best[(wave * CT + ct) * 64 + lane] = extreme[ct];
+        __syncthreads();
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct)
+            if (wave == ct) {
+                float m = best[ct * 64 + lane];
+#pragma unroll
+                for (int q = 1; q < 4; ++q)
+                    m = __builtin_elementwise_maximum(m, best[(q * CT + ct) * 64 + lane]);
+                results.put_extreme(p, b, ct, base, half, m);
+            }
+    }
+    if constexpr (OUT == OUT_MASK) {
+        __syncthreads();
+        double2 *part = reinterpret_cast<double2 *>(lds);  // [NW][32 CT]
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) {
+            double s1 = results.sum1[ct], s2 = results.sum2[ct];
+            s1 += __shfl_xor(s1, 32);
+            s2 += __shfl_xor(s2, 32);
+            if (half == 0)
+                part[wave * (32 * CT) + ct * 32 + col] = double2{s1, s2};
+        }
+        __syncthreads();
+        if (tid < 32 * CT && cbase + tid < p.C) {
+            double2 s = part[tid];
+            for (int w = 1; w < NW; ++w) {
                 s.x += part[w * (32 * CT) + tid].x;
                 s.y += part[w * (32 * CT) + tid].y;
             }
@@ -1281,6 +1536,33 @@ Shape pick_shape(int out, const tk3d_mlp_product &p)
     return {1, 1};
 }
 
+// The tile of mlp_split_kernel for a product, or {0, 0} where mlp_product_kernel is faster (times of that
+// kernel -> split, us):
+// - 32 x 32 instead of wave tiles of that size, up to one per SIMD or on 128 channels and more: 512 -> 1024
+//   channels, 128 positions 27 -> 8; 1024 -> 512, 16 x 128 masked 90 -> 44; 64 -> 64, 16384 positions 8.1 ->
+//   6.5; 256 -> 128, 8 x 2048 31 -> 26. (Two per SIMD on few channels: 6 -> 128, 8 x 2048 8.2 against 9.0.)
+// - 64 x 64 for gradients of 128 channels and more on up to two waves a SIMD: 512 -> 256, 8 x 2048 92 -> 76,
+//   1024 -> 320 227 -> 180; twice the positions 129 against 144. Evaluation of these sizes has short chains
+//   of the same length either way, and stays.
+// - 64 positions for groups of 64 that leave SIMDs idle: 64 -> 128, 2048 positions 12 -> 4.8; 128 -> 256, 8192
+//   positions 20 -> 11.6.
+Shape pick_split(int out, const tk3d_mlp_product &p, bool two)
+{
+    const int simds = 4 * tk_cu_count();
+    const auto waves = [&](int pt, int ct) {
+        return (int64_t)p.B * ((p.P + 32 * pt - 1) / (32 * pt)) * ((p.C + 32 * ct - 1) / (32 * ct));
+    };
+    const bool deep = (two ? p.src[0].K + p.src[1].K : p.src[0].K) > 120;
+    const Shape s = pick_shape(out, p);
+    if (s.pt == 1)
+        return waves(1, 1) <= simds || (deep && waves(1, 1) <= 4 * simds) ? Shape{1, 1} : Shape{0, 0};
+    if (s.pt != 2)
+        return {0, 0};
+    if (out == TK3D_MLP_OUT_POOL_EVAL && p.group == 64 && waves(2, 2) < simds)
+        return waves(2, 2) <= simds / 4 ? Shape{2, 1} : Shape{2, 2};
+    return deep && !short_chains_of(out) && waves(4, 2) < simds ? Shape{2, 2} : Shape{0, 0};
+}
+
 int fill(const tk3d_mlp_product &p, int in, int out, Shape s, GemmArgs &g)
 {
     g.p = p;
@@ -1299,6 +1581,11 @@ int fill(const tk3d_mlp_product &p, int in, int out, Shape s, GemmArgs &g)
     // (a multiple of the XCDs, so that the channel blocks of a position share an L2)
     most = (most + 7) & ~7;
     g.slots = wgs < most ? wgs : most;
+    g.rows4 = 1;
+    for (int i = 0; i < (two ? 2 : 1); ++i)
+        if (p.src[i].wk != 1 || p.src[i].K % 8 != 0 || p.src[i].wc % 4 != 0 ||
+            (reinterpret_cast<uintptr_t>(p.src[i].w) & 15) != 0)
+            g.rows4 = 0;
     return cblocks;
 }
 
@@ -1328,6 +1615,32 @@ int launch_shape(const GemmArgs &g, Shape s, int cblocks, hipStream_t stream)
     if (s.pt == 2)
         return launch_product<IN, OUT, 2, 2>(g, cblocks, stream);
     return launch_product<IN, OUT, 1, 1>(g, cblocks, stream);
+}
+
+template <int IN, int OUT, int PT, int CT>
+int launch_split(const GemmArgs &g, int cblocks, hipStream_t stream)
+{
+    const int sum_bytes = kWaves * 4 * CT * PT * 1024;
+    const int bytes = sum_bytes > g.coef_bytes ? sum_bytes : g.coef_bytes;
+    if (bytes > 150 << 10)
+        return TK3D_ERR_UNSUPPORTED;
+    const int rc = tk_allow_dynamic_lds<mlp_split_kernel<IN, OUT, PT, CT>>(150 << 10);
+    if (rc != TK3D_OK)
+        return rc;
+    mlp_split_kernel<IN, OUT, PT, CT><<<dim3(g.total, cblocks), kBlock, bytes, stream>>>(g);
+    return tk_launch_status();
+}
+
+template <int IN, int OUT>
+int launch_split_shape(const GemmArgs &g, Shape s, int cblocks, hipStream_t stream)
+{
+    if constexpr (OUT == OUT_POOL_EVAL)
+        if (s.pt == 2 && s.ct == 1)
+            return launch_split<IN, OUT, 2, 1>(g, cblocks, stream);
+    if constexpr (OUT == OUT_POOL_EVAL || !short_chains(OUT))
+        if (s.pt == 2)
+            return launch_split<IN, OUT, 2, 2>(g, cblocks, stream);
+    return launch_split<IN, OUT, 1, 1>(g, cblocks, stream);
 }
 
 template <int ROW, int COL, int TA, int TB>
@@ -1373,8 +1686,9 @@ extern "C" {
 int tk3d_mlp_product_slots(int in, int out, const tk3d_mlp_product *p)
 {
     GemmArgs g;
-    fill(*p, in, out, pick_shape(out, *p), g);
-    return g.slots;
+    const Shape split = pick_split(out, *p, in == TK3D_MLP_IN_RAW2);
+    fill(*p, in, out, split.pt ? split : pick_shape(out, *p), g);
+    return split.pt ? g.total : g.slots;
 }
 
 int tk3d_mlp_product_f32(int in, int out, const tk3d_mlp_product *p, void *stream_)
@@ -1393,13 +1707,17 @@ int tk3d_mlp_product_f32(int in, int out, const tk3d_mlp_product *p, void *strea
         return TK3D_ERR_UNSUPPORTED;
     if (in == TK3D_MLP_IN_CENTRED && out == TK3D_MLP_OUT_MASK && (!p->add || p->P % 32 != 0))
         return TK3D_ERR_BAD_SIZE;
-    const Shape s = pick_shape(out, *p);
+    const Shape split = pick_split(out, *p, two);
+    const Shape s = split.pt ? split : pick_shape(out, *p);
     GemmArgs g;
     const int cblocks = fill(*p, in, out, s, g);
+    if (split.pt)
+        g.slots = g.total;
     const hipStream_t stream = (hipStream_t)stream_;
 #define TK_CASE(IN, OUT)                                                                        \
     if (in == TK3D_MLP_##IN && out == TK3D_MLP_##OUT)                                           \
-        return launch_shape<IN, OUT>(g, s, cblocks, stream);
+        return split.pt ? launch_split_shape<IN, OUT>(g, split, cblocks, stream)                \
+                        : launch_shape<IN, OUT>(g, s, cblocks, stream);
     TK_CASE(IN_RAW, OUT_EVAL)
     TK_CASE(IN_RAW, OUT_PLAIN)
     TK_CASE(IN_RAW, OUT_POINTS)
