@@ -1,5 +1,5 @@
 /*
- * tk3d_mlp.h - C ABI of the shared-MLP kernels (torkit3d_amd/csrc/mlp.hip): the pieces of
+ * tk3d_mlp.h - C ABI of the shared-MLP kernels (torkit3d_amd/csrc/mlp*.hip): the pieces of
  * "1x1 convolution, batch norm, ReLU" chains on [B, C, P] fp32 tensors, forward and backward,
  * that the reference runs as stock torch modules (torkit3d/nn/modules/mlp.py,
  * torkit3d/nn/modules/conv.py) on the tensors its ops produce (torkit3d/layers/pointnet2.py,
@@ -102,6 +102,14 @@ typedef struct {
 } tk3d_mlp_outer;
 int tk3d_mlp_outer_splits(const tk3d_mlp_outer *p);
 int tk3d_mlp_outer_f32(int row, int col, const tk3d_mlp_outer *p, void *stream);
+
+/* Both of a layer in one launch, where they read the same: the product IN_GRAD, IN_GRAD_OUT (weights
+ * K = R output channels to C input channels) or IN_CENTRED (K = R = C) to OUT_MASK, and the weight gradient
+ * with rows of the same kind and the product's yprev as COL_ACT (COL_CENTRED behind IN_CENTRED); or one to
+ * OUT_PLAIN (C0 = C), columns COL_RAW. tk3d_mlp_pair_slots: slots and splits of the partial sums, 0 where the two
+ * have to be called apart (more than 128 channels, 128 from 32, rows that are not 16-byte aligned). */
+int tk3d_mlp_pair_slots(int in, const tk3d_mlp_product *p, const tk3d_mlp_outer *o);
+int tk3d_mlp_pair_f32(int in, int out, const tk3d_mlp_product *p, const tk3d_mlp_outer *o, void *stream);
 
 /* out[r * ld + c] = sum over the splits of partial[r][c], rows of C, `stride` elements from one split
  * to the next; n of them in one launch. */

@@ -107,6 +107,23 @@ def test_maximum_over_neighbours(cuda, monkeypatch, b, m, s, widths, training):
           [(randn(m, b, widths[0], m, s), True)], monkeypatch)
 
 
+# Input and weight gradient of a layer in one launch: every shape in tiles of 32 channels on either side (the
+# widths' neighbours), widths and positions off the tiles, one tile in all, a few tiles a workgroup and many.
+@pytest.mark.parametrize("b,p", [(2, 4), (3, 36), (2, 1000), (5, 20004)])
+@pytest.mark.parametrize("widths", [(64, 128, 128, 64, 64, 32, 32), (100, 30, 128, 40, 128), (33, 65, 33, 20, 64)])
+def test_both_gradients_of_a_layer(cuda, monkeypatch, b, p, widths):
+    mlp = make(mlp1d_bn_relu, widths[0], widths[1:], True, cuda)
+    check(mlp, lambda m, x: m(x), lambda m, x: m(x), [(randn(p, b, widths[0], p), True)], monkeypatch)
+
+
+@pytest.mark.parametrize("b,m,s,widths", [(1, 3, 32, (64, 128, 128)), (4, 1025, 32, (70, 100, 64, 40)),
+                                          (3, 700, 64, (128, 128, 32, 128))])
+def test_both_gradients_under_a_maximum(cuda, monkeypatch, b, m, s, widths):
+    mlp = make(mlp2d_bn_relu, widths[0], widths[1:], True, cuda)
+    check(mlp, lambda n, x: n.forward_max(x), lambda n, x: n(x).max(dim=3)[0],
+          [(randn(m, b, widths[0], m, s), True)], monkeypatch)
+
+
 # Products whose waves share a tile: gradients in tiles of 64 x 64 with remainders of both, groups of 32 and
 # of 64 in evaluation (one channel tile and two), channels that leave waves without a group of eight.
 @pytest.mark.parametrize("b,p,widths,pool,training", [

@@ -336,16 +336,47 @@ struct Pending {
     std::vector<Tensor> alive;
 };
 
+void pending_sum(const Tensor &partial, const tk3d_mlp_outer &o, float *out, int64_t ld, Pending &pending)
+{
+    pending.sums.push_back({f32(partial), out, (int64_t)o.row.K * o.col.K, (int32_t)partial.size(0),
+                            o.row.K, o.col.K, (int32_t)ld});
+    pending.alive.push_back(partial);
+}
+
 void outer(int row, int col, tk3d_mlp_outer &o, const Tensor &like, float *out, int64_t ld,
            Pending &pending, void *stream)
 {
-    const int splits = tk3d_mlp_outer_splits(&o);
-    const Tensor partial = at::empty({splits, o.row.K, o.col.K}, like.options());
+    const Tensor partial = at::empty({tk3d_mlp_outer_splits(&o), o.row.K, o.col.K}, like.options());
     o.partial = f32(partial);
     done(tk3d_mlp_outer_f32(row, col, &o, stream), "tk3d_mlp_outer_f32");
-    pending.sums.push_back({f32(partial), out, (int64_t)o.row.K * o.col.K, splits, o.row.K,
-                            o.col.K, (int32_t)ld});
-    pending.alive.push_back(partial);
+    pending_sum(partial, o, out, ld, pending);
+}
+
+// A layer's product and its weight gradient in one launch, where there is one for its size. Returns the
+// partial sums of a masked product and their slots, and leaves those of the weight gradient (and of the rows)
+// in o; 0 slots: nothing was launched.
+struct Paired {
+    int slots = 0;
+    Tensor sums, outer, rows;
+};
+Paired pair(int in, int out, tk3d_mlp_product &p, tk3d_mlp_outer &o, const Tensor &like, void *stream)
+{
+    Paired r;
+    r.slots = tk3d_mlp_pair_slots(in, &p, &o);
+    if (r.slots == 0)
+        return r;
+    r.outer = at::empty({r.slots, o.row.K, o.col.K}, like.options());
+    o.partial = f32(r.outer);
+    if (out == TK3D_MLP_OUT_MASK) {
+        r.sums = partial_sums(like, p.C, r.slots);
+        p.partial = r.sums.data_ptr();
+    }
+    if (in == TK3D_MLP_IN_CENTRED) {
+        r.rows = at::empty({r.slots, o.row.K}, like.options());
+        o.rowsum = f32(r.rows);
+    }
+    done(tk3d_mlp_pair_f32(in, out, &p, &o, stream), "tk3d_mlp_pair_f32");
+    return r;
 }
 
 Grads backward(const Call &c, const Kept &k, const Tensor &g, bool want_x, bool want_x2)
@@ -400,8 +431,6 @@ Grads backward(const Call &c, const Kept &k, const Tensor &g, bool want_x, bool 
         p.yprev = f32(k.y[l - 1]);
         p.bias = f32(gram) + I * I;
         p.add = p.out = f32(e);
-        const auto sums = summed_product(TK3D_MLP_IN_CENTRED, TK3D_MLP_OUT_MASK, p, like, stream);
-
         const int sparse_splits = tk3d_mlp_pool_outer_splits((int)B, (int)O, (int)I, (int)M);
         const Tensor sparse = at::empty({sparse_splits, O, I}, like.options());
         done(tk3d_mlp_pool_outer_f32(sel.data_ptr(), f32(k.y[l - 1]), &inner, (int)B, (int)O, (int)I,
@@ -413,19 +442,24 @@ Grads backward(const Call &c, const Kept &k, const Tensor &g, bool want_x, bool 
         o.col = source(k.y[l - 1], nullptr, 0, 0);
         o.col_norm = o.row_norm = inner;
         o.row = o.col;
-        const int splits = tk3d_mlp_outer_splits(&o);
-        const Tensor xx = at::empty({splits, I, I}, like.options());
-        const Tensor xsum = at::empty({splits, I}, like.options());
-        o.partial = f32(xx);
-        o.rowsum = f32(xsum);
-        done(tk3d_mlp_outer_f32(TK3D_MLP_ROW_CENTRED, TK3D_MLP_COL_CENTRED, &o, stream),
-             "tk3d_mlp_outer_f32");
+        Paired both = pair(TK3D_MLP_IN_CENTRED, TK3D_MLP_OUT_MASK, p, o, like, stream);
+        if (both.slots == 0) {
+            std::tie(both.sums, both.slots) =
+                summed_product(TK3D_MLP_IN_CENTRED, TK3D_MLP_OUT_MASK, p, like, stream);
+            const int splits = tk3d_mlp_outer_splits(&o);
+            both.outer = at::empty({splits, I, I}, like.options());
+            both.rows = at::empty({splits, I}, like.options());
+            o.partial = f32(both.outer);
+            o.rowsum = f32(both.rows);
+            done(tk3d_mlp_outer_f32(TK3D_MLP_ROW_CENTRED, TK3D_MLP_COL_CENTRED, &o, stream),
+                 "tk3d_mlp_outer_f32");
+        }
         const Tensor scratch = at::empty({I + 1, I}, like.options());
-        done(tk3d_mlp_pool_weight_grad_f32(f32(sparse), sparse_splits, f32(xx), f32(xsum), splits, w,
-                                           f32(coef[l]), (int)O, (int)I, f32(scratch),
-                                           f32(out.params[3 * l]), stream),
+        done(tk3d_mlp_pool_weight_grad_f32(f32(sparse), sparse_splits, f32(both.outer), f32(both.rows),
+                                           (int)both.outer.size(0), w, f32(coef[l]), (int)O, (int)I,
+                                           f32(scratch), f32(out.params[3 * l]), stream),
              "tk3d_mlp_pool_weight_grad_f32");
-        coefficients(l - 1, sums.first.data_ptr(), sums.second);
+        coefficients(l - 1, both.sums.data_ptr(), both.slots);
         masked = true;
         --l;
     } else {
@@ -463,14 +497,19 @@ Grads backward(const Call &c, const Kept &k, const Tensor &g, bool want_x, bool 
         if (l > 0) {
             o.col = source(k.y[l - 1], nullptr, 0, 0);
             o.col_norm = norm_of(c, k, l - 1);
-            outer(row, TK3D_MLP_COL_ACT, o, like, dw, I, pending, stream);
             tk3d_mlp_product p = gradient_product(I);
             p.out_norm = o.col_norm;
             p.yprev = f32(k.y[l - 1]);
             const Tensor before = at::empty({B, I, P}, like.options());
             p.out = f32(before);
-            const auto sums = summed_product(in, TK3D_MLP_OUT_MASK, p, like, stream);
-            coefficients(l - 1, sums.first.data_ptr(), sums.second);
+            Paired both = pair(in, TK3D_MLP_OUT_MASK, p, o, like, stream);
+            if (both.slots) {
+                pending_sum(both.outer, o, dw, I, pending);
+            } else {
+                outer(row, TK3D_MLP_COL_ACT, o, like, dw, I, pending, stream);
+                std::tie(both.sums, both.slots) = summed_product(in, TK3D_MLP_OUT_MASK, p, like, stream);
+            }
+            coefficients(l - 1, both.sums.data_ptr(), both.slots);
             e = before;
             masked = true;
             continue;
@@ -478,16 +517,25 @@ Grads backward(const Call &c, const Kept &k, const Tensor &g, bool want_x, bool 
         if (!c.grouped()) {
             const int64_t C1 = c.x.size(1);
             o.col = source(c.x, nullptr, 0, 0);
-            outer(row, TK3D_MLP_COL_RAW, o, like, dw, I, pending, stream);
+            if (want_x)
+                out.x = at::empty(c.x.sizes(), like.options());
+            Paired both;
+            if (want_x && !want_x2) {
+                tk3d_mlp_product p = gradient_product(C1);
+                p.out = f32(out.x);
+                both = pair(in, TK3D_MLP_OUT_PLAIN, p, o, like, stream);
+            }
+            if (both.slots)
+                pending_sum(both.outer, o, dw, I, pending);
+            else
+                outer(row, TK3D_MLP_COL_RAW, o, like, dw, I, pending, stream);
             if (c.x2.defined()) {
                 o.col = source(c.x2, nullptr, 0, 0);
                 outer(row, TK3D_MLP_COL_RAW, o, like, dw + C1, I, pending, stream);
             }
-            if (want_x || want_x2) {
+            if ((want_x || want_x2) && !both.slots) {
                 tk3d_mlp_product p = gradient_product(I);
                 p.C0 = (int32_t)C1;
-                if (want_x)
-                    out.x = at::empty(c.x.sizes(), like.options());
                 if (want_x2)
                     out.x2 = at::empty(c.x2.sizes(), like.options());
                 p.out = f32(out.x);
