@@ -124,7 +124,29 @@ def test_both_gradients_under_a_maximum(cuda, monkeypatch, b, m, s, widths):
           [(randn(m, b, widths[0], m, s), True)], monkeypatch)
 
 
-# Products whose waves share a tile: gradients in tiles of 64 x 64 with remainders of both, groups of 32 and
+# Layers too wide for that, in tiles in LDS: three, four and five tiles of channels a workgroup with remainders
+# of all of them, of 128 positions and of 32 input channels; rows in parts of a block of 128; two inputs.
+@pytest.mark.parametrize("b,p,widths", [(6, 4100, (330, 160, 384, 260, 140)), (200, 36, (129, 70, 300)),
+                                        (1, 24580, (65, 129, 512, 66))])
+def test_wide_layers(cuda, monkeypatch, b, p, widths):
+    mlp = make(mlp1d_bn_relu, widths[0], widths[1:], True, cuda)
+    check(mlp, lambda m, x: m(x), lambda m, x: m(x), [(randn(p, b, widths[0], p), True)], monkeypatch)
+
+
+def test_wide_layers_of_two_inputs(cuda, monkeypatch):
+    mlp = make(mlp1d_bn_relu, 100 + 35, (140,), True, cuda)
+    check(mlp, lambda m, x, y: m.forward_cat(x, y), lambda m, x, y: m(torch.cat([x, y], 1)),
+          [(randn(1, 4, 100, 8200), True), (randn(2, 4, 35, 8200), True)], monkeypatch)
+
+
+@pytest.mark.parametrize("b,m,s,widths", [(4, 225, 32, (20, 200, 300)), (3, 150, 64, (9, 256, 96))])
+def test_wide_layers_under_a_maximum(cuda, monkeypatch, b, m, s, widths):
+    mlp = make(mlp2d_bn_relu, widths[0], widths[1:], True, cuda)
+    check(mlp, lambda n, x: n.forward_max(x), lambda n, x: n(x).max(dim=3)[0],
+          [(randn(m, b, widths[0], m, s), True)], monkeypatch)
+
+
+# Products whose waves share a tile: groups of 32 and
 # of 64 in evaluation (one channel tile and two), channels that leave waves without a group of eight.
 @pytest.mark.parametrize("b,p,widths,pool,training", [
     (4, 4100, (260, 256, 140), 0, True), (2, 8252, (131, 192, 128), 0, True), (3, 130, (20, 9, 200), 0, True),

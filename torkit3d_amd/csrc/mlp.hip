@@ -9,6 +9,7 @@
 // (up to 64 channels) are bound by HBM, wide ones by the fp32 matrix rate (157 TFLOP/s), which is
 // why the products are fp32 v_mfma_f32_32x32x2 and nothing is rounded to a shorter type.
 #include "mlp_common.h"
+#include "mlp_wide.h"
 
 namespace {
 
@@ -1541,9 +1542,6 @@ Shape pick_shape(int out, const tk3d_mlp_product &p)
 // - 32 x 32 instead of wave tiles of that size, up to one per SIMD or on 128 channels and more: 512 -> 1024
 //   channels, 128 positions 27 -> 8; 1024 -> 512, 16 x 128 masked 90 -> 44; 64 -> 64, 16384 positions 8.1 ->
 //   6.5; 256 -> 128, 8 x 2048 31 -> 26. (Two per SIMD on few channels: 6 -> 128, 8 x 2048 8.2 against 9.0.)
-// - 64 x 64 for gradients of 128 channels and more on up to two waves a SIMD: 512 -> 256, 8 x 2048 92 -> 76,
-//   1024 -> 320 227 -> 180; twice the positions 129 against 144. Evaluation of these sizes has short chains
-//   of the same length either way, and stays.
 // - 64 positions for groups of 64 that leave SIMDs idle: 64 -> 128, 2048 positions 12 -> 4.8; 128 -> 256, 8192
 //   positions 20 -> 11.6.
 Shape pick_split(int out, const tk3d_mlp_product &p, bool two)
@@ -1560,7 +1558,7 @@ Shape pick_split(int out, const tk3d_mlp_product &p, bool two)
         return {0, 0};
     if (out == TK3D_MLP_OUT_POOL_EVAL && p.group == 64 && waves(2, 2) < simds)
         return waves(2, 2) <= simds / 4 ? Shape{2, 1} : Shape{2, 2};
-    return deep && !short_chains_of(out) && waves(4, 2) < simds ? Shape{2, 2} : Shape{0, 0};
+    return {0, 0};
 }
 
 int fill(const tk3d_mlp_product &p, int in, int out, Shape s, GemmArgs &g)
@@ -1637,7 +1635,7 @@ int launch_split_shape(const GemmArgs &g, Shape s, int cblocks, hipStream_t stre
     if constexpr (OUT == OUT_POOL_EVAL)
         if (s.pt == 2 && s.ct == 1)
             return launch_split<IN, OUT, 2, 1>(g, cblocks, stream);
-    if constexpr (OUT == OUT_POOL_EVAL || !short_chains(OUT))
+    if constexpr (OUT == OUT_POOL_EVAL)
         if (s.pt == 2)
             return launch_split<IN, OUT, 2, 2>(g, cblocks, stream);
     return launch_split<IN, OUT, 1, 1>(g, cblocks, stream);
@@ -1685,6 +1683,8 @@ extern "C" {
 
 int tk3d_mlp_product_slots(int in, int out, const tk3d_mlp_product *p)
 {
+    if (const int wide = tk_mlp_wide_product_slots(in, out, *p))
+        return wide;
     GemmArgs g;
     const Shape split = pick_split(out, *p, in == TK3D_MLP_IN_RAW2);
     fill(*p, in, out, split.pt ? split : pick_shape(out, *p), g);
@@ -1707,6 +1707,8 @@ int tk3d_mlp_product_f32(int in, int out, const tk3d_mlp_product *p, void *strea
         return TK3D_ERR_UNSUPPORTED;
     if (in == TK3D_MLP_IN_CENTRED && out == TK3D_MLP_OUT_MASK && (!p->add || p->P % 32 != 0))
         return TK3D_ERR_BAD_SIZE;
+    if (tk_mlp_wide_product_slots(in, out, *p))
+        return tk_mlp_wide_product(in, out, *p, (hipStream_t)stream_);
     const Shape split = pick_split(out, *p, two);
     const Shape s = split.pt ? split : pick_shape(out, *p);
     GemmArgs g;
@@ -1736,6 +1738,8 @@ int tk3d_mlp_product_f32(int in, int out, const tk3d_mlp_product *p, void *strea
 
 int tk3d_mlp_outer_splits(const tk3d_mlp_outer *p)
 {
+    if (const int wide = tk_mlp_wide_outer_splits(*p))
+        return wide;
     const int ta = p->row.K > 32 ? 2 : 1, tb = p->col.K > 32 ? 2 : 1;
     const int blocks = ((p->row.K + 32 * ta - 1) / (32 * ta)) * ((p->col.K + 32 * tb - 1) / (32 * tb));
     const int64_t units = (int64_t)p->B * ((p->P + 31) / 32);
@@ -1754,6 +1758,8 @@ int tk3d_mlp_outer_f32(int row, int col, const tk3d_mlp_outer *p, void *stream_)
         return TK3D_ERR_BAD_SIZE;
     if (!indexable(p->row.K, p->P) || !indexable(p->col.K, p->P))
         return TK3D_ERR_UNSUPPORTED;
+    if (tk_mlp_wide_outer_splits(*p))
+        return tk_mlp_wide_outer(row, col, *p, (hipStream_t)stream_);
     OuterArgs a;
     a.p = *p;
     a.units = (p->P + 31) / 32;
