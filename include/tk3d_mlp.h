@@ -168,11 +168,13 @@ int tk3d_mlp_grad_apply_f32(float *e, const float *y, const float *coef, int B, 
 
 /* Backward of a pooled layer, before the products: from g [B,C,M], the extremes and their places
  * the coefficients (a, b, d'), dgamma, dbeta and sel, [B, C, M] of (float a e, int32 place in the
- * group); positions = B * group * M, w [C][I], inner the norm in front of the layer. */
+ * group); positions = B * group * M, w [C][I], inner the norm in front of the layer; partial: doubles
+ * [C][slots][2] of scratch memory, slots of tk3d_mlp_pool_grad_slots. */
+int tk3d_mlp_pool_grad_slots(int B, int C, int M);
 int tk3d_mlp_pool_grad_f32(const float *g, const float *extreme, const unsigned char *arg, int B,
                            int C, int M, int64_t positions, const tk3d_mlp_norm *norm, const float *w,
-                           int I, const tk3d_mlp_norm *inner, void *sel, float *coef, float *dgamma,
-                           float *dbeta, void *stream);
+                           int I, const tk3d_mlp_norm *inner, void *partial, void *sel, float *coef,
+                           float *dgamma, float *dbeta, void *stream);
 /* The sparse half of W^T dy, [B, I, M * group] (groups of 32 or 64; W [O][I]), and that of dW in
  * partial sums [splits][O][I] (y [B, I, M * group], norm of y). */
 int tk3d_mlp_pool_scatter_f32(const void *sel, const float *w, int B, int O, int I, int M, int group,

@@ -117,7 +117,9 @@ def test_both_gradients_of_a_layer(cuda, monkeypatch, b, p, widths):
 
 
 @pytest.mark.parametrize("b,m,s,widths", [(1, 3, 32, (64, 128, 128)), (4, 1025, 32, (70, 100, 64, 40)),
-                                          (3, 700, 64, (128, 128, 32, 128))])
+                                          (3, 700, 64, (128, 128, 32, 128)),
+                                          # (more than 128 outputs: waves share a group; 9000 groups: sums first)
+                                          (3, 70, 64, (6, 33, 300)), (9, 1000, 32, (3, 20, 24))])
 def test_both_gradients_under_a_maximum(cuda, monkeypatch, b, m, s, widths):
     mlp = make(mlp2d_bn_relu, widths[0], widths[1:], True, cuda)
     check(mlp, lambda n, x: n.forward_max(x), lambda n, x: n(x).max(dim=3)[0],

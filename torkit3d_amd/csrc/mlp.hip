@@ -944,83 +944,58 @@ struct SumArgs {
     tk3d_mlp_sum s[kMaxSums];
 };
 
-// Sixteen outputs to a workgroup, sixteen threads to an output: the partial sums are up to 512 of
-// few values (one thread per output took 123 us on 512 sums of 32 x 32).
-__global__ void __launch_bounds__(kBlock) mlp_sum_kernel(SumArgs a)
+// Sixteen threads to an output, or to four from 32768 outputs on (12 sums of 1024 x 320 9.7 -> 7.2 us, 32 of 256 x
+// 512 6.6 -> 4.3, 256 of 128 x 128 3.9 for 4.7): the partial sums are up to 512 of few values (one thread per
+// output took 123 us on 512 sums of 32 x 32).
+template <int V> __device__ __forceinline__ void add_up(const tk3d_mlp_sum &s, double (*lds)[16][4])
 {
-    const tk3d_mlp_sum &s = a.s[blockIdx.y];
-    __shared__ double lds[kWaves][16];
     const int n = s.R * s.C;
     const int at = threadIdx.x & 15, lane = threadIdx.x >> 4;
-    for (int first = blockIdx.x * 16; first < n; first += gridDim.x * 16) {
-        const int i = first + at < n ? first + at : n - 1;
-        double sum = 0.0;
-#pragma unroll 4
-        for (int k = lane; k < s.splits; k += 16)
-            sum += (double)s.partial[k * s.stride + i];
-        sum += __shfl_xor(sum, 16);
-        sum += __shfl_xor(sum, 32);
-        if ((threadIdx.x & 63) < 16)
-            lds[threadIdx.x >> 6][at] = sum;
+    for (int first = blockIdx.x * (16 * V); first < n; first += gridDim.x * (16 * V)) {
+        const int i = first + V * at < n ? first + V * at : n - V;
+        double sum[V] = {};
+#pragma unroll 8
+        for (int k = lane; k < s.splits; k += 16) {
+            const float *part = s.partial + k * s.stride + i;
+            if constexpr (V == 4) {
+                const f32x4 v = *reinterpret_cast<const f32x4 *>(part);
+#pragma unroll
+                for (int j = 0; j < V; ++j)
+                    sum[j] += (double)v[j];
+            } else {
+                sum[0] += (double)*part;
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < V; ++j) {
+            sum[j] += __shfl_xor(sum[j], 16);
+            sum[j] += __shfl_xor(sum[j], 32);
+            if ((threadIdx.x & 63) < 16)
+                lds[threadIdx.x >> 6][at][j] = sum[j];
+        }
         __syncthreads();
-        if (threadIdx.x < 16 && first + at < n) {
-            sum = lds[0][at] + lds[1][at] + lds[2][at] + lds[3][at];
-            const int r = i / s.C;
-            s.out[(int64_t)r * s.ld + (i - r * s.C)] = (float)sum;
+        const int e = threadIdx.x / V, j = threadIdx.x % V, to = first + threadIdx.x;
+        if (threadIdx.x < 16 * V && to < n) {
+            const int r = to / s.C;
+            s.out[(int64_t)r * s.ld + (to - r * s.C)] =
+                (float)(lds[0][e][j] + lds[1][e][j] + lds[2][e][j] + lds[3][e][j]);
         }
         __syncthreads();
     }
 }
 
+__global__ void __launch_bounds__(kBlock) mlp_sum_kernel(SumArgs a)
+{
+    const tk3d_mlp_sum &s = a.s[blockIdx.y];
+    __shared__ double lds[kWaves][16][4];
+    if (s.stride % 4 == 0 && s.R * s.C % 4 == 0 && (reinterpret_cast<uintptr_t>(s.partial) & 15) == 0 &&
+        s.R * s.C >= 32768)
+        add_up<4>(s, lds);
+    else
+        add_up<1>(s, lds);
+}
+
 // ---- statistics and coefficients ---------------------------------------------------------------------
-
-// Sum of (x, y) over the block; the result is valid in every thread.
-__device__ __forceinline__ double2 block_sum(double2 v, double2 *lds)
-{
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        v.x += __shfl_xor(v.x, off);
-        v.y += __shfl_xor(v.y, off);
-    }
-    const int waves = blockDim.x >> 6;
-    if ((threadIdx.x & 63) == 0)
-        lds[threadIdx.x >> 6] = v;
-    __syncthreads();
-    double2 s = lds[0];
-    for (int w = 1; w < waves; ++w) {
-        s.x += lds[w].x;
-        s.y += lds[w].y;
-    }
-    return s;
-}
-
-__device__ __forceinline__ double2 slot_sum(const void *partial, int slots, int c, double2 *lds)
-{
-    const double2 *row = reinterpret_cast<const double2 *>(partial) + (int64_t)c * slots;
-    double2 v{0.0, 0.0};
-    for (int i = threadIdx.x; i < slots; i += blockDim.x) {
-        v.x += row[i].x;
-        v.y += row[i].y;
-    }
-    return block_sum(v, lds);
-}
-
-struct Coefficients {
-    f32x4 abd;
-    float dgamma, dbeta;
-};
-
-// (`origin`: the y from which the b y of the caller is counted)
-__device__ __forceinline__ Coefficients grad_coefficients(double2 s, double n, const tk3d_mlp_norm &norm,
-                                                          int c, double origin = 0.0)
-{
-    const double is = norm.eps < 0.0f ? (double)norm.var[c]
-                                      : 1.0 / __builtin_sqrt((double)norm.var[c] + (double)norm.eps);
-    const double gamma = norm.gamma[c], mean = norm.mean[c];
-    const double b = -gamma * is * is * is * s.y / n;
-    const double d0 = -gamma * is * s.x / n, d = d0 - b * (mean - origin);
-    return {f32x4{(float)(gamma * is), (float)b, (float)d, (float)d0}, (float)(s.y * is), (float)s.x};
-}
 
 __global__ void __launch_bounds__(kBlock)
     mlp_grad_coefficients_kernel(const void *partial, int slots, double n, tk3d_mlp_norm norm,
@@ -1111,254 +1086,6 @@ __global__ void __launch_bounds__(kBlock)
     } else {
         for (int i = blockIdx.x * kBlock + threadIdx.x; i < P; i += gridDim.x * kBlock)
             e[row + i] = f(e[row + i], y[row + i]);
-    }
-}
-
-// ---- pooled layers, backward ---------------------------------------------------------------------------
-
-// One workgroup per channel: the sums, then the coefficients, then the sparse gradient.
-__global__ void __launch_bounds__(1024)
-    mlp_pool_grad_kernel(const float *g, const float *extreme, const unsigned char *arg, int B, int C,
-                         int M, double n, tk3d_mlp_norm norm, const float *w, int I,
-                         tk3d_mlp_norm inner, int2 *sel, float *coef, float *dgamma, float *dbeta)
-{
-    __shared__ double2 lds[16], lds2[16];
-    const int c = blockIdx.x;
-    const f32x4 ss = constants_of(norm, c);
-    const float mean = norm.mean[c];
-    const int count = B * M;
-    const auto at = [&](int i) {
-        const int b = i / M;
-        return ((int64_t)b * C + c) * M + (i - b * M);
-    };
-    double2 v{0.0, 0.0};
-    for (int i = threadIdx.x; i < count; i += blockDim.x) {
-        const int64_t j = at(i);
-        const float y = extreme[j];
-        const float e = passes(normalised(y, ss)) ? g[j] : 0.0f;
-        v.x += e;
-        v.y += (double)e * (double)(y - mean);
-    }
-    double2 wm{0.0, 0.0};
-    for (int i = threadIdx.x; i < I; i += blockDim.x)
-        wm.x += (double)w[(int64_t)c * I + i] * (double)centre_of(constants_of(inner, i));
-    wm = block_sum(wm, lds2);
-    const Coefficients k = grad_coefficients(block_sum(v, lds), n, norm, c, wm.x);
-    if (threadIdx.x == 0) {
-        reinterpret_cast<f32x4 *>(coef)[c] = k.abd;
-        dgamma[c] = k.dgamma;
-        dbeta[c] = k.dbeta;
-    }
-    for (int i = threadIdx.x; i < count; i += blockDim.x) {
-        const int64_t j = at(i);
-        const float e = passes(normalised(extreme[j], ss)) ? g[j] : 0.0f;
-        sel[j] = int2{__float_as_int(k.abd.x * e), (int)arg[j]};
-    }
-}
-
-// The sparse halves. In a group of S positions a channel o has one value a e, at one place, so that
-// W^T (a e) and (a e) x^T take O x I operations a group. As products over all positions (matrix cores,
-// zeros among the rows) they took S times as many: on 16 x 512 groups of 32, O = 128, I = 64, both
-// halves of W^T dy in one product 174 us, (a e) x^T 78 us; now 46 and 72 (the product), and 31 us. A
-// wave has a group, lanes are input channels, the places are scalars, and the group's tile of S x 64
-// lies in LDS (rows of 65: read by channels and by positions).
-
-constexpr int kRow = 65;
-
-__device__ __forceinline__ float scalar_of(float v, int lane)
-{
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
-}
-
-struct SparseArgs {
-    const int2 *sel;       // [B, O, M]
-    const float *w;        // [O][I] (scatter)
-    const float *y;        // [B, I, P] (outer)
-    tk3d_mlp_norm norm;    // of y
-    float *out;            // [B, I, P] (scatter), partial sums [splits][O][I] (outer)
-    int O, I, M, run;      // a wave takes `run` consecutive groups at once
-    int units, total;      // runs: per batch element, in all
-};
-
-// out[b, i, (m, place)] = sum over o of w[o][i] a e; zero at the other places. A
-// lane adds to a column of its own, in the order of o: 12 to 16 waves a CU cover the trips to LDS (as LDS
-// atomics, without the trips, the additions took 341 us for 42 on 16 x 512 groups of 32).
-template <int S>
-__global__ void __launch_bounds__(kBlock) mlp_pool_scatter_kernel(SparseArgs a)
-{
-    extern __shared__ float tiles[];
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    float *tile = tiles + wave * (S * kRow);
-    const int i0 = blockIdx.y * 64, c = i0 + lane < a.I ? i0 + lane : a.I - 1;
-    const int p = lane & (S - 1), first = lane / S;  // of the loop over positions
-    for (int unit = blockIdx.x * kWaves + wave; unit < a.total; unit += gridDim.x * kWaves) {
-        const int b = unit / a.units, from = (unit - b * a.units) * a.run;
-        const int to = from + a.run < a.M ? from + a.run : a.M;
-        for (int m = from; m < to; ++m) {
-#pragma unroll 8
-            for (int q = 0; q < S; ++q)
-                tile[q * kRow + lane] = 0.0f;
-            for (int o0 = 0; o0 < a.O; o0 += 64) {
-                const int o = o0 + lane < a.O ? o0 + lane : a.O - 1;
-                const int2 s = a.sel[((int64_t)b * a.O + o) * a.M + m];
-                const float e = o0 + lane < a.O ? __int_as_float(s.x) : 0.0f;
-                const int n = a.O - o0 < 64 ? a.O - o0 : 64;
-                for (int k = 0; k < n; k += 8) {
-                    float w[8];
-#pragma unroll
-                    for (int j = 0; j < 8; ++j)
-                        w[j] = a.w[(int64_t)(o0 + (k + j < n ? k + j : n - 1)) * a.I + c];
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) {  // (lanes from n on: zeros at a place of the tile)
-                        float &at = tiles[wave * (S * kRow) + __builtin_amdgcn_readlane(s.y, k + j) * kRow + lane];
-                        at = __builtin_fmaf(scalar_of(e, k + j), w[j], at);
-                    }
-                }
-            }
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            const int64_t P = (int64_t)a.M * S;
-            float *out = a.out + ((int64_t)b * a.I + i0) * P + (int64_t)m * S + p;
-#pragma unroll 8
-            for (int i = first; i < 64; i += 64 / S)
-                if (i0 + i < a.I)
-                    out[i * P] = tile[p * kRow + i];
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-        }
-    }
-}
-
-// partial[split][o][i] = sum over groups of a e (relu(norm(y[i, (m, place)])) less the centre of i): 64
-// rows and 64 columns a workgroup, rows in registers.
-template <int S>
-__global__ void __launch_bounds__(kBlock) mlp_pool_outer_kernel(SparseArgs a)
-{
-    extern __shared__ float tiles[];
-    __shared__ f32x4 constants[64];
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    float *tile = tiles + wave * (S * kRow);
-    const int o0 = blockIdx.y * 64, i0 = blockIdx.z * 64;
-    const int o = o0 + lane < a.O ? o0 + lane : a.O - 1;
-    const int p = lane & (S - 1), first = lane / S;
-    if (tid < 64)
-        constants[tid] = constants_of(a.norm, i0 + tid < a.I ? i0 + tid : a.I - 1);
-    __syncthreads();
-    float acc[64];
-#pragma unroll
-    for (int k = 0; k < 64; ++k)
-        acc[k] = 0.0f;
-    // The values of the next group are requested before the present one's rows are added up.
-    const int64_t P = (int64_t)a.M * S;
-    float v[S];
-    int2 sel{0, 0};
-    const auto load = [&](int b, int m) {
-        sel = a.sel[((int64_t)b * a.O + o) * a.M + m];
-        const float *y = a.y + (int64_t)b * a.I * P + (int64_t)m * S + p;
-#pragma unroll
-        for (int q = 0; q < S; ++q) {
-            const int i = i0 + first + q * (64 / S);
-            v[q] = y[(i < a.I ? i : a.I - 1) * P];
-        }
-    };
-    int unit = blockIdx.x * kWaves + wave, b = unit / a.units, m = (unit - b * a.units) * a.run;
-    bool more = unit < a.total;
-    if (more)
-        load(b, m);
-    while (more) {
-#pragma unroll
-        for (int q = 0; q < S; ++q) {
-            const int i = first + q * (64 / S);
-            tile[p * kRow + i] = relu(normalised(v[q], constants[i])) - centre_of(constants[i]);
-        }
-        const float e = o0 + lane < a.O ? __int_as_float(sel.x) : 0.0f;
-        const int place = sel.y;
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        const int to = (unit - b * a.units + 1) * a.run;
-        if (++m >= (to < a.M ? to : a.M)) {
-            unit += gridDim.x * kWaves;
-            b = unit / a.units;
-            m = (unit - b * a.units) * a.run;
-            more = unit < a.total;
-        }
-        if (more)
-            load(b, m);
-#pragma unroll
-        for (int k = 0; k < 64; ++k)
-            acc[k] = __builtin_fmaf(scalar_of(e, k),
-                                    tile[__builtin_amdgcn_readlane(place, k) * kRow + lane], acc[k]);
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-    }
-    // (one wave after the other: 16 KB, within the tiles of four waves)
-    for (int w = 0; w < kWaves; ++w) {
-        __syncthreads();
-        if (w == wave)
-#pragma unroll
-            for (int k = 0; k < 64; ++k)
-                tiles[k * 64 + lane] = w ? tiles[k * 64 + lane] + acc[k] : acc[k];
-    }
-    __syncthreads();
-    for (int e = tid; e < 64 * 64; e += kBlock) {
-        const int k = e >> 6, i = e & 63;
-        if (o0 + k < a.O && i0 + i < a.I)
-            a.out[((int64_t)blockIdx.x * a.O + o0 + k) * a.I + i0 + i] = tiles[e];
-    }
-}
-
-constexpr int kT = 16;
-
-// gram[k][c] = sum_o W[o][k] b[o] W[o][c]; the first row of blocks also adds up bias[c].
-__global__ void __launch_bounds__(kT *kT)
-    mlp_pool_gram_kernel(const float *w, const float *coef, int O, int I, float *gram, float *bias)
-{
-    __shared__ float wk[kT][kT + 1], wc[kT][kT + 1];
-    __shared__ float dd[kT];
-    const int x = threadIdx.x % kT, y = threadIdx.x / kT;
-    const int k = blockIdx.y * kT, c = blockIdx.x * kT;
-    float sum = 0.0f, off = 0.0f;
-    for (int o = 0; o < O; o += kT) {
-        const bool in = o + y < O;
-        wk[y][x] = in && k + x < I ? w[(int64_t)(o + y) * I + k + x] * coef[(o + y) * 4 + 1] : 0.0f;
-        wc[y][x] = in && c + x < I ? w[(int64_t)(o + y) * I + c + x] : 0.0f;
-        if (x == 0)
-            dd[y] = in ? coef[(o + y) * 4 + 2] : 0.0f;
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < kT; ++i) {
-            sum = __builtin_fmaf(wk[i][y], wc[i][x], sum);
-            off = __builtin_fmaf(dd[i], wc[i][x], off);
-        }
-        __syncthreads();
-    }
-    if (k + y < I && c + x < I)
-        gram[(int64_t)(k + y) * I + c + x] = sum;
-    if (blockIdx.y == 0 && y == 0 && c + x < I)
-        bias[c + x] = off;
-}
-
-// dw[o][i] += b[o] (W xx)[o][i] + d[o] xsum[i]
-__global__ void __launch_bounds__(kT *kT)
-    mlp_pool_weight_grad_kernel(const float *w, const float *coef, const float *xx, const float *xsum,
-                                int O, int I, float *dw)
-{
-    __shared__ float wt[kT][kT + 1], xt[kT][kT + 1];
-    const int x = threadIdx.x % kT, y = threadIdx.x / kT;
-    const int o = blockIdx.y * kT + y, i = blockIdx.x * kT + x;
-    float sum = 0.0f;
-    for (int k = 0; k < I; k += kT) {
-        wt[y][x] = o < O && k + x < I ? w[(int64_t)o * I + k + x] : 0.0f;
-        xt[y][x] = k + y < I && i < I ? xx[(int64_t)(k + y) * I + i] : 0.0f;
-        __syncthreads();
-#pragma unroll
-        for (int j = 0; j < kT; ++j)
-            sum = __builtin_fmaf(wt[y][j], xt[j][x], sum);
-        __syncthreads();
-    }
-    if (o < O && i < I) {
-        float &out = dw[(int64_t)o * I + i];
-        out = __builtin_fmaf(coef[o * 4 + 1], sum, __builtin_fmaf(coef[o * 4 + 2], xsum[i], out));
     }
 }
 
@@ -1493,15 +1220,6 @@ __global__ void __launch_bounds__(kBlock)
 }
 
 // ---- launches ------------------------------------------------------------------------------------------
-
-// Runs of four groups read whole sectors of sel ([B, O, M]), as long as every SIMD keeps a wave.
-void fill_sparse(SparseArgs &a, int B)
-{
-    a.run = (int64_t)B * a.M >= 16 * tk_cu_count() ? 4 : 1;
-    a.units = (a.M + a.run - 1) / a.run;
-    a.total = B * a.units;
-}
-int sparse_bytes(int group) { return kWaves * group * kRow * 4; }
 
 constexpr int kWeightBytes = 64 << 10;  // weights in LDS: two workgroups to a CU
 
@@ -1860,109 +1578,6 @@ int tk3d_mlp_grad_apply_f32(float *e, const float *y, const float *coef, int B, 
     for (int64_t r = 0; r < rows; r += step)
         mlp_grad_apply_kernel<<<dim3(row_blocks(P), (unsigned)(rows - r < step ? rows - r : step)), kBlock, 0,
                                 (hipStream_t)stream>>>(e + r * P, y + r * P, coef, C, P);
-    return tk_launch_status();
-}
-
-int tk3d_mlp_pool_grad_f32(const float *g, const float *extreme, const unsigned char *arg, int B,
-                           int C, int M, int64_t positions, const tk3d_mlp_norm *norm, const float *w,
-                           int I, const tk3d_mlp_norm *inner, void *sel, float *coef, float *dgamma,
-                           float *dbeta, void *stream)
-{
-    mlp_pool_grad_kernel<<<C, 1024, 0, (hipStream_t)stream>>>(
-        g, extreme, arg, B, C, M, (double)positions, *norm, w, I, *inner,
-        reinterpret_cast<int2 *>(sel), coef, dgamma, dbeta);
-    return tk_launch_status();
-}
-
-int tk3d_mlp_pool_scatter_f32(const void *sel, const float *w, int B, int O, int I, int M, int group,
-                              float *out, void *stream_)
-{
-    if (B <= 0 || O <= 0 || I <= 0 || M <= 0)
-        return TK3D_ERR_BAD_SIZE;
-    if ((group != 32 && group != 64) || !tk_fits(TK_MAX_I32, B, M) || I > 65535 * 64)
-        return TK3D_ERR_UNSUPPORTED;
-    SparseArgs a{};
-    a.sel = reinterpret_cast<const int2 *>(sel);
-    a.w = w;
-    a.out = out;
-    a.O = O;
-    a.I = I;
-    a.M = M;
-    fill_sparse(a, B);
-    const int rc = group == 32 ? tk_allow_dynamic_lds<mlp_pool_scatter_kernel<32>>(sparse_bytes(32))
-                               : tk_allow_dynamic_lds<mlp_pool_scatter_kernel<64>>(sparse_bytes(64));
-    if (rc != TK3D_OK)
-        return rc;
-    const int wgs = (a.total + kWaves - 1) / kWaves, most = 4 * tk_cu_count();
-    const dim3 grid(wgs < most ? wgs : most, (I + 63) / 64);
-    if (group == 32)
-        mlp_pool_scatter_kernel<32><<<grid, kBlock, sparse_bytes(32), (hipStream_t)stream_>>>(a);
-    else
-        mlp_pool_scatter_kernel<64><<<grid, kBlock, sparse_bytes(64), (hipStream_t)stream_>>>(a);
-    return tk_launch_status();
-}
-
-// Two workgroups to a CU, and no more than there are runs for.
-int tk3d_mlp_pool_outer_splits(int B, int O, int I, int M)
-{
-    SparseArgs a{};
-    a.M = M;
-    fill_sparse(a, B);
-    const int blocks = ((O + 63) / 64) * ((I + 63) / 64), wgs = (a.total + kWaves - 1) / kWaves;
-    const int most = (2 * tk_cu_count() + blocks - 1) / blocks;
-    return wgs < most ? wgs : most;
-}
-
-int tk3d_mlp_pool_outer_f32(const void *sel, const float *y, const tk3d_mlp_norm *norm, int B, int O,
-                            int I, int M, int group, float *partial, void *stream_)
-{
-    if (B <= 0 || O <= 0 || I <= 0 || M <= 0)
-        return TK3D_ERR_BAD_SIZE;
-    if ((group != 32 && group != 64) || !tk_fits(TK_MAX_I32, B, M) || I > 65535 * 64 || O > 65535 * 64)
-        return TK3D_ERR_UNSUPPORTED;
-    SparseArgs a{};
-    a.sel = reinterpret_cast<const int2 *>(sel);
-    a.y = y;
-    a.norm = *norm;
-    a.out = partial;
-    a.O = O;
-    a.I = I;
-    a.M = M;
-    fill_sparse(a, B);
-    const int rc = group == 32 ? tk_allow_dynamic_lds<mlp_pool_outer_kernel<32>>(sparse_bytes(32))
-                               : tk_allow_dynamic_lds<mlp_pool_outer_kernel<64>>(sparse_bytes(64));
-    if (rc != TK3D_OK)
-        return rc;
-    const dim3 grid(tk3d_mlp_pool_outer_splits(B, O, I, M), (O + 63) / 64, (I + 63) / 64);
-    if (group == 32)
-        mlp_pool_outer_kernel<32><<<grid, kBlock, sparse_bytes(32), (hipStream_t)stream_>>>(a);
-    else
-        mlp_pool_outer_kernel<64><<<grid, kBlock, sparse_bytes(64), (hipStream_t)stream_>>>(a);
-    return tk_launch_status();
-}
-
-int tk3d_mlp_pool_gram_f32(const float *w, const float *coef, int O, int I, float *gram, float *bias,
-                           void *stream)
-{
-    const int n = (I + kT - 1) / kT;
-    mlp_pool_gram_kernel<<<dim3(n, n), kT * kT, 0, (hipStream_t)stream>>>(w, coef, O, I, gram, bias);
-    return tk_launch_status();
-}
-
-int tk3d_mlp_pool_weight_grad_f32(const float *sparse, int sparse_splits, const float *xx,
-                                  const float *xsum, int xx_splits, const float *w,
-                                  const float *coef, int O, int I, float *scratch, float *dw,
-                                  void *stream)
-{
-    const tk3d_mlp_sum sums[3] = {
-        {sparse, dw, (int64_t)O * I, sparse_splits, O, I, I},
-        {xx, scratch, (int64_t)I * I, xx_splits, I, I, I},
-        {xsum, scratch + (int64_t)I * I, I, xx_splits, 1, I, I}};
-    const int rc = tk3d_mlp_sum_f32(sums, 3, stream);
-    if (rc != TK3D_OK)
-        return rc;
-    mlp_pool_weight_grad_kernel<<<dim3((I + kT - 1) / kT, (O + kT - 1) / kT), kT * kT, 0, (hipStream_t)stream>>>(
-        w, coef, scratch, scratch + (int64_t)I * I, O, I, dw);
     return tk_launch_status();
 }
 

@@ -50,4 +50,54 @@ __device__ __forceinline__ void take_larger(float &best, int &where, float s, in
     where = up ? at : where;
 }
 
+// ---- sums and coefficients of a gradient --------------------------------------------------------------
+
+// Sum of (x, y) over the block; the result is valid in every thread.
+__device__ __forceinline__ double2 block_sum(double2 v, double2 *lds)
+{
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        v.x += __shfl_xor(v.x, off);
+        v.y += __shfl_xor(v.y, off);
+    }
+    const int waves = blockDim.x >> 6;
+    if ((threadIdx.x & 63) == 0)
+        lds[threadIdx.x >> 6] = v;
+    __syncthreads();
+    double2 s = lds[0];
+    for (int w = 1; w < waves; ++w) {
+        s.x += lds[w].x;
+        s.y += lds[w].y;
+    }
+    return s;
+}
+
+__device__ __forceinline__ double2 slot_sum(const void *partial, int slots, int c, double2 *lds)
+{
+    const double2 *row = reinterpret_cast<const double2 *>(partial) + (int64_t)c * slots;
+    double2 v{0.0, 0.0};
+    for (int i = threadIdx.x; i < slots; i += blockDim.x) {
+        v.x += row[i].x;
+        v.y += row[i].y;
+    }
+    return block_sum(v, lds);
+}
+
+struct Coefficients {
+    f32x4 abd;
+    float dgamma, dbeta;
+};
+
+// (`origin`: the y from which the b y of the caller is counted)
+__device__ __forceinline__ Coefficients grad_coefficients(double2 s, double n, const tk3d_mlp_norm &norm,
+                                                          int c, double origin = 0.0)
+{
+    const double is = norm.eps < 0.0f ? (double)norm.var[c]
+                                      : 1.0 / __builtin_sqrt((double)norm.var[c] + (double)norm.eps);
+    const double gamma = norm.gamma[c], mean = norm.mean[c];
+    const double b = -gamma * is * is * is * s.y / n;
+    const double d0 = -gamma * is * s.x / n, d = d0 - b * (mean - origin);
+    return {f32x4{(float)(gamma * is), (float)b, (float)d, (float)d0}, (float)(s.y * is), (float)s.x};
+}
+
 }  // namespace

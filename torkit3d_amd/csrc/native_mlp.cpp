@@ -411,10 +411,11 @@ Grads backward(const Call &c, const Kept &k, const Tensor &g, bool want_x, bool 
         const int64_t O = c.out_channels(l), I = c.in_channels(l), M = P / c.pool;
         const tk3d_mlp_norm norm = norm_of(c, k, l), inner = norm_of(c, k, l - 1);
         const Tensor sel = at::empty({B, O, M, 2}, like.options());
+        const Tensor scratch_sums = partial_sums(like, O, tk3d_mlp_pool_grad_slots((int)B, (int)O, (int)M));
         const float *w = f32(c.weight(l));
         done(tk3d_mlp_pool_grad_f32(f32(g), f32(k.y[l]), k.arg.data_ptr<uint8_t>(), (int)B, (int)O,
-                                    (int)M, B * P, &norm, w, (int)I, &inner, sel.data_ptr(),
-                                    f32(coef[l]), f32(out.params[3 * l + 1]),
+                                    (int)M, B * P, &norm, w, (int)I, &inner, scratch_sums.data_ptr(),
+                                    sel.data_ptr(), f32(coef[l]), f32(out.params[3 * l + 1]),
                                     f32(out.params[3 * l + 2]), stream),
              "tk3d_mlp_pool_grad_f32");
         const Tensor gram = at::empty({I + 1, I}, like.options());
