@@ -57,6 +57,7 @@ enum {
     TK3D_MLP_IN_GRAD = 3,     /* a x + b y + d */
     TK3D_MLP_IN_GRAD_OUT = 4, /* the same with x masked by relu(in_norm(y)) first */
     TK3D_MLP_IN_CENTRED = 5,  /* relu(in_norm(x)) - relu(beta of in_norm) */
+    TK3D_MLP_IN_SHIFTED = 7,  /* x - relu(beta of in_norm); to OUT_PLAIN, + add, alone; slots 0: not for this size */
     TK3D_MLP_OUT_PLAIN = 1,     /* out + bias, channels from C0 on in out2; either may be NULL */
     TK3D_MLP_OUT_POINTS = 2,    /* out as [B, P, C] */
     TK3D_MLP_OUT_EVAL = 3,      /* relu(out_norm(out)) */
@@ -71,7 +72,7 @@ typedef struct {
     float *out, *out2;
     const float *yprev; /* [B, C, P] */
     const float *bias;  /* [C] or NULL */
-    const float *add;   /* [B, C, P], may be out itself; IN_CENTRED to OUT_MASK alone (P % 32 == 0) */
+    const float *add;   /* [B, C, P], may be out itself; IN_CENTRED (P % 4 == 0) and IN_SHIFTED alone */
     void *partial;      /* OUT_MASK: doubles [C][slots][2]; tk3d_mlp_product_slots gives slots */
     int32_t B, C, C0, P;
     int32_t group, M;   /* pooled forms: P == group * M, group 32 or 64 */
@@ -84,15 +85,18 @@ int tk3d_mlp_product_f32(int in, int out, const tk3d_mlp_product *p, void *strea
 /* Weight gradient: out[r][c] = sum over (b, p) of row(r, p) * colv(c, p), r < R, c < C, in
  * `splits` partial sums [splits][R][C]. Rows: raw x, gradient (a x + b y + d, masked or not),
  * or activations less relu(beta); columns: raw x, activations, or these less relu(beta). rowsum (NULL or [splits][R]) gets the
- * sums of the rows themselves. */
+ * sums of the rows themselves. Activations less a centre come as rows and columns of one tensor: the result is
+ * symmetric, and below the diagonal of more than 64 rows nothing need be written. */
 enum {
     TK3D_MLP_ROW_RAW = 0,
     TK3D_MLP_ROW_GRAD = 1,
     TK3D_MLP_ROW_GRAD_OUT = 2,
     TK3D_MLP_ROW_CENTRED = 4,
+    TK3D_MLP_ROW_SHIFTED = 5, /* x - relu(beta of row_norm), with COL_SHIFTED; more than 64 rows */
     TK3D_MLP_COL_RAW = 0,
     TK3D_MLP_COL_ACT = 1,
-    TK3D_MLP_COL_CENTRED = 2
+    TK3D_MLP_COL_CENTRED = 2,
+    TK3D_MLP_COL_SHIFTED = 3
 };
 typedef struct {
     tk3d_mlp_source row, col; /* K = R and C; weights unused */
@@ -142,6 +146,12 @@ int tk3d_mlp_batch_relu_f32(const float *y, const tk3d_mlp_batch_norm *norm, flo
 int tk3d_mlp_batch_pool_f32(const float *y, const tk3d_mlp_batch_norm *norm, int size, float *out,
                             float *extreme, unsigned char *arg, void *stream);
 
+/* out = relu(max norm(y)) over whole rows, [B, C]; arg the place of the maximum, extreme the y there and index the
+ * place of the maximum of relu(norm(y)), the first of equal ones. z: norm(y) where it is there, else norm is
+ * as above. */
+int tk3d_mlp_batch_rows_f32(const float *y, const float *z, const tk3d_mlp_batch_norm *norm, int B, int C, int P,
+                            float *out, float *extreme, int32_t *arg, int64_t *index, void *stream);
+
 /* A normalised layer's ReLU and maximum over groups of `size` <= 255 consecutive values: out =
  * relu(max z), arg the place of the maximum and extreme the y at that place, [groups] each. */
 int tk3d_mlp_pool_max_f32(const float *z, const float *y, int64_t groups, int size, float *out,
@@ -169,10 +179,11 @@ int tk3d_mlp_grad_apply_f32(float *e, const float *y, const float *coef, int B, 
 /* Backward of a pooled layer, before the products: from g [B,C,M], the extremes and their places
  * the coefficients (a, b, d'), dgamma, dbeta and sel, [B, C, M] of (float a e, int32 place in the
  * group); positions = B * group * M, w [C][I], inner the norm in front of the layer; partial: doubles
- * [C][slots][2] of scratch memory, slots of tk3d_mlp_pool_grad_slots. */
+ * [C][slots][2] of scratch memory, slots of tk3d_mlp_pool_grad_slots. The places come as bytes or, with
+ * arg NULL, in arg32. */
 int tk3d_mlp_pool_grad_slots(int B, int C, int M);
-int tk3d_mlp_pool_grad_f32(const float *g, const float *extreme, const unsigned char *arg, int B,
-                           int C, int M, int64_t positions, const tk3d_mlp_norm *norm, const float *w,
+int tk3d_mlp_pool_grad_f32(const float *g, const float *extreme, const unsigned char *arg,
+                           const int32_t *arg32, int B, int C, int M, int64_t positions, const tk3d_mlp_norm *norm, const float *w,
                            int I, const tk3d_mlp_norm *inner, void *partial, void *sel, float *coef,
                            float *dgamma, float *dbeta, void *stream);
 /* The sparse half of W^T dy, [B, I, M * group] (groups of 32 or 64; W [O][I]), and that of dW in
@@ -182,10 +193,19 @@ int tk3d_mlp_pool_scatter_f32(const void *sel, const float *w, int B, int O, int
 int tk3d_mlp_pool_outer_splits(int B, int O, int I, int M);
 int tk3d_mlp_pool_outer_f32(const void *sel, const float *y, const tk3d_mlp_norm *norm, int B, int O,
                             int I, int M, int group, float *partial, void *stream);
+/* The same where a group is a whole row of P values (M == 1, P % 4 == 0): the sparse half of W^T dy [B, I, P], and
+ * that of dW [O][I] itself, from the activations of x [B, I, P] (or, shifted != 0, x - relu(beta of norm)). */
+int tk3d_mlp_rows_scatter_f32(const void *sel, const float *w, int B, int O, int I, int P, float *out,
+                              void *stream);
+int tk3d_mlp_rows_outer_f32(const void *sel, const float *x, int shifted, const tk3d_mlp_norm *norm, int B, int O,
+                            int I, int P, float *dw, void *stream);
+/* mean[c] of x [B, C, P] */
+int tk3d_mlp_channel_means_f32(const float *x, int B, int C, int P, float *mean, void *stream);
 /* gram[k][c] = sum_o W[o][k] b[o] W[o][c] and bias[c] = sum_o W[o][c] d'[o]; W [O][I]. */
 int tk3d_mlp_pool_gram_f32(const float *w, const float *coef, int O, int I, float *gram, float *bias,
                            void *stream);
-/* dW[o][i] = sparse[o][i] + b[o] (W xx)[o][i] + d'[o] xsum[i]; sparse, xx, xsum as partial sums. */
+/* dW[o][i] = sparse[o][i] + b[o] (W xx)[o][i] + d'[o] xsum[i]; sparse, xx, xsum as partial sums, of xx what is on
+ * and above the diagonal. */
 int tk3d_mlp_pool_weight_grad_f32(const float *sparse, int sparse_splits, const float *xx,
                                   const float *xsum, int xx_splits, const float *w,
                                   const float *coef, int O, int I, float *scratch, float *dw,

@@ -11,6 +11,7 @@ import pytest
 import torch
 from torch import nn
 
+from torkit3d_amd import _native
 from torkit3d_amd.nn import SharedMLP, mlp1d_bn_relu, mlp2d_bn_relu
 from torkit3d_amd.ops.group_points import group_points_with_xyz
 
@@ -53,9 +54,13 @@ def check(mlp, fused, reference, inputs, monkeypatch):
     real = SharedMLP._chain
     monkeypatch.setattr(SharedMLP, "_chain",
                         lambda self, *a, **k: used.append(real(self, *a, **k)) or used[-1])
+    compare_forms(mlp, fused, reference, inputs)
+    assert len(used) == 1 and used[0] is not None, "the fused chain did not run"
+
+
+def compare_forms(mlp, fused, reference, inputs):
     plain32, plain64 = stock(mlp, torch.float32), stock(mlp, torch.float64)
     got = everything(mlp, fused, inputs)
-    assert len(used) == 1 and used[0] is not None, "the fused chain did not run"
     single = everything(plain32, reference, inputs)
     exact = everything(plain64, reference, [(t.double() if t.is_floating_point() else t, g)
                                             for t, g in inputs])
@@ -146,6 +151,32 @@ def test_wide_layers_under_a_maximum(cuda, monkeypatch, b, m, s, widths):
     mlp = make(mlp2d_bn_relu, widths[0], widths[1:], True, cuda)
     check(mlp, lambda n, x: n.forward_max(x), lambda n, x: n(x).max(dim=3)[0],
           [(randn(m, b, widths[0], m, s), True)], monkeypatch)
+
+
+# A maximum over all points behind the last layer: on the layer's own input (tiles of it as for wide layers) and on
+# activations of up to 128 channels and more, several and single clouds, rows off the tiles of 64 positions, channels
+# whose maximum is negative, equal maxima; sizes that stay with the dense backward.
+@pytest.mark.parametrize("b,p,widths", [
+    (6, 4100, (330, 700)), (13, 2048, (70, 160)), (3, 1400, (9, 64, 128)), (1, 5000, (40, 33, 70)), (2, 2084, (6, 160, 330)),
+    (5, 1028, (3, 30, 100)), (40, 128, (12, 65, 140)),
+    (2, 2048, (64, 100)), (3, 37, (8, 16, 40)), (2, 512, (320, 1024))])
+def test_maximum_over_points(cuda, monkeypatch, b, p, widths):
+    mlp = make(mlp1d_bn_relu, widths[0], widths[1:], True, cuda)
+    with torch.no_grad():
+        mlp[-1].bn.bias[0::5] = -40.0  # (nothing passes the ReLU)
+    x = randn(p, b, widths[0], p)
+    x[:, :, 1::3] = x[:, :, 0:1]  # copies of a point
+    reference = stock(mlp, torch.float32)
+    values, places = mlp.forward_points_max(x.clone().requires_grad_())
+    want = torch.max(reference(x), 2)
+    assert torch.equal(values, want[0]) and torch.equal(places, want[1])
+    used = []
+    real = _native.mlp_max
+    monkeypatch.setattr(_native, "mlp_max", lambda *a: used.append(real(*a)) or used[-1])
+    mlp2 = make(mlp1d_bn_relu, widths[0], widths[1:], True, cuda)
+    compare_forms(mlp2, lambda m, x: m.forward_points_max(x)[0], lambda m, x: m(x).max(dim=2)[0],
+                  [(randn(p + 1, b, widths[0], p), True)])
+    assert bool(used[0]) == (widths[-1] >= 2 * widths[-2] and b * p >= 4096 and p % 4 == 0)
 
 
 # Products whose waves share a tile: groups of 32 and

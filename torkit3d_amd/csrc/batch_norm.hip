@@ -20,7 +20,8 @@
 // -> the two kernels with ReLU, or with maximum): [16, 64, 512, 32] 110 -> 35, 33; [16, 128, 128, 64] 59
 // -> 33, 32; [8, 32, 2048, 32] 214 -> 37, 34; [8, 128, 16384] 59 -> 32; [8, 1024, 2048] 34 -> 34; [8, 64,
 // 2048, 20] 138 -> 40, 31 (84 MB: sums 14.6 us, 5.7 TB/s). The ReLU (10 to 14 us) and the maximum (40 to
-// 57 us) that the library needed behind it come on top of its times. Every workgroup of the second adds up the sixteen results of its channel itself.
+// 57 us) that the library needed behind it come on top of its times. Every workgroup of the second adds up the
+// sixteen results of its channel itself.
 #include "mlp_common.h"
 
 namespace {
@@ -228,6 +229,57 @@ __global__ void __launch_bounds__(kBlock) batch_pool_kernel(const float *__restr
     }
 }
 
+// The same over whole rows, a wave a row; Z: from the normalised values z.
+template <bool Z>
+__global__ void __launch_bounds__(kBlock)
+    batch_rows_kernel(const float *__restrict__ y, const float *__restrict__ z, tk3d_mlp_batch_norm n, int rows, int C,
+                      int P, float *__restrict__ out, float *__restrict__ extreme, int *__restrict__ arg,
+                      int64_t *__restrict__ index)
+{
+    const int row = blockIdx.x * kWaves + threadIdx.x / TK_WAVE, lane = threadIdx.x % TK_WAVE;
+    if (row >= rows)
+        return;
+    f32x4 k{0.0f, 0.0f, 0.0f, 0.0f};
+    if constexpr (!Z)
+        k = batch_constants(n, row % C, row < C && lane == 0);
+    const float *__restrict__ values = (Z ? z : y) + (int64_t)row * P;
+    float best = -__builtin_huge_valf();
+    int where = 0x7fffffff;  // (of no value: any other is before it)
+    const auto look = [&](float v, int at) { take_larger(best, where, Z ? v : normalised(v, k), at); };
+    if ((P & 3) == 0) {
+        constexpr int U = 4;
+        for (int i = 4 * lane; i < P; i += U * 4 * TK_WAVE) {
+            f32x4 v[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int at = i + u * 4 * TK_WAVE;
+                v[u] = *reinterpret_cast<const f32x4 *>(values + (at < P ? at : i));
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (i + u * 4 * TK_WAVE < P)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        look(v[u][j], i + u * 4 * TK_WAVE + j);
+        }
+    } else {
+        for (int i = lane; i < P; i += TK_WAVE)
+            look(values[i], i);
+    }
+#pragma unroll
+    for (int off = 1; off < TK_WAVE; off <<= 1) {
+        const float other = __shfl_xor(best, off);
+        const int at = __shfl_xor(where, off);
+        take_larger(best, where, other, at);
+    }
+    if (lane == 0) {
+        out[row] = relu(best);
+        extreme[row] = y[(int64_t)row * P + where];
+        arg[row] = where;
+        index[row] = best <= 0.0f ? 0 : where;  // (behind the ReLU all are zero then)
+    }
+}
+
 // Workgroups per row, so that the chip has sixteen per CU of them and none has under 4096 values.
 int stretches_of(int64_t rows, int P)
 {
@@ -298,6 +350,26 @@ int tk3d_mlp_batch_pool_f32(const float *y, const tk3d_mlp_batch_norm *norm, int
         batch_pool_kernel<16><<<grid, kBlock, 0, stream>>>(y, *norm, size, out, extreme, arg, stretches);
     else
         batch_pool_kernel<0><<<grid, kBlock, 0, stream>>>(y, *norm, size, out, extreme, arg, stretches);
+    return tk_launch_status();
+}
+
+int tk3d_mlp_batch_rows_f32(const float *y, const float *z, const tk3d_mlp_batch_norm *norm, int B, int C, int P,
+                            float *out, float *extreme, int32_t *arg, int64_t *index, void *stream_)
+{
+    if (B <= 0 || C <= 0 || P <= 0)
+        return TK3D_ERR_BAD_SIZE;
+    if (!tk_fits(TK_MAX_I32, B, C) || (P % 4 == 0 && (((uintptr_t)y | (uintptr_t)z) & 15) != 0))
+        return TK3D_ERR_UNSUPPORTED;
+    const int rows = B * C;
+    const unsigned grid = (unsigned)((rows + kWaves - 1) / kWaves);
+    const hipStream_t stream = (hipStream_t)stream_;
+    if (z)
+        batch_rows_kernel<true><<<grid, kBlock, 0, stream>>>(y, z, tk3d_mlp_batch_norm{}, rows, C, P, out, extreme, arg,
+                                                            index);
+    else if (tk3d_mlp_batch_norm_supported(norm->B, norm->C, norm->P))
+        batch_rows_kernel<false><<<grid, kBlock, 0, stream>>>(y, z, *norm, rows, C, P, out, extreme, arg, index);
+    else
+        return TK3D_ERR_UNSUPPORTED;
     return tk_launch_status();
 }
 

@@ -239,7 +239,7 @@ template <int IN, int OUT, int PT, int CT> struct Results {
                 for (int i = 0; i < RUN; ++i)
                     before[i] = yrow[pos + i > P - 1 ? P - 1 : pos + i];
             }
-            if constexpr (IN == IN_CENTRED) {  // (P is a multiple of 32 here)
+            if constexpr (IN == IN_CENTRED) {  // (P is a multiple of four here)
                 const float *arow = p.add + ((int64_t)b * p.C + (mine ? c : p.C - 1)) * P;
 #pragma unroll
                 for (int i = 0; i < PT; ++i) {
@@ -1401,7 +1401,8 @@ extern "C" {
 
 int tk3d_mlp_product_slots(int in, int out, const tk3d_mlp_product *p)
 {
-    if (const int wide = tk_mlp_wide_product_slots(in, out, *p))
+    const int wide = tk_mlp_wide_product_slots(in, out, *p);
+    if (wide || in == TK3D_MLP_IN_SHIFTED)
         return wide;
     GemmArgs g;
     const Shape split = pick_split(out, *p, in == TK3D_MLP_IN_RAW2);
@@ -1423,7 +1424,7 @@ int tk3d_mlp_product_f32(int in, int out, const tk3d_mlp_product *p, void *strea
         return TK3D_ERR_UNSUPPORTED;
     if (out == TK3D_MLP_OUT_POOL_EVAL && ((p->group != 32 && p->group != 64) || p->M * p->group != p->P))
         return TK3D_ERR_UNSUPPORTED;
-    if (in == TK3D_MLP_IN_CENTRED && out == TK3D_MLP_OUT_MASK && (!p->add || p->P % 32 != 0))
+    if (in == TK3D_MLP_IN_CENTRED && out == TK3D_MLP_OUT_MASK && (!p->add || p->P % 4 != 0))
         return TK3D_ERR_BAD_SIZE;
     if (tk_mlp_wide_product_slots(in, out, *p))
         return tk_mlp_wide_product(in, out, *p, (hipStream_t)stream_);

@@ -12,6 +12,7 @@ namespace {
 struct PoolGradArgs {
     const float *g, *extreme;
     const unsigned char *arg;
+    const int *arg32;
     int B, C, M, count;  // count = B * M
     tk3d_mlp_norm norm;
     double2 *partial;    // [C][slots], or NULL: a workgroup has the whole of its channel
@@ -65,7 +66,7 @@ __global__ void __launch_bounds__(1024)
     }
     for_groups(a, [&](int64_t j) {
         const float e = passes(normalised(a.extreme[j], ss)) ? a.g[j] : 0.0f;
-        sel[j] = int2{__float_as_int(k.abd.x * e), (int)a.arg[j]};
+        sel[j] = int2{__float_as_int(k.abd.x * e), a.arg ? (int)a.arg[j] : a.arg32[j]};
     });
 }
 
@@ -244,48 +245,140 @@ __global__ void __launch_bounds__(WO * kBlock) mlp_pool_outer_kernel(SparseArgs 
     }
 }
 
-// ---- small products of the weights -----------------------------------------------------------------------
+// ---- a group that is a whole row --------------------------------------------------------------------------------
 //
-// 32 x 32 results a workgroup on the matrix cores, the sum shared by its four waves: these are chains of trips to
-// L2 (in tiles of 16 x 16 through LDS, two barriers per 16 of the sum, gram took 25 us on O = 512, I = 256).
+// One value per channel and batch element: of a layer under a maximum over all points dy is dense only through b y
+// + d, whose products are as wide as the layer's input and not as its output (1024 channels of 320, 8 x 2048
+// points, both gradients and what led to them: 337 us dense, 216 us so; 1024 of 128, 32 x 2048 points, with its forward
+// and backward in front 1216 -> 663).
 
-constexpr int kStep = 8;  // steps of two of the sum that are requested at once
-
-// The four waves' sums of a tile added up, in wave 0's order: result r of lane l.
-__device__ __forceinline__ void add_up(tk_f32x16 &sum, f32x4 (*lds)[4][64], int wave, int lane)
+// out[b, i, p] = sum over the o whose place is p of w[o][i] a e, in the order of o. A wave has 64 positions and 64
+// channels: it looks through the places, and takes eight o of its own at once.
+__global__ void __launch_bounds__(kBlock)
+    mlp_rows_scatter_kernel(const int2 *sel, const float *w, int O, int I, int P, int tiles, int total, float *out)
 {
+    constexpr int AT_ONCE = 8;
+    extern __shared__ float tiles_[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    float *tile = tiles_ + wave * (64 * kRow);
+    const int i0 = blockIdx.y * 64, c = i0 + lane < I ? i0 + lane : I - 1;
+    for (int unit = blockIdx.x * kWaves + wave; unit < total; unit += gridDim.x * kWaves) {
+        const int b = unit / tiles, from = (unit - b * tiles) * 64;
+#pragma unroll 8
+        for (int q = 0; q < 64; ++q)
+            tile[q * kRow + lane] = 0.0f;
+        int2 next = sel[(int64_t)b * O + (lane < O ? lane : O - 1)];
+        for (int o0 = 0; o0 < O; o0 += 64) {
+            const int2 s = next;
+            const int after = o0 + 64 + lane;
+            next = sel[(int64_t)b * O + (after < O ? after : O - 1)];
+            const float e = __int_as_float(s.x);
+            unsigned long long mine =
+                __ballot(o0 + lane < O && (unsigned)s.y < (unsigned)P && (unsigned)(s.y - from) < 64u);
+            while (mine) {
+                int at[AT_ONCE];
+                float v[AT_ONCE];
+                int n = 0;
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
-        lds[wave][q][lane] = f32x4{sum[4 * q], sum[4 * q + 1], sum[4 * q + 2], sum[4 * q + 3]};
-    __syncthreads();
+                for (int j = 0; j < AT_ONCE; ++j) {
+                    at[j] = mine ? __builtin_ctzll(mine) : at[0];
+                    n += mine ? 1 : 0;
+                    mine &= mine - 1;  // (zero stays zero)
+                    v[j] = w[(int64_t)(o0 + at[j]) * I + c];
+                }
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const f32x4 v = (lds[0][q][lane] + lds[1][q][lane]) + (lds[2][q][lane] + lds[3][q][lane]);
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            sum[4 * q + j] = v[j];
+                for (int j = 0; j < AT_ONCE; ++j)
+                    if (j < n) {
+                        float &sum = tile[(__builtin_amdgcn_readlane(s.y, at[j]) - from) * kRow + lane];
+                        sum = __builtin_fmaf(scalar_of(e, at[j]), v[j], sum);
+                    }
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        float *to = out + ((int64_t)b * I + i0) * P + from + lane;
+#pragma unroll 8
+        for (int i = 0; i < 64; ++i)
+            if (i0 + i < I && from + lane < P)
+                to[(int64_t)i * P] = tile[lane * kRow + i];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
     }
 }
 
-// gram[k][c] = sum_o W[o][k] b[o] W[o][c]; the first row of blocks also adds up bias[c].
+// dw[o][i] = sum over b of a e x', x' that of channel i at the place of o. Neighbouring lanes have neighbouring o,
+// whose places are within one row of x: the row stays in L1 for all of them.
+template <bool SHIFTED>
+__global__ void __launch_bounds__(kBlock) mlp_rows_outer_kernel(const int2 *sel, const float *x, tk3d_mlp_norm norm, int B,
+                                                                int O, int I, int P, float *dw)
+{
+    const int i = blockIdx.x, o = blockIdx.y * kBlock + threadIdx.x;
+    const f32x4 k = constants_of(norm, i);
+    if (o >= O)
+        return;
+    float sum = 0.0f;
+#pragma unroll 4
+    for (int b = 0; b < B; ++b) {
+        const int2 s = sel[(int64_t)b * O + o];
+        const float v = x[((int64_t)b * I + i) * P + ((unsigned)s.y < (unsigned)P ? s.y : 0)];
+        sum = __builtin_fmaf(__int_as_float(s.x), (SHIFTED ? v : relu(normalised(v, k))) - centre_of(k), sum);
+    }
+    dw[(int64_t)o * I + i] = sum;
+}
+
+// mean[c], a workgroup a channel. (Where a sum is counted from need not be known to the last bit.)
+__global__ void __launch_bounds__(kBlock) mlp_channel_means_kernel(const float *x, int B, int C, int P, float *mean)
+{
+    __shared__ double2 lds[kWaves];
+    const int c = blockIdx.x;
+    float sum = 0.0f;
+    for (int b = 0; b < B; ++b)
+#pragma unroll 8
+        for (int i = threadIdx.x; i < P; i += kBlock)
+            sum += x[((int64_t)b * C + c) * P + i];
+    const double2 s = block_sum(double2{sum, 0.0}, lds);
+    if (threadIdx.x == 0)
+        mean[c] = (float)(s.x / ((double)B * P));
+}
+
+// ---- small products of the weights -----------------------------------------------------------------------
+//
+// A tile of results a workgroup on the matrix cores, the sum shared by its four waves: these are chains of trips to
+// L2 (in tiles of 16 x 16 through LDS, two barriers per 16 of the sum, gram took 19 us on O = 512, I = 256; in fp32 on the
+// matrix cores 14.5, in fp64 8.5).
+
+constexpr int kStep = 16, kStepGrad = 8;  // steps of four of the sum that are requested at once
+
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+
+// The four waves' sums of a tile of 16 x 16 added up: wave r returns the result in row 4 r + lane / 16.
+__device__ __forceinline__ double add_up(const f64x4 &sum, double (*lds)[4][64], int wave, int lane)
+{
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+        lds[wave][r][lane] = sum[r];
+    __syncthreads();
+    return (lds[0][wave][lane] + lds[1][wave][lane]) + (lds[2][wave][lane] + lds[3][wave][lane]);
+}
+
+// gram[k][c] = sum_o W[o][k] b[o] W[o][c]; the first row of blocks also adds up bias[c]. In fp64, rounded once: an
+// error here is the same at all positions, and what is added up over them next, the gradients of the batch norm in
+// front, is small (dbeta under a maximum over 2048 points from sums in fp32 twice as far from 64 bits as from a
+// dense backward, now no farther).
 __global__ void __launch_bounds__(kBlock)
     mlp_pool_gram_kernel(const float *w, const float *coef, int O, int I, float *gram, float *bias)
 {
-    __shared__ f32x4 lds[kWaves][4][64];
-    __shared__ float part[kWaves][32];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, half = lane >> 5, l32 = lane & 31;
-    const int k = blockIdx.y * 32 + l32, c = blockIdx.x * 32 + l32;
+    __shared__ double lds[kWaves][4][64], part[kWaves][16];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, quarter = lane >> 4, l16 = lane & 15;
+    const int k = blockIdx.y * 16 + l16, c = blockIdx.x * 16 + l16;
     const int kk = k < I ? k : I - 1, cc = c < I ? c : I - 1;
-    tk_f32x16 sum;
-#pragma unroll
-    for (int r = 0; r < 16; ++r)
-        sum[r] = 0.0f;
-    float off = 0.0f;
-    for (int o0 = wave * (2 * kStep); o0 < O; o0 += kWaves * 2 * kStep) {
+    f64x4 sum{0.0, 0.0, 0.0, 0.0};
+    double off = 0.0;
+    for (int o0 = wave * (4 * kStep); o0 < O; o0 += kWaves * 4 * kStep) {
         float x[kStep], y[kStep], b[kStep], d[kStep];
 #pragma unroll
         for (int s = 0; s < kStep; ++s) {
-            const int o = o0 + 2 * s + half, at = o < O ? o : O - 1;
+            const int o = o0 + 4 * s + quarter, at = o < O ? o : O - 1;
             x[s] = w[(int64_t)at * I + kk];
             y[s] = w[(int64_t)at * I + cc];
             b[s] = o < O ? coef[at * 4 + 1] : 0.0f;
@@ -293,59 +386,50 @@ __global__ void __launch_bounds__(kBlock)
         }
 #pragma unroll
         for (int s = 0; s < kStep; ++s) {
-            sum = __builtin_amdgcn_mfma_f32_32x32x2f32(x[s] * b[s], y[s], sum, 0, 0, 0);
-            off = __builtin_fmaf(d[s], y[s], off);
+            sum = __builtin_amdgcn_mfma_f64_16x16x4f64((double)x[s] * (double)b[s], (double)y[s], sum, 0, 0, 0);
+            off = __builtin_fma((double)d[s], (double)y[s], off);
         }
     }
+    off += __shfl_xor(off, 16);
     off += __shfl_xor(off, 32);
-    if (half == 0)
-        part[wave][l32] = off;
-    add_up(sum, lds, wave, lane);
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const int row = blockIdx.y * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
-        if (r >> 2 == wave && row < I && c < I)
-            gram[(int64_t)row * I + c] = sum[r];
-    }
-    if (blockIdx.y == 0 && threadIdx.x < 32 && c < I)
-        bias[c] = (part[0][l32] + part[1][l32]) + (part[2][l32] + part[3][l32]);
+    if (quarter == 0)
+        part[wave][l16] = off;
+    const double total = add_up(sum, lds, wave, lane);
+    const int row = blockIdx.y * 16 + 4 * wave + quarter;
+    if (row < I && c < I)
+        gram[(int64_t)row * I + c] = (float)total;
+    if (blockIdx.y == 0 && threadIdx.x < 16 && c < I)
+        bias[c] = (float)((part[0][l16] + part[1][l16]) + (part[2][l16] + part[3][l16]));
 }
 
-// dw[o][i] += b[o] (W xx)[o][i] + d[o] xsum[i]
+// dw[o][i] += b[o] (W xx)[o][i] + d[o] xsum[i], terms of which the sum is a small part: in fp64 as well
 __global__ void __launch_bounds__(kBlock)
     mlp_pool_weight_grad_kernel(const float *w, const float *coef, const float *xx, const float *xsum,
                                 int O, int I, float *dw)
 {
-    __shared__ f32x4 lds[kWaves][4][64];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, half = lane >> 5, l32 = lane & 31;
-    const int o = blockIdx.y * 32 + l32, i = blockIdx.x * 32 + l32;
+    __shared__ double lds[kWaves][4][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, quarter = lane >> 4, l16 = lane & 15;
+    const int o = blockIdx.y * 16 + l16, i = blockIdx.x * 16 + l16, ii = i < I ? i : I - 1;
     const float *row = w + (int64_t)(o < O ? o : O - 1) * I;
-    const int ii = i < I ? i : I - 1;
-    tk_f32x16 sum;
+    f64x4 sum{0.0, 0.0, 0.0, 0.0};
+    for (int k0 = wave * (4 * kStepGrad); k0 < I; k0 += kWaves * 4 * kStepGrad) {
+        float x[kStepGrad], y[kStepGrad];
 #pragma unroll
-    for (int r = 0; r < 16; ++r)
-        sum[r] = 0.0f;
-    // (a lane takes runs of a row of w: its steps are those of the product's order only within both halves)
-    for (int k0 = wave * (2 * kStep); k0 < I; k0 += kWaves * 2 * kStep) {
-        float x[kStep], y[kStep];
-#pragma unroll
-        for (int s = 0; s < kStep; ++s) {
-            const int k = k0 + kStep * half + s, at = k < I ? k : I - 1;
+        for (int s = 0; s < kStepGrad; ++s) {
+            const int k = k0 + 4 * s + quarter, at = k < I ? k : I - 1;
             x[s] = k < I ? row[at] : 0.0f;
-            y[s] = k < I ? xx[(int64_t)at * I + ii] : 0.0f;
+            y[s] = k < I ? xx[(int64_t)(at < ii ? at : ii) * I + (at < ii ? ii : at)] : 0.0f;
         }
 #pragma unroll
-        for (int s = 0; s < kStep; ++s)
-            sum = __builtin_amdgcn_mfma_f32_32x32x2f32(x[s], y[s], sum, 0, 0, 0);
+        for (int s = 0; s < kStepGrad; ++s)
+            sum = __builtin_amdgcn_mfma_f64_16x16x4f64((double)x[s], (double)y[s], sum, 0, 0, 0);
     }
-    add_up(sum, lds, wave, lane);
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const int to = blockIdx.y * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
-        if (r >> 2 == wave && to < O && i < I) {
-            float &out = dw[(int64_t)to * I + i];
-            out = __builtin_fmaf(coef[to * 4 + 1], sum[r], __builtin_fmaf(coef[to * 4 + 2], xsum[i], out));
-        }
+    const double total = add_up(sum, lds, wave, lane);
+    const int to = blockIdx.y * 16 + 4 * wave + quarter;
+    if (to < O && i < I) {
+        float &out = dw[(int64_t)to * I + i];
+        out = (float)__builtin_fma((double)coef[to * 4 + 1], total,
+                                   __builtin_fma((double)coef[to * 4 + 2], (double)xsum[i], (double)out));
     }
 }
 
@@ -396,8 +480,8 @@ extern "C" {
 
 int tk3d_mlp_pool_grad_slots(int B, int C, int M) { return grad_slots(B, C, M); }
 
-int tk3d_mlp_pool_grad_f32(const float *g, const float *extreme, const unsigned char *arg, int B,
-                           int C, int M, int64_t positions, const tk3d_mlp_norm *norm, const float *w,
+int tk3d_mlp_pool_grad_f32(const float *g, const float *extreme, const unsigned char *arg,
+                           const int32_t *arg32, int B, int C, int M, int64_t positions, const tk3d_mlp_norm *norm, const float *w,
                            int I, const tk3d_mlp_norm *inner, void *partial, void *sel, float *coef,
                            float *dgamma, float *dbeta, void *stream_)
 {
@@ -406,7 +490,7 @@ int tk3d_mlp_pool_grad_f32(const float *g, const float *extreme, const unsigned 
     if (!tk_fits(TK_MAX_I32 - (1 << 24), B, M) || C > 65535)
         return TK3D_ERR_UNSUPPORTED;
     const dim3 grid(grad_slots(B, C, M), C);
-    const PoolGradArgs a{g, extreme, arg, B, C, M, B * M, *norm,
+    const PoolGradArgs a{g, extreme, arg, arg32, B, C, M, B * M, *norm,
                          grid.x > 1 ? reinterpret_cast<double2 *>(partial) : nullptr};
     const hipStream_t stream = (hipStream_t)stream_;
     if (grid.x > 1) {
@@ -415,7 +499,7 @@ int tk3d_mlp_pool_grad_f32(const float *g, const float *extreme, const unsigned 
         if (rc != TK3D_OK)
             return rc;
     }
-    mlp_pool_grad_kernel<<<grid, grid.x > 1 ? kBlock : 1024, 0, stream>>>(
+    mlp_pool_grad_kernel<<<grid, grid.x > 1 || a.count <= 1024 ? kBlock : 1024, 0, stream>>>(
         a, (double)positions, w, I, *inner, reinterpret_cast<int2 *>(sel), coef, dgamma, dbeta);
     return tk_launch_status();
 }
@@ -482,10 +566,47 @@ int tk3d_mlp_pool_outer_f32(const void *sel, const float *y, const tk3d_mlp_norm
                        : launch_outer<64>(a, splits, (hipStream_t)stream_);
 }
 
+int tk3d_mlp_rows_scatter_f32(const void *sel, const float *w, int B, int O, int I, int P, float *out, void *stream)
+{
+    if (B <= 0 || O <= 0 || I <= 0 || P <= 0)
+        return TK3D_ERR_BAD_SIZE;
+    const int tiles = (P + 63) / 64;
+    if (!tk_fits(1 << 30, B, tiles) || I > 65535 * 64)
+        return TK3D_ERR_UNSUPPORTED;
+    constexpr int bytes = kWaves * 64 * kRow * 4;
+    const int rc = tk_allow_dynamic_lds<mlp_rows_scatter_kernel>(bytes);
+    if (rc != TK3D_OK)
+        return rc;
+    const int wgs = (B * tiles + kWaves - 1) / kWaves, most = 4 * tk_cu_count();
+    mlp_rows_scatter_kernel<<<dim3(wgs < most ? wgs : most, (I + 63) / 64), kBlock, bytes, (hipStream_t)stream>>>(
+        reinterpret_cast<const int2 *>(sel), w, O, I, P, tiles, B * tiles, out);
+    return tk_launch_status();
+}
+
+int tk3d_mlp_rows_outer_f32(const void *sel, const float *x, int shifted, const tk3d_mlp_norm *norm, int B, int O,
+                            int I, int P, float *dw, void *stream_)
+{
+    if (B <= 0 || O <= 0 || I <= 0 || P <= 0)
+        return TK3D_ERR_BAD_SIZE;
+    const dim3 grid(I, (O + kBlock - 1) / kBlock);
+    const hipStream_t stream = (hipStream_t)stream_;
+    if (shifted)
+        mlp_rows_outer_kernel<true><<<grid, kBlock, 0, stream>>>(reinterpret_cast<const int2 *>(sel), x, *norm, B, O, I, P, dw);
+    else
+        mlp_rows_outer_kernel<false><<<grid, kBlock, 0, stream>>>(reinterpret_cast<const int2 *>(sel), x, *norm, B, O, I, P, dw);
+    return tk_launch_status();
+}
+
+int tk3d_mlp_channel_means_f32(const float *x, int B, int C, int P, float *mean, void *stream)
+{
+    mlp_channel_means_kernel<<<C, kBlock, 0, (hipStream_t)stream>>>(x, B, C, P, mean);
+    return tk_launch_status();
+}
+
 int tk3d_mlp_pool_gram_f32(const float *w, const float *coef, int O, int I, float *gram, float *bias,
                            void *stream)
 {
-    const int n = (I + 31) / 32;
+    const int n = (I + 15) / 16;
     mlp_pool_gram_kernel<<<dim3(n, n), kBlock, 0, (hipStream_t)stream>>>(w, coef, O, I, gram, bias);
     return tk_launch_status();
 }
@@ -502,7 +623,7 @@ int tk3d_mlp_pool_weight_grad_f32(const float *sparse, int sparse_splits, const 
     const int rc = tk3d_mlp_sum_f32(sums, 3, stream);
     if (rc != TK3D_OK)
         return rc;
-    mlp_pool_weight_grad_kernel<<<dim3((I + 31) / 32, (O + 31) / 32), kBlock, 0, (hipStream_t)stream>>>(
+    mlp_pool_weight_grad_kernel<<<dim3((I + 15) / 16, (O + 15) / 16), kBlock, 0, (hipStream_t)stream>>>(
         w, coef, scratch, scratch + (int64_t)I * I, O, I, dw);
     return tk_launch_status();
 }

@@ -9,8 +9,9 @@
 //
 // us, before -> now (TFLOP/s of the matrix rate's 157): weight gradient of 320 -> 1024 channels, 16384 positions
 // 217 -> 120 (90), of 512 -> 1024, 2048 positions 38 -> 28 (77), of 256 -> 256, 1024 positions 14.5 -> 5.8; input
-// gradient of 320 -> 1024, 16384 positions 165 -> 124 (87), of 320 -> 256 45 -> 36 (75). Errors against 64 bits:
-// dW 4.4e-7 -> 1.6e-7, dx 2.9e-7 -> 1.3e-7 of the result for the first.
+// gradient of 320 -> 1024, 16384 positions 165 -> 124 (87), of 320 -> 256 45 -> 36 (75). Activations times
+// themselves (the dense half under a maximum), 320 x 320 on 16384 positions: 63 us, 42 without the blocks below
+// the diagonal. Errors against 64 bits: dW 4.4e-7 -> 1.6e-7, dx 2.9e-7 -> 1.3e-7 of the result for the first.
 #include "mlp_common.h"
 #include "mlp_wide.h"
 
@@ -50,6 +51,7 @@ __global__ void __launch_bounds__(kWide, 4) mlp_wide_outer_kernel(WideOuterArgs 
     constexpr int STEP = kWide / 8, RL = 32 * RB / STEP, CL = 32 * CB / STEP;  // 16-byte loads of a thread, rows apart
     constexpr int ROWS = 32 * RB * STRIDE, HALF = ROWS + 32 * CB * STRIDE;
     constexpr bool kGrad = ROW == TK3D_MLP_ROW_GRAD || ROW == TK3D_MLP_ROW_GRAD_OUT;
+    constexpr bool kRowSums = ROW == TK3D_MLP_ROW_CENTRED || ROW == TK3D_MLP_ROW_SHIFTED;
     __shared__ __attribute__((aligned(16))) float lds[2 * HALF];
     const tk3d_mlp_outer &p = a.p;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -57,6 +59,8 @@ __global__ void __launch_bounds__(kWide, 4) mlp_wide_outer_kernel(WideOuterArgs 
     const int R = p.row.K, C = p.col.K, P = p.P;
     int group, cblock;
     if (!place_of(blockIdx.x, a.splits * a.rblocks, a.cblocks, group, cblock))
+        return;
+    if (kRowSums && 2 * (group % a.rblocks) > cblock)  // (symmetric: nothing below the diagonal is read)
         return;
     const int split = group / a.rblocks, rbase = group % a.rblocks * (32 * RB), cbase = cblock * (32 * CB);
 
@@ -68,7 +72,7 @@ __global__ void __launch_bounds__(kWide, 4) mlp_wide_outer_kernel(WideOuterArgs 
         const int r = rbase + first + i * STEP, row = r < R ? r : R - 1;
         if constexpr (kGrad)
             coef[i] = reinterpret_cast<const f32x4 *>(p.row.coef)[row];
-        if constexpr (ROW == TK3D_MLP_ROW_GRAD_OUT || ROW == TK3D_MLP_ROW_CENTRED)
+        if constexpr (ROW == TK3D_MLP_ROW_GRAD_OUT || ROW == TK3D_MLP_ROW_CENTRED || ROW == TK3D_MLP_ROW_SHIFTED)
             row_act[i] = constants_of(p.row_norm, row);
     }
 #pragma unroll
@@ -113,6 +117,8 @@ __global__ void __launch_bounds__(kWide, 4) mlp_wide_outer_kernel(WideOuterArgs 
                     g = __builtin_fmaf(coef[i].x, g, __builtin_fmaf(coef[i].y, y[kGrad ? i : 0][j], coef[i].z));
                 if constexpr (ROW == TK3D_MLP_ROW_CENTRED)
                     g = relu(normalised(g, row_act[i])) - centre_of(row_act[i]);
+                if constexpr (ROW == TK3D_MLP_ROW_SHIFTED)
+                    g -= centre_of(row_act[i]);
                 v[j] = in ? g : 0.0f;
             }
             *reinterpret_cast<f32x4 *>(to + i * STEP * STRIDE) = v;
@@ -123,9 +129,9 @@ __global__ void __launch_bounds__(kWide, 4) mlp_wide_outer_kernel(WideOuterArgs 
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 float h = c[i][j];
-                if constexpr (COL != TK3D_MLP_COL_RAW)
+                if constexpr (COL == TK3D_MLP_COL_ACT || COL == TK3D_MLP_COL_CENTRED)
                     h = relu(normalised(h, col_act[i]));
-                if constexpr (COL == TK3D_MLP_COL_CENTRED)
+                if constexpr (COL == TK3D_MLP_COL_CENTRED || COL == TK3D_MLP_COL_SHIFTED)
                     h -= centre_of(col_act[i]);
                 v[j] = in ? h : 0.0f;
             }
@@ -161,7 +167,7 @@ __global__ void __launch_bounds__(kWide, 4) mlp_wide_outer_kernel(WideOuterArgs 
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-                if constexpr (ROW == TK3D_MLP_ROW_CENTRED)
+                if constexpr (kRowSums)
                     row_sum += g[step & 1][k];
                 acc = __builtin_amdgcn_mfma_f32_32x32x2f32(g[step & 1][k], h[step & 1][k], acc, 0, 0, 0);
             }
@@ -190,10 +196,10 @@ __global__ void __launch_bounds__(kWide, 4) mlp_wide_outer_kernel(WideOuterArgs 
         if (row < R && column < C)
             p.partial[((int64_t)split * R + row) * C + column] = total[r];
     }
-    if constexpr (ROW == TK3D_MLP_ROW_CENTRED) {
+    if constexpr (kRowSums) {
         row_total += __shfl_xor(row_total, 32);
         const int row = rbase + wrow + l32;
-        if (p.rowsum && cblock == 0 && wave % CB == 0 && half == 0 && row < R)
+        if (p.rowsum && cbase == rbase && wave % CB == 0 && half == 0 && row < R)
             p.rowsum[(int64_t)split * R + row] = row_total;
     }
 }
@@ -218,7 +224,7 @@ __global__ void __launch_bounds__(kWide) mlp_wide_product_kernel(WideProductArgs
     constexpr int G = KC * GS, HALF = G + KC * WS;
     constexpr int QUADS = NP / 4, STEP = kWide / QUADS, GL = KC / STEP;
     constexpr int WQUADS = 8 * CT, WL = (KC * WQUADS + kWide - 1) / kWide;
-    constexpr bool kGrad = IN != TK3D_MLP_IN_CENTRED;
+    constexpr bool kGrad = IN == TK3D_MLP_IN_GRAD || IN == TK3D_MLP_IN_GRAD_OUT;
     extern __shared__ __attribute__((aligned(16))) float lds[];
     const tk3d_mlp_product &p = a.p;
     const tk3d_mlp_source &s = p.src[0];
@@ -283,8 +289,10 @@ __global__ void __launch_bounds__(kWide) mlp_wide_product_kernel(WideProductArgs
                 if constexpr (kGrad)
                     g = __builtin_fmaf(grad_coef[k].x, g,
                                        __builtin_fmaf(grad_coef[k].y, y[kGrad ? i : 0][j], grad_coef[k].z));
-                else
+                else if constexpr (IN == TK3D_MLP_IN_CENTRED)
                     g = relu(normalised(g, act_coef[k])) - centre_of(act_coef[k]);
+                else
+                    g -= centre_of(act_coef[k]);
                 v[j] = in && k < K ? g : 0.0f;
             }
             *reinterpret_cast<f32x4 *>(to + (first + i * STEP) * GS + 4 * quad) = v;
@@ -378,7 +386,7 @@ __global__ void __launch_bounds__(kWide) mlp_wide_product_kernel(WideProductArgs
             const bool inside = pos < P;
             const int64_t offset = ((int64_t)b * C + c) * P + (inside ? pos : P - 4);
             v += bias;
-            if constexpr (IN == TK3D_MLP_IN_CENTRED)
+            if constexpr (!kGrad)
                 v += *reinterpret_cast<const f32x4 *>(p.add + offset);
             if constexpr (OUT == TK3D_MLP_OUT_MASK) {
                 const f32x4 was = *reinterpret_cast<const f32x4 *>(p.yprev + offset);
@@ -459,9 +467,10 @@ ProductShape product_shape(int in, int out, const tk3d_mlp_product &p)
 {
     const ProductShape none{0, 0, 0, 0};
     const tk3d_mlp_source &s = p.src[0];
-    if ((in != TK3D_MLP_IN_GRAD && in != TK3D_MLP_IN_GRAD_OUT && in != TK3D_MLP_IN_CENTRED) ||
+    const bool grad = in == TK3D_MLP_IN_GRAD || in == TK3D_MLP_IN_GRAD_OUT;
+    if ((!grad && in != TK3D_MLP_IN_CENTRED && in != TK3D_MLP_IN_SHIFTED) ||
         (out != TK3D_MLP_OUT_MASK && out != TK3D_MLP_OUT_PLAIN) || s.K <= 64 || s.K > 2048 || p.C <= 64 ||
-        p.P % 4 != 0 || !aligned(s.x) || (in != TK3D_MLP_IN_CENTRED && !aligned(s.y)) || s.batch_stride % 4 != 0 ||
+        p.P % 4 != 0 || !aligned(s.x) || (grad && !aligned(s.y)) || s.batch_stride % 4 != 0 ||
         !aligned(p.out) || !aligned(p.out2) || !aligned(p.yprev) || !aligned(p.add))
         return none;
     const int ctiles = (p.C + 31) / 32;
@@ -474,6 +483,10 @@ ProductShape product_shape(int in, int out, const tk3d_mlp_product &p)
 
 }  // namespace
 
+// Rows and columns are the same activations, less the same centres: half of the blocks leave at once. (For the
+// number of splits alone.)
+static bool symmetric(const tk3d_mlp_outer &p) { return p.row.x == p.col.x && p.row.y == nullptr && p.row.K == p.col.K; }
+
 // Rows of one or two tiles of 32, and columns of one, waste too much of 128 x 64. No fewer positions than
 // a tile for a workgroup, else two workgroups to a CU.
 int tk_mlp_wide_outer_splits(const tk3d_mlp_outer &p)
@@ -481,7 +494,10 @@ int tk_mlp_wide_outer_splits(const tk3d_mlp_outer &p)
     if (p.row.K <= 64 || p.col.K <= 32 || p.P % 4 != 0 || !aligned(p.row.x) || !aligned(p.row.y) || !aligned(p.col.x) ||
         p.row.batch_stride % 4 != 0 || p.col.batch_stride % 4 != 0)
         return 0;
-    const int64_t blocks = (int64_t)((p.row.K + 127) / 128) * ((p.col.K + 63) / 64);
+    const int64_t rblocks = (p.row.K + 127) / 128, cblocks = (p.col.K + 63) / 64;
+    int64_t blocks = rblocks * cblocks;
+    if (symmetric(p))  // blocks on and above the diagonal: cblocks - 2 r of row block r
+        blocks -= rblocks * (rblocks - 1);
     const int64_t total = (int64_t)p.B * ((p.P + 31) / 32);
     if (total > (1 << 29) || blocks > (1 << 20))
         return 0;
@@ -508,6 +524,7 @@ int tk_mlp_wide_outer(int row, int col, const tk3d_mlp_outer &p, hipStream_t str
     TK_CASE(TK3D_MLP_ROW_GRAD_OUT, TK3D_MLP_COL_RAW)
     TK_CASE(TK3D_MLP_ROW_GRAD_OUT, TK3D_MLP_COL_ACT)
     TK_CASE(TK3D_MLP_ROW_CENTRED, TK3D_MLP_COL_CENTRED)
+    TK_CASE(TK3D_MLP_ROW_SHIFTED, TK3D_MLP_COL_SHIFTED)
 #undef TK_CASE
     return TK3D_ERR_UNSUPPORTED;
 }
@@ -533,6 +550,7 @@ int tk_mlp_wide_product(int in, int out, const tk3d_mlp_product &p, hipStream_t 
     TK_CASE(TK3D_MLP_IN_GRAD_OUT, TK3D_MLP_OUT_MASK)
     TK_CASE(TK3D_MLP_IN_GRAD_OUT, TK3D_MLP_OUT_PLAIN)
     TK_CASE(TK3D_MLP_IN_CENTRED, TK3D_MLP_OUT_MASK)
+    TK_CASE(TK3D_MLP_IN_SHIFTED, TK3D_MLP_OUT_PLAIN)
 #undef TK_CASE
 #undef TK_SHAPE
     return TK3D_ERR_UNSUPPORTED;

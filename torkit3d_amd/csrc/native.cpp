@@ -745,8 +745,19 @@ PYBIND11_MODULE(_host, m)
         const Tensor t[] = {optional_arg("x", x), optional_arg("x2", x2), optional_arg("xyz", xyz),
                             optional_arg("centre", centre), optional_arg("index", index)};
         return unlocked([&] {
-            return mlp(t[0], t[1], t[2], t[3], t[4], std::move(params), std::move(buffers),
-                       std::move(eps), std::move(momentum), training, pool);
+            const variable_list made = mlp(t[0], t[1], t[2], t[3], t[4], std::move(params),
+                                           std::move(buffers), std::move(eps), std::move(momentum),
+                                           training, pool);
+            return made.empty() ? Tensor() : made[0];
+        });
+    });
+    // (values, places), or an empty list
+    m.def("mlp_max", [](py::handle x, std::vector<Tensor> params, std::vector<Tensor> buffers,
+                        std::vector<double> eps, std::vector<double> momentum, bool training) {
+        const Tensor in = tensor_arg("x", x), none;
+        return unlocked([&] {
+            return mlp(in, none, none, none, none, std::move(params), std::move(buffers),
+                       std::move(eps), std::move(momentum), training, -1);
         });
     });
     m.def("edge_lists", [](py::handle index, int64_t n) {

@@ -46,9 +46,9 @@ bool watched();
 // Saved tensors come back through hooks, which may lay them out anew.
 variable_list dense(variable_list saved);
 
-Tensor mlp(Tensor x, Tensor x2, const Tensor &xyz, const Tensor &centre, const Tensor &index,
-           std::vector<Tensor> params, std::vector<Tensor> buffers, std::vector<double> eps,
-           std::vector<double> momentum, bool training, int64_t pool);
+variable_list mlp(Tensor x, Tensor x2, const Tensor &xyz, const Tensor &centre, const Tensor &index,
+                  std::vector<Tensor> params, std::vector<Tensor> buffers, std::vector<double> eps,
+                  std::vector<double> momentum, bool training, int64_t pool);
 
 Tensor edge_lists(const Tensor &index, int64_t n);
 Tensor edge_conv(const Tensor &x, const Tensor &index, const Tensor &lists,

@@ -70,6 +70,7 @@ struct Call {
     // centre [B, 3, M], index [B, M, S]
     Tensor xyz, centre, index;
     int64_t pool = 0;  // maximum over groups of this many consecutive positions, 0: none
+    bool whole = false;  // maximum over all positions (pool is their number), and its place
     int64_t rows = 0;  // of a dense input given as [B, C, rows, P / rows]
     bool training = false;
     std::vector<double> eps, momentum;
@@ -91,7 +92,7 @@ struct Call {
 // 1 / sqrt(variance + eps), as batch norm saves it).
 struct Kept {
     std::vector<Tensor> y, mean, var;
-    Tensor arg;
+    Tensor arg;  // uint8; of a maximum over all positions int32
 };
 
 tk3d_mlp_norm norm_of(const Call &c, const Kept &k, int64_t l)
@@ -281,6 +282,21 @@ Tensor pool_max(const Normalised &n, Tensor &extreme, Tensor &arg)
     return out;
 }
 
+// The same over all positions, with the places as torch.max gives them behind a ReLU.
+Tensor row_max(const Normalised &n, Tensor &extreme, Tensor &arg, Tensor &index)
+{
+    const Tensor y = n.y.contiguous(), z = n.z.defined() ? n.z.contiguous() : n.z;
+    const int64_t B = y.size(0), C = y.size(1), P = y.numel() / (B * C);
+    const Tensor out = at::empty({B, C}, y.options());
+    extreme = at::empty({B, C}, y.options());
+    arg = at::empty({B, C}, y.options().dtype(at::kInt));
+    index = at::empty({B, C}, y.options().dtype(at::kLong));
+    done(tk3d_mlp_batch_rows_f32(f32(y), f32(z), &n.norm, (int)B, (int)C, (int)P, f32(out), f32(extreme),
+                                 arg.data_ptr<int32_t>(), index.data_ptr<int64_t>(), stream_of(y)),
+         "tk3d_mlp_batch_rows_f32");
+    return out;
+}
+
 // Training: the activations of the stock modules, bit by bit. The gradient of a training step
 // follows the signs and places that last-bit differences decide: with products and statistics of
 // its own, however exact, one step in six of a PointNet++ or DGCNN had single gradients off by more
@@ -288,7 +304,7 @@ Tensor pool_max(const Normalised &n, Tensor &extreme, Tensor &arg)
 // products are the library's, and the batch norms' sums come in its order (csrc/batch_norm.hip). Fused
 // are the grouping, the batch norm with the ReLU or the maximum behind it, what is kept (the products
 // alone, no activations, no edge of a pooled layer), and the whole backward.
-Tensor forward_training(const Call &c, Kept &k)
+Tensor forward_training(const Call &c, Kept &k, Tensor &index)
 {
     const int64_t B = c.batch(), L = c.layers();
     Tensor h = c.x2.defined() ? at::cat({c.x, c.x2}, 1) : c.x;
@@ -311,7 +327,7 @@ Tensor forward_training(const Call &c, Kept &k)
         k.var.push_back(n.inv_std);
         if (c.pool && l == L - 1) {
             Tensor extreme;
-            h = pool_max(n, extreme, k.arg);
+            h = c.whole ? row_max(n, extreme, k.arg, index) : pool_max(n, extreme, k.arg);
             k.y.push_back(extreme);
         } else {
             h = activate(n);
@@ -407,13 +423,89 @@ Grads backward(const Call &c, const Kept &k, const Tensor &g, bool want_x, bool 
     int64_t l = L - 1;
     Tensor e = g;
     bool masked = false;  // whether e already is the gradient behind the norm
-    if (c.pool) {
+    if (c.whole) {
+        // As below with a group that is a row. The layer's input is the activation of the layer in front, or
+        // x itself, counted from its mean.
+        const int64_t O = c.out_channels(l), I = c.in_channels(l);
+        const bool first = l == 0;
+        Tensor x = first ? c.x : k.y[l - 1];
+        if (reinterpret_cast<uintptr_t>(x.data_ptr()) & 15)  // (a hook's doing)
+            x = x.clone();
+        Tensor mean;
+        if (first) {
+            mean = at::empty({I}, like.options());
+            done(tk3d_mlp_channel_means_f32(f32(x), (int)B, (int)I, (int)P, f32(mean), stream),
+                 "tk3d_mlp_channel_means_f32");
+        }
+        const tk3d_mlp_norm norm = norm_of(c, k, l),
+                            inner = first ? tk3d_mlp_norm{f32(mean), f32(mean), f32(mean), f32(mean), -1.0f}
+                                          : norm_of(c, k, l - 1);
+        const Tensor sel = at::empty({B, O, 2}, like.options());
+        const Tensor sums = partial_sums(like, O, tk3d_mlp_pool_grad_slots((int)B, (int)O, 1));
+        const float *w = f32(c.weight(l));
+        done(tk3d_mlp_pool_grad_f32(f32(g), f32(k.y[l]), nullptr, k.arg.data_ptr<int32_t>(), (int)B, (int)O, 1,
+                                    B * P, &norm, w, (int)I, &inner, sums.data_ptr(), sel.data_ptr(),
+                                    f32(coef[l]), f32(out.params[3 * l + 1]), f32(out.params[3 * l + 2]),
+                                    stream),
+             "tk3d_mlp_pool_grad_f32");
+        tk3d_mlp_outer o{};
+        o.B = (int32_t)B;
+        o.P = (int32_t)P;
+        o.row = o.col = source(x, nullptr, 0, 0);
+        o.row_norm = o.col_norm = inner;
+        Paired both;
+        if (!first || want_x) {
+            const Tensor gram = at::empty({I + 1, I}, like.options());
+            done(tk3d_mlp_pool_gram_f32(w, f32(coef[l]), (int)O, (int)I, f32(gram), f32(gram) + I * I, stream),
+                 "tk3d_mlp_pool_gram_f32");
+            e = at::empty({B, I, P}, like.options());
+            done(tk3d_mlp_rows_scatter_f32(sel.data_ptr(), w, (int)B, (int)O, (int)I, (int)P, f32(e), stream),
+                 "tk3d_mlp_rows_scatter_f32");
+            tk3d_mlp_product p = product(B, I, P);
+            p.src[0] = source(x, f32(gram), I, 1);
+            p.in_norm = p.out_norm = inner;
+            p.yprev = first ? nullptr : f32(x);
+            p.bias = f32(gram) + I * I;
+            p.add = p.out = f32(e);
+            if (first) {
+                run_product(TK3D_MLP_IN_SHIFTED, TK3D_MLP_OUT_PLAIN, p, stream);
+                out.x = e;
+            } else {
+                both = pair(TK3D_MLP_IN_CENTRED, TK3D_MLP_OUT_MASK, p, o, like, stream);
+                if (both.slots == 0)
+                    std::tie(both.sums, both.slots) =
+                        summed_product(TK3D_MLP_IN_CENTRED, TK3D_MLP_OUT_MASK, p, like, stream);
+            }
+        }
+        if (!both.outer.defined()) {
+            const int splits = tk3d_mlp_outer_splits(&o);
+            both.outer = at::empty({splits, I, I}, like.options());
+            both.rows = at::empty({splits, I}, like.options());
+            o.partial = f32(both.outer);
+            o.rowsum = f32(both.rows);
+            done(tk3d_mlp_outer_f32(first ? TK3D_MLP_ROW_SHIFTED : TK3D_MLP_ROW_CENTRED,
+                                    first ? TK3D_MLP_COL_SHIFTED : TK3D_MLP_COL_CENTRED, &o, stream),
+                 "tk3d_mlp_outer_f32");
+        }
+        const Tensor sparse = at::empty({1, O, I}, like.options()), scratch = at::empty({I + 1, I}, like.options());
+        done(tk3d_mlp_rows_outer_f32(sel.data_ptr(), f32(x), first, &inner, (int)B, (int)O, (int)I, (int)P,
+                                     f32(sparse), stream),
+             "tk3d_mlp_rows_outer_f32");
+        done(tk3d_mlp_pool_weight_grad_f32(f32(sparse), 1, f32(both.outer), f32(both.rows),
+                                           (int)both.outer.size(0), w, f32(coef[l]), (int)O, (int)I,
+                                           f32(scratch), f32(out.params[3 * l]), stream),
+             "tk3d_mlp_pool_weight_grad_f32");
+        if (!first)
+            coefficients(l - 1, both.sums.data_ptr(), both.slots);
+        masked = true;
+        --l;
+    } else if (c.pool) {
         const int64_t O = c.out_channels(l), I = c.in_channels(l), M = P / c.pool;
         const tk3d_mlp_norm norm = norm_of(c, k, l), inner = norm_of(c, k, l - 1);
         const Tensor sel = at::empty({B, O, M, 2}, like.options());
         const Tensor scratch_sums = partial_sums(like, O, tk3d_mlp_pool_grad_slots((int)B, (int)O, (int)M));
         const float *w = f32(c.weight(l));
-        done(tk3d_mlp_pool_grad_f32(f32(g), f32(k.y[l]), k.arg.data_ptr<uint8_t>(), (int)B, (int)O,
+        done(tk3d_mlp_pool_grad_f32(f32(g), f32(k.y[l]), k.arg.data_ptr<uint8_t>(), nullptr, (int)B, (int)O,
                                     (int)M, B * P, &norm, w, (int)I, &inner, scratch_sums.data_ptr(),
                                     sel.data_ptr(), f32(coef[l]), f32(out.params[3 * l + 1]),
                                     f32(out.params[3 * l + 2]), stream),
@@ -613,6 +705,8 @@ Tensor in_stock_operators(const Call &c)
                            c.eps[l], false);
         h = at::relu(h);
     }
+    if (c.whole)
+        return std::get<0>(at::max(h, 2));
     if (c.pool)
         h = std::get<0>(at::max(h.view({h.size(0), h.size(1), h.size(2) / c.pool, c.pool}), 3));
     return h;
@@ -621,11 +715,13 @@ Tensor in_stock_operators(const Call &c)
 struct Node : torch::autograd::Function<Node> {  // (made in training mode alone)
     // Saved: x, x2, xyz, centre, index, arg, then of every layer weight, gamma, beta, y, mean, var.
     // (The tensors in front of the call are what autograd sees; the call holds them too.)
-    static Tensor forward(AutogradContext *ctx, const std::optional<Tensor> &, const std::optional<Tensor> &,
-                          at::TensorList, const Call &call)
+    // The maximum over all positions has their places behind it.
+    static variable_list forward(AutogradContext *ctx, const std::optional<Tensor> &,
+                                 const std::optional<Tensor> &, at::TensorList, const Call &call)
     {
         Kept k;
-        const Tensor z = forward_training(call, k);
+        Tensor index;
+        const Tensor z = forward_training(call, k, index);
         variable_list saved = {call.x, call.x2, call.xyz, call.centre, call.index, k.arg};
         for (int64_t l = 0; l < call.layers(); ++l) {
             for (int64_t i = 0; i < 3; ++i)
@@ -636,10 +732,14 @@ struct Node : torch::autograd::Function<Node> {  // (made in training mode alone
         }
         ctx->save_for_backward(std::move(saved));
         ctx->saved_data["pool"] = call.pool;
+        ctx->saved_data["whole"] = call.whole;
         ctx->saved_data["eps"] = call.eps;
         ctx->saved_data["want_x"] = call.x.defined() && call.x.requires_grad();
         ctx->saved_data["want_x2"] = call.x2.defined() && call.x2.requires_grad();
-        return z;
+        if (!call.whole)
+            return {z};
+        ctx->mark_non_differentiable({index});
+        return {z, index};
     }
 
     static variable_list backward(AutogradContext *ctx, variable_list grads)
@@ -654,6 +754,7 @@ struct Node : torch::autograd::Function<Node> {  // (made in training mode alone
         c.index = s[4];
         k.arg = s[5];
         c.pool = ctx->saved_data["pool"].toInt();
+        c.whole = ctx->saved_data["whole"].toBool();
         c.training = true;
         c.eps = ctx->saved_data["eps"].toDoubleVector();
         const int64_t L = ((int64_t)s.size() - 6) / 6;
@@ -882,55 +983,77 @@ bool usable_layer(const Tensor *params, const Tensor *buffers, const Tensor &lik
 
 }  // namespace
 
+// Whether the backward of a maximum over all positions takes this layer: its products are as wide as its input.
+// That pays from twice as many outputs and 4096 positions on (64 -> 128 -> 256 channels, 4 x 1024 forward and backward
+// 296 -> 277 us; 256 -> 512 -> 1024, 16 x 128 276 for 314: more launches, each of its 5 us).
+bool whole_rows(const Call &c)
+{
+    const int64_t l = c.layers() - 1, O = c.out_channels(l), I = c.in_channels(l), B = c.batch(), P = c.positions();
+    if (P % 4 != 0 || O < 2 * I || B * P < 4096 || B > (1 << 20))
+        return false;
+    if (l > 0)
+        return true;
+    tk3d_mlp_product p = product(B, I, P);
+    p.src[0] = source(c.x, nullptr, I, 1);
+    return tk3d_mlp_product_slots(TK3D_MLP_IN_SHIFTED, TK3D_MLP_OUT_PLAIN, &p) > 0;
+}
+
 // x [B,C,P] (or [B,C,M,S]); a chain applied to it. Declines (undefined result) what the kernels
 // do not take: the caller then runs the stock modules.
-Tensor mlp(Tensor x, Tensor x2, const Tensor &xyz, const Tensor &centre, const Tensor &index,
-           std::vector<Tensor> params, std::vector<Tensor> buffers, std::vector<double> eps,
-           std::vector<double> momentum, bool training, int64_t pool)
+// With pool -1 the maximum over all positions: [B, C] and the places, for training alone.
+variable_list mlp(Tensor x, Tensor x2, const Tensor &xyz, const Tensor &centre, const Tensor &index,
+                  std::vector<Tensor> params, std::vector<Tensor> buffers, std::vector<double> eps,
+                  std::vector<double> momentum, bool training, int64_t pool)
 {
     Call c;
     const int64_t L = (int64_t)params.size() / 3;
+    c.whole = pool < 0;
+    if (c.whole) {
+        if (!training || !x.defined() || x.dim() != 3 || x.size(2) == 0)
+            return {};
+        pool = 0;
+    }
     // (Pooled forms: groups of 32 or 64, which fill whole tiles of every shape; other groups take
     // the dense chain and a maximum behind it.)
     if (L == 0 || (pool && (L < 2 || (pool != 32 && pool != 64))) || watched())
-        return Tensor();
+        return {};
     const bool grouped = xyz.defined();
     std::vector<int64_t> shape;
     if (grouped) {
         if (L < 2 || !pool || !usable(xyz, xyz) || !usable(centre, xyz) || !usable_index(index, xyz) ||
             xyz.dim() != 3 || centre.dim() != 3 || index.dim() != 3 || index.size(2) != pool || centre.size(2) != index.size(1) || xyz.size(1) != 3 ||
             centre.size(1) != 3 || index.size(0) != xyz.size(0) || centre.size(0) != xyz.size(0))
-            return Tensor();
+            return {};
         c.xyz = xyz.contiguous();
         c.centre = centre.contiguous();
         c.index = index.contiguous();
         if (x.defined() && (x.dim() != 3 || x.size(2) != xyz.size(2) || x.size(0) != xyz.size(0)))
-            return Tensor();
+            return {};
     } else {
         if (!x.defined() || x.dim() < 3 || x.dim() > 4 || (pool && x.size(-1) != pool))
-            return Tensor();
+            return {};
         if (x2.defined() && (x.dim() != 3 || x2.dim() != 3 || x2.size(0) != x.size(0) ||
                              x2.size(2) != x.size(2)))
-            return Tensor();
+            return {};
         shape = x.sizes().vec();
     }
     const bool has_x = x.defined(), has_x2 = x2.defined();
     const Tensor &first = grouped ? xyz : x;
     if ((has_x && !usable(x, first)) || (has_x2 && !usable(x2, first)))
-        return Tensor();
+        return {};
     int64_t channels = (has_x ? x.size(1) : 0) + (has_x2 ? x2.size(1) : 0) + (grouped ? 3 : 0);
     bool tracked = (has_x && x.requires_grad()) || (has_x2 && x2.requires_grad());
     for (int64_t l = 0; l < L; ++l) {
         if (!usable_layer(&params[3 * l], &buffers[3 * l], first))
-            return Tensor();
+            return {};
         for (int i = 0; i < 3; ++i)
             tracked = tracked || params[3 * l + i].requires_grad();
         if (params[3 * l].size(1) != channels)
-            return Tensor();
+            return {};
         channels = params[3 * l].size(0);
     }
     if (params[0].dim() != (grouped ? 4 : x.dim()))
-        return Tensor();  // (a Conv1d on [B, C, M, S] and the like: stock torch has the error)
+        return {};  // (a Conv1d on [B, C, M, S] and the like: stock torch has the error)
     c.rows = !grouped && x.dim() == 4 ? x.size(2) : 0;
     if (has_x)
         c.x = x.dim() == 4 ? x.flatten(2).contiguous() : x.contiguous();
@@ -947,7 +1070,12 @@ Tensor mlp(Tensor x, Tensor x2, const Tensor &xyz, const Tensor &centre, const T
     // too, signs and places decide the gradients, and nothing of the forward would be left to fuse.
     const bool grads = c10::GradMode::is_enabled() && tracked;
     if (training != grads || (training && !same_gradients(P)))
-        return Tensor();
+        return {};
+    if (c.whole) {
+        c.pool = P;
+        if (!whole_rows(c))
+            return {};
+    }
     int64_t widest = has_x ? c.x.size(1) : 0;
     if (has_x2)
         widest = std::max(widest, c.x2.size(1));
@@ -957,27 +1085,30 @@ Tensor mlp(Tensor x, Tensor x2, const Tensor &xyz, const Tensor &centre, const T
     // (one value per channel has no variance: stock batch norm raises the error)
     if (B == 0 || P == 0 || longest == 0 || B * P < 2 || widest > 2048 ||
         (widest + 8) * longest > (1 << 29) || B * longest > (1 << 30))
-        return Tensor();
+        return {};
     OnDeviceOf guard(c.like().device());
     for (int64_t l = 0; training && l < L; ++l) {
         const int64_t C = c.out_channels(l), rows = grouped ? index.size(1) : c.rows;
         const std::vector<int64_t> y =
             rows ? std::vector<int64_t>{B, C, rows, P / rows} : std::vector<int64_t>{B, C, P};
         if (!library_norm(c.like(), y, &c.params[3 * l], &c.buffers[3 * l], c.eps[l]))
-            return Tensor();
+            return {};
     }
     Tensor z;
     if (training) {
         const auto given = [](const Tensor &t) {
             return t.defined() ? std::optional<Tensor>(t) : std::nullopt;
         };
-        z = Node::apply(given(c.x), given(c.x2), at::TensorList(c.params), c);
+        const variable_list made = Node::apply(given(c.x), given(c.x2), at::TensorList(c.params), c);
+        if (c.whole)
+            return made;
+        z = made[0];
     } else {
         z = evaluate(c);
     }
     if (!grouped && x.dim() == 4 && !pool)
         z = z.reshape({shape[0], z.size(1), shape[2], shape[3]});
-    return z;
+    return {z};
 }
 
 // The inverse of a graph [B, N, K] over N points, for edge_conv(); undefined where the kernels do

@@ -2,7 +2,7 @@
 import torch
 from torch import nn
 
-from ...nn import mlp1d_bn_relu, mlp_bn_relu
+from ...nn import forward_points_max, mlp1d_bn_relu, mlp_bn_relu
 from ...ops import native
 from ...ops.edge_conv import EdgeConvBlock, edge_lists
 from ...ops.knn_points import knn_points
@@ -72,8 +72,7 @@ class DGCNN(nn.Module):
                     graph = {} if lists is None else {"lists": lists}
             x = edge_conv(x, x, knn_ind, **graph)
             outputs.append(x)
-        x = self.mlp_local(torch.cat(outputs, dim=1))
-        pooled, max_indices = torch.max(x, 2)
+        pooled, max_indices = forward_points_max(self.mlp_local, torch.cat(outputs, dim=1))
         return {"feature": self.mlp_global(pooled), "max_indices": max_indices}
 
     def reset_parameters(self):

@@ -2,7 +2,7 @@
 import torch
 from torch import nn
 
-from ...nn import mlp1d_bn_relu, mlp_bn_relu
+from ...nn import forward_points_max, mlp1d_bn_relu, mlp_bn_relu
 from .._common import zero_biases
 
 __all__ = ["PointNet"]
@@ -26,6 +26,10 @@ class PointNet(nn.Module):
         """points [B,3,N], points_feature [B,C,N] or None, points_mask [B,N] bool or None
         -> {"feature": [B, out_channels], "max_indices": [B, local_channels[-1]]}."""
         x = points if points_feature is None else torch.cat([points, points_feature], dim=1)
+        if not torch.jit.is_scripting():
+            if points_mask is None:
+                pooled, max_indices = forward_points_max(self.mlp_local, x)
+                return {"feature": self.mlp_global(pooled), "max_indices": max_indices}
         x = self.mlp_local(x)
         if points_mask is not None:
             x = torch.where(points_mask.unsqueeze(1), x, torch.zeros_like(x))

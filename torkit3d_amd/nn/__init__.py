@@ -98,6 +98,12 @@ class SharedMLP(nn.Sequential):
         out = self._chain(x, pool=x.size(-1))
         return torch.max(self(x), dim=3)[0] if out is None else out
 
+    def forward_points_max(self, x):
+        """``torch.max(self(x), 2)`` for x [B, C, N]: values and places, [B, C'] each."""
+        plan = self._plan(x)
+        out = _native.mlp_max(x, *plan) if plan is not None and plan[-1] else None
+        return (out[0], out[1]) if out else torch.max(self(x), 2)
+
     def forward_grouped_max(self, feature, xyz, centre, index):
         """``self(group_points_with_xyz(feature, xyz, centre, index)).max(dim=3)[0]``, or None
         where the fused chain does not take it."""
@@ -181,6 +187,12 @@ def forward_max(mlp, x):
     if isinstance(mlp, SharedMLP):
         return mlp.forward_max(x)
     return torch.max(mlp(x), dim=3)[0]
+
+
+def forward_points_max(mlp, x):
+    if isinstance(mlp, SharedMLP):
+        return mlp.forward_points_max(x)
+    return torch.max(mlp(x), 2)
 
 
 def forward_grouped_max(mlp, feature, xyz, centre, index):
