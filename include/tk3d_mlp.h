@@ -172,9 +172,11 @@ int tk3d_mlp_mask_sums_f32(const float *g, const float *y, int B, int C, int P,
 /* z = relu(norm(y)), n rows of P values, channel = row modulo C. */
 int tk3d_mlp_activate_f32(const float *y, int64_t rows, int C, int P, const tk3d_mlp_norm *norm,
                           float *z, void *stream);
-/* dy = a e + b y + d over e itself. */
-int tk3d_mlp_grad_apply_f32(float *e, const float *y, const float *coef, int B, int C, int P,
-                            void *stream);
+/* dy = a e + b y + d over e itself, and dy rel^T, rel [B, 3, P], in partial sums [splits][C][3] (at most 2^31 - 1
+ * rows B C). */
+int tk3d_mlp_grad_apply_splits(int B, int P);
+int tk3d_mlp_grad_apply_f32(float *e, const float *y, const float *coef, const float *rel, int B, int C, int P,
+                            float *partial, void *stream);
 
 /* Backward of a pooled layer, before the products: from g [B,C,M], the extremes and their places
  * the coefficients (a, b, d'), dgamma, dbeta and sel, [B, C, M] of (float a e, int32 place in the

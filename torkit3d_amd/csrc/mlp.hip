@@ -1066,26 +1066,54 @@ __global__ void __launch_bounds__(kBlock)
     }
 }
 
+// dy = a e + b y + d over e, and its products with the three rows of rel (the coordinates that a grouping adds to a
+// layer's input) in partial sums of a workgroup: apart these read dy once more (128 channels, 131072 positions 31 +
+// 20 us, now 38).
 __global__ void __launch_bounds__(kBlock)
-    mlp_grad_apply_kernel(float *e, const float *y, const float *coef, int C, int P)
+    mlp_grad_apply_kernel(float *e, const float *y, const float *coef, const float *rel, int C, int P, int first_row,
+                          float *partial)
 {
-    const int64_t row = (int64_t)blockIdx.y * P;
-    const f32x4 k = reinterpret_cast<const f32x4 *>(coef)[blockIdx.y % C];
+    __shared__ double2 lds[kWaves], lds2[kWaves];
+    const int row = first_row + blockIdx.y, b = row / C, c = row % C;
+    const f32x4 k = reinterpret_cast<const f32x4 *>(coef)[c];
+    e += (int64_t)row * P;
+    y += (int64_t)row * P;
+    rel += (int64_t)b * 3 * P;
     const auto f = [&](float ev, float yv) {
         return __builtin_fmaf(k.x, ev, __builtin_fmaf(k.y, yv, k.z));
     };
+    float sum[3] = {0.0f, 0.0f, 0.0f};
     if ((P & 3) == 0) {
+#pragma unroll 4
         for (int i = (blockIdx.x * kBlock + threadIdx.x) * 4; i < P; i += gridDim.x * kBlock * 4) {
-            f32x4 v = *reinterpret_cast<const f32x4 *>(e + row + i);
-            const f32x4 w = *reinterpret_cast<const f32x4 *>(y + row + i);
+            f32x4 v = *reinterpret_cast<const f32x4 *>(e + i);
+            const f32x4 w = *reinterpret_cast<const f32x4 *>(y + i);
 #pragma unroll
             for (int j = 0; j < 4; ++j)
                 v[j] = f(v[j], w[j]);
-            *reinterpret_cast<f32x4 *>(e + row + i) = v;
+            *reinterpret_cast<f32x4 *>(e + i) = v;
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                const f32x4 r = *reinterpret_cast<const f32x4 *>(rel + (int64_t)d * P + i);
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    sum[d] = __builtin_fmaf(v[j], r[j], sum[d]);
+            }
         }
     } else {
-        for (int i = blockIdx.x * kBlock + threadIdx.x; i < P; i += gridDim.x * kBlock)
-            e[row + i] = f(e[row + i], y[row + i]);
+        for (int i = blockIdx.x * kBlock + threadIdx.x; i < P; i += gridDim.x * kBlock) {
+            e[i] = f(e[i], y[i]);
+#pragma unroll
+            for (int d = 0; d < 3; ++d)
+                sum[d] = __builtin_fmaf(e[i], rel[(int64_t)d * P + i], sum[d]);
+        }
+    }
+    const double2 s = block_sum(double2{sum[0], sum[1]}, lds), t = block_sum(double2{sum[2], 0.0}, lds2);
+    if (threadIdx.x == 0) {
+        float *to = partial + (((int64_t)b * gridDim.x + blockIdx.x) * C + c) * 3;
+        to[0] = (float)s.x;
+        to[1] = (float)s.y;
+        to[2] = (float)t.x;
     }
 }
 
@@ -1572,13 +1600,15 @@ int tk3d_mlp_activate_f32(const float *y, int64_t rows, int C, int P, const tk3d
     return tk_launch_status();
 }
 
-int tk3d_mlp_grad_apply_f32(float *e, const float *y, const float *coef, int B, int C, int P,
-                            void *stream)
+int tk3d_mlp_grad_apply_splits(int B, int P) { return B * row_blocks(P); }
+
+int tk3d_mlp_grad_apply_f32(float *e, const float *y, const float *coef, const float *rel, int B, int C, int P,
+                            float *partial, void *stream)
 {
     const int64_t rows = (int64_t)B * C, step = rows_at_once(C);
     for (int64_t r = 0; r < rows; r += step)
         mlp_grad_apply_kernel<<<dim3(row_blocks(P), (unsigned)(rows - r < step ? rows - r : step)), kBlock, 0,
-                                (hipStream_t)stream>>>(e + r * P, y + r * P, coef, C, P);
+                                (hipStream_t)stream>>>(e, y, coef, rel, C, P, (int)r, partial);
     return tk_launch_status();
 }
 

@@ -655,11 +655,12 @@ Grads backward(const Call &c, const Kept &k, const Tensor &g, bool want_x, bool 
         done(tk3d_group_points_concat_forward_f32(nullptr, f32(c.xyz), f32(c.centre), index, B, 0, N,
                                                   M, S, f32(rel), stream),
              "tk3d_group_points_concat_forward_f32");
-        done(tk3d_mlp_grad_apply_f32(f32(e), f32(k.y[0]), f32(coef[0]), (int)B, (int)O, (int)P,
-                                     stream),
+        const Tensor partial = at::empty({tk3d_mlp_grad_apply_splits((int)B, (int)P), O, 3}, like.options());
+        done(tk3d_mlp_grad_apply_f32(f32(e), f32(k.y[0]), f32(coef[0]), f32(rel), (int)B, (int)O, (int)P,
+                                     f32(partial), stream),
              "tk3d_mlp_grad_apply_f32");
         o.col = source(rel, nullptr, 0, 0);
-        outer(TK3D_MLP_ROW_RAW, TK3D_MLP_COL_RAW, o, like, dw + F, I, pending, stream);
+        pending_sum(partial, o, dw + F, I, pending);
         const Tensor du = at::empty({B, O, N}, like.options());
         done(tk3d_group_points_backward_f32(f32(e), index, B, O, N, M, S, f32(du), stream),
              "tk3d_group_points_backward_f32");
