@@ -112,7 +112,7 @@ int tk3d_mlp_outer_f32(int row, int col, const tk3d_mlp_outer *p, void *stream);
  * with rows of the same kind and the product's yprev as COL_ACT (COL_CENTRED behind IN_CENTRED); or one to
  * OUT_PLAIN (C0 = C), columns COL_RAW. tk3d_mlp_pair_slots: slots and splits of the partial sums, 0 where the two
  * have to be called apart (more than 128 channels, 128 from 32, rows that are not 16-byte aligned). */
-int tk3d_mlp_pair_slots(int in, const tk3d_mlp_product *p, const tk3d_mlp_outer *o);
+int tk3d_mlp_pair_slots(const tk3d_mlp_product *p, const tk3d_mlp_outer *o);
 int tk3d_mlp_pair_f32(int in, int out, const tk3d_mlp_product *p, const tk3d_mlp_outer *o, void *stream);
 
 /* out[r * ld + c] = sum over the splits of partial[r][c], rows of C, `stride` elements from one split

@@ -480,7 +480,7 @@ struct PairShape {
 // not fit in LDS twice, and 16-byte rows. At any number of positions: 128 -> 128 channels, 2048 positions 18.9
 // apart, 12.2 us together.
 bool aligned(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
-PairShape pair_shape(int in, const tk3d_mlp_product &p, const tk3d_mlp_outer &o)
+PairShape pair_shape(const tk3d_mlp_product &p, const tk3d_mlp_outer &o)
 {
     const int O = o.row.K, I = p.C;
     PairShape s{0, 0, 0, 0, 0};
@@ -505,16 +505,16 @@ PairShape pair_shape(int in, const tk3d_mlp_product &p, const tk3d_mlp_outer &o)
 
 extern "C" {
 
-int tk3d_mlp_pair_slots(int in, const tk3d_mlp_product *p, const tk3d_mlp_outer *o)
+int tk3d_mlp_pair_slots(const tk3d_mlp_product *p, const tk3d_mlp_outer *o)
 {
-    return pair_shape(in, *p, *o).grid;
+    return pair_shape(*p, *o).grid;
 }
 
 int tk3d_mlp_pair_f32(int in, int out, const tk3d_mlp_product *p, const tk3d_mlp_outer *o, void *stream_)
 {
     if (!p || !o)
         return TK3D_ERR_NULL_POINTER;
-    const PairShape s = pair_shape(in, *p, *o);
+    const PairShape s = pair_shape(*p, *o);
     if (s.grid == 0 || p->B != o->B || p->P != o->P || p->C != o->col.K || p->src[0].K != o->row.K)
         return TK3D_ERR_UNSUPPORTED;
     PairArgs a{*p, *o, s.tiles, s.total};

@@ -378,7 +378,7 @@ struct Paired {
 Paired pair(int in, int out, tk3d_mlp_product &p, tk3d_mlp_outer &o, const Tensor &like, void *stream)
 {
     Paired r;
-    r.slots = tk3d_mlp_pair_slots(in, &p, &o);
+    r.slots = tk3d_mlp_pair_slots(&p, &o);
     if (r.slots == 0)
         return r;
     r.outer = at::empty({r.slots, o.row.K, o.col.K}, like.options());
