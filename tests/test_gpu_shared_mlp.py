@@ -13,6 +13,7 @@ from torch import nn
 
 from torkit3d_amd import _native
 from torkit3d_amd.nn import SharedMLP, mlp1d_bn_relu, mlp2d_bn_relu
+from torkit3d_amd.ops.edge_conv import edge_lists
 from torkit3d_amd.ops.group_points import group_points_with_xyz
 
 pytestmark = pytest.mark.gpu
@@ -479,7 +480,7 @@ def stock_forward(mlp, x):
     (2, 15, 65, 5, 70, False), (2, 16, 64, 20, 64, False), (3, 130, 17, 3, 40, True),
 ])
 def test_edge_conv(cuda, b, c, n, k, o, lists, training):
-    from torkit3d_amd.ops.edge_conv import EdgeConvBlock, edge_lists, get_edge_feature_builtin
+    from torkit3d_amd.ops.edge_conv import EdgeConvBlock, get_edge_feature_builtin
 
     torch.manual_seed(1)
     block = EdgeConvBlock(c, [o])
@@ -560,7 +561,7 @@ def test_edge_conv_is_as_exact_as_the_stock_modules(cuda, c, o, far):
 def test_edge_conv_lists_are_checked(cuda):
     """What is not the inverse of a graph of this size is refused, and whatever such a tensor holds,
     the backward stays inside it and inside the cloud."""
-    from torkit3d_amd.ops.edge_conv import EdgeConvBlock, edge_lists
+    from torkit3d_amd.ops.edge_conv import EdgeConvBlock
 
     block = EdgeConvBlock(4, [8]).to(cuda).train()
     b, n, k = 2, 50, 6
@@ -600,3 +601,18 @@ def test_edge_conv_with_indices_outside(cuda):
     (out * weight).sum().backward()
     (ref * weight).sum().backward()
     torch.testing.assert_close(x.grad, y.grad, rtol=1e-4, atol=1e-4)
+
+
+# The inverse of a graph: several slices of a cloud and one, points without edges, a cloud whose edges all go to one
+# point, indices outside.
+@pytest.mark.parametrize("b,n,k", [(8, 2048, 20), (3, 1000, 20), (2, 32768, 4), (300, 70, 2), (1, 129, 3), (1, 1, 1)])
+def test_edge_lists(cuda, b, n, k):
+    index = torch.randint(-1, n + 1, (b, n, k), generator=torch.Generator().manual_seed(n))
+    index[0] = n // 2
+    lists = edge_lists(index.to(cuda), n).cpu()
+    for i in range(b):
+        counts = torch.bincount(index[i][(index[i] >= 0) & (index[i] < n)], minlength=n)
+        assert torch.equal(lists[i, :n + 1], torch.cat([counts.new_zeros(1), counts.cumsum(0)]).int())
+        edges = lists[i, n + 1:n + 1 + int(counts.sum())].long()
+        assert torch.equal(index[i][edges >> 8, edges & 255], torch.repeat_interleave(torch.arange(n), counts))
+        assert len(set(edges.tolist())) == len(edges)

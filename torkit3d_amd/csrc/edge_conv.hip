@@ -116,30 +116,50 @@ __global__ void __launch_bounds__(kBlock)
     }
 }
 
-// The inverse of the graph, one workgroup per batch element: start [N + 1], then the edges into
-// every point as i << 8 | k. (Their order within a point is arbitrary; the backward adds them up in
-// double.)
+// The inverse of the graph: start [N + 1], then the edges into every point as i << 8 | k. (Their order within
+// a point is arbitrary; the backward adds them up in double.) A workgroup has `own` points of a batch element and
+// looks through all its edges, counting those into lower points on the way; a thread's indices come eight at a
+// time. What bounds it are these trips to memory, and the scattered entries, 64 cache lines a store, of which
+// one workgroup per batch element had all (8 x 2048 points, 20 neighbours 43 us, now 20).
 __global__ void __launch_bounds__(1024)
-    edge_lists_kernel(const int64_t *index, int N, int K, int *lists)
+    edge_lists_kernel(const int64_t *index, int N, int K, int own, int slices, int *lists)
 {
-    extern __shared__ int cursor[];  // [N]
-    __shared__ int waves[16];
-    const int tid = threadIdx.x, edges = N * K;
-    const int64_t *row = index + (int64_t)blockIdx.x * edges;
-    int *start = lists + (int64_t)blockIdx.x * (N + 1 + edges);
+    constexpr int AT_ONCE = 8;
+    extern __shared__ int cursor[];  // [own]
+    __shared__ int waves[16], lower[16];
+    const int tid = threadIdx.x, edges = N * K, b = blockIdx.x / slices;
+    const int first = blockIdx.x % slices * own, last = min(first + own, N);
+    if (first >= N)
+        return;
+    const int64_t *row = index + (int64_t)b * edges;
+    int *start = lists + (int64_t)b * (N + 1 + edges);
     int *entries = start + N + 1;
-    for (int j = tid; j < N; j += 1024)
+    for (int j = tid; j < own; j += 1024)
         cursor[j] = 0;
     __syncthreads();
-    for (int e = tid; e < edges; e += 1024) {
-        const int64_t j = row[e];
-        if (j >= 0 && j < N)
-            atomicAdd(&cursor[(int)j], 1);
-    }
+    const auto for_edges = [&](const auto &f) {  // f(edge, point)
+        for (int e0 = tid; e0 < edges; e0 += AT_ONCE * 1024) {
+            int64_t j[AT_ONCE];
+#pragma unroll
+            for (int i = 0; i < AT_ONCE; ++i)
+                j[i] = row[e0 + i * 1024 < edges ? e0 + i * 1024 : e0];
+#pragma unroll
+            for (int i = 0; i < AT_ONCE; ++i)
+                if (e0 + i * 1024 < edges && j[i] >= 0 && j[i] < last)
+                    f(e0 + i * 1024, (int)j[i]);
+        }
+    };
+    int below = 0;
+    for_edges([&](int, int j) {
+        if (j >= first)
+            atomicAdd(&cursor[j - first], 1);
+        else
+            ++below;
+    });
     __syncthreads();
-    // exclusive prefix sums: a run of points per thread, then over the threads
-    const int run = (N + 1023) / 1024, from = tid * run < N ? tid * run : N;
-    const int to = from + run < N ? from + run : N;
+    // exclusive prefix sums: a run of points per thread, then over the threads; in front of them `below` of all
+    const int n = last - first, run = (n + 1023) / 1024, from = tid * run < n ? tid * run : n;
+    const int to = from + run < n ? from + run : n;
     int mine = 0;
     for (int j = from; j < to; ++j)
         mine += cursor[j];
@@ -148,27 +168,29 @@ __global__ void __launch_bounds__(1024)
     for (int off = 1; off < 64; off <<= 1) {
         const int other = __shfl_up(scan, off);
         scan += (tid & 63) >= off ? other : 0;
+        below += __shfl_xor(below, off);
     }
-    if ((tid & 63) == 63)
+    if ((tid & 63) == 63) {
         waves[tid >> 6] = scan;
+        lower[tid >> 6] = below;
+    }
     __syncthreads();
     int base = scan - mine;
-    for (int w = 0; w < (tid >> 6); ++w)
-        base += waves[w];
+    for (int w = 0; w < 16; ++w)
+        base += lower[w] + (w < (tid >> 6) ? waves[w] : 0);
     for (int j = from; j < to; ++j) {
         const int count = cursor[j];
         cursor[j] = base;
-        start[j] = base;
+        start[first + j] = base;
         base += count;
     }
-    if (tid == 1023)
+    if (tid == 1023 && last == N)
         start[N] = base;
     __syncthreads();
-    for (int e = tid; e < edges; e += 1024) {
-        const int64_t j = row[e];
-        if (j >= 0 && j < N)
-            entries[atomicAdd(&cursor[(int)j], 1)] = (e / K) << 8 | (e % K);
-    }
+    for_edges([&](int e, int j) {
+        if (j >= first)
+            entries[atomicAdd(&cursor[j - first], 1)] = (e / K) << 8 | (e % K);
+    });
 }
 
 // The edges into point j, as positions of the entries. (The lists come from the caller: whatever they
@@ -278,9 +300,33 @@ __global__ void __launch_bounds__(kBlock) edge_rows_kernel(const float *x, int C
     }
 }
 
+// The edges into a wave's kEach consecutive points, 64 entries of each on their way before the first is used: a lane
+// holds an entry, from which its row is read at an address of the whole wave.
+constexpr int kEach = kGather / kWaves;
+struct Edges {
+    Run run[kEach];
+    int entry[kEach];
+    __device__ __forceinline__ void request(const int *start, const int *entries, int first, int N, int K, int lane)
+    {
+#pragma unroll
+        for (int q = 0; q < kEach; ++q)
+            run[q] = edges_into(start, min(first + q, N - 1), N, K);
+#pragma unroll
+        for (int q = 0; q < kEach; ++q)
+            entry[q] = more(entries, q, 0, lane);
+    }
+    __device__ __forceinline__ int more(const int *entries, int q, int c0, int lane) const
+    {
+        return run[q].to > run[q].from ? entries[min(run[q].from + c0 + lane, run[q].to - 1)] : 0;
+    }
+};
+
 // The sums of the differences to the neighbours, out [B, 2 C, N]: s = sum of x_i - x_j over the edges
 // i -> j into a point, then t = sum of x_j - x_i over the edges out of it (x_j = 0 outside the cloud).
-// W of them lie side by side in a wave: channels of one point.
+// W of them lie side by side in a wave: channels of one point. With 64, bounds, edges and neighbours of a wave's points
+// are requested at once, and rows of both kinds go together: one behind the other they were twelve trips to memory a
+// point (8 x 2048 points, 64 channels, 20 neighbours 34 us, now 24.5; the same for edge_sparse_kernel gave nothing, nor
+// did places of a byte there, read in front of the values: 23 -> 26).
 template <int W>
 __global__ void __launch_bounds__(kBlock)
     edge_neighbours_kernel(const float *__restrict__ rows, const int64_t *__restrict__ index,
@@ -297,34 +343,88 @@ __global__ void __launch_bounds__(kBlock)
     const float *x = rows + (int64_t)b * N * C + c;
     const int *start = lists + (int64_t)b * (N + 1 + (int64_t)N * K);
     const int *entries = start + N + 1;
-    for (int local = sub; local < kGather && first + local < N; local += AT_ONCE) {
-        const int p = first + local;
-        const float own = x[(int64_t)p * C];
-        const Run run = edges_into(start, p, N, K);
-        double s = 0.0, t = 0.0;
-        for (int e0 = run.from; e0 < run.to; e0 += kAtOnce) {
-            float v[kAtOnce];
+    if constexpr (W == 64) {  // (in the same order as below, edges into and out of a point side by side)
+        Edges mine;
+        mine.request(start, entries, first + sub * kEach, N, K, lane);
+        const int64_t *neighbours = index + (int64_t)b * N * K;
+        const auto neighbour = [&](int p, int k) {
+            const int64_t j = neighbours[(int64_t)min(p, N - 1) * K + min(k, K - 1)];
+            return j >= 0 && j < N ? (int)j : -1;
+        };
+        int out_of[kEach];
+        float own[kEach];
 #pragma unroll
-            for (int i = 0; i < kAtOnce; ++i)
-                v[i] = x[(int64_t)point_of(entries[e0 + i < run.to ? e0 + i : run.to - 1], N) * C];
-#pragma unroll
-            for (int i = 0; i < kAtOnce; ++i)
-                s += e0 + i < run.to ? (double)(v[i] - own) : 0.0;
+        for (int q = 0; q < kEach; ++q) {
+            out_of[q] = neighbour(first + sub * kEach + q, lane);
+            own[q] = x[(int64_t)min(first + sub * kEach + q, N - 1) * C];
         }
-        const int64_t *neighbours = index + ((int64_t)b * N + p) * K;
-        for (int k0 = 0; k0 < K; k0 += kAtOnce) {
-            float v[kAtOnce];
 #pragma unroll
-            for (int i = 0; i < kAtOnce; ++i) {
-                const int64_t j = neighbours[k0 + i < K ? k0 + i : K - 1];
-                v[i] = j >= 0 && j < N ? x[j * C] : 0.0f;
+        for (int q = 0; q < kEach; ++q) {
+            const int local = sub * kEach + q, p = first + local;
+            if (p >= N)
+                break;
+            double s = 0.0, t = 0.0;
+            const int count = mine.run[q].to - mine.run[q].from;
+            for (int c0 = 0; c0 < max(count, K); c0 += 64) {
+                const int entry = c0 && c0 < count ? mine.more(entries, q, c0, lane) : mine.entry[q];
+                const int near = c0 && c0 < K ? neighbour(p, c0 + lane) : out_of[q];
+                const int n = min(count - c0, 64), m = min(K - c0, 64);
+                for (int e0 = 0; e0 < max(n, m); e0 += kAtOnce) {
+                    float v[kAtOnce], u[kAtOnce];
+                    if (e0 < n)
+#pragma unroll
+                        for (int i = 0; i < kAtOnce; ++i)
+                            v[i] = x[(int64_t)point_of(__builtin_amdgcn_readlane(entry, min(e0 + i, n - 1)), N) * C];
+                    if (e0 < m)
+#pragma unroll
+                        for (int i = 0; i < kAtOnce; ++i) {
+                            const int j = __builtin_amdgcn_readlane(near, min(e0 + i, m - 1));
+                            u[i] = x[(int64_t)max(j, 0) * C];
+                            u[i] = j >= 0 ? u[i] : 0.0f;
+                        }
+                    if (e0 < n)
+#pragma unroll
+                        for (int i = 0; i < kAtOnce; ++i)
+                            s += e0 + i < n ? (double)(v[i] - own[q]) : 0.0;
+                    if (e0 < m)
+#pragma unroll
+                        for (int i = 0; i < kAtOnce; ++i)
+                            t += e0 + i < m ? (double)(u[i] - own[q]) : 0.0;
+                }
             }
-#pragma unroll
-            for (int i = 0; i < kAtOnce; ++i)
-                t += k0 + i < K ? (double)(v[i] - own) : 0.0;
+            into[lane][local] = (float)s;
+            from[lane][local] = (float)t;
         }
-        into[lane][local] = (float)s;
-        from[lane][local] = (float)t;
+    } else {
+        for (int local = sub; local < kGather && first + local < N; local += AT_ONCE) {
+            const int p = first + local;
+            const float own = x[(int64_t)p * C];
+            const Run run = edges_into(start, p, N, K);
+            double s = 0.0, t = 0.0;
+            for (int e0 = run.from; e0 < run.to; e0 += kAtOnce) {
+                float v[kAtOnce];
+#pragma unroll
+                for (int i = 0; i < kAtOnce; ++i)
+                    v[i] = x[(int64_t)point_of(entries[e0 + i < run.to ? e0 + i : run.to - 1], N) * C];
+#pragma unroll
+                for (int i = 0; i < kAtOnce; ++i)
+                    s += e0 + i < run.to ? (double)(v[i] - own) : 0.0;
+            }
+            const int64_t *neighbours = index + ((int64_t)b * N + p) * K;
+            for (int k0 = 0; k0 < K; k0 += kAtOnce) {
+                float v[kAtOnce];
+#pragma unroll
+                for (int i = 0; i < kAtOnce; ++i) {
+                    const int64_t j = neighbours[k0 + i < K ? k0 + i : K - 1];
+                    v[i] = j >= 0 && j < N ? x[j * C] : 0.0f;
+                }
+#pragma unroll
+                for (int i = 0; i < kAtOnce; ++i)
+                    t += k0 + i < K ? (double)(v[i] - own) : 0.0;
+            }
+            into[lane][local] = (float)s;
+            from[lane][local] = (float)t;
+        }
     }
     __syncthreads();
     for (int e = tid; e < W * kGather; e += kBlock) {
@@ -703,7 +803,13 @@ int tk3d_mlp_edge_lists(const int64_t *index, int B, int N, int K, int32_t *list
     const int rc = tk_allow_dynamic_lds<edge_lists_kernel>(32768 * 4);
     if (rc != TK3D_OK)
         return rc;
-    edge_lists_kernel<<<B, 1024, N * 4, (hipStream_t)stream>>>(index, N, K, lists);
+    // eight slices of a batch element, as long as every workgroup has a CU and 64 points
+    int slices = tk_cu_count() / B;
+    slices = slices > 8 ? 8 : slices;
+    slices = slices > N / 64 ? N / 64 : slices;
+    slices = slices < 1 ? 1 : slices;
+    const int own = (N + slices - 1) / slices;
+    edge_lists_kernel<<<B * slices, 1024, own * 4, (hipStream_t)stream>>>(index, N, K, own, slices, lists);
     return tk_launch_status();
 }
 
