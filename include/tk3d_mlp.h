@@ -111,7 +111,8 @@ int tk3d_mlp_outer_f32(int row, int col, const tk3d_mlp_outer *p, void *stream);
  * K = R output channels to C input channels) or IN_CENTRED (K = R = C) to OUT_MASK, and the weight gradient
  * with rows of the same kind and the product's yprev as COL_ACT (COL_CENTRED behind IN_CENTRED); or one to
  * OUT_PLAIN (C0 = C), columns COL_RAW. tk3d_mlp_pair_slots: slots and splits of the partial sums, 0 where the two
- * have to be called apart (more than 128 channels, 128 from 32, rows that are not 16-byte aligned). */
+ * have to be called apart (more than 128 channels, 128 from 32, rows that are not 16-byte aligned, channels by
+ * positions beyond 32-bit byte offsets). */
 int tk3d_mlp_pair_slots(const tk3d_mlp_product *p, const tk3d_mlp_outer *o);
 int tk3d_mlp_pair_f32(int in, int out, const tk3d_mlp_product *p, const tk3d_mlp_outer *o, void *stream);
 

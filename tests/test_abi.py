@@ -184,3 +184,34 @@ def test_chamfer_clouds_are_copied_where_it_pays(lib, b, n1, n2, channels_first,
         padded = sum((n + 3) // 4 * 4 for n in sizes)
         want = b * padded * 12 if copied else 0
         assert fn(i64(b), i64(sizes[0]), i64(sizes[1]), ctypes.c_int(channels_first)) == want
+
+
+# The kernel's byte offsets within a batch element are 32-bit: (channels + 8) * positions up to 2^29, as in the
+# products on their own. No pointer is read.
+@pytest.mark.parametrize("rows,columns,positions,taken", [
+    (128, 128, 3947580, True), (128, 128, 3947584, False), (16, 128, 3947584, False), (128, 64, 3947584, False),
+    (16, 16, 3947584, True), (16, 16, 22369620, True), (16, 16, 22369624, False), (128, 128, 2**31 - 4, False),
+    (128, 128, 2046, False), (129, 64, 64, False), (64, 129, 64, False), (128, 32, 64, False), (32, 128, 64, True)])
+def test_layers_whose_two_gradients_share_a_launch(lib, rows, columns, positions, taken):
+    pointer, i32 = ctypes.c_void_p, ctypes.c_int32
+
+    class Source(ctypes.Structure):
+        _fields_ = [(n, pointer) for n in ("x", "y", "coef", "w")] + [("batch_stride", ctypes.c_int64)] + [
+            (n, i32) for n in ("K", "wk", "wc")]
+
+    class Norm(ctypes.Structure):
+        _fields_ = [(n, pointer) for n in ("mean", "var", "gamma", "beta")] + [("eps", ctypes.c_float)]
+
+    class Product(ctypes.Structure):
+        _fields_ = [("src", Source * 2), ("in_norm", Norm), ("out_norm", Norm)] + [
+            (n, pointer) for n in ("out", "out2", "yprev", "bias", "add", "partial")] + [
+            (n, i32) for n in ("B", "C", "C0", "P", "group", "M")]
+
+    class Outer(ctypes.Structure):
+        _fields_ = [("row", Source), ("col", Source), ("row_norm", Norm), ("col_norm", Norm),
+                    ("partial", pointer), ("rowsum", pointer), ("B", i32), ("P", i32)]
+
+    product, outer = Product(B=1, C=columns, C0=columns, P=positions), Outer(B=1, P=positions)
+    product.src[0].K = outer.row.K = rows
+    outer.col.K = columns
+    assert (lib.tk3d_mlp_pair_slots(ctypes.byref(product), ctypes.byref(outer)) > 0) is taken

@@ -99,7 +99,7 @@ __global__ void __launch_bounds__(kPairBlock) mlp_pair_kernel(PairArgs a)
         at = pos < P ? pos : P - 4;
         return pos < P;
     };
-    const auto row_of = [&](int r, int rows, int at) {  // (32-bit byte offsets: indexable() of the caller)
+    const auto row_of = [&](int r, int rows, int at) {  // (32-bit byte offsets, see pair_shape)
         return ((unsigned)(r < rows ? r : rows - 1) * (unsigned)P + (unsigned)at) * 4u;
     };
     // Rows and positions past the last ones are zero, so that nothing comes of them.
@@ -477,14 +477,15 @@ struct PairShape {
 };
 
 // The tiles of a layer, or {0}: up to 128 channels on either side, except 128 from 32, whose gradient does
-// not fit in LDS twice, and 16-byte rows. At any number of positions: 128 -> 128 channels, 2048 positions 18.9
-// apart, 12.2 us together.
+// not fit in LDS twice, 16-byte rows, and 32-bit byte offsets within a batch element. At any number of positions:
+// 128 -> 128 channels, 2048 positions 18.9 apart, 12.2 us together.
 bool aligned(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 PairShape pair_shape(const tk3d_mlp_product &p, const tk3d_mlp_outer &o)
 {
     const int O = o.row.K, I = p.C;
     PairShape s{0, 0, 0, 0, 0};
     if (O > 128 || I > 128 || p.P % 4 != 0 || p.B <= 0 || p.P <= 0 ||
+        !tk_fits(1 << 29, (O > I ? O : I) + 8, p.P) ||
         !aligned(p.src[0].x) || !aligned(p.src[0].y) || !aligned(p.out) || !aligned(p.yprev) || !aligned(p.add) ||
         !aligned(o.col.x) || p.src[0].batch_stride % 4 != 0 || o.col.batch_stride % 4 != 0)
         return s;
