@@ -222,7 +222,7 @@ def test_points_at_infinity(cuda):
 
 # ---- 513 to 16384 points, 256 samples or more: the kernel that lays the points out by region
 # (Morton order), skips the blocks a new centre cannot reach and accepts from a candidate per
-# group of lanes. The lane order is no longer the reference's priority order there, so ties are
+# lane's blocks. The lane order is no longer the reference's priority order there, so ties are
 # resolved explicitly. ----
 
 def _region_cloud(kind, g, b, n):
@@ -332,7 +332,7 @@ def test_shapes_the_reference_author_profiled(cuda, b, n, k):
     np.testing.assert_array_equal(run(pts, k, cuda), oracle.sample_farthest_points(pts.numpy(), k))
 
 
-# ---- 513 points or more and 256 samples or more: one candidate per group of lanes ----
+# ---- 192 samples or more: the points of a band below the largest minimum ----
 
 @pytest.mark.parametrize("n,k", [(513, 256), (1024, 1024), (2048, 256), (2049, 1025), (4096, 257),
                                  (8192, 1024), (8193, 511), (8193, 512), (16384, 1025)])
@@ -389,3 +389,38 @@ def test_claims_of_many_clouds(cuda):
     which = torch.arange(256) * 5 % len(kinds)
     got = run(kinds[which].contiguous(), 256, cuda)
     np.testing.assert_array_equal(got, want[which.numpy()])
+
+
+@pytest.mark.parametrize("n,k", [(192, 192), (200, 191), (512, 192), (1000, 999), (1024, 512), (1025, 192),
+                                 (2049, 600), (4097, 700)])
+@pytest.mark.parametrize("kind", ["uniform", "lattice", "coarse_lattice", "tail", "overflow", "outliers",
+                                  "denormal", "equidistant", "steps"])
+def test_bands_of_every_kind(cuda, n, k, kind):
+    # bands that hold too many points or none again and again (minima spread over many powers of two,
+    # jumps between them, infinite ones), more points at the largest minimum than are judged at once,
+    # minima that end at zero, and the smallest and largest cloud of a launch shape
+    g = gen(n + 3 * k)
+    if kind == "tail":
+        pts = torch.randn(2, n, 3, generator=g) ** 7
+    elif kind == "overflow":         # squares beyond the largest float: infinite distances, all equal
+        pts = (torch.rand(2, n, 3, generator=g) - 0.5) * 4e20
+    elif kind == "outliers":         # a few far away at scales of their own, the rest in a small cube
+        pts = torch.rand(2, n, 3, generator=g) * 1e-3
+        pts[:, 5:45] = torch.randn(2, 40, 3, generator=g) * torch.logspace(-2, 12, 40)[:, None]
+    elif kind == "denormal":
+        pts = torch.rand(2, n, 3, generator=g) * 3e-21
+    elif kind == "equidistant":      # unit vectors around point 0: every minimum is 1 after one step
+        pts = torch.zeros(2, n, 3)
+        axis = torch.randint(0, 3, (2, n), generator=g)
+        sign = torch.randint(0, 2, (2, n), generator=g) * 2.0 - 1.0
+        pts.scatter_(2, axis[:, :, None], sign[:, :, None])
+        pts[:, 0] = 0.0
+    elif kind == "steps":            # on a line, gaps that halve: a new scale at every step
+        pts = torch.zeros(2, n, 3)
+        pts[:, :, 0] = 2.0 ** -(torch.arange(n) % 60).float()
+    else:
+        pts = _region_cloud(kind, g, 2, n - n % 2)
+        pts = torch.cat([pts, pts[:, : n % 2]], dim=1)
+    want = oracle.sample_farthest_points(pts.numpy(), k)
+    np.testing.assert_array_equal(run(pts, k, cuda), want)
+    np.testing.assert_array_equal(run(pts.transpose(1, 2).contiguous(), k, cuda, True), want)

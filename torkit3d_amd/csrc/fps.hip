@@ -22,6 +22,8 @@
 // laid out here in exactly that priority order ("positions"), lanes take
 // consecutive positions, and every reduction keeps the lowest position among
 // equal values, which reproduces the reference's choice.
+#include <type_traits>
+
 #include "tk3d_common.h"
 
 namespace {
@@ -506,81 +508,118 @@ constexpr int64_t FPS_CLAIM = -2;   // the cloud looks as if in sampling order: 
 constexpr int64_t FPS_BROKEN = -3;  // it is not
 constexpr int FPS_CLAIM_MAX = 1024;
 
-// The largest and the second-largest running minimum (bits) of some of a lane's points, and
-// the point that holds the largest.
-struct FpsTop {
-    int m, s;
-    float x, y, z;
-    int p;
-};
-
 __device__ __forceinline__ int fps_max(int a, int b) { return a > b ? a : b; }
 __device__ __forceinline__ int fps_min(int a, int b) { return a < b ? a : b; }
 
-// (the left one stays among equals: a tie shows as s == m and is settled elsewhere)
-__device__ __forceinline__ FpsTop fps_merge(const FpsTop &a, const FpsTop &b, bool leaves)
+// Place of the cell (x, y, z) of a 16^3 grid along a Hilbert curve (J. Skilling, "Programming the
+// Hilbert curve", AIP Conference Proceedings 707, 2004).
+__device__ __forceinline__ unsigned fps_hilbert(unsigned x, unsigned y, unsigned z)
 {
-    const bool right = b.m > a.m;
-    FpsTop o;
-    o.m = fps_max(a.m, b.m);
-    o.s = fps_min(a.m, b.m);
-    if (!leaves)
-        o.s = fps_max(o.s, fps_max(a.s, b.s));
-    o.x = right ? b.x : a.x;
-    o.y = right ? b.y : a.y;
-    o.z = right ? b.z : a.z;
-    o.p = right ? b.p : a.p;
-    return o;
+    unsigned c[3] = {x, y, z};
+#pragma unroll
+    for (unsigned q = 8u; q > 1u; q >>= 1) {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            const bool flip = (c[a] & q) != 0u;
+            const unsigned swap = flip ? 0u : (c[0] ^ c[a]) & (q - 1u);
+            c[0] ^= flip ? q - 1u : swap;
+            c[a] ^= swap;
+        }
+    }
+    c[1] ^= c[0];
+    c[2] ^= c[1];
+    unsigned gray = 0u;
+#pragma unroll
+    for (unsigned q = 8u; q > 1u; q >>= 1)
+        gray ^= (c[2] & q) != 0u ? q - 1u : 0u;
+    unsigned place = 0u;
+#pragma unroll
+    for (int b = 3; b >= 0; --b) {
+#pragma unroll
+        for (int a = 0; a < 3; ++a)
+            place = 2u * place + (((c[a] ^ gray) >> b) & 1u);
+    }
+    return place;
 }
 
-// fp32 kernel for clouds of 513 to 16384 points: several selection steps per exchange as in the
-// multi-step kernel above, with the points laid out by region, so that an update only visits the
-// points a new centre can reach, and with one candidate from each of 64 (GM = 2: 128) groups of
-// lanes, so that an exchange has many candidates to accept from.
+// Adds to a counter in LDS, lane by lane, and returns what it held before. (As an atomicAdd the
+// compiler turns it into a scan over the lanes, for a handful of which it is.)
+__device__ __forceinline__ int fps_lds_add(int *counter, int v)
+{
+    int before;
+    const unsigned at = (unsigned)(size_t)(__attribute__((address_space(3))) int *)counter;
+    asm volatile("ds_add_rtn_u32 %0, %1, %2\n\ts_waitcnt lgkmcnt(0)"
+                 : "=v"(before)
+                 : "v"(at), "v"(v)
+                 : "memory");
+    return before;
+}
+
+// Appends the lane's bit of a mask to a number: 2 bits + (mask >> lane & 1), in one instruction.
+__device__ __forceinline__ unsigned fps_append(unsigned bits, unsigned long long mask)
+{
+    asm("v_addc_co_u32_e64 %0, vcc, %0, %0, %1" : "+v"(bits) : "s"(mask) : "vcc");
+    return bits;
+}
+
+// Width of a band for `target` points where one of width `was` held n. (Any number will do, as long as
+// all waves have the same; a wave-uniform result.)
+__device__ __forceinline__ int fps_band(int was, float target, int n)
+{
+    const float w = (float)was * (target * __builtin_amdgcn_rcpf((float)n));
+    return __builtin_amdgcn_readfirstlane((int)__builtin_fmaxf(__builtin_fminf(w, 1e9f), 1.0f));
+}
+
+// fp32 kernel for clouds of up to 16384 points: dozens of selection steps per exchange between the
+// waves, with the points laid out by region, so that an update only visits the points a new centre
+// can reach.
 //
-// Update. Every running minimum is at most tau, the value of the last exchange's first winner (it
-// was the largest of them all, and minima only shrink), so a centre can lower a point's minimum
-// only if it lies within sqrt(tau) of it - a ball that shrinks as the sampling proceeds. The
-// prologue sorts the points along a Morton curve (a counting sort by cell in LDS) and cuts the
-// sequence into 4 NW regions; region R goes to wave R % NW as block R / NW of the lanes' registers
-// (P / 4 points per lane and block), so neighbouring regions sit on different SIMDs. Lane (a, q)
-// evaluates the canonical distance from winner a to the box of block q - the same rounded
-// operations as tk_dist2 on the per-axis gaps, each of which is monotone, so the result is a lower
-// bound of the canonical distance to every point of the box - and a block is updated only if that
-// bound is below tau. Skipping is therefore exact. A wave none of whose blocks is reached leaves
-// its candidates as they are.
+// Band. With an upper bound `base` of all minima, the points whose running minimum lies above
+// theta = base - step are listed in LDS, at most 64, a lane each; every other point is at or below
+// theta. So as long as the steps' maxima stay above theta, the coming winners are found among the
+// listed points alone: in order of (minimum, position), a listed point is a winner unless an earlier
+// winner lies nearer to it than its minimum. Such a point falls to that distance, nearly always
+// below theta (its neighbour in the same hole was taken); where it stays above, the list counts only
+// down to that distance, `stop`, which takes theta's place. After the exchange nothing is above `stop`:
+// the next `base`. The band's width follows the last one's (40 points are aimed at, 20 to 64 come):
+// too many or none, and the points are listed again with another width, in two consecutive bands of
+// that kind with the largest minimum looked for as well. 457 -> 139 exchanges at 16384 -> 4096, 155 -> 53
+// at 4096 -> 1024, against a candidate from each of 128 groups of lanes and a list of sixteen.
 //
-// Candidates. A group is GL = NW / GM neighbouring lanes of a wave (its points are a quarter, an
-// eighth, ... of each of the wave's blocks), because GL lanes agree on their largest and second-
-// largest minimum in log2(GL) DPP steps for all groups of the wave at once, and the lane that holds
-// the largest has its coordinates at hand: no walk, no scalar unit. The kernel before this one had a
-// candidate per wave: 4.4 winners an exchange of sixteen candidates, where 64 groups give 7.5 and
-// 128 groups 8.8 (16384 -> 4096, uniform), and an exchange costs hardly more.
+// Judgement. Eight waves take eight listed points each and compare them with all 64 lanes: which
+// come after, which of these are nearer than their minimum, a bit each, appended lane by lane with
+// an add-with-carry. From the other waves' bits in LDS every wave then has, for its lane's point, the
+// earlier points that would knock it out, and settles all of them in a few turns: a point none of whose
+// opponents is undecided or a winner is a winner, one with a winner among them is out. (The list
+// needs no order: a winner's turn is the number of winners before it.)
 //
-// Judgement. A candidate above every group's second-largest minimum is listed (at most sixteen are,
-// the upper ones); four waves, one per SIMD and at raised priority, compare four listed candidates
-// each with all of them. Candidates in order of (value, position) are the winners of the following
-// steps up to the first that an earlier one lies nearer to than its value: their updates leave it
-// alone, and everything not listed is below it. They meet in LDS, by order, behind a second barrier.
+// Update. A winner with minimum v lowers minima only within sqrt(v) of itself, since no minimum is
+// larger at its step. The prologue sorts the points along a Hilbert curve (a counting sort by cell in
+// LDS) and cuts the sequence into NB NW regions; region R goes to wave R % NW as block R / NW of the
+// lanes' registers (P / NB points per lane and block). A lane evaluates the canonical distance from
+// its point to the box of every block of the wave - the same rounded operations as tk_dist2 on the per-axis
+// gaps, each of which is monotone, so the result is a lower bound of the canonical distance to every point
+// of the box - and a winner updates a block only if that bound is below v. Skipping is therefore
+// exact. (Along a Morton curve, whose runs jump, a winner reached 6.9 of 64 blocks and the busiest wave
+// had 22.8 of an exchange's visits; now 4.2 and 9.5.)
 //
-// Ties. The lane order is not the reference's priority order (see the top of the file), so equal
-// maxima are resolved explicitly. A group that holds its maximum more than once puts up the point
-// with the lowest reference position and counts as second-largest what the others will be once that
-// one is chosen (copies of a point vanish with it); if the largest minimum of all is still held twice
-// in a group, the candidates in front of the second holder's position are listed. Lattices take
-// several steps per exchange this way: 8 x 4096 -> 1024 on one of 9 x 9 x 9 points 1.61 -> 0.33 ms.
+// Ties. Equal minima are ordered by the reference's positions (see the top of the file), looked up only
+// where two listed minima are equal. Where more than 64 points share the largest minimum, the band is
+// the part of them below a position that moves up. Lattices take many steps per exchange this way: 16 x
+// 4096 -> 1024 on one of 9 x 9 x 9 points 0.35 -> 0.19 ms.
 //
-// What bounds it: one workgroup has one compute unit, and an exchange is a chain of short phases
-// (clocks at 4096 -> 1024, 8 waves, of 4100: update 1230 on average and 1880 in the slowest wave,
-// group maxima 300, judgement 1070, both with the trips through LDS; winners against boxes 600). A
-// lone wave issues an instruction every 6 clocks, two waves on a SIMD one every 4.6 together, so what
-// counts is the number of instructions on the chain. Measured (ms, before: the kernels with a
-// candidate per wave; both with what runs behind them): 8 x 16384 -> 4096 1.87 -> 1.35, 8 x 16384 ->
-// 2048 on a noisy sphere 0.95 -> 0.69, 16 x 8192 -> 2048 0.85 -> 0.58, 16 x 4096 -> 1024 0.39 -> 0.29,
-// 16 x 2048 -> 512 0.185 -> 0.155, 1 x 1024 -> 512 0.140 -> 0.117. Tried: every wave judging by itself
-// without the second barrier (1100 clocks of instructions in every wave instead of 850 in four: 16 x
-// 4096 -> 1024 0.37), blocks of half the size (0.33 for 0.29), no regions for up to 2048 points (8 %
-// faster at 1024 points in random order, three times slower on lattices).
+// What bounds it: one workgroup has one compute unit, and an exchange is a chain of short phases (clocks
+// at 16 x 4096 -> 1024, 16 waves, of 6700 for 19 winners: listing 1100, judgement 1700, resolving and
+// turns 800, update 1540 on average and 2050 in the slowest wave, with the boxes; the rest is waiting at the
+// barriers, and 14 of 67 bands are listed again). Measured (us; before: a candidate per group; both
+// with what runs behind them): 8 x 16384 -> 4096 1390-1450 -> 590, on a noisy sphere 1120-1200 -> 560,
+// in clusters 1180-1330 -> 700-730; 16 x 8192 -> 2048 590 -> 285; 16 x 4096 -> 1024 285 -> 160; 16 x 2048 -> 512
+// 160 -> 97; 1 x 1024 -> 512 120 -> 76; on lattices, copies and a line 0.2 to 0.9 of the time before.
+// Tried: listing up to 256 and judging the upper 64 (0 to 5 % faster up to 8192 points, 4 % slower
+// at 16384, lattices 10 % slower), aiming at 28, 34, 56 or 80 points, blocks of half and twice the
+// size and half as many waves with twice the points (all slower by 2 to 20 % at the sizes where another
+// instance is used), a point's names and the loop's boxes kept in registers (they went to scratch: 2.1 times the
+// time at 16384).
 //
 // A cloud that is itself a farthest point sample, in sampling order from its point 0 (the next level
 // of a PointNet++ encoder), has 0, 1, 2, ... as its answer. Where point 1 is the point farthest from
@@ -589,33 +628,33 @@ __device__ __forceinline__ FpsTop fps_merge(const FpsTop &a, const FpsTop &b, bo
 // chip; the instance with LAST behind them writes the answer, or does the work if the claim was wrong.
 // (A cloud in random order passes the test of point 1 once in n, and then takes twice the time: with that
 // test alone 256 x 2048 -> 512 took 330 us for 177 in one batch of eight. Point 2 is looked at behind it.)
-template <int P, int NW, int GM, bool SOA, bool LAST>
-__device__ __forceinline__ void fps_groups(const float *__restrict__ pts, int64_t *__restrict__ out,
+template <int P, int NW, int NB, bool SOA, bool LAST>
+__device__ __forceinline__ void fps_band(const float *__restrict__ pts, int64_t *__restrict__ out,
                                            const FpsLayout &L, bool claims)
 {
-    constexpr int NB = 4, NT = NW * TK_WAVE, PB = P / NB, S = NT * P, RS = TK_WAVE * PB;
-    constexpr int GL = NW / GM, GW = TK_WAVE / GL;  // lanes of a group, groups of a wave
-    constexpr int G = NW * GW;                      // 64 GM groups in all
-    constexpr int MAXM = 16;                        // candidates judged at once
-    constexpr int NJ = 4;                           // waves that judge
+    constexpr int NT = NW * TK_WAVE, PB = P / NB, S = NT * P, RS = TK_WAVE * PB;
+    constexpr int LIST = TK_WAVE;                   // points judged at once, a lane each
+    constexpr int QUAD = P < 4 ? P : 4;
+    constexpr float TARGET = 40.0f;                 // points a band is meant to hold
+    constexpr int NJ = NW < 8 ? NW : 8;             // waves that judge
+    constexpr int RJ = TK_WAVE / NJ;                // points for which each of them does
+    constexpr int RJ_LOG2 = RJ == 8 ? 3 : 4;
+    using Piece = typename std::conditional<RJ == 8, unsigned char, unsigned short>::type;
+    struct Relation {  // of a listed point to the others, a bit each
+        Piece before[NJ];  // is before it
+        Piece hit[NJ];     // and nearer to it than its minimum
+    };
     constexpr int CELLS = 4096;                     // 16^3 cells for the sort
-    constexpr bool BOX_IN_LDS = P * NW >= 256;      // (the registers are full)
-    static_assert((P & (P - 1)) == 0 && P % NB == 0 && G == TK_WAVE * GM && NW >= NJ, "shape");
-    static_assert(GL == 2 || GL == 4 || GL == 8 || GL == 16, "groups");
-    static_assert(CELLS % NT == 0 && S < (1 << 19), "sort");
-    constexpr int F32_INF = 0x7f800000;
+    static_assert((P & (P - 1)) == 0 && P % NB == 0 && (NW & (NW - 1)) == 0 && NW >= 4, "shape");
+    static_assert(CELLS % NT == 0 && S < (1 << 19) && S >= 8 * LIST && P % QUAD == 0, "sort");
     constexpr int F32_NEG1 = (int)0xbf800000;
-    extern __shared__ __align__(16) unsigned char fps_groups_lds[];
-    unsigned *const keys = reinterpret_cast<unsigned *>(fps_groups_lds);  // [S] points, sorted
+    extern __shared__ __align__(16) unsigned char fps_band_lds[];
+    unsigned *const keys = reinterpret_cast<unsigned *>(fps_band_lds);  // [S] points, sorted
     unsigned *const cnt = keys + S;                                       // [CELLS + 1]
-    __shared__ float4 s_cand[G];         // a group's candidate: x, y, z, running minimum (bits)
-    __shared__ int2 s_aux[G];            // the group's second-largest minimum, the candidate
-    __shared__ int s_next[G];            // position of the next point with the same minimum
-    __shared__ float4 s_list[NJ][MAXM];  // the listed candidates, a copy for every judge
-    __shared__ int s_name[NJ][MAXM];     // which points those are
-    __shared__ float4 s_win[MAXM];       // the same in order
-    __shared__ int2 s_ent[MAXM];         // the exchange's number * 2 + (it is a winner), the point
-    __shared__ float4 s_box[NW][NB][2];  // lo, hi of a wave's block
+    __shared__ float4 s_cand[LIST + 1];  // the band's points: x, y, z, running minimum (bits)
+    __shared__ int s_name[LIST + 1];     // which points those are
+    __shared__ __align__(16) Relation s_rel[LIST];
+    __shared__ int s_count[3], s_stop[3], s_most[3];
     __shared__ float s_red[NW][8];
 
     const int tid = threadIdx.x;
@@ -653,9 +692,8 @@ __device__ __forceinline__ void fps_groups(const float *__restrict__ pts, int64_
             hi[a] = __builtin_fmaxf(hi[a], own[a][k]);
             odd |= !(own[a][k] - own[a][k] == 0.0f);
         }
-        if constexpr (!LAST)
-            far = __builtin_fmaxf(far, tk_dist2<float>(own[0][k], own[1][k], own[2][k], p0[0],
-                                                       p0[1], p0[2]));
+        far = __builtin_fmaxf(far, tk_dist2<float>(own[0][k], own[1][k], own[2][k], p0[0], p0[1],
+                                                   p0[2]));
     }
     far = wave_max<float>(far);
     odd = __builtin_amdgcn_ballot_w64(odd) != 0ull;
@@ -674,15 +712,17 @@ __device__ __forceinline__ void fps_groups(const float *__restrict__ pts, int64_
     }
     for (int i = tid; i <= CELLS; i += NT)
         cnt[i] = 0u;
+    if (tid < 3)
+        s_count[tid] = s_stop[tid] = s_most[tid] = 0;
     __syncthreads();
-    if constexpr (!LAST) {
-        float reached = 0.0f;
-        bool any_odd = false;
+    float reached = 0.0f;
+    bool any_odd = false;
 #pragma unroll
-        for (int w = 0; w < NW; ++w) {
-            reached = __builtin_fmaxf(reached, s_red[w][6]);
-            any_odd |= s_red[w][6] < 0.0f;
-        }
+    for (int w = 0; w < NW; ++w) {
+        reached = __builtin_fmaxf(reached, s_red[w][6]);
+        any_odd |= s_red[w][6] < 0.0f;
+    }
+    if constexpr (!LAST) {
         const float p1[3] = {fps_coord<SOA>(pts, L.n, 1, 0), fps_coord<SOA>(pts, L.n, 1, 1),
                              fps_coord<SOA>(pts, L.n, 1, 2)};
         bool claim = claims && !any_odd &&
@@ -700,12 +740,12 @@ __device__ __forceinline__ void fps_groups(const float *__restrict__ pts, int64_
             if (lane == 0)
                 s_red[wave][7] = far;
             __syncthreads();
-            reached = 0.0f;
+            float both = 0.0f;
 #pragma unroll
             for (int w = 0; w < NW; ++w)
-                reached = __builtin_fmaxf(reached, s_red[w][7]);
+                both = __builtin_fmaxf(both, s_red[w][7]);
             claim = from_both(fps_coord<SOA>(pts, L.n, 2, 0), fps_coord<SOA>(pts, L.n, 2, 1),
-                              fps_coord<SOA>(pts, L.n, 2, 2)) >= reached;
+                              fps_coord<SOA>(pts, L.n, 2, 2)) >= both;
         }
         if (any_odd || claim) {  // uniform over the workgroup
             if (tid == 0) {
@@ -731,11 +771,6 @@ __device__ __forceinline__ void fps_groups(const float *__restrict__ pts, int64_
     // ---- the points in the order of their cells along a Morton curve; slots beyond the cloud
     // last. A counting sort: any order that keeps neighbours together is a valid layout, so 16
     // steps per axis are enough and the order within a cell is whatever the atomics give. ----
-    auto spread = [](unsigned v) {  // 4 bits -> every third bit
-        v = (v | (v << 4)) & 0x0c3u;
-        v = (v | (v << 2)) & 0x249u;
-        return v;
-    };
     unsigned where[P];  // cell, and the point's turn within it from bit 13
 #pragma unroll
     for (int k = 0; k < P; ++k) {
@@ -748,7 +783,7 @@ __device__ __forceinline__ void fps_groups(const float *__restrict__ pts, int64_
                 // (a NaN or an out-of-range value lands in cell 0 or 15)
                 c3[a] = (unsigned)(int)__builtin_fminf(__builtin_fmaxf(f, 0.0f), 15.0f);
             }
-            cell = spread(c3[0]) | (spread(c3[1]) << 1) | (spread(c3[2]) << 2);
+            cell = fps_hilbert(c3[0], c3[1], c3[2]);
         }
         where[k] = cell | (atomicAdd(&cnt[cell], 1u) << 13);
     }
@@ -812,70 +847,249 @@ __device__ __forceinline__ void fps_groups(const float *__restrict__ pts, int64_
 #pragma unroll
     for (int p = 0; p < P; ++p) {
         z[p] = plane1[name_of(lane, p)];
-        t[p] = (int)keys[name_of(lane, p)] < L.n ? F32_INF : F32_NEG1;
     }
-    // boxes of the wave's blocks (an empty block gets an empty box: never reached)
+    // ---- minima after point 0, boxes of the wave's blocks (an empty block gets an empty box: never
+    // reached), wave-uniform ----
+    float box[NB][6];
 #pragma unroll
     for (int q = 0; q < NB; ++q) {
         float bl[3] = {INF, INF, INF}, bh[3] = {-INF, -INF, -INF};
 #pragma unroll
         for (int u = 0; u < PB; ++u) {
             const int p = q * PB + u;
-            const bool ok = t[p] == F32_INF;
+            const bool ok = name_of(lane, p) < L.n;  // (the slots beyond the cloud come last)
             const float v[3] = {x[p], y[p], z[p]};
 #pragma unroll
             for (int a = 0; a < 3; ++a) {
                 bl[a] = __builtin_fminf(bl[a], ok ? v[a] : INF);
                 bh[a] = __builtin_fmaxf(bh[a], ok ? v[a] : -INF);
             }
+            const float d = tk_dist2<float>(x[p], y[p], z[p], p0[0], p0[1], p0[2]);
+            t[p] = ok ? __builtin_bit_cast(int, d) : F32_NEG1;
         }
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
-            bl[a] = -wave_max<float>(-bl[a]);
-            bh[a] = wave_max<float>(bh[a]);
-        }
-        if (lane == 0) {
-            s_box[wave][q][0] = make_float4(bl[0], bl[1], bl[2], 0.0f);
-            s_box[wave][q][1] = make_float4(bh[0], bh[1], bh[2], 0.0f);
+            box[q][a] = -wave_max<float>(-bl[a]);
+            box[q][3 + a] = wave_max<float>(bh[a]);
         }
     }
-    if (tid < MAXM)
-        s_ent[tid] = make_int2(-1, 0);
-    __syncthreads();  // the boxes are written
-    // After an exchange lane (a, q) = (lane / 4, lane % 4) stands for candidate a of the list and
-    // tests it against the wave's blocks q, q + 4, ..., whose boxes it keeps in registers.
-    const int ca = lane >> 2, cb = lane & 3;
-    float4 box_lo, box_hi;
-    if constexpr (!BOX_IN_LDS) {
-        box_lo = s_box[wave][cb][0];
-        box_hi = s_box[wave][cb][1];
-    }
-    constexpr unsigned long long QUADS = 0x1111111111111111ull;  // the lanes (a, 0)
-    // The first update is point 0 against every block.
-    float ax = p0[0], ay = p0[1], az = p0[2];
-    unsigned long long reach = 15ull;  // bit 4 a + q: winner a can lower a minimum in block q
-    int last_name = -1;                // the last point emitted; -1: point 0
-    // What the last wave has still to write, lanes (a, 0): the look-up of a point's index would
-    // hold it up behind the barrier that everybody waits at.
-    int pend_at = -1, pend_name = 0;
-    FpsTop top[NB];
-#pragma unroll
-    for (int q = 0; q < NB; ++q)
-        top[q] = FpsTop{F32_NEG1, F32_NEG1, 0.0f, 0.0f, 0.0f, q * PB};
-    if (tid == 0)
-        out[0] = 0;
+    __syncthreads();  // plane1 is read
+    // The picks by name, in order, where the sort had its counters (k <= n <= S).
+    int *const order = reinterpret_cast<int *>(plane1);
+    int base = __builtin_bit_cast(int, reached);  // no minimum is above it
+    int step = 1 << 19;                           // width of the band below it, in steps of a float
+    // With `tied` the band is part of the points whose minimum is `base` itself: those at positions
+    // before tie_end (and from tie_from on, there are none before it).
+    bool tied = false;
+    int tie_from = 0, tie_end = 0, tie_step = S / 8;
+    int wide = step;  // the last band that was not of equals
 
-    int nc = 1;
-    int round = 0;
-    for (int it = 1; it < L.k; it += nc, ++round) {
-        // ---- running minima of the blocks a winner can reach, and those blocks' two largest ----
+    int it = 1, n = 0, round = 0;
+    while (it < L.k) {  // (uniform over the workgroup, as is all of this state)
+        // ---- the points of the band; anew with another band if they are too many or none ----
+        int theta;
+        int crowd = 1 << 20;
+        bool again = false;  // (then the largest minimum is looked for as well)
+        for (;; ++round, again = true) {
+            theta = tied ? base - 1 : fps_max(base - step, 0);
+            int *const count = &s_count[round % 3];
+            if (tid == 0)  // (their last readers are two barriers back)
+                s_count[(round + 1) % 3] = s_stop[(round + 1) % 3] = s_most[(round + 1) % 3] = 0;
+            int first = wave * RS + lane;  // a point's name is this and a constant
+            asm volatile("" : "+v"(first));  // (added where it is wanted, not kept in P registers)
+            const auto enlist = [&](int p, int &at) {
+                const int to = fps_min(at, LIST);  // (what is too much goes to a spare place)
+                s_cand[to] = make_float4(x[p], y[p], z[p], __builtin_bit_cast(float, t[p]));
+                s_name[to] = first + (p / PB) * NW * RS + (p % PB) * TK_WAVE;
+                ++at;
+            };
+            if (__builtin_expect(!tied, 1)) {  // uniform
+                int upto[P / QUAD], mine = 0;  // how many there are in the lane's first points
+#pragma unroll
+                for (int g = 0; g < P / QUAD; ++g) {
+#pragma unroll
+                    for (int p = g * QUAD; p < (g + 1) * QUAD; ++p)
+                        mine += t[p] > theta ? 1 : 0;
+                    upto[g] = mine;
+                }
+                if (mine > 0) {
+                    int at = fps_lds_add(count, mine);
+#pragma unroll
+                    for (int g = 0; g < P / QUAD; ++g) {
+                        if (upto[g] > (g > 0 ? upto[g - 1] : 0)) {
+#pragma unroll
+                            for (int p = g * QUAD; p < (g + 1) * QUAD; ++p) {
+                                if (t[p] > theta)
+                                    enlist(p, at);
+                            }
+                        }
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int p = 0; p < P; ++p) {
+                    if (t[p] > theta &&
+                        fps_position_of_point(point_of(first + (p / PB) * NW * RS + (p % PB) * TK_WAVE), L) < tie_end) {
+                        int at = fps_lds_add(count, 1);
+                        enlist(p, at);
+                    }
+                }
+            }
+            if (again && !tied) {  // uniform
+                int most = t[0];
+#pragma unroll
+                for (int p = 1; p < P; ++p)
+                    most = fps_max(most, t[p]);
+                most = wave_max_i32(fps_max(most, 0));
+                if (lane == 0)
+                    atomicMax(&s_most[round % 3], most);
+            }
+            __syncthreads();
+            n = __builtin_amdgcn_readfirstlane(*count);
+            if ((unsigned)(n - 1) < (unsigned)LIST)
+                break;
+            if (n == 0) {
+                if (tied) {  // none before tie_end
+                    if (tie_end < S) {
+                        tie_step = 2 * tie_step;
+                        tie_from = tie_end;
+                        tie_end = fps_min(tie_from + tie_step, S);
+                    } else {
+                        tied = false;
+                        base -= 1;
+                        step = wide;
+                    }
+                } else {
+                    if (theta == 0)
+                        break;  // no point lies away from the chosen set, and none will
+                    base = again ? __builtin_amdgcn_readfirstlane(s_most[round % 3]) : theta;
+                    step = fps_min(2 * step, 1 << 24);
+                }
+            } else if (tied) {  // (positions differ: LIST of them hold no more points)
+                tie_step = (tie_end - tie_from) >> 1;
+                tie_end = tie_from + tie_step;
+            } else if (base - theta == 1) {  // too many points share the largest minimum
+                tied = true;
+                tie_from = 0;
+                tie_end = fps_min(tie_step, S);
+            } else {
+                step = base - theta;
+                if (again)
+                    base = __builtin_amdgcn_readfirstlane(s_most[round % 3]);
+                // (where a narrower band has not made them fewer, they are equal)
+                step = 4 * n > 3 * crowd ? 1 : fps_band(step, TARGET, n);
+                crowd = n;
+            }
+        }
+        if (n == 0)
+            break;
+        // ---- lane 8 w + i has candidate w + 8 i ----
+        const int own_slot = (lane >> RJ_LOG2) + NJ * (lane & (RJ - 1));
+        const float4 C = s_cand[own_slot];
+        const int my_name = s_name[own_slot];
+        const int v = own_slot < n ? __builtin_bit_cast(int, C.w) : -1;
+        if (wave < NJ) {
+            // wave w relates the candidates of lanes RJ w .. to all of them
+            unsigned hits = 0u, befores = 0u;
+            int pos = -1;
+            bool have_pos = false;
+            const int rows = (n - wave + NJ - 1) / NJ;
+            int over = 0;
+            const auto relate = [&](auto pair, int r) {  // the candidates of lanes r and, with pair, r + 1
+                constexpr int R = decltype(pair)::value;
+                float d[R];
+                int rv[R];
+                unsigned long long after[R], hit[R], same[R], kept = 0ull;
+                int equals = 0;
+#pragma unroll
+                for (int j = 0; j < R; ++j) {
+                    rv[j] = read_lane(v, r + j);
+                    d[j] = tk_dist2<float>(C.x, C.y, C.z, read_lane(C.x, r + j), read_lane(C.y, r + j),
+                                           read_lane(C.z, r + j));
+                    after[j] = __builtin_amdgcn_ballot_w64(rv[j] > v);
+                    same[j] = __builtin_amdgcn_ballot_w64(rv[j] == v);
+                    equals += __builtin_popcountll(same[j]);
+                }
+                if (__builtin_expect(equals != R, 0)) {  // uniform
+                    if (!have_pos) {
+                        pos = fps_position_of_point(point_of(v >= 0 ? my_name : 0), L);
+                        have_pos = true;
+                    }
+#pragma unroll
+                    for (int j = 0; j < R; ++j)
+                        after[j] |= same[j] & __builtin_amdgcn_ballot_w64(read_lane(pos, r + j) < pos);
+                }
+#pragma unroll
+                for (int j = 0; j < R; ++j) {
+                    hit[j] = after[j] & __builtin_amdgcn_ballot_w64(__builtin_bit_cast(int, d[j]) < v);
+                    kept |= hit[j] & __builtin_amdgcn_ballot_w64(__builtin_bit_cast(int, d[j]) > theta);
+                }
+#pragma unroll
+                for (int j = R - 1; j >= 0; --j) {
+                    befores = fps_append(befores, after[j]);
+                    hits = fps_append(hits, hit[j]);
+                }
+                if (__builtin_expect(kept != 0ull, 0)) {  // uniform
+#pragma unroll
+                    for (int j = 0; j < R; ++j)
+                        over = fps_max(over, ((hit[j] >> lane) & 1ull) != 0ull ? __builtin_bit_cast(int, d[j]) : 0);
+                }
+            };
+            if (rows & 1)  // uniform
+                relate(std::integral_constant<int, 1>{}, RJ * wave + rows - 1);
+#pragma unroll 1
+            for (int i = (rows & ~1) - 2; i >= 0; i -= 2)
+                relate(std::integral_constant<int, 2>{}, RJ * wave + i);
+            s_rel[lane].before[wave] = (Piece)befores;
+            s_rel[lane].hit[wave] = (Piece)hits;
+            if (__builtin_expect(__builtin_amdgcn_ballot_w64(over > 0) != 0ull, 0)) {  // uniform
+                over = wave_max_i32(over);
+                if (lane == 0)
+                    atomicMax(&s_stop[round % 3], over);
+            }
+        }
+        __syncthreads();
+        const ulonglong2 rel = *reinterpret_cast<const ulonglong2 *>(&s_rel[lane]);
+        const unsigned long long before = rel.x, hit = rel.y;
+        const int stop = __builtin_amdgcn_readfirstlane(fps_max(theta, s_stop[round % 3]));
+        unsigned long long open = __builtin_amdgcn_ballot_w64(v >= 0), winners = 0ull;
+        while (open != 0ull) {  // (the first of the open ones is decided in every turn)
+            const unsigned long long may = open | winners;
+            const unsigned long long won = __builtin_amdgcn_ballot_w64((hit & may) == 0ull) & open;
+            winners |= won;
+            const unsigned long long lost = __builtin_amdgcn_ballot_w64((hit & winners) != 0ull) & open;
+            open &= ~(won | lost);
+        }
+        winners &= __builtin_amdgcn_ballot_w64(v > stop);
+        // ---- their turns, and the minima they lower ----
+        if (wave == NW - 1) {  // uniform
+            const int at = it + __builtin_popcountll(before & winners);
+            if (((winners >> lane) & 1ull) != 0ull && at < L.k)
+                order[at] = my_name;
+        }
+        it += __builtin_popcountll(winners);
+        if (!tied) {
+            const int was = base - theta;
+            step = fps_max(fps_min(fps_max(fps_band(was, TARGET, n), was >> 1), 2 * was), 1);
+            step = fps_min(step, 1 << 24);
+            wide = fps_max(step, wide >> 1);
+            base = stop;
+        } else {
+            tie_step = n < LIST / 2 ? fps_min(2 * tie_step, S) : tie_step;
+            tie_from = tie_end;
+            tie_end = fps_min(tie_from + tie_step, S);
+        }
 #pragma unroll
         for (int q = 0; q < NB; ++q) {
-            unsigned long long todo = reach & (QUADS << q);
+            const float gx = __builtin_fmaxf(__builtin_fmaxf(box[q][0] - C.x, C.x - box[q][3]), 0.0f);
+            const float gy = __builtin_fmaxf(__builtin_fmaxf(box[q][1] - C.y, C.y - box[q][4]), 0.0f);
+            const float gz = __builtin_fmaxf(__builtin_fmaxf(box[q][2] - C.z, C.z - box[q][5]), 0.0f);
+            const float bound = __builtin_fmaf(gz, gz, __builtin_fmaf(gy, gy, gx * gx));
+            unsigned long long todo = __builtin_amdgcn_ballot_w64(__builtin_bit_cast(int, bound) < v) & winners;
             if (todo != 0ull) {  // uniform
                 if (__builtin_popcountll(todo) & 1) {  // uniform
                     const int l = __builtin_ctzll(todo);
-                    const float sx = read_lane(ax, l), sy = read_lane(ay, l), sz = read_lane(az, l);
+                    const float sx = read_lane(C.x, l), sy = read_lane(C.y, l), sz = read_lane(C.z, l);
 #pragma unroll
                     for (int u = 0; u < PB; ++u) {
                         const int p = q * PB + u;
@@ -886,10 +1100,10 @@ __device__ __forceinline__ void fps_groups(const float *__restrict__ pts, int64_
                 }
                 while (todo != 0ull) {  // two at a time
                     const int l = __builtin_ctzll(todo);
-                    const float sx = read_lane(ax, l), sy = read_lane(ay, l), sz = read_lane(az, l);
+                    const float sx = read_lane(C.x, l), sy = read_lane(C.y, l), sz = read_lane(C.z, l);
                     todo &= todo - 1;
                     const int h = __builtin_ctzll(todo);
-                    const float hx = read_lane(ax, h), hy = read_lane(ay, h), hz = read_lane(az, h);
+                    const float hx = read_lane(C.x, h), hy = read_lane(C.y, h), hz = read_lane(C.z, h);
                     todo &= todo - 1;
 #pragma unroll
                     for (int u = 0; u < PB; ++u) {
@@ -900,282 +1114,30 @@ __device__ __forceinline__ void fps_groups(const float *__restrict__ pts, int64_
                                        __builtin_bit_cast(int, e));
                     }
                 }
-                FpsTop node[PB];
-#pragma unroll
-                for (int u = 0; u < PB; ++u) {
-                    const int p = q * PB + u;
-                    node[u] = FpsTop{t[p], F32_NEG1, x[p], y[p], z[p], p};
-                }
-#pragma unroll
-                for (int w = PB / 2; w >= 1; w /= 2) {
-#pragma unroll
-                    for (int i = 0; i < w; ++i)
-                        node[i] = fps_merge(node[2 * i], node[2 * i + 1], w == PB / 2);
-                }
-                top[q] = node[0];
             }
         }
-        // (a wave without a touched block has left its groups' candidates already)
-        if (reach != 0ull) {  // uniform
-            FpsTop best[NB];
-#pragma unroll
-            for (int q = 0; q < NB; ++q)
-                best[q] = top[q];
-#pragma unroll
-            for (int w = NB / 2; w >= 1; w /= 2) {
-#pragma unroll
-                for (int i = 0; i < w; ++i)
-                    best[i] = fps_merge(best[2 * i], best[2 * i + 1], PB == 1 && w == NB / 2);
-            }
-            // ---- the group's two largest, in all its lanes ----
-            int gm = best[0].m, gs = best[0].s;
-#define TK3D_GROUP_STEPS(STEP)                                                         \
-            STEP(0xb1) /* quad_perm 1,0,3,2 */                                         \
-            if constexpr (GL >= 4) {                                                   \
-                STEP(0x4e) /* quad_perm 2,3,0,1 */                                     \
-            }                                                                          \
-            if constexpr (GL >= 8) {                                                   \
-                STEP(0x141) /* row_half_mirror */                                      \
-            }                                                                          \
-            if constexpr (GL >= 16) {                                                  \
-                STEP(0x140) /* row_mirror */                                           \
-            }
-#define TK3D_GROUP_TOP(ctrl)                                                           \
-            {                                                                          \
-                const int om = __builtin_amdgcn_update_dpp(gm, gm, ctrl, 0xf, 0xf, true); \
-                const int os = __builtin_amdgcn_update_dpp(gs, gs, ctrl, 0xf, 0xf, true); \
-                gs = fps_max(fps_min(gm, om), fps_max(gs, os));                        \
-                gm = fps_max(gm, om);                                                  \
-            }
-            TK3D_GROUP_STEPS(TK3D_GROUP_TOP)
-#undef TK3D_GROUP_TOP
-            // Only points strictly above zero are candidates (the reference starts its scan from
-            // max_dist = 0 with strict '>'); of a group without one, the lanes that write are many,
-            // and what they write is not looked at.
-            bool holds = best[0].m == gm;
-            int pick = best[0].p;
-            float px = best[0].x, py = best[0].y, pz = best[0].z;
-            if (__builtin_expect(__builtin_amdgcn_ballot_w64(gs == gm && gm > 0) != 0ull, 0)) {  // uniform
-                // A group holds its maximum more than once: the reference takes the point with
-                // the lowest position in its own order.
-                int lane_pos = 0x7fffffff;
-#pragma unroll
-                for (int p = 0; p < P; ++p) {
-                    const int pos = fps_position_of_point(point_of(name_of(lane, p)), L);
-                    const bool take = t[p] == gm && pos < lane_pos;
-                    lane_pos = take ? pos : lane_pos;
-                    pick = take ? p : pick;
-                    px = take ? x[p] : px;
-                    py = take ? y[p] : py;
-                    pz = take ? z[p] : pz;
-                }
-                int group_pos = lane_pos;
-#define TK3D_GROUP_MIN(ctrl)                                                           \
-                group_pos = fps_min(group_pos, __builtin_amdgcn_update_dpp(            \
-                                                   group_pos, group_pos, ctrl, 0xf, 0xf, true));
-                TK3D_GROUP_STEPS(TK3D_GROUP_MIN)
-                holds = lane_pos == group_pos;
-                // The largest of the others counts as it will be once this one is chosen: a
-                // cloud that holds points more than once would accept one winner an exchange
-                // otherwise.
-                if (holds)
-                    s_cand[wave * GW + lane / GL] = make_float4(px, py, pz, 0.0f);
-                tk_wave_fence();
-                const float4 w = s_cand[wave * GW + lane / GL];
-                gs = F32_NEG1;
-#pragma unroll
-                for (int p = 0; p < P; ++p) {
-                    const float d = tk_dist2<float>(x[p], y[p], z[p], w.x, w.y, w.z);
-                    gs = fps_max(gs, fps_min(t[p], __builtin_bit_cast(int, d)));
-                }
-#define TK3D_GROUP_MAX(ctrl)                                                           \
-                gs = fps_max(gs, __builtin_amdgcn_update_dpp(gs, gs, ctrl, 0xf, 0xf, true));
-                TK3D_GROUP_STEPS(TK3D_GROUP_MAX)
-#undef TK3D_GROUP_MAX
-                group_pos = 0x7fffffff;
-                if (__builtin_amdgcn_ballot_w64(gs == gm && gm > 0) != 0ull) {  // uniform
-#pragma unroll
-                    for (int p = 0; p < P; ++p) {
-                        const float d = tk_dist2<float>(x[p], y[p], z[p], w.x, w.y, w.z);
-                        const int pos = fps_position_of_point(point_of(name_of(lane, p)), L);
-                        const bool same = t[p] == gm && __builtin_bit_cast(int, d) >= gm;
-                        group_pos = same ? fps_min(group_pos, pos) : group_pos;
-                    }
-                    TK3D_GROUP_STEPS(TK3D_GROUP_MIN)
-                }
-#undef TK3D_GROUP_MIN
-                if (holds)
-                    s_next[wave * GW + lane / GL] = group_pos;
-            }
-            if (holds) {
-                s_cand[wave * GW + lane / GL] = make_float4(px, py, pz, __builtin_bit_cast(float, gm));
-                s_aux[wave * GW + lane / GL] = make_int2(gs, name_of(lane, pick));
-            }
-        }
-#undef TK3D_GROUP_STEPS
-        __syncthreads();
-        // ---- which of the candidates are certain winners of the coming steps ----
-        if (wave == NW - 1) {  // uniform
-            const int j = point_of(pend_name);
-            if (pend_at >= 0)
-                out[pend_at] = (int64_t)j;
-        }
-        if (wave < NJ) {  // uniform
-            __builtin_amdgcn_s_setprio(3);
-            // lane b holds candidates b (, b + 64)
-            float4 C[GM];
-            int name_of_mine[GM], v[GM], second[GM], limit = 0, vmax = 0;
-#pragma unroll
-            for (int g = 0; g < GM; ++g) {
-                C[g] = s_cand[g * TK_WAVE + lane];
-                const int2 X = s_aux[g * TK_WAVE + lane];
-                asm volatile("" ::"v"(C[g].x), "v"(C[g].y), "v"(C[g].z));  // (loaded once, here)
-                v[g] = __builtin_bit_cast(int, C[g].w);
-                name_of_mine[g] = X.y;
-                second[g] = X.x;
-                limit = fps_max(limit, X.x);
-                vmax = fps_max(vmax, v[g]);
-            }
-            limit = wave_max_i32(limit);
-            bool in_list[GM];
-            int slot[GM], n;
-            auto place = [](unsigned long long m, int from) {
-                return (int)__builtin_amdgcn_mbcnt_hi(
-                    (unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, (unsigned)from));
-            };
-            auto enlist = [&]() {
-                n = 0;
-#pragma unroll
-                for (int g = 0; g < GM; ++g) {
-                    in_list[g] = v[g] > limit;
-                    const unsigned long long m = __builtin_amdgcn_ballot_w64(in_list[g]);
-                    slot[g] = place(m, n);
-                    n += __builtin_popcountll(m);
-                }
-            };
-            enlist();
-            if ((unsigned)(n - 1) >= (unsigned)MAXM) {  // uniform: too many, or none
-                vmax = wave_max_i32(vmax);
-                while (n > MAXM) {  // the upper ones (ends at the latest above vmax)
-                    limit += (vmax - limit + 3) >> 2;
-                    enlist();
-                }
-                if (n == 0 && vmax > 0) {
-                    // The largest minimum is there more than once, also in one group: its
-                    // candidates in front of the first point that no group has put up.
-                    int pos[GM], low = 0x7fffffff, end = 0x7fffffff;
-#pragma unroll
-                    for (int g = 0; g < GM; ++g) {
-                        pos[g] = v[g] == vmax ? fps_position_of_point(point_of(name_of_mine[g]), L)
-                                              : 0x7fffffff;
-                        low = fps_min(low, pos[g]);
-                        if (second[g] == vmax)
-                            end = fps_min(end, s_next[g * TK_WAVE + lane]);
-                    }
-                    low = 0x7fffffff - wave_max_i32(0x7fffffff - low);
-                    end = 0x7fffffff - wave_max_i32(0x7fffffff - end);
-                    do {  // (ends at the latest at one candidate)
-                        n = 0;
-#pragma unroll
-                        for (int g = 0; g < GM; ++g) {
-                            in_list[g] = pos[g] < end;
-                            const unsigned long long m = __builtin_amdgcn_ballot_w64(in_list[g]);
-                            slot[g] = place(m, n);
-                            n += __builtin_popcountll(m);
-                        }
-                        end = low + (int)(((unsigned)end - (unsigned)low + 1u) >> 1);
-                    } while (n > MAXM);
-                }
-            }
-#pragma unroll
-            for (int g = 0; g < GM; ++g) {
-                if (in_list[g]) {
-                    s_list[wave][slot[g]] = C[g];
-                    s_name[wave][slot[g]] = name_of_mine[g];
-                }
-            }
-            tk_wave_fence();
-            // lane (c, b) = (lane / 16, lane % 16) compares candidate 4 wave + c of the list
-            // with candidate b
-            const int c = NJ * wave + (lane >> 4), b = lane & 15;
-            const float4 A = s_list[wave][c], B = s_list[wave][b];
-            const int name = s_name[wave][c];
-            const int va = __builtin_bit_cast(int, A.w), vb = __builtin_bit_cast(int, B.w);
-            const unsigned long long there = (unsigned long long)((1u << n) - 1u) * 0x0001000100010001ull;
-            constexpr unsigned long long SELF = 0x0008000400020001ull;
-            unsigned long long before = __builtin_amdgcn_ballot_w64(vb > va) & there;
-            const unsigned long long equal =
-                __builtin_amdgcn_ballot_w64(vb == va && c < n) & there & ~(SELF << (NJ * wave));
-            if (equal != 0ull) {  // uniform
-                const int pa = fps_position_of_point(point_of(c < n ? name : 0), L);
-                const int other = s_name[wave][b];
-                const int pb = fps_position_of_point(point_of(b < n ? other : 0), L);
-                before |= equal & __builtin_amdgcn_ballot_w64(pb < pa);
-            }
-            const float d = tk_dist2<float>(A.x, A.y, A.z, B.x, B.y, B.z);
-            const unsigned long long clash =
-                __builtin_amdgcn_ballot_w64(__builtin_bit_cast(int, d) < va) & before;
-            const int group = lane & 48;
-            const int order = __builtin_popcount((unsigned)(before >> group) & 0xffffu);
-            const bool clear = ((unsigned)(clash >> group) & 0xffffu) == 0u;
-            if (b == 0 && c < n) {
-                s_win[order] = A;
-                s_ent[order] = make_int2(round * 2 + (clear ? 1 : 0), name);
-            }
-            __builtin_amdgcn_s_setprio(0);
-        }
-        if constexpr (BOX_IN_LDS) {
-            box_lo = s_box[wave][cb][0];
-            box_hi = s_box[wave][cb][1];
-        }
-        __syncthreads();
-        const float4 A = s_win[ca];
-        const int2 E = s_ent[ca];
-        ax = A.x;
-        ay = A.y;
-        az = A.z;
-        const unsigned long long missing = ~__builtin_amdgcn_ballot_w64(E.x == round * 2 + 1);
-        int good = missing != 0ull ? __builtin_ctzll(missing) >> 2 : 16;  // winners in a row
-        good = fps_min(good, L.k - it);
-        pend_at = -1;
-        if (good > 0) {  // uniform
-            const float gx = __builtin_fmaxf(__builtin_fmaxf(box_lo.x - A.x, A.x - box_hi.x), 0.0f);
-            const float gy = __builtin_fmaxf(__builtin_fmaxf(box_lo.y - A.y, A.y - box_hi.y), 0.0f);
-            const float gz = __builtin_fmaxf(__builtin_fmaxf(box_lo.z - A.z, A.z - box_hi.z), 0.0f);
-            const float bound = __builtin_fmaf(gz, gz, __builtin_fmaf(gy, gy, gx * gx));
-            const float tau = read_lane(A.w, 0);
-            reach = __builtin_amdgcn_ballot_w64(!(bound >= tau) && ca < good);
-            if (cb == 0 && ca < good)
-                pend_at = it + ca;
-            pend_name = E.y;
-            last_name = read_lane(E.y, 4 * (good - 1));
-            nc = good;
-        } else {
-            // No point lies away from the chosen set, and none will: the previous choice is
-            // emitted from here on.
-            const int64_t j = last_name >= 0 ? (int64_t)point_of(last_name) : (int64_t)0;
-            for (int i = it + tid; i < L.k; i += NT)
-                out[i] = j;
-            break;
-        }
+        ++round;
     }
-    if (wave == NW - 1 && pend_at >= 0)
-        out[pend_at] = (int64_t)point_of(pend_name);
+    __syncthreads();
+    // (after the last point that lies away from the chosen ones the previous choice is repeated)
+    const int64_t again = it > 1 ? (int64_t)point_of(order[fps_min(it, L.k) - 1]) : 0;
+    for (int i = tid; i < L.k; i += NT)
+        out[i] = i == 0 ? 0 : i < it ? (int64_t)point_of(order[i]) : again;
 }
 
-template <int P, int NW, int GM, bool SOA>
-__global__ __launch_bounds__(NW * 64) void fps_groups_kernel_f32(const float *__restrict__ points,
+template <int P, int NW, int NB, bool SOA>
+__global__ __launch_bounds__(NW * 64) void fps_band_kernel_f32(const float *__restrict__ points,
                                                                  int64_t *__restrict__ index,
                                                                  FpsLayout L, bool claims)
 {
-    fps_groups<P, NW, GM, SOA, false>(points + (int64_t)blockIdx.x * L.n * 3,
+    fps_band<P, NW, NB, SOA, false>(points + (int64_t)blockIdx.x * L.n * 3,
                                       index + (int64_t)blockIdx.x * L.k, L, claims);
 }
 
 // Behind the kernel above and the check of its claims: the clouds that it has left, then the
 // coordinates of the picks if wanted ([B,K,3], or [B,3,K] with SOA). One launch for what took two
 // (a second look at every coordinate, the gather): 4.7 us less per call.
-template <int P, int NW, int GM, bool SOA>
+template <int P, int NW, int NB, bool SOA>
 __global__ __launch_bounds__(NW * 64) void fps_last_kernel_f32(const float *__restrict__ points,
                                                                int64_t *__restrict__ index,
                                                                float *__restrict__ sampled,
@@ -1191,7 +1153,7 @@ __global__ __launch_bounds__(NW * 64) void fps_last_kernel_f32(const float *__re
             for (int i = threadIdx.x; i < L.k; i += NT)
                 out[i] = (int64_t)i;
         } else if (left == FPS_BROKEN) {
-            fps_groups<P, NW, GM, SOA, true>(pts, out, L, false);
+            fps_band<P, NW, NB, SOA, true>(pts, out, L, false);
         } else {
             fps_plain<float, P, NT, SOA>(pts, out, L);
         }
@@ -1518,16 +1480,16 @@ void fps_launch_f32(const float *points, bool soa, int64_t B, int64_t *index,
     }
 }
 
-// The groups kernel, the check of its claims and what is left.
-template <int P, int NW, int GM, bool SOA>
-int fps_groups_launch(const float *points, int64_t B, int64_t *index, float *sampled,
+// The band kernel, the check of its claims and what is left.
+template <int P, int NW, int NB, bool SOA>
+int fps_band_launch(const float *points, int64_t B, int64_t *index, float *sampled,
                       const FpsLayout &L, hipStream_t s)
 {
     constexpr int NT = NW * TK_WAVE;
     // the sorted list, and behind it the sort's counters, then one coordinate of every point
     constexpr int LDS = NT * P * 4 + (NT * P > 4100 ? NT * P : 4100) * 4;
-    constexpr auto kernel = fps_groups_kernel_f32<P, NW, GM, SOA>;
-    constexpr auto last = fps_last_kernel_f32<P, NW, GM, SOA>;
+    constexpr auto kernel = fps_band_kernel_f32<P, NW, NB, SOA>;
+    constexpr auto last = fps_last_kernel_f32<P, NW, NB, SOA>;
     int allowed = tk_allow_dynamic_lds<kernel>(LDS);
     if (allowed == TK3D_OK)
         allowed = tk_allow_dynamic_lds<last>(LDS);
@@ -1552,40 +1514,36 @@ int fps_groups_launch(const float *points, int64_t B, int64_t *index, float *sam
     return TK3D_OK;
 }
 
-template <int P, int NW, int GM>
-int fps_groups_launch_f32(const float *points, bool soa, int64_t B, int64_t *index, float *sampled,
+template <int P, int NW, int NB>
+int fps_band_launch_f32(const float *points, bool soa, int64_t B, int64_t *index, float *sampled,
                           const FpsLayout &L, hipStream_t s)
 {
-    return soa ? fps_groups_launch<P, NW, GM, true>(points, B, index, sampled, L, s)
-               : fps_groups_launch<P, NW, GM, false>(points, B, index, sampled, L, s);
+    return soa ? fps_band_launch<P, NW, NB, true>(points, B, index, sampled, L, s)
+               : fps_band_launch<P, NW, NB, false>(points, B, index, sampled, L, s);
 }
 
-// fp32, the groups kernel: whether it takes the call, and its launch if so. It needs 256 samples to
+// fp32, the band kernel: whether it takes the call, and its launch if so. It needs 192 samples to
 // be paid for: its prologue sorts the cloud, which costs 5 us at 1024 points and 25 at 16384, and
-// early in a sampling, where a centre reaches every block, an exchange is no faster than the
-// multi-step kernel's. At 256 samples (us, multi-step against this one, with what runs behind
-// them): 16 x 16384 284, 240; 16 x 8192 185, 168; 16 x 4096 131, 129; from there on it gains with every
-// sample. Clouds of 1024 and 2048 points, on which no lane of the multi-step kernel idles, lose at 256
-// samples in random order (16 x 1024 84, 92; 16 x 2048 97, 110; equal from 320 and 384 on; 16 x 600 83, 84,
-// 16 x 1500 104, 97), but gain more in sampling order, in which an encoder's levels come (4 x 1024 63, 14).
-// Up to 512 points the multi-step kernel has four launches less to wait for. 128 groups instead of 64
-// accept 10-14 % more winners and cost a step of the judgement: with 16 points per lane they lose up to
-// 512 samples (229 against 220 us at 256).
-bool fps_groups_dispatch_f32(const float *points, bool soa, int64_t B, int64_t *index, float *sampled,
+// early in a sampling, where the points far from all centres are neighbours, a band of 64 holds one or
+// two winners. Multi-step kernel against this one, with what runs behind them, us, at 128 samples:
+// 1 x 300 42, 35; 16 x 600 48, 55; 16 x 1024 50, 59; 16 x 4096 77, 83; 16 x 16384 159, 161; at 192: 65, 45;
+// 67, 53; 69, 56; 104, 86; 222, 177. In sampling order, in which an encoder's levels come, it has 16 for
+// 46 to 210 at 192 samples.
+bool fps_band_dispatch_f32(const float *points, bool soa, int64_t B, int64_t *index, float *sampled,
                              const FpsLayout &L, int64_t npos, hipStream_t s, int &rc)
 {
-    if (npos <= 512 || npos > 1024 * 16 || L.k < 256)
+    if (npos > 1024 * 16 || L.k < 192)
         return false;
-    if (npos <= 512 * 4)
-        rc = fps_groups_launch_f32<4, 8, 1>(points, soa, B, index, sampled, L, s);
-    else if (npos <= 512 * 8)
-        rc = fps_groups_launch_f32<8, 8, 2>(points, soa, B, index, sampled, L, s);
+    if (npos <= 512 * 2)
+        rc = fps_band_launch_f32<2, 8, 2>(points, soa, B, index, sampled, L, s);
+    else if (npos <= 512 * 4)
+        rc = fps_band_launch_f32<4, 8, 2>(points, soa, B, index, sampled, L, s);
+    else if (npos <= 1024 * 4)
+        rc = fps_band_launch_f32<4, 16, 2>(points, soa, B, index, sampled, L, s);
     else if (npos <= 1024 * 8)
-        rc = fps_groups_launch_f32<8, 16, 2>(points, soa, B, index, sampled, L, s);
-    else if (L.k < 512)
-        rc = fps_groups_launch_f32<16, 16, 1>(points, soa, B, index, sampled, L, s);
+        rc = fps_band_launch_f32<8, 16, 4>(points, soa, B, index, sampled, L, s);
     else
-        rc = fps_groups_launch_f32<16, 16, 2>(points, soa, B, index, sampled, L, s);
+        rc = fps_band_launch_f32<16, 16, 4>(points, soa, B, index, sampled, L, s);
     return true;
 }
 
@@ -1676,7 +1634,7 @@ int fps(const T *points, bool soa, int64_t B, int64_t N, int64_t K, int64_t *ind
     if (npos <= fps_register_capacity(sizeof(T))) {
         if constexpr (sizeof(T) == 4) {
             int rc;
-            if (fps_groups_dispatch_f32(points, soa, B, index, sampled, L, npos, s, rc))
+            if (fps_band_dispatch_f32(points, soa, B, index, sampled, L, npos, s, rc))
                 return rc != TK3D_OK ? rc : tk_launch_status();
             fps_dispatch_f32(points, soa, B, index, L, npos, s);
         } else {
