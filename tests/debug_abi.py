@@ -76,7 +76,7 @@ def chamfer_sorted(x1, x2, counted=False, stages=7, ws=None, out=None):
 
 def knn_filter(query, key, k):
     """(distance, index) of KNN through the pre-filtered kernel, or None when it does not take
-    the shape (k > 16 or under 256 keys)."""
+    the shape (k > 32)."""
     from torkit3d_amd import _lib
     from torkit3d_amd._lib import i64, ptr, stream_of
 

@@ -360,6 +360,23 @@ def test_prefiltered_kernel_with_sorted_slots_on_equal_distances(cuda, steps, k)
     check_raw(0.01 * uniform_cloud(g, 4, 8192 + 5), key, k, cuda)
 
 
+@pytest.mark.parametrize("k", [1, 3, 4, 5, 8, 9, 16, 17, 32])
+@pytest.mark.parametrize("n2", [64, 65, 96, 97, 511, 512, 513, 700, 1024])
+def test_prefiltered_kernel_on_short_clouds(cuda, n2, k):
+    # the smallest clouds it is launched on: less than a stage, parts of a chunk, one key into
+    # the second stage; in random order, on a lattice, and from far to near (every key inserted)
+    b, n1 = 74, 256 + 5                      # beyond what a wave per query takes
+    assert b * n1 > 18432
+    g = gen(n2 + k)
+    key = uniform_cloud(g, b, n2)
+    key[1::3] = lattice_cloud(g, len(key[1::3]), n2, 4)
+    order = key[2::3].norm(dim=2).argsort(dim=1, descending=True)
+    key[2::3] = torch.gather(key[2::3], 1, order[:, :, None].expand(-1, -1, 3))
+    q = uniform_cloud(g, b, n1)
+    q[1::3] = lattice_cloud(g, len(q[1::3]), n1, 4)
+    check_raw(q, key, k, cuda)
+
+
 # ---- k = 17..32 with 32768 to 131071 queries against 4096 keys or more: the same matrix
 # sweep feeding the LDS tournament tree (one query per lane, two blocks of 32 per wave) ----
 

@@ -373,129 +373,50 @@ __global__ __launch_bounds__(KNN_BLOCK) void knn_batched_kernel_f32(
                                          k, skey);
 }
 
-// The slot number of every position of a sorted list of KMAX distances (see SORTED below).
-// Up to 16 positions: a nibble each in one 64-bit word. 32 positions: the low nibbles in two
-// 64-bit words and the fifth bits in a 32-bit word.
-template <int KMAX> struct KnnSlotNumbers;
-
-template <> struct KnnSlotNumbers<16> {
-    unsigned long long w;
-    __device__ __forceinline__ void identity() { w = 0xfedcba9876543210ull; }
-    __device__ __forceinline__ unsigned head() const { return (unsigned)w & 15u; }
-    __device__ __forceinline__ unsigned at(int p) const
+// A slot of the sorted list below: the bit pattern of the distance above (flag, KMAX - 1 - slot, key
+// index). As a double it orders by distance and, among equal distances, by the low word: no pattern of
+// a float is one of a NaN or an infinity up there, zero is a (kept) subnormal, the negative patterns
+// of the placeholders are below all others.
+template <int KMAX> struct KnnSlot {
+    static constexpr int SLOT_BITS = KMAX == 32 ? 5 : KMAX == 16 ? 4 : KMAX == 8 ? 3 : 2;
+    static constexpr int KEY_BITS = 31 - SLOT_BITS;
+    static constexpr unsigned FLAG = 0x80000000u;
+    static constexpr unsigned SLOT = (unsigned)(KMAX - 1) << KEY_BITS;  // mask of the slot's bits
+    static constexpr unsigned KEY = (1u << KEY_BITS) - 1u;
+    static_assert((1 << SLOT_BITS) == KMAX, "4, 8, 16 or 32 slots");
+    static __device__ __forceinline__ double pack(int distance, unsigned low)
     {
-        return (unsigned)(w >> ((4 * p) & 63)) & 15u;
+        return __builtin_bit_cast(double, ((unsigned long long)(unsigned)distance << 32) | low);
     }
-    // positions 0..m turn by one towards the head; `slot` (the old head's) goes to position m
-    __device__ __forceinline__ void turn(int m, unsigned slot)
+    static __device__ __forceinline__ int distance(double v)
     {
-        const unsigned long long turning = ~0ull >> (60 - 4 * m);
-        w = (w & ~turning) | ((w & turning) >> 4) | ((unsigned long long)slot << (4 * m));
+        return (int)(__builtin_bit_cast(unsigned long long, v) >> 32);
     }
-    // positions m..s move one position down (s is a compile-time constant, s > 0), `slot`
-    // enters at position m
-    __device__ __forceinline__ void make_room(int m, int s, unsigned slot)
+    static __device__ __forceinline__ unsigned low(double v)
     {
-        const unsigned long long field = (~0ull >> (60 - 4 * s)) & (~0ull << (4 * m));
-        w = (w & ~field) | (((w & field) << 4) & field) | ((unsigned long long)slot << (4 * m));
+        return (unsigned)__builtin_bit_cast(unsigned long long, v);
     }
-    __device__ __forceinline__ void keep() { asm volatile("" : "+v"(w)); }
-};
-
-template <> struct KnnSlotNumbers<32> {
-    unsigned long long w0, w1;  // low nibbles of positions 0..15 and 16..31
-    unsigned fifth;             // bit p: the fifth bit of position p's slot
-    __device__ __forceinline__ void identity()
+    static __device__ __forceinline__ int slot(double v)
     {
-        w0 = w1 = 0xfedcba9876543210ull;
-        fifth = 0xffff0000u;
-    }
-    __device__ __forceinline__ unsigned head() const
-    {
-        return ((unsigned)w0 & 15u) | ((fifth & 1u) << 4);
-    }
-    __device__ __forceinline__ unsigned at(int p) const
-    {
-        const unsigned long long w = p < 16 ? w0 : w1;
-        return ((unsigned)(w >> ((4 * p) & 63)) & 15u) | (((fifth >> (p & 31)) & 1u) << 4);
-    }
-    __device__ __forceinline__ void turn(int m, unsigned slot)
-    {
-        const unsigned turning5 = ~0u >> (31 - m);
-        fifth = (fifth & ~turning5) | ((fifth & turning5) >> 1) | ((slot >> 4) << m);
-        const bool far = m >= 16;
-        const unsigned long long low = slot & 15u;
-        // the first word turns as far as m reaches in it and takes the second word's first
-        // nibble, or the slot, at the end of that range
-        const int m0 = far ? 15 : m;
-        const unsigned long long t0 = ~0ull >> (60 - 4 * m0);
-        const unsigned long long in0 = far ? (w1 & 15ull) : low;
-        w0 = (w0 & ~t0) | ((w0 & t0) >> 4) | (in0 << (4 * m0));
-        const int m1 = far ? m - 16 : 0;
-        const unsigned long long t1 = far ? ~0ull >> (60 - 4 * m1) : 0ull;
-        w1 = (w1 & ~t1) | ((w1 & t1) >> 4) | (far ? low << (4 * m1) : 0ull);
-    }
-    __device__ __forceinline__ void make_room(int m, int s, unsigned slot)
-    {
-        const unsigned field5 = (~0u >> (31 - s)) & (~0u << m);
-        fifth = (fifth & ~field5) | (((fifth & field5) << 1) & field5) | ((slot >> 4) << m);
-        const unsigned long long low = slot & 15u;
-        if (s < 16) {  // (compile-time) only the first word
-            const unsigned long long field = (~0ull >> (60 - 4 * s)) & (~0ull << (4 * m));
-            w0 = (w0 & ~field) | (((w0 & field) << 4) & field) | (low << (4 * m));
-        } else {
-            const bool far = m >= 16;  // the first word stays as it is
-            // second word: positions max(m, 16)..s move down; what enters at its start is
-            // the first word's last nibble, or the slot itself
-            const int m1 = far ? m - 16 : 0;
-            const unsigned long long f1 = (~0ull >> (60 - 4 * (s - 16))) & (~0ull << (4 * m1));
-            const unsigned long long in1 = far ? low : (w0 >> 60);
-            w1 = (w1 & ~f1) | (((w1 & f1) << 4) & f1) | (in1 << (4 * m1));
-            const unsigned long long f0 = far ? 0ull : ~0ull << (4 * m);
-            w0 = (w0 & ~f0) | ((w0 & f0) << 4) | (far ? 0ull : low << (4 * m));
-        }
-    }
-    __device__ __forceinline__ void keep()
-    {
-        asm volatile("" : "+v"(w0), "+v"(w1), "+v"(fifth));
+        return KMAX - 1 - (int)((low(v) & SLOT) >> KEY_BITS);
     }
 };
 
-// How many of positions 1..KMAX-1 of a descending list satisfy `above` (true for a prefix of
-// them), by bisection through the registers: the pivot of a level is chosen among its 2^level
-// possible places by selects on the outcomes so far (KMAX - 1 - log2 KMAX selects in all).
-// `last` returns the last position's value that satisfied it (`none` without one).
-template <int KMAX, typename Above>
-__device__ __forceinline__ int knn_sorted_position(const int (&v)[KMAX], Above above, int none,
-                                                   int &last)
+// (the builtins quiet their operands first, an instruction each)
+__device__ __forceinline__ double knn_min_f64(double a, double b)
 {
-    constexpr int LEVELS = KMAX == 32 ? 5 : KMAX == 16 ? 4 : KMAX == 8 ? 3 : 2;
-    static_assert((1 << LEVELS) == KMAX, "KMAX is a power of two from 4 to 32");
-    bool taken[LEVELS];
-    int m = 0;
-    last = none;
-#pragma unroll
-    for (int level = 0; level < LEVELS; ++level) {
-        const int step = KMAX >> (level + 1);
-        int c[1 << (LEVELS - 1)];
-#pragma unroll
-        for (int j = 0; j < (1 << level); ++j)
-            c[j] = v[(2 * j + 1) * step];
-        // the outcome of the previous level is the lowest bit of the place, and so on
-#pragma unroll
-        for (int d = level - 1; d >= 0; --d) {
-#pragma unroll
-            for (int j = 0; j < (1 << d); ++j)
-                c[j] = taken[d] ? c[2 * j + 1] : c[2 * j];
-        }
-        taken[level] = above(c[0]);
-        last = taken[level] ? c[0] : last;
-        m = 2 * m + (taken[level] ? 1 : 0);
-    }
-    return m;
+    double o;
+    asm("v_min_f64 %0, %1, %2" : "=v"(o) : "v"(a), "v"(b));
+    return o;
+}
+__device__ __forceinline__ double knn_max_f64(double a, double b)
+{
+    double o;
+    asm("v_max_f64 %0, %1, %2" : "=v"(o) : "v"(a), "v"(b));
+    return o;
 }
 
-// fp32, k <= 16, launches with many queries: pre-filtered sweep with deferred insertions.
+// fp32, k <= 32, launches with many queries: pre-filtered sweep with deferred insertions.
 //
 // Two costs dominate the batched kernel above: its sweep spends 8 vector instructions per
 // pair (six for the canonical distance), and its insertion rounds run after every chunk
@@ -504,90 +425,74 @@ __device__ __forceinline__ int knn_sorted_position(const int (&v)[KMAX], Above a
 // Sweep. As in the chamfer kernel, most pairs only need to be ruled out, which the score
 //     s(q,k) = |k'|^2 - 2 q'.k'      (k' = k - c, q' = q - c, c the centre of the key
 //                                      cloud's bounding box)
-// does with three fused multiply-adds: d2(q,k) = s + |q'|^2 up to rounding. A key can
-// only be inserted if its canonical distance is below the query's current maximum M, so
-// the sweep evaluates t = s - thr, thr = (M - |q'|^2) + slack, by starting the three fmas
-// from |k'|^2 - thr, and collects the sign bits of t: 5 instructions per pair. With
-// u = 2^-24, rho = |k'| + |q'|, R = (max|k'| + |q'|)^2:
-//     canonical d2 against the exact distance of the centred points   7.02 u rho^2
-//         (three rounded differences, a product and two fmas of non-negative terms,
-//          plus the rounding of k' and q' themselves)
-//     |k'|^2 as staged                                                 3 u |k'|^2
-//     |k'|^2 - thr and the three fmas: four roundings of partial sums
-//         bounded by R + |thr|                                         4.04 u (R + |thr|)
-//     thr itself: M - |q'|^2 and the added slack                      3 u (M + R)
-// With |thr| <= M + R the total is below 21.2 u R + 7.1 u M; the kernel uses
-// slack = 32 u R + 16 u M (+1e-37 against underflow), R from max|k'| and |q'| inflated by
-// 1e-6 for their own rounding. Every key with canonical d2 < M therefore has t < 0: the
-// sign bits are a superset of MinK's insertions. Queries or key clouds that are
-// non-finite or huge (where the bound means nothing) take every key as a candidate, or
-// the workgroup runs the exact batched sweep.
-//
-// Insertions. A candidate is re-evaluated with the canonical arithmetic and inserted
-// under MinK's strict test against the maximum as it stands then, in ascending key
-// order per query, so the slots go through exactly MinK's states. But insertion does not
-// follow every chunk: a lane keeps up to CAP non-empty chunk masks per query in a small
-// register queue and the wave runs a service step (every lane with a pending candidate
-// takes its first one) only while some lane holds T candidates or a full queue; the
-// rest waits for company. Deferring only makes M - and with it thr - a little stale,
-// i.e. admits more candidates, each rejected by the strict test when it is served.
-// Per 2048 keys a wave runs 68 steps at k = 3 and 145 at k = 16 instead of 142 and 253
-// rounds. Keys are centred and staged in LDS as (x', y', z', |k'|^2); a lane serves QPL
-// queries, so one LDS read feeds QPL pairs and the steps of its queries interleave.
-//
-// MATRIX. The scores of a chunk of 32 keys come from the matrix cores instead: one
-// v_mfma_f32_32x32x16_f16 gives t = s - thr for 32 keys x 32 queries as a 16-term dot
-// product of fp16 pieces, and a lane only has to collect the 16 sign bits it is handed
-// (1.1 vector instructions per pair instead of 5). Coordinates are centred and multiplied
-// by a power of two that brings the largest centred key norm into [1, 2) (exact; outside
-// 2^-40 .. 2^40 the workgroup takes the exact sweep), then split into two fp16 pieces
-// each, x = xh + xl + e with |e| <= 2^-23 |x| + 2^-25, |k'|^2 into two and -thr into two:
+// does: d2(q,k) = s + |q'|^2 up to rounding. A key can only be inserted if its canonical
+// distance is below the query's current maximum M, so the sweep takes the sign of t = s - thr,
+// thr = (M - |q'|^2) + slack: candidates are the keys with t < 0. The scores come from the matrix
+// cores: one v_mfma_f32_32x32x16_f16 gives t for 32 keys x 32 queries as a 16-term dot product of
+// fp16 pieces, and a lane only has to collect the 16 sign bits it is handed (1.1 vector
+// instructions per pair). Coordinates are centred and multiplied by a power of two that brings
+// the largest centred key norm into [1, 2) (exact; outside 2^-40 .. 2^40 the workgroup takes the
+// exact sweep), then split into two fp16 pieces each, x = xh + xl + e with |e| <= 2^-23 |x| +
+// 2^-25, |k'|^2 into two and -thr into two:
 //     key   : xh xh xl  yh yh yl  1  1  | zh zh zl  n0 n1 0  1  1
 //     query : Xh Xl Xh  Yh Yl Yh  T0 T1 | Zh Zl Zh  1  1  0  T0 T1        (X = -2 q'x)
 // In the 32 x 32 result lane l holds rows (keys) 16 h .. 16 h + 15, h = l / 32, of column
 // (query) l % 32; the keys of a tile are stored in that row order, so the sign bits of a
-// lane are 16 consecutive bits of the chunk mask. The wave's 64 QPL queries are 2 QPL
-// blocks of 32; lane l owns the queries of column l % 32 in blocks h, 2 + h, ..., computes
-// their thr and writes -thr into the T terms of its own half only (the other half holds
-// zeros there), so no thr crosses lanes; the two halves of a mask meet through one exchange
-// between lanes l and l ^ 32 per chunk. The library runs it with one query per lane in
-// workgroups of 512 lanes (LANES): 120 registers, four waves per SIMD, where two queries
-// per lane need 238 and leave two. Error budget in the rescaled units, on top of the
-// one above (products of the second pieces are left out, thr is rounded to two pieces):
+// lane are 16 consecutive bits of the chunk mask. The wave's 64 queries are two blocks of 32,
+// block h the queries of the lanes of half h; a lane computes its thr and writes -thr into the T
+// terms of its own half only (the other half holds zeros there), so no thr crosses lanes; the
+// halves of a mask meet through one exchange of registers between lanes l and l ^ 32. With
+// u = 2^-24, rho = |k'| + |q'|, R = (max|k'| + |q'|)^2, in the rescaled units:
+//     canonical d2 against the exact distance of the centred points   7.02 u rho^2
+//         (three rounded differences, a product and two fmas of non-negative terms,
+//          plus the rounding of k' and q' themselves)
+//     |k'|^2 as staged, thr itself                         3 u |k'|^2 + 3 u (M + R)
 //     pieces dropped from 2 q'.k', subnormal pieces                       5 u R
 //     |k'|^2 and thr in two pieces                           4 u R + 4 u (M + R)
 //     the matrix core's 16 additions: 32 u times the sum of the products' magnitudes
 //         as the matrix core sees them (a subnormal fp16 factor counts as 2^-14; see
 //         the chamfer kernel and tests/test_gpu_mfma_bound.py), which is below
 //         1.02 (M + R) here because the scale makes max|k'| >= 1     33 u (M + R)
-//     canonical d2, |k'|^2 as staged, thr itself             10 u R + 3 u (M + R)
-// below 59 u R + 40 u M; the kernel uses slack = 64 u R + 48 u M. Queries further than 200
-// from the centre (rescaled; thr would leave fp16's range) take every key as a candidate.
-// KI_LDS: the key indices of the slots live in LDS (16-bit, so clouds of up to 65536 keys),
-// one column per lane: they are only written during the sweep, and a write into a column of
-// one's own is one instruction where the slot in registers takes a select per slot.
+// below 59 u R + 40 u M; the kernel uses slack = 64 u R + 48 u M (+1e-37 against underflow), R from
+// max|k'| and |q'| inflated by 1e-6 for their own rounding. Every key with canonical d2 < M
+// therefore has t < 0: the sign bits are a superset of MinK's insertions. Queries further than 200
+// from the centre (rescaled; thr would leave fp16's range) take every key as a candidate, key clouds
+// that are non-finite or huge the exact batched sweep.
 //
-// SORTED (8 to 32 slots, key indices in LDS; described for 16): the registers hold the
-// distances in descending order instead of slot order, and a 64-bit word holds the slot
-// number of every position, a nibble each. MinK's maximum is then position 0, and an
-// insertion is one v_med3_i32 per position (remove the head, let the new key x sink to its place: position p becomes the
-// median of its old value, its lower neighbour's and x) plus a rotation of the nibbles of
-// positions 0..m, m being x's new position, found by a binary search through the registers
-// (4 compares, 11 selects): 86 instructions per step where the slot-ordered registers take
-// 116 (a select per slot to write, a max3 tree and a sign-bit scan for the first slot that
-// holds the new maximum). MinK's order among equal distances (mink.cuh:74-87: the rescan
-// starts from the inserted key and moves on only to a strictly larger one, so the maximum
-// is the inserted slot if nothing is strictly above it, else the lowest slot holding the
-// largest distance) becomes: equal distances are kept in ascending slot order, except
-// that a key with nothing strictly above it goes to the head. With R the list without its
-// head, x goes to position 0 if no element of R is above it, else behind the elements of R
-// that are above it or equal to it with a lower slot number. Equal distances are rare
-// outside quantised clouds: the binary search counts the elements >= x and hands back the
-// last of them; only when that equals x in some lane does the wave search again, for the
-// elements strictly above x, and walk the run of equals between the two results comparing
-// slot numbers.
-template <int KMAX, int QPL, bool SOA, bool WEIGHTS, bool MATRIX, int LANES = KNN_BLOCK,
-          bool KI_LDS = false, bool SORTED = false>
+// Insertions. A candidate is re-evaluated with the canonical arithmetic and inserted
+// under MinK's strict test against the maximum as it stands then, in ascending key
+// order per query, so the slots go through exactly MinK's states. But insertion does not
+// follow every chunk: a lane keeps up to CAP non-empty chunk masks in a small
+// register queue and the wave runs a service step (every lane with a pending candidate
+// takes its first one) only while some lane holds T candidates or a full queue; the
+// rest waits for company. Deferring only makes M - and with it thr - a little stale,
+// i.e. admits more candidates, each rejected by the strict test when it is served.
+// Per 2048 keys a wave runs 68 steps at k = 3 and 145 at k = 16 instead of 142 and 253
+// rounds.
+//
+// Slots. They are kept in descending order, each a double made of the distance's bit pattern above
+// (flag, KMAX - 1 - slot, key index): v_min_f64 and v_max_f64 run at the rate of 32-bit
+// instructions, compare both words at once and need no selects, so an insertion (the head leaves, x sinks
+// to its place: position p becomes the larger of its lower neighbour and the smaller of itself and
+// x) is 2 KMAX - 1 instructions, slot numbers, key indices and ties included. MinK's order among equal
+// distances (mink.cuh:74-87: the rescan starts from the inserted key and moves on only to a strictly
+// larger one, so the maximum is the inserted slot if nothing is strictly above it, else the lowest slot
+// holding the largest distance) is the order of the low words - equal distances in ascending slot
+// order - except that a key with nothing strictly above it goes to the head: it gets the flag, which
+// leaves with it at the next insertion. 64 instructions a step at k = 16 where a list of distances with
+// the slot numbers as nibbles of a 64-bit word and the key indices in LDS took 86 (a median per
+// position, a binary search, the nibbles' rotation), and 40 at k = 3 where slots in registers in their
+// own order took 112 (selects, a maximum, a scan for its first slot).
+//
+// Bound by vector issue, of which the steps are half to two thirds: a lane is a query whose
+// candidates are served in key order, so 59 % of the lanes are busy in a step at k = 16, a third at k =
+// 3. 512 lanes share the staged keys (113 registers up to 16 slots, four waves per SIMD); 32 slots run
+// in 256 (up to 6 % faster; bounded to three waves per SIMD the registers spill, 3 to 30 % slower).
+// us, list with nibbles (slot order up to 4) and this: 32 x 8192 queries on 2048 keys k = 3 74, 63, k = 8 101,
+// 82, k = 16 152, 125, k = 32 376, 254; 32 x 2048 on 8192 k = 3 137, 96, k = 16 190, 130, k = 32 272, 191; 4 x 16384
+// on 16384 k = 16 316, 213; on lattices of 5 positions an axis, where nearly every step meets equal
+// distances, k = 16 407, 166, k = 32 1391, 342.
+template <int KMAX, bool SOA, bool WEIGHTS, int LANES>
 __global__ __launch_bounds__(LANES) void knn_filter_kernel_f32(
     const float *__restrict__ query, const float *__restrict__ key,
     float *__restrict__ distance, int64_t *__restrict__ index, float *__restrict__ weight,
@@ -600,17 +505,15 @@ __global__ __launch_bounds__(LANES) void knn_filter_kernel_f32(
     constexpr int CAP = 4;
     constexpr int T = 6;
     constexpr int PER = STAGE / BLOCK;
+    using Slot = KnnSlot<KMAX>;
     static_assert(STAGE % BLOCK == 0 && STAGE % CHUNK == 0, "stage shape");
-    static_assert(!SORTED || (KI_LDS && QPL == 1 && KMAX >= 4 && KMAX <= 32 && !WEIGHTS),
-                  "the sorted list is for one query of 4 to 32 slots per lane, no weights");
-    static_assert(2 * STAGE * 4 * (int)sizeof(float) >= KNN_STAGE * 4 * (int)sizeof(float),
-                  "the staging buffers double as the exact sweep's stage");
-    // Two stage buffers of centred keys (x', y', z', |k'|^2) (+ 8 keys the read-ahead of
-    // the sweep runs into), then two of raw keys (x, y, z, 0) for the service steps.
-    // (MATRIX: two stage buffers of key terms, [tile][half][row] x 16 bytes, instead.)
-    static_assert(!MATRIX || QPL == 1 || QPL == 2, "two or four blocks of 32 queries per wave");
-    constexpr int SCORE_FLOATS = MATRIX ? 2 * STAGE * 8 : 2 * STAGE * 4 + 32;
+    static_assert(!WEIGHTS || KMAX == 4, "weights of three neighbours");
+    // Two stage buffers of key terms, [tile][half][row] x 16 bytes, then two of raw keys
+    // (x, y, z, 0) for the service steps.
+    constexpr int SCORE_FLOATS = 2 * STAGE * 8;
     constexpr int STAGING_FLOATS = SCORE_FLOATS + 2 * STAGE * 4;
+    static_assert(STAGING_FLOATS >= KNN_STAGE * 4,
+                  "the staging buffers double as the exact sweep's stage");
     // waves that transpose their results together (32 slots: two, 34 KB of LDS)
     constexpr int TWAVES = NW < 4 ? NW : KMAX > 16 ? 2 : 4;
     constexpr int TRANSPOSE_FLOATS = TWAVES * 2 * TK_WAVE * (KMAX + 1);  // see the end of the kernel
@@ -618,7 +521,6 @@ __global__ __launch_bounds__(LANES) void knn_filter_kernel_f32(
         skey[STAGING_FLOATS > TRANSPOSE_FLOATS ? STAGING_FLOATS : TRANSPOSE_FLOATS];
     float4 *const sraw = reinterpret_cast<float4 *>(skey + SCORE_FLOATS);
     uint4 *const sterm = reinterpret_cast<uint4 *>(skey);
-    extern __shared__ __align__(16) unsigned short knn_filter_ski[];  // KI_LDS: [QPL][KMAX][LANES]
     const int half = (threadIdx.x >> 5) & 1;
     __shared__ float sred[NW][8];
     const int tid = threadIdx.x;
@@ -686,464 +588,218 @@ __global__ __launch_bounds__(LANES) void knn_filter_kernel_f32(
     for (int w = 0; w < NW; ++w)
         kmax2 = __builtin_fmaxf(kmax2, sred[w][6]);
     bool safe = (c0 - c0 == 0.0f) && (c1 - c1 == 0.0f) && (c2 - c2 == 0.0f) && (kmax2 < 1e30f);
-    float scale = 1.0f;  // MATRIX: 2^-(exponent of the largest centred key norm)
-    if constexpr (MATRIX) {
-        const float ext = __builtin_sqrtf(kmax2);
-        const int ebits = (int)((__builtin_bit_cast(unsigned, ext) >> 23) & 0xffu) - 127;
-        safe = safe && (ext == 0.0f || (ebits >= -40 && ebits <= 40));
-        scale = (!safe || ext == 0.0f) ? 1.0f
-                                       : __builtin_bit_cast(float, (unsigned)(127 - ebits) << 23);
-    }
+    const float ext = __builtin_sqrtf(kmax2);
+    const int ebits = (int)((__builtin_bit_cast(unsigned, ext) >> 23) & 0xffu) - 127;
+    safe = safe && (ext == 0.0f || (ebits >= -40 && ebits <= 40));
+    // 2^-(exponent of the largest centred key norm)
+    const float scale = (!safe || ext == 0.0f) ? 1.0f
+                                               : __builtin_bit_cast(float, (unsigned)(127 - ebits) << 23);
+
     if (!safe) {  // uniform over the workgroup
-#pragma unroll 1
-        for (int i = 0; i < QPL; ++i)
-            knn_batched_body<KMAX, SOA, WEIGHTS>(query, key, distance, index, weight, eps, b,
-                                                 (qblock * QPL + i) * BLOCK + tid, n1, n2, k,
-                                                 skey);
+        knn_batched_body<KMAX, SOA, WEIGHTS>(query, key, distance, index, weight, eps, b,
+                                             qblock * BLOCK + tid, n1, n2, k, skey);
         return;
     }
     const float kmax = __builtin_sqrtf(kmax2) * scale * 1.000001f;
     const float scale2 = scale * scale;  // <= 2^80
 
-    // ---- queries ----
-    float qx[QPL], qy[QPL], qz[QPL], ax[QPL], ay[QPL], az[QPL], qn[QPL], slack_r[QPL];
-    bool active[QPL], usable[QPL];
-    // Slots hold the bit patterns of the distances: squared distances are non-negative, so
-    // their patterns order as signed integers. A NaN can only enter during the fill (a later
-    // key must compare below the maximum) and MinK never selects such a slot as maximum
-    // unless it is slot 0, in which case it never inserts again: here a NaN slot holds the
-    // pattern of -inf (below everything) and is recomputed when the results are written, and
-    // a NaN in slot 0 freezes the query (maximum -inf: no key compares below it).
-    int kd[QPL][KMAX];
-    int ki[QPL][KI_LDS ? 1 : KMAX];
-    auto ski = [&](int i, int slot) -> unsigned short & {
-        return knn_filter_ski[(i * KMAX + slot) * LANES + threadIdx.x];
-    };
-    float max_key[QPL];
-    int max_idx[QPL];
-    unsigned nan_slots[QPL];
-    KnnSlotNumbers<(KMAX > 16 ? 32 : 16)> ids[QPL];  // SORTED: the slot of every position of kd
-    constexpr int NEG_INF_BITS = (int)0xff800000u;
-    constexpr int INT_LOWEST = (int)0x80000000u, INT_HIGHEST = 0x7fffffff;
-    // the median of three (v_med3_i32)
-    auto med3 = [](int a, int b, int c) {
-        const int lo = a < b ? a : b, hi = a < b ? b : a;
-        const int t = hi < c ? hi : c;
-        return lo > t ? lo : t;
-    };
-    // Pending chunk masks per query, oldest first (bit 31 = first key of the chunk), and
-    // the key index of bit 31 of each. Named members and no loops over the queue, so it
-    // stays in registers (an array indexed through a loop ends up in scratch memory).
-    static_assert(CAP == 4, "the queue is written out for four entries");
-    struct Pending {
-        unsigned m0, m1, m2, m3;
-        int b0, b1, b2, b3;
-    } pq[QPL];
-    int qlen[QPL], pending[QPL];
-#pragma unroll
-    for (int i = 0; i < QPL; ++i) {
-        const int qi = (qblock * QPL + i) * BLOCK + tid;
-        active[i] = qi < n1;
-        qx[i] = active[i] ? knn_coord<SOA>(Q, n1, qi, 0) : c0;
-        qy[i] = active[i] ? knn_coord<SOA>(Q, n1, qi, 1) : c1;
-        qz[i] = active[i] ? knn_coord<SOA>(Q, n1, qi, 2) : c2;
-        const float px = (qx[i] - c0) * scale, py = (qy[i] - c1) * scale, pz = (qz[i] - c2) * scale;
-        ax[i] = -2.0f * px;
-        ay[i] = -2.0f * py;
-        az[i] = -2.0f * pz;
-        qn[i] = __builtin_fmaf(pz, pz, __builtin_fmaf(py, py, px * px));
-        const float qnorm = __builtin_sqrtf(qn[i]) * 1.000001f;
+    // ---- the lane's query ----
+    const int qi = qblock * BLOCK + tid;
+    const bool active = qi < n1;
+    const float qx = active ? knn_coord<SOA>(Q, n1, qi, 0) : c0;
+    const float qy = active ? knn_coord<SOA>(Q, n1, qi, 1) : c1;
+    const float qz = active ? knn_coord<SOA>(Q, n1, qi, 2) : c2;
+    float qn, slack_r;
+    bool usable;
+    // The query side of the 16 terms for the wave's two blocks of 32 queries, block h being the
+    // queries of the lanes of half h. This lane supplies terms 8 half .. 8 half + 7 of column
+    // lane % 32 in either block, from its own coordinates or, for the other half's block, its
+    // partner's. The T terms (.w) are written whenever the maximum has changed.
+    uint4 qterm[2];
+    {
+        const float px = (qx - c0) * scale, py = (qy - c1) * scale, pz = (qz - c2) * scale;
+        qn = __builtin_fmaf(pz, pz, __builtin_fmaf(py, py, px * px));
+        const float qnorm = __builtin_sqrtf(qn) * 1.000001f;
         const float r = kmax + qnorm;
-        if constexpr (MATRIX) {
-            slack_r[i] = r * r * 3.8146973e-06f + 1e-37f * scale2;  // 64 u R
-            usable[i] = qnorm <= 200.0f;                            // false for NaN
-            ax[i] = usable[i] ? ax[i] : 0.0f;
-            ay[i] = usable[i] ? ay[i] : 0.0f;
-            az[i] = usable[i] ? az[i] : 0.0f;
-        } else {
-            slack_r[i] = r * r * 1.9073486e-06f + 1e-37f;  // 32 u R
-            usable[i] = slack_r[i] < 1e30f;                  // false for NaN / inf / huge
-        }
-        // fill: keys 0..k-1 go to slots 0..k-1 (mink.cuh:63-72); unused slots stay at -inf
-        max_key[i] = 0.0f;
-        max_idx[i] = 0;
-        nan_slots[i] = 0u;
-        bool frozen = false;
-        ids[i].identity();
+        slack_r = r * r * 3.8146973e-06f + 1e-37f * scale2;  // 64 u R
+        usable = qnorm <= 200.0f;                            // false for NaN
+        const float ax = usable ? -2.0f * px : 0.0f, ay = usable ? -2.0f * py : 0.0f,
+                    az = usable ? -2.0f * pz : 0.0f;
+        const float ox = __shfl_xor(ax, 32), oy = __shfl_xor(ay, 32), oz = __shfl_xor(az, 32);
 #pragma unroll
-        for (int s = 0; s < KMAX; ++s)
-            kd[i][s] = NEG_INF_BITS;
-#pragma unroll
-        for (int s = 0; s < KMAX; ++s) {
-            if constexpr (KI_LDS)
-                ski(i, s) = (unsigned short)(s < k ? s : 0);
-            else
-                ki[i][s] = 0;
-            if constexpr (SORTED) {
-                if (s < k) {  // uniform
-                    const float d = tk_dist2<float>(knn_coord<SOA>(K, n2, s, 0),
-                                                    knn_coord<SOA>(K, n2, s, 1),
-                                                    knn_coord<SOA>(K, n2, s, 2), qx[i], qy[i], qz[i]);
-                    const bool isnan = d != d;
-                    const int x = isnan ? NEG_INF_BITS : __builtin_bit_cast(int, d);
-                    nan_slots[i] |= isnan ? (1u << s) : 0u;
-                    frozen |= isnan && s == 0;
-                    // Positions 0..s-1 hold the keys so far, all of lower slot numbers: key s
-                    // goes behind those that are >= it, the rest move down one position
-                    // (position s held the placeholder of slot s).
-                    int m = 0;
-#pragma unroll
-                    for (int p = 0; p < s; ++p)
-                        m += kd[i][p] >= x ? 1 : 0;
-#pragma unroll
-                    for (int p = s; p >= 1; --p)
-                        kd[i][p] = med3(kd[i][p - 1], kd[i][p], x);
-                    kd[i][0] = kd[i][0] > x ? kd[i][0] : x;
-                    if (s > 0)
-                        ids[i].make_room(m, s, (unsigned)s);
-                }
-                continue;
-            }
-            if (s < k) {  // uniform
-                const float d = tk_dist2<float>(knn_coord<SOA>(K, n2, s, 0),
-                                                knn_coord<SOA>(K, n2, s, 1),
-                                                knn_coord<SOA>(K, n2, s, 2), qx[i], qy[i], qz[i]);
-                const bool isnan = d != d;
-                kd[i][s] = isnan ? NEG_INF_BITS : __builtin_bit_cast(int, d);
-                if constexpr (!KI_LDS)
-                    ki[i][s] = s;
-                nan_slots[i] |= isnan ? (1u << s) : 0u;
-                frozen |= isnan && s == 0;
-                if (s == 0 || d > max_key[i]) {
-                    max_key[i] = d;
-                    max_idx[i] = s;
-                }
-            }
-        }
-        if constexpr (SORTED)
-            max_key[i] = __builtin_bit_cast(float, kd[i][0]);  // (-inf if every key is a NaN)
-        max_key[i] = frozen ? -INF : max_key[i];
-        pq[i] = Pending{0u, 0u, 0u, 0u, 0, 0, 0, 0};
-        qlen[i] = 0;
-        pending[i] = 0;
-    }
-
-    // MATRIX: the query side of the 16 terms for the wave's 2 QPL blocks of 32 queries.
-    // Block 2 i + h' holds query i of the lanes of half h'; this lane supplies terms
-    // 8 h .. 8 h + 7 of column lane % 32 in every block, from its own coordinates or, for
-    // the other half's blocks, its partner's. The T terms (.w) are written per chunk.
-    uint4 qterm[MATRIX ? 2 * QPL : 1];
-    if constexpr (MATRIX) {
-#pragma unroll
-        for (int i = 0; i < QPL; ++i) {
-            const float ox = __shfl_xor(ax[i], 32), oy = __shfl_xor(ay[i], 32),
-                        oz = __shfl_xor(az[i], 32);
-#pragma unroll
-            for (int hb = 0; hb < 2; ++hb) {  // the block owned by half hb
-                const bool own = half == hb;
-                const float X = own ? ax[i] : ox, Y = own ? ay[i] : oy, Z = own ? az[i] : oz;
-                const unsigned sx = tk_f16_split2(X), sy = tk_f16_split2(Y), sz = tk_f16_split2(Z);
-                const unsigned xh = sx & 0xffffu, yh = sy & 0xffffu, zh = sz & 0xffffu;
-                qterm[2 * i + hb] =
-                    half == 0 ? make_uint4(sx, xh | (yh << 16), (sy >> 16) | (yh << 16), 0u)
-                              : make_uint4(sz, zh | 0x3c000000u, 0x00003c00u, 0u);
-            }
+        for (int hb = 0; hb < 2; ++hb) {
+            const bool own = half == hb;
+            const float X = own ? ax : ox, Y = own ? ay : oy, Z = own ? az : oz;
+            const unsigned sx = tk_f16_split2(X), sy = tk_f16_split2(Y), sz = tk_f16_split2(Z);
+            const unsigned xh = sx & 0xffffu, yh = sy & 0xffffu, zh = sz & 0xffffu;
+            qterm[hb] = half == 0 ? make_uint4(sx, xh | (yh << 16), (sy >> 16) | (yh << 16), 0u)
+                                  : make_uint4(sz, zh | 0x3c000000u, 0x00003c00u, 0u);
         }
     }
 
-    // One service step: every query with a pending candidate takes its first one. Written
-    // without branches so that the chains of a lane's queries interleave.
+    // ---- the slots, in descending order of their distances. A NaN can only enter during the
+    // fill (a later key must compare below the maximum) and MinK never selects such a slot as
+    // maximum unless it is slot 0, in which case it never inserts again: here a NaN slot holds
+    // the pattern of -inf (below every distance) and is recomputed when the results are written,
+    // and a NaN in slot 0 freezes the query (maximum -inf: no key compares below it). Unused
+    // slots hold the double's -inf, below all others. ----
+    constexpr int NEG_INF_BITS = (int)0xff800000u;
+    const double UNUSED = -__builtin_huge_val();
+    double v[KMAX];
+    unsigned nan_slots = 0u;
+    bool frozen = false;
+#pragma unroll
+    for (int s = 0; s < KMAX; ++s)
+        v[s] = UNUSED;
+    // fill: keys 0..k-1 go to slots 0..k-1 (mink.cuh:63-72)
+#pragma unroll
+    for (int s = 0; s < KMAX; ++s) {
+        if (s < k) {  // uniform
+            const float d = tk_dist2<float>(knn_coord<SOA>(K, n2, s, 0), knn_coord<SOA>(K, n2, s, 1),
+                                            knn_coord<SOA>(K, n2, s, 2), qx, qy, qz);
+            const bool isnan = d != d;
+            nan_slots |= isnan ? (1u << s) : 0u;
+            frozen |= isnan && s == 0;
+            const double x = Slot::pack(isnan ? NEG_INF_BITS : __builtin_bit_cast(int, d),
+                                        ((unsigned)(KMAX - 1 - s) << Slot::KEY_BITS) | (unsigned)s);
+#pragma unroll
+            for (int p = s; p >= 1; --p)
+                v[p] = knn_max_f64(v[p], knn_min_f64(v[p - 1], x));
+            v[0] = knn_max_f64(v[0], x);
+        }
+    }
+    float max_key = frozen ? -INF : __builtin_bit_cast(float, Slot::distance(v[0]));
+    // Pending chunk masks, oldest first (bit 31 = first key of the chunk), and the key index of
+    // bit 31 of each. Named and no loops over the queue, so it stays in registers.
+    static_assert(CAP == 4, "the queue is written out for four entries");
+    unsigned m0 = 0u, m1 = 0u, m2 = 0u, m3 = 0u;
+    int b0 = 0, b1 = 0, b2 = 0, b3 = 0;
+    int qlen = 0, pending = 0;
+
+    // One service step: every query with a pending candidate takes its first one.
     auto service = [&]() {
-        float4 raw[QPL];
-        int kj[QPL];
-        bool has[QPL];
+        const bool has = qlen > 0;
+        // (an empty queue has m0 == 0: the bit number is then meaningless, the address
+        // below stays inside the buffer and nothing is inserted)
+        const int bit = __builtin_clz(m0 | 1u);
+        const int kj = b0 + bit;
+        // resident: candidates are never older than the previous stage (see below)
+        const float4 raw = sraw[kj & (2 * STAGE - 1)];
+        const unsigned rest = m0 & ~(0x80000000u >> bit);
+        const bool shift = has && rest == 0u;
+        m0 = shift ? m1 : rest;
+        b0 = shift ? b1 : b0;
+        m1 = shift ? m2 : m1;
+        b1 = shift ? b2 : b1;
+        m2 = shift ? m3 : m2;
+        b2 = shift ? b3 : b2;
+        m3 = shift ? 0u : m3;
+        qlen -= shift ? 1 : 0;
+        pending -= has ? 1 : 0;
+        const float d = tk_dist2<float>(raw.x, raw.y, raw.z, qx, qy, qz);
+        const bool ins = has && d < max_key;  // MinK's strict test (mink.cuh:74)
+        const int dbits = __builtin_bit_cast(int, d);
+        // The key takes the slot of the maximum, which leaves. With nothing that stays strictly
+        // above it, it is the next maximum: the flag puts it in front of its equals. A key that is
+        // not inserted sinks nowhere: above every pattern.
+        const unsigned low = (Slot::low(v[0]) & Slot::SLOT) | (unsigned)kj;
+        const unsigned flag = dbits >= Slot::distance(v[1]) ? Slot::FLAG : 0u;
+        const double x = Slot::pack(ins ? dbits : 0x7fe00000, low | flag);
 #pragma unroll
-        for (int i = 0; i < QPL; ++i) {
-            Pending &p = pq[i];
-            has[i] = qlen[i] > 0;
-            // (an empty queue has m0 == 0: the bit number is then meaningless, the address
-            // below stays inside the buffer and nothing is inserted)
-            const int bit = __builtin_clz(p.m0 | 1u);
-            kj[i] = p.b0 + bit;
-            // resident: candidates are never older than the previous stage (see below)
-            raw[i] = sraw[kj[i] & (2 * STAGE - 1)];
-            const unsigned rest = p.m0 & ~(0x80000000u >> bit);
-            const bool shift = has[i] && rest == 0u;
-            p.m0 = shift ? p.m1 : rest;
-            p.b0 = shift ? p.b1 : p.b0;
-            p.m1 = shift ? p.m2 : p.m1;
-            p.b1 = shift ? p.b2 : p.b1;
-            p.m2 = shift ? p.m3 : p.m2;
-            p.b2 = shift ? p.b3 : p.b2;
-            p.m3 = shift ? 0u : p.m3;
-            qlen[i] -= shift ? 1 : 0;
-            pending[i] -= has[i] ? 1 : 0;
-        }
-#pragma unroll
-        for (int i = 0; i < QPL; ++i) {
-            const float d = tk_dist2<float>(raw[i].x, raw[i].y, raw[i].z, qx[i], qy[i], qz[i]);
-            const bool ins = has[i] && d < max_key[i];  // MinK's strict test (mink.cuh:74)
-            const int dbits = __builtin_bit_cast(int, d);
-            if constexpr (SORTED) {
-                int(&v)[KMAX] = kd[i];
-                // a key that is not inserted sinks nowhere: above every pattern
-                const int x = ins ? dbits : INT_HIGHEST;
-                // m: how many of positions 1..KMAX-1 are >= x; last: the last of them
-                int last;
-                int m = knn_sorted_position<KMAX>(v, [&](int pivot) { return pivot >= x; },
-                                                  INT_LOWEST, last);
-                const unsigned slot = ids[i].head();  // of the maximum: x takes it
-                if (__builtin_amdgcn_ballot_w64(last == x) != 0) {  // uniform: equal distances
-                    // the same search for the positions strictly above x ...
-                    int unused;
-                    const int above = knn_sorted_position<KMAX>(
-                        v, [&](int pivot) { return pivot > x; }, INT_LOWEST, unused);
-                    // ... and positions above + 1 .. m hold x, in ascending slot order: x goes
-                    // behind those of lower slots
-                    const int equal = m - above;
-                    int before = 0;
-                    for (int q = 0; __builtin_amdgcn_ballot_w64(q < equal) != 0; ++q) {
-                        const unsigned other = ids[i].at((above + 1 + q) & (KMAX - 1));
-                        before += (q < equal && other < slot) ? 1 : 0;
-                    }
-                    m = above == 0 ? 0 : above + before;
-                }
-#pragma unroll
-                for (int p = 0; p < KMAX; ++p)
-                    v[p] = med3(v[p], p + 1 < KMAX ? v[p + 1] : INT_LOWEST, x);
-                ids[i].turn(m, slot);  // the head's slot goes with x to position m
-                if (ins)
-                    ski(i, slot) = (unsigned short)kj[i];
-                max_key[i] = ins ? __builtin_bit_cast(float, v[0]) : max_key[i];
-                continue;
-            }
-            // the key takes the slot of the maximum ...
-#pragma unroll
-            for (int s = 0; s < KMAX; ++s) {
-                const bool here = ins && s == max_idx[i];
-                kd[i][s] = here ? dbits : kd[i][s];
-                if constexpr (!KI_LDS)
-                    ki[i][s] = here ? kj[i] : ki[i][s];
-            }
-            if constexpr (KI_LDS) {
-                if (ins)
-                    ski(i, max_idx[i]) = (unsigned short)kj[i];
-            }
-            // ... and the new maximum is the largest pattern: it stays in the written slot
-            // when nothing is strictly above the new key, otherwise it is the first slot
-            // holding the largest pattern ((top - 1 - bits) is negative exactly there; the
-            // sign bits shifted together put slot 0 in the highest position).
-            int t[KMAX];
-#pragma unroll
-            for (int s = 0; s < KMAX; ++s)
-                t[s] = kd[i][s];
-#pragma unroll
-            for (int n = KMAX; n > 1; n = (n + 2) / 3) {
-#pragma unroll
-                for (int j = 0; 3 * j < n; ++j) {
-                    int v = t[3 * j];
-                    if (3 * j + 1 < n)
-                        v = t[3 * j + 1] > v ? t[3 * j + 1] : v;
-                    if (3 * j + 2 < n)
-                        v = t[3 * j + 2] > v ? t[3 * j + 2] : v;
-                    t[j] = v;
-                }
-            }
-            const int top = t[0];
-            const unsigned below = (unsigned)top - 1u;
-            constexpr int GS = 4;
-            unsigned eq = 0u;
-#pragma unroll
-            for (int g0 = 0; g0 < KMAX; g0 += GS) {
-                unsigned part = 0u;
-#pragma unroll
-                for (int s = g0; s < g0 + GS; ++s)
-                    part = __builtin_amdgcn_alignbit(part, below - (unsigned)kd[i][s], 31);
-                eq = (eq << GS) | part;
-            }
-            // (eq | 1 keeps the count defined; eq is never 0 when it matters)
-            const int first_top = __builtin_clz(eq | 1u) - (32 - KMAX);
-            const int new_idx = top != dbits ? first_top : max_idx[i];
-            max_key[i] = ins ? __builtin_bit_cast(float, top) : max_key[i];
-            max_idx[i] = ins ? new_idx : max_idx[i];
-        }
+        for (int p = 0; p < KMAX - 1; ++p)
+            v[p] = knn_max_f64(v[p + 1], knn_min_f64(v[p], x));
+        v[KMAX - 1] = knn_min_f64(v[KMAX - 1], x);
+        max_key = ins ? __builtin_bit_cast(float, Slot::distance(v[0])) : max_key;
         // Keep the loop-carried state where it is: without this the register allocator
         // rotates some forty values through copies on every step.
+        asm volatile("" : "+v"(m0), "+v"(m1), "+v"(m2), "+v"(m3));
+        asm volatile("" : "+v"(b0), "+v"(b1), "+v"(b2), "+v"(b3));
+        asm volatile("" : "+v"(qlen), "+v"(pending), "+v"(max_key));
 #pragma unroll
-        for (int i = 0; i < QPL; ++i) {
-            asm volatile("" : "+v"(pq[i].m0), "+v"(pq[i].m1), "+v"(pq[i].m2), "+v"(pq[i].m3));
-            asm volatile("" : "+v"(pq[i].b0), "+v"(pq[i].b1), "+v"(pq[i].b2), "+v"(pq[i].b3));
-            asm volatile("" : "+v"(qlen[i]), "+v"(pending[i]), "+v"(max_key[i]), "+v"(max_idx[i]));
-            if constexpr (SORTED)
-                ids[i].keep();
-#pragma unroll
-            for (int s = 0; s < KMAX; ++s) {
-                asm volatile("" : "+v"(kd[i][s]));
-                if constexpr (!KI_LDS)
-                    asm volatile("" : "+v"(ki[i][s]));
-            }
-        }
+        for (int s = 0; s < KMAX; ++s)
+            asm volatile("" : "+v"(v[s]));
     };
     auto must_serve = [&]() {
-        bool need = false;
-#pragma unroll
-        for (int i = 0; i < QPL; ++i)
-            need |= pending[i] >= T || qlen[i] >= CAP;
-        return __builtin_amdgcn_ballot_w64(need) != 0;
+        return __builtin_amdgcn_ballot_w64(pending >= T || qlen >= CAP) != 0;
     };
 
     // ---- sweep: keys centred and staged in two LDS buffers, one barrier per stage ----
     const int nstages = (n2 + STAGE - 1) / STAGE;
-    float4 pre[PER], pre_raw[PER];
+    float4 pre[PER];
     auto fetch = [&](int st) {
 #pragma unroll
         for (int r = 0; r < PER; ++r) {
             const int kj = st * STAGE + r * BLOCK + tid;
-            float4 e = make_float4(0.0f, 0.0f, 0.0f, INF);  // past the end: never a candidate
-            float4 w = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            if (kj < n2) {
-                w.x = knn_coord<SOA>(K, n2, kj, 0);
-                w.y = knn_coord<SOA>(K, n2, kj, 1);
-                w.z = knn_coord<SOA>(K, n2, kj, 2);
-                e.x = w.x - c0;
-                e.y = w.y - c1;
-                e.z = w.z - c2;
-                e.w = __builtin_fmaf(e.z, e.z, __builtin_fmaf(e.y, e.y, e.x * e.x));
-            }
-            pre[r] = e;
-            pre_raw[r] = w;
+            pre[r] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (kj < n2)
+                pre[r] = make_float4(knn_coord<SOA>(K, n2, kj, 0), knn_coord<SOA>(K, n2, kj, 1),
+                                     knn_coord<SOA>(K, n2, kj, 2), 1.0f);
         }
     };
     auto stash = [&](int buf) {
 #pragma unroll
         for (int r = 0; r < PER; ++r) {
             const int j = r * BLOCK + tid;  // key within the stage
-            if constexpr (MATRIX) {
-                const float4 e = pre[r];
-                const float x = e.x * scale, y = e.y * scale, z = e.z * scale;
-                const float n = e.w * scale2;  // (+inf past the end)
-                const unsigned sx = tk_f16_split2(x), sy = tk_f16_split2(y), sz = tk_f16_split2(z);
-                const unsigned xh = sx & 0xffffu, yh = sy & 0xffffu, zh = sz & 0xffffu;
-                const unsigned sn = tk_f16_split2(n);
-                const bool exists = e.w < INF || e.w != e.w;
-                const unsigned n0 = exists ? (sn & 0xffffu) : 0x7c00u, n1 = exists ? (sn >> 16) : 0u;
-                // row of the tile: lane half h of the result holds rows 8 a + 4 h + c
-                const int row = ((j & 12) << 1) | ((j & 16) >> 2) | (j & 3);
-                uint4 *t = sterm + buf * (STAGE * 2) + (j >> 5) * 64 + row;
-                t[0] = make_uint4(xh * 0x10001u, (sx >> 16) | (yh << 16), yh | (sy & 0xffff0000u),
-                                  0x3c003c00u);
-                t[32] = make_uint4(zh * 0x10001u, (sz >> 16) | (n0 << 16), n1, 0x3c003c00u);
-            } else {
-                reinterpret_cast<float4 *>(skey)[buf * STAGE + j] = pre[r];
-            }
-            sraw[buf * STAGE + j] = pre_raw[r];
+            const bool exists = pre[r].w != 0.0f;
+            const float ex = pre[r].x - c0, ey = pre[r].y - c1, ez = pre[r].z - c2;
+            const float x = ex * scale, y = ey * scale, z = ez * scale;
+            const float n = __builtin_fmaf(ez, ez, __builtin_fmaf(ey, ey, ex * ex)) * scale2;
+            const unsigned sx = tk_f16_split2(x), sy = tk_f16_split2(y), sz = tk_f16_split2(z);
+            const unsigned xh = sx & 0xffffu, yh = sy & 0xffffu, zh = sz & 0xffffu;
+            const unsigned sn = tk_f16_split2(n);
+            // (past the end: an infinite norm, never a candidate)
+            const unsigned n0 = exists ? (sn & 0xffffu) : 0x7c00u, n1 = exists ? (sn >> 16) : 0u;
+            // row of the tile: lane half h of the result holds rows 8 a + 4 h + c
+            const int row = ((j & 12) << 1) | ((j & 16) >> 2) | (j & 3);
+            uint4 *t = sterm + buf * (STAGE * 2) + (j >> 5) * 64 + row;
+            t[0] = make_uint4(xh * 0x10001u, (sx >> 16) | (yh << 16), yh | (sy & 0xffff0000u),
+                              0x3c003c00u);
+            t[32] = make_uint4(zh * 0x10001u, (sz >> 16) | (n0 << 16), n1, 0x3c003c00u);
+            sraw[buf * STAGE + j] = pre[r];
         }
     };
     __syncthreads();
     fetch(0);
     stash(0);
     __syncthreads();
+    bool stale = true;  // the T terms do not belong to the maximum any more
     for (int st = 0; st < nstages; ++st) {
         const int stage0 = st * STAGE;
         if (st + 1 < nstages)
             fetch(st + 1);
-        const float4 *sbuf = reinterpret_cast<const float4 *>(skey) + (st & 1) * STAGE;
         const int left = n2 - stage0;
         const int cnt = left < STAGE ? left : STAGE;
         for (int c0k = 0; c0k < cnt; c0k += CHUNK) {
             const int first = stage0 + c0k;  // key index of bit 31
-            float thr[QPL];
-            unsigned mask[QPL];
-#pragma unroll
-            for (int i = 0; i < QPL; ++i) {
-                if constexpr (MATRIX) {  // rescaled units; slack 64 u R + 48 u M
-                    const float m = max_key[i] * scale2;
-                    thr[i] = (m - qn[i]) + __builtin_fmaf(m, 2.8610229e-06f, slack_r[i]);
-                } else {
-                    thr[i] = (max_key[i] - qn[i]) +
-                             __builtin_fmaf(max_key[i], 9.5367432e-07f, slack_r[i]);
-                }
-                mask[i] = 0u;
+            const tk_f16x8 ka = __builtin_bit_cast(
+                tk_f16x8, sterm[(st & 1) * (STAGE * 2) + (c0k >> 5) * 64 + lane]);
+            if (stale) {  // uniform
+                const float m = max_key * scale2;  // rescaled units; slack 64 u R + 48 u M
+                const float thr = (m - qn) + __builtin_fmaf(m, 2.8610229e-06f, slack_r);
+                const unsigned tp = tk_f16_split2(-thr);
+                qterm[0].w = half == 0 ? tp : 0u;
+                qterm[1].w = half == 1 ? tp : 0u;
+                stale = false;
             }
-            if constexpr (MATRIX) {
-                const tk_f16x8 ka = __builtin_bit_cast(
-                    tk_f16x8, sterm[(st & 1) * (STAGE * 2) + (c0k >> 5) * 64 + lane]);
+            unsigned m16[2];
+            const tk_f32x16 zero = {};
 #pragma unroll
-                for (int i = 0; i < QPL; ++i) {
-                    const unsigned tp = tk_f16_split2(-thr[i]);
-                    qterm[2 * i].w = half == 0 ? tp : 0u;
-                    qterm[2 * i + 1].w = half == 1 ? tp : 0u;
+            for (int g = 0; g < 2; ++g) {
+                const tk_f32x16 acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                    ka, __builtin_bit_cast(tk_f16x8, qterm[g]), zero, 0, 0, 0);
+                unsigned m = 0u;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const float t = acc[r];  // (a bit_cast applied to acc[r] itself reads element 0)
+                    m = __builtin_amdgcn_alignbit(m, __builtin_bit_cast(unsigned, t), 31);
                 }
-                const tk_f32x16 zero = {};
-                unsigned m16[2 * QPL];
-#pragma unroll
-                for (int g = 0; g < 2 * QPL; ++g) {
-                    const tk_f32x16 acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-                        ka, __builtin_bit_cast(tk_f16x8, qterm[g]), zero, 0, 0, 0);
-                    unsigned m = 0u;
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        const float t = acc[r];  // (a bit_cast applied to acc[r] itself reads element 0)
-                        m = __builtin_amdgcn_alignbit(m, __builtin_bit_cast(unsigned, t), 31);
-                    }
-                    m16[g] = m;
-                }
-                // rows of this half: keys 16 h .. 16 h + 15 of the chunk, first key in the
-                // highest bit; the other half's rows of this lane's blocks come from lane ^ 32
-                if constexpr (QPL == 2) {
-                    const unsigned send =
-                        half == 0 ? (m16[1] | (m16[3] << 16)) : (m16[0] | (m16[2] << 16));
-                    const unsigned recv = __shfl_xor(send, 32);
-                    const unsigned own0 = half == 0 ? m16[0] : m16[1],
-                                   own1 = half == 0 ? m16[2] : m16[3];
-                    const unsigned oth0 = recv & 0xffffu, oth1 = recv >> 16;
-                    mask[0] = half == 0 ? ((own0 << 16) | oth0) : ((oth0 << 16) | own0);
-                    mask[1] = half == 0 ? ((own1 << 16) | oth1) : ((oth1 << 16) | own1);
-                } else {
-                    const unsigned recv = __shfl_xor(half == 0 ? m16[1] : m16[0], 32);
-                    const unsigned own = half == 0 ? m16[0] : m16[1];
-                    mask[0] = half == 0 ? ((own << 16) | recv) : ((recv << 16) | own);
-                }
-            } else {
-            const float4 *ck = sbuf + c0k;
-            // Groups of G keys: the next group is read from LDS before the current one is
-            // used, and the G scores of a query are independent chains.
-            constexpr int G = 4;
-            float4 cur[G];
-#pragma unroll
-            for (int g = 0; g < G; ++g)
-                cur[g] = ck[g];
-#pragma unroll
-            for (int j = 0; j < CHUNK; j += G) {
-                float4 nxt[G];
-#pragma unroll
-                for (int g = 0; g < G; ++g)
-                    nxt[g] = ck[j + G + g];  // runs into the next chunk / the pad at the end
-#pragma unroll
-                for (int i = 0; i < QPL; ++i) {
-                    float t[G];
-#pragma unroll
-                    for (int g = 0; g < G; ++g)
-                        t[g] = cur[g].w - thr[i];
-#pragma unroll
-                    for (int g = 0; g < G; ++g)
-                        t[g] = __builtin_fmaf(cur[g].z, az[i], t[g]);
-#pragma unroll
-                    for (int g = 0; g < G; ++g)
-                        t[g] = __builtin_fmaf(cur[g].y, ay[i], t[g]);
-#pragma unroll
-                    for (int g = 0; g < G; ++g)
-                        t[g] = __builtin_fmaf(cur[g].x, ax[i], t[g]);
-#pragma unroll
-                    for (int g = 0; g < G; ++g)
-                        mask[i] = __builtin_amdgcn_alignbit(mask[i],
-                                                            __builtin_bit_cast(unsigned, t[g]), 31);
-                }
-#pragma unroll
-                for (int g = 0; g < G; ++g)
-                    cur[g] = nxt[g];
+                m16[g] = m;
             }
-            }
+            // Lane l has rows (keys) 16 half .. of column l % 32 of both blocks, the first key in
+            // the highest bit. The upper lanes of block 0 change places with the lower ones of
+            // block 1: then it has both halves of the rows of its own column of its own block.
+            const auto both = __builtin_amdgcn_permlane32_swap(m16[0], m16[1], false, false);
+            const unsigned mask = ((unsigned)both[0] << 16) | (unsigned)both[1];
             // Keys that do not exist, or that the fill phase took, are no candidates.
             int vlo = k - first;
             vlo = vlo < 0 ? 0 : (vlo > CHUNK ? CHUNK : vlo);
@@ -1151,27 +807,24 @@ __global__ __launch_bounds__(LANES) void knn_filter_kernel_f32(
             vhi = vhi > CHUNK ? CHUNK : vhi;
             unsigned valid = (vlo >= CHUNK) ? 0u : (0xffffffffu >> vlo);
             valid &= (vhi >= CHUNK) ? 0xffffffffu : ~(0xffffffffu >> vhi);
-#pragma unroll
-            for (int i = 0; i < QPL; ++i) {
-                unsigned m = usable[i] ? mask[i] : 0xffffffffu;
-                m = active[i] ? (m & valid) : 0u;
-                const bool nz = m != 0u;
-                Pending &p = pq[i];
-                const int at = nz ? qlen[i] : -1;
-                p.m0 = at == 0 ? m : p.m0;
-                p.b0 = at == 0 ? first : p.b0;
-                p.m1 = at == 1 ? m : p.m1;
-                p.b1 = at == 1 ? first : p.b1;
-                p.m2 = at == 2 ? m : p.m2;
-                p.b2 = at == 2 ? first : p.b2;
-                p.m3 = at == 3 ? m : p.m3;
-                p.b3 = at == 3 ? first : p.b3;
-                qlen[i] += nz ? 1 : 0;
-                pending[i] += __builtin_popcount(m);
-            }
+            unsigned m = usable ? mask : 0xffffffffu;
+            m = active ? (m & valid) : 0u;
+            const bool nz = m != 0u;
+            const int at = nz ? qlen : -1;
+            m0 = at == 0 ? m : m0;
+            b0 = at == 0 ? first : b0;
+            m1 = at == 1 ? m : m1;
+            b1 = at == 1 ? first : b1;
+            m2 = at == 2 ? m : m2;
+            b2 = at == 2 ? first : b2;
+            m3 = at == 3 ? m : m3;
+            b3 = at == 3 ? first : b3;
+            qlen += nz ? 1 : 0;
+            pending += __builtin_popcount(m);
             // (two steps per trip: the loop-carried state is copied between registers once
             // per trip, some forty moves)
             while (must_serve()) {
+                stale = true;
                 service();
                 if (!must_serve())
                     break;
@@ -1181,13 +834,8 @@ __global__ __launch_bounds__(LANES) void knn_filter_kernel_f32(
         if (st + 1 < nstages) {
             // The next stage replaces the previous one in LDS: whatever is still pending
             // from it is served first (the queue is in key order, so its head tells).
-            for (;;) {
-                bool old = false;
-#pragma unroll
-                for (int i = 0; i < QPL; ++i)
-                    old |= qlen[i] > 0 && pq[i].b0 < stage0;
-                if (!__builtin_amdgcn_ballot_w64(old))
-                    break;
+            while (__builtin_amdgcn_ballot_w64(qlen > 0 && b0 < stage0) != 0) {
+                stale = true;
                 service();
             }
             __syncthreads();  // every wave is done with the previous stage
@@ -1195,15 +843,8 @@ __global__ __launch_bounds__(LANES) void knn_filter_kernel_f32(
         }
         __syncthreads();
     }
-    for (;;) {
-        bool any = false;
-#pragma unroll
-        for (int i = 0; i < QPL; ++i)
-            any |= qlen[i] > 0;
-        if (!__builtin_amdgcn_ballot_w64(any))
-            break;
+    while (__builtin_amdgcn_ballot_w64(qlen > 0) != 0)
         service();
-    }
 
     // ---- results: a wave's 64 queries own 64 * k consecutive output elements; the slots
     // are transposed through LDS (row stride KMAX + 1: no bank conflicts) so that the
@@ -1214,39 +855,25 @@ __global__ __launch_bounds__(LANES) void knn_filter_kernel_f32(
     int *const ibuf = reinterpret_cast<int *>(tbuf + TK_WAVE * ROW);
     static_assert(TWAVES * 2 * TK_WAVE * ROW == TRANSPOSE_FLOATS, "LDS for the transpose");
     auto emit = [&]() {
+        const int q0 = qblock * BLOCK + wave * TK_WAVE;  // first query of the wave
 #pragma unroll
-    for (int i = 0; i < QPL; ++i) {
-        const int q0 = (qblock * QPL + i) * BLOCK + wave * TK_WAVE;  // first query of the wave
-        if constexpr (SORTED) {
-#pragma unroll
-            for (int p = 0; p < KMAX; ++p) {
-                const int slot = (int)ids[i].at(p);
-                tbuf[lane * ROW + slot] = __builtin_bit_cast(float, kd[i][p]);
-                ibuf[lane * ROW + p] = (int)ski(i, p);
-            }
-            if (nan_slots[i] != 0u) {  // NaNs of the fill, still in their slots
-#pragma unroll
-                for (int s = 0; s < KMAX; ++s) {
-                    if (s < k && ((nan_slots[i] >> s) & 1u))
-                        tbuf[lane * ROW + s] = tk_dist2<float>(
-                            knn_coord<SOA>(K, n2, s, 0), knn_coord<SOA>(K, n2, s, 1),
-                            knn_coord<SOA>(K, n2, s, 2), qx[i], qy[i], qz[i]);
-                }
+        for (int p = 0; p < KMAX; ++p) {
+            if (p < k) {  // uniform
+                const int slot = Slot::slot(v[p]);
+                tbuf[lane * ROW + slot] = __builtin_bit_cast(float, Slot::distance(v[p]));
+                ibuf[lane * ROW + slot] = (int)(Slot::low(v[p]) & Slot::KEY);
             }
         }
+        if (nan_slots != 0u) {  // NaNs of the fill, still in their slots
 #pragma unroll
-        for (int s = 0; s < (SORTED ? 0 : KMAX); ++s) {
-            float d = __builtin_bit_cast(float, kd[i][s]);
-            if (s < k && ((nan_slots[i] >> s) & 1u))  // a NaN of the fill, still in its slot
-                d = tk_dist2<float>(knn_coord<SOA>(K, n2, s, 0), knn_coord<SOA>(K, n2, s, 1),
-                                    knn_coord<SOA>(K, n2, s, 2), qx[i], qy[i], qz[i]);
-            kd[i][s] = __builtin_bit_cast(int, d);
-            tbuf[lane * ROW + s] = d;
-            if constexpr (KI_LDS)
-                ibuf[lane * ROW + s] = (int)ski(i, s);
-            else
-                ibuf[lane * ROW + s] = ki[i][s];
+            for (int s = 0; s < KMAX; ++s) {
+                if (s < k && ((nan_slots >> s) & 1u))
+                    tbuf[lane * ROW + s] = tk_dist2<float>(
+                        knn_coord<SOA>(K, n2, s, 0), knn_coord<SOA>(K, n2, s, 1),
+                        knn_coord<SOA>(K, n2, s, 2), qx, qy, qz);
+            }
         }
+        tk_wave_fence();
         const int nvalid = n1 - q0 < TK_WAVE ? n1 - q0 : TK_WAVE;  // may be <= 0
         const int total = nvalid * k;
         float *od = distance + ((int64_t)b * n1 + q0) * k;
@@ -1261,15 +888,12 @@ __global__ __launch_bounds__(LANES) void knn_filter_kernel_f32(
                 oi[e] = (int64_t)ibuf[row * ROW + col];
             }
         }
-        if constexpr (WEIGHTS && KMAX >= 3) {  // k == 3
-            if (active[i]) {
-                const float d3[3] = {__builtin_bit_cast(float, kd[i][0]),
-                                     __builtin_bit_cast(float, kd[i][1]),
-                                     __builtin_bit_cast(float, kd[i][2])};
+        if constexpr (WEIGHTS) {  // k == 3
+            if (active) {
+                const float d3[3] = {tbuf[lane * ROW], tbuf[lane * ROW + 1], tbuf[lane * ROW + 2]};
                 knn_three_weights<float>(d3, eps, weight + ((int64_t)b * n1 + q0 + lane) * 3);
             }
         }
-    }
     };
     if constexpr (NW == TWAVES) {
         emit();
@@ -1804,30 +1428,16 @@ void knn_launch(const T *query, const T *key, T *distance, int64_t *index, int64
                            index, weight, eps, bpb, n1, n2, k);
 }
 
-// Where the pre-filtered kernel is the fastest route for k <= 16, from timing it against
-// every other kernel here on an MI355X (k = 1..16, 128 to 524288 queries, 128 to 65536
-// keys, 1100 shapes): 1.1-2.0 times faster inside these bounds, 0.7-1.0 outside. Short key
-// clouds do not amortise its prologue (two passes over the keys per workgroup); with few
-// queries and very long clouds the kernels that share the keys of 64 queries among several
-// waves win, from k = 5 on.
-inline bool knn_filter_pays(int64_t queries, int n2, int k)
-{
-    if (k <= 4)
-        return n2 >= 512 || (n2 >= 256 && queries >= 4096);
-    if (k > 16)  // 32 slots as a sorted list, key indices in LDS; the tree kernel keeps
-                 // short clouds with many queries (B=24, 4096 x 700: 117 against 137 us)
-        return n2 <= 65536 && queries >= 4096 && (n2 >= 1024 || (n2 >= 512 && queries <= 32768));
-    if (queries < 32768 && n2 > (k <= 8 ? 8192 : 32768))
-        return false;
-    return n2 >= (k <= 8 ? 512 : 1024) || (n2 >= 512 && queries >= 131072);
-}
-
-// Whether knn_filter_launch takes this launch: the one test both entry points and the
-// launch itself go by.
+// Whether knn_filter_launch takes this launch: the one test both entry points and the launch itself
+// go by. Behind the wave kernel, which has the launches of few queries, it is the fastest route
+// wherever a cloud holds 64 keys (timed against every other kernel here at 19000 to 262144 queries, 33 to
+// 70000 keys, k = 3 to 32; us, others and this one: 19000 queries on 64 keys k = 3 12, 12, k = 16 22, 18,
+// k = 32 28, 28; 65536 on 256, k = 8 33, 20, on 768, k = 16 97, 41, on 70000, k = 20 4470, 900; on 33
+// keys k = 32 16, 20). A slot has 27 bits or more for its key, of 32 slots 26.
 inline bool knn_filter_takes(int64_t B, int n1, int n2, int k)
 {
-    const int64_t bpb = ((int64_t)n1 + 511) / 512;
-    return k <= 32 && knn_filter_pays(B * n1, n2, k) && B * bpb <= TK_MAX_I32;
+    const int64_t bpb = ((int64_t)n1 + 255) / 256;
+    return k <= 32 && n2 >= 64 && (k <= 4 || n2 <= (k <= 16 ? 1 << 27 : 1 << 26)) && B * bpb <= TK_MAX_I32;
 }
 
 template <int KMAX, bool SOA, bool WEIGHTS, int LANES>
@@ -1835,25 +1445,8 @@ int knn_filter_launch_as(const float *query, const float *key, float *distance, 
                          float *weight, float eps, int64_t B, int n1, int n2, int k, hipStream_t s)
 {
     const int64_t bpb = ((int64_t)n1 + LANES - 1) / LANES;
-    if constexpr (KMAX >= 8) {  // (4 slots: the slot-ordered registers are 2-7 % faster)
-        if (n2 <= 65536) {  // the slots' key indices in LDS, 16 bits each
-            constexpr auto kernel =
-                knn_filter_kernel_f32<KMAX, 1, SOA, WEIGHTS, true, LANES, true, !WEIGHTS>;
-            constexpr int lds = KMAX * LANES * (int)sizeof(unsigned short);
-            const int allowed = tk_allow_dynamic_lds<kernel>(lds);
-            if (allowed != TK3D_OK)
-                return allowed;
-            hipLaunchKernelGGL(kernel, dim3((unsigned)(B * bpb)), dim3(LANES), lds, s, query, key,
-                               distance, index, weight, eps, (int)bpb, n1, n2, k);
-            return tk_launch_status();
-        }
-        if constexpr (KMAX > 16)
-            return TK3D_ERR_UNSUPPORTED;  // 32 slots exist as a sorted list only
-    }
-    if constexpr (KMAX <= 16)
-        hipLaunchKernelGGL((knn_filter_kernel_f32<KMAX, 1, SOA, WEIGHTS, true, LANES>),
-                           dim3((unsigned)(B * bpb)), dim3(LANES), 0, s, query, key, distance,
-                           index, weight, eps, (int)bpb, n1, n2, k);
+    hipLaunchKernelGGL((knn_filter_kernel_f32<KMAX, SOA, WEIGHTS, LANES>), dim3((unsigned)(B * bpb)),
+                       dim3(LANES), 0, s, query, key, distance, index, weight, eps, (int)bpb, n1, n2, k);
     return tk_launch_status();
 }
 
@@ -1862,21 +1455,21 @@ int knn_filter_launch(const float *query, const float *key, float *distance, int
                       float *weight, float eps, int64_t B, int n1, int n2, int k, hipStream_t s,
                       bool whatever_the_size = false)
 {
-    // One query per lane, 512 lanes: two workgroups (16 waves) per CU. Two queries per lane
-    // in 256 lanes need twice the registers, which leaves two waves per SIMD, and were 1.1
-    // to 1.4 times slower on every shape (k = 16 at B=32, 8192 x 2048: 222 -> 191 us).
-    // A launch of few such workgroups leaves CUs without one: 256 lanes then (128 workgroups,
-    // B=8, 8192 x 2048: k = 3 52 -> 48 us, k = 16 96 -> 85 us, k = 32 189 -> 142 us; at 160
-    // workgroups with up to 8 slots, at 192 with more, the larger workgroup wins: its staged
-    // keys serve more queries).
-    const int64_t bpb = ((int64_t)n1 + 511) / 512;
-    if (B * bpb > TK_MAX_I32 || !(whatever_the_size || knn_filter_takes(B, n1, n2, k)))
+    // 512 lanes: two workgroups (16 waves) per CU. A launch of few such workgroups leaves CUs
+    // without one: 256 lanes then (128 workgroups, B=8, 8192 x 2048, with a list of nibbles: k = 3 52 ->
+    // 48 us, k = 16 96 -> 85 us; at 160 workgroups with up to 8 slots, at 192 with more, the larger
+    // workgroup wins: its staged keys serve more queries). 32 slots leave room for two waves per SIMD,
+    // which 256 lanes use better from 131072 queries on (k = 20 226, 211 us) and no worse below.
+    if (!(whatever_the_size || knn_filter_takes(B, n1, n2, k)))
         return TK3D_ERR_UNSUPPORTED;
-    if (B * bpb <= (KMAX <= 8 ? 128 : 160))
-        return knn_filter_launch_as<KMAX, SOA, WEIGHTS, 256>(query, key, distance, index, weight,
-                                                             eps, B, n1, n2, k, s);
-    return knn_filter_launch_as<KMAX, SOA, WEIGHTS, 512>(query, key, distance, index, weight, eps,
-                                                         B, n1, n2, k, s);
+    if constexpr (KMAX <= 16) {
+        const int64_t bpb = ((int64_t)n1 + 511) / 512;
+        if (B * bpb > (KMAX <= 8 ? 128 : 160))
+            return knn_filter_launch_as<KMAX, SOA, WEIGHTS, 512>(query, key, distance, index, weight,
+                                                                 eps, B, n1, n2, k, s);
+    }
+    return knn_filter_launch_as<KMAX, SOA, WEIGHTS, 256>(query, key, distance, index, weight, eps, B,
+                                                         n1, n2, k, s);
 }
 
 // Rows of k <= 64 results in place: ascending distance (equal ones in slot order, NaNs last, as a
@@ -2264,8 +1857,9 @@ int tk3d_debug_knn_filter_f32(const float *query, const float *key, int64_t B, i
         return TK3D_ERR_BAD_SIZE;
     if (k <= 0 || k > N2)
         return TK3D_ERR_BAD_K;
-    if (k > 16 || N2 < 256 || N1 > TK_MAX_I32 / 4 || N2 > TK_MAX_I32 / 4 ||
-        !tk_fits(TK_MAX_ELEMS, B, N1, k) || !tk_fits(TK_MAX_ELEMS, B, N2, 3))
+    if (k > 32 || N1 > TK_MAX_I32 / 4 || N2 > TK_MAX_I32 / 4 ||
+        !tk_fits(TK_MAX_ELEMS, B, N1, k) || !tk_fits(TK_MAX_ELEMS, B, N2, 3) ||
+        N2 > ((int64_t)1 << 26) || !tk_fits(TK_MAX_I32, B, (N1 + 255) / 256))
         return TK3D_ERR_UNSUPPORTED;
     if (B * N1 == 0)
         return TK3D_OK;
@@ -2279,8 +1873,11 @@ int tk3d_debug_knn_filter_f32(const float *query, const float *key, int64_t B, i
     if (k <= 8)
         return knn_filter_launch<8, false, false>(query, key, distance, index, nullptr, 0.0f, B,
                                                   n1, n2, kk, s, true);
-    return knn_filter_launch<16, false, false>(query, key, distance, index, nullptr, 0.0f, B, n1,
-                                               n2, kk, s, true);
+    if (k <= 16)
+        return knn_filter_launch<16, false, false>(query, key, distance, index, nullptr, 0.0f, B, n1,
+                                                   n2, kk, s, true);
+    return knn_filter_launch<32, false, false>(query, key, distance, index, nullptr, 0.0f, B, n1, n2,
+                                               kk, s, true);
 }
 
 }  // extern "C"

@@ -71,7 +71,7 @@ int tk3d_debug_knn_wave_f32(const float *query, const float *key, int channels_f
                             void *stream);
 
 /* tk3d_knn_distance_f32 through the pre-filtered kernel (knn_filter_kernel_f32, scores on
- * the matrix cores) whatever the launch size; k <= 16 and at least 256 keys. */
+ * the matrix cores) whatever the launch size; k <= 32. */
 int tk3d_debug_knn_filter_f32(const float *query, const float *key, int64_t B, int64_t N1,
                               int64_t N2, int64_t k, float *distance, int64_t *index,
                               void *stream);
