@@ -378,12 +378,12 @@ __global__ __launch_bounds__(KNN_BLOCK) void knn_batched_kernel_f32(
 // a float is one of a NaN or an infinity up there, zero is a (kept) subnormal, the negative patterns
 // of the placeholders are below all others.
 template <int KMAX> struct KnnSlot {
-    static constexpr int SLOT_BITS = KMAX == 32 ? 5 : KMAX == 16 ? 4 : KMAX == 8 ? 3 : 2;
+    static constexpr int SLOT_BITS = KMAX == 64 ? 6 : KMAX == 32 ? 5 : KMAX == 16 ? 4 : KMAX == 8 ? 3 : 2;
     static constexpr int KEY_BITS = 31 - SLOT_BITS;
     static constexpr unsigned FLAG = 0x80000000u;
     static constexpr unsigned SLOT = (unsigned)(KMAX - 1) << KEY_BITS;  // mask of the slot's bits
     static constexpr unsigned KEY = (1u << KEY_BITS) - 1u;
-    static_assert((1 << SLOT_BITS) == KMAX, "4, 8, 16 or 32 slots");
+    static_assert((1 << SLOT_BITS) == KMAX, "4 to 64 slots");
     static __device__ __forceinline__ double pack(int distance, unsigned low)
     {
         return __builtin_bit_cast(double, ((unsigned long long)(unsigned)distance << 32) | low);
@@ -407,6 +407,12 @@ __device__ __forceinline__ double knn_min_f64(double a, double b)
 {
     double o;
     asm("v_min_f64 %0, %1, %2" : "=v"(o) : "v"(a), "v"(b));
+    return o;
+}
+__device__ __forceinline__ double knn_min_f64_uniform(double a, double b)  // b wave-uniform
+{
+    double o;
+    asm("v_min_f64 %0, %1, %2" : "=v"(o) : "v"(a), "s"(b));
     return o;
 }
 __device__ __forceinline__ double knn_max_f64(double a, double b)
@@ -1166,39 +1172,24 @@ int knn_tree_launch(const T *query, const T *key, T *distance, int64_t *index,
 //
 // With a lane per query a launch needs 65536 queries to give every SIMD a wave, and an insertion
 // is a chain of dependent LDS or register steps for the whole wave. Here a wave has ONE query and
-// up to 64 slots, a slot per lane: 64 keys are measured at once, and those below the maximum are
+// up to 64 slots, one per lane: 64 keys are measured at once, and those below the maximum are
 // inserted one after the other in key order, which are MinK's insertions in MinK's order. The
-// kernel is bound by what an insertion issues, about k (1 + ln(N2 / k)) times per query in random
-// key order: two selects and a maximum over the lanes that hold slots (4, 5 or 6 steps). (A list
-// of the lanes in descending order, which needs no maximum, moves three values per insertion and
-// was 1.1 to 1.3 times slower.)
-// Distances are kept as bit patterns, which order as integers; a NaN is -1 in a slot, where no
-// maximum picks it, and above every maximum as a candidate, where no comparison takes it.
+// kernel is bound by the chain of an insertion, about k (1 + ln(N2 / k)) times per query in random key
+// order. The lanes hold the slots in descending order, as the doubles of the kernel above
+// (distance, flag, slot, key; KnnSlot): the head leaves, and a lane takes the larger of its lower
+// neighbour's and the smaller of its own and the new key's - two moves between lanes, a minimum and a
+// maximum, where slots that stay in their lanes take two selects and a maximum over the lanes (4, 5 or
+// 6 steps). A list of the lanes that moves distance, slot and key by selects was slower than either.
+// us, before and now: 4 x 512 queries, 10000 keys,
+// k = 64 57.6, 47.6, k = 16 31.9, 28.1; 8 x 2048 on 2048 k = 20 61, 56, k = 64 125, 112; 1 x 16384 on 16384 k = 64
+// 284, 262; on 128 keys, where ordering the first k counts, k = 64 10.6, 12.5. Tried: insertions in a row
+// without a look at the new maximum (longer for few neighbours, whose maximum falls fast).
+// A NaN of the fill holds the pattern of -inf, below every distance; one in slot 0 freezes the query,
+// and no comparison takes one as a candidate.
 
-// Maximum over the first KMAX lanes.
-template <int KMAX> __device__ __forceinline__ int knn_wave_max(int v)
-{
-    const int none = -2147483647 - 1;
-#define TK_MAX_STEP(CTRL)                                                                      \
-    {                                                                                          \
-        const int o = __builtin_amdgcn_update_dpp(none, v, CTRL, 0xf, 0xf, false);             \
-        v = o > v ? o : v;                                                                     \
-    }
-    TK_MAX_STEP(0x111)  // row_shr:1
-    TK_MAX_STEP(0x112)
-    TK_MAX_STEP(0x114)
-    TK_MAX_STEP(0x118)
-    if constexpr (KMAX > 16)
-        TK_MAX_STEP(0x142)  // row_bcast:15
-    if constexpr (KMAX > 32)
-        TK_MAX_STEP(0x143)  // row_bcast:31
-#undef TK_MAX_STEP
-    return __builtin_amdgcn_readlane(v, KMAX - 1);
-}
+constexpr int KNN_WAVE_CHUNKS = 8;  // 64 keys each, requested together
 
-constexpr int KNN_WAVE_CHUNKS = 4;  // 64 keys each, requested together
-
-template <int KMAX, bool SOA, bool WEIGHTS>
+template <bool SOA, bool WEIGHTS>
 __global__ __launch_bounds__(KNN_BLOCK) void knn_wave_kernel_f32(
     const float *__restrict__ query, const float *__restrict__ key, float *__restrict__ distance,
     int64_t *__restrict__ index, float *__restrict__ weight, float eps, int64_t queries, int n1,
@@ -1235,15 +1226,31 @@ __global__ __launch_bounds__(KNN_BLOCK) void knn_wave_kernel_f32(
     };
     load(0);
 
-    // The first k keys fill the slots (mink.cuh:63-72); with a NaN in slot 0 MinK's maximum is a
-    // NaN, which nothing is below.
+    using Slot = KnnSlot<64>;
+    // The first k keys fill the slots (mink.cuh:63-72): key s in slot s, put in order here. With a
+    // NaN in slot 0 MinK's maximum is a NaN, which nothing is below.
     const float filled = tk_dist2<float>(px[0], py[0], pz[0], qx, qy, qz);
     const bool nan = filled != filled;
-    int value = lane < k && !nan ? __float_as_int(filled) : -1, where = lane;
-    int best, most = knn_wave_max<KMAX>(value);  // the slot of the maximum, the maximum
-    best = (int)__builtin_ctzll(__ballot(value == most));
+    constexpr int UNUSED = (int)0xfff00000u;  // a double's -inf, below all others
+    int vh = lane >= k ? UNUSED : nan ? (int)0xff800000u : __float_as_int(filled);
+    int vl = lane >= k ? 0 : ((63 - lane) << Slot::KEY_BITS) | lane;
+    {
+        const double mine = Slot::pack(vh, (unsigned)vl);
+        int place = 0;
+        for (int l = 0; l < k; l += 4) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                place += Slot::pack(__builtin_amdgcn_readlane(vh, l + i),
+                                    (unsigned)__builtin_amdgcn_readlane(vl, l + i)) > mine ? 1 : 0;
+        }
+        place = lane < k ? place : lane;
+        vh = __builtin_amdgcn_ds_permute(4 * place, vh);
+        vl = __builtin_amdgcn_ds_permute(4 * place, vl);
+    }
     const bool frozen = __builtin_amdgcn_readfirstlane((int)nan) != 0;
-    unsigned top = frozen || most < 0 ? 0u : (unsigned)most;  // what a key has to be below
+    // what a key has to be below
+    unsigned top = (unsigned)__builtin_amdgcn_readfirstlane(vh);
+    top = frozen || (int)top < 0 ? 0u : top;
 
     for (int base = 0; base < n2; base += 64 * KNN_WAVE_CHUNKS) {
         unsigned d[KNN_WAVE_CHUNKS];
@@ -1259,17 +1266,23 @@ __global__ __launch_bounds__(KNN_BLOCK) void knn_wave_kernel_f32(
 #pragma unroll
         for (int c = 0; c < KNN_WAVE_CHUNKS; ++c) {
             unsigned long long mask = __ballot(d[c] < top);
+            const int keys = base + 64 * c + lane;
             while (mask) {
                 const int l = (int)__builtin_ctzll(mask);
-                const int x = __builtin_amdgcn_readlane((int)d[c], l);
-                value = lane == best ? x : value;
-                where = lane == best ? base + 64 * c + l : where;
-                // the slot just written is the maximum unless another holds more: then the first
-                // of those that hold the most (mink.cuh:74-87)
-                most = knn_wave_max<KMAX>(value);
-                if (most > x)
-                    best = (int)__builtin_ctzll(__ballot(value == most));
-                top = (unsigned)most;
+                const int xh = __builtin_amdgcn_readlane((int)d[c], l);
+                // the slot of the maximum, which leaves; with nothing that stays strictly above it
+                // the key goes to the head, also in front of its equals (mink.cuh:74-87)
+                const unsigned slot = (unsigned)__builtin_amdgcn_readfirstlane(vl) & Slot::SLOT;
+                const unsigned flag = xh >= __builtin_amdgcn_readlane(vh, 1) ? Slot::FLAG : 0u;
+                const double x = Slot::pack(xh, slot | flag | (unsigned)__builtin_amdgcn_readlane(keys, l));
+                const double mine = Slot::pack(vh, (unsigned)vl);
+                const double next = Slot::pack(
+                    __builtin_amdgcn_update_dpp(UNUSED, vh, 0x130, 0xf, 0xf, false),  // wave_shl:1
+                    (unsigned)__builtin_amdgcn_update_dpp(0, vl, 0x130, 0xf, 0xf, true));
+                const double v = knn_max_f64(next, knn_min_f64_uniform(mine, x));
+                vh = Slot::distance(v);
+                vl = (int)Slot::low(v);
+                top = (unsigned)__builtin_amdgcn_readfirstlane(vh);
                 mask = __ballot(d[c] < top) & (~1ull << l);
             }
         }
@@ -1277,27 +1290,35 @@ __global__ __launch_bounds__(KNN_BLOCK) void knn_wave_kernel_f32(
 
     // An entry goes to its slot, or to its place in ascending order (equal distances in slot
     // order, NaNs last, as a stable sort of the slots leaves them).
-    float out = value < 0 ? filled : __int_as_float(value);  // (a NaN never leaves its slot)
-    int place = lane;
+    const int slot = 63 - (int)(((unsigned)vl & Slot::SLOT) >> Slot::KEY_BITS);
+    const float refilled = __int_as_float(__builtin_amdgcn_ds_bpermute(4 * slot, __float_as_int(filled)));
+    float out = vh < 0 ? refilled : __int_as_float(vh);  // (a NaN never leaves its slot)
+    int place = slot;
     if (sorted) {
-        const unsigned mine = (unsigned)value;  // (NaN: the largest)
-        place = 0;
-        for (int l = 0; l < k; ++l) {
-            const unsigned other = (unsigned)__builtin_amdgcn_readlane(value, l);
-            place += other < mine || (other == mine && l < lane) ? 1 : 0;
+        // equal neighbours, or NaNs: counted
+        const int below = __builtin_amdgcn_update_dpp(UNUSED, vh, 0x130, 0xf, 0xf, false);
+        place = k - 1 - lane;
+        if (__ballot(lane < k && (vh < 0 || vh == below))) {
+            place = 0;
+            for (int l = 0; l < k; ++l) {
+                const unsigned other = (unsigned)__builtin_amdgcn_readlane(vh, l);  // (NaN: the largest)
+                const int there = __builtin_amdgcn_readlane(slot, l);
+                place += other < (unsigned)vh || (other == (unsigned)vh && there < slot) ? 1 : 0;
+            }
         }
     }
     if (root)
         out = __builtin_sqrtf(out);
     if (lane < k) {
         distance[row * k + place] = out;
-        index[row * k + place] = where;
+        index[row * k + place] = (int64_t)((unsigned)vl & Slot::KEY);
     }
     if constexpr (WEIGHTS) {  // k == 3
+        const int of_slot = __builtin_amdgcn_ds_permute(4 * (lane < k ? slot : lane), __float_as_int(out));
         float d3[3];
 #pragma unroll
         for (int i = 0; i < 3; ++i)
-            d3[i] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(out), i));
+            d3[i] = __int_as_float(__builtin_amdgcn_readlane(of_slot, i));
         float w[3];
         knn_three_weights<float>(d3, eps, w);
         if (lane < 3)
@@ -1312,9 +1333,10 @@ __global__ __launch_bounds__(KNN_BLOCK) void knn_wave_kernel_f32(
 // and 64 to 10^6 keys, it never lost: equal at k = 48 and 64 on 256 keys, else 1.1 to 7 times faster,
 // also with keys sorted along an axis or a Morton curve (an insertion costs k (1 + ln(keys / k)) of
 // them on keys in random order; on sorted keys there are more, and the other kernels have them too).
-inline bool knn_wave_pays(int64_t queries, int k)
+// (A slot has 25 bits for its key.)
+inline bool knn_wave_pays(int64_t queries, int n2, int k)
 {
-    return k <= 64 && queries <= (k <= 32 ? 18432 : 36864);
+    return k <= 64 && n2 <= (1 << 25) && queries <= (k <= 32 ? 18432 : 36864);
 }
 
 template <bool SOA, bool WEIGHTS>
@@ -1323,19 +1345,10 @@ int knn_wave_launch(const float *query, const float *key, float *distance, int64
                     int root, hipStream_t s)
 {
     const int64_t queries = B * n1, blocks = (queries + KNN_BLOCK / 64 - 1) / (KNN_BLOCK / 64);
-    if (k > 64 || blocks > TK_MAX_I32)
+    if (k > 64 || n2 > (1 << 25) || blocks > TK_MAX_I32)
         return TK3D_ERR_UNSUPPORTED;
-#define TK_WAVE_LAUNCH(KMAX)                                                                      \
-    hipLaunchKernelGGL((knn_wave_kernel_f32<KMAX, SOA, WEIGHTS>), dim3((unsigned)blocks),         \
-                       dim3(KNN_BLOCK), 0, s, query, key, distance, index, weight, eps, queries,  \
-                       n1, n2, k, sorted, root)
-    if (k <= 16)
-        TK_WAVE_LAUNCH(16);
-    else if (k <= 32)
-        TK_WAVE_LAUNCH(32);
-    else
-        TK_WAVE_LAUNCH(64);
-#undef TK_WAVE_LAUNCH
+    hipLaunchKernelGGL((knn_wave_kernel_f32<SOA, WEIGHTS>), dim3((unsigned)blocks), dim3(KNN_BLOCK), 0, s,
+                       query, key, distance, index, weight, eps, queries, n1, n2, k, sorted, root);
     return tk_launch_status();
 }
 
@@ -1550,7 +1563,7 @@ int knn(const T *query, const T *key, int64_t B, int64_t N1, int64_t N2, int64_t
     hipStream_t s = (hipStream_t)stream;
     const int n1 = (int)N1, n2 = (int)N2, kk = (int)k;
     if constexpr (sizeof(T) == 4) {
-        if (knn_wave_pays(B * N1, kk))
+        if (knn_wave_pays(B * N1, n2, kk))
             return knn_wave_launch<false, false>(query, key, distance, index, nullptr, 0.0f, B, n1,
                                                  n2, kk, 0, 0, s);
     }
@@ -1650,7 +1663,7 @@ int knn_bcn(const T *query, const T *key, int64_t B, int64_t N1, int64_t N2, int
         return TK3D_ERR_NULL_POINTER;
     hipStream_t s = (hipStream_t)stream;
     if constexpr (sizeof(T) == 4) {
-        if (knn_wave_pays(B * N1, kk))
+        if (knn_wave_pays(B * N1, n2, kk))
             return knn_wave_launch<true, false>(query, key, distance, index, nullptr, 0.0f, B, n1, n2,
                                                 kk, 0, 0, s);
         if (k > 4 && !knn_filter_takes(B, n1, n2, kk)) {
@@ -1708,7 +1721,7 @@ int knn_ordered(const T *query, const T *key, bool channels_first, int64_t B, in
     if constexpr (sizeof(T) == 4) {
         if (B > 0 && N1 > 0 && k > 0 && k <= N2 && query && key && distance && index &&
             N1 <= TK_MAX_I32 / 4 && N2 <= TK_MAX_I32 / 4 && tk_fits(TK_MAX_ELEMS, B, N2, 3) &&
-            knn_wave_pays(B * N1, (int)k)) {
+            knn_wave_pays(B * N1, (int)N2, (int)k)) {
             const auto launch = channels_first ? knn_wave_launch<true, false> : knn_wave_launch<false, false>;
             return launch(query, key, distance, index, nullptr, 0.0f, B, (int)N1, (int)N2, (int)k,
                           sorted, root, (hipStream_t)stream);
@@ -1742,7 +1755,7 @@ int three_nn(const T *query, const T *key, bool channels_first, int64_t B, int64
         return TK3D_ERR_UNSUPPORTED;
     hipStream_t s = (hipStream_t)stream;
     if constexpr (sizeof(T) == 4) {
-        if (knn_wave_pays(B * N1, 3)) {
+        if (knn_wave_pays(B * N1, (int)N2, 3)) {
             const auto launch = channels_first ? knn_wave_launch<true, true> : knn_wave_launch<false, true>;
             return launch(query, key, distance, index, weight, (float)eps, B, (int)N1, (int)N2, 3, 0, 0,
                           s);
