@@ -452,6 +452,69 @@ def test_batch_norm_is_the_librarys_bit_by_bit(cuda, b, c, m, size):
         assert lib.tk3d_mlp_batch_norm_supported(*(ctypes.c_int64(v) for v in shape)) == 0
 
 
+@pytest.mark.parametrize("size", [20, 32, 64])
+def test_a_maximum_is_the_first_of_equals(cuda, size):
+    # quantised values (and their order is that of their norm: ascending or, with gamma < 0, descending), a
+    # channel of one value, NaNs above all
+    import ctypes
+
+    from torkit3d_amd import _lib
+
+    class Norm(ctypes.Structure):
+        _fields_ = [(n, ctypes.c_void_p) for n in
+                    ("partial", "gamma", "beta", "running_mean", "running_var", "mean", "inv_std")] + [
+                        ("eps", ctypes.c_double), ("momentum", ctypes.c_float),
+                        ("B", ctypes.c_int32), ("C", ctypes.c_int32), ("P", ctypes.c_int32)]
+
+    def pointers(*tensors):
+        return [ctypes.c_void_p(t.data_ptr()) for t in tensors]
+
+    b, c, m = 2, 6, 103
+    y = (randn(size, b, c, m, size) * 1.5).round() / 2
+    y[:, 3] = 0.25
+    gamma, beta = torch.tensor([1.0, -1.0, 0.5, 2.0, 1.0, -2.0], device=cuda), randn(4, c)
+    lib, p, stream = _lib.lib(), m * size, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    lib.tk3d_mlp_batch_norm_partial_bytes.restype = ctypes.c_int64
+    partial = torch.empty(lib.tk3d_mlp_batch_norm_partial_bytes(ctypes.c_int64(c)), dtype=torch.uint8, device=cuda)
+    state = [randn(5, c), randn(6, c).abs(), torch.empty(c, device=cuda), torch.empty(c, device=cuda)]
+    norm = Norm(*(t.data_ptr() for t in (partial, gamma, beta, *state)), 1e-3, 0.3, b, c, p)
+    assert lib.tk3d_mlp_batch_sums_f32(*pointers(y), b, c, p, *pointers(partial), stream) == 0
+    y[0, :, ::5, 7] = float("nan")      # (behind the sums: the other values keep their norm)
+    y[0, :, ::10, size - 1] = float("nan")
+    out, extreme = torch.empty(b, c, m, device=cuda), torch.empty(b, c, m, device=cuda)
+    arg = torch.empty(b, c, m, dtype=torch.uint8, device=cuda)
+    assert lib.tk3d_mlp_batch_pool_f32(*pointers(y), ctypes.byref(norm), size, *pointers(out, extreme, arg),
+                                       stream) == 0
+    order = (y * gamma.sign()[:, None, None]).nan_to_num(float("inf"))
+    first = (order == order.max(dim=3, keepdim=True)[0]).int().argmax(dim=3)
+    assert torch.equal(arg.long(), first)
+    there = y.gather(3, first[..., None])[..., 0]
+    assert torch.equal(extreme.nan_to_num(7.0), there.nan_to_num(7.0)) and torch.equal(out.isnan(), there.isnan())
+
+
+@pytest.mark.parametrize("b,m,s", [(1, 4097, 32), (3, 2731, 32), (5, 3277, 32), (1, 2049, 64), (3, 1366, 64), (3, 2731, 64)])
+def test_scatter_of_several_groups_a_wave(cuda, b, m, s):
+    # around the numbers of groups from which a wave takes two and four in a row, numbers that neither divides
+    import ctypes
+
+    from torkit3d_amd import _lib
+
+    o, i = 5, 3
+    place = torch.randint(0, s, (b, o, m), device=cuda, dtype=torch.int32)
+    value, w = randn(m, b, o, m), randn(s, o, i)
+    sel = torch.stack([value.view(torch.int32), place], dim=3).contiguous()
+    out = torch.full((b, i, m, s), 7.0, device=cuda)
+    ptr = [ctypes.c_void_p(t.data_ptr()) for t in (sel, w)]
+    assert _lib.lib().tk3d_mlp_pool_scatter_f32(*ptr, b, o, i, m, s, ctypes.c_void_p(out.data_ptr()),
+                                                ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+    e = torch.zeros(b, o, m, s, dtype=torch.float64, device=cuda).scatter_(3, place.long()[..., None],
+                                                                           value.double()[..., None])
+    want = torch.einsum("oi,bop->bip", w.double(), e.flatten(2)).view_as(out)
+    # (up to five terms of one sum, each rounded once, and the sum after each)
+    assert ((out - want).abs() <= 6 * 2.0 ** -24 * torch.einsum(
+        "oi,bop->bip", w.double().abs(), e.abs().flatten(2)).view_as(out) + 1e-30).all()
+
+
 @pytest.mark.parametrize("form", ["dense", "edges"])
 def test_without_the_library_training_is_left_to_stock(cuda, form):
     """torch's own batch norm rounds in another order than the backward takes its signs by."""

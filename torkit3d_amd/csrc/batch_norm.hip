@@ -142,8 +142,42 @@ __global__ void __launch_bounds__(kBlock) batch_relu_kernel(const float *__restr
     }
 }
 
-// out = relu(max norm(y)) over groups of `size` values, where the maximum is and the y there.
-// LANES lanes share a group of 4 LANES values; 0: a lane walks a group.
+// Largest value of a group of LANES neighbouring lanes, in all of them; NaN above all.
+template <int LANES> __device__ __forceinline__ float group_maximum(float v)
+{
+#define TK_MAXIMUM_STEP(ctrl)                                                                         \
+    v = __builtin_elementwise_maximum(                                                                \
+        v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), ctrl, 0xf, 0xf, true)));
+    TK_MAXIMUM_STEP(0xb1)  // quad_perm 1,0,3,2
+    TK_MAXIMUM_STEP(0x4e)  // quad_perm 2,3,0,1
+    TK_MAXIMUM_STEP(0x141)  // row_half_mirror
+    if constexpr (LANES > 8)
+        TK_MAXIMUM_STEP(0x140)  // row_mirror
+#undef TK_MAXIMUM_STEP
+    return v;
+}
+template <int LANES> __device__ __forceinline__ int group_first(int v)
+{
+#define TK_FIRST_STEP(ctrl)                                                                           \
+    {                                                                                                 \
+        const int o = __builtin_amdgcn_update_dpp(0, v, ctrl, 0xf, 0xf, true);                        \
+        v = o < v ? o : v;                                                                            \
+    }
+    TK_FIRST_STEP(0xb1)
+    TK_FIRST_STEP(0x4e)
+    TK_FIRST_STEP(0x141)
+    if constexpr (LANES > 8)
+        TK_FIRST_STEP(0x140)
+#undef TK_FIRST_STEP
+    return v;
+}
+
+// out = relu(max norm(y)) over groups of `size` values, where the maximum is and the y there, the first of
+// equals, NaN above all. LANES lanes share a group of 4 LANES values; 0: a lane walks a group.
+// The largest value first, then the first place that holds it: three instructions a value beside the
+// norm, where a maximum that carries its place and its y along takes nine, and three exchanges through LDS
+// a step between lanes. Bound by memory (and the last-level cache) now: [16, 64, 512, 32] 18.2 -> 15.5 us, [16, 128, 512, 32]
+// 29.9 -> 24.3, [16, 256, 128, 64] 31.8 -> 24.0. (Over groups of 20, a lane a group, it made no difference.)
 template <int LANES>
 __global__ void __launch_bounds__(kBlock) batch_pool_kernel(const float *__restrict__ y,
                                                             tk3d_mlp_batch_norm n, int size,
@@ -152,6 +186,7 @@ __global__ void __launch_bounds__(kBlock) batch_pool_kernel(const float *__restr
                                                             unsigned char *__restrict__ arg,
                                                             int stretches)
 {
+    constexpr int NONE = 0x7fffffff;
     const int part = blockIdx.x % stretches, row = blockIdx.x / stretches, c = row % n.C;
     const f32x4 k = batch_constants(n, c, row < n.C && part == 0 && threadIdx.x == 0);
     const int M = n.P / size;
@@ -174,23 +209,24 @@ __global__ void __launch_bounds__(kBlock) batch_pool_kernel(const float *__restr
             }
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                float best = normalised(v[u][0], k);
-                int where = 4 * l;
-                float raw = v[u][0];
+                f32x4 z;
 #pragma unroll
-                for (int i = 1; i < 4; ++i) {
-                    const int before = where;
-                    take_larger(best, where, normalised(v[u][i], k), 4 * l + i);
-                    raw = where != before ? v[u][i] : raw;
-                }
+                for (int i = 0; i < 4; ++i)
+                    z[i] = normalised(v[u][i], k);
+                const float best = group_maximum<LANES>(__builtin_elementwise_maximum(
+                    __builtin_elementwise_maximum(z[0], z[1]), __builtin_elementwise_maximum(z[2], z[3])));
+                // (nothing is above `best`, and a NaN is where it is one)
+                const bool nan = best != best;
+                int own = NONE;
+                float raw = 0.0f;
 #pragma unroll
-                for (int off = 1; off < LANES; off <<= 1) {
-                    const float other = __shfl_xor(best, off), y_there = __shfl_xor(raw, off);
-                    const int at = __shfl_xor(where, off), before = where;
-                    take_larger(best, where, other, at);
-                    raw = where != before ? y_there : raw;
+                for (int i = 3; i >= 0; --i) {
+                    const bool here = nan ? z[i] != z[i] : z[i] == best;
+                    own = here ? 4 * l + i : own;
+                    raw = here ? v[u][i] : raw;
                 }
-                if (l == 0 && g0 + u * step < M)
+                const int where = group_first<LANES>(own);
+                if (own == where && g0 + u * step < M)  // (one lane of the group has it)
                     put(g0 + u * step, best, raw, where);
             }
         }

@@ -435,9 +435,11 @@ __global__ void __launch_bounds__(kBlock)
 // ---- launches ----------------------------------------------------------------------------------------------
 
 // Runs of four groups read whole sectors of sel ([B, O, M]), as long as every SIMD keeps a wave.
-void fill_sparse(SparseArgs &a, int B)
+int outer_run(int B, int M) { return (int64_t)B * M >= 16 * tk_cu_count() ? 4 : 1; }
+
+void fill_sparse(SparseArgs &a, int B, int run)
 {
-    a.run = (int64_t)B * a.M >= 16 * tk_cu_count() ? 4 : 1;
+    a.run = run;
     a.units = (a.M + a.run - 1) / a.run;
     a.total = B * a.units;
 }
@@ -517,7 +519,13 @@ int tk3d_mlp_pool_scatter_f32(const void *sel, const float *w, int B, int O, int
     a.O = O;
     a.I = I;
     a.M = M;
-    fill_sparse(a, B);
+    // Groups in a row share the lines of `sel` they come from, but a launch that leaves lanes idle for it
+    // loses more: as many as the resident waves (16 of a CU, 8 with 64 places, by LDS) have rounds for, up to
+    // four. us, four of them from 4096 groups on, and now: O = 128, I = 64, 8 x 512 groups of 32 38, 19; 16 x
+    // 512 46, 34 (two); 32 x 512 63, 63 (four; one 66); O = 256, I = 128, 16 x 128 groups of 64 48, 46.
+    const int64_t waves = (int64_t)B * M * ((I + 63) / 64);
+    const int64_t rounds = waves / ((group == 32 ? 16 : 8) * (int64_t)tk_cu_count());
+    fill_sparse(a, B, rounds >= 4 ? 4 : rounds >= 2 ? 2 : 1);
     const int bytes = kWaves * group * kRow * 4;
     const int rc = group == 32 ? tk_allow_dynamic_lds<mlp_pool_scatter_kernel<32>>(bytes)
                                : tk_allow_dynamic_lds<mlp_pool_scatter_kernel<64>>(bytes);
@@ -537,7 +545,7 @@ int tk3d_mlp_pool_outer_splits(int B, int O, int I, int M)
 {
     SparseArgs a{};
     a.M = M;
-    fill_sparse(a, B);
+    fill_sparse(a, B, outer_run(B, M));
     const int wo = sharing(O);
     const int blocks = ((O + 64 * wo - 1) / (64 * wo)) * ((I + 63) / 64), wgs = (a.total + kWaves - 1) / kWaves;
     const int most = ((wo == 1 ? 2 : 1) * tk_cu_count() + blocks - 1) / blocks;
@@ -559,7 +567,7 @@ int tk3d_mlp_pool_outer_f32(const void *sel, const float *y, const tk3d_mlp_norm
     a.O = O;
     a.I = I;
     a.M = M;
-    fill_sparse(a, B);
+    fill_sparse(a, B, outer_run(B, M));
     const int splits = tk3d_mlp_pool_outer_splits(B, O, I, M);
     return group == 32 ? launch_outer<32>(a, splits, (hipStream_t)stream_)
                        : launch_outer<64>(a, splits, (hipStream_t)stream_);
