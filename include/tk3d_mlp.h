@@ -221,6 +221,23 @@ int tk3d_mlp_group_f32(const float *u, const float *xyz, const float *centre, co
                        const float *wx, int ldw, int B, int C, int N, int M, int S, float *y,
                        void *stream);
 
+/* Evaluation of three layers behind a grouping, pooled over the S neighbours: y of tk3d_mlp_group_f32 with C[0]
+ * channels, ReLU of its norm[0]; w2 [C[1]][C[0]] and norm[1], w3 [C[2]][C[1]] and norm[2] on top; out [B,C[2],M]
+ * is the maximum over each group. `supported`: C multiples of 32 whose activations of 64 positions fit in LDS
+ * (C[0] + C[1] up to 512 or so), S 32 or 64, u (or NULL), w2 and w3 16-byte aligned, and work enough for the chip; others
+ * are refused. */
+typedef struct tk3d_mlp_grouped_pool {
+    const float *u, *xyz, *centre;
+    const int64_t *index;
+    const float *wx, *w2, *w3;
+    tk3d_mlp_norm norm[3];
+    float *out;
+    int32_t ldw, B, N, M, S;
+    int32_t C[3];
+} tk3d_mlp_grouped_pool;
+int tk3d_mlp_grouped_pool_supported(const tk3d_mlp_grouped_pool *p);
+int tk3d_mlp_grouped_pool_f32(const tk3d_mlp_grouped_pool *p, void *stream);
+
 /* EdgeConv (torkit3d/ops/edge_conv.py) with one layer, on a graph of a cloud with itself, pooled
  * over the K neighbours: y(i, k) = W1 (x_j - x_i) + W2 x_i, j = index[b, i, k] (x_j = 0 for an index
  * outside [0,N)), where w [O][2 C] = [W1 W2] and x [B, C, N].

@@ -6,12 +6,13 @@ about as close to float64 (2-norm of the difference over 2-norm of the result) a
 float32 is: within four times its error plus 2e-6 (a few rounding errors of 2^-24 through up
 to four layers)."""
 import copy
+import ctypes
 
 import pytest
 import torch
 from torch import nn
 
-from torkit3d_amd import _native
+from torkit3d_amd import _lib, _native
 from torkit3d_amd.nn import SharedMLP, mlp1d_bn_relu, mlp2d_bn_relu
 from torkit3d_amd.ops.edge_conv import edge_lists
 from torkit3d_amd.ops.group_points import group_points_with_xyz
@@ -268,6 +269,50 @@ def test_grouped(cuda, monkeypatch, features, tracked, n, m, s, training):
     check(mlp, fused, reference, inputs, monkeypatch)
 
 
+# Three layers behind a grouping in one launch, in evaluation: tiles of 32 and of 64 positions, with half a tile left
+# over; four waves and eight, with fewer channel blocks than waves and with more; the last layer's channels in one part
+# and in several; activations that nearly fill LDS.
+class GroupedPool(ctypes.Structure):  # tk3d_mlp_grouped_pool
+    _fields_ = [("pointers", ctypes.c_void_p * 7), ("norms", ctypes.c_void_p * 15), ("out", ctypes.c_void_p),
+                ("sizes", ctypes.c_int32 * 8)]
+
+
+@pytest.mark.parametrize("b,features,n,m,s,widths", [
+    (1, 0, 100, 7, 32, (32, 32, 32)), (1, 64, 100, 1, 64, (96, 128, 160)), (2, 3, 333, 257, 32, (64, 96, 32)),
+    (3, 0, 40, 50, 32, (64, 128, 96)), (2, 5, 64, 64, 64, (128, 160, 256)), (9, 12, 50, 61, 32, (256, 256, 512)),
+    (2, 3, 70, 80, 64, (32, 480, 64)), (5, 1, 300, 999, 32, (32, 64, 288)),
+])
+def test_grouped_in_one_launch(cuda, monkeypatch, b, features, n, m, s, widths):
+    sizes = GroupedPool(sizes=(features + 3, b, n, m, s, *widths))
+    assert _lib.lib().tk3d_mlp_grouped_pool_supported(ctypes.byref(sizes)) == 1
+    for other in ((30, *widths[1:]), (widths[0], 4096, widths[2])):  # (the general chain's)
+        sizes = GroupedPool(sizes=(features + 3, b, n, m, s, *other))
+        assert _lib.lib().tk3d_mlp_grouped_pool_supported(ctypes.byref(sizes)) == 0
+    mlp = make(mlp2d_bn_relu, features + 3, widths, False, cuda)
+    xyz, centre = randn(1, b, 3, n), randn(2, b, 3, m)
+    index = torch.randint(0, n, (b, m, s), generator=torch.Generator().manual_seed(n))
+    index[0, 0] = -1
+    inputs = [(xyz, False), (centre, False), (index.cuda(), False)]
+    if features:
+        inputs.append((randn(3, b, features, n), False))
+
+    def fused(mod, xyz, centre, index, f=None):
+        return mod.forward_grouped_max(f, xyz, centre, index)
+
+    def reference(mod, xyz, centre, index, f=None):
+        return mod(group_points_with_xyz(f, xyz, centre, index)).max(dim=3)[0]
+
+    check(mlp, fused, reference, inputs, monkeypatch)
+    xyz[0, 0, 0], xyz[-1, 2, -1] = float("inf"), float("nan")
+    # (these stay where they are. In float64: a float32 convolution of the library's carries them over to the
+    # positions beside.)
+    with torch.no_grad():
+        args = [t for t, _ in inputs]
+        got = fused(mlp, *args)
+        want = reference(stock(mlp, torch.float64), *[t.double() if t.is_floating_point() else t for t in args])
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+
+
 # Products in evaluation add up in several chains. Roundings of at most u = 2^-24 to numbers that grow as a
 # random walk over n terms make an error of about 0.21 u sqrt(n) of the result (one chain over all K:
 # 1.9 u at 64 channels, 3.4 u at 256, 6.9 u at 1024), in four chains half of it, in chains of 16 or
@@ -374,10 +419,6 @@ def test_pooled_layer_far_from_zero(cuda, b, m, s, widths, far):
 def test_the_backward_takes_the_signs_of_the_library(cuda, b, c, p):
     """The activations as the backward works them out are those of the library's batch norm, bit by
     bit."""
-    import ctypes
-
-    from torkit3d_amd import _lib
-
     class Norm(ctypes.Structure):
         _fields_ = [(n, ctypes.c_void_p) for n in ("mean", "var", "gamma", "beta")] + [("eps", ctypes.c_float)]
 
@@ -405,10 +446,6 @@ def test_the_backward_takes_the_signs_of_the_library(cuda, b, c, p):
     (8, 64, 2048, 32), (32, 4, 2048, 32), (512, 3, 1023, 4), (1, 3, 32768, 64), (511, 3, 1026, 4),
 ])
 def test_batch_norm_is_the_librarys_bit_by_bit(cuda, b, c, m, size):
-    import ctypes
-
-    from torkit3d_amd import _lib
-
     class Norm(ctypes.Structure):
         _fields_ = [(n, ctypes.c_void_p) for n in
                     ("partial", "gamma", "beta", "running_mean", "running_var", "mean", "inv_std")] + [
@@ -456,10 +493,6 @@ def test_batch_norm_is_the_librarys_bit_by_bit(cuda, b, c, m, size):
 def test_a_maximum_is_the_first_of_equals(cuda, size):
     # quantised values (and their order is that of their norm: ascending or, with gamma < 0, descending), a
     # channel of one value, NaNs above all
-    import ctypes
-
-    from torkit3d_amd import _lib
-
     class Norm(ctypes.Structure):
         _fields_ = [(n, ctypes.c_void_p) for n in
                     ("partial", "gamma", "beta", "running_mean", "running_var", "mean", "inv_std")] + [
@@ -495,10 +528,6 @@ def test_a_maximum_is_the_first_of_equals(cuda, size):
 @pytest.mark.parametrize("b,m,s", [(1, 4097, 32), (3, 2731, 32), (5, 3277, 32), (1, 2049, 64), (3, 1366, 64), (3, 2731, 64)])
 def test_scatter_of_several_groups_a_wave(cuda, b, m, s):
     # around the numbers of groups from which a wave takes two and four in a row, numbers that neither divides
-    import ctypes
-
-    from torkit3d_amd import _lib
-
     o, i = 5, 3
     place = torch.randint(0, s, (b, o, m), device=cuda, dtype=torch.int32)
     value, w = randn(m, b, o, m), randn(s, o, i)

@@ -146,6 +146,21 @@ void run_product(int in, int out, tk3d_mlp_product &p, void *stream)
     done(tk3d_mlp_product_f32(in, out, &p, stream), "tk3d_mlp_product_f32");
 }
 
+// The product of the features with their weights in the first layer behind a grouping: [B, N, C], or
+// undefined without features.
+Tensor feature_product(const Call &c)
+{
+    if (!c.x.defined())
+        return {};
+    const int64_t B = c.batch(), C = c.out_channels(0), N = c.xyz.size(2);
+    const Tensor u = at::empty({B, N, C}, c.xyz.options());
+    tk3d_mlp_product q = product(B, C, N);
+    q.src[0] = source(c.x, f32(c.weight(0)), 1, c.in_channels(0));
+    q.out = f32(u);
+    run_product(TK3D_MLP_IN_RAW, TK3D_MLP_OUT_POINTS, q, stream_of(c.xyz));
+    return u;
+}
+
 // The product of the first layer behind a grouping, without the grouped tensor.
 void first_grouped(const Call &c, const Tensor &y)
 {
@@ -153,14 +168,7 @@ void first_grouped(const Call &c, const Tensor &y)
     const int64_t M = c.index.size(1), S = c.index.size(2), N = c.xyz.size(2);
     const float *w = f32(c.weight(0));
     void *stream = stream_of(c.xyz);
-    Tensor u;
-    if (c.x.defined()) {
-        u = at::empty({B, N, C}, c.xyz.options());
-        tk3d_mlp_product q = product(B, C, N);
-        q.src[0] = source(c.x, w, 1, K);
-        q.out = f32(u);
-        run_product(TK3D_MLP_IN_RAW, TK3D_MLP_OUT_POINTS, q, stream);
-    }
+    const Tensor u = feature_product(c);
     done(tk3d_mlp_group_f32(f32(u), f32(c.xyz), f32(c.centre), c.index.data_ptr<int64_t>(), w + (K - 3),
                             (int)K, (int)B, (int)C, (int)N, (int)M, (int)S, f32(y), stream),
          "tk3d_mlp_group_f32");
@@ -176,6 +184,31 @@ Tensor evaluate(const Call &c)
     for (int64_t l = 0; l < L; ++l) {
         k.mean.push_back(c.buffers[3 * l]);
         k.var.push_back(c.buffers[3 * l + 1]);
+    }
+    if (c.grouped() && c.pool && L == 3) {
+        tk3d_mlp_grouped_pool p{};
+        p.xyz = f32(c.xyz);
+        p.centre = f32(c.centre);
+        p.index = c.index.data_ptr<int64_t>();
+        p.ldw = (int32_t)c.in_channels(0);
+        p.wx = f32(c.weight(0)) + (p.ldw - 3);
+        p.w2 = f32(c.weight(1));
+        p.w3 = f32(c.weight(2));
+        p.B = (int32_t)B;
+        p.N = (int32_t)c.xyz.size(2);
+        p.M = (int32_t)c.index.size(1);
+        p.S = (int32_t)c.index.size(2);
+        for (int l = 0; l < 3; ++l) {
+            p.norm[l] = norm_of(c, k, l);
+            p.C[l] = (int32_t)c.out_channels(l);
+        }
+        if (tk3d_mlp_grouped_pool_supported(&p)) {
+            const Tensor u = feature_product(c), out = at::empty({B, p.C[2], p.M}, like.options());
+            p.u = f32(u);
+            p.out = f32(out);
+            done(tk3d_mlp_grouped_pool_f32(&p, stream), "tk3d_mlp_grouped_pool_f32");
+            return out;
+        }
     }
     Tensor h;
     for (int64_t l = 0; l < L; ++l) {
