@@ -369,7 +369,7 @@ def test_groups_kernel_edges(cuda, n, k, kind):
 
 
 def test_claims_of_many_clouds(cuda):
-    # workgroups that take several groups of a cloud's points in turn (17 groups, 8 workgroups a cloud):
+    # workgroups that take several groups of a cloud's points in turn (17 groups, one workgroup a cloud):
     # clouds in sampling order, and copies of them with two samples exchanged at the first steps that the kernel
     # does not look at itself, in the middle and at the end, or a point moved in the last group of points
     g = gen(11)
@@ -389,6 +389,34 @@ def test_claims_of_many_clouds(cuda):
     which = torch.arange(256) * 5 % len(kinds)
     got = run(kinds[which].contiguous(), 256, cuda)
     np.testing.assert_array_equal(got, want[which.numpy()])
+
+
+@pytest.mark.parametrize("b,n,k", [(5, 1000, 193), (40, 1025, 300), (60, 2100, 1024), (3, 8193, 1000)])
+def test_claims_shared_by_workgroups(cuda, b, n, k):
+    # one and several groups of a cloud's points to each of several workgroups, of which the last one through
+    # finishes the cloud: with a claim that holds, that fails in the last group only, among points that are
+    # not samples, that is made of distances which overflow, and without one
+    from torkit3d_amd.ops.sample_farthest_points import sample_farthest_points_gather
+
+    big = torch.rand(1, n + 300, 3, generator=gen(n))
+    first = torch.from_numpy(oracle.sample_farthest_points(big.numpy(), n))
+    order = torch.gather(big, 1, first[:, :, None].expand(-1, -1, 3))[0]
+    moved = order.clone()
+    moved[n - 1] = 0.5 * (order[0] + order[k - 1])  # (nearer to others than step k - 1's sample, or not)
+    outlier = order.clone()
+    outlier[n - 1] = order[2] + 0.9 * (order[2] - order[0])
+    odd = order.clone()
+    odd[n // 2, 1] = float("nan")
+    kinds = torch.stack([order, moved, outlier, order * 1e20, odd, order.flip(0)])
+    want = oracle.sample_farthest_points(kinds.numpy(), k)
+    which = torch.arange(b) % len(kinds)
+    pts = kinds[which].contiguous()
+    for transpose in (False, True):
+        dev = (pts.transpose(1, 2) if transpose else pts).contiguous().to(cuda)
+        index, sampled = sample_farthest_points_gather(dev, k, transpose=transpose)
+        np.testing.assert_array_equal(index.cpu().numpy(), want[which.numpy()])
+        got = (sampled.transpose(1, 2) if transpose else sampled).cpu().numpy()
+        np.testing.assert_array_equal(got, np.take_along_axis(pts.numpy(), want[which.numpy()][:, :, None], 1))
 
 
 @pytest.mark.parametrize("n,k", [(192, 192), (200, 191), (512, 192), (1000, 999), (1024, 512), (1025, 192),

@@ -505,7 +505,6 @@ __device__ __forceinline__ int fps_position_of_point(int j, const FpsLayout &L)
 // What one of these kernels leaves as a cloud's first index for the ones behind it.
 constexpr int64_t FPS_ODD = -1;     // a coordinate is not finite: the plain loop has to do it
 constexpr int64_t FPS_CLAIM = -2;   // the cloud looks as if in sampling order: to be checked
-constexpr int64_t FPS_BROKEN = -3;  // it is not
 constexpr int FPS_CLAIM_MAX = 1024;
 
 __device__ __forceinline__ int fps_max(int a, int b) { return a > b ? a : b; }
@@ -624,8 +623,8 @@ __device__ __forceinline__ int fps_band(int was, float target, int n)
 // A cloud that is itself a farthest point sample, in sampling order from its point 0 (the next level
 // of a PointNet++ encoder), has 0, 1, 2, ... as its answer. Where point 1 is the point farthest from
 // point 0, point 2 the one farthest from both and at most 1024 samples are wanted, this kernel
-// only leaves the claim, which fps_claim_minima_kernel and fps_claim_check_kernel test with the whole
-// chip; the instance with LAST behind them writes the answer, or does the work if the claim was wrong.
+// only leaves the claim, which fps_claim_minima_kernel and fps_settle_kernel_f32 test with the whole
+// chip; the latter writes the answer, or does the work (LAST) if the claim was wrong.
 // (A cloud in random order passes the test of point 1 once in n, and then takes twice the time: with that
 // test alone 256 x 2048 -> 512 took 330 us for 177 in one batch of eight. Point 2 is looked at behind it.)
 template <int P, int NW, int NB, bool SOA, bool LAST>
@@ -750,6 +749,7 @@ __device__ __forceinline__ void fps_band(const float *__restrict__ pts, int64_t 
         if (any_odd || claim) {  // uniform over the workgroup
             if (tid == 0) {
                 out[0] = any_odd ? FPS_ODD : FPS_CLAIM;
+                out[1] = 0;
             }
             return;
         }
@@ -1134,51 +1134,12 @@ __global__ __launch_bounds__(NW * 64) void fps_band_kernel_f32(const float *__re
                                       index + (int64_t)blockIdx.x * L.k, L, claims);
 }
 
-// Behind the kernel above and the check of its claims: the clouds that it has left, then the
-// coordinates of the picks if wanted ([B,K,3], or [B,3,K] with SOA). One launch for what took two
-// (a second look at every coordinate, the gather): 4.7 us less per call.
-template <int P, int NW, int NB, bool SOA>
-__global__ __launch_bounds__(NW * 64) void fps_last_kernel_f32(const float *__restrict__ points,
-                                                               int64_t *__restrict__ index,
-                                                               float *__restrict__ sampled,
-                                                               FpsLayout L)
-{
-    constexpr int NT = NW * TK_WAVE;
-    const float *__restrict__ pts = points + (int64_t)blockIdx.x * L.n * 3;
-    int64_t *out = index + (int64_t)blockIdx.x * L.k;
-    const int64_t left = out[0];  // uniform over the workgroup
-    if (left < 0) {
-        __syncthreads();  // everybody has read it
-        if (left == FPS_CLAIM) {
-            for (int i = threadIdx.x; i < L.k; i += NT)
-                out[i] = (int64_t)i;
-        } else if (left == FPS_BROKEN) {
-            fps_band<P, NW, NB, SOA, true>(pts, out, L, false);
-        } else {
-            fps_plain<float, P, NT, SOA>(pts, out, L);
-        }
-        __syncthreads();
-    }
-    if (sampled) {
-        float *__restrict__ so = sampled + (int64_t)blockIdx.x * L.k * 3;
-        for (int i = threadIdx.x; i < L.k; i += NT) {
-            const int64_t j = out[i];
-#pragma unroll
-            for (int a = 0; a < 3; ++a)
-                so[SOA ? (int64_t)a * L.k + i : (int64_t)i * 3 + a] = fps_coord<SOA>(pts, L.n, j, a);
-        }
-    }
-}
-
-// The check of a claim that a cloud's first k points, in this order, are its farthest point sample:
-// step s takes point s exactly if no point has a larger running minimum after the centres 0 .. s - 1,
-// nor an equal one at a lower position. The minimum of point s itself at that time, v_s, is the
-// threshold, worked out by a first kernel into the index row, which nobody else needs yet. Both read
-// the centres at uniform addresses and cut the centres into 16 stretches, a wave each, so that a
-// group of 64 points is done in k / 16 dependent steps, twice in the check (a stretch needs the
-// minimum over those before it). 8 x 4096 -> 1024: 333 us of sampling before, under 30 us with both.
-// A cloud's workgroups take its groups in turn, eight workgroups to a CU in all: clouds without a claim,
-// which is most of them, pay for the launch alone.
+// A claim that a cloud's first k points, in this order, are its farthest point sample: step s takes point s
+// exactly if no point has a larger running minimum after the centres 0 .. s - 1, nor an equal one at a
+// lower position. The minimum of point s itself at that time, v_s, is the threshold, worked out by a first
+// kernel into the index row, which nobody else needs yet; fps_settle_kernel_f32 compares. Both read the centres at
+// uniform addresses and cut them into stretches, a wave each. A cloud's workgroups take its groups of 64 points in
+// turn. 8 x 4096 -> 1024: 333 us of sampling before, 36 us in all.
 constexpr int FPS_CLAIM_PARTS = 16;
 
 template <bool SOA>
@@ -1219,57 +1180,138 @@ __global__ __launch_bounds__(1024) void fps_claim_minima_kernel(const float *__r
     }
 }
 
-template <bool SOA>
-__global__ __launch_bounds__(1024) void fps_claim_check_kernel(const float *__restrict__ points,
-                                                               int64_t *__restrict__ index,
-                                                               FpsLayout L, int slices)
+// Whether a claim fails on one of the workgroup's points (of one thread's, in that thread).
+template <int NW, bool SOA>
+__device__ __forceinline__ bool fps_claim_fails(const float *__restrict__ pts, const int64_t *out,
+                                                const FpsLayout &L, int slice, int slices)
 {
-    const int b = blockIdx.x / slices;
-    const float *__restrict__ pts = points + (int64_t)b * L.n * 3;
-    int64_t *__restrict__ out = index + (int64_t)b * L.k;
-    __shared__ float s_min[FPS_CLAIM_PARTS][TK_WAVE];
-    __shared__ int s_open;
-    if (threadIdx.x == 0)
-        s_open = out[0] == FPS_CLAIM;  // (another workgroup may be writing it: read once)
-    __syncthreads();
-    if (!s_open)  // uniform over the workgroup
-        return;
+    // Centres that a wave takes at a time. Their distances stay in registers until the minima over the waves
+    // before it are there, and the differences to the thresholds run into one maximum: worked out twice, and
+    // compared step by step, the check took 35 us at 8 x 4096 -> 1024 and 5 more for the launch behind it, both
+    // now 24.
+    constexpr int C = 32;
+    __shared__ __align__(16) float s_v[FPS_CLAIM_MAX + C * NW];  // [i]: v of step i + 1, which follows centre i
+    __shared__ float s_min[2][NW][TK_WAVE];
     const int lane = threadIdx.x & (TK_WAVE - 1);
-    const int part = __builtin_amdgcn_readfirstlane(threadIdx.x / TK_WAVE);
-    const int centres = L.k - 1;  // after centre i comes the choice of step i + 1
-    const int step = (centres + FPS_CLAIM_PARTS - 1) / FPS_CLAIM_PARTS;
-    const int from = part * step, to = fps_min(from + step, centres);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / TK_WAVE);
+    const int centres = L.k - 1;
     bool bad = false;
-    for (int first = blockIdx.x % slices * TK_WAVE; first < L.n; first += slices * TK_WAVE) {
+    for (int i = threadIdx.x; i < FPS_CLAIM_MAX + C * NW; i += NW * TK_WAVE) {
+        const float v = i < centres ? __builtin_bit_cast(float, (int)out[i + 1]) : __builtin_huge_valf();
+        bad |= !(v > 0.0f && (v < __builtin_huge_valf() || i >= centres));
+        s_v[i] = v;
+    }
+    __syncthreads();
+    int turn = 0;
+    for (int first = slice * TK_WAVE; first < L.n; first += slices * TK_WAVE) {
         const int j = first + lane, me = j < L.n ? j : L.n - 1;
         const float x = fps_coord<SOA>(pts, L.n, me, 0), y = fps_coord<SOA>(pts, L.n, me, 1),
                     z = fps_coord<SOA>(pts, L.n, me, 2);
-        float m = __builtin_huge_valf();
-#pragma unroll 4
-        for (int i = from; i < to; ++i)
-            m = __builtin_fminf(m, tk_dist2<float>(x, y, z, fps_coord<SOA>(pts, L.n, i, 0),
-                                                   fps_coord<SOA>(pts, L.n, i, 1),
-                                                   fps_coord<SOA>(pts, L.n, i, 2)));
-        s_min[part][lane] = m;
-        __syncthreads();
-        m = __builtin_huge_valf();
-        for (int w = 0; w < part; ++w)
-            m = __builtin_fminf(m, s_min[w][lane]);
-#pragma unroll 4
-        for (int i = from; i < to; ++i) {
-            m = __builtin_fminf(m, tk_dist2<float>(x, y, z, fps_coord<SOA>(pts, L.n, i, 0),
-                                                   fps_coord<SOA>(pts, L.n, i, 1),
-                                                   fps_coord<SOA>(pts, L.n, i, 2)));
-            const float v = __builtin_bit_cast(float, (int)out[i + 1]);
-            if (m >= v && me != i + 1)  // (a point already taken has m = 0: there only if v is)
-                bad |= m > v || !(v > 0.0f) ||
-                       fps_position_of_point(me, L) < fps_position_of_point(i + 1, L);
-            bad |= !(v > 0.0f);
+        float before = __builtin_huge_valf();  // the minimum over the centres up to this turn's
+        for (int start = 0; start < centres; start += C * NW, turn ^= 1) {
+            const int from = start + wave * C;
+            float m[C];
+            const auto minima = [&](auto whole) {  // (whole: at addresses that the compiler sees are side by side)
+#pragma unroll
+                for (int u = 0; u < C; ++u) {  // (beyond the last centre v is infinite)
+                    const int i = whole ? from + u : fps_min(from + u, centres - 1);
+                    const float d = tk_dist2<float>(x, y, z, fps_coord<SOA>(pts, L.n, i, 0),
+                                                    fps_coord<SOA>(pts, L.n, i, 1), fps_coord<SOA>(pts, L.n, i, 2));
+                    m[u] = u ? __builtin_fminf(m[u ? u - 1 : 0], d) : d;
+                }
+            };
+            if (from + C <= centres)
+                minima(std::true_type());
+            else
+                minima(std::false_type());
+            s_min[turn][wave][lane] = m[C - 1];
+            __syncthreads();
+            float here = before;
+#pragma unroll
+            for (int w = 0; w < NW; ++w) {
+                const float o = s_min[turn][w][lane];
+                here = w < wave ? __builtin_fminf(here, o) : here;
+                before = __builtin_fminf(before, o);
+            }
+            float over = -1.0f;  // the largest minimum less its threshold
+            const auto compare = [&](auto meets) {
+#pragma unroll
+                for (int u = 0; u < C; ++u) {
+                    const float d = __builtin_fminf(m[u], here) - s_v[from + u];
+                    over = __builtin_fmaxf(over, meets && me == from + u + 1 ? -1.0f : d);
+                }
+            };
+            if (first <= from + C && from < first + TK_WAVE)  // a point of the group meets its own v here
+                compare(std::true_type());
+            else
+                compare(std::false_type());
+            bad |= over > 0.0f;
+            if (__builtin_amdgcn_ballot_w64(over == 0.0f) != 0ull)  // a tie
+                for (int i = from; i < fps_min(from + C, centres); ++i) {
+                    here = __builtin_fminf(here, tk_dist2<float>(x, y, z, fps_coord<SOA>(pts, L.n, i, 0),
+                                                                 fps_coord<SOA>(pts, L.n, i, 1),
+                                                                 fps_coord<SOA>(pts, L.n, i, 2)));
+                    const float v = s_v[i];
+                    if (here == v && me != i + 1)
+                        bad |= fps_position_of_point(me, L) < fps_position_of_point(i + 1, L);
+                }
         }
-        __syncthreads();  // (the next turn writes s_min)
     }
-    if (bad)
-        out[0] = FPS_BROKEN;  // (the same from whoever writes it)
+    return bad;
+}
+
+// Behind the band kernel: claims are checked, the clouds that it has left done, and the coordinates follow the
+// indices. A cloud's workgroups share the check and the copying; what has to be done by one of them is done by
+// the last one through. Its turn is counted, with who has found the claim wrong from bit 16, in the upper half of
+// out[1], which is zero until then (out[1] holds v_1, a float); nobody waits for anybody, and what a cloud is
+// in for is read from out[0] before the turn is taken, so only the last one changes it, after all have read it.
+// (Against a launch for the check and one for the rest, us: 4 x 1024 -> 512 75.3, 74.0; 8 x 16384 -> 1024 304,
+// 300, where one workgroup copied a cloud's coordinates; a claim that fails late 16 x 4096 -> 1024 249, 255.)
+template <int P, int NW, int NB, bool SOA>
+__global__ __launch_bounds__(NW * 64) void fps_settle_kernel_f32(const float *__restrict__ points,
+                                                                 int64_t *__restrict__ index,
+                                                                 float *__restrict__ sampled,
+                                                                 FpsLayout L, int slices)
+{
+    constexpr int NT = NW * TK_WAVE;
+    const int b = blockIdx.x / slices;
+    int slice = blockIdx.x % slices, of = slices;
+    const float *__restrict__ pts = points + (int64_t)b * L.n * 3;
+    int64_t *out = index + (int64_t)b * L.k;
+    const int64_t left = out[0];  // uniform over the workgroup
+    if (left < 0) {
+        __shared__ unsigned s_turn;
+        bool bad = false;
+        if (left == FPS_CLAIM)
+            bad = fps_claim_fails<NW, SOA>(pts, out, L, slice, slices);
+        bad = __syncthreads_or(bad);
+        if (threadIdx.x == 0)
+            s_turn = __hip_atomic_fetch_add(reinterpret_cast<unsigned *>(out + 1) + 1, bad ? 0x10001u : 1u,
+                                            __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        const unsigned turn = s_turn;
+        if ((turn & 0xffffu) != (unsigned)(slices - 1))
+            return;
+        if (left == FPS_ODD)
+            fps_plain<float, P, NT, SOA>(pts, out, L);
+        else if (bad || turn >> 16)
+            fps_band<P, NW, NB, SOA, true>(pts, out, L, false);
+        else
+            for (int i = threadIdx.x; i < L.k; i += NT)
+                out[i] = (int64_t)i;
+        __syncthreads();
+        slice = 0;
+        of = 1;
+    }
+    if (sampled) {
+        float *__restrict__ so = sampled + (int64_t)b * L.k * 3;
+        for (int i = slice * NT + threadIdx.x; i < L.k; i += of * NT) {
+            const int64_t j = out[i];
+#pragma unroll
+            for (int a = 0; a < 3; ++a)
+                so[SOA ? (int64_t)a * L.k + i : (int64_t)i * 3 + a] = fps_coord<SOA>(pts, L.n, j, a);
+        }
+    }
 }
 
 // Clouds that do not fit in one workgroup's registers: every selection step is one
@@ -1489,28 +1531,28 @@ int fps_band_launch(const float *points, int64_t B, int64_t *index, float *sampl
     // the sorted list, and behind it the sort's counters, then one coordinate of every point
     constexpr int LDS = NT * P * 4 + (NT * P > 4100 ? NT * P : 4100) * 4;
     constexpr auto kernel = fps_band_kernel_f32<P, NW, NB, SOA>;
-    constexpr auto last = fps_last_kernel_f32<P, NW, NB, SOA>;
+    constexpr auto settle = fps_settle_kernel_f32<P, NW, NB, SOA>;
     int allowed = tk_allow_dynamic_lds<kernel>(LDS);
     if (allowed == TK3D_OK)
-        allowed = tk_allow_dynamic_lds<last>(LDS);
+        allowed = tk_allow_dynamic_lds<settle>(LDS);
     if (allowed != TK3D_OK)
         return allowed;
-    // up to a workgroup per 64 points, and a launch holds less than 2^32 lanes
-    const int64_t most = (8 * tk_cu_count() + B - 1) / B;
-    const auto slices = [&](int n) {
-        const int groups = (n + TK_WAVE - 1) / TK_WAVE;
+    // up to a workgroup per 64 points: eight to a CU in all of the light first kernel, one of the second; and a
+    // launch holds less than 2^32 lanes
+    const auto slices = [&](int points_of, int each) {
+        const int groups = (points_of + TK_WAVE - 1) / TK_WAVE;
+        const int64_t most = (each * tk_cu_count() + B - 1) / B;
         return groups < most ? groups : (int)most;
     };
-    const int of_k = slices(L.k), of_n = slices(L.n);
     const bool claims = L.k <= FPS_CLAIM_MAX && B < ((int64_t)1 << 22);
     hipLaunchKernelGGL(kernel, dim3((unsigned)B), dim3(NT), LDS, s, points, index, L, claims);
     if (claims) {
+        const int of_k = slices(L.k, 8);
         hipLaunchKernelGGL((fps_claim_minima_kernel<SOA>), dim3((unsigned)(B * of_k)), dim3(1024), 0,
                            s, points, index, L, of_k);
-        hipLaunchKernelGGL((fps_claim_check_kernel<SOA>), dim3((unsigned)(B * of_n)), dim3(1024), 0,
-                           s, points, index, L, of_n);
     }
-    hipLaunchKernelGGL(last, dim3((unsigned)B), dim3(NT), LDS, s, points, index, sampled, L);
+    const int of_n = slices(claims ? L.n : L.k, 1);
+    hipLaunchKernelGGL(settle, dim3((unsigned)(B * of_n)), dim3(NT), LDS, s, points, index, sampled, L, of_n);
     return TK3D_OK;
 }
 
