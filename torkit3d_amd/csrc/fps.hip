@@ -561,6 +561,17 @@ __device__ __forceinline__ unsigned fps_append(unsigned bits, unsigned long long
     return bits;
 }
 
+// Zero exactly if the lane's bits have none in common with the mask. (Of 64 bits compared at once, the
+// comparison alone takes as long as all of this.)
+__device__ __forceinline__ unsigned fps_common(unsigned long long bits, unsigned long long mask)
+{
+    unsigned some;
+    asm("v_and_or_b32 %0, %1, %2, %3"
+        : "=v"(some)
+        : "v"((unsigned)(bits >> 32)), "s"((unsigned)(mask >> 32)), "v"((unsigned)bits & (unsigned)mask));
+    return some;
+}
+
 // Width of a band for `target` points where one of width `was` held n. (Any number will do, as long as
 // all waves have the same; a wave-uniform result.)
 __device__ __forceinline__ int fps_band(int was, float target, int n)
@@ -653,7 +664,7 @@ __device__ __forceinline__ void fps_band(const float *__restrict__ pts, int64_t 
     __shared__ float4 s_cand[LIST + 1];  // the band's points: x, y, z, running minimum (bits)
     __shared__ int s_name[LIST + 1];     // which points those are
     __shared__ __align__(16) Relation s_rel[LIST];
-    __shared__ int s_count[3], s_stop[3], s_most[3];
+    __shared__ int s_count[3], s_stop[3], s_most[3], s_step;
     __shared__ float s_red[NW][8];
 
     const int tid = threadIdx.x;
@@ -884,17 +895,21 @@ __device__ __forceinline__ void fps_band(const float *__restrict__ pts, int64_t 
     int tie_from = 0, tie_end = 0, tie_step = S / 8;
     int wide = step;  // the last band that was not of equals
 
-    int it = 1, n = 0, round = 0;
+    const int own_slot = (lane >> RJ_LOG2) + NJ * (lane & (RJ - 1));  // lane 8 w + i has candidate w + 8 i
+    const auto after = [](int turn) { return turn == 2 ? 0 : turn + 1; };
+    int it = 1, n = 0, turn = 0;  // (turn: which of three counters)
     while (it < L.k) {  // (uniform over the workgroup, as is all of this state)
         // ---- the points of the band; anew with another band if they are too many or none ----
         int theta;
         int crowd = 1 << 20;
         bool again = false;  // (then the largest minimum is looked for as well)
-        for (;; ++round, again = true) {
+        float4 C;
+        int my_name;
+        for (;; turn = after(turn), again = true) {
             theta = tied ? base - 1 : fps_max(base - step, 0);
-            int *const count = &s_count[round % 3];
+            int *const count = &s_count[turn];
             if (tid == 0)  // (their last readers are two barriers back)
-                s_count[(round + 1) % 3] = s_stop[(round + 1) % 3] = s_most[(round + 1) % 3] = 0;
+                s_count[after(turn)] = s_stop[after(turn)] = s_most[after(turn)] = 0;
             int first = wave * RS + lane;  // a point's name is this and a constant
             asm volatile("" : "+v"(first));  // (added where it is wanted, not kept in P registers)
             const auto enlist = [&](int p, int &at) {
@@ -942,10 +957,13 @@ __device__ __forceinline__ void fps_band(const float *__restrict__ pts, int64_t 
                     most = fps_max(most, t[p]);
                 most = wave_max_i32(fps_max(most, 0));
                 if (lane == 0)
-                    atomicMax(&s_most[round % 3], most);
+                    atomicMax(&s_most[turn], most);
             }
             __syncthreads();
-            n = __builtin_amdgcn_readfirstlane(*count);
+            const int listed = *count;
+            C = s_cand[own_slot];  // (requested before the count is looked at)
+            my_name = s_name[own_slot];
+            n = __builtin_amdgcn_readfirstlane(listed);
             if ((unsigned)(n - 1) < (unsigned)LIST)
                 break;
             if (n == 0) {
@@ -962,7 +980,7 @@ __device__ __forceinline__ void fps_band(const float *__restrict__ pts, int64_t 
                 } else {
                     if (theta == 0)
                         break;  // no point lies away from the chosen set, and none will
-                    base = again ? __builtin_amdgcn_readfirstlane(s_most[round % 3]) : theta;
+                    base = again ? __builtin_amdgcn_readfirstlane(s_most[turn]) : theta;
                     step = fps_min(2 * step, 1 << 24);
                 }
             } else if (tied) {  // (positions differ: LIST of them hold no more points)
@@ -975,7 +993,7 @@ __device__ __forceinline__ void fps_band(const float *__restrict__ pts, int64_t 
             } else {
                 step = base - theta;
                 if (again)
-                    base = __builtin_amdgcn_readfirstlane(s_most[round % 3]);
+                    base = __builtin_amdgcn_readfirstlane(s_most[turn]);
                 // (where a narrower band has not made them fewer, they are equal)
                 step = 4 * n > 3 * crowd ? 1 : fps_band(step, TARGET, n);
                 crowd = n;
@@ -983,23 +1001,29 @@ __device__ __forceinline__ void fps_band(const float *__restrict__ pts, int64_t 
         }
         if (n == 0)
             break;
-        // ---- lane 8 w + i has candidate w + 8 i ----
-        const int own_slot = (lane >> RJ_LOG2) + NJ * (lane & (RJ - 1));
-        const float4 C = s_cand[own_slot];
-        const int my_name = s_name[own_slot];
+        const auto next_step = [&] {
+            const int was = base - theta;
+            const int w = fps_max(fps_min(fps_max(fps_band(was, TARGET, n), was >> 1), 2 * was), 1);
+            return fps_min(w, 1 << 24);
+        };
+        if (NW > NJ && wave == NW - 1 && !tied) {  // uniform; it has nothing to judge
+            const int w = next_step();
+            if (lane == 0)
+                s_step = w;
+        }
         const int v = own_slot < n ? __builtin_bit_cast(int, C.w) : -1;
         if (wave < NJ) {
             // wave w relates the candidates of lanes RJ w .. to all of them
             unsigned hits = 0u, befores = 0u;
+            int over = 0;  // the largest distance to which a candidate falls
             int pos = -1;
             bool have_pos = false;
             const int rows = (n - wave + NJ - 1) / NJ;
-            int over = 0;
             const auto relate = [&](auto pair, int r) {  // the candidates of lanes r and, with pair, r + 1
                 constexpr int R = decltype(pair)::value;
                 float d[R];
                 int rv[R];
-                unsigned long long after[R], hit[R], same[R], kept = 0ull;
+                unsigned long long after[R], hit[R], same[R];
                 int equals = 0;
 #pragma unroll
                 for (int j = 0; j < R; ++j) {
@@ -1022,17 +1046,12 @@ __device__ __forceinline__ void fps_band(const float *__restrict__ pts, int64_t 
 #pragma unroll
                 for (int j = 0; j < R; ++j) {
                     hit[j] = after[j] & __builtin_amdgcn_ballot_w64(__builtin_bit_cast(int, d[j]) < v);
-                    kept |= hit[j] & __builtin_amdgcn_ballot_w64(__builtin_bit_cast(int, d[j]) > theta);
+                    over = fps_max(over, __builtin_amdgcn_inverse_ballot_w64(hit[j]) ? __builtin_bit_cast(int, d[j]) : 0);
                 }
 #pragma unroll
                 for (int j = R - 1; j >= 0; --j) {
                     befores = fps_append(befores, after[j]);
                     hits = fps_append(hits, hit[j]);
-                }
-                if (__builtin_expect(kept != 0ull, 0)) {  // uniform
-#pragma unroll
-                    for (int j = 0; j < R; ++j)
-                        over = fps_max(over, ((hit[j] >> lane) & 1ull) != 0ull ? __builtin_bit_cast(int, d[j]) : 0);
                 }
             };
             if (rows & 1)  // uniform
@@ -1042,36 +1061,37 @@ __device__ __forceinline__ void fps_band(const float *__restrict__ pts, int64_t 
                 relate(std::integral_constant<int, 2>{}, RJ * wave + i);
             s_rel[lane].before[wave] = (Piece)befores;
             s_rel[lane].hit[wave] = (Piece)hits;
-            if (__builtin_expect(__builtin_amdgcn_ballot_w64(over > 0) != 0ull, 0)) {  // uniform
+            if (__builtin_expect(__builtin_amdgcn_ballot_w64(over > theta) != 0ull, 0)) {  // uniform
                 over = wave_max_i32(over);
                 if (lane == 0)
-                    atomicMax(&s_stop[round % 3], over);
+                    atomicMax(&s_stop[turn], over);
             }
         }
         __syncthreads();
         const ulonglong2 rel = *reinterpret_cast<const ulonglong2 *>(&s_rel[lane]);
         const unsigned long long before = rel.x, hit = rel.y;
-        const int stop = __builtin_amdgcn_readfirstlane(fps_max(theta, s_stop[round % 3]));
+        const int stop = __builtin_amdgcn_readfirstlane(fps_max(theta, s_stop[turn]));
+        const int its_step = s_step;
         unsigned long long open = __builtin_amdgcn_ballot_w64(v >= 0), winners = 0ull;
         while (open != 0ull) {  // (the first of the open ones is decided in every turn)
             const unsigned long long may = open | winners;
-            const unsigned long long won = __builtin_amdgcn_ballot_w64((hit & may) == 0ull) & open;
+            const unsigned long long won = __builtin_amdgcn_ballot_w64(fps_common(hit, may) == 0u) & open;
             winners |= won;
-            const unsigned long long lost = __builtin_amdgcn_ballot_w64((hit & winners) != 0ull) & open;
+            const unsigned long long lost = __builtin_amdgcn_ballot_w64(fps_common(hit, winners) != 0u) & open;
             open &= ~(won | lost);
         }
         winners &= __builtin_amdgcn_ballot_w64(v > stop);
         // ---- their turns, and the minima they lower ----
         if (wave == NW - 1) {  // uniform
-            const int at = it + __builtin_popcountll(before & winners);
-            if (((winners >> lane) & 1ull) != 0ull && at < L.k)
+            unsigned long long mine = before;
+            asm volatile("" : "+v"(mine));  // (the others are not to work it out as well)
+            const int at = it + __builtin_popcountll(mine & winners);
+            if (__builtin_amdgcn_inverse_ballot_w64(winners) && at < L.k)
                 order[at] = my_name;
         }
         it += __builtin_popcountll(winners);
         if (!tied) {
-            const int was = base - theta;
-            step = fps_max(fps_min(fps_max(fps_band(was, TARGET, n), was >> 1), 2 * was), 1);
-            step = fps_min(step, 1 << 24);
+            step = NW > NJ ? __builtin_amdgcn_readfirstlane(its_step) : next_step();
             wide = fps_max(step, wide >> 1);
             base = stop;
         } else {
@@ -1116,7 +1136,7 @@ __device__ __forceinline__ void fps_band(const float *__restrict__ pts, int64_t 
                 }
             }
         }
-        ++round;
+        turn = after(turn);
     }
     __syncthreads();
     // (after the last point that lies away from the chosen ones the previous choice is repeated)
