@@ -512,12 +512,10 @@ __device__ __forceinline__ int fps_min(int a, int b) { return a < b ? a : b; }
 
 // Place of the cell (x, y, z) of a 16^3 grid along a Hilbert curve (J. Skilling, "Programming the
 // Hilbert curve", AIP Conference Proceedings 707, 2004).
-__device__ __forceinline__ unsigned fps_hilbert(unsigned x, unsigned y, unsigned z)
+constexpr unsigned fps_hilbert(unsigned x, unsigned y, unsigned z)
 {
     unsigned c[3] = {x, y, z};
-#pragma unroll
     for (unsigned q = 8u; q > 1u; q >>= 1) {
-#pragma unroll
         for (int a = 0; a < 3; ++a) {
             const bool flip = (c[a] & q) != 0u;
             const unsigned swap = flip ? 0u : (c[0] ^ c[a]) & (q - 1u);
@@ -528,17 +526,43 @@ __device__ __forceinline__ unsigned fps_hilbert(unsigned x, unsigned y, unsigned
     c[1] ^= c[0];
     c[2] ^= c[1];
     unsigned gray = 0u;
-#pragma unroll
     for (unsigned q = 8u; q > 1u; q >>= 1)
         gray ^= (c[2] & q) != 0u ? q - 1u : 0u;
     unsigned place = 0u;
-#pragma unroll
-    for (int b = 3; b >= 0; --b) {
-#pragma unroll
+    for (int b = 3; b >= 0; --b)
         for (int a = 0; a < 3; ++a)
             place = 2u * place + (((c[a] ^ gray) >> b) & 1u);
-    }
     return place;
+}
+
+// The places of all cells, by 256 x + 16 y + z. (Worked out for every point they took 150 operations, 13 us of
+// the 612 at 8 x 16384 -> 4096 and 3 of the 155 at 16 x 4096 -> 1024.)
+struct FpsCurve {
+    unsigned short place[4096];
+};
+constexpr FpsCurve fps_make_curve()
+{
+    FpsCurve t{};
+    for (unsigned i = 0; i < 4096u; ++i)
+        t.place[i] = (unsigned short)fps_hilbert(i >> 8, (i >> 4) & 15u, i & 15u);
+    return t;
+}
+__device__ constexpr FpsCurve fps_curve alignas(16) = fps_make_curve();
+
+// The maxima over the 64 lanes of six values at once, left in lane 63: the steps of one value are the wait
+// between those of another, and the maximum takes its operand from the other lane itself.
+__device__ __forceinline__ void wave_max_six(float (&v)[6])
+{
+#define TK_STEP(HOW)                                              \
+    "v_max_f32_dpp %0, %0, %0 " HOW "\n\tv_max_f32_dpp %1, %1, %1 " HOW \
+    "\n\tv_max_f32_dpp %2, %2, %2 " HOW "\n\tv_max_f32_dpp %3, %3, %3 " HOW \
+    "\n\tv_max_f32_dpp %4, %4, %4 " HOW "\n\tv_max_f32_dpp %5, %5, %5 " HOW "\n\t"
+    asm("s_nop 1\n\t" TK_STEP("row_shr:1 row_mask:0xf bank_mask:0xf") TK_STEP("row_shr:2 row_mask:0xf bank_mask:0xf")
+            TK_STEP("row_shr:4 row_mask:0xf bank_mask:0xf") TK_STEP("row_shr:8 row_mask:0xf bank_mask:0xf")
+                TK_STEP("row_bcast:15 row_mask:0xa bank_mask:0xf") TK_STEP("row_bcast:31 row_mask:0xc bank_mask:0xf")
+        "s_nop 1"
+        : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]));
+#undef TK_STEP
 }
 
 // Adds to a counter in LDS, lane by lane, and returns what it held before. (As an atomicAdd the
@@ -619,12 +643,12 @@ __device__ __forceinline__ int fps_band(int was, float target, int n)
 // 4096 -> 1024 on one of 9 x 9 x 9 points 0.35 -> 0.19 ms.
 //
 // What bounds it: one workgroup has one compute unit, and an exchange is a chain of short phases (clocks
-// at 16 x 4096 -> 1024, 16 waves, of 6700 for 19 winners: listing 1100, judgement 1700, resolving and
-// turns 800, update 1540 on average and 2050 in the slowest wave, with the boxes; the rest is waiting at the
+// at 16 x 4096 -> 1024, 16 waves, of 6700 for 19 winners, of which shorter chains of instructions have since
+// taken 250: listing 1100, judgement 1700, resolving and turns 800, update 1540 on average and 2050 in the slowest wave, with the boxes; the rest is waiting at the
 // barriers, and 14 of 67 bands are listed again). Measured (us; before: a candidate per group; both
-// with what runs behind them): 8 x 16384 -> 4096 1390-1450 -> 590, on a noisy sphere 1120-1200 -> 560,
-// in clusters 1180-1330 -> 700-730; 16 x 8192 -> 2048 590 -> 285; 16 x 4096 -> 1024 285 -> 160; 16 x 2048 -> 512
-// 160 -> 97; 1 x 1024 -> 512 120 -> 76; on lattices, copies and a line 0.2 to 0.9 of the time before.
+// with what runs behind them): 8 x 16384 -> 4096 1390-1450 -> 545, on a noisy sphere 1120-1200 -> 520,
+// in clusters 1180-1330 -> 695; 16 x 8192 -> 2048 590 -> 275; 16 x 4096 -> 1024 285 -> 150; 16 x 2048 -> 512
+// 160 -> 94; 1 x 1024 -> 512 120 -> 69; on lattices, copies and a line 0.2 to 0.9 of the time before.
 // Tried: listing up to 256 and judging the upper 64 (0 to 5 % faster up to 8192 points, 4 % slower
 // at 16384, lattices 10 % slower), aiming at 28, 34, 56 or 80 points, blocks of half and twice the
 // size and half as many waves with twice the points (all slower by 2 to 20 % at the sizes where another
@@ -707,19 +731,23 @@ __device__ __forceinline__ void fps_band(const float *__restrict__ pts, int64_t 
     }
     far = wave_max<float>(far);
     odd = __builtin_amdgcn_ballot_w64(odd) != 0ull;
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        lo[a] = -wave_max<float>(-lo[a]);
-        hi[a] = wave_max<float>(hi[a]);
-    }
-    if (lane == 0) {
+    float ends[6] = {-lo[0], -lo[1], -lo[2], hi[0], hi[1], hi[2]};
+    wave_max_six(ends);
+    if (lane == TK_WAVE - 1) {
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
-            s_red[wave][a] = lo[a];
-            s_red[wave][3 + a] = hi[a];
+            s_red[wave][a] = -ends[a];
+            s_red[wave][3 + a] = ends[3 + a];
         }
         s_red[wave][6] = odd ? -1.0f : far;
     }
+    // (the table where the list comes later, if there is room)
+    constexpr bool NEAR = S * 4 >= (int)sizeof(FpsCurve);
+    if constexpr (NEAR)
+        for (int i = tid; i < (int)sizeof(FpsCurve) / 16; i += NT)
+            reinterpret_cast<uint4 *>(fps_band_lds)[i] = reinterpret_cast<const uint4 *>(&fps_curve)[i];
+    const unsigned short *const curve =
+        NEAR ? reinterpret_cast<const unsigned short *>(fps_band_lds) : fps_curve.place;
     for (int i = tid; i <= CELLS; i += NT)
         cnt[i] = 0u;
     if (tid < 3)
@@ -779,7 +807,7 @@ __device__ __forceinline__ void fps_band(const float *__restrict__ pts, int64_t 
         scale[a] = extent > 0.0f ? 15.99f / extent : 0.0f;  // also 0 for NaN / inf extents
     }
 
-    // ---- the points in the order of their cells along a Morton curve; slots beyond the cloud
+    // ---- the points in the order of their cells along the curve; slots beyond the cloud
     // last. A counting sort: any order that keeps neighbours together is a valid layout, so 16
     // steps per axis are enough and the order within a cell is whatever the atomics give. ----
     unsigned where[P];  // cell, and the point's turn within it from bit 13
@@ -787,14 +815,14 @@ __device__ __forceinline__ void fps_band(const float *__restrict__ pts, int64_t 
     for (int k = 0; k < P; ++k) {
         unsigned cell = CELLS;
         if (tid + k * NT < L.n) {
-            unsigned c3[3];
+            unsigned at = 0u;
 #pragma unroll
             for (int a = 0; a < 3; ++a) {
                 const float f = (own[a][k] - origin[a]) * scale[a];
                 // (a NaN or an out-of-range value lands in cell 0 or 15)
-                c3[a] = (unsigned)(int)__builtin_fminf(__builtin_fmaxf(f, 0.0f), 15.0f);
+                at = 16u * at + (unsigned)(int)__builtin_fminf(__builtin_fmaxf(f, 0.0f), 15.0f);
             }
-            cell = fps_hilbert(c3[0], c3[1], c3[2]);
+            cell = curve[at];
         }
         where[k] = cell | (atomicAdd(&cnt[cell], 1u) << 13);
     }
@@ -864,7 +892,7 @@ __device__ __forceinline__ void fps_band(const float *__restrict__ pts, int64_t 
     float box[NB][6];
 #pragma unroll
     for (int q = 0; q < NB; ++q) {
-        float bl[3] = {INF, INF, INF}, bh[3] = {-INF, -INF, -INF};
+        float reach[6] = {-INF, -INF, -INF, -INF, -INF, -INF};  // -lowest, highest
 #pragma unroll
         for (int u = 0; u < PB; ++u) {
             const int p = q * PB + u;
@@ -872,16 +900,17 @@ __device__ __forceinline__ void fps_band(const float *__restrict__ pts, int64_t 
             const float v[3] = {x[p], y[p], z[p]};
 #pragma unroll
             for (int a = 0; a < 3; ++a) {
-                bl[a] = __builtin_fminf(bl[a], ok ? v[a] : INF);
-                bh[a] = __builtin_fmaxf(bh[a], ok ? v[a] : -INF);
+                reach[a] = __builtin_fmaxf(reach[a], ok ? -v[a] : -INF);
+                reach[3 + a] = __builtin_fmaxf(reach[3 + a], ok ? v[a] : -INF);
             }
             const float d = tk_dist2<float>(x[p], y[p], z[p], p0[0], p0[1], p0[2]);
             t[p] = ok ? __builtin_bit_cast(int, d) : F32_NEG1;
         }
+        wave_max_six(reach);
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
-            box[q][a] = -wave_max<float>(-bl[a]);
-            box[q][3 + a] = wave_max<float>(bh[a]);
+            box[q][a] = -read_lane(reach[a], TK_WAVE - 1);
+            box[q][3 + a] = read_lane(reach[3 + a], TK_WAVE - 1);
         }
     }
     __syncthreads();  // plane1 is read
@@ -1585,11 +1614,11 @@ int fps_band_launch_f32(const float *points, bool soa, int64_t B, int64_t *index
 }
 
 // fp32, the band kernel: whether it takes the call, and its launch if so. It needs 192 samples to
-// be paid for: its prologue sorts the cloud, which costs 5 us at 1024 points and 25 at 16384, and
+// be paid for: its prologue sorts the cloud, which costs 4 us at 1024 points and about 10 at 16384, and
 // early in a sampling, where the points far from all centres are neighbours, a band of 64 holds one or
-// two winners. Multi-step kernel against this one, with what runs behind them, us, at 128 samples:
-// 1 x 300 42, 35; 16 x 600 48, 55; 16 x 1024 50, 59; 16 x 4096 77, 83; 16 x 16384 159, 161; at 192: 65, 45;
-// 67, 53; 69, 56; 104, 86; 222, 177. In sampling order, in which an encoder's levels come, it has 16 for
+// two winners. Multi-step kernel against this one, with what runs behind them, us, at 128 samples (this
+// one 2 to 20 us slower than now): 1 x 300 42, 35; 16 x 600 48, 55; 16 x 1024 50, 59; 16 x 4096 77, 83; 16 x 16384
+// 159, 161; at 192: 65, 43; 67, 47; 69, 54; 104, 82; 222, 153. In sampling order, in which an encoder's levels come, it has 16 for
 // 46 to 210 at 192 samples.
 bool fps_band_dispatch_f32(const float *points, bool soa, int64_t B, int64_t *index, float *sampled,
                              const FpsLayout &L, int64_t npos, hipStream_t s, int &rc)
