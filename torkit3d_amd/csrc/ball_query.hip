@@ -9,6 +9,12 @@
 // fraction of the cloud - whereas the reference always scans to the end.
 // Remaining slots repeat the first hit; a query with no hit gets -1 everywhere
 // (ball_query_kernel.cu:94-101, :123).
+//
+// What bounds it: the seven vector instructions of a test, 28 clocks per query and 64 keys on one SIMD, where hits
+// are few (8 x 4096 queries, 16384 keys, radius 0.02 of the unit cube: 99 us, 29 clocks); at radius 0.1 the scan ends
+// early and every fourth chunk has a hit, 92 us. Whether a query is full is asked once per trip and not per chunk
+// (96 -> 92 us there; 8 x 2048 queries 62 -> 54; 16 x 1024 on a sphere of 8000 keys 39 -> 36). Tried: hits of 2, 4
+// or 8 chunks looked for together (99, 133, 170 us), since the chunks' hits are then handled where there are none.
 #include "tk3d_common.h"
 
 namespace {
@@ -78,24 +84,23 @@ __global__ __launch_bounds__(256) void ball_query_kernel(const T *__restrict__ q
         bool all_done = true;
 #pragma unroll
         for (int q = 0; q < QW; ++q) {
+            if (cnt[q] < k) {  // wave-uniform; a query that is full by the end of the trip drops its later hits
 #pragma unroll
-            for (int u = 0; u < UNROLL; ++u) {
-                if (cnt[q] >= k)  // wave-uniform
-                    continue;
-                const int j = j0 + u * TK_WAVE + lane;
-                const T d = tk_dist2<T>(kx[u], ky[u], kz[u], qx[q], qy[q], qz[q]);
-                const bool hit = d < r2;  // false for the NaN of a key that does not exist
-                const unsigned long long mask = __builtin_amdgcn_ballot_w64(hit);
-                if (mask == 0)
-                    continue;
-                const int below = __builtin_amdgcn_mbcnt_hi(
-                    (unsigned)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0));
-                const int slot = cnt[q] + below;
-                if (hit && slot < k)
-                    out[(int64_t)q * k + slot] = (int64_t)j;
-                if (cnt[q] == 0)
-                    first[q] = j0 + u * TK_WAVE + __builtin_ctzll(mask);
-                cnt[q] += __builtin_popcountll(mask);
+                for (int u = 0; u < UNROLL; ++u) {
+                    // (false for the NaN of a key that does not exist)
+                    const unsigned long long mask = __builtin_amdgcn_ballot_w64(
+                        tk_dist2<T>(kx[u], ky[u], kz[u], qx[q], qy[q], qz[q]) < r2);
+                    if (mask == 0)
+                        continue;
+                    const int below = __builtin_amdgcn_mbcnt_hi(
+                        (unsigned)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0));
+                    const int j = j0 + u * TK_WAVE + lane, slot = cnt[q] + below;
+                    if (__builtin_amdgcn_inverse_ballot_w64(mask) && slot < k)
+                        out[(int64_t)q * k + slot] = (int64_t)j;
+                    if (cnt[q] == 0)
+                        first[q] = j0 + u * TK_WAVE + __builtin_ctzll(mask);
+                    cnt[q] += __builtin_popcountll(mask);
+                }
             }
             all_done = all_done && (cnt[q] >= k);
         }
