@@ -290,37 +290,16 @@ __global__ __launch_bounds__(BLOCK) void chamfer_forward_kernel(ChamferFwdArgs<T
 // exact sweep for the whole workgroup or the exact scan for the query.
 // Results are therefore bit-identical to the exact sweep for every input.
 
-// Minimum / maximum over the wave, the same value in every lane (NaNs are passed over, as
-// fminf / fmaxf do). A scan along rows of 16 lanes with row shifts, the rows' results carried
-// on with row broadcasts, the total read from lane 63: six short steps on the vector ALU where
-// six exchanges through the LDS crossbar (ds_bpermute) took a hundred clocks each.
-template <bool MAX> __device__ __forceinline__ float wave_reduce_extreme(float v)
-{
-#define TK_WAVE_STEP(ctrl, rows)                                                              \
-    {                                                                                         \
-        const float o = __builtin_bit_cast(                                                   \
-            float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, v),                    \
-                                               __builtin_bit_cast(int, v), ctrl, rows, 0xf,   \
-                                               false));                                       \
-        v = MAX ? __builtin_fmaxf(v, o) : __builtin_fminf(v, o);                              \
-    }
-    TK_WAVE_STEP(0x111, 0xf)  // row_shr:1
-    TK_WAVE_STEP(0x112, 0xf)  // row_shr:2
-    TK_WAVE_STEP(0x114, 0xf)  // row_shr:4
-    TK_WAVE_STEP(0x118, 0xf)  // row_shr:8
-    TK_WAVE_STEP(0x142, 0xa)  // row_bcast:15 into rows 1 and 3
-    TK_WAVE_STEP(0x143, 0xc)  // row_bcast:31 into rows 2 and 3
-#undef TK_WAVE_STEP
-    return __builtin_bit_cast(float,
-                              __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), TK_WAVE - 1));
-}
+// Minimum / maximum over the wave, the same value in every lane: a scan along rows of 16 lanes with row shifts,
+// the rows' results carried on with row broadcasts, the total read from lane 63, where six exchanges through the LDS
+// crossbar (ds_bpermute) took a hundred clocks each.
 __device__ __forceinline__ float wave_reduce_min(float v)
 {
-    return wave_reduce_extreme<false>(v);
+    return tk_wave_extreme<false>(v);
 }
 __device__ __forceinline__ float wave_reduce_max(float v)
 {
-    return wave_reduce_extreme<true>(v);
+    return tk_wave_extreme<true>(v);
 }
 
 // Exact nearest neighbour of one query, the whole workgroup cooperating: lane t scans
@@ -2757,26 +2736,6 @@ __device__ __forceinline__ float tk_order_float(int i)
     return __builtin_bit_cast(float, i ^ ((i >> 31) & 0x7fffffff));
 }
 
-// Minimum (MAX: maximum) over each half of the wave, left in lanes 31 and 63: a scan along
-// rows of 16 lanes with row shifts, then row 0's result carried into row 1 (2's into 3).
-// On integers: a floating-point minimum quiets its operands first, one more instruction per
-// step and operand (57 of the 271 instructions a sorted point cost went there).
-template <bool MAX> __device__ __forceinline__ int half_wave_reduce_to_last(int v)
-{
-#define TK_HALF_WAVE_STEP(ctrl, rows)                                                  \
-    {                                                                                  \
-        const int o = __builtin_amdgcn_update_dpp(v, v, ctrl, rows, 0xf, false);       \
-        v = MAX ? (o > v ? o : v) : (o < v ? o : v);                                   \
-    }
-    TK_HALF_WAVE_STEP(0x111, 0xf)  // row_shr:1
-    TK_HALF_WAVE_STEP(0x112, 0xf)  // row_shr:2
-    TK_HALF_WAVE_STEP(0x114, 0xf)  // row_shr:4
-    TK_HALF_WAVE_STEP(0x118, 0xf)  // row_shr:8
-    TK_HALF_WAVE_STEP(0x142, 0xa)  // row_bcast:15 into rows 1 and 3
-#undef TK_HALF_WAVE_STEP
-    return v;
-}
-
 // Everything the pruned sweep needs of one cloud of up to 16384 points, in one launch.
 // `parts` workgroups of 1024 lanes (16 points per lane) serve a cloud. Each works out, for
 // itself, what needs the whole cloud:
@@ -2918,22 +2877,22 @@ __global__ __launch_bounds__(1024) void chamfer_prepare_kernel(ChamferSortArgs a
     }
 #pragma unroll
     for (int ax = 0; ax < 3; ++ax) {
-        lo[ax] = wave_reduce_min(lo[ax]);
-        hi[ax] = wave_reduce_max(hi[ax]);
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1)
             dev[ax] += __shfl_xor(dev[ax], o);
     }
+    float ends[6] = {-lo[0], -lo[1], -lo[2], hi[0], hi[1], hi[2]};
+    tk_wave_max_six<64>(ends);
     if (tid == 0) {
         sbad = 0;
         sfar = 0;
     }
     __syncthreads();
-    if (lane == 0) {
+    if (lane == TK_WAVE - 1) {
 #pragma unroll
         for (int ax = 0; ax < 3; ++ax) {
-            sred[wave][ax] = lo[ax];
-            sred[wave][3 + ax] = hi[ax];
+            sred[wave][ax] = -ends[ax];
+            sred[wave][3 + ax] = ends[3 + ax];
             sdev[wave][ax] = dev[ax];
         }
     }
@@ -3163,24 +3122,19 @@ __global__ __launch_bounds__(1024) void chamfer_prepare_kernel(ChamferSortArgs a
                 tile[0] = h0;
                 tile[32] = h1;
             }
-            int bl[3], bh[3];
-            bl[0] = half_wave_reduce_to_last<false>(swept ? tk_float_order(x) : ORDER_POS_INF);
-            bl[1] = half_wave_reduce_to_last<false>(swept ? tk_float_order(y) : ORDER_POS_INF);
-            bl[2] = half_wave_reduce_to_last<false>(swept ? tk_float_order(z) : ORDER_POS_INF);
-            bh[0] = half_wave_reduce_to_last<true>(swept ? tk_float_order(x) : ORDER_NEG_INF);
-            bh[1] = half_wave_reduce_to_last<true>(swept ? tk_float_order(y) : ORDER_NEG_INF);
-            bh[2] = half_wave_reduce_to_last<true>(swept ? tk_float_order(z) : ORDER_NEG_INF);
+            float ends[6] = {swept ? -x : -INF, swept ? -y : -INF, swept ? -z : -INF,
+                             swept ? x : -INF,  swept ? y : -INF,  swept ? z : -INF};
+            tk_wave_max_six<32>(ends);
             // the tile's box comes from the part that owns the tile's first position
             if ((i & 31) == 31 && i - 31 >= s_lo) {
+                float fl[3] = {-ends[0], -ends[1], -ends[2]}, fh[3] = {ends[3], ends[4], ends[5]};
                 if (i + 1 == shared_end) {
 #pragma unroll
                     for (int ax = 0; ax < 3; ++ax) {
-                        bl[ax] = sextra[ax] < bl[ax] ? sextra[ax] : bl[ax];
-                        bh[ax] = sextra[3 + ax] > bh[ax] ? sextra[3 + ax] : bh[ax];
+                        fl[ax] = __builtin_fminf(fl[ax], tk_order_float(sextra[ax]));
+                        fh[ax] = __builtin_fmaxf(fh[ax], tk_order_float(sextra[3 + ax]));
                     }
                 }
-                const float fl[3] = {tk_order_float(bl[0]), tk_order_float(bl[1]), tk_order_float(bl[2])};
-                const float fh[3] = {tk_order_float(bh[0]), tk_order_float(bh[1]), tk_order_float(bh[2])};
                 boxes[i >> 5] = chamfer_box_bits(fl, fh);
             }
         }
@@ -3443,10 +3397,14 @@ __global__ __launch_bounds__(256) void chamfer_pruned_kernel(ChamferPrunedArgs a
             qnmax = __builtin_fmaxf(qnmax, qnorm[g]);
         }
     }
+    {
+        float ends[6] = {-blo[0], -blo[1], -blo[2], bhi[0], bhi[1], bhi[2]};
+        tk_wave_max_six<64>(ends);
 #pragma unroll
-    for (int ax = 0; ax < 3; ++ax) {
-        blo[ax] = wave_reduce_min(blo[ax]);
-        bhi[ax] = wave_reduce_max(bhi[ax]);
+        for (int ax = 0; ax < 3; ++ax) {
+            blo[ax] = -__builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, ends[ax]), 63));
+            bhi[ax] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, ends[3 + ax]), 63));
+        }
     }
     const bool nothing_to_sweep = !(blo[0] <= bhi[0]);  // padding and strays only (uniform)
     if (nothing_to_sweep && nstray == 0)

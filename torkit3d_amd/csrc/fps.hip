@@ -71,6 +71,8 @@ __device__ __forceinline__ double read_lane(double v, int lane)
 // the row totals up so that lane 63 holds the result.
 template <typename T> __device__ __forceinline__ T wave_max(T v)
 {
+    if constexpr (std::is_same<T, float>::value)
+        return tk_wave_extreme<true>(v);
     v = tk_max<T>(v, dpp_move<0x111, 0xF>(v));
     v = tk_max<T>(v, dpp_move<0x112, 0xF>(v));
     v = tk_max<T>(v, dpp_move<0x114, 0xF>(v));
@@ -549,22 +551,6 @@ constexpr FpsCurve fps_make_curve()
 }
 __device__ constexpr FpsCurve fps_curve alignas(16) = fps_make_curve();
 
-// The maxima over the 64 lanes of six values at once, left in lane 63: the steps of one value are the wait
-// between those of another, and the maximum takes its operand from the other lane itself.
-__device__ __forceinline__ void wave_max_six(float (&v)[6])
-{
-#define TK_STEP(HOW)                                              \
-    "v_max_f32_dpp %0, %0, %0 " HOW "\n\tv_max_f32_dpp %1, %1, %1 " HOW \
-    "\n\tv_max_f32_dpp %2, %2, %2 " HOW "\n\tv_max_f32_dpp %3, %3, %3 " HOW \
-    "\n\tv_max_f32_dpp %4, %4, %4 " HOW "\n\tv_max_f32_dpp %5, %5, %5 " HOW "\n\t"
-    asm("s_nop 1\n\t" TK_STEP("row_shr:1 row_mask:0xf bank_mask:0xf") TK_STEP("row_shr:2 row_mask:0xf bank_mask:0xf")
-            TK_STEP("row_shr:4 row_mask:0xf bank_mask:0xf") TK_STEP("row_shr:8 row_mask:0xf bank_mask:0xf")
-                TK_STEP("row_bcast:15 row_mask:0xa bank_mask:0xf") TK_STEP("row_bcast:31 row_mask:0xc bank_mask:0xf")
-        "s_nop 1"
-        : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]));
-#undef TK_STEP
-}
-
 // Adds to a counter in LDS, lane by lane, and returns what it held before. (As an atomicAdd the
 // compiler turns it into a scan over the lanes, for a handful of which it is.)
 __device__ __forceinline__ int fps_lds_add(int *counter, int v)
@@ -732,7 +718,7 @@ __device__ __forceinline__ void fps_band(const float *__restrict__ pts, int64_t 
     far = wave_max<float>(far);
     odd = __builtin_amdgcn_ballot_w64(odd) != 0ull;
     float ends[6] = {-lo[0], -lo[1], -lo[2], hi[0], hi[1], hi[2]};
-    wave_max_six(ends);
+    tk_wave_max_six<64>(ends);
     if (lane == TK_WAVE - 1) {
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
@@ -906,7 +892,7 @@ __device__ __forceinline__ void fps_band(const float *__restrict__ pts, int64_t 
             const float d = tk_dist2<float>(x[p], y[p], z[p], p0[0], p0[1], p0[2]);
             t[p] = ok ? __builtin_bit_cast(int, d) : F32_NEG1;
         }
-        wave_max_six(reach);
+        tk_wave_max_six<64>(reach);
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
             box[q][a] = -read_lane(reach[a], TK_WAVE - 1);

@@ -135,6 +135,49 @@ template <auto Kernel> static inline int tk_allow_dynamic_lds(int bytes)
     return TK3D_OK;
 }
 
+// The maxima over the wave (LANES 64, left in lane 63) or over each half of it (32, in lanes 31 and 63) of six values
+// at once: the steps of one value are the wait between those of another, and a maximum takes its operand from the
+// other lane itself. One by one, through moves, the compiler makes it five instructions a step.
+template <int LANES> __device__ __forceinline__ void tk_wave_max_six(float (&v)[6])
+{
+#define TK_STEP(HOW)                                                           \
+    "v_max_f32_dpp %0, %0, %0 " HOW "\n\tv_max_f32_dpp %1, %1, %1 " HOW      \
+    "\n\tv_max_f32_dpp %2, %2, %2 " HOW "\n\tv_max_f32_dpp %3, %3, %3 " HOW \
+    "\n\tv_max_f32_dpp %4, %4, %4 " HOW "\n\tv_max_f32_dpp %5, %5, %5 " HOW "\n\t"
+    asm("s_nop 1\n\t"
+        TK_STEP("row_shr:1 row_mask:0xf bank_mask:0xf")
+        TK_STEP("row_shr:2 row_mask:0xf bank_mask:0xf")
+        TK_STEP("row_shr:4 row_mask:0xf bank_mask:0xf")
+        TK_STEP("row_shr:8 row_mask:0xf bank_mask:0xf")
+        TK_STEP("row_bcast:15 row_mask:0xa bank_mask:0xf")
+        "s_nop 1"
+        : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]));
+    if constexpr (LANES == 64)
+        asm("s_nop 1\n\t"
+            TK_STEP("row_bcast:31 row_mask:0xc bank_mask:0xf")
+            "s_nop 1"
+            : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]));
+#undef TK_STEP
+}
+
+// Minimum or maximum over the wave, the same value in every lane (quiet NaNs are passed over).
+template <bool MAX> __device__ __forceinline__ float tk_wave_extreme(float v)
+{
+#define TK_STEPS(OP)                                                     \
+    "s_nop 1\n\t" OP " %0, %0, %0 row_shr:1 row_mask:0xf bank_mask:0xf\n\t"  \
+    "s_nop 1\n\t" OP " %0, %0, %0 row_shr:2 row_mask:0xf bank_mask:0xf\n\t"  \
+    "s_nop 1\n\t" OP " %0, %0, %0 row_shr:4 row_mask:0xf bank_mask:0xf\n\t"  \
+    "s_nop 1\n\t" OP " %0, %0, %0 row_shr:8 row_mask:0xf bank_mask:0xf\n\t"  \
+    "s_nop 1\n\t" OP " %0, %0, %0 row_bcast:15 row_mask:0xa bank_mask:0xf\n\t" \
+    "s_nop 1\n\t" OP " %0, %0, %0 row_bcast:31 row_mask:0xc bank_mask:0xf\n\ts_nop 1"
+    if constexpr (MAX)
+        asm(TK_STEPS("v_max_f32_dpp") : "+v"(v));
+    else
+        asm(TK_STEPS("v_min_f32_dpp") : "+v"(v));
+#undef TK_STEPS
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), TK_WAVE - 1));
+}
+
 // Compute units of the current device (256 when the query fails), looked up once per device.
 static inline int tk_cu_count()
 {
