@@ -93,6 +93,20 @@ def test_hard_inputs_on_longer_clouds(cuda, kind):
     check_sorted(a.contiguous(), c.contiguous(), cuda)
 
 
+@pytest.mark.parametrize("n1", [1, 5, 64, 65, 1030, 4100])
+@pytest.mark.parametrize("size,spread", [(20, 1e-3), (40, 1e-3), (56, 3e-4), (64, 0.0)])
+def test_several_candidate_half_tiles_a_query(cuda, n1, size, spread):
+    # keys in knots of 20 to 64 that lie in one tile or two, all about as near to a query beside them: up to both
+    # halves of both tiles are evaluated for it, or the query is scanned, and waves with few queries have few
+    g = gen(size + n1)
+    knots = uniform_cloud(g, 2, 9600 // size)
+    keys = knots.repeat_interleave(size, dim=1)
+    keys = keys + spread * torch.rand(keys.shape, generator=g)
+    keys = keys[:, torch.randperm(keys.size(1), generator=g)]
+    queries = knots[:, torch.arange(n1) % knots.size(1)] + 2e-3 * torch.rand(2, n1, 3, generator=g)
+    check_sorted(queries, keys, cuda)
+
+
 def test_ties_go_to_the_lowest_original_index(cuda):
     # every key position occurs many times, at indices far apart: sorted order puts the
     # copies next to each other in an order of its own, the result must still name the

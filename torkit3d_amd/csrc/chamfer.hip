@@ -2219,7 +2219,7 @@ int chamfer_forward(const T *xyz1, const T *xyz2, int64_t B, int64_t N1, int64_t
 //     terms of every key (the layout the matrix kernel stages in LDS) and the tile's
 //     bounding box in centred, scaled coordinates; keys far outside the frame go on a
 //     short list instead.
-//   chamfer_pruned_kernel (waves work alone, no LDS): a wave takes NQB x 32 consecutive
+//   chamfer_pruned_kernel (waves work alone): a wave takes NQB x 32 consecutive
 //     sorted queries - a compact patch - and sweeps a key tile only if the squared gap
 //     between the patch's box and the tile's box does not exceed T, an upper bound of
 //     every query's distance to the nearest key met so far: first the tiles that overlap
@@ -3141,6 +3141,36 @@ __global__ __launch_bounds__(1024) void chamfer_prepare_kernel(ChamferSortArgs a
     }
 }
 
+// A double of another lane of the quad.
+template <int CTRL> __device__ __forceinline__ double quad_move(double v)
+{
+    const unsigned long long bits = __builtin_bit_cast(unsigned long long, v);
+    const auto half = [](unsigned w) { return (unsigned)__builtin_amdgcn_mov_dpp((int)w, CTRL, 0xf, 0xf, true); };
+    return __builtin_bit_cast(double, (unsigned long long)half((unsigned)(bits >> 32)) << 32 | half((unsigned)bits));
+}
+
+// The nearest of the keys of a half tile (four runs of four, eight keys apart) to a query, for each quad of lanes
+// one: a key of every run a lane. The nearest as a (distance bits, index) word: distances are non-negative, so the
+// words order as such pairs, also as doubles, all of them finite, of which a minimum is one instruction. The NaN of
+// padding, whose sign is clear, lies above +inf. `task`: tile, half, query (see where they are listed).
+__device__ __forceinline__ double chamfer_half_tile_nearest(const float4 *SK, const float4 *queries, int task)
+{
+    const float4 q = queries[task & 127];
+    const unsigned at = (unsigned)((task >> 8) * 32 + (task >> 7 & 1) * 4 + (int)(threadIdx.x & 3)) * 16u;
+    const char *base = reinterpret_cast<const char *>(SK);
+    double best = 0.0;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const float4 f = *reinterpret_cast<const float4 *>(base + at + r * 128u);
+        const float dd = tk_dist2<float>(f.x, f.y, f.z, q.x, q.y, q.z);
+        const double word = __builtin_bit_cast(double, (unsigned long long)__builtin_bit_cast(unsigned, dd) << 32 |
+                                                           __builtin_bit_cast(unsigned, f.w));
+        best = r == 0 ? word : tk_min_f64(best, word);
+    }
+    best = tk_min_f64(best, quad_move<0xb1>(best));
+    return tk_min_f64(best, quad_move<0x4e>(best));
+}
+
 struct ChamferPrunedArgs {
     const float4 *sorted[2];
     const uint4 *terms[2];
@@ -3218,8 +3248,10 @@ __device__ __attribute__((noinline)) bool chamfer_most_tiles_within_reach(
 // (Launched one wave per workgroup - waves share nothing, and a finished wave frees its
 // slot at once: 2-3 % over four waves per workgroup. The bound of 256 lanes only caps the
 // registers at four waves per SIMD.)
+// (Eight rounds of boxes: 96 registers and five waves to a SIMD; with 109 and four, 102 us for 95 on the sphere
+// above, with six waves and values in scratch 105.)
 template <int NQB, int RMAX, bool COUNT = false>
-__global__ __launch_bounds__(256) void chamfer_pruned_kernel(ChamferPrunedArgs a)
+__global__ __launch_bounds__(256, RMAX == 8 ? 5 : 1) void chamfer_pruned_kernel(ChamferPrunedArgs a)
 {
     const int tid = threadIdx.x;
     const int lane = tid & (TK_WAVE - 1);
@@ -3471,7 +3503,7 @@ __global__ __launch_bounds__(256) void chamfer_pruned_kernel(ChamferPrunedArgs a
             id0[g] = lt0 ? t : id0[g];
             v2[g] = __builtin_amdgcn_fmed3f(v1[g], v2[g], x);
             v1[g] = __builtin_amdgcn_fmed3f(v0[g], v1[g], x);
-            v0[g] = __builtin_amdgcn_fmed3f(-INF, v0[g], x);
+            v0[g] = tk_min_f32(v0[g], x);
         }
     };
     unsigned swept = 0;  // bit r: tile r * 64 + lane has been swept
@@ -3532,18 +3564,18 @@ __global__ __launch_bounds__(256) void chamfer_pruned_kernel(ChamferPrunedArgs a
 #pragma unroll 1
         for (int r = 0; r < rounds; ++r) {
             unsigned long long m = __builtin_amdgcn_ballot_w64(((takes >> r) & 1u) != 0);
-            while (m != 0) {  // four tiles in flight at a time
+            // Four tiles in flight at a time, the first again where there are fewer: with loads that depend on how many
+            // there are, the first product waited for the last of them (clusters 212 -> 206 us).
+            while (m != 0) {
                 int t[4];
                 uint4 ka[4];
 #pragma unroll
                 for (int u = 0; u < 4; ++u) {
-                    t[u] = -1;
-                    if (m != 0) {
-                        t[u] = r * TK_WAVE + (int)__builtin_ctzll(m);
-                        m &= m - 1;
-                        ka[u] = TK[(int64_t)t[u] * 64 + lane];
-                    }
+                    t[u] = m != 0 ? r * TK_WAVE + (int)__builtin_ctzll(m) : -1;
+                    m &= m - 1;
+                    ka[u] = TK[(int64_t)(t[u] < 0 ? t[0] : t[u]) * 64 + lane];
                 }
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int u = 0; u < 4; ++u) {
                     if (t[u] >= 0) {
@@ -3561,57 +3593,81 @@ __global__ __launch_bounds__(256) void chamfer_pruned_kernel(ChamferPrunedArgs a
             atomicAdd(a.counters + 1, 1ull);
         }
     }
-    // ---- exact evaluation of each half's candidate tiles, then the merge ----
+    // ---- exact evaluation of each half's candidate tiles ----
+    // Of a query's halves mostly one has a candidate, and a second one is rare: 64 queries have 70 half tiles to
+    // look at, of 256 that they could have. They are listed and dealt out to the quads. (A lane with its own half's
+    // candidates, one after the other, spent 660 of a wave's 2050 instructions here: forward, 32 x 16384 points on a
+    // sphere both ways 109 -> 102 us.)
+    static_assert(NQB <= 4, "seven bits for a query");
+    __shared__ float4 s_query[32 * NQB];
+    __shared__ unsigned long long s_best[32 * NQB];
+    __shared__ int s_task[128 * NQB];  // tile << 8 | half << 7 | query
     unsigned over_mask[NQB], stray_mask[NQB];
-    int nover = 0;
+    bool evaluates[NQB];
+    int nover = 0, ntasks = 0;
 #pragma unroll
     for (int g = 0; g < NQB; ++g) {
-        const bool ok = live[g];
         stray_mask[g] = (unsigned)__builtin_amdgcn_ballot_w64(stray[g] && half == 0);
         const float best_score = __builtin_fminf(v0[g], __shfl_xor(v0[g], 32));
         const float r = kmax + qnorm[g];
         const float thr = best_score + (r * r * 7.6293945e-06f + guard);  // 2^-17 R
         const bool crowded = v2[g] <= thr;  // three or more candidate tiles in this half
         const bool over =
-            ok && ((__builtin_amdgcn_ballot_w64(crowded) >> col & 0x100000001ull) != 0);
+            live[g] && ((__builtin_amdgcn_ballot_w64(crowded) >> col & 0x100000001ull) != 0);
+        evaluates[g] = live[g] && !over;
+        over_mask[g] = (unsigned)__builtin_amdgcn_ballot_w64(over && half == 0);
+        nover += __builtin_popcount(over_mask[g]);
+        const int query = g * 32 + col;
+        if (half == 0) {
+            s_query[query] = make_float4(rx[g], ry[g], rz[g], 0.0f);
+            s_best[query] = (0x7f800000ull << 32) | 0xffffffffull;
+        }
+#pragma unroll
+        for (int pass = 0; pass < 2; ++pass) {
+            const int tile = pass == 0 ? id0[g] : id1[g];
+            const bool takes = evaluates[g] && (pass == 0 ? v0[g] : v1[g]) <= thr && tile >= 0;
+            const unsigned long long mask = __builtin_amdgcn_ballot_w64(takes);
+            const int at = ntasks + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32),
+                                                                  __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0));
+            if (takes)
+                s_task[at] = tile << 8 | half << 7 | query;
+            ntasks += __builtin_popcountll(mask);
+        }
+    }
+    __syncthreads();  // (of one wave)
+    const auto look = [&](int first, auto quads) {  // (a task too many is the last one again)
+        constexpr int N = decltype(quads)::value;
+        int task[N];
+        double word[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const int at = first + i * 16 + (lane >> 2);
+            task[i] = s_task[at < ntasks ? at : ntasks - 1];
+        }
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+            word[i] = chamfer_half_tile_nearest(SK, s_query, task[i]);
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+            if ((lane & 3) == 0)
+                atomicMin(&s_best[task[i] & 127], __builtin_bit_cast(unsigned long long, word[i]));
+    };
+    int done = 0;
+    for (; ntasks - done > 16; done += 64)
+        look(done, std::integral_constant<int, 4>());
+    for (; done < ntasks; done += 16)
+        look(done, std::integral_constant<int, 1>());
+    __syncthreads();
+#pragma unroll
+    for (int g = 0; g < NQB; ++g) {
         float bestd = INF;
         int bestj = -1;
-        // (distance bits << 32 | original index): distances are non-negative, so the words
-        // order as (distance, index) pairs; a NaN (padding) is above +inf and never taken
-        unsigned long long best = (0x7f800000ull << 32) | 0xffffffffull;
-        if (ok && !over) {
-            const int ta = v0[g] <= thr ? id0[g] : -1, tb = v1[g] <= thr ? id1[g] : -1;
-#pragma unroll
-            for (int pass = 0; pass < 2; ++pass) {
-                const int tile = pass == 0 ? ta : tb;
-                if (tile < 0)
-                    continue;
-                // this half's keys of the tile: runs of 4 keys, 8 keys apart
-                const float4 *p = SK + (int64_t)tile * 32 + half * 4;
-                float4 f[16];
-#pragma unroll
-                for (int e = 0; e < 16; ++e)
-                    f[e] = p[(e >> 2) * 8 + (e & 3)];
-#pragma unroll
-                for (int e = 0; e < 16; ++e) {
-                    const float dd = tk_dist2<float>(f[e].x, f[e].y, f[e].z, rx[g], ry[g], rz[g]);
-                    const unsigned long long word =
-                        ((unsigned long long)__builtin_bit_cast(unsigned, dd) << 32) |
-                        __builtin_bit_cast(unsigned, f[e].w);
-                    best = word < best ? word : best;
-                }
-            }
+        if (evaluates[g]) {
+            const unsigned long long best = s_best[g * 32 + col];
             // (a distance that overflowed is no match: strict '<' from +inf)
             const float d = __builtin_bit_cast(float, (unsigned)(best >> 32));
             bestd = d < INF ? d : INF;
             bestj = d < INF ? (int)(unsigned)best : -1;
-        }
-        // the other half's result: smaller distance, then lower key index
-        const float od = __shfl_xor(bestd, 32);
-        const int oj = __shfl_xor(bestj, 32);
-        if (oj >= 0 && (bestj < 0 || od < bestd || (od == bestd && oj < bestj))) {
-            bestd = od;
-            bestj = oj;
         }
         for (int e = 0; e < nfar; ++e) {  // (uniform; usually none)
             const float4 f = FK[e];
@@ -3622,13 +3678,11 @@ __global__ __launch_bounds__(256) void chamfer_pruned_kernel(ChamferPrunedArgs a
                 bestj = fj;
             }
         }
-        if (half == 0 && ok && !over) {
+        if (half == 0 && evaluates[g]) {
             const int64_t o = (int64_t)b * nq + qid[g];
             a.dist[which][o] = bestd;
             a.idx[which][o] = (int64_t)bestj;
         }
-        over_mask[g] = (unsigned)__builtin_amdgcn_ballot_w64(over && half == 0);
-        nover += __builtin_popcount(over_mask[g]);
     }
     if (nover == 0 && nstray == 0)
         return;

@@ -402,13 +402,7 @@ template <int KMAX> struct KnnSlot {
     }
 };
 
-// (the builtins quiet their operands first, an instruction each)
-__device__ __forceinline__ double knn_min_f64(double a, double b)
-{
-    double o;
-    asm("v_min_f64 %0, %1, %2" : "=v"(o) : "v"(a), "v"(b));
-    return o;
-}
+// (written out as tk_min_f64 is)
 __device__ __forceinline__ double knn_min_f64_uniform(double a, double b)  // b wave-uniform
 {
     double o;
@@ -670,7 +664,7 @@ __global__ __launch_bounds__(LANES) void knn_filter_kernel_f32(
                                         ((unsigned)(KMAX - 1 - s) << Slot::KEY_BITS) | (unsigned)s);
 #pragma unroll
             for (int p = s; p >= 1; --p)
-                v[p] = knn_max_f64(v[p], knn_min_f64(v[p - 1], x));
+                v[p] = knn_max_f64(v[p], tk_min_f64(v[p - 1], x));
             v[0] = knn_max_f64(v[0], x);
         }
     }
@@ -713,8 +707,8 @@ __global__ __launch_bounds__(LANES) void knn_filter_kernel_f32(
         const double x = Slot::pack(ins ? dbits : 0x7fe00000, low | flag);
 #pragma unroll
         for (int p = 0; p < KMAX - 1; ++p)
-            v[p] = knn_max_f64(v[p + 1], knn_min_f64(v[p], x));
-        v[KMAX - 1] = knn_min_f64(v[KMAX - 1], x);
+            v[p] = knn_max_f64(v[p + 1], tk_min_f64(v[p], x));
+        v[KMAX - 1] = tk_min_f64(v[KMAX - 1], x);
         max_key = ins ? __builtin_bit_cast(float, Slot::distance(v[0])) : max_key;
         // Keep the loop-carried state where it is: without this the register allocator
         // rotates some forty values through copies on every step.

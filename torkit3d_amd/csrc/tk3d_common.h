@@ -135,6 +135,20 @@ template <auto Kernel> static inline int tk_allow_dynamic_lds(int bytes)
     return TK3D_OK;
 }
 
+// Minima without the instruction by which the builtins quiet each operand first.
+__device__ __forceinline__ float tk_min_f32(float a, float b)
+{
+    float o;
+    asm("v_min_f32 %0, %1, %2" : "=v"(o) : "v"(a), "v"(b));
+    return o;
+}
+__device__ __forceinline__ double tk_min_f64(double a, double b)
+{
+    double o;
+    asm("v_min_f64 %0, %1, %2" : "=v"(o) : "v"(a), "v"(b));
+    return o;
+}
+
 // The maxima over the wave (LANES 64, left in lane 63) or over each half of it (32, in lanes 31 and 63) of six values
 // at once: the steps of one value are the wait between those of another, and a maximum takes its operand from the
 // other lane itself. One by one, through moves, the compiler makes it five instructions a step.
