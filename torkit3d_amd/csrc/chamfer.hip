@@ -1083,7 +1083,7 @@ __device__ __forceinline__ void chamfer_mfma_block(const ChamferDir<float> &d, c
         const int slot = (wave * NQB + g) * 32 + col;
         const int qi = qblock * QB + slot;
         const bool ok = qi < nq;
-        const float best_score = __builtin_fminf(v0[g], __shfl_xor(v0[g], 32));
+        const float best_score = tk_min_of_halves(v0[g]);
         const float r = kmax + qnorm[g];
         const float thr = best_score + (r * r * 7.6293945e-06f + guard);  // 2^-17 R
         const bool filtered = qnorm[g] <= 16000.0f;  // false for NaN / inf / out of range
@@ -2846,7 +2846,7 @@ __global__ __launch_bounds__(1024) void chamfer_prepare_kernel(ChamferSortArgs a
                                         // once do not fit the registers)
     float lo[3] = {INF, INF, INF}, hi[3] = {-INF, -INF, -INF};
     float dev[3] = {0.0f, 0.0f, 0.0f};
-    bool bad = false;
+    float zero = 0.0f;
     // (the table of Hilbert positions comes along, into the LDS that the windows use later:
     // looked up in global memory, one cache line per lane, the look-ups took 8 us)
     unsigned short *const cell_of = reinterpret_cast<unsigned short *>(win);
@@ -2865,7 +2865,7 @@ __global__ __launch_bounds__(1024) void chamfer_prepare_kernel(ChamferSortArgs a
             const bool counts = u * NT + tid < n;
 #pragma unroll
             for (int ax = 0; ax < 3; ++ax) {
-                bad |= !(v[ax] - v[ax] == 0.0f);
+                zero = __builtin_fmaf(v[ax], 0.0f, zero);  // (NaN once one is not finite)
                 lo[ax] = __builtin_fminf(lo[ax], v[ax]);
                 hi[ax] = __builtin_fmaxf(hi[ax], v[ax]);
                 dev[ax] += counts ? __builtin_fminf(__builtin_fabsf(v[ax] - pilot[ax]), cap[ax]) : 0.0f;
@@ -2896,7 +2896,7 @@ __global__ __launch_bounds__(1024) void chamfer_prepare_kernel(ChamferSortArgs a
             sdev[wave][ax] = dev[ax];
         }
     }
-    if (bad)
+    if (!(zero == 0.0f))
         sbad = 1;
     __syncthreads();
     float cc[3], flo[3], ext;
@@ -3513,7 +3513,7 @@ __global__ __launch_bounds__(256, RMAX == 8 ? 5 : 1) void chamfer_pruned_kernel(
         float ub = -INF;
 #pragma unroll
         for (int g = 0; g < NQB; ++g) {
-            const float best = __builtin_fminf(v0[g], __shfl_xor(v0[g], 32));
+            const float best = tk_min_of_halves(v0[g]);
             ub = live[g] ? __builtin_fmaxf(ub, best + qn2[g]) : ub;
         }
         return wave_reduce_max(ub);
@@ -3608,7 +3608,7 @@ __global__ __launch_bounds__(256, RMAX == 8 ? 5 : 1) void chamfer_pruned_kernel(
 #pragma unroll
     for (int g = 0; g < NQB; ++g) {
         stray_mask[g] = (unsigned)__builtin_amdgcn_ballot_w64(stray[g] && half == 0);
-        const float best_score = __builtin_fminf(v0[g], __shfl_xor(v0[g], 32));
+        const float best_score = tk_min_of_halves(v0[g]);
         const float r = kmax + qnorm[g];
         const float thr = best_score + (r * r * 7.6293945e-06f + guard);  // 2^-17 R
         const bool crowded = v2[g] <= thr;  // three or more candidate tiles in this half

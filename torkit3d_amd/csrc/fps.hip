@@ -695,7 +695,7 @@ __device__ __forceinline__ void fps_band(const float *__restrict__ pts, int64_t 
     const float p0[3] = {fps_coord<SOA>(pts, L.n, 0, 0), fps_coord<SOA>(pts, L.n, 0, 1),
                          fps_coord<SOA>(pts, L.n, 0, 2)};
     float far = 0.0f;
-    bool odd = false;
+    float zero = 0.0f;
     float own[3][P];  // point tid + k * NT (beyond the cloud: its last point), read coalesced
 #pragma unroll
     for (int k = 0; k < P; ++k) {
@@ -710,13 +710,13 @@ __device__ __forceinline__ void fps_band(const float *__restrict__ pts, int64_t 
         for (int a = 0; a < 3; ++a) {
             lo[a] = __builtin_fminf(lo[a], own[a][k]);
             hi[a] = __builtin_fmaxf(hi[a], own[a][k]);
-            odd |= !(own[a][k] - own[a][k] == 0.0f);
+            zero = __builtin_fmaf(own[a][k], 0.0f, zero);  // (NaN once one is not finite)
         }
         far = __builtin_fmaxf(far, tk_dist2<float>(own[0][k], own[1][k], own[2][k], p0[0], p0[1],
                                                    p0[2]));
     }
     far = wave_max<float>(far);
-    odd = __builtin_amdgcn_ballot_w64(odd) != 0ull;
+    const bool odd = __builtin_amdgcn_ballot_w64(!(zero == 0.0f)) != 0ull;
     float ends[6] = {-lo[0], -lo[1], -lo[2], hi[0], hi[1], hi[2]};
     tk_wave_max_six<64>(ends);
     if (lane == TK_WAVE - 1) {

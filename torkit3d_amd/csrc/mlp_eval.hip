@@ -195,7 +195,8 @@ __global__ void __launch_bounds__(NW *TK_WAVE, 4) mlp_grouped_pool_kernel(Groupe
 #pragma unroll
                 for (int i = 0; i < 16; ++i)
                     best[t] = __builtin_elementwise_maximum(best[t], normalised(sums[t][i], k));
-                best[t] = __builtin_elementwise_maximum(best[t], __shfl_xor(best[t], 32));
+                const float2 halves = tk_both_halves(best[t]);
+                best[t] = __builtin_elementwise_maximum(halves.x, halves.y);
             }
             float *out = p.out + ((int64_t)b * C3 + cbase + c) * p.M;
             const int group = base / p.S;

@@ -149,6 +149,20 @@ __device__ __forceinline__ double tk_min_f64(double a, double b)
     return o;
 }
 
+// The values of the two lanes 32 apart, the lower one's first.
+__device__ __forceinline__ float2 tk_both_halves(float v)
+{
+    const unsigned bits = __builtin_bit_cast(unsigned, v);
+    const auto r = __builtin_amdgcn_permlane32_swap(bits, bits, false, false);
+    const unsigned lower = r[0], upper = r[1];  // (a bit_cast applied to r[1] itself reads element 0)
+    return make_float2(__builtin_bit_cast(float, lower), __builtin_bit_cast(float, upper));
+}
+__device__ __forceinline__ float tk_min_of_halves(float v)
+{
+    const float2 b = tk_both_halves(v);
+    return tk_min_f32(b.x, b.y);
+}
+
 // The maxima over the wave (LANES 64, left in lane 63) or over each half of it (32, in lanes 31 and 63) of six values
 // at once: the steps of one value are the wait between those of another, and a maximum takes its operand from the
 // other lane itself. One by one, through moves, the compiler makes it five instructions a step.
