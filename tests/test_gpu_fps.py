@@ -220,9 +220,9 @@ def test_points_at_infinity(cuda):
     np.testing.assert_array_equal(run(pts, 30, cuda), want)
 
 
-# ---- 513 to 16384 points, 256 samples or more: the kernel that lays the points out by region
-# (Morton order), skips the blocks a new centre cannot reach and accepts from a candidate per
-# lane's blocks. The lane order is no longer the reference's priority order there, so ties are
+# ---- up to 16384 points, 192 samples or more: the kernel that lays the points out by region
+# (along a Hilbert curve), skips the blocks a new centre cannot reach and takes its winners from the points of
+# a band below the largest minimum. The lane order is not the reference's priority order there, so ties are
 # resolved explicitly. ----
 
 def _region_cloud(kind, g, b, n):
