@@ -153,6 +153,15 @@ int tk3d_mlp_batch_pool_f32(const float *y, const tk3d_mlp_batch_norm *norm, int
 int tk3d_mlp_batch_rows_f32(const float *y, const float *z, const tk3d_mlp_batch_norm *norm, int B, int C, int P,
                             float *out, float *extreme, int32_t *arg, int64_t *index, void *stream);
 
+/* The three with one added to *count, the norm's count of batches (NULL: none). */
+int tk3d_mlp_batch_relu_counted_f32(const float *y, const tk3d_mlp_batch_norm *norm, int64_t *count, float *z,
+                                    void *stream);
+int tk3d_mlp_batch_pool_counted_f32(const float *y, const tk3d_mlp_batch_norm *norm, int64_t *count, int size,
+                                    float *out, float *extreme, unsigned char *arg, void *stream);
+int tk3d_mlp_batch_rows_counted_f32(const float *y, const float *z, const tk3d_mlp_batch_norm *norm, int64_t *count,
+                                    int B, int C, int P, float *out, float *extreme, int32_t *arg, int64_t *index,
+                                    void *stream);
+
 /* A normalised layer's ReLU and maximum over groups of `size` <= 255 consecutive values: out =
  * relu(max z), arg the place of the maximum and extreme the y at that place, [groups] each. */
 int tk3d_mlp_pool_max_f32(const float *z, const float *y, int64_t groups, int size, float *out,

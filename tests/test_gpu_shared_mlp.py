@@ -489,6 +489,26 @@ def test_batch_norm_is_the_librarys_bit_by_bit(cuda, b, c, m, size):
         assert lib.tk3d_mlp_batch_norm_supported(*(ctypes.c_int64(v) for v in shape)) == 0
 
 
+@pytest.mark.parametrize("form", ["relu", "pool", "rows"])
+def test_batches_are_counted(cuda, form):
+    # by the pass that normalises, once a call and layer; where the count is not beside the values, or no int64, as before
+    mlp = make(mlp2d_bn_relu if form == "pool" else mlp1d_bn_relu, 16, (32, 64, 32), True, cuda)
+    norms = [m for m in mlp.modules() if isinstance(m, (nn.BatchNorm1d, nn.BatchNorm2d))]
+    norms[0]._buffers["num_batches_tracked"] = torch.tensor(3)
+    norms[1]._buffers["num_batches_tracked"] = torch.tensor(5, dtype=torch.int32, device=cuda)
+    x = randn(4, 4, 16, 64, 32) if form == "pool" else randn(4, 4, 16, 2048)
+    versions = [m.num_batches_tracked._version for m in norms]
+    for call in (1, 2):
+        if form == "pool":
+            mlp.forward_max(x.requires_grad_())
+        elif form == "rows":
+            mlp.forward_points_max(x.requires_grad_())
+        else:
+            mlp(x.requires_grad_())
+        assert [int(m.num_batches_tracked) for m in norms] == [3 + call, 5 + call, call]
+        assert [m.num_batches_tracked._version for m in norms] == [v + call for v in versions]
+
+
 @pytest.mark.parametrize("size", [20, 32, 64])
 def test_a_maximum_is_the_first_of_equals(cuda, size):
     # quantised values (and their order is that of their norm: ascending or, with gamma < 0, descending), a

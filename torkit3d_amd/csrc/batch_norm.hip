@@ -110,11 +110,20 @@ __device__ __forceinline__ f32x4 batch_constants(const tk3d_mlp_batch_norm &n, i
     return f32x4{mean, inv_std, n.gamma[c], n.beta[c]};
 }
 
+// The batch norm's count of batches, where the caller has one. (A launch of its own for the layers of a chain took 3
+// to 4 us.)
+__device__ __forceinline__ void count_batch(int64_t *count)
+{
+    if (count && blockIdx.x == 0 && threadIdx.x == 0)
+        *count += 1;
+}
+
 // z = relu(norm(y)), a stretch of a row per workgroup.
 __global__ void __launch_bounds__(kBlock) batch_relu_kernel(const float *__restrict__ y,
-                                                            tk3d_mlp_batch_norm n,
+                                                            tk3d_mlp_batch_norm n, int64_t *count,
                                                             float *__restrict__ z, int stretches)
 {
+    count_batch(count);
     const int part = blockIdx.x % stretches, row = blockIdx.x / stretches, c = row % n.C;
     const f32x4 k = batch_constants(n, c, row < n.C && part == 0 && threadIdx.x == 0);
     const int64_t base = (int64_t)row * n.P;
@@ -184,8 +193,9 @@ __global__ void __launch_bounds__(kBlock) batch_pool_kernel(const float *__restr
                                                             float *__restrict__ out,
                                                             float *__restrict__ extreme,
                                                             unsigned char *__restrict__ arg,
-                                                            int stretches)
+                                                            int stretches, int64_t *count)
 {
+    count_batch(count);
     constexpr int NONE = 0x7fffffff;
     const int part = blockIdx.x % stretches, row = blockIdx.x / stretches, c = row % n.C;
     const f32x4 k = batch_constants(n, c, row < n.C && part == 0 && threadIdx.x == 0);
@@ -270,8 +280,9 @@ template <bool Z>
 __global__ void __launch_bounds__(kBlock)
     batch_rows_kernel(const float *__restrict__ y, const float *__restrict__ z, tk3d_mlp_batch_norm n, int rows, int C,
                       int P, float *__restrict__ out, float *__restrict__ extreme, int *__restrict__ arg,
-                      int64_t *__restrict__ index)
+                      int64_t *__restrict__ index, int64_t *count)
 {
+    count_batch(count);
     const int row = blockIdx.x * kWaves + threadIdx.x / TK_WAVE, lane = threadIdx.x % TK_WAVE;
     if (row >= rows)
         return;
@@ -359,18 +370,30 @@ int tk3d_mlp_batch_sums_f32(const float *y, int B, int C, int P, void *partial, 
 
 int tk3d_mlp_batch_relu_f32(const float *y, const tk3d_mlp_batch_norm *norm, float *z, void *stream)
 {
+    return tk3d_mlp_batch_relu_counted_f32(y, norm, nullptr, z, stream);
+}
+
+int tk3d_mlp_batch_relu_counted_f32(const float *y, const tk3d_mlp_batch_norm *norm, int64_t *count, float *z,
+                                    void *stream)
+{
     if (!tk3d_mlp_batch_norm_supported(norm->B, norm->C, norm->P) ||
         (((uintptr_t)y | (uintptr_t)z) & 15) != 0)
         return TK3D_ERR_UNSUPPORTED;
     const int64_t rows = (int64_t)norm->B * norm->C;
     const int stretches = stretches_of(rows, norm->P);
-    batch_relu_kernel<<<(unsigned)(rows * stretches), kBlock, 0, (hipStream_t)stream>>>(y, *norm, z,
-                                                                                      stretches);
+    batch_relu_kernel<<<(unsigned)(rows * stretches), kBlock, 0, (hipStream_t)stream>>>(
+        y, *norm, count, z, stretches);
     return tk_launch_status();
 }
 
 int tk3d_mlp_batch_pool_f32(const float *y, const tk3d_mlp_batch_norm *norm, int size, float *out,
-                            float *extreme, unsigned char *arg, void *stream_)
+                            float *extreme, unsigned char *arg, void *stream)
+{
+    return tk3d_mlp_batch_pool_counted_f32(y, norm, nullptr, size, out, extreme, arg, stream);
+}
+
+int tk3d_mlp_batch_pool_counted_f32(const float *y, const tk3d_mlp_batch_norm *norm, int64_t *count, int size,
+                                    float *out, float *extreme, unsigned char *arg, void *stream_)
 {
     if (!tk3d_mlp_batch_norm_supported(norm->B, norm->C, norm->P) || ((uintptr_t)y & 15) != 0)
         return TK3D_ERR_UNSUPPORTED;
@@ -381,16 +404,23 @@ int tk3d_mlp_batch_pool_f32(const float *y, const tk3d_mlp_batch_norm *norm, int
     const unsigned grid = (unsigned)(rows * stretches);
     const hipStream_t stream = (hipStream_t)stream_;
     if (size == 32)
-        batch_pool_kernel<8><<<grid, kBlock, 0, stream>>>(y, *norm, size, out, extreme, arg, stretches);
+        batch_pool_kernel<8><<<grid, kBlock, 0, stream>>>(y, *norm, size, out, extreme, arg, stretches, count);
     else if (size == 64)
-        batch_pool_kernel<16><<<grid, kBlock, 0, stream>>>(y, *norm, size, out, extreme, arg, stretches);
+        batch_pool_kernel<16><<<grid, kBlock, 0, stream>>>(y, *norm, size, out, extreme, arg, stretches, count);
     else
-        batch_pool_kernel<0><<<grid, kBlock, 0, stream>>>(y, *norm, size, out, extreme, arg, stretches);
+        batch_pool_kernel<0><<<grid, kBlock, 0, stream>>>(y, *norm, size, out, extreme, arg, stretches, count);
     return tk_launch_status();
 }
 
 int tk3d_mlp_batch_rows_f32(const float *y, const float *z, const tk3d_mlp_batch_norm *norm, int B, int C, int P,
-                            float *out, float *extreme, int32_t *arg, int64_t *index, void *stream_)
+                            float *out, float *extreme, int32_t *arg, int64_t *index, void *stream)
+{
+    return tk3d_mlp_batch_rows_counted_f32(y, z, norm, nullptr, B, C, P, out, extreme, arg, index, stream);
+}
+
+int tk3d_mlp_batch_rows_counted_f32(const float *y, const float *z, const tk3d_mlp_batch_norm *norm, int64_t *count,
+                                    int B, int C, int P, float *out, float *extreme, int32_t *arg, int64_t *index,
+                                    void *stream_)
 {
     if (B <= 0 || C <= 0 || P <= 0)
         return TK3D_ERR_BAD_SIZE;
@@ -401,9 +431,10 @@ int tk3d_mlp_batch_rows_f32(const float *y, const float *z, const tk3d_mlp_batch
     const hipStream_t stream = (hipStream_t)stream_;
     if (z)
         batch_rows_kernel<true><<<grid, kBlock, 0, stream>>>(y, z, tk3d_mlp_batch_norm{}, rows, C, P, out, extreme, arg,
-                                                            index);
+                                                            index, count);
     else if (tk3d_mlp_batch_norm_supported(norm->B, norm->C, norm->P))
-        batch_rows_kernel<false><<<grid, kBlock, 0, stream>>>(y, z, *norm, rows, C, P, out, extreme, arg, index);
+        batch_rows_kernel<false><<<grid, kBlock, 0, stream>>>(y, z, *norm, rows, C, P, out, extreme, arg, index,
+                                                             count);
     else
         return TK3D_ERR_UNSUPPORTED;
     return tk_launch_status();

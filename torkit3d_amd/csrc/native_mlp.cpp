@@ -258,6 +258,19 @@ struct Normalised {
     Tensor z;                 // the library's, where it took the batch norm
     tk3d_mlp_batch_norm norm{};  // else what the pass over y needs
     Tensor partial;
+    int64_t *count = nullptr;    // the norm's count of batches, if that pass counts
+
+    // Whether the pass over y takes the count along: a single int64 beside y. (Its version goes up
+    // as with an addition in place.)
+    bool counts(const Tensor &batches)
+    {
+        if (z.defined() || batches.device() != y.device() || batches.scalar_type() != at::kLong ||
+            batches.numel() != 1)
+            return false;
+        batches.unsafeGetTensorImpl()->bump_version();
+        count = batches.data_ptr<int64_t>();
+        return true;
+    }
 };
 
 Normalised stock_layer(const Tensor &h, const Tensor &weight, const Tensor &gamma, const Tensor &beta,
@@ -290,7 +303,8 @@ Tensor activate(const Normalised &n)
     if (n.z.defined())
         return Tensor(n.z).relu_();
     const Tensor z = at::empty_like(n.y);
-    done(tk3d_mlp_batch_relu_f32(f32(n.y), &n.norm, f32(z), stream_of(z)), "tk3d_mlp_batch_relu_f32");
+    done(tk3d_mlp_batch_relu_counted_f32(f32(n.y), &n.norm, n.count, f32(z), stream_of(z)),
+         "tk3d_mlp_batch_relu_f32");
     return z;
 }
 
@@ -308,8 +322,8 @@ Tensor pool_max(const Normalised &n, Tensor &extreme, Tensor &arg)
                                    arg.data_ptr<uint8_t>(), stream_of(y)),
              "tk3d_mlp_pool_max_f32");
     } else {
-        done(tk3d_mlp_batch_pool_f32(f32(y), &n.norm, (int)y.size(3), f32(out), f32(extreme),
-                                     arg.data_ptr<uint8_t>(), stream_of(y)),
+        done(tk3d_mlp_batch_pool_counted_f32(f32(y), &n.norm, n.count, (int)y.size(3), f32(out), f32(extreme),
+                                             arg.data_ptr<uint8_t>(), stream_of(y)),
              "tk3d_mlp_batch_pool_f32");
     }
     return out;
@@ -324,8 +338,9 @@ Tensor row_max(const Normalised &n, Tensor &extreme, Tensor &arg, Tensor &index)
     extreme = at::empty({B, C}, y.options());
     arg = at::empty({B, C}, y.options().dtype(at::kInt));
     index = at::empty({B, C}, y.options().dtype(at::kLong));
-    done(tk3d_mlp_batch_rows_f32(f32(y), f32(z), &n.norm, (int)B, (int)C, (int)P, f32(out), f32(extreme),
-                                 arg.data_ptr<int32_t>(), index.data_ptr<int64_t>(), stream_of(y)),
+    done(tk3d_mlp_batch_rows_counted_f32(f32(y), f32(z), &n.norm, n.count, (int)B, (int)C, (int)P, f32(out),
+                                         f32(extreme), arg.data_ptr<int32_t>(), index.data_ptr<int64_t>(),
+                                         stream_of(y)),
          "tk3d_mlp_batch_rows_f32");
     return out;
 }
@@ -352,10 +367,12 @@ Tensor forward_training(const Call &c, Kept &k, Tensor &index)
     } else if (c.params[0].dim() == 4) {
         h = h.view({B, h.size(1), c.rows, -1});
     }
-    std::vector<Tensor> counts;  // (one launch for all layers)
+    std::vector<Tensor> counts;  // of the layers whose own passes don't count (one launch for all of them)
     for (int64_t l = 0; l < L; ++l) {
         const Tensor *w = &c.params[3 * l], *s = &c.buffers[3 * l];
-        const Normalised n = stock_layer(h, w[0], w[1], w[2], s[0], s[1], c.momentum[l], c.eps[l]);
+        Normalised n = stock_layer(h, w[0], w[1], w[2], s[0], s[1], c.momentum[l], c.eps[l]);
+        if (s[2].defined() && !n.counts(s[2]))
+            counts.push_back(s[2]);
         k.mean.push_back(n.mean);
         k.var.push_back(n.inv_std);
         if (c.pool && l == L - 1) {
@@ -366,8 +383,6 @@ Tensor forward_training(const Call &c, Kept &k, Tensor &index)
             h = activate(n);
             k.y.push_back(n.y.flatten(2).contiguous());
         }
-        if (s[2].defined())
-            counts.push_back(s[2]);
     }
     if (!counts.empty())
         at::_foreach_add_(counts, 1);
@@ -871,9 +886,9 @@ Tensor edge_forward(const EdgeCall &c, EdgeKept &k)
         done(tk3d_mlp_edge_features_f32(f32(c.x), c.index.data_ptr<int64_t>(), (int)B, (int)C, (int)N,
                                         (int)K, f32(edges), stream),
              "tk3d_mlp_edge_features_f32");
-        const Normalised n = stock_layer(edges, c.weight, c.gamma, c.beta, c.running_mean,
-                                         c.running_var, c.momentum, c.eps);
-        if (c.batches.defined())
+        Normalised n = stock_layer(edges, c.weight, c.gamma, c.beta, c.running_mean, c.running_var, c.momentum,
+                                   c.eps);
+        if (c.batches.defined() && !n.counts(c.batches))
             Tensor(c.batches).add_(1);
         k.mean = n.mean;
         k.var = n.inv_std;
