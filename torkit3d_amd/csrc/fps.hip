@@ -630,8 +630,9 @@ __device__ __forceinline__ int fps_band(int was, float target, int n)
 //
 // What bounds it: one workgroup has one compute unit, and an exchange is a chain of short phases (clocks
 // at 16 x 4096 -> 1024, 16 waves, of 6700 for 19 winners, of which shorter chains of instructions have since
-// taken 250: listing 1100, judgement 1700, resolving and turns 800, update 1540 on average and 2050 in the slowest wave, with the boxes; the rest is waiting at the
-// barriers, and 14 of 67 bands are listed again). Measured (us; before: a candidate per group; both
+// taken 250: listing 1100, judgement 1700, resolving and turns 800, update 1540 on average and 2050 in
+// the slowest wave, with the boxes; the rest is waiting at the barriers, and 14 of 67 bands are listed
+// again). Measured (us; before: a candidate per group; both
 // with what runs behind them): 8 x 16384 -> 4096 1390-1450 -> 545, on a noisy sphere 1120-1200 -> 520,
 // in clusters 1180-1330 -> 695; 16 x 8192 -> 2048 590 -> 275; 16 x 4096 -> 1024 285 -> 150; 16 x 2048 -> 512
 // 160 -> 94; 1 x 1024 -> 512 120 -> 69; on lattices, copies and a line 0.2 to 0.9 of the time before.
@@ -1604,7 +1605,8 @@ int fps_band_launch_f32(const float *points, bool soa, int64_t B, int64_t *index
 // early in a sampling, where the points far from all centres are neighbours, a band of 64 holds one or
 // two winners. Multi-step kernel against this one, with what runs behind them, us, at 128 samples (this
 // one 2 to 20 us slower than now): 1 x 300 42, 35; 16 x 600 48, 55; 16 x 1024 50, 59; 16 x 4096 77, 83; 16 x 16384
-// 159, 161; at 192: 65, 43; 67, 47; 69, 54; 104, 82; 222, 153. In sampling order, in which an encoder's levels come, it has 16 for
+// 159, 161; at 192: 65, 43; 67, 47; 69, 54; 104, 82; 222, 153. In sampling order, in which an encoder's
+// levels come, it has 16 for
 // 46 to 210 at 192 samples.
 bool fps_band_dispatch_f32(const float *points, bool soa, int64_t B, int64_t *index, float *sampled,
                              const FpsLayout &L, int64_t npos, hipStream_t s, int &rc)
