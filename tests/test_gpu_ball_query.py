@@ -87,3 +87,26 @@ def test_edge_cases(cuda):
     out = _C.ball_query_cuda(query.to(cuda), torch.zeros(2, 0, 3, device=cuda), 0.5, 5)
     assert (out == -1).all()
     assert _C.ball_query_cuda(query.to(cuda), key.to(cuda), 0.5, 0).shape == (2, 48, 0)
+
+
+@pytest.mark.parametrize("channels_first", [False, True])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("first", [0, 63, 64, 255, 256, 300, 448, 511, 512, 700])
+def test_query_full_within_a_trip(cuda, first, dtype, channels_first):
+    # A trip is 512 keys in chunks of 64. Keys that every query reaches begin at key `first` and go on beyond
+    # the place where a query is full, with stretches out of reach in between.
+    from torkit3d_amd import _C, _fused
+
+    rng = np.random.default_rng(first)
+    key = rng.uniform(5.0, 6.0, (2, 1300, 3)).astype(dtype)
+    near = np.zeros(1300, bool)
+    near[first:first + 3] = near[first + 40:first + 290] = near[first + 400:] = True
+    key[:, near] = rng.uniform(-0.3, 0.3, (2, int(near.sum()), 3)).astype(dtype)
+    query = np.zeros((2, 9, 3), dtype)
+    for k in (1, 3, 4, 64, 100, 253, 254, 400):
+        q, x = torch.from_numpy(query).to(cuda), torch.from_numpy(key).to(cuda)
+        if channels_first:
+            got = _fused.ball_query_bcn(q.transpose(1, 2).contiguous(), x.transpose(1, 2).contiguous(), 1.0, k)
+        else:
+            got = _C.ball_query_cuda(q, x, 1.0, k)
+        np.testing.assert_array_equal(got.cpu().numpy(), oracle.ball_query(query, key, 1.0, k))

@@ -10,11 +10,16 @@
 // Remaining slots repeat the first hit; a query with no hit gets -1 everywhere
 // (ball_query_kernel.cu:94-101, :123).
 //
-// What bounds it: the seven vector instructions of a test, 28 clocks per query and 64 keys on one SIMD, where hits
-// are few (8 x 4096 queries, 16384 keys, radius 0.02 of the unit cube: 99 us, 29 clocks); at radius 0.1 the scan ends
-// early and every fourth chunk has a hit, 92 us. Whether a query is full is asked once per trip and not per chunk
-// (96 -> 92 us there; 8 x 2048 queries 62 -> 54; 16 x 1024 on a sphere of 8000 keys 39 -> 36). Tried: hits of 2, 4
-// or 8 chunks looked for together (99, 133, 170 us), since the chunks' hits are then handled where there are none.
+// What bounds it: the seven vector instructions of a test, 27 clocks per query and 64 keys on one SIMD, where hits
+// are few (8 x 4096 queries, 16384 keys, radius 0.02 of the unit cube: 90 us); at radius 0.1 the scan ends early and
+// every fourth chunk has a hit, 88 us. Whether a query is full is asked twice per trip, and a hit that fills it takes the
+// reach of the chunks up to the next question away: asked per chunk, the tests of several chunks do not overlap; asked
+// per trip alone, a query that is full after its first chunk handles the hits of seven more. us, per chunk, per trip and
+// now: 16 x 1024 queries on 4096 keys, 32 neighbours, radius 0.02 20.1, 18.6, 18.6, radius 0.4 8.2, 9.3, 8.3, radius 2
+// 5.2, 7.9, 5.4; 32 x 2048 on 2048, 8 neighbours, radius 2 9.9, 18.0, 10.1; 8 x 4096 on 16384, 32 neighbours, radius 0.1
+// 92.0, 88.1, 88.2. Tried: leaving the trip at the chunk that fills the query (18.6 -> 24 at radius 0.02: the tests
+// do not overlap either), a form that asks per chunk for queries more than half full (16 x 777 on 3001 15.9 -> 18.4),
+// hits of 2, 4 or 8 chunks looked for together, since the chunks' hits are then handled where there are none.
 #include "tk3d_common.h"
 
 namespace {
@@ -45,6 +50,7 @@ __global__ __launch_bounds__(256) void ball_query_kernel(const T *__restrict__ q
     int64_t *__restrict__ out = index + ((int64_t)b * n1 + q0) * k;
 
     T qx[QW], qy[QW], qz[QW];
+    T reach[QW];  // r2, of a full query less than any distance
     int cnt[QW], first[QW];
     int nq = n1 - q0;
     nq = nq < QW ? nq : QW;
@@ -54,6 +60,7 @@ __global__ __launch_bounds__(256) void ball_query_kernel(const T *__restrict__ q
         qx[q] = ok ? Q[q * qps] : (T)0;
         qy[q] = ok ? Q[q * qps + qcs] : (T)0;
         qz[q] = ok ? Q[q * qps + 2 * qcs] : (T)0;
+        reach[q] = r2;
         cnt[q] = ok ? 0 : k;  // absent queries count as finished
         first[q] = -1;
     }
@@ -84,12 +91,14 @@ __global__ __launch_bounds__(256) void ball_query_kernel(const T *__restrict__ q
         bool all_done = true;
 #pragma unroll
         for (int q = 0; q < QW; ++q) {
-            if (cnt[q] < k) {  // wave-uniform; a query that is full by the end of the trip drops its later hits
+            if (cnt[q] < k) {  // wave-uniform
 #pragma unroll
                 for (int u = 0; u < UNROLL; ++u) {
+                    if (u == UNROLL / 2 && cnt[q] >= k)  // wave-uniform
+                        break;
                     // (false for the NaN of a key that does not exist)
                     const unsigned long long mask = __builtin_amdgcn_ballot_w64(
-                        tk_dist2<T>(kx[u], ky[u], kz[u], qx[q], qy[q], qz[q]) < r2);
+                        tk_dist2<T>(kx[u], ky[u], kz[u], qx[q], qy[q], qz[q]) < reach[q]);
                     if (mask == 0)
                         continue;
                     const int below = __builtin_amdgcn_mbcnt_hi(
@@ -100,6 +109,7 @@ __global__ __launch_bounds__(256) void ball_query_kernel(const T *__restrict__ q
                     if (cnt[q] == 0)
                         first[q] = j0 + u * TK_WAVE + __builtin_ctzll(mask);
                     cnt[q] += __builtin_popcountll(mask);
+                    reach[q] = cnt[q] < k ? r2 : (T)-1;
                 }
             }
             all_done = all_done && (cnt[q] >= k);
