@@ -233,8 +233,8 @@ int tk3d_mlp_group_f32(const float *u, const float *xyz, const float *centre, co
 /* Evaluation of three layers behind a grouping, pooled over the S neighbours: y of tk3d_mlp_group_f32 with C[0]
  * channels, ReLU of its norm[0]; w2 [C[1]][C[0]] and norm[1], w3 [C[2]][C[1]] and norm[2] on top; out [B,C[2],M]
  * is the maximum over each group. `supported`: C multiples of 32 whose activations of 64 positions fit in LDS
- * (C[0] + C[1] up to 512 or so), S 32 or 64, u (or NULL), w2 and w3 16-byte aligned, and work enough for the chip; others
- * are refused. */
+ * (C[0] + C[1] up to 512 or so), S 32 or 64, u (or NULL), w2 and w3 16-byte aligned, and widths and sizes for which it is
+ * the faster way; others are refused. */
 typedef struct tk3d_mlp_grouped_pool {
     const float *u, *xyz, *centre;
     const int64_t *index;

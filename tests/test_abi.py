@@ -275,3 +275,24 @@ def test_products_whose_waves_share_tiles(lib, rows, columns, b, positions, eval
         product.src[0].wk, product.src[0].wc = wk, wc
         slots = lib.tk3d_mlp_product_slots(way, out, ctypes.byref(product))
         assert (slots == b * -(-positions // 32)) is taken
+
+
+class GroupedPool(ctypes.Structure):  # tk3d_mlp_grouped_pool
+    _fields_ = [("pointers", pointer * 7), ("norms", pointer * 15), ("out", pointer), ("sizes", i32 * 8)]
+
+
+# Three layers behind a grouping go in one launch unless that is slower: chains of products that are long for the tiles
+# there are, layers that leave most waves of a CU's only workgroup idle. (256 CUs, b x m groups of s)
+@pytest.mark.parametrize("widths,b,m,s,taken", [
+    ((64, 64, 128), 1, 1, 64, True), ((96, 96, 96), 1, 32, 64, True), ((128, 128, 256), 1, 32, 64, True),
+    ((192, 64, 64), 1, 32, 64, False), ((256, 32, 64), 1, 32, 64, False), ((256, 32, 64), 1, 32, 32, True),
+    ((32, 480, 64), 1, 32, 32, False), ((480, 32, 64), 1, 32, 32, False), ((256, 256, 512), 1, 32, 32, False),
+    ((128, 256, 512), 1, 32, 32, True), ((256, 256, 512), 1, 64, 64, False),
+    ((256, 256, 512), 2, 64, 64, True), ((32, 480, 64), 2, 64, 64, True),
+    ((224, 32, 64), 2, 64, 64, False), ((448, 64, 64), 2, 64, 64, False), ((480, 32, 64), 2, 64, 64, False),
+    ((480, 32, 64), 32, 128, 64, False), ((224, 32, 64), 32, 128, 64, True), ((256, 64, 128), 16, 32, 32, True),
+    ((256, 64, 128), 32, 128, 64, False), ((32, 480, 64), 32, 128, 64, False), ((96, 256, 32), 32, 128, 64, False),
+    ((96, 256, 32), 16, 32, 32, True), ((128, 192, 32), 32, 128, 64, True), ((256, 256, 512), 32, 128, 64, True)])
+def test_grouped_layers_that_share_a_launch(lib, widths, b, m, s, taken):
+    sizes = GroupedPool(sizes=(67, b, 4 * m, m, s, *widths))
+    assert bool(lib.tk3d_mlp_grouped_pool_supported(ctypes.byref(sizes))) is taken

@@ -242,15 +242,60 @@ int64_t tiles_of(const tk3d_mlp_grouped_pool &p, int tile)
     return (int64_t)p.B * (((int64_t)p.M * p.S + tile - 1) / tile);
 }
 int pick_tile(const tk3d_mlp_grouped_pool &p) { return p.S == 32 && tiles_of(p, 64) < tk_cu_count() ? 32 : 64; }
+// Eight waves share a tile if the second layer has a block of channels for every other one at least (four and
+// eight, us: 32 x 777 groups of 32, 64-96-128 channels 331, 359; 32 x 128, 128-128-256 146, 143; 8 x 32,
+// 256-256-512 51, 43).
+int waves_of(const tk3d_mlp_grouped_pool &p) { return p.C[1] < 128 ? 4 : 8; }
+// Fewer tiles than CUs: the third layer's channels over several workgroups, each of which works the first two
+// layers out again (1 x 128 groups of 64, 128-128-256 channels: 24 us in one part, 21 in two, 28 in four).
+int part_of(const tk3d_mlp_grouped_pool &p, int64_t tiles)
+{
+    const int blocks = p.C[2] / 32;
+    int64_t parts = tk_cu_count() / tiles;
+    parts = parts < 1 ? 1 : parts > blocks ? blocks : parts;
+    return (int)((blocks + parts - 1) / parts) * 32;
+}
+
+// Whether one launch is the better choice (us, three launches and this one, 64 features in front of the first layer).
+bool pays(const tk3d_mlp_grouped_pool &p)
+{
+    const int tile = pick_tile(p), waves = waves_of(p), cus = tk_cu_count();
+    const int64_t tiles = tiles_of(p, tile);
+    const int C1 = p.C[0], C2 = p.C[1], C3 = p.C[2];
+    if (tiles < cus) {
+        // A tile is a chain of products on one CU, which three launches spread over the chip: here the channels that a wave
+        // multiplies one behind the other. A short one (two tiles of 32 at once take half as long again as one) is hidden
+        // by the host's time for two launches more: a pass among others, and one that is waited for, 32 groups of 64,
+        // 96-96-96 (192) 22.5, 17.4 and 35.8, 36.6; 128-128-256 (256) 22.3, 20.1 and 37.0, 38.9; with four waves 192-64-64
+        // (256) 22.7, 21.7 and 36.3, 40.8, 256-32-64 (288) 22.3, 23.9 and 36.9, 43.0; 32 of 32, 128-256-512 (384) 22.6, 20.5
+        // and 37.6, 40.2; GPU time, 256-256-512 (512) 23.5, 27.7.
+        // A longer one pays with the tiles that the three have to spread. GPU time, 128 groups of 64: 256-256-512 (512) 69.5,
+        // 47.3, 32-480-64 (544) 35.9, 33.0; with four waves 192-64-64 (256) 23, 23, 224-32-64 (256) 21, 23, 448-64-64 (512)
+        // 33, 38; 64 groups of 64, 256-256-512 (512) 37.7, 39.9.
+        const auto turns = [&](int channels) { return (channels / 32 + waves - 1) / waves; };
+        const int64_t chain = C1 * turns(C2) + C2 * turns(part_of(p, tiles)), all = chain * (tile / 32);
+        return chain * (tile == 64 ? 3 : 2) <= (waves == 4 ? 704 : 768) || (waves == 4 ? all < 4 * tiles : all <= 9 * tiles);
+    }
+    // Layers for which a CU holds one workgroup need work for all of its waves. A second layer of one or two blocks of
+    // channels leaves most of four waves idle through the longest product: 32 x 128 groups of 64, 256-32-64 191, 289,
+    // 480-32-64 367, 502, 256-64-128 267, 319 (with up to four tiles a CU two blocks gain: 16 x 32 of 32 40, 29);
+    // 224-32-64, two workgroups to a CU, 174, 159. So does a third layer of one or two blocks behind a wide second one, on
+    // more than four tiles a CU: 32 x 128 groups of 64, 96-256-32 270, 326, 32-480-64 380, 423, 64-256-64 248, 283;
+    // 16 x 32 of 32, 96-256-32 43, 28. (128-192-32 304, 316 there and 687, 632 at 32 x 512 of 32; 256-256-512, whose
+    // workgroups are alone too, 1056, 929.)
+    if (2 * lds_bytes(C1, C2, C3, 64) > 160 << 10) {
+        if (C2 <= 64)
+            return C2 == 64 && tiles <= 4 * cus;
+        if (C3 <= 64 && C2 >= 2 * C1)
+            return tiles <= 4 * cus;
+    }
+    return true;
+}
 
 }  // namespace
 
 extern "C" {
 
-// Not taken either are wide layers on tiles for less than every fourth CU, where each CU's share of the second layer
-// takes longer than three launches that spread it over the chip (three launches and this one, us: 1 x 32 groups
-// of 32, 256-256-512 channels 23.5, 27.7; 1 x 64 groups of 64 37.7, 39.9; 2 x 64 groups of 32 40.8, 32.5; 1 x 64
-// groups of 64, 128-128-256 23.7, 20.6).
 int tk3d_mlp_grouped_pool_supported(const tk3d_mlp_grouped_pool *p)
 {
     for (int l = 0; l < 3; ++l)
@@ -260,8 +305,7 @@ int tk3d_mlp_grouped_pool_supported(const tk3d_mlp_grouped_pool *p)
         tiles_of(*p, 32) > TK_MAX_I32 / 2 || lds_bytes(p->C[0], p->C[1], p->C[2], 64) > kMostLds ||
         !aligned(p->u) || !aligned(p->w2) || !aligned(p->w3))
         return 0;
-    const int tile = pick_tile(*p);
-    return p->C[0] * p->C[1] * tile <= 1 << 20 || tiles_of(*p, tile) > tk_cu_count() / 4;
+    return pays(*p);
 }
 
 int tk3d_mlp_grouped_pool_f32(const tk3d_mlp_grouped_pool *p, void *stream_)
@@ -271,22 +315,14 @@ int tk3d_mlp_grouped_pool_f32(const tk3d_mlp_grouped_pool *p, void *stream_)
     if (!tk3d_mlp_grouped_pool_supported(p))
         return TK3D_ERR_UNSUPPORTED;
     const hipStream_t stream = (hipStream_t)stream_;
-    const int cus = tk_cu_count(), tile = pick_tile(*p);
+    const int tile = pick_tile(*p);
     GroupedArgs a;
     a.p = *p;
     a.tiles = (p->M * p->S + tile - 1) / tile;
     a.total = (int)tiles_of(*p, tile);
-    // Fewer tiles than CUs: the third layer's channels over several workgroups, each of which works the first two
-    // layers out again (1 x 128 groups of 64, 128-128-256 channels: 24 us in one part, 21 in two, 28 in four).
-    const int blocks = p->C[2] / 32;
-    int parts = cus / a.total;
-    parts = parts < 1 ? 1 : parts > blocks ? blocks : parts;
-    a.part = (blocks + parts - 1) / parts * 32;
-    parts = (p->C[2] + a.part - 1) / a.part;
-    // Eight waves share a tile if the second layer has a block of channels for every other one at least (four and
-    // eight, us: 32 x 777 groups of 32, 64-96-128 channels 331, 359; 32 x 128, 128-128-256 146, 143; 8 x 32,
-    // 256-256-512 51, 43).
-    if (p->C[1] < 128)
+    a.part = part_of(*p, a.total);
+    const int parts = (p->C[2] + a.part - 1) / a.part;
+    if (waves_of(*p) == 4)
         return tile == 32 ? launch<4, 32>(a, parts, stream) : launch<4, 64>(a, parts, stream);
     return tile == 32 ? launch<8, 32>(a, parts, stream) : launch<8, 64>(a, parts, stream);
 }
