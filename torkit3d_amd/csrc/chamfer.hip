@@ -3245,13 +3245,14 @@ __device__ __attribute__((noinline)) bool chamfer_most_tiles_within_reach(
     return within_reach * 4 >= ntiles * 3;
 }
 
-// (Launched one wave per workgroup - waves share nothing, and a finished wave frees its
-// slot at once: 2-3 % over four waves per workgroup. The bound of 256 lanes only caps the
-// registers at four waves per SIMD.)
+// One wave to a workgroup: a finished wave frees its slot at once, the lists in LDS are one wave's, and so are the
+// barriers between those who write them and those who read them, behind returns that a wave takes alone.
 // (Eight rounds of boxes: 96 registers and five waves to a SIMD; with 109 and four, 102 us for 95 on the sphere
 // above, with six waves and values in scratch 105.)
+constexpr int CHAMFER_PRUNED_LANES = TK_WAVE;
+
 template <int NQB, int RMAX, bool COUNT = false>
-__global__ __launch_bounds__(256, RMAX == 8 ? 5 : 1) void chamfer_pruned_kernel(ChamferPrunedArgs a)
+__global__ __launch_bounds__(CHAMFER_PRUNED_LANES, RMAX == 8 ? 5 : 1) void chamfer_pruned_kernel(ChamferPrunedArgs a)
 {
     const int tid = threadIdx.x;
     const int lane = tid & (TK_WAVE - 1);
@@ -3634,7 +3635,8 @@ __global__ __launch_bounds__(256, RMAX == 8 ? 5 : 1) void chamfer_pruned_kernel(
             ntasks += __builtin_popcountll(mask);
         }
     }
-    __syncthreads();  // (of one wave)
+    static_assert(CHAMFER_PRUNED_LANES == TK_WAVE, "the lists belong to one wave");
+    __syncthreads();
     const auto look = [&](int first, auto quads) {  // (a task too many is the last one again)
         constexpr int N = decltype(quads)::value;
         int task[N];
@@ -3927,15 +3929,15 @@ int chamfer_forward_sorted(const float *xyz1, const float *xyz2, int64_t B, int6
     if (!(stages & 2)) {
     } else if (counters != nullptr) {  // (the counting build: tests and the benchmark's untimed repeat)
         if (small)
-            hipLaunchKernelGGL((chamfer_pruned_kernel<NQB, 8, true>), grid, dim3(64), 0, s, pa);
+            hipLaunchKernelGGL((chamfer_pruned_kernel<NQB, 8, true>), grid, dim3(CHAMFER_PRUNED_LANES), 0, s, pa);
         else
-            hipLaunchKernelGGL((chamfer_pruned_kernel<NQB, 32, true>), grid, dim3(64), 0, s, pa);
+            hipLaunchKernelGGL((chamfer_pruned_kernel<NQB, 32, true>), grid, dim3(CHAMFER_PRUNED_LANES), 0, s, pa);
         hipLaunchKernelGGL(chamfer_count_flags_kernel, dim3(1), dim3(256), 0, s, sa.flags,
                            (int)(2 * B), counters);
     } else if (small) {
-        hipLaunchKernelGGL((chamfer_pruned_kernel<NQB, 8>), grid, dim3(64), 0, s, pa);
+        hipLaunchKernelGGL((chamfer_pruned_kernel<NQB, 8>), grid, dim3(CHAMFER_PRUNED_LANES), 0, s, pa);
     } else {
-        hipLaunchKernelGGL((chamfer_pruned_kernel<NQB, 32>), grid, dim3(64), 0, s, pa);
+        hipLaunchKernelGGL((chamfer_pruned_kernel<NQB, 32>), grid, dim3(CHAMFER_PRUNED_LANES), 0, s, pa);
     }
     const int rc = tk_launch_status();
     if (rc != TK3D_OK)
