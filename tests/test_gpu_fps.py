@@ -452,3 +452,31 @@ def test_bands_of_every_kind(cuda, n, k, kind):
     want = oracle.sample_farthest_points(pts.numpy(), k)
     np.testing.assert_array_equal(run(pts, k, cuda), want)
     np.testing.assert_array_equal(run(pts.transpose(1, 2).contiguous(), k, cuda, True), want)
+
+
+@pytest.mark.parametrize("n,k", [(2049, 192), (2049, 2049), (3000, 600), (4096, 256), (4096, 1025)])
+def test_more_clouds_than_compute_units(cuda, n, k):
+    # Clouds of 2049 to 4096 points go through workgroups of eight waves then: bands of every kind, in sampling
+    # order (a claim that holds, and one that fails late), and with a coordinate that is not finite.
+    from torkit3d_amd.ops.sample_farthest_points import sample_farthest_points_gather
+
+    g = gen(n + k)
+    kinds = [_region_cloud(kind, g, 1, n - n % 2) for kind in ("uniform", "lattice", "coarse_lattice", "half_duplicates",
+                                                               "clusters", "line", "shell", "far_from_origin")]
+    kinds = [torch.cat([pts, pts[:, : n % 2]], dim=1)[0] for pts in kinds]
+    big = torch.rand(1, n + 300, 3, generator=g)
+    first = torch.from_numpy(oracle.sample_farthest_points(big.numpy(), n))
+    order = torch.gather(big, 1, first[:, :, None].expand(-1, -1, 3))[0]
+    late, odd = order.clone(), order.clone()
+    late[[k - 2, k - 1]] = order[[k - 1, k - 2]]
+    odd[n - 1, 2] = float("inf")
+    kinds = torch.stack(kinds + [order, late, odd, order * 1e20, order * 3e-21])
+    want = oracle.sample_farthest_points(kinds.numpy(), k)
+    which = torch.arange(torch.cuda.get_device_properties(cuda).multi_processor_count + 3) % len(kinds)
+    pts = kinds[which].contiguous()
+    for transpose in (False, True):
+        dev = (pts.transpose(1, 2) if transpose else pts).contiguous().to(cuda)
+        index, sampled = sample_farthest_points_gather(dev, k, transpose=transpose)
+        np.testing.assert_array_equal(index.cpu().numpy(), want[which.numpy()])
+        got = (sampled.transpose(1, 2) if transpose else sampled).cpu().numpy()
+        np.testing.assert_array_equal(got, np.take_along_axis(pts.numpy(), want[which.numpy()][:, :, None], 1))

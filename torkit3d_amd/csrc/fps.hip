@@ -1608,6 +1608,9 @@ int fps_band_launch_f32(const float *points, bool soa, int64_t B, int64_t *index
 // 159, 161; at 192: 65, 43; 67, 47; 69, 54; 104, 82; 222, 153. In sampling order, in which an encoder's
 // levels come, it has 16 for
 // 46 to 210 at 192 samples.
+// Of the clouds that sixteen waves finish soonest, a CU takes two of eight waves at once, which is the faster way where there
+// are more clouds than CUs. us, multi-step kernel, sixteen waves and eight: 257 x 4096 -> 192 144, 128, 94; 512 x 3000 ->
+// 256 199, 165, 119; 1024 x 4096 -> 192 262, 317, 209, -> 512 602, 434, 310.
 bool fps_band_dispatch_f32(const float *points, bool soa, int64_t B, int64_t *index, float *sampled,
                              const FpsLayout &L, int64_t npos, hipStream_t s, int &rc)
 {
@@ -1617,6 +1620,8 @@ bool fps_band_dispatch_f32(const float *points, bool soa, int64_t B, int64_t *in
         rc = fps_band_launch_f32<2, 8, 2>(points, soa, B, index, sampled, L, s);
     else if (npos <= 512 * 4)
         rc = fps_band_launch_f32<4, 8, 2>(points, soa, B, index, sampled, L, s);
+    else if (npos <= 1024 * 4 && B > tk_cu_count())
+        rc = fps_band_launch_f32<8, 8, 2>(points, soa, B, index, sampled, L, s);
     else if (npos <= 1024 * 4)
         rc = fps_band_launch_f32<4, 16, 2>(points, soa, B, index, sampled, L, s);
     else if (npos <= 1024 * 8)
