@@ -47,6 +47,19 @@ def test_slots(cuda, kind, n2, k, channels_first):
     same(knn_points(a, b, k, transpose=channels_first), want)
 
 
+# The first k keys put in order by networks of 2, 4, 8, 16, 32 and 64 lanes, full and not, on clouds of one chunk of
+# keys to more than eight.
+@pytest.mark.parametrize("kind", ["uniform", "lattice", "broken"])
+@pytest.mark.parametrize("n2", [64, 65, 128, 129, 256, 257, 512, 513])
+def test_order_of_the_first_keys(cuda, kind, n2):
+    q, c = cloud("uniform", n2, 2, 19), cloud(kind, n2, 2, n2)
+    a, b = torch.from_numpy(q).to(cuda), torch.from_numpy(c).to(cuda)
+    for k in (1, 2, 3, 4, 5, 8, 9, 16, 17, 31, 32, 33, 48, 63, 64):
+        same(knn_wave(a, b, k, False), oracle.knn(q, c, k))
+        few = np.ascontiguousarray(c[:, : k + 1])
+        same(knn_wave(a, torch.from_numpy(few).to(cuda), k, False), oracle.knn(q, few, k))
+
+
 def in_order(want, root):
     """A stable sort of the slots, NaNs last (numpy sorts NaNs last)."""
     order = np.argsort(want[0], axis=2, kind="stable")

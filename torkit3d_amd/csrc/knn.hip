@@ -13,8 +13,6 @@
 // k above the largest register variant falls back to a kernel that keeps the
 // structure in the output arrays in global memory, as the reference's generic
 // variant does (knn_distance_kernel.cu:102-177).
-#include <type_traits>
-
 #include "tk3d_common.h"
 #include "tk3d_debug.h"
 
@@ -1174,16 +1172,82 @@ int knn_tree_launch(const T *query, const T *key, T *distance, int64_t *index,
 // neighbour's and the smaller of its own and the new key's - two moves between lanes, a minimum and a
 // maximum, where slots that stay in their lanes take two selects and a maximum over the lanes (4, 5 or
 // 6 steps). A list of the lanes that moves distance, slot and key by selects was slower than either.
-// us, before and now: 4 x 512 queries, 10000 keys,
-// k = 64 57.6, 47.6, k = 16 31.9, 28.1; 8 x 2048 on 2048 k = 20 61, 56, k = 64 125, 112; 1 x 16384 on 16384 k = 64
-// 284, 262; on 128 keys, where ordering the first k counts, k = 64 10.6, 12.5. Tried: insertions in a row
+// us, slots that stay in their lanes and now: 4 x 512 queries on 16384 keys k = 16 39.2, 33.3, k = 64 70.6, 54.4; 1 x
+// 4096 on 16384 k = 64 93, 76; 8 x 2048 on 4096 k = 20 79, 68, k = 64 159, 124; on short clouds, where ordering the
+// first k counts, 8 x 2048 on 128 k = 64 27.6, 23.9, on 64 k = 32 16.4, 14.3. Tried: insertions in a row
 // without a look at the new maximum (longer for few neighbours, whose maximum falls fast).
 // A NaN of the fill holds the pattern of -inf, below every distance; one in slot 0 freezes the query,
 // and no comparison takes one as a candidate.
 
-constexpr int KNN_WAVE_CHUNKS = 8;  // 64 keys each, requested together
+// The value of lane (l ^ X) for X below 32, or 63.
+template <int X> __device__ __forceinline__ int knn_lane_xor(int v)
+{
+    constexpr int DPP = X == 1 ? 0xb1 : X == 2 ? 0x4e : X == 3 ? 0x1b  // quad_perm
+                        : X == 7 ? 0x141 : X == 15 ? 0x140             // row_half_mirror, row_mirror
+                        : X == 8 ? 0x128 : 0;                          // row_ror:8
+    if constexpr (DPP != 0)
+        return __builtin_amdgcn_mov_dpp(v, DPP, 0xf, 0xf, true);
+    else if constexpr (X < 32)
+        return __builtin_amdgcn_ds_swizzle(v, (X << 10) | 0x1f);
+    else
+        return __shfl_xor(v, X);
+}
 
-template <bool SOA, bool WEIGHTS>
+// A step of the network below: the lower lane of a pair l, l ^ X keeps the larger double.
+template <int X> __device__ __forceinline__ void knn_order_step(int &vh, int &vl, int lane)
+{
+    const int oh = knn_lane_xor<X>(vh), ol = knn_lane_xor<X>(vl);
+    const bool lower = (lane & (X == 63 ? 32 : X == 31 ? 16 : X == 15 ? 8 : X == 7 ? 4 : X == 3 ? 2 : X)) == 0;
+    const double mine = __builtin_bit_cast(double, (unsigned long long)(unsigned)vh << 32 | (unsigned)vl);
+    const double other = __builtin_bit_cast(double, (unsigned long long)(unsigned)oh << 32 | (unsigned)ol);
+    const bool take = (other > mine) == lower;
+    vh = take ? oh : vh;
+    vl = take ? ol : vl;
+}
+
+// The doubles of the first k lanes in descending order, -inf in the others: a bitonic network of 1, 3, 6, 10, 15 or
+// 21 steps, of the size that holds k lanes. (Counting, for every lane, the values above its own took four instructions
+// a value: 8 x 2048 queries on 128 keys, k = 64 30.4 us, 23.9 now.)
+__device__ __forceinline__ void knn_order_lanes(int &vh, int &vl, int lane, int k)
+{
+    if (k > 1)  // (uniform)
+        knn_order_step<1>(vh, vl, lane);
+    if (k > 2) {
+        knn_order_step<3>(vh, vl, lane);
+        knn_order_step<1>(vh, vl, lane);
+    }
+    if (k > 4) {
+        knn_order_step<7>(vh, vl, lane);
+        knn_order_step<2>(vh, vl, lane);
+        knn_order_step<1>(vh, vl, lane);
+    }
+    if (k > 8) {
+        knn_order_step<15>(vh, vl, lane);
+        knn_order_step<4>(vh, vl, lane);
+        knn_order_step<2>(vh, vl, lane);
+        knn_order_step<1>(vh, vl, lane);
+    }
+    if (k > 16) {
+        knn_order_step<31>(vh, vl, lane);
+        knn_order_step<8>(vh, vl, lane);
+        knn_order_step<4>(vh, vl, lane);
+        knn_order_step<2>(vh, vl, lane);
+        knn_order_step<1>(vh, vl, lane);
+    }
+    if (k > 32) {
+        knn_order_step<63>(vh, vl, lane);
+        knn_order_step<16>(vh, vl, lane);
+        knn_order_step<8>(vh, vl, lane);
+        knn_order_step<4>(vh, vl, lane);
+        knn_order_step<2>(vh, vl, lane);
+        knn_order_step<1>(vh, vl, lane);
+    }
+}
+
+// CHUNKS: of 64 keys each, requested together, eight or as many as a short cloud has (8 x 2048 queries on 64 keys, k = 3:
+// 10.2 us with eight, 8.5 with one).
+
+template <int CHUNKS, bool SOA, bool WEIGHTS>
 __global__ __launch_bounds__(KNN_BLOCK) void knn_wave_kernel_f32(
     const float *__restrict__ query, const float *__restrict__ key, float *__restrict__ distance,
     int64_t *__restrict__ index, float *__restrict__ weight, float eps, int64_t queries, int n1,
@@ -1200,10 +1264,10 @@ __global__ __launch_bounds__(KNN_BLOCK) void knn_wave_kernel_f32(
     const float qx = knn_coord<SOA>(Q, n1, qi, 0), qy = knn_coord<SOA>(Q, n1, qi, 1),
                 qz = knn_coord<SOA>(Q, n1, qi, 2);
 
-    float px[KNN_WAVE_CHUNKS], py[KNN_WAVE_CHUNKS], pz[KNN_WAVE_CHUNKS];
+    float px[CHUNKS], py[CHUNKS], pz[CHUNKS];
     const auto load = [&](int base) {
 #pragma unroll
-        for (int c = 0; c < KNN_WAVE_CHUNKS; ++c) {
+        for (int c = 0; c < CHUNKS; ++c) {
             int j = base + 64 * c + lane;
             j = j < n2 ? j : n2 - 1;
             if constexpr (SOA) {
@@ -1211,7 +1275,9 @@ __global__ __launch_bounds__(KNN_BLOCK) void knn_wave_kernel_f32(
                 py[c] = K[n2 + j];
                 pz[c] = K[2 * n2 + j];
             } else {
-                const TkPoint3<float> p = tk_load3<float>(K + (int64_t)j * 3);
+                // (a 32-bit offset to a uniform address: at most 2^25 keys)
+                const TkPoint3<float> p = *reinterpret_cast<const TkPoint3<float> *>(
+                    reinterpret_cast<const char *>(K) + (unsigned)j * 12u);
                 px[c] = p.x;
                 py[c] = p.y;
                 pz[c] = p.z;
@@ -1228,39 +1294,27 @@ __global__ __launch_bounds__(KNN_BLOCK) void knn_wave_kernel_f32(
     constexpr int UNUSED = (int)0xfff00000u;  // a double's -inf, below all others
     int vh = lane >= k ? UNUSED : nan ? (int)0xff800000u : __float_as_int(filled);
     int vl = lane >= k ? 0 : ((63 - lane) << Slot::KEY_BITS) | lane;
-    {
-        const double mine = Slot::pack(vh, (unsigned)vl);
-        int place = 0;
-        for (int l = 0; l < k; l += 4) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                place += Slot::pack(__builtin_amdgcn_readlane(vh, l + i),
-                                    (unsigned)__builtin_amdgcn_readlane(vl, l + i)) > mine ? 1 : 0;
-        }
-        place = lane < k ? place : lane;
-        vh = __builtin_amdgcn_ds_permute(4 * place, vh);
-        vl = __builtin_amdgcn_ds_permute(4 * place, vl);
-    }
+    if (k < n2 || sorted)  // (else nothing leaves, and every key goes to its slot)
+        knn_order_lanes(vh, vl, lane, k);
     const bool frozen = __builtin_amdgcn_readfirstlane((int)nan) != 0;
     // what a key has to be below
     unsigned top = (unsigned)__builtin_amdgcn_readfirstlane(vh);
     top = frozen || (int)top < 0 ? 0u : top;
 
-    for (int base = 0; base < n2; base += 64 * KNN_WAVE_CHUNKS) {
-        unsigned d[KNN_WAVE_CHUNKS];
+    for (int base = 0; base < n2; base += 64 * CHUNKS) {
+        unsigned d[CHUNKS];
 #pragma unroll
-        for (int c = 0; c < KNN_WAVE_CHUNKS; ++c) {
+        for (int c = 0; c < CHUNKS; ++c) {
             const int j = base + 64 * c + lane;
             const unsigned bits =
                 __float_as_uint(tk_dist2<float>(px[c], py[c], pz[c], qx, qy, qz));
             d[c] = j >= k && j < n2 ? bits : 0xffffffffu;
         }
-        if (base + 64 * KNN_WAVE_CHUNKS < n2)
-            load(base + 64 * KNN_WAVE_CHUNKS);
+        if (base + 64 * CHUNKS < n2)
+            load(base + 64 * CHUNKS);
 #pragma unroll
-        for (int c = 0; c < KNN_WAVE_CHUNKS; ++c) {
+        for (int c = 0; c < CHUNKS; ++c) {
             unsigned long long mask = __ballot(d[c] < top);
-            const int keys = base + 64 * c + lane;
             while (mask) {
                 const int l = (int)__builtin_ctzll(mask);
                 const int xh = __builtin_amdgcn_readlane((int)d[c], l);
@@ -1268,7 +1322,7 @@ __global__ __launch_bounds__(KNN_BLOCK) void knn_wave_kernel_f32(
                 // the key goes to the head, also in front of its equals (mink.cuh:74-87)
                 const unsigned slot = (unsigned)__builtin_amdgcn_readfirstlane(vl) & Slot::SLOT;
                 const unsigned flag = xh >= __builtin_amdgcn_readlane(vh, 1) ? Slot::FLAG : 0u;
-                const double x = Slot::pack(xh, slot | flag | (unsigned)__builtin_amdgcn_readlane(keys, l));
+                const double x = Slot::pack(xh, slot | flag | (unsigned)(base + 64 * c + l));
                 const double mine = Slot::pack(vh, (unsigned)vl);
                 const double next = Slot::pack(
                     __builtin_amdgcn_update_dpp(UNUSED, vh, 0x130, 0xf, 0xf, false),  // wave_shl:1
@@ -1341,8 +1395,18 @@ int knn_wave_launch(const float *query, const float *key, float *distance, int64
     const int64_t queries = B * n1, blocks = (queries + KNN_BLOCK / 64 - 1) / (KNN_BLOCK / 64);
     if (k > 64 || n2 > (1 << 25) || blocks > TK_MAX_I32)
         return TK3D_ERR_UNSUPPORTED;
-    hipLaunchKernelGGL((knn_wave_kernel_f32<SOA, WEIGHTS>), dim3((unsigned)blocks), dim3(KNN_BLOCK), 0, s,
-                       query, key, distance, index, weight, eps, queries, n1, n2, k, sorted, root);
+#define TK_WAVE_LAUNCH(CHUNKS)                                                                              \
+    hipLaunchKernelGGL((knn_wave_kernel_f32<CHUNKS, SOA, WEIGHTS>), dim3((unsigned)blocks), dim3(KNN_BLOCK), 0, \
+                       s, query, key, distance, index, weight, eps, queries, n1, n2, k, sorted, root)
+    if (n2 <= 64)
+        TK_WAVE_LAUNCH(1);
+    else if (n2 <= 128)
+        TK_WAVE_LAUNCH(2);
+    else if (n2 <= 256)
+        TK_WAVE_LAUNCH(4);
+    else
+        TK_WAVE_LAUNCH(8);
+#undef TK_WAVE_LAUNCH
     return tk_launch_status();
 }
 
