@@ -90,6 +90,33 @@ def test_knn_against_very_many_keys(cuda, k):
     assert np.array_equal(d.cpu().numpy(), want_d)
 
 
+def test_knn_against_more_keys_than_a_slot_has_bits_for(cuda):
+    # 2^25 + 700 keys, the last ones beyond what 25 bits count, on a lattice that repeats every position some
+    # hundred times; a corner of it is met at the very end alone.
+    from torkit3d_amd import _C, _fused
+    from torkit3d_amd.ops.knn_points import knn_points
+
+    n2 = 2 ** 25 + 700
+    rng = np.random.default_rng(7)
+    key = rng.integers(1, 64, (1, n2, 3), dtype=np.int8).astype(np.float32)
+    key[0, -600:] = 0.25 * rng.integers(-8, 3, (600, 3))
+    query = np.concatenate([np.zeros((1, 2, 3), np.float32), rng.integers(0, 64, (1, 3, 3)).astype(np.float32)], 1)
+    q, x = torch.from_numpy(query).to(cuda), torch.from_numpy(key).to(cuda)
+    planes = q.transpose(1, 2).contiguous(), x.transpose(1, 2).contiguous()
+    for k in (3, 20, 64):
+        want = oracle.knn(query, key, k)
+        assert (want[1][0, :2] >= 2 ** 25).all()
+        for got in (_C.knn_distance_cuda(q, x, k, 1), _fused.knn_distance_bcn(*planes, k, 1)):
+            np.testing.assert_array_equal(got[0].cpu().numpy(), want[0])
+            np.testing.assert_array_equal(got[1].cpu().numpy(), want[1])
+        order = np.argsort(want[0], axis=2, kind="stable")
+        distance, index = knn_points(q, x, k, sorted=True)
+        np.testing.assert_array_equal(distance.cpu().numpy(), np.take_along_axis(want[0], order, 2))
+        np.testing.assert_array_equal(index.cpu().numpy(), np.take_along_axis(want[1], order, 2))
+    got = _fused.three_nn(q, x, False)
+    np.testing.assert_array_equal(got[1].cpu().numpy(), oracle.knn(query, key, 3)[1])
+
+
 def test_ball_query_against_very_many_keys(cuda):
     from torkit3d_amd import _C
 

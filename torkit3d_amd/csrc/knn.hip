@@ -13,6 +13,8 @@
 // k above the largest register variant falls back to a kernel that keeps the
 // structure in the output arrays in global memory, as the reference's generic
 // variant does (knn_distance_kernel.cu:102-177).
+#include <type_traits>
+
 #include "tk3d_common.h"
 #include "tk3d_debug.h"
 
@@ -1245,9 +1247,12 @@ __device__ __forceinline__ void knn_order_lanes(int &vh, int &vl, int lane, int 
 }
 
 // CHUNKS: of 64 keys each, requested together, eight or as many as a short cloud has (8 x 2048 queries on 64 keys, k = 3:
-// 10.2 us with eight, 8.5 with one).
+// 10.2 us with eight, 8.5 with one). LONG: clouds of more than KNN_SLOT_KEYS keys, whose numbers do not fit beside a slot
+// and go along in a register of their own (16 queries on 2^25 + 4096 keys, k = 32, by the kernel of a lane per query 487 ms,
+// here 44; k = 64, with slots in a tree in LDS, 2870 and 45).
+constexpr int KNN_SLOT_KEYS = 1 << 25;
 
-template <int CHUNKS, bool SOA, bool WEIGHTS>
+template <int CHUNKS, bool LONG, bool SOA, bool WEIGHTS>
 __global__ __launch_bounds__(KNN_BLOCK) void knn_wave_kernel_f32(
     const float *__restrict__ query, const float *__restrict__ key, float *__restrict__ distance,
     int64_t *__restrict__ index, float *__restrict__ weight, float eps, int64_t queries, int n1,
@@ -1275,9 +1280,10 @@ __global__ __launch_bounds__(KNN_BLOCK) void knn_wave_kernel_f32(
                 py[c] = K[n2 + j];
                 pz[c] = K[2 * n2 + j];
             } else {
-                // (a 32-bit offset to a uniform address: at most 2^25 keys)
+                // (a 32-bit offset to a uniform address, if it fits)
+                using Offset = typename std::conditional<LONG, int64_t, unsigned>::type;
                 const TkPoint3<float> p = *reinterpret_cast<const TkPoint3<float> *>(
-                    reinterpret_cast<const char *>(K) + (unsigned)j * 12u);
+                    reinterpret_cast<const char *>(K) + (Offset)j * 12);
                 px[c] = p.x;
                 py[c] = p.y;
                 pz[c] = p.z;
@@ -1293,9 +1299,13 @@ __global__ __launch_bounds__(KNN_BLOCK) void knn_wave_kernel_f32(
     const bool nan = filled != filled;
     constexpr int UNUSED = (int)0xfff00000u;  // a double's -inf, below all others
     int vh = lane >= k ? UNUSED : nan ? (int)0xff800000u : __float_as_int(filled);
-    int vl = lane >= k ? 0 : ((63 - lane) << Slot::KEY_BITS) | lane;
+    int vl = lane >= k ? 0 : (63 - lane) << Slot::KEY_BITS;
+    if constexpr (!LONG)
+        vl |= lane >= k ? 0 : lane;
     if (k < n2 || sorted)  // (else nothing leaves, and every key goes to its slot)
         knn_order_lanes(vh, vl, lane, k);
+    const auto slot_of = [](int low) { return 63 - (int)(((unsigned)low & Slot::SLOT) >> Slot::KEY_BITS); };
+    int vk = LONG ? slot_of(vl) : 0;
     const bool frozen = __builtin_amdgcn_readfirstlane((int)nan) != 0;
     // what a key has to be below
     unsigned top = (unsigned)__builtin_amdgcn_readfirstlane(vh);
@@ -1322,12 +1332,17 @@ __global__ __launch_bounds__(KNN_BLOCK) void knn_wave_kernel_f32(
                 // the key goes to the head, also in front of its equals (mink.cuh:74-87)
                 const unsigned slot = (unsigned)__builtin_amdgcn_readfirstlane(vl) & Slot::SLOT;
                 const unsigned flag = xh >= __builtin_amdgcn_readlane(vh, 1) ? Slot::FLAG : 0u;
-                const double x = Slot::pack(xh, slot | flag | (unsigned)(base + 64 * c + l));
+                const int number = base + 64 * c + l;
+                const double x = Slot::pack(xh, slot | flag | (LONG ? 0u : (unsigned)number));
                 const double mine = Slot::pack(vh, (unsigned)vl);
                 const double next = Slot::pack(
                     __builtin_amdgcn_update_dpp(UNUSED, vh, 0x130, 0xf, 0xf, false),  // wave_shl:1
                     (unsigned)__builtin_amdgcn_update_dpp(0, vl, 0x130, 0xf, 0xf, true));
                 const double v = knn_max_f64(next, knn_min_f64_uniform(mine, x));
+                if constexpr (LONG) {  // (no two slots are equal: v is one of the three)
+                    const int below = __builtin_amdgcn_update_dpp(0, vk, 0x130, 0xf, 0xf, true);
+                    vk = v == next ? below : v == mine ? vk : number;
+                }
                 vh = Slot::distance(v);
                 vl = (int)Slot::low(v);
                 top = (unsigned)__builtin_amdgcn_readfirstlane(vh);
@@ -1338,7 +1353,7 @@ __global__ __launch_bounds__(KNN_BLOCK) void knn_wave_kernel_f32(
 
     // An entry goes to its slot, or to its place in ascending order (equal distances in slot
     // order, NaNs last, as a stable sort of the slots leaves them).
-    const int slot = 63 - (int)(((unsigned)vl & Slot::SLOT) >> Slot::KEY_BITS);
+    const int slot = slot_of(vl);
     const float refilled = __int_as_float(__builtin_amdgcn_ds_bpermute(4 * slot, __float_as_int(filled)));
     float out = vh < 0 ? refilled : __int_as_float(vh);  // (a NaN never leaves its slot)
     int place = slot;
@@ -1359,7 +1374,7 @@ __global__ __launch_bounds__(KNN_BLOCK) void knn_wave_kernel_f32(
         out = __builtin_sqrtf(out);
     if (lane < k) {
         distance[row * k + place] = out;
-        index[row * k + place] = (int64_t)((unsigned)vl & Slot::KEY);
+        index[row * k + place] = LONG ? (int64_t)vk : (int64_t)((unsigned)vl & Slot::KEY);
     }
     if constexpr (WEIGHTS) {  // k == 3
         const int of_slot = __builtin_amdgcn_ds_permute(4 * (lane < k ? slot : lane), __float_as_int(out));
@@ -1381,10 +1396,9 @@ __global__ __launch_bounds__(KNN_BLOCK) void knn_wave_kernel_f32(
 // and 64 to 10^6 keys, it never lost: equal at k = 48 and 64 on 256 keys, else 1.1 to 7 times faster,
 // also with keys sorted along an axis or a Morton curve (an insertion costs k (1 + ln(keys / k)) of
 // them on keys in random order; on sorted keys there are more, and the other kernels have them too).
-// (A slot has 25 bits for its key.)
-inline bool knn_wave_pays(int64_t queries, int n2, int k)
+inline bool knn_wave_pays(int64_t queries, int k)
 {
-    return k <= 64 && n2 <= (1 << 25) && queries <= (k <= 32 ? 18432 : 36864);
+    return k <= 64 && queries <= (k <= 32 ? 18432 : 36864);
 }
 
 template <bool SOA, bool WEIGHTS>
@@ -1393,19 +1407,21 @@ int knn_wave_launch(const float *query, const float *key, float *distance, int64
                     int root, hipStream_t s)
 {
     const int64_t queries = B * n1, blocks = (queries + KNN_BLOCK / 64 - 1) / (KNN_BLOCK / 64);
-    if (k > 64 || n2 > (1 << 25) || blocks > TK_MAX_I32)
+    if (k > 64 || blocks > TK_MAX_I32)
         return TK3D_ERR_UNSUPPORTED;
-#define TK_WAVE_LAUNCH(CHUNKS)                                                                              \
-    hipLaunchKernelGGL((knn_wave_kernel_f32<CHUNKS, SOA, WEIGHTS>), dim3((unsigned)blocks), dim3(KNN_BLOCK), 0, \
-                       s, query, key, distance, index, weight, eps, queries, n1, n2, k, sorted, root)
+#define TK_WAVE_LAUNCH(CHUNKS, LONG)                                                                             \
+    hipLaunchKernelGGL((knn_wave_kernel_f32<CHUNKS, LONG, SOA, WEIGHTS>), dim3((unsigned)blocks), dim3(KNN_BLOCK), \
+                       0, s, query, key, distance, index, weight, eps, queries, n1, n2, k, sorted, root)
     if (n2 <= 64)
-        TK_WAVE_LAUNCH(1);
+        TK_WAVE_LAUNCH(1, false);
     else if (n2 <= 128)
-        TK_WAVE_LAUNCH(2);
+        TK_WAVE_LAUNCH(2, false);
     else if (n2 <= 256)
-        TK_WAVE_LAUNCH(4);
+        TK_WAVE_LAUNCH(4, false);
+    else if (n2 <= KNN_SLOT_KEYS)
+        TK_WAVE_LAUNCH(8, false);
     else
-        TK_WAVE_LAUNCH(8);
+        TK_WAVE_LAUNCH(8, true);
 #undef TK_WAVE_LAUNCH
     return tk_launch_status();
 }
@@ -1621,7 +1637,7 @@ int knn(const T *query, const T *key, int64_t B, int64_t N1, int64_t N2, int64_t
     hipStream_t s = (hipStream_t)stream;
     const int n1 = (int)N1, n2 = (int)N2, kk = (int)k;
     if constexpr (sizeof(T) == 4) {
-        if (knn_wave_pays(B * N1, n2, kk))
+        if (knn_wave_pays(B * N1, kk))
             return knn_wave_launch<false, false>(query, key, distance, index, nullptr, 0.0f, B, n1,
                                                  n2, kk, 0, 0, s);
     }
@@ -1721,7 +1737,7 @@ int knn_bcn(const T *query, const T *key, int64_t B, int64_t N1, int64_t N2, int
         return TK3D_ERR_NULL_POINTER;
     hipStream_t s = (hipStream_t)stream;
     if constexpr (sizeof(T) == 4) {
-        if (knn_wave_pays(B * N1, n2, kk))
+        if (knn_wave_pays(B * N1, kk))
             return knn_wave_launch<true, false>(query, key, distance, index, nullptr, 0.0f, B, n1, n2,
                                                 kk, 0, 0, s);
         if (k > 4 && !knn_filter_takes(B, n1, n2, kk)) {
@@ -1779,7 +1795,7 @@ int knn_ordered(const T *query, const T *key, bool channels_first, int64_t B, in
     if constexpr (sizeof(T) == 4) {
         if (B > 0 && N1 > 0 && k > 0 && k <= N2 && query && key && distance && index &&
             N1 <= TK_MAX_I32 / 4 && N2 <= TK_MAX_I32 / 4 && tk_fits(TK_MAX_ELEMS, B, N2, 3) &&
-            knn_wave_pays(B * N1, (int)N2, (int)k)) {
+            knn_wave_pays(B * N1, (int)k)) {
             const auto launch = channels_first ? knn_wave_launch<true, false> : knn_wave_launch<false, false>;
             return launch(query, key, distance, index, nullptr, 0.0f, B, (int)N1, (int)N2, (int)k,
                           sorted, root, (hipStream_t)stream);
@@ -1813,7 +1829,7 @@ int three_nn(const T *query, const T *key, bool channels_first, int64_t B, int64
         return TK3D_ERR_UNSUPPORTED;
     hipStream_t s = (hipStream_t)stream;
     if constexpr (sizeof(T) == 4) {
-        if (knn_wave_pays(B * N1, (int)N2, 3)) {
+        if (knn_wave_pays(B * N1, 3)) {
             const auto launch = channels_first ? knn_wave_launch<true, true> : knn_wave_launch<false, true>;
             return launch(query, key, distance, index, weight, (float)eps, B, (int)N1, (int)N2, 3, 0, 0,
                           s);
