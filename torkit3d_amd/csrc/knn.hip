@@ -487,11 +487,12 @@ __device__ __forceinline__ double knn_max_f64(double a, double b)
 // Bound by vector issue, of which the steps are half to two thirds: a lane is a query whose
 // candidates are served in key order, so 59 % of the lanes are busy in a step at k = 16, a third at k =
 // 3. 512 lanes share the staged keys (113 registers up to 16 slots, four waves per SIMD); 32 slots run
-// in 256 (up to 6 % faster; bounded to three waves per SIMD the registers spill, 3 to 30 % slower).
+// in 256, of which a CU holds three workgroups (161 registers; with 256 of them, two workgroups, 32 x 8192 queries on 4096
+// keys k = 20 took 473 us for 289 now, and up to 65536 queries, a workgroup to a CU, 5 % less than now or as much).
 // us, list with nibbles (slot order up to 4) and this: 32 x 8192 queries on 2048 keys k = 3 74, 63, k = 8 101,
-// 82, k = 16 152, 125, k = 32 376, 254; 32 x 2048 on 8192 k = 3 137, 96, k = 16 190, 130, k = 32 272, 191; 4 x 16384
+// 82, k = 16 152, 125, k = 32 372, 260; 32 x 2048 on 8192 k = 3 137, 96, k = 16 190, 130, k = 32 268, 208; 4 x 16384
 // on 16384 k = 16 316, 213; on lattices of 5 positions an axis, where nearly every step meets equal
-// distances, k = 16 407, 166, k = 32 1391, 342.
+// distances, 32 x 8192 on 2048 k = 16 413, 170, k = 32 1380, 324.
 template <int KMAX, bool SOA, bool WEIGHTS, int LANES>
 __global__ __launch_bounds__(LANES) void knn_filter_kernel_f32(
     const float *__restrict__ query, const float *__restrict__ key,
@@ -859,6 +860,8 @@ __global__ __launch_bounds__(LANES) void knn_filter_kernel_f32(
 #pragma unroll
         for (int p = 0; p < KMAX; ++p) {
             if (p < k) {  // uniform
+                if constexpr (KMAX > 16)
+                    asm volatile("" : "+v"(v[p]));  // (and the slots' addresses, ahead of the passes)
                 const int slot = Slot::slot(v[p]);
                 tbuf[lane * ROW + slot] = __builtin_bit_cast(float, Slot::distance(v[p]));
                 ibuf[lane * ROW + slot] = (int)(Slot::low(v[p]) & Slot::KEY);
@@ -878,8 +881,10 @@ __global__ __launch_bounds__(LANES) void knn_filter_kernel_f32(
         const int total = nvalid * k;
         float *od = distance + ((int64_t)b * n1 + q0) * k;
         int64_t *oi = index + ((int64_t)b * n1 + q0) * k;
-#pragma unroll
-        for (int r = 0; r < KMAX; ++r) {
+        // (With 32 slots one after the other: side by side, their addresses, the same in every pass, took the kernel from
+        // 161 registers to 256, two waves to a SIMD instead of three.)
+#pragma unroll (KMAX > 16 ? 1 : KMAX)
+        for (int r = 0; r < (KMAX > 16 ? k : KMAX); ++r) {
             const int e = r * TK_WAVE + lane;
             if (e < total) {
                 const int row = e / k;
@@ -1545,8 +1550,8 @@ int knn_filter_launch(const float *query, const float *key, float *distance, int
     // 512 lanes: two workgroups (16 waves) per CU. A launch of few such workgroups leaves CUs
     // without one: 256 lanes then (128 workgroups, B=8, 8192 x 2048, with a list of nibbles: k = 3 52 ->
     // 48 us, k = 16 96 -> 85 us; at 160 workgroups with up to 8 slots, at 192 with more, the larger
-    // workgroup wins: its staged keys serve more queries). 32 slots leave room for two waves per SIMD,
-    // which 256 lanes use better from 131072 queries on (k = 20 226, 211 us) and no worse below.
+    // workgroup wins: its staged keys serve more queries). 32 slots leave room for three waves per
+    // SIMD, twelve a CU: three workgroups of 256 lanes or one of 512.
     if (!(whatever_the_size || knn_filter_takes(B, n1, n2, k)))
         return TK3D_ERR_UNSUPPORTED;
     if constexpr (KMAX <= 16) {
