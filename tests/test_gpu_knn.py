@@ -136,9 +136,8 @@ def test_errors(cuda):
         _C.knn_distance_cuda(q.transpose(0, 1), q, 2, 1)
 
 
-# ---- few queries, many keys: four waves share the keys of every 64 queries, the waves
-# other than the first log what they insert and the first replays the logs. The result
-# must still be MinK's, slot for slot. ----
+# ---- few queries, many keys: a wave per query, on the shapes and inputs on which several waves once shared
+# the keys of 64 queries. The result must be MinK's, slot for slot. ----
 
 @pytest.mark.parametrize("b,n1,n2,k", [(1, 1000, 4096, 16), (2, 700, 5001, 9), (1, 64, 2048, 5),
                                         (3, 2000, 4100, 8), (1, 16384, 16384, 16),
@@ -273,8 +272,8 @@ def test_slot_order_of_the_hand_worked_mink_run(cuda, k, dtype):
 # ---- many queries: the pre-filtered kernel. A cheaper score rules pairs out, candidates wait
 # in per-lane queues and are inserted later with the exact arithmetic. Whatever the input,
 # distances, indices and slot order must be MinK's: these cases aim at its error bound, its
-# queues, its stage boundaries and its fallbacks. (Sizes are chosen inside the range where
-# the dispatcher takes this kernel: 65536 queries or more against 2048 keys or more.) ----
+# queues, its stage boundaries and its fallbacks. (Sizes are inside the range where the dispatcher takes this
+# kernel: more than 18432 queries, 64 keys or more.) ----
 
 def _filter_case(kind, g, k, b=8, n1=8192 + 5, n2=2048 + 37):  # ragged: partial workgroup, partial chunk
     q, key = uniform_cloud(g, b, n1), uniform_cloud(g, b, n2)
@@ -377,15 +376,31 @@ def test_prefiltered_kernel_on_short_clouds(cuda, n2, k):
     check_raw(q, key, k, cuda)
 
 
-# ---- k = 17..32 with 32768 to 131071 queries against 4096 keys or more: the same matrix
-# sweep feeding the LDS tournament tree (one query per lane, two blocks of 32 per wave) ----
+@pytest.mark.parametrize("channels_first", [False, True])
+@pytest.mark.parametrize("b,n1", [(74, 261), (16, 8200)])  # beyond a wave per query; 131072 queries and more
+@pytest.mark.parametrize("n2,k", [(4, 4), (33, 3), (63, 5), (8, 8), (40, 9), (16, 16), (63, 17), (33, 32)])
+def test_clouds_below_the_prefiltered_kernel(cuda, n2, k, b, n1, channels_first):
+    # under 64 keys: slots in registers (up to 4 neighbours, and up to 8 below 131072 queries), else in the LDS tree
+    from torkit3d_amd.ops.knn_points import knn_points
+
+    g = gen(n2 + k)
+    key, q = uniform_cloud(g, b, n2), uniform_cloud(g, b, n1)
+    key[1::2], q[1::2] = lattice_cloud(g, len(key[1::2]), n2, 4), lattice_cloud(g, len(q[1::2]), n1, 4)
+    want_d, want_i = oracle.knn(q.numpy(), key.numpy(), k)
+    a, c = ((t.transpose(1, 2).contiguous() if channels_first else t).to(cuda) for t in (q, key))
+    distance, index = knn_points(a, c, k, transpose=channels_first)
+    np.testing.assert_array_equal(distance.cpu().numpy(), want_d)
+    np.testing.assert_array_equal(index.cpu().numpy(), want_i)
+
+
+# ---- k = 17..32: the same kernel with 32 slots, in workgroups of 256 lanes ----
 
 @pytest.mark.parametrize("k", [17, 32])
 @pytest.mark.parametrize("kind", ["uniform", "lattice", "far_to_near", "near_to_far",
                                   "far_from_origin", "separated", "tiny", "huge", "huge_queries",
                                   "scaled_small", "scaled_large", "far_queries",
                                   "clusters", "duplicates", "nan_and_inf"])
-def test_tree_kernel_with_matrix_sweep_on_hard_inputs(cuda, kind, k):
+def test_prefiltered_kernel_with_32_slots_on_hard_inputs(cuda, kind, k):
     q, key = _filter_case(kind, gen(sum(map(ord, kind)) + k), k, b=8, n1=4096 + 5, n2=4096 + 37)
     assert 32768 <= q.shape[0] * q.shape[1] < 131072 and key.shape[1] >= 4096
     check_raw(q, key, k, cuda)
@@ -393,7 +408,7 @@ def test_tree_kernel_with_matrix_sweep_on_hard_inputs(cuda, kind, k):
 
 @pytest.mark.parametrize("b,n1,n2,k", [(32, 2048, 8192, 32), (16, 2048, 4096, 20), (5, 8000, 4097, 31),
                                         (2, 20000, 65536, 24), (33, 1000, 4096 + 255, 18)])
-def test_tree_kernel_with_matrix_sweep_shapes(cuda, b, n1, n2, k):
+def test_prefiltered_kernel_with_32_slots_shapes(cuda, b, n1, n2, k):
     g = gen(n1 + n2 + k)
     check_raw(uniform_cloud(g, b, n1), uniform_cloud(g, b, n2), k, cuda)
 

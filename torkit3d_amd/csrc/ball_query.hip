@@ -12,14 +12,14 @@
 //
 // What bounds it: the seven vector instructions of a test, 27 clocks per query and 64 keys on one SIMD, where hits
 // are few (8 x 4096 queries, 16384 keys, radius 0.02 of the unit cube: 90 us); at radius 0.1 the scan ends early and
-// every fourth chunk has a hit, 88 us. Whether a query is full is asked twice per trip, and a hit that fills it takes the
-// reach of the chunks up to the next question away: asked per chunk, the tests of several chunks do not overlap; asked
-// per trip alone, a query that is full after its first chunk handles the hits of seven more. us, per chunk, per trip and
-// now: 16 x 1024 queries on 4096 keys, 32 neighbours, radius 0.02 20.1, 18.6, 18.6, radius 0.4 8.2, 9.3, 8.3, radius 2
-// 5.2, 7.9, 5.4; 32 x 2048 on 2048, 8 neighbours, radius 2 9.9, 18.0, 10.1; 8 x 4096 on 16384, 32 neighbours, radius 0.1
-// 92.0, 88.1, 88.2. Tried: leaving the trip at the chunk that fills the query (18.6 -> 24 at radius 0.02: the tests
-// do not overlap either), a form that asks per chunk for queries more than half full (16 x 777 on 3001 15.9 -> 18.4),
-// hits of 2, 4 or 8 chunks looked for together, since the chunks' hits are then handled where there are none.
+// every fourth chunk has a hit, 88 us. Whether a query is full is asked twice per trip, and a hit that fills it takes
+// the reach of the chunks up to the next question away: asked per chunk, the tests of several chunks do not overlap;
+// asked per trip alone, a query that is full after its first chunk handles the hits of seven more. us, per chunk, per
+// trip and now: 16 x 1024 queries on 4096 keys, 32 neighbours, radius 0.02 20.1, 18.6, 18.6, radius 0.4 8.2, 9.3, 8.3,
+// radius 2 5.2, 7.9, 5.4; 32 x 2048 on 2048, 8 neighbours, radius 2 9.9, 18.0, 10.1; 8 x 4096 on 16384, 32 neighbours,
+// radius 0.1 92.0, 88.1, 88.2. Tried: leaving the trip at the chunk that fills the query (18.6 -> 24 at radius 0.02:
+// the tests do not overlap either), a form that asks per chunk for queries more than half full (16 x 777 on 3001 15.9
+// -> 18.4), hits of 2, 4 or 8 chunks looked for together, since the chunks' hits are then handled where there are none.
 #include "tk3d_common.h"
 
 namespace {

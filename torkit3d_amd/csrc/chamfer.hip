@@ -2225,10 +2225,10 @@ int chamfer_forward(const T *xyz1, const T *xyz2, int64_t B, int64_t N1, int64_t
 //     every query's distance to the nearest key met so far: first the tiles that overlap
 //     the patch, then (if those were few) the tiles within T/4, then those within T,
 //     with T taken anew each time. The
-//     sweep, the three smallest tile minima per lane and the exact re-evaluation of the
-//     candidate tiles are those of the matrix kernel; ties between equal distances go to
-//     the lower original index, compared explicitly because sorted order is not index
-//     order. Queries with three or more candidate tiles are scanned exactly over the
+//     sweep and the three smallest tile minima per lane are those of the matrix kernel; the
+//     candidates' half tiles are evaluated exactly by quads of lanes; ties between equal
+//     distances go to the lower original index, which the compared words hold below the
+//     distance, because sorted order is not index order. Queries with three or more candidate tiles are scanned exactly over the
 //     swept tiles only.
 //
 // Why a skipped tile cannot matter. With the notation of the matrix kernel (k', q' the

@@ -295,8 +295,8 @@ __device__ __forceinline__ int wave_max_i32(int v)
     return __builtin_amdgcn_readlane(v, 63);
 }
 
-// FpsWalk that also reports the largest value it passed by: the walk from the root to
-// the first leaf equal to `wmax` sees the sibling of every node on its path, and the
+// The walk through a lane's tree of maxima from the root to the first leaf equal to `wmax`, which also reports the
+// largest value it passed by: it sees the sibling of every node on its path, and the
 // largest of those siblings is the lane's second-largest minimum (equal to `wmax` when
 // the lane holds the maximum twice).
 template <int P, int NODE> struct FpsWalk2 {
@@ -1302,7 +1302,8 @@ __device__ __forceinline__ bool fps_claim_fails(const float *__restrict__ pts, c
 // out[1], which is zero until then (out[1] holds v_1, a float); nobody waits for anybody, and what a cloud is
 // in for is read from out[0] before the turn is taken, so only the last one changes it, after all have read it.
 // (Against a launch for the check and one for the rest, us: 4 x 1024 -> 512 75.3, 74.0; 8 x 16384 -> 1024 304,
-// 300, where one workgroup copied a cloud's coordinates; a claim that fails late 16 x 4096 -> 1024 249, 255.)
+// 300, where one workgroup copied a cloud's coordinates; a claim that fails late 16 x 4096 -> 1024 249, 255, and 175
+// with the shorter exchanges since.)
 template <int P, int NW, int NB, bool SOA>
 __global__ __launch_bounds__(NW * 64) void fps_settle_kernel_f32(const float *__restrict__ points,
                                                                  int64_t *__restrict__ index,
@@ -1608,9 +1609,9 @@ int fps_band_launch_f32(const float *points, bool soa, int64_t B, int64_t *index
 // 159, 161; at 192: 65, 43; 67, 47; 69, 54; 104, 82; 222, 153. In sampling order, in which an encoder's
 // levels come, it has 16 for
 // 46 to 210 at 192 samples.
-// Of the clouds that sixteen waves finish soonest, a CU takes two of eight waves at once, which is the faster way where there
-// are more clouds than CUs. us, multi-step kernel, sixteen waves and eight: 257 x 4096 -> 192 144, 128, 94; 512 x 3000 ->
-// 256 199, 165, 119; 1024 x 4096 -> 192 262, 317, 209, -> 512 602, 434, 310.
+// Of the clouds that sixteen waves finish soonest, a CU takes two of eight waves at once, which is the faster way where
+// there are more clouds than CUs. us, multi-step kernel, sixteen waves and eight: 257 x 4096 -> 192 144, 128, 94; 512 x
+// 3000 -> 256 199, 165, 119; 1024 x 4096 -> 192 262, 317, 209, -> 512 602, 434, 310.
 bool fps_band_dispatch_f32(const float *points, bool soa, int64_t B, int64_t *index, float *sampled,
                              const FpsLayout &L, int64_t npos, hipStream_t s, int &rc)
 {

@@ -487,12 +487,12 @@ __device__ __forceinline__ double knn_max_f64(double a, double b)
 // Bound by vector issue, of which the steps are half to two thirds: a lane is a query whose
 // candidates are served in key order, so 59 % of the lanes are busy in a step at k = 16, a third at k =
 // 3. 512 lanes share the staged keys (113 registers up to 16 slots, four waves per SIMD); 32 slots run
-// in 256, of which a CU holds three workgroups (161 registers; with 256 of them, two workgroups, 32 x 8192 queries on 4096
-// keys k = 20 took 473 us for 289 now, and up to 65536 queries, a workgroup to a CU, 5 % less than now or as much).
-// us, list with nibbles (slot order up to 4) and this: 32 x 8192 queries on 2048 keys k = 3 74, 63, k = 8 101,
-// 82, k = 16 152, 125, k = 32 372, 260; 32 x 2048 on 8192 k = 3 137, 96, k = 16 190, 130, k = 32 268, 208; 4 x 16384
-// on 16384 k = 16 316, 213; on lattices of 5 positions an axis, where nearly every step meets equal
-// distances, 32 x 8192 on 2048 k = 16 413, 170, k = 32 1380, 324.
+// in 256, of which a CU holds three workgroups (161 registers; with 256 of them, two workgroups, 32 x 8192 queries on
+// 4096 keys k = 20 took 473 us for 289 now, and up to 65536 queries, a workgroup to a CU, 5 % less than now or as
+// much). us, list with nibbles (slot order up to 4) and this: 32 x 8192 queries on 2048 keys k = 3 74, 63, k = 8 101,
+// 82, k = 16 152, 125, k = 32 372, 260; 32 x 2048 on 8192 k = 3 137, 96, k = 16 190, 130, k = 32 268, 208; 4 x 16384 on
+// 16384 k = 16 316, 213; on lattices of 5 positions an axis, where nearly every step meets equal distances, 32 x 8192
+// on 2048 k = 16 413, 170, k = 32 1380, 324.
 template <int KMAX, bool SOA, bool WEIGHTS, int LANES>
 __global__ __launch_bounds__(LANES) void knn_filter_kernel_f32(
     const float *__restrict__ query, const float *__restrict__ key,
@@ -881,8 +881,8 @@ __global__ __launch_bounds__(LANES) void knn_filter_kernel_f32(
         const int total = nvalid * k;
         float *od = distance + ((int64_t)b * n1 + q0) * k;
         int64_t *oi = index + ((int64_t)b * n1 + q0) * k;
-        // (With 32 slots one after the other: side by side, their addresses, the same in every pass, took the kernel from
-        // 161 registers to 256, two waves to a SIMD instead of three.)
+        // (With 32 slots one after the other: side by side, their addresses, the same in every pass, took the kernel
+        // from 161 registers to 256, two waves to a SIMD instead of three.)
 #pragma unroll (KMAX > 16 ? 1 : KMAX)
         for (int r = 0; r < (KMAX > 16 ? k : KMAX); ++r) {
             const int e = r * TK_WAVE + lane;
@@ -1251,10 +1251,10 @@ __device__ __forceinline__ void knn_order_lanes(int &vh, int &vl, int lane, int 
     }
 }
 
-// CHUNKS: of 64 keys each, requested together, eight or as many as a short cloud has (8 x 2048 queries on 64 keys, k = 3:
-// 10.2 us with eight, 8.5 with one). LONG: clouds of more than KNN_SLOT_KEYS keys, whose numbers do not fit beside a slot
-// and go along in a register of their own (16 queries on 2^25 + 4096 keys, k = 32, by the kernel of a lane per query 487 ms,
-// here 44; k = 64, with slots in a tree in LDS, 2870 and 45).
+// CHUNKS: of 64 keys each, requested together, eight or as many as a short cloud has (8 x 2048 queries on 64 keys, k =
+// 3: 10.2 us with eight, 8.5 with one). LONG: clouds of more than KNN_SLOT_KEYS keys, whose numbers do not fit beside a
+// slot and go along in a register of their own (16 queries on 2^25 + 4096 keys, k = 32, by the kernel of a lane per
+// query 487 ms, here 44; k = 64, with slots in a tree in LDS, 2870 and 45).
 constexpr int KNN_SLOT_KEYS = 1 << 25;
 
 template <int CHUNKS, bool LONG, bool SOA, bool WEIGHTS>
@@ -1394,13 +1394,13 @@ __global__ __launch_bounds__(KNN_BLOCK) void knn_wave_kernel_f32(
     }
 }
 
-// Where a wave per query wins (timed against every other kernel here on 260 shapes, 256 to 131072
-// queries, 64 to 16384 keys, k = 1 to 64; the ratio goes with the number of queries): 1.1 to 19
-// times faster up to 16384 queries, even at about 20000 (32768 with more than 32 neighbours,
-// which the lane-per-query kernels keep in LDS). At the limits themselves, with twelve k from 1 to 64
-// and 64 to 10^6 keys, it never lost: equal at k = 48 and 64 on 256 keys, else 1.1 to 7 times faster,
-// also with keys sorted along an axis or a Morton curve (an insertion costs k (1 + ln(keys / k)) of
-// them on keys in random order; on sorted keys there are more, and the other kernels have them too).
+// Where a wave per query wins: its time goes with the number of queries, that of the kernels of a lane per query hardly
+// does while they leave CUs idle. At the limits, 18432 queries, and 36864 with more than 32 neighbours, which the
+// others keep in a tree in LDS, it is the faster one throughout. us, it and the pre-filtered kernel, 18432 queries: on
+// 64 keys k = 3 9.7, 11.6, k = 8 12.7, 14.0, k = 16 15.6, 18.8, k = 32 16.6, 30.1; on 512 k = 3 14.8, 19.0, k = 8 22.1,
+// 24.0, k = 16 32.0, 34.6, k = 32 45.8, 64.0; on 16384 k = 3 152, 211, k = 16 171, 244, k = 32 197, 307. With the tree,
+// 36864 queries: on 64 keys k = 64 10.7, 37, on 16384 492, 1570. (Up to k = 16 the two are even at 20000 to 24000
+// queries, at 32 at 32000 to 40000.)
 inline bool knn_wave_pays(int64_t queries, int k)
 {
     return k <= 64 && queries <= (k <= 32 ? 18432 : 36864);
@@ -1647,7 +1647,7 @@ int knn(const T *query, const T *key, int64_t B, int64_t N1, int64_t N2, int64_t
                                                  n2, kk, 0, 0, s);
     }
     if (k <= 4) {
-        // the pre-filtered kernel wherever it pays (512 keys or more), else the batched kernel
+        // the pre-filtered kernel from 64 keys on, else the batched kernel
         if constexpr (sizeof(T) == 4) {
             const int rc = knn_filter_launch<4, false, false>(query, key, distance, index, nullptr,
                                                               0.0f, B, n1, n2, kk, s);
@@ -1656,11 +1656,9 @@ int knn(const T *query, const T *key, int64_t B, int64_t N1, int64_t N2, int64_t
         }
         knn_launch<T, 4>(query, key, distance, index, B, (int)bpb, n1, n2, kk, s);
     } else if constexpr (sizeof(T) == 4) {
-        // fp32, k >= 5: slots in LDS as a tournament tree (k = 16 at B=32, 8192 x 2048:
-        // 0.30 ms against 0.41 ms with the slots in registers). Small launches with k <= 8
-        // are a little faster in registers.
+        // fp32, k >= 5
         if (k <= 32) {
-            // pre-filtered sweep on the matrix cores, slots in registers: wherever it pays
+            // the pre-filtered kernel from 64 keys on
             const int rc =
                 k <= 8 ? knn_filter_launch<8, false, false>(query, key, distance, index, nullptr,
                                                             0.0f, B, n1, n2, kk, s)
@@ -1672,6 +1670,8 @@ int knn(const T *query, const T *key, int64_t B, int64_t N1, int64_t N2, int64_t
             if (rc != TK3D_ERR_UNSUPPORTED)
                 return rc;
         }
+        // Slots in LDS as a tournament tree: more than 32 neighbours, and clouds of under 64 keys, on which launches
+        // with k <= 8 below 131072 queries are a little faster with slots in registers.
         if (k <= 8 && B * N1 < 131072)
             knn_launch<T, 8>(query, key, distance, index, B, (int)bpb, n1, n2, kk, s);
         else if (k <= 8)
@@ -1715,10 +1715,8 @@ int knn(const T *query, const T *key, int64_t B, int64_t N1, int64_t N2, int64_t
 
 // KNN on [B,3,N] clouds with the kernels that read either layout, k <= 64 (beyond:
 // TK3D_ERR_UNSUPPORTED before anything is launched; the caller copies the clouds and calls
-// knn()). fp32: the pre-filtered sweep where knn() would launch it, the register kernel for
-// k <= 4, else the LDS tree kernel (the variants of it that share keys among several waves,
-// or sweep on the matrix cores, read [B,N,3] only). fp64 runs the same kernels on either
-// layout.
+// knn()). fp32: the wave and pre-filtered kernels where knn() would launch them, else the batched kernel
+// for k <= 4 and the LDS tree kernel. fp64: slots in registers.
 template <typename T>
 int knn_bcn(const T *query, const T *key, int64_t B, int64_t N1, int64_t N2, int64_t k,
             int version, T *distance, int64_t *index, void *stream)
@@ -1746,8 +1744,7 @@ int knn_bcn(const T *query, const T *key, int64_t B, int64_t N1, int64_t N2, int
             return knn_wave_launch<true, false>(query, key, distance, index, nullptr, 0.0f, B, n1, n2,
                                                 kk, 0, 0, s);
         if (k > 4 && !knn_filter_takes(B, n1, n2, kk)) {
-            // k = 17..64, or a launch the pre-filtered sweep does not pay for: the LDS tree,
-            // reading the coordinate planes
+            // more than 32 neighbours, or fewer than 64 keys: the LDS tree, reading the coordinate planes
             if (k <= 8)
                 return knn_tree_launch<8, float, true>(query, key, distance, index, B, n1, n2, kk, s);
             if (k <= 16)

@@ -263,24 +263,25 @@ bool pays(const tk3d_mlp_grouped_pool &p)
     const int64_t tiles = tiles_of(p, tile);
     const int C1 = p.C[0], C2 = p.C[1], C3 = p.C[2];
     if (tiles < cus) {
-        // A tile is a chain of products on one CU, which three launches spread over the chip: here the channels that a wave
-        // multiplies one behind the other. A short one (two tiles of 32 at once take half as long again as one) is hidden
-        // by the host's time for two launches more: a pass among others, and one that is waited for, 32 groups of 64,
-        // 96-96-96 (192) 22.5, 17.4 and 35.8, 36.6; 128-128-256 (256) 22.3, 20.1 and 37.0, 38.9; with four waves 192-64-64
-        // (256) 22.7, 21.7 and 36.3, 40.8, 256-32-64 (288) 22.3, 23.9 and 36.9, 43.0; 32 of 32, 128-256-512 (384) 22.6, 20.5
-        // and 37.6, 40.2; GPU time, 256-256-512 (512) 23.5, 27.7.
-        // A longer one pays with the tiles that the three have to spread. GPU time, 128 groups of 64: 256-256-512 (512) 69.5,
-        // 47.3, 32-480-64 (544) 35.9, 33.0; with four waves 192-64-64 (256) 23, 23, 224-32-64 (256) 21, 23, 448-64-64 (512)
-        // 33, 38; 64 groups of 64, 256-256-512 (512) 37.7, 39.9.
+        // A tile is a chain of products on one CU, which three launches spread over the chip: here the channels that a
+        // wave multiplies one behind the other. A short one (two tiles of 32 at once take half as long again as one) is
+        // hidden by the host's time for two launches more: a pass among others, and one that is waited for, 32 groups
+        // of 64, 96-96-96 (192) 22.5, 17.4 and 35.8, 36.6; 128-128-256 (256) 22.3, 20.1 and 37.0, 38.9; with four waves
+        // 192-64-64 (256) 22.7, 21.7 and 36.3, 40.8, 256-32-64 (288) 22.3, 23.9 and 36.9, 43.0; 32 of 32, 128-256-512
+        // (384) 22.6, 20.5 and 37.6, 40.2; GPU time, 256-256-512 (512) 23.5, 27.7. A longer one pays with the tiles
+        // that the three have to spread. GPU time, 128 groups of 64: 256-256-512 (512) 69.5, 47.3, 32-480-64 (544)
+        // 35.9, 33.0; with four waves 192-64-64 (256) 23, 23, 224-32-64 (256) 21, 23, 448-64-64 (512) 33, 38; 64 groups
+        // of 64, 256-256-512 (512) 37.7, 39.9.
         const auto turns = [&](int channels) { return (channels / 32 + waves - 1) / waves; };
         const int64_t chain = C1 * turns(C2) + C2 * turns(part_of(p, tiles)), all = chain * (tile / 32);
-        return chain * (tile == 64 ? 3 : 2) <= (waves == 4 ? 704 : 768) || (waves == 4 ? all < 4 * tiles : all <= 9 * tiles);
+        return chain * (tile == 64 ? 3 : 2) <= (waves == 4 ? 704 : 768) ||
+               (waves == 4 ? all < 4 * tiles : all <= 9 * tiles);
     }
     // Layers for which a CU holds one workgroup need work for all of its waves. A second layer of one or two blocks of
     // channels leaves most of four waves idle through the longest product: 32 x 128 groups of 64, 256-32-64 191, 289,
     // 480-32-64 367, 502, 256-64-128 267, 319 (with up to four tiles a CU two blocks gain: 16 x 32 of 32 40, 29);
-    // 224-32-64, two workgroups to a CU, 174, 159. So does a third layer of one or two blocks behind a wide second one, on
-    // more than four tiles a CU: 32 x 128 groups of 64, 96-256-32 270, 326, 32-480-64 380, 423, 64-256-64 248, 283;
+    // 224-32-64, two workgroups to a CU, 174, 159. So does a third layer of one or two blocks behind a wide second one,
+    // on more than four tiles a CU: 32 x 128 groups of 64, 96-256-32 270, 326, 32-480-64 380, 423, 64-256-64 248, 283;
     // 16 x 32 of 32, 96-256-32 43, 28. (128-192-32 304, 316 there and 687, 632 at 32 x 512 of 32; 256-256-512, whose
     // workgroups are alone too, 1056, 929.)
     if (2 * lds_bytes(C1, C2, C3, 64) > 160 << 10) {
