@@ -516,3 +516,24 @@ def test_prefilter_kernel_around_the_16_bit_index_limit(cuda, n2, k):
     np.testing.assert_array_equal(got[0].cpu().numpy(), od)
     np.testing.assert_array_equal(got[1].cpu().numpy(), oi)
     assert int(oi.max()) >= n2 - 40
+
+
+@pytest.mark.parametrize("k", [1, 4, 8, 16, 17, 32])
+@pytest.mark.parametrize("n1,n2", [(128, 1024), (129, 1024), (513, 1023), (1029, 1025), (600, 2048 + 65), (512, 4096)])
+def test_prefiltered_kernel_on_sorted_queries(cuda, n1, n2, k):
+    # From 1024 keys and 129 queries on a workgroup sorts its queries and passes over keys outside a wave's box:
+    # a box's edges (queries on a lattice, all in one point), keys far off, and queries that no box holds.
+    from debug_abi import knn_filter
+
+    g = gen(n1 + n2 + k)
+    q, key = uniform_cloud(g, 5, n1), uniform_cloud(g, 5, n2)
+    q[1], key[1] = lattice_cloud(g, 1, n1, 5)[0], lattice_cloud(g, 1, n2, 5)[0]
+    q[2] = q[2, :1]
+    key[3, : n2 // 2] += 1e4
+    q[4, 7, 1], q[4, 9, 0], q[4, 11, 2] = float("inf"), float("nan"), -1e30
+    key[4, n2 - 5, 2] = float("nan")
+    got = knn_filter(q.to(cuda), key.to(cuda), k)
+    assert got is not None
+    od, oi = oracle.knn(q.numpy(), key.numpy(), k)
+    np.testing.assert_array_equal(got[0].cpu().numpy(), od)  # (a NaN equals a NaN)
+    np.testing.assert_array_equal(got[1].cpu().numpy(), oi)

@@ -25,6 +25,7 @@
 #include <type_traits>
 
 #include "tk3d_common.h"
+#include "tk3d_curve.h"
 
 namespace {
 
@@ -512,44 +513,9 @@ constexpr int FPS_CLAIM_MAX = 1024;
 __device__ __forceinline__ int fps_max(int a, int b) { return a > b ? a : b; }
 __device__ __forceinline__ int fps_min(int a, int b) { return a < b ? a : b; }
 
-// Place of the cell (x, y, z) of a 16^3 grid along a Hilbert curve (J. Skilling, "Programming the
-// Hilbert curve", AIP Conference Proceedings 707, 2004).
-constexpr unsigned fps_hilbert(unsigned x, unsigned y, unsigned z)
-{
-    unsigned c[3] = {x, y, z};
-    for (unsigned q = 8u; q > 1u; q >>= 1) {
-        for (int a = 0; a < 3; ++a) {
-            const bool flip = (c[a] & q) != 0u;
-            const unsigned swap = flip ? 0u : (c[0] ^ c[a]) & (q - 1u);
-            c[0] ^= flip ? q - 1u : swap;
-            c[a] ^= swap;
-        }
-    }
-    c[1] ^= c[0];
-    c[2] ^= c[1];
-    unsigned gray = 0u;
-    for (unsigned q = 8u; q > 1u; q >>= 1)
-        gray ^= (c[2] & q) != 0u ? q - 1u : 0u;
-    unsigned place = 0u;
-    for (int b = 3; b >= 0; --b)
-        for (int a = 0; a < 3; ++a)
-            place = 2u * place + (((c[a] ^ gray) >> b) & 1u);
-    return place;
-}
-
-// The places of all cells, by 256 x + 16 y + z. (Worked out for every point they took 150 operations, 13 us of
+// The places of all cells of a 16^3 grid. (Worked out for every point they took 150 operations, 13 us of
 // the 612 at 8 x 16384 -> 4096 and 3 of the 155 at 16 x 4096 -> 1024.)
-struct FpsCurve {
-    unsigned short place[4096];
-};
-constexpr FpsCurve fps_make_curve()
-{
-    FpsCurve t{};
-    for (unsigned i = 0; i < 4096u; ++i)
-        t.place[i] = (unsigned short)fps_hilbert(i >> 8, (i >> 4) & 15u, i & 15u);
-    return t;
-}
-__device__ constexpr FpsCurve fps_curve alignas(16) = fps_make_curve();
+__device__ constexpr TkCurve fps_curve alignas(16) = tk_make_curve();
 
 // Adds to a counter in LDS, lane by lane, and returns what it held before. (As an atomicAdd the
 // compiler turns it into a scan over the lanes, for a handful of which it is.)
@@ -729,9 +695,9 @@ __device__ __forceinline__ void fps_band(const float *__restrict__ pts, int64_t 
         s_red[wave][6] = odd ? -1.0f : far;
     }
     // (the table where the list comes later, if there is room)
-    constexpr bool NEAR = S * 4 >= (int)sizeof(FpsCurve);
+    constexpr bool NEAR = S * 4 >= (int)sizeof(TkCurve);
     if constexpr (NEAR)
-        for (int i = tid; i < (int)sizeof(FpsCurve) / 16; i += NT)
+        for (int i = tid; i < (int)sizeof(TkCurve) / 16; i += NT)
             reinterpret_cast<uint4 *>(fps_band_lds)[i] = reinterpret_cast<const uint4 *>(&fps_curve)[i];
     const unsigned short *const curve =
         NEAR ? reinterpret_cast<const unsigned short *>(fps_band_lds) : fps_curve.place;

@@ -16,6 +16,7 @@
 #include <type_traits>
 
 #include "tk3d_common.h"
+#include "tk3d_curve.h"
 #include "tk3d_debug.h"
 
 namespace {
@@ -431,13 +432,14 @@ __device__ __forceinline__ double knn_max_f64(double a, double b)
 // cores: one v_mfma_f32_32x32x16_f16 gives t for 32 keys x 32 queries as a 16-term dot product of
 // fp16 pieces, and a lane only has to collect the 16 sign bits it is handed (1.1 vector
 // instructions per pair). Coordinates are centred and multiplied by a power of two that brings
-// the largest centred key norm into [1, 2) (exact; outside 2^-40 .. 2^40 the workgroup takes the
-// exact sweep), then split into two fp16 pieces each, x = xh + xl + e with |e| <= 2^-23 |x| +
+// half the diagonal of the keys' bounding box, which no centred key norm exceeds, into [2, 4) (exact; outside
+// 2^-40 .. 2^40 the workgroup takes the exact sweep; a key lies on the box's longest side, 2 / sqrt(3) or more from
+// the centre), then split into two fp16 pieces each, x = xh + xl + e with |e| <= 2^-23 |x| +
 // 2^-25, |k'|^2 into two and -thr into two:
 //     key   : xh xh xl  yh yh yl  1  1  | zh zh zl  n0 n1 0  1  1
 //     query : Xh Xl Xh  Yh Yl Yh  T0 T1 | Zh Zl Zh  1  1  0  T0 T1        (X = -2 q'x)
 // In the 32 x 32 result lane l holds rows (keys) 16 h .. 16 h + 15, h = l / 32, of column
-// (query) l % 32; the keys of a tile are stored in that row order, so the sign bits of a
+// (query) l % 32; lane l puts the key of that row into the tile, so the sign bits of a
 // lane are 16 consecutive bits of the chunk mask. The wave's 64 queries are two blocks of 32,
 // block h the queries of the lanes of half h; a lane computes its thr and writes -thr into the T
 // terms of its own half only (the other half holds zeros there), so no thr crosses lanes; the
@@ -452,12 +454,24 @@ __device__ __forceinline__ double knn_max_f64(double a, double b)
 //     the matrix core's 16 additions: 32 u times the sum of the products' magnitudes
 //         as the matrix core sees them (a subnormal fp16 factor counts as 2^-14; see
 //         the chamfer kernel and tests/test_gpu_mfma_bound.py), which is below
-//         1.02 (M + R) here because the scale makes max|k'| >= 1     33 u (M + R)
+//         1.02 (M + R) here because the scale makes max|k'| > 1      33 u (M + R)
 // below 59 u R + 40 u M; the kernel uses slack = 64 u R + 48 u M (+1e-37 against underflow), R from
-// max|k'| and |q'| inflated by 1e-6 for their own rounding. Every key with canonical d2 < M
+// the bound of |k'| and |q'| inflated by 1e-6 for their own rounding. Every key with canonical d2 < M
 // therefore has t < 0: the sign bits are a superset of MinK's insertions. Queries further than 200
 // from the centre (rescaled; thr would leave fp16's range) take every key as a candidate, key clouds
 // that are non-finite or huge the exact batched sweep.
+//
+// Boxes. From 1024 keys on the workgroup's queries are sorted along a Hilbert curve, so that a wave has
+// neighbours: its 64 queries' box is small, and a key whose distance to that box - by the operations of the canonical distance
+// on the per-axis gaps, each of which is monotone, hence a bound for every query in the box - is not below the
+// largest of the wave's maxima is a candidate of none of them. A lane tests a key, and what passes goes into the
+// wave's list in LDS, in key order; the sweep takes its chunks of 32 from there. Of 2048 keys 780 pass
+// for waves of 512 sorted queries at k = 3 and 1050 at k = 16 (sorted along a Morton curve 980 and 1190; 8192 queries
+// sorted together 300 and 470, but they take a kernel and a workspace of their own). Of fewer keys too many pass.
+//
+// The first keys behind the fill are below the maximum of half of the queries or more: up to 3 k (2 k with 32 slots) they
+// are put to all of them, without a sweep and a queue (a third less work than the steps they save: 142 -> 109 of
+// them at k = 16).
 //
 // Insertions. A candidate is re-evaluated with the canonical arithmetic and inserted
 // under MinK's strict test against the maximum as it stands then, in ascending key
@@ -467,8 +481,6 @@ __device__ __forceinline__ double knn_max_f64(double a, double b)
 // takes its first one) only while some lane holds T candidates or a full queue; the
 // rest waits for company. Deferring only makes M - and with it thr - a little stale,
 // i.e. admits more candidates, each rejected by the strict test when it is served.
-// Per 2048 keys a wave runs 68 steps at k = 3 and 145 at k = 16 instead of 142 and 253
-// rounds.
 //
 // Slots. They are kept in descending order, each a double made of the distance's bit pattern above
 // (flag, KMAX - 1 - slot, key index): v_min_f64 and v_max_f64 run at the rate of 32-bit
@@ -486,13 +498,32 @@ __device__ __forceinline__ double knn_max_f64(double a, double b)
 //
 // Bound by vector issue, of which the steps are half to two thirds: a lane is a query whose
 // candidates are served in key order, so 59 % of the lanes are busy in a step at k = 16, a third at k =
-// 3. 512 lanes share the staged keys (113 registers up to 16 slots, four waves per SIMD); 32 slots run
-// in 256, of which a CU holds three workgroups (161 registers; with 256 of them, two workgroups, 32 x 8192 queries on
-// 4096 keys k = 20 took 473 us for 289 now, and up to 65536 queries, a workgroup to a CU, 5 % less than now or as
-// much). us, list with nibbles (slot order up to 4) and this: 32 x 8192 queries on 2048 keys k = 3 74, 63, k = 8 101,
-// 82, k = 16 152, 125, k = 32 372, 260; 32 x 2048 on 8192 k = 3 137, 96, k = 16 190, 130, k = 32 268, 208; 4 x 16384 on
-// 16384 k = 16 316, 213; on lattices of 5 positions an axis, where nearly every step meets equal distances, 32 x 8192
-// on 2048 k = 16 413, 170, k = 32 1380, 324.
+// 3. 512 lanes share the staged keys and the sort (up to 123 registers and 66 KB of LDS up to 16 slots: four waves
+// per SIMD); 32 slots run in 256, of which a CU holds three workgroups. us, all keys swept and this, uniform
+// clouds unless said otherwise: 32 x 8192 queries on 2048 keys k = 3 69.6, 54.9 (in clusters 68.1, 66.0), k = 8 83.2, 70.1, k = 16
+// 128, 114 (on a sphere 130, 113); 16 x 16384 on 4096 k = 3 103, 75; 4 x 16384 on 16384 k = 16 249, 204; 20 x 1000 on 16384
+// k = 8 232, 160; 1 x 40000 on 40000 k = 16 546, 498; 32 slots, whose waves' boxes are of 256 queries, 24 x 8192 on 2048 k = 32
+// 212, 203, 32 x 2048 on 8192 208, 211; on 64 to 512 keys 0.9 to 1.02 of the time before; clouds of 128 queries, which
+// two waves have anyway, up to 1.12.
+constexpr int knn_max4(int a, int b, int c, int d)
+{
+    const int ab = a > b ? a : b, cd = c > d ? c : d;
+    return ab > cd ? ab : cd;
+}
+
+// The places of all cells of an 8^3 grid along a Hilbert curve.
+struct KnnCurve {
+    unsigned short place[512];
+};
+constexpr KnnCurve knn_make_curve()
+{
+    KnnCurve t{};
+    for (unsigned i = 0; i < 512u; ++i)  // (eight neighbours along the curve of 16^3 are a cell of 8^3)
+        t.place[i] = (unsigned short)(tk_hilbert(2u * (i >> 6), 2u * ((i >> 3) & 7u), 2u * (i & 7u)) >> 3);
+    return t;
+}
+__device__ constexpr KnnCurve knn_curve alignas(16) = knn_make_curve();
+
 template <int KMAX, bool SOA, bool WEIGHTS, int LANES>
 __global__ __launch_bounds__(LANES) void knn_filter_kernel_f32(
     const float *__restrict__ query, const float *__restrict__ key,
@@ -501,100 +532,122 @@ __global__ __launch_bounds__(LANES) void knn_filter_kernel_f32(
 {
     constexpr int BLOCK = LANES;
     constexpr int NW = BLOCK / TK_WAVE;
-    constexpr int STAGE = 512;
+    constexpr int STAGE = KMAX > 16 ? 256 : 512;
     constexpr int CHUNK = 32;
+    constexpr int TEST = KMAX > 16 ? 4 : 2;  // keys a lane tests against the box at once
     constexpr int CAP = 4;
     constexpr int T = 6;
-    constexpr int PER = STAGE / BLOCK;
+    constexpr int PER = STAGE > BLOCK ? STAGE / BLOCK : 1;
+    constexpr int RING = 2 * STAGE;  // a wave's list: it goes back to the first key of the stage before
     using Slot = KnnSlot<KMAX>;
-    static_assert(STAGE % BLOCK == 0 && STAGE % CHUNK == 0, "stage shape");
+    static_assert((STAGE % BLOCK == 0 || BLOCK % STAGE == 0) && STAGE % (TEST * TK_WAVE) == 0, "stage shape");
     static_assert(!WEIGHTS || KMAX == 4, "weights of three neighbours");
-    // Two stage buffers of key terms, [tile][half][row] x 16 bytes, then two of raw keys
-    // (x, y, z, 0) for the service steps.
+    // Two stage buffers of key terms, [key][half] x 16 bytes, then two of raw keys (x, y, z, 0) for the
+    // boxes' test and the service steps; before them the sort's counters, behind them the results.
     constexpr int SCORE_FLOATS = 2 * STAGE * 8;
     constexpr int STAGING_FLOATS = SCORE_FLOATS + 2 * STAGE * 4;
-    static_assert(STAGING_FLOATS >= KNN_STAGE * 4,
-                  "the staging buffers double as the exact sweep's stage");
-    // waves that transpose their results together (32 slots: two, 34 KB of LDS)
-    constexpr int TWAVES = NW < 4 ? NW : KMAX > 16 ? 2 : 4;
-    constexpr int TRANSPOSE_FLOATS = TWAVES * 2 * TK_WAVE * (KMAX + 1);  // see the end of the kernel
-    __shared__ __align__(16) float
-        skey[STAGING_FLOATS > TRANSPOSE_FLOATS ? STAGING_FLOATS : TRANSPOSE_FLOATS];
+    constexpr int CELLS = 512;
+    constexpr int PRUNE = 1024;
+    // rows of results that leave together (36 KB of LDS with 8 slots, 40 at most)
+    constexpr int ROW = KMAX + 1;
+    constexpr int ROWS_FIT = KMAX == 4 ? 1024 : 4096 / KMAX;
+    constexpr int ROWS = ROWS_FIT < BLOCK ? ROWS_FIT : BLOCK;
+    constexpr int LDS_FLOATS = knn_max4(STAGING_FLOATS, ROWS * ROW * 2, CELLS + 4 + CELLS / 2 + 4 * BLOCK, KNN_STAGE * 4);
+    __shared__ __align__(16) float skey[LDS_FLOATS];
+    __shared__ __align__(16) unsigned short sring[NW][RING + CHUNK];  // (its beginning once more behind it)
     float4 *const sraw = reinterpret_cast<float4 *>(skey + SCORE_FLOATS);
     uint4 *const sterm = reinterpret_cast<uint4 *>(skey);
     const int half = (threadIdx.x >> 5) & 1;
-    __shared__ float sred[NW][8];
+    __shared__ float sred[NW][13];
     const int tid = threadIdx.x;
     const int lane = tid & (TK_WAVE - 1);
-    const int wave = tid / TK_WAVE;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / TK_WAVE);
     const int b = blockIdx.x / blocks_per_batch;
     const int qblock = blockIdx.x - b * blocks_per_batch;
     const float *__restrict__ K = key + (int64_t)b * n2 * 3;
     const float *__restrict__ Q = query + (int64_t)b * n1 * 3;
     const float INF = __builtin_huge_valf();
 
-    // ---- bounding box of the key cloud -> centre; largest centred norm ----
-    float lo[3] = {INF, INF, INF}, hi[3] = {-INF, -INF, -INF};
+    // ---- bounding boxes of the key cloud (its centre, and a bound of the centred norms) and of the
+    // workgroup's queries ----
+    const int mine0 = qblock * BLOCK + tid;
+    float ends[6] = {-INF, -INF, -INF, -INF, -INF, -INF};  // -lowest, highest
+    const auto reach_out = [&](float (&e)[6], const float (&v)[3]) {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            e[a] = __builtin_fmaxf(e[a], -v[a]);
+            e[3 + a] = __builtin_fmaxf(e[3 + a], v[a]);
+        }
+    };
     for (int j = tid; j < n2; j += BLOCK) {
+        const float v[3] = {knn_coord<SOA>(K, n2, j, 0), knn_coord<SOA>(K, n2, j, 1), knn_coord<SOA>(K, n2, j, 2)};
+        reach_out(ends, v);
+    }
+    const int nstages = (n2 + STAGE - 1) / STAGE;
+    float4 pre[PER];
+    auto fetch = [&](int st) {
 #pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            const float v = knn_coord<SOA>(K, n2, j, a);
-            lo[a] = __builtin_fminf(lo[a], v);
-            hi[a] = __builtin_fmaxf(hi[a], v);
+        for (int r = 0; r < PER; ++r) {
+            const int kj = st * STAGE + r * BLOCK + tid;
+            pre[r] = make_float4(INF, INF, INF, __builtin_bit_cast(float, kj));  // (past the end: in no box's reach)
+            if (kj < n2 && (BLOCK <= STAGE || tid < STAGE))
+                pre[r] = make_float4(knn_coord<SOA>(K, n2, kj, 0), knn_coord<SOA>(K, n2, kj, 1),
+                                     knn_coord<SOA>(K, n2, kj, 2), __builtin_bit_cast(float, kj));
+        }
+    };
+    fetch(0);
+    float own[3] = {0.0f, 0.0f, 0.0f};  // (of a query that does not exist)
+    float qends[6] = {-INF, -INF, -INF, -INF, -INF, -INF};
+    if (mine0 < n1) {
+#pragma unroll
+        for (int a = 0; a < 3; ++a)
+            own[a] = knn_coord<SOA>(Q, n1, mine0, a);
+        reach_out(qends, own);
+    }
+    tk_wave_max_six<64>(ends);
+    tk_wave_max_six<64>(qends);
+    if (lane == TK_WAVE - 1) {
+#pragma unroll
+        for (int a = 0; a < 6; ++a) {
+            sred[wave][a] = ends[a];
+            sred[wave][6 + a] = qends[a];
         }
     }
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            lo[a] = __builtin_fminf(lo[a], __shfl_xor(lo[a], o));
-            hi[a] = __builtin_fmaxf(hi[a], __shfl_xor(hi[a], o));
-        }
-    }
-    if (lane == 0) {
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            sred[wave][a] = lo[a];
-            sred[wave][3 + a] = hi[a];
-        }
-    }
+    unsigned *const cnt = reinterpret_cast<unsigned *>(skey);
+    unsigned short *const curve = reinterpret_cast<unsigned short *>(cnt + CELLS + 4);
+    if (tid < CELLS / 8)
+        reinterpret_cast<uint4 *>(curve)[tid] = reinterpret_cast<const uint4 *>(knn_curve.place)[tid];
+    for (int i = tid; i <= CELLS; i += BLOCK)
+        cnt[i] = 0u;
     __syncthreads();
-    float cc[3];
+    float cc[3], origin[3], cells[3];
+    float kmax2 = 0.0f;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-        float l = INF, h = -INF;
+        float l = -INF, h = -INF, ql = -INF, qh = -INF;
 #pragma unroll
         for (int w = 0; w < NW; ++w) {
-            l = __builtin_fminf(l, sred[w][a]);
+            l = __builtin_fmaxf(l, sred[w][a]);
             h = __builtin_fmaxf(h, sred[w][3 + a]);
+            ql = __builtin_fmaxf(ql, sred[w][6 + a]);
+            qh = __builtin_fmaxf(qh, sred[w][9 + a]);
         }
-        cc[a] = 0.5f * l + 0.5f * h;
+        cc[a] = 0.5f * h - 0.5f * l;
+        const float side = __builtin_fmaxf(h - cc[a], cc[a] + l);
+        // (the operations of a norm, each of which is monotone: no centred key is beyond it)
+        kmax2 = a == 0 ? side * side : __builtin_fmaf(side, side, kmax2);
+        origin[a] = -ql;
+        const float extent = qh + ql;
+        cells[a] = extent > 0.0f ? 7.99f / extent : 0.0f;  // also 0 for NaN / inf extents
     }
     const float c0 = cc[0], c1 = cc[1], c2 = cc[2];
-    float kmax2 = 0.0f;
-    for (int j = tid; j < n2; j += BLOCK) {
-        const float x = knn_coord<SOA>(K, n2, j, 0) - c0;
-        const float y = knn_coord<SOA>(K, n2, j, 1) - c1;
-        const float z = knn_coord<SOA>(K, n2, j, 2) - c2;
-        kmax2 = __builtin_fmaxf(kmax2, __builtin_fmaf(z, z, __builtin_fmaf(y, y, x * x)));
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1)
-        kmax2 = __builtin_fmaxf(kmax2, __shfl_xor(kmax2, o));
-    if (lane == 0)
-        sred[wave][6] = kmax2;
-    __syncthreads();
-    kmax2 = 0.0f;
-#pragma unroll
-    for (int w = 0; w < NW; ++w)
-        kmax2 = __builtin_fmaxf(kmax2, sred[w][6]);
     bool safe = (c0 - c0 == 0.0f) && (c1 - c1 == 0.0f) && (c2 - c2 == 0.0f) && (kmax2 < 1e30f);
     const float ext = __builtin_sqrtf(kmax2);
     const int ebits = (int)((__builtin_bit_cast(unsigned, ext) >> 23) & 0xffu) - 127;
     safe = safe && (ext == 0.0f || (ebits >= -40 && ebits <= 40));
-    // 2^-(exponent of the largest centred key norm)
+    // Half the box's diagonal comes to [2, 4): its largest side is 1/sqrt(3) of that or more, and a key on it.
     const float scale = (!safe || ext == 0.0f) ? 1.0f
-                                               : __builtin_bit_cast(float, (unsigned)(127 - ebits) << 23);
+                                               : __builtin_bit_cast(float, (unsigned)(128 - ebits) << 23);
 
     if (!safe) {  // uniform over the workgroup
         knn_batched_body<KMAX, SOA, WEIGHTS>(query, key, distance, index, weight, eps, b,
@@ -602,14 +655,81 @@ __global__ __launch_bounds__(LANES) void knn_filter_kernel_f32(
         return;
     }
     const float kmax = __builtin_sqrtf(kmax2) * scale * 1.000001f;
-    const float scale2 = scale * scale;  // <= 2^80
+    const float scale2 = scale * scale;  // <= 2^82
+
+    // ---- the workgroup's queries in the order of their cells along a Hilbert curve, those that do not exist last
+    // (a counting sort; the order within a cell is whatever the atomics give, which no result depends on) ----
+    int mine = tid;
+    float qx = own[0], qy = own[1], qz = own[2];
+    const bool prune = n2 >= PRUNE && n1 > 128;  // uniform
+    if (prune) {
+        unsigned cell = CELLS;
+        if (mine0 < n1) {
+            unsigned at = 0u;
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                const float f = (own[a] - origin[a]) * cells[a];
+                // (a NaN or an out-of-range value lands in cell 0 or 7)
+                at = 8u * at + (unsigned)(int)__builtin_fminf(__builtin_fmaxf(f, 0.0f), 7.0f);
+            }
+            cell = curve[at];
+        }
+        const unsigned turn = atomicAdd(&cnt[cell], 1u);
+        __syncthreads();
+        constexpr int RUN = CELLS / BLOCK;
+        static_assert(RUN * BLOCK == CELLS, "a run of cells to a lane");
+        unsigned c[RUN], sum = 0u;
+#pragma unroll
+        for (int i = 0; i < RUN; ++i) {
+            c[i] = cnt[tid * RUN + i];
+            sum += c[i];
+        }
+        unsigned incl = sum;
+#pragma unroll
+        for (int o = 1; o < TK_WAVE; o <<= 1) {
+            const unsigned up = (unsigned)__shfl_up((int)incl, o);
+            incl += lane >= o ? up : 0u;
+        }
+        if (lane == TK_WAVE - 1)
+            sred[wave][12] = __builtin_bit_cast(float, incl);
+        __syncthreads();
+        unsigned start = incl - sum;
+#pragma unroll
+        for (int w = 0; w < NW; ++w)
+            start += w < wave ? __builtin_bit_cast(unsigned, sred[w][12]) : 0u;
+#pragma unroll
+        for (int i = 0; i < RUN; ++i) {
+            cnt[tid * RUN + i] = start;
+            start += c[i];
+        }
+        if (tid == BLOCK - 1)
+            cnt[CELLS] = start;
+        __syncthreads();
+        float4 *const order = reinterpret_cast<float4 *>(curve + CELLS);
+        order[cnt[cell] + turn] = make_float4(own[0], own[1], own[2], __builtin_bit_cast(float, tid));
+        __syncthreads();
+        const float4 q = order[tid];
+        qx = q.x;
+        qy = q.y;
+        qz = q.z;
+        mine = __builtin_bit_cast(int, q.w);
+    }
 
     // ---- the lane's query ----
-    const int qi = qblock * BLOCK + tid;
+    const int qi = qblock * BLOCK + mine;
     const bool active = qi < n1;
-    const float qx = active ? knn_coord<SOA>(Q, n1, qi, 0) : c0;
-    const float qy = active ? knn_coord<SOA>(Q, n1, qi, 1) : c1;
-    const float qz = active ? knn_coord<SOA>(Q, n1, qi, 2) : c2;
+    // the box of the wave's queries
+    float box[6] = {-INF, -INF, -INF, -INF, -INF, -INF};
+    if (active) {
+        const float v[3] = {qx, qy, qz};
+        reach_out(box, v);
+    }
+    tk_wave_max_six<64>(box);
+#pragma unroll
+    for (int a = 0; a < 6; ++a) {
+        const int end = __builtin_amdgcn_readlane(__builtin_bit_cast(int, box[a]), TK_WAVE - 1);
+        box[a] = __builtin_bit_cast(float, prune ? end : 0x7f7fffff);  // (else all keys)
+    }
     float qn, slack_r;
     bool usable;
     // The query side of the 16 terms for the wave's two blocks of 32 queries, block h being the
@@ -652,51 +772,25 @@ __global__ __launch_bounds__(LANES) void knn_filter_kernel_f32(
 #pragma unroll
     for (int s = 0; s < KMAX; ++s)
         v[s] = UNUSED;
-    // fill: keys 0..k-1 go to slots 0..k-1 (mink.cuh:63-72)
-#pragma unroll
-    for (int s = 0; s < KMAX; ++s) {
-        if (s < k) {  // uniform
-            const float d = tk_dist2<float>(knn_coord<SOA>(K, n2, s, 0), knn_coord<SOA>(K, n2, s, 1),
-                                            knn_coord<SOA>(K, n2, s, 2), qx, qy, qz);
-            const bool isnan = d != d;
-            nan_slots |= isnan ? (1u << s) : 0u;
-            frozen |= isnan && s == 0;
-            const double x = Slot::pack(isnan ? NEG_INF_BITS : __builtin_bit_cast(int, d),
-                                        ((unsigned)(KMAX - 1 - s) << Slot::KEY_BITS) | (unsigned)s);
-#pragma unroll
-            for (int p = s; p >= 1; --p)
-                v[p] = knn_max_f64(v[p], tk_min_f64(v[p - 1], x));
-            v[0] = knn_max_f64(v[0], x);
-        }
-    }
-    float max_key = frozen ? -INF : __builtin_bit_cast(float, Slot::distance(v[0]));
-    // Pending chunk masks, oldest first (bit 31 = first key of the chunk), and the key index of
-    // bit 31 of each. Named and no loops over the queue, so it stays in registers.
+    float max_key = 0.0f;
+    // Pending chunk masks, oldest first (bit 31 = first key of the chunk), and the place in the wave's list
+    // of bit 31 of each. Named and no loops over the queue, so it stays in registers.
     static_assert(CAP == 4, "the queue is written out for four entries");
     unsigned m0 = 0u, m1 = 0u, m2 = 0u, m3 = 0u;
     int b0 = 0, b1 = 0, b2 = 0, b3 = 0;
     int qlen = 0, pending = 0;
 
-    // One service step: every query with a pending candidate takes its first one.
-    auto service = [&]() {
-        const bool has = qlen > 0;
-        // (an empty queue has m0 == 0: the bit number is then meaningless, the address
-        // below stays inside the buffer and nothing is inserted)
-        const int bit = __builtin_clz(m0 | 1u);
-        const int kj = b0 + bit;
-        // resident: candidates are never older than the previous stage (see below)
-        const float4 raw = sraw[kj & (2 * STAGE - 1)];
-        const unsigned rest = m0 & ~(0x80000000u >> bit);
-        const bool shift = has && rest == 0u;
-        m0 = shift ? m1 : rest;
-        b0 = shift ? b1 : b0;
-        m1 = shift ? m2 : m1;
-        b1 = shift ? b2 : b1;
-        m2 = shift ? m3 : m2;
-        b2 = shift ? b3 : b2;
-        m3 = shift ? 0u : m3;
-        qlen -= shift ? 1 : 0;
-        pending -= has ? 1 : 0;
+    // The wave's list: 16 times which key of the two buffers. (Zeros: a place that nothing was listed at is
+    // read where a query has no candidate.)
+    unsigned short *const ring = sring[wave];
+    unsigned char *const lds_raw = reinterpret_cast<unsigned char *>(sraw);
+    unsigned char *const lds_term = reinterpret_cast<unsigned char *>(sterm);
+    for (int i = lane; i < (RING + CHUNK) / 8; i += TK_WAVE)
+        reinterpret_cast<uint4 *>(ring)[i] = make_uint4(0u, 0u, 0u, 0u);
+    int head = 0, tail = 0;  // places of the list: swept up to, filled up to (uniform)
+
+    // Puts a key to the lane's query.
+    auto put = [&](const float4 &raw, int kj, bool has) {
         const float d = tk_dist2<float>(raw.x, raw.y, raw.z, qx, qy, qz);
         const bool ins = has && d < max_key;  // MinK's strict test (mink.cuh:74)
         const int dbits = __builtin_bit_cast(int, d);
@@ -711,6 +805,35 @@ __global__ __launch_bounds__(LANES) void knn_filter_kernel_f32(
             v[p] = knn_max_f64(v[p + 1], tk_min_f64(v[p], x));
         v[KMAX - 1] = tk_min_f64(v[KMAX - 1], x);
         max_key = ins ? __builtin_bit_cast(float, Slot::distance(v[0])) : max_key;
+    };
+
+    // With 32 slots, one to three waves a SIMD: where the first candidate lies is looked up a step ahead, beside the insertion before it.
+    constexpr bool AHEAD = KMAX > 16 || LANES == 256;
+    unsigned coming = 0u;
+    auto look = [&]() { coming = ring[b0 + __builtin_clz(m0 | 1u)]; };
+    // One service step: every query with a pending candidate takes its first one.
+    auto service = [&]() {
+        const bool has = qlen > 0;
+        // (an empty queue has m0 == 0: the bit number is then meaningless, the address
+        // below stays inside the buffer and nothing is inserted)
+        const int bit = __builtin_clz(m0 | 1u);
+        // resident: candidates are never older than the previous stage (see below)
+        const float4 raw = *reinterpret_cast<const float4 *>(lds_raw + (AHEAD ? coming : ring[b0 + bit]));
+        const int kj = __builtin_bit_cast(int, raw.w);
+        const unsigned rest = m0 & ~(0x80000000u >> bit);
+        const bool shift = has && rest == 0u;
+        m0 = shift ? m1 : rest;
+        b0 = shift ? b1 : b0;
+        m1 = shift ? m2 : m1;
+        b1 = shift ? b2 : b1;
+        m2 = shift ? m3 : m2;
+        b2 = shift ? b3 : b2;
+        m3 = shift ? 0u : m3;
+        qlen -= shift ? 1 : 0;
+        pending -= has ? 1 : 0;
+        if constexpr (AHEAD)
+            look();
+        put(raw, kj, has);
         // Keep the loop-carried state where it is: without this the register allocator
         // rotates some forty values through copies on every step.
         asm volatile("" : "+v"(m0), "+v"(m1), "+v"(m2), "+v"(m3));
@@ -725,190 +848,239 @@ __global__ __launch_bounds__(LANES) void knn_filter_kernel_f32(
     };
 
     // ---- sweep: keys centred and staged in two LDS buffers, one barrier per stage ----
-    const int nstages = (n2 + STAGE - 1) / STAGE;
-    float4 pre[PER];
-    auto fetch = [&](int st) {
-#pragma unroll
-        for (int r = 0; r < PER; ++r) {
-            const int kj = st * STAGE + r * BLOCK + tid;
-            pre[r] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            if (kj < n2)
-                pre[r] = make_float4(knn_coord<SOA>(K, n2, kj, 0), knn_coord<SOA>(K, n2, kj, 1),
-                                     knn_coord<SOA>(K, n2, kj, 2), 1.0f);
-        }
-    };
     auto stash = [&](int buf) {
+        if (BLOCK > STAGE && tid >= STAGE)
+            return;
 #pragma unroll
         for (int r = 0; r < PER; ++r) {
-            const int j = r * BLOCK + tid;  // key within the stage
-            const bool exists = pre[r].w != 0.0f;
+            const int j = buf * STAGE + r * BLOCK + tid;
             const float ex = pre[r].x - c0, ey = pre[r].y - c1, ez = pre[r].z - c2;
             const float x = ex * scale, y = ey * scale, z = ez * scale;
             const float n = __builtin_fmaf(ez, ez, __builtin_fmaf(ey, ey, ex * ex)) * scale2;
             const unsigned sx = tk_f16_split2(x), sy = tk_f16_split2(y), sz = tk_f16_split2(z);
             const unsigned xh = sx & 0xffffu, yh = sy & 0xffffu, zh = sz & 0xffffu;
             const unsigned sn = tk_f16_split2(n);
-            // (past the end: an infinite norm, never a candidate)
-            const unsigned n0 = exists ? (sn & 0xffffu) : 0x7c00u, n1 = exists ? (sn >> 16) : 0u;
-            // row of the tile: lane half h of the result holds rows 8 a + 4 h + c
-            const int row = ((j & 12) << 1) | ((j & 16) >> 2) | (j & 3);
-            uint4 *t = sterm + buf * (STAGE * 2) + (j >> 5) * 64 + row;
-            t[0] = make_uint4(xh * 0x10001u, (sx >> 16) | (yh << 16), yh | (sy & 0xffff0000u),
-                              0x3c003c00u);
-            t[32] = make_uint4(zh * 0x10001u, (sz >> 16) | (n0 << 16), n1, 0x3c003c00u);
-            sraw[buf * STAGE + j] = pre[r];
+            sterm[2 * j] = make_uint4(xh * 0x10001u, (sx >> 16) | (yh << 16), yh | (sy & 0xffff0000u),
+                                      0x3c003c00u);
+            sterm[2 * j + 1] = make_uint4(zh * 0x10001u, (sz >> 16) | (sn << 16), sn >> 16, 0x3c003c00u);
+            sraw[j] = pre[r];
+        }
+    };
+    bool stale = true;    // the T terms do not belong to the maximum any more
+    bool moved = true;    // nor does the wave's reach
+    float reach = 0.0f;   // the largest of the queries' maxima
+    // The key of a chunk in this lane's row of the tile: lane half h of the result holds rows 8 a + 4 h + c.
+    const int row = (lane & 3) | ((lane >> 1) & 12) | ((lane & 4) << 2);
+    // Sweeps the next `count` <= 32 keys of the list, and serves what has to be.
+    auto sweep = [&](int count) {
+        tk_wave_fence();  // (the list is the wave's own)
+        const int first = head & (RING - 1);  // (a chunk goes on into the ring's beginning behind its end)
+        const int at = ring[first + (row < count ? row : 0)];
+        const tk_f16x8 ka = *reinterpret_cast<const tk_f16x8 *>(lds_term + 2 * at + 16 * half);
+        if (stale) {  // uniform
+            const float m = max_key * scale2;  // rescaled units; slack 64 u R + 48 u M
+            const float thr = (m - qn) + __builtin_fmaf(m, 2.8610229e-06f, slack_r);
+            const unsigned tp = tk_f16_split2(-thr);
+            qterm[0].w = half == 0 ? tp : 0u;
+            qterm[1].w = half == 1 ? tp : 0u;
+            stale = false;
+        }
+        unsigned m16[2];
+        const tk_f32x16 zero = {};
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+            const tk_f32x16 acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                ka, __builtin_bit_cast(tk_f16x8, qterm[g]), zero, 0, 0, 0);
+            unsigned m = 0u;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const float t = acc[r];  // (a bit_cast applied to acc[r] itself reads element 0)
+                m = __builtin_amdgcn_alignbit(m, __builtin_bit_cast(unsigned, t), 31);
+            }
+            m16[g] = m;
+        }
+        // Lane l has rows (keys) 16 half .. of column l % 32 of both blocks, the first key in
+        // the highest bit. The upper lanes of block 0 change places with the lower ones of
+        // block 1: then it has both halves of the rows of its own column of its own block.
+        const auto both = __builtin_amdgcn_permlane32_swap(m16[0], m16[1], false, false);
+        const unsigned mask = ((unsigned)both[0] << 16) | (unsigned)both[1];
+        const unsigned valid = ~(unsigned)(0xffffffffull >> count);
+        const unsigned m = active ? (usable ? mask : 0xffffffffu) & valid : 0u;
+        const bool nz = m != 0u;
+        const int to = nz ? qlen : -1;
+        m0 = to == 0 ? m : m0;
+        b0 = to == 0 ? first : b0;
+        m1 = to == 1 ? m : m1;
+        b1 = to == 1 ? first : b1;
+        m2 = to == 2 ? m : m2;
+        b2 = to == 2 ? first : b2;
+        m3 = to == 3 ? m : m3;
+        b3 = to == 3 ? first : b3;
+        qlen += nz ? 1 : 0;
+        pending += __builtin_popcount(m);
+        head += count;
+        if constexpr (AHEAD)
+            look();
+        // (two steps per trip: the loop-carried state is copied between registers once
+        // per trip, some forty moves)
+        while (must_serve()) {
+            stale = moved = true;
+            service();
+            if (!must_serve())
+                break;
+            service();
         }
     };
     __syncthreads();
-    fetch(0);
     stash(0);
     __syncthreads();
-    bool stale = true;  // the T terms do not belong to the maximum any more
+    // fill: keys 0..k-1 go to slots 0..k-1 (mink.cuh:63-72)
+#pragma unroll
+    for (int s = 0; s < KMAX; ++s) {
+        if (s < k) {  // uniform
+            const float4 raw = sraw[s];
+            const float d = tk_dist2<float>(raw.x, raw.y, raw.z, qx, qy, qz);
+            const bool isnan = d != d;
+            nan_slots |= isnan ? (1u << s) : 0u;
+            frozen |= isnan && s == 0;
+            const double x = Slot::pack(isnan ? NEG_INF_BITS : __builtin_bit_cast(int, d),
+                                        ((unsigned)(KMAX - 1 - s) << Slot::KEY_BITS) | (unsigned)s);
+#pragma unroll
+            for (int p = s; p >= 1; --p)
+                v[p] = knn_max_f64(v[p], tk_min_f64(v[p - 1], x));
+            v[0] = knn_max_f64(v[0], x);
+        }
+    }
+    max_key = frozen ? -INF : __builtin_bit_cast(float, Slot::distance(v[0]));
+    int before = 0;  // where the list was when this stage began
+    // The first keys behind the fill are below the maximum of so many queries that they are put to all of them.
+    const int taken_fit = KMAX <= 16 ? 3 * k : 2 * k;
+    const int taken = taken_fit < n2 ? taken_fit : n2;
+    for (int j = k; j < taken; ++j) {
+        const float4 raw = sraw[j];
+        put(raw, j, active);
+    }
     for (int st = 0; st < nstages; ++st) {
-        const int stage0 = st * STAGE;
+        const int stage0 = st * STAGE, buf = (st & 1) * STAGE;
         if (st + 1 < nstages)
             fetch(st + 1);
         const int left = n2 - stage0;
         const int cnt = left < STAGE ? left : STAGE;
-        for (int c0k = 0; c0k < cnt; c0k += CHUNK) {
-            const int first = stage0 + c0k;  // key index of bit 31
-            const tk_f16x8 ka = __builtin_bit_cast(
-                tk_f16x8, sterm[(st & 1) * (STAGE * 2) + (c0k >> 5) * 64 + lane]);
-            if (stale) {  // uniform
-                const float m = max_key * scale2;  // rescaled units; slack 64 u R + 48 u M
-                const float thr = (m - qn) + __builtin_fmaf(m, 2.8610229e-06f, slack_r);
-                const unsigned tp = tk_f16_split2(-thr);
-                qterm[0].w = half == 0 ? tp : 0u;
-                qterm[1].w = half == 1 ? tp : 0u;
-                stale = false;
+#pragma unroll 1
+        for (int j0 = 0; j0 < cnt; j0 += TEST * TK_WAVE) {
+            if (moved) {  // uniform
+                reach = tk_wave_extreme<true>(active ? max_key : -INF);
+                moved = false;
             }
-            unsigned m16[2];
-            const tk_f32x16 zero = {};
+            float4 raw[TEST];
+            unsigned long long in[TEST];
 #pragma unroll
-            for (int g = 0; g < 2; ++g) {
-                const tk_f32x16 acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-                    ka, __builtin_bit_cast(tk_f16x8, qterm[g]), zero, 0, 0, 0);
-                unsigned m = 0u;
+            for (int u = 0; u < TEST; ++u)
+                raw[u] = sraw[buf + j0 + u * TK_WAVE + lane];
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const float t = acc[r];  // (a bit_cast applied to acc[r] itself reads element 0)
-                    m = __builtin_amdgcn_alignbit(m, __builtin_bit_cast(unsigned, t), 31);
+            for (int u = 0; u < TEST; ++u) {
+                // (box[a] is -lowest)
+                const float gx = __builtin_fmaxf(__builtin_fmaxf(-box[0] - raw[u].x, raw[u].x - box[3]), 0.0f);
+                const float gy = __builtin_fmaxf(__builtin_fmaxf(-box[1] - raw[u].y, raw[u].y - box[4]), 0.0f);
+                const float gz = __builtin_fmaxf(__builtin_fmaxf(-box[2] - raw[u].z, raw[u].z - box[5]), 0.0f);
+                const float bound = __builtin_fmaf(gz, gz, __builtin_fmaf(gy, gy, gx * gx));
+                in[u] = __builtin_amdgcn_ballot_w64(bound < reach);
+            }
+            if (st == 0 && j0 == 0) {  // uniform; these have been taken
+                in[0] = taken < TK_WAVE ? in[0] & (~0ull << taken) : 0ull;
+                in[1] = taken > TK_WAVE ? in[1] & (~0ull << (taken - TK_WAVE)) : in[1];
+            }
+#pragma unroll
+            for (int u = 0; u < TEST; ++u) {
+                const int below = __builtin_amdgcn_mbcnt_hi((unsigned)(in[u] >> 32),
+                                                            __builtin_amdgcn_mbcnt_lo((unsigned)in[u], 0));
+                if (__builtin_amdgcn_inverse_ballot_w64(in[u])) {
+                    const int to = (tail + below) & (RING - 1);
+                    const unsigned short key = (unsigned short)(16 * (buf + j0 + u * TK_WAVE + lane));
+                    ring[to] = key;
+                    if (to < CHUNK)
+                        ring[RING + to] = key;
                 }
-                m16[g] = m;
+                tail += __builtin_popcountll(in[u]);
             }
-            // Lane l has rows (keys) 16 half .. of column l % 32 of both blocks, the first key in
-            // the highest bit. The upper lanes of block 0 change places with the lower ones of
-            // block 1: then it has both halves of the rows of its own column of its own block.
-            const auto both = __builtin_amdgcn_permlane32_swap(m16[0], m16[1], false, false);
-            const unsigned mask = ((unsigned)both[0] << 16) | (unsigned)both[1];
-            // Keys that do not exist, or that the fill phase took, are no candidates.
-            int vlo = k - first;
-            vlo = vlo < 0 ? 0 : (vlo > CHUNK ? CHUNK : vlo);
-            int vhi = cnt - c0k;
-            vhi = vhi > CHUNK ? CHUNK : vhi;
-            unsigned valid = (vlo >= CHUNK) ? 0u : (0xffffffffu >> vlo);
-            valid &= (vhi >= CHUNK) ? 0xffffffffu : ~(0xffffffffu >> vhi);
-            unsigned m = usable ? mask : 0xffffffffu;
-            m = active ? (m & valid) : 0u;
-            const bool nz = m != 0u;
-            const int at = nz ? qlen : -1;
-            m0 = at == 0 ? m : m0;
-            b0 = at == 0 ? first : b0;
-            m1 = at == 1 ? m : m1;
-            b1 = at == 1 ? first : b1;
-            m2 = at == 2 ? m : m2;
-            b2 = at == 2 ? first : b2;
-            m3 = at == 3 ? m : m3;
-            b3 = at == 3 ? first : b3;
-            qlen += nz ? 1 : 0;
-            pending += __builtin_popcount(m);
-            // (two steps per trip: the loop-carried state is copied between registers once
-            // per trip, some forty moves)
-            while (must_serve()) {
-                stale = true;
-                service();
-                if (!must_serve())
-                    break;
-                service();
-            }
+            while (tail - head >= CHUNK)
+                sweep(CHUNK);
         }
         if (st + 1 < nstages) {
-            // The next stage replaces the previous one in LDS: whatever is still pending
-            // from it is served first (the queue is in key order, so its head tells).
-            while (__builtin_amdgcn_ballot_w64(qlen > 0 && b0 < stage0) != 0) {
-                stale = true;
+            // The next stage replaces the previous one in LDS: whatever is still to be swept or pending
+            // from it comes first (the queue is in key order, so its head tells).
+            if (head < before)
+                sweep(tail - head);
+            // (no chunk begins more than a stage before or behind `before`)
+            while (__builtin_amdgcn_ballot_w64(qlen > 0 && ((b0 - before) & STAGE) != 0) != 0) {
+                stale = moved = true;
                 service();
             }
+            before = tail;
             __syncthreads();  // every wave is done with the previous stage
             stash((st + 1) & 1);
         }
         __syncthreads();
     }
+    if (tail > head)
+        sweep(tail - head);
     while (__builtin_amdgcn_ballot_w64(qlen > 0) != 0)
         service();
 
-    // ---- results: a wave's 64 queries own 64 * k consecutive output elements; the slots
-    // are transposed through LDS (row stride KMAX + 1: no bank conflicts) so that the
-    // stores are runs of consecutive elements instead of one element per k ----
-    __syncthreads();
-    constexpr int ROW = KMAX + 1;
-    float *const tbuf = skey + (wave % TWAVES) * (2 * TK_WAVE * ROW);  // values, then indices
-    int *const ibuf = reinterpret_cast<int *>(tbuf + TK_WAVE * ROW);
-    static_assert(TWAVES * 2 * TK_WAVE * ROW == TRANSPOSE_FLOATS, "LDS for the transpose");
-    auto emit = [&]() {
-        const int q0 = qblock * BLOCK + wave * TK_WAVE;  // first query of the wave
+    // ---- results: the workgroup's queries own consecutive rows of k; the slots go to their rows
+    // through LDS (row stride KMAX + 1), a part of the rows at a time, so that the stores are runs
+    // of consecutive elements ----
+    float *const tbuf = skey;  // values, then indices
+    int *const ibuf = reinterpret_cast<int *>(skey + ROWS * ROW);
+#pragma unroll 1
+    for (int part = 0; part < BLOCK / ROWS; ++part) {
+        const int row0 = qblock * BLOCK + part * ROWS;  // of the cloud's queries
+        int rows = n1 - row0;
+        if (rows <= 0)  // uniform
+            break;
+        rows = rows < ROWS ? rows : ROWS;
+        __syncthreads();  // the last stage, or the part before, has been read
+        if (active && mine / ROWS == part) {
+            const int r = (mine & (ROWS - 1)) * ROW;
 #pragma unroll
-        for (int p = 0; p < KMAX; ++p) {
-            if (p < k) {  // uniform
-                if constexpr (KMAX > 16)
-                    asm volatile("" : "+v"(v[p]));  // (and the slots' addresses, ahead of the passes)
-                const int slot = Slot::slot(v[p]);
-                tbuf[lane * ROW + slot] = __builtin_bit_cast(float, Slot::distance(v[p]));
-                ibuf[lane * ROW + slot] = (int)(Slot::low(v[p]) & Slot::KEY);
+            for (int p = 0; p < KMAX; ++p) {
+                if (p < k) {  // uniform
+                    if constexpr (KMAX > 16)
+                        asm volatile("" : "+v"(v[p]));  // (and the slots' addresses, ahead of the parts)
+                    const int slot = Slot::slot(v[p]);
+                    tbuf[r + slot] = __builtin_bit_cast(float, Slot::distance(v[p]));
+                    ibuf[r + slot] = (int)(Slot::low(v[p]) & Slot::KEY);
+                }
+            }
+            if (nan_slots != 0u) {  // NaNs of the fill, still in their slots
+#pragma unroll
+                for (int s = 0; s < KMAX; ++s) {
+                    if (s < k && ((nan_slots >> s) & 1u))
+                        tbuf[r + s] = tk_dist2<float>(knn_coord<SOA>(K, n2, s, 0), knn_coord<SOA>(K, n2, s, 1),
+                                                      knn_coord<SOA>(K, n2, s, 2), qx, qy, qz);
+                }
             }
         }
-        if (nan_slots != 0u) {  // NaNs of the fill, still in their slots
-#pragma unroll
-            for (int s = 0; s < KMAX; ++s) {
-                if (s < k && ((nan_slots >> s) & 1u))
-                    tbuf[lane * ROW + s] = tk_dist2<float>(
-                        knn_coord<SOA>(K, n2, s, 0), knn_coord<SOA>(K, n2, s, 1),
-                        knn_coord<SOA>(K, n2, s, 2), qx, qy, qz);
-            }
-        }
-        tk_wave_fence();
-        const int nvalid = n1 - q0 < TK_WAVE ? n1 - q0 : TK_WAVE;  // may be <= 0
-        const int total = nvalid * k;
-        float *od = distance + ((int64_t)b * n1 + q0) * k;
-        int64_t *oi = index + ((int64_t)b * n1 + q0) * k;
-        // (With 32 slots one after the other: side by side, their addresses, the same in every pass, took the kernel
-        // from 161 registers to 256, two waves to a SIMD instead of three.)
-#pragma unroll (KMAX > 16 ? 1 : KMAX)
-        for (int r = 0; r < (KMAX > 16 ? k : KMAX); ++r) {
-            const int e = r * TK_WAVE + lane;
-            if (e < total) {
-                const int row = e / k;
-                const int col = e - row * k;
-                od[e] = tbuf[row * ROW + col];
-                oi[e] = (int64_t)ibuf[row * ROW + col];
-            }
+        __syncthreads();
+        const int total = rows * k;
+        float *od = distance + ((int64_t)b * n1 + row0) * k;
+        int64_t *oi = index + ((int64_t)b * n1 + row0) * k;
+        int r = tid / k, col = tid - r * k;
+        const int dr = BLOCK / k, dcol = BLOCK - dr * k;
+#pragma unroll 1
+        for (int e = tid; e < total; e += BLOCK) {
+            od[e] = tbuf[r * ROW + col];
+            oi[e] = (int64_t)ibuf[r * ROW + col];
+            r += dr;
+            col += dcol;
+            r += col >= k ? 1 : 0;
+            col -= col >= k ? k : 0;
         }
         if constexpr (WEIGHTS) {  // k == 3
-            if (active) {
-                const float d3[3] = {tbuf[lane * ROW], tbuf[lane * ROW + 1], tbuf[lane * ROW + 2]};
-                knn_three_weights<float>(d3, eps, weight + ((int64_t)b * n1 + q0 + lane) * 3);
+            for (int i = tid; i < rows; i += BLOCK) {
+                const float d3[3] = {tbuf[i * ROW], tbuf[i * ROW + 1], tbuf[i * ROW + 2]};
+                knn_three_weights<float>(d3, eps, weight + ((int64_t)b * n1 + row0 + i) * 3);
             }
-        }
-    };
-    if constexpr (NW == TWAVES) {
-        emit();
-    } else {
-#pragma unroll 1
-        for (int pass = 0; pass < NW / TWAVES; ++pass) {
-            if (pass > 0)
-                __syncthreads();  // the waves of the previous pass are done with the buffers
-            if (wave / TWAVES == pass)
-                emit();
         }
     }
 }
@@ -1548,15 +1720,15 @@ int knn_filter_launch(const float *query, const float *key, float *distance, int
                       bool whatever_the_size = false)
 {
     // 512 lanes: two workgroups (16 waves) per CU. A launch of few such workgroups leaves CUs
-    // without one: 256 lanes then (128 workgroups, B=8, 8192 x 2048, with a list of nibbles: k = 3 52 ->
-    // 48 us, k = 16 96 -> 85 us; at 160 workgroups with up to 8 slots, at 192 with more, the larger
-    // workgroup wins: its staged keys serve more queries). 32 slots leave room for three waves per
+    // without one: 256 lanes then, unless there are keys enough for the boxes of 512 sorted queries to pay (us, 256 and 512
+    // lanes: 5 x 4096 queries on 512 keys k = 8 24.4, 28.0, 8 x 4096 on 1024 k = 3 26.2, 25.3, 2 x 16384 on 4096 k = 3 64, 49,
+    // 5 x 5000 on 1024 k = 16 46.5, 52.8, 3 x 8192 on 16384 k = 16 256, 191). 32 slots leave room for three waves per
     // SIMD, twelve a CU: three workgroups of 256 lanes or one of 512.
     if (!(whatever_the_size || knn_filter_takes(B, n1, n2, k)))
         return TK3D_ERR_UNSUPPORTED;
     if constexpr (KMAX <= 16) {
         const int64_t bpb = ((int64_t)n1 + 511) / 512;
-        if (B * bpb > (KMAX <= 8 ? 128 : 160))
+        if (B * bpb > (KMAX <= 8 ? 128 : 160) || n2 >= (KMAX <= 8 ? 1024 : 2048))
             return knn_filter_launch_as<KMAX, SOA, WEIGHTS, 512>(query, key, distance, index, weight,
                                                                  eps, B, n1, n2, k, s);
     }
