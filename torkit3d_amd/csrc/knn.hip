@@ -1429,8 +1429,13 @@ __device__ __forceinline__ void knn_order_lanes(int &vh, int &vl, int lane, int 
 // query 487 ms, here 44; k = 64, with slots in a tree in LDS, 2870 and 45).
 constexpr int KNN_SLOT_KEYS = 1 << 25;
 
+// A trip inside the cloud loads from uniform addresses at the lane's offset and asks about no key whether it exists or
+// was filled (17 vector instructions a chunk, one of them a product of integers, became 8), and 64 registers leave room for eight
+// waves a SIMD (67 before). us, before and now: 4 x 512 queries on 10000 keys k = 1 16.6, 14.2, k = 64 45.4, 42.4; 8 x
+// 2048 on 2048 k = 20 50, 45; 1 x 16384 on 16384 k = 3 123, 119 (its loads from L1), k = 16 163, 140, k = 64 232, 183; planes, 1 x
+// 16384 on 4096 k = 3 43.7, 36.3; one trip, 8 x 2048 on 300 k = 16 24.9, 23.9.
 template <int CHUNKS, bool LONG, bool SOA, bool WEIGHTS>
-__global__ __launch_bounds__(KNN_BLOCK) void knn_wave_kernel_f32(
+__global__ __launch_bounds__(KNN_BLOCK, LONG ? 1 : 8) void knn_wave_kernel_f32(
     const float *__restrict__ query, const float *__restrict__ key, float *__restrict__ distance,
     int64_t *__restrict__ index, float *__restrict__ weight, float eps, int64_t queries, int n1,
     int n2, int k, int sorted, int root)
@@ -1447,7 +1452,26 @@ __global__ __launch_bounds__(KNN_BLOCK) void knn_wave_kernel_f32(
                 qz = knn_coord<SOA>(Q, n1, qi, 2);
 
     float px[CHUNKS], py[CHUNKS], pz[CHUNKS];
+    constexpr int TRIP = 64 * CHUNKS;
+    const unsigned lane_bytes = (unsigned)lane * (SOA ? 4u : 12u);
     const auto load = [&](int base) {
+        if (CHUNKS == 8 && base > 0 && base + TRIP <= n2) {  // uniform: a lane's offset to uniform addresses
+#pragma unroll
+            for (int c = 0; c < CHUNKS; ++c) {
+                const char *const at = reinterpret_cast<const char *>(K + (int64_t)(base + 64 * c) * (SOA ? 1 : 3));
+                if constexpr (SOA) {
+                    px[c] = *reinterpret_cast<const float *>(at + lane_bytes);
+                    py[c] = *reinterpret_cast<const float *>(at + (int64_t)n2 * 4 + lane_bytes);
+                    pz[c] = *reinterpret_cast<const float *>(at + (int64_t)n2 * 8 + lane_bytes);
+                } else {
+                    const TkPoint3<float> p = *reinterpret_cast<const TkPoint3<float> *>(at + lane_bytes);
+                    px[c] = p.x;
+                    py[c] = p.y;
+                    pz[c] = p.z;
+                }
+            }
+            return;
+        }
 #pragma unroll
         for (int c = 0; c < CHUNKS; ++c) {
             int j = base + 64 * c + lane;
@@ -1488,17 +1512,20 @@ __global__ __launch_bounds__(KNN_BLOCK) void knn_wave_kernel_f32(
     unsigned top = (unsigned)__builtin_amdgcn_readfirstlane(vh);
     top = frozen || (int)top < 0 ? 0u : top;
 
-    for (int base = 0; base < n2; base += 64 * CHUNKS) {
+    for (int base = 0; base < n2; base += TRIP) {
         unsigned d[CHUNKS];
 #pragma unroll
-        for (int c = 0; c < CHUNKS; ++c) {
-            const int j = base + 64 * c + lane;
-            const unsigned bits =
-                __float_as_uint(tk_dist2<float>(px[c], py[c], pz[c], qx, qy, qz));
-            d[c] = j >= k && j < n2 ? bits : 0xffffffffu;
+        for (int c = 0; c < CHUNKS; ++c)
+            d[c] = __float_as_uint(tk_dist2<float>(px[c], py[c], pz[c], qx, qy, qz));
+        if (base == 0 || base + TRIP > n2) {  // uniform
+#pragma unroll
+            for (int c = 0; c < CHUNKS; ++c) {
+                const int j = base + 64 * c + lane;
+                d[c] = j >= k && j < n2 ? d[c] : 0xffffffffu;
+            }
         }
-        if (base + 64 * CHUNKS < n2)
-            load(base + 64 * CHUNKS);
+        if (base + TRIP < n2)
+            load(base + TRIP);
 #pragma unroll
         for (int c = 0; c < CHUNKS; ++c) {
             unsigned long long mask = __ballot(d[c] < top);
