@@ -72,3 +72,36 @@ def test_square_roots(cuda, transpose, dtype):
     with torch.no_grad():
         for f, p in zip(chamfer_distance(x, y, transpose=transpose, sqrt=True, eps=eps), plain):
             assert torch.equal(f, p)
+
+
+# lengths on either side of a range of the backward kernel and of the longest cloud whose layout and roots it takes itself
+@pytest.mark.parametrize("sqrt", [False, True])
+@pytest.mark.parametrize("b,n1,n2", [(2, 1, 3), (3, 4095, 4097), (2, 8192, 5), (1, 8193, 700)])
+def test_backward_of_planes_and_roots(cuda, b, n1, n2, sqrt):
+    rows = [t.to(cuda).requires_grad_() for t in clouds(b, n1, n2)]
+    planes = [t.detach().transpose(1, 2).contiguous().requires_grad_() for t in rows]
+    grads = [torch.randn(b, n, device=cuda) for n in (n1, n2)]
+    eps = 1e-6
+    dists = chamfer_distance(*rows)
+    want = torch.autograd.grad([safe_sqrt(d, eps) for d in dists] if sqrt else dists, rows, grads)
+    roots = chamfer_distance(*rows, sqrt=sqrt, eps=eps)
+    for got, w in zip(torch.autograd.grad(roots, rows, grads), want):
+        assert torch.equal(got, w)
+    for some in ((0, 1), (0,), (1,)):  # (both gradients, or one)
+        leaves = [p.detach().requires_grad_(i in some) for i, p in enumerate(planes)]
+        out = chamfer_distance(*leaves, transpose=True, sqrt=sqrt, eps=eps)
+        for i, got in zip(some, torch.autograd.grad(out, [leaves[i] for i in some], grads)):
+            assert torch.equal(got, want[i].transpose(1, 2))
+
+
+def test_backward_of_planes_and_roots_with_infinite_gradients(cuda):
+    x, y = [t.to(cuda).transpose(1, 2).contiguous().requires_grad_() for t in clouds(2, 300, 513)]
+    grads = [torch.randn(2, n, device=cuda) for n in (300, 513)]
+    grads[1][0, 7] = float("inf")  # (a batch element with sums through atomics)
+    rows = [t.detach().transpose(1, 2).contiguous().requires_grad_() for t in (x, y)]
+    plain = [safe_sqrt(d) for d in chamfer_distance(*rows)]
+    want = torch.autograd.grad(plain, rows, grads)
+    got = torch.autograd.grad(chamfer_distance(x, y, transpose=True, sqrt=True), (x, y), grads)
+    # (the distances' gradients agree to the bit; sums of the same float32 terms in another order: a few of them a point)
+    for g, w in zip(got, want):
+        torch.testing.assert_close(g.transpose(1, 2), w, rtol=1e-5, atol=1e-5, equal_nan=True)

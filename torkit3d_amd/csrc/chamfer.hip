@@ -1323,12 +1323,33 @@ __global__ __launch_bounds__(256) void chamfer_backward_scatter_kernel(
 // floating-point path.
 // The own terms are fetched first, while the accumulators are cleared and the first
 // match indices arrive, and meet the sums at the end.
-template <int R, int NT>
+//
+// SOA: clouds as planes, [B,3,N] (the gradients come as [B,N,3] all the same). ROOT: gradients of the roots of the
+// distances, from which those of the distances are made where they are read.
+template <typename T> __device__ __forceinline__ T chamfer_root_grad(T g, T d, T root, T eps)
+{
+    const T of_root = g / (root * 2);
+    return d >= eps ? of_root : (T)0;
+}
+
+// Up to two ranges a cloud: every range reads what it is sent anew, roots and distances as well, and points at random
+// places from three planes. (Kernels of a backward call in us, [B,3,N] with roots, with launches in front that copy the
+// clouds to rows and form the gradients, and without: 8 x 2500 x 3001 10.6 + 2.7, 13.5, and 4 to 7 us less of the
+// host's time; without roots 32 x 2048 x 2048 9.9 + 3.0, 10.8, 16 x 8192 x 8192 13.0 + 3.9, 17.6; 32 x 16384 x 16384 21.1 +
+// 9.0, 39.2, without roots 21.1 + 8.7, 31.0.)
+constexpr int64_t CHAMFER_FORMS_POINTS = 8192;
+
+struct ChamferRootGrads {
+    const float *dist[2], *root[2];
+    float eps;
+};
+
+template <int R, int NT, bool SOA, bool ROOT>
 __global__ __launch_bounds__(NT) void chamfer_backward_fixed_kernel(
     const float *__restrict__ gd1, const float *__restrict__ gd2,
     const float *__restrict__ xyz1, const float *__restrict__ xyz2,
     const int64_t *__restrict__ idx1, const int64_t *__restrict__ idx2, int n1, int n2,
-    int ranges1, int ranges2, float *__restrict__ gx1, float *__restrict__ gx2)
+    int ranges1, int ranges2, float *__restrict__ gx1, float *__restrict__ gx2, ChamferRootGrads roots)
 {
     extern __shared__ __align__(16) unsigned long long acc[];  // [R * 3], then the range
     float *sx = reinterpret_cast<float *>(acc + R * 3);        // of X itself: [R * 3] floats
@@ -1387,8 +1408,33 @@ __global__ __launch_bounds__(NT) void chamfer_backward_fixed_kernel(
     auto load_f = [](__amdgpu_buffer_rsrc_t rs, int at) {
         return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, at, 0, 0));
     };
-    auto load_f3 = [](__amdgpu_buffer_rsrc_t rs, int at) {
-        return __builtin_bit_cast(f3, __builtin_amdgcn_raw_buffer_load_b96(rs, at, 0, 0));
+    // point i of a cloud of n
+    auto load_point = [](__amdgpu_buffer_rsrc_t rs, int i, int n) {
+        if constexpr (SOA) {
+            f3 p;
+            p.x = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, i * 4, 0, 0));
+            p.y = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, i * 4, n * 4, 0));
+            p.z = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, i * 4, n * 8, 0));
+            return p;
+        } else {
+            return __builtin_bit_cast(f3, __builtin_amdgcn_raw_buffer_load_b96(rs, i * 12, 0, 0));
+        }
+    };
+    const int from_y = second ? 0 : 1;  // whose distances and roots belong to Y
+    const auto of_cloud = [&](const float *const (&both)[2], bool y) {
+        return ROOT ? both[y ? from_y : 1 - from_y] + (int64_t)b * (y ? ny : nx) : gX;
+    };
+    const float *const dX = of_cloud(roots.dist, false), *const tX = of_cloud(roots.root, false);
+    const float *const dY = of_cloud(roots.dist, true), *const tY = of_cloud(roots.root, true);
+    const __amdgpu_buffer_rsrc_t rdX = rsrc(dX, (int64_t)nx * 4), rtX = rsrc(tX, (int64_t)nx * 4);
+    const __amdgpu_buffer_rsrc_t rdY = rsrc(dY, (int64_t)ny * 4), rtY = rsrc(tY, (int64_t)ny * 4);
+    // the gradient of distance i
+    auto load_grad = [&](__amdgpu_buffer_rsrc_t g, __amdgpu_buffer_rsrc_t d, __amdgpu_buffer_rsrc_t t, int i) {
+        const float grad = load_f(g, i * 4);
+        if constexpr (ROOT)
+            return chamfer_root_grad<float>(grad, load_f(d, i * 4), load_f(t, i * 4), roots.eps);
+        else
+            return grad;
     };
     auto load_i64 = [](__amdgpu_buffer_rsrc_t rs, int at) {
         return __builtin_bit_cast(int64_t, __builtin_amdgcn_raw_buffer_load_b64(rs, at, 0, 0));
@@ -1422,8 +1468,8 @@ __global__ __launch_bounds__(NT) void chamfer_backward_fixed_kernel(
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int is = jj[u] >= 0 ? sender(round, u) : 0;
-            g[u] = load_f(rgY, is * 4) * 2;
-            y[u] = load_f3(rY, is * 12);
+            g[u] = load_grad(rgY, rdY, rtY, is) * 2;
+            y[u] = load_point(rY, is, ny);
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -1502,7 +1548,7 @@ __global__ __launch_bounds__(NT) void chamfer_backward_fixed_kernel(
 #pragma unroll
             for (int f = 0; f < F; ++f) {
                 const int j = j0 + tid + f * NT;
-                xs[f] = load_f3(rX, (j < j1 ? j : j0) * 12);
+                xs[f] = load_point(rX, j < j1 ? j : j0, nx);
             }
             if (rounds > 0)
                 load_matches(0, jj);
@@ -1522,8 +1568,8 @@ __global__ __launch_bounds__(NT) void chamfer_backward_fixed_kernel(
 #pragma unroll
         for (int f = 0; f < F; ++f) {
             const int j = j0 + tid + f * NT;
-            gg[f] = load_f(rgX, (j < j1 ? j : j0) * 4);
-            ys[f] = load_f3(rY, (mj[f] >= 0 ? mj[f] : 0) * 12);
+            gg[f] = load_grad(rgX, rdX, rtX, j < j1 ? j : j0);
+            ys[f] = load_point(rY, mj[f] >= 0 ? mj[f] : 0, ny);
         }
 #pragma unroll
         for (int f = 0; f < F; ++f) {
@@ -1653,10 +1699,11 @@ __global__ __launch_bounds__(NT) void chamfer_backward_fixed_kernel(
         const int64_t j = iY[i];
         if (j < j0 || j >= j1)
             continue;
-        const float g = gY[i] * 2;
+        const float g = load_grad(rgY, rdY, rtY, i) * 2;
+        const f3 y = load_point(rY, i, ny), x = load_point(rX, (int)j, nx);
 #pragma unroll
         for (int a = 0; a < 3; ++a)
-            atomicAdd(&facc[(j - j0) * 3 + a], -(g * (Y[(int64_t)i * 3 + a] - X[j * 3 + a])));
+            atomicAdd(&facc[(j - j0) * 3 + a], -(g * (y[a] - x[a])));
     }
     __syncthreads();
     for (int t = tid; t < (j1 - j0) * 3; t += NT) {
@@ -1664,7 +1711,7 @@ __global__ __launch_bounds__(NT) void chamfer_backward_fixed_kernel(
         const int64_t jm = iX[j];
         float o = 0.0f;
         if (jm >= 0 && jm < ny)
-            o = (gX[j] * 2) * (X[(int64_t)j * 3 + a] - Y[jm * 3 + a]);
+            o = (load_grad(rgX, rdX, rtX, j) * 2) * (load_point(rX, j, nx)[a] - load_point(rY, (int)jm, ny)[a]);
         out[(int64_t)j * 3 + a] = o + facc[t];
     }
 }
@@ -3953,10 +4000,10 @@ int chamfer_forward_sorted(const float *xyz1, const float *xyz2, int64_t B, int6
                                                   idx2, s, sa.flags);
 }
 
-template <typename T>
+template <typename T, bool SOA = false, bool ROOT = false>
 int chamfer_backward(const T *gd1, const T *gd2, const T *xyz1, const T *xyz2,
                      const int64_t *idx1, const int64_t *idx2, int64_t B, int64_t N1,
-                     int64_t N2, T *gx1, T *gx2, void *stream)
+                     int64_t N2, T *gx1, T *gx2, void *stream, const ChamferRootGrads &roots = {})
 {
     if (B < 0 || N1 < 0 || N2 < 0)
         return TK3D_ERR_BAD_SIZE;
@@ -3981,17 +4028,19 @@ int chamfer_backward(const T *gd1, const T *gd2, const T *xyz1, const T *xyz2,
             return TK3D_OK;
         // (the kernel addresses a cloud with 32-bit byte offsets: 12 bytes a point)
         if (B * (r1 + r2) <= TK_MAX_I32 && N1 <= (1 << 27) && N2 <= (1 << 27)) {
-            constexpr auto kernel = chamfer_backward_fixed_kernel<R, NT>;
+            constexpr auto kernel = chamfer_backward_fixed_kernel<R, NT, SOA, ROOT>;
             constexpr size_t lds = (size_t)R * 3 * (sizeof(unsigned long long) + sizeof(float));
             const int allowed = tk_allow_dynamic_lds<kernel>((int)lds);
             if (allowed != TK3D_OK)
                 return allowed;
             hipLaunchKernelGGL(kernel, dim3((unsigned)(B * (r1 + r2))), dim3(NT), lds, s, gd1,
                                gd2, xyz1, xyz2, idx1, idx2, (int)N1, (int)N2, (int)r1, (int)r2,
-                               gx1, gx2);
+                               gx1, gx2, roots);
             return tk_launch_status();
         }
     }
+    if constexpr (SOA || ROOT)
+        return TK3D_ERR_UNSUPPORTED;
     if ((t1 > 0 && !gx1) || (t2 > 0 && !gx2))
         return TK3D_ERR_UNSUPPORTED;  // (longer clouds than the kernel above takes: both or none)
     int64_t blocks = (t1 + t2 + 255) / 256;
@@ -4092,12 +4141,6 @@ __global__ __launch_bounds__(256) void chamfer_roots_kernel(const T *__restrict_
     if (i >= n)
         return;
     (i < n1 ? r1[i] : r2[i - n1]) = chamfer_root<T>(i < n1 ? d1[i] : d2[i - n1], eps);
-}
-
-template <typename T> __device__ __forceinline__ T chamfer_root_grad(T g, T d, T root, T eps)
-{
-    const T of_root = g / (root * 2);
-    return d >= eps ? of_root : (T)0;
 }
 
 template <typename T>
@@ -4399,6 +4442,25 @@ int tk3d_chamfer_roots_f32(const float *dist1, const float *dist2, int64_t n1, i
     hipLaunchKernelGGL((chamfer_roots_kernel<float>), dim3((unsigned)blocks), dim3(256), 0,
                        (hipStream_t)stream, dist1, dist2, n1, n1 + n2, (float)eps, root1, root2);
     return tk_launch_status();
+}
+
+int tk3d_chamfer_distance_backward_forms_f32(const float *grad1, const float *grad2, const float *xyz1,
+                                             const float *xyz2, const int64_t *idx1, const int64_t *idx2,
+                                             const float *dist1, const float *dist2, const float *root1,
+                                             const float *root2, double eps, int channels_first, int64_t B,
+                                             int64_t N1, int64_t N2, float *grad_xyz1, float *grad_xyz2,
+                                             void *stream)
+{
+    const bool roots = dist1 || dist2 || root1 || root2;
+    if (N1 > CHAMFER_FORMS_POINTS || N2 > CHAMFER_FORMS_POINTS)
+        return TK3D_ERR_UNSUPPORTED;
+    if (roots && ((B * N1 > 0 && (!dist1 || !root1)) || (B * N2 > 0 && (!dist2 || !root2))))
+        return TK3D_ERR_NULL_POINTER;
+    const ChamferRootGrads r{{dist1, dist2}, {root1, root2}, (float)eps};
+    const auto run = roots ? channels_first ? chamfer_backward<float, true, true> : chamfer_backward<float, false, true>
+                           : channels_first ? chamfer_backward<float, true, false>
+                                            : chamfer_backward<float, false, false>;
+    return run(grad1, grad2, xyz1, xyz2, idx1, idx2, B, N1, N2, grad_xyz1, grad_xyz2, stream, r);
 }
 
 int tk3d_chamfer_root_grads_f32(const float *grad1, const float *grad2, const float *dist1,

@@ -324,6 +324,60 @@ std::vector<Tensor> chamfer_backward(const Tensor &grad1, const Tensor &grad2, c
     return {grad_xyz1, grad_xyz2};
 }
 
+// The same of what the forward call leaves, in one launch: clouds of either layout, and gradients of the distances or
+// of their roots (`of` then holds both distances and both roots). False, with nothing launched, for what the kernel
+// does not take.
+bool chamfer_backward_forms(const Tensor &grad1, const Tensor &grad2, const Tensor &xyz1, const Tensor &xyz2,
+                            const Tensor &idx1, const Tensor &idx2, const Tensor *of, double eps,
+                            bool channels_first, Tensor *grad_xyz1, Tensor *grad_xyz2)
+{
+    if (!is_f32(xyz1))
+        return false;
+    check_contiguous_cuda("grad_dist1", grad1);
+    check_contiguous_cuda("grad_dist2", grad2);
+    check_contiguous_cuda("xyz1", xyz1);
+    check_contiguous_cuda("xyz2", xyz2);
+    check_contiguous_cuda("idx1", idx1);
+    check_contiguous_cuda("idx2", idx2);
+    check(grad1.dim() == 2 && grad2.dim() == 2, "grad_dist must be 2-D tensors.");
+    check(xyz1.dim() == 3 && xyz2.dim() == 3, "xyz1 and xyz2 must be 3-D tensors.");
+    const int64_t b = grad1.size(0), n1 = grad1.size(1), n2 = grad2.size(1);
+    const int64_t points = channels_first ? 2 : 1, coords = 3 - points;
+    check(grad2.size(0) == b && xyz1.size(0) == b && xyz2.size(0) == b, "grad_dist and clouds differ in batch size.");
+    check(xyz1.size(points) == n1 && xyz2.size(points) == n2, "grad_dist and clouds differ in points.");
+    check(xyz1.size(coords) == 3 && xyz2.size(coords) == 3, "clouds must have three coordinates.");
+    check(idx1.sizes() == grad1.sizes() && idx2.sizes() == grad2.sizes(), "idx and grad_dist differ in shape.");
+    check_index("idx1", idx1);
+    check_index("idx2", idx2);
+    check_same("grad_dist1", grad1, "xyz1", xyz1);
+    check_same("grad_dist2", grad2, "xyz2", xyz2);
+    check_same("xyz1", xyz1, "xyz2", xyz2);
+    for (int i = 0; of && i < 4; ++i) {
+        check_contiguous_cuda("dist", of[i]);
+        check_same("dist", of[i], "xyz1", xyz1);
+        check(of[i].sizes() == (i % 2 ? grad2 : grad1).sizes(), "distances and grad_dist differ in shape.");
+    }
+    OnDeviceOf guard(xyz1.device());
+    Tensor g1, g2;
+    if (grad_xyz1)
+        g1 = like(xyz1, {b, n1, 3});
+    if (grad_xyz2)
+        g2 = like(xyz2, {b, n2, 3});
+    const int rc = tk3d_chamfer_distance_backward_forms_f32(
+        (const float *)ptr(grad1), (const float *)ptr(grad2), (const float *)ptr(xyz1), (const float *)ptr(xyz2),
+        ptr(idx1), ptr(idx2), of ? (const float *)ptr(of[0]) : nullptr, of ? (const float *)ptr(of[1]) : nullptr,
+        of ? (const float *)ptr(of[2]) : nullptr, of ? (const float *)ptr(of[3]) : nullptr, eps, channels_first, b, n1,
+        n2, grad_xyz1 ? (float *)ptr(g1) : nullptr, grad_xyz2 ? (float *)ptr(g2) : nullptr, stream_of(xyz1));
+    if (rc == TK3D_ERR_UNSUPPORTED)
+        return false;
+    done(rc, "tk3d_chamfer_distance_backward_forms_f32");
+    if (grad_xyz1)
+        *grad_xyz1 = g1;
+    if (grad_xyz2)
+        *grad_xyz2 = g2;
+    return true;
+}
+
 // Like the reference (which goes through at::gather) non-contiguous tensors are accepted.
 Tensor group_forward(const Tensor &input_, const Tensor &index_)
 {
@@ -485,13 +539,26 @@ struct ChamferNode : torch::autograd::Function<ChamferNode> {
         Tensor g1 = grads[0].contiguous(), g2 = grads[1].contiguous();
         Tensor a = saved[0], c = saved[1];
         OnDeviceOf guard(a.device());
-        // (the backward kernel works on [B,N,3])
+        const double eps = saved.size() > 4 ? ctx->saved_data["eps"].toDouble() : 0.0;
+        const auto result = [&](std::vector<Tensor> g) {
+            for (int i = 0; i < 2; ++i) {
+                if (!(want & (1 << i)))
+                    g[i] = Tensor();
+                else if (channels_first)
+                    g[i] = g[i].transpose(1, 2);
+            }
+            return variable_list{g[0], g[1], Tensor(), Tensor(), Tensor()};
+        };
+        std::vector<Tensor> g(2);
+        if (chamfer_backward_forms(g1, g2, a, c, saved[2], saved[3], saved.size() > 4 ? &saved[4] : nullptr, eps,
+                                   channels_first, want & 1 ? &g[0] : nullptr, want & 2 ? &g[1] : nullptr))
+            return result(std::move(g));
+        // (the other backward kernels work on [B,N,3] and gradients of distances)
         const int64_t b = a.size(0), n1 = g1.size(1), n2 = g2.size(1);
         const Tensor a3 = channels_first ? like(a, {b, n1, 3}) : a;
         const Tensor c3 = channels_first ? like(c, {b, n2, 3}) : c;
         bool copied = !channels_first;
         if (saved.size() > 4) {
-            const double eps = ctx->saved_data["eps"].toDouble();
             const Tensor o1 = like(g1, g1.sizes()), o2 = like(g2, g2.sizes());
             if (channels_first && is_f32(a)) {
                 done(tk3d_chamfer_root_grads_rows_f32(ptr(g1), ptr(g2), ptr(saved[4]), ptr(saved[5]),
@@ -513,15 +580,7 @@ struct ChamferNode : torch::autograd::Function<ChamferNode> {
                       ptr(c3), stream_of(a));
         a = a3;
         c = c3;
-        std::vector<Tensor> g = chamfer_backward(g1, g2, a, c, saved[2], saved[3], (want & 1) != 0,
-                                                 (want & 2) != 0);
-        for (int i = 0; i < 2; ++i) {
-            if (!(want & (1 << i)))
-                g[i] = Tensor();
-            else if (channels_first)
-                g[i] = g[i].transpose(1, 2);
-        }
-        return {g[0], g[1], Tensor(), Tensor(), Tensor()};
+        return result(chamfer_backward(g1, g2, a, c, saved[2], saved[3], (want & 1) != 0, (want & 2) != 0));
     }
 };
 
