@@ -405,3 +405,23 @@ def test_whole_row_scatter_shapes_retries_and_bad_indices(cuda, b, c, n1, n2):
             np.testing.assert_allclose(got[bi, ci], want[bi, ci], rtol=RTOL, atol=top * 2.0 ** -40 + atol)
             got[bi, ci] = want[bi, ci]
         np.testing.assert_allclose(got, want, rtol=RTOL, atol=atol)
+
+
+@pytest.mark.parametrize("n1", [4160, 8383, 8385, 16384])  # two channels a workgroup up to 8384, then one
+@pytest.mark.parametrize("b,n2", [(1, 1), (2, 255), (2, 257), (3, 8192 + 511), (3, 8192 + 513)])
+def test_long_row_scatter_at_the_edges_of_its_chunks(cuda, n1, b, n2):
+    """Rows that leave room for one or two channels take chunks of eight and four points a lane: lengths around
+    one chunk and around one chunk for each of the sixteen waves, the last channel alone in its group. Whole
+    numbers make every sum exact, so the result equals torch's scatter_add; the largest term lies at the end, where
+    the first chunks, which set the scale, do not see it."""
+    from torkit3d_amd import _C
+
+    g = gen(n1 + n2)
+    c, k = 3, 2
+    index = torch.randint(0, n1, (b, n2, k), generator=g)
+    index[:, -1] = n1 - 1
+    grad = torch.randint(-3, 4, (b, c, n2, k), generator=g).float()
+    grad[:, 1, -1] = 4096.0
+    got = _C.group_points_backward_cuda(grad.to(cuda), index.to(cuda), n1).cpu()
+    want = torch.zeros(b, c, n1).scatter_add_(2, index.view(b, 1, -1).expand(b, c, -1), grad.view(b, c, -1))
+    assert torch.equal(got, want)

@@ -1208,6 +1208,18 @@ int scatter(const T *gout, const int64_t *idx, const T *w, int64_t B, int64_t C,
                                            (unsigned)gy, (unsigned)B);
                         return tk_launch_status();
                     };
+                    // Long rows leave room for one or two channels, and a wave then waits for its chunk rather
+                    // than for LDS: a longer chunk keeps as many loads on their way as four channels do. us, two
+                    // points a lane and now: 8 x 32 rows of 16384 (one channel, eight points) from 131072 points
+                    // 45.3 -> 35.2 (four points 38.4, twelve 35.7), 4 x 64 rows of 10000 from 160000 82.8 -> 72.6;
+                    // 16 x 16 rows of 6000 (two channels, four points) from 36000 21.1 -> 19.8. With four channels
+                    // it gives nothing: 8 x 64 rows of 4096 from 32768 37.4, four points 36.9; 16 x 64 68.2, 70.0.
+                    if constexpr (KK == 1) {
+                        if (!two && cg == 1)
+                            return launch(ScatterRowsKernel<KK, HAS_W, 1024, 1, 8>{}, 1024);
+                        if (!two && cg == 2)
+                            return launch(ScatterRowsKernel<KK, HAS_W, 1024, 2, 4>{}, 1024);
+                    }
                     if (two)
                         return launch(ScatterRowsKernel<KK, HAS_W, 512, 4, PTS>{}, 512);
                     return launch(ScatterRowsKernel<KK, HAS_W, 1024, 4, PTS>{}, 1024);
