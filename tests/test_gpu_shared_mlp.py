@@ -693,6 +693,17 @@ def test_edge_conv(cuda, b, c, n, k, o, lists, training):
         assert mine <= 4 * theirs + 2e-6, (i, tuple(e.shape), mine, theirs)
 
 
+# The sums over the edges whose value is the maximum, in LDS: rows around the 2048 points of a part, the last channel
+# alone in its workgroup of two, rows that fit LDS once but not twice, few rows just beyond those that are added there
+# (four neighbours: the fused training takes more than 512 edges of a cloud only in multiples of four).
+@pytest.mark.parametrize("b,c,n,k,o", [
+    (2, 4, 2047, 4, 5), (1, 4, 2049, 4, 6), (1, 3, 4096 + 511, 4, 3), (172, 3, 40, 3, 3), (104, 3, 2049, 4, 5),
+    (64, 3, 7168, 4, 8), (64, 3, 7169, 4, 8), (1, 3, 6144, 4, 6), (1, 3, 6145, 4, 6),
+])
+def test_edge_sums_of_maxima(cuda, b, c, n, k, o):
+    test_edge_conv(cuda, b, c, n, k, o, False, True)
+
+
 # On a graph of near neighbours, with the cloud at `far` from the origin: y taken apart into a term
 # of the neighbour and one of the point loses what their difference keeps, unless the products are more
 # exact than float32 (with float32 products the error of the activations was 1.1 to 1.7 times the stock

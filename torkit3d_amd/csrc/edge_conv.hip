@@ -20,6 +20,9 @@ constexpr int kChannels = 64;  // channels of a workgroup: a lane is a channel
 constexpr int kGather = 16;    // points of a workgroup that gathers in the backward: waves to hide trips
 constexpr int kRounded = 16;   // channels from which u and v may be rounded before they are added
 constexpr int kAtOnce = 8;     // rows requested before the first is used
+constexpr int kOwners = 512;   // lanes of a workgroup that adds what belongs to neighbours in LDS
+constexpr int kPart = 2048;    // its points at a time: every wave's run of 64 x kAtOnce within it
+constexpr int kOwnersLds = 144 * 1024;
 
 // The extreme of y = u_j + v_i over the neighbours.
 // A workgroup takes 32 points, a wave eight of them, a lane one of 64 output channels. Consecutive
@@ -293,6 +296,110 @@ __global__ void __launch_bounds__(kBlock)
             row[(int64_t)O * N] = dv[ch][p];
         }
     }
+}
+
+// The same from g, extreme and arg themselves: a workgroup has CH channels of a cloud, whose sums lie in LDS. kPart
+// points at a time, every lane finds the values of its points and the neighbours that they belong to; then one wave a
+// channel adds them, in the order of the points, so that every run adds in the same order. The two kernels above look
+// at all K edges into a point for the few that count, 8 bytes a channel of each, and pass 8 bytes a value through
+// memory; here a value looks up its one neighbour. 8 x 2048 points, 20 neighbours, 64 channels: 26.4 us in two launches,
+// now 10.5, most of it the trips to g, to the neighbours and through LDS, one behind the other; 128 channels 40.8, 14.
+// A step of DGCNN's training on them 74 us less.
+template <int CH>
+__global__ void __launch_bounds__(kOwners)
+    edge_owners_kernel(const float *__restrict__ g, const float *__restrict__ extreme,
+                       const unsigned char *__restrict__ arg, const int64_t *__restrict__ index, int B, int N, int K,
+                       int O, tk3d_mlp_norm norm, const float *__restrict__ coef, float *__restrict__ out)
+{
+    extern __shared__ double sums[];  // CH rows of N, then values and neighbours, CH rows of kPart each
+    float *values = reinterpret_cast<float *>(sums + CH * N);
+    int *owners = reinterpret_cast<int *>(values + CH * kPart);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int b = blockIdx.x % B, c0 = blockIdx.x / B * CH;
+    const int64_t *neighbours = index + (int64_t)b * N * K;
+    f32x4 ss[CH];
+    float a[CH];
+    int64_t row[CH];
+#pragma unroll
+    for (int ch = 0; ch < CH; ++ch) {
+        const int c = min(c0 + ch, O - 1);
+        ss[ch] = constants_of(norm, c);
+        a[ch] = coef[c * 4];
+        row[ch] = ((int64_t)b * O + c) * N;
+    }
+    for (int e = tid; e < CH * N; e += kOwners)
+        sums[e] = 0.0;
+    constexpr int STEPS = kPart / kOwners;
+    for (int from = 0; from < N; from += kPart) {
+        float y[STEPS][CH], gv[STEPS][CH];
+        int place[STEPS][CH];
+        int64_t j[STEPS][CH];
+#pragma unroll
+        for (int i = 0; i < STEPS; ++i) {
+            const int p = min(from + i * kOwners + tid, N - 1);
+#pragma unroll
+            for (int ch = 0; ch < CH; ++ch) {
+                place[i][ch] = arg[row[ch] + p];
+                y[i][ch] = extreme[row[ch] + p];
+                gv[i][ch] = g[row[ch] + p];
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < STEPS; ++i) {
+            const int p = min(from + i * kOwners + tid, N - 1);
+#pragma unroll
+            for (int ch = 0; ch < CH; ++ch)
+                j[i][ch] = neighbours[(int64_t)p * K + min(place[i][ch], K - 1)];
+        }
+#pragma unroll
+        for (int i = 0; i < STEPS; ++i) {
+            const int p = from + i * kOwners + tid;
+#pragma unroll
+            for (int ch = 0; ch < CH; ++ch) {
+                const float v = a[ch] * (passes(normalised(y[i][ch], ss[ch])) ? gv[i][ch] : 0.0f);
+                const bool counts = p < N && place[i][ch] < K && j[i][ch] >= 0 && j[i][ch] < N && v != 0.0f;
+                values[ch * kPart + i * kOwners + tid] = v;
+                owners[ch * kPart + i * kOwners + tid] = counts ? (int)j[i][ch] : -1;
+                if (p < N && c0 + ch < O)
+                    out[((int64_t)b * 2 * O + O + c0 + ch) * N + p] = v;
+            }
+        }
+        __syncthreads();
+        if (wave < CH)
+            for (int e0 = 0; e0 < min(kPart, N - from); e0 += 64 * kAtOnce) {
+                int to[kAtOnce];
+                float v[kAtOnce];
+#pragma unroll
+                for (int i = 0; i < kAtOnce; ++i) {
+                    to[i] = owners[wave * kPart + e0 + i * 64 + lane];
+                    v[i] = values[wave * kPart + e0 + i * 64 + lane];
+                }
+#pragma unroll
+                for (int i = 0; i < kAtOnce; ++i)
+                    if (to[i] >= 0)
+                        unsafeAtomicAdd(&sums[wave * N + to[i]], (double)v[i]);
+            }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int ch = 0; ch < CH; ++ch)
+        if (c0 + ch < O)
+            for (int p = tid; p < N; p += kOwners)
+                out[((int64_t)b * 2 * O + c0 + ch) * N + p] = (float)sums[ch * N + p];
+}
+
+int64_t owners_lds(int N, int channels) { return (int64_t)channels * (N * 8 + kPart * 8); }
+
+template <int CH>
+int edge_owners(const float *g, const float *extreme, const unsigned char *arg, const int64_t *index, int B, int N,
+                int K, int O, const tk3d_mlp_norm &norm, const float *coef, float *out, hipStream_t stream)
+{
+    const int rc = tk_allow_dynamic_lds<edge_owners_kernel<CH>>(kOwnersLds);
+    if (rc != TK3D_OK)
+        return rc;
+    edge_owners_kernel<CH><<<(O + CH - 1) / CH * B, kOwners, owners_lds(N, CH), stream>>>(g, extreme, arg, index, B,
+                                                                                         N, K, O, norm, coef, out);
+    return tk_launch_status();
 }
 
 // x [B, C, N] as rows of points [B, N, C].
@@ -854,9 +961,22 @@ int tk3d_mlp_edge_backward_f32(const float *g, const float *extreme, const unsig
     float *rows = duv + (int64_t)B * N * 2 * O, *st = rows + (int64_t)B * N * C;
     const int tiles = (N + kPoints - 1) / kPoints, blocks = (O + kChannels - 1) / kChannels;
     const int gathers = (N + kGather - 1) / kGather * B;
-    edge_select_kernel<<<dim3(tiles, blocks, B), kBlock, 0, stream>>>(g, extreme, arg, N, O, *norm, coef,
-                                                                    sel);
-    edge_sparse_kernel<<<dim3(gathers, blocks), kBlock, 0, stream>>>(sel, lists, B, N, K, O, duv);
+    int rc = TK3D_OK;
+    // Few long rows are better off gathered (us of the whole backward, gathered and owned, 64 -> 64 channels, one
+    // cloud of 16384 points 119.5, 128.1; of 8192 97.6, 98.1; of 6000 96.5, 93.0; of 2048 88.2, 77.2; 128 rows of
+    // 16384 182.3, 174.8), as are rows that LDS does not hold. Two channels of a workgroup share the lines of the
+    // neighbours, as long as that leaves every CU a workgroup (512 rows of 2048: 10.5 us, one channel 12.5).
+    const int64_t channels = (int64_t)B * O;
+    if (owners_lds(N, 1) <= kOwnersLds && (channels * 2 >= tk_cu_count() || N <= 3 * kPart)) {
+        const bool two = channels >= 2 * tk_cu_count() && owners_lds(N, 2) <= kOwnersLds;
+        rc = two ? edge_owners<2>(g, extreme, arg, index, B, N, K, O, *norm, coef, duv, stream)
+                 : edge_owners<1>(g, extreme, arg, index, B, N, K, O, *norm, coef, duv, stream);
+        if (rc != TK3D_OK)
+            return rc;
+    } else {
+        edge_select_kernel<<<dim3(tiles, blocks, B), kBlock, 0, stream>>>(g, extreme, arg, N, O, *norm, coef, sel);
+        edge_sparse_kernel<<<dim3(gathers, blocks), kBlock, 0, stream>>>(sel, lists, B, N, K, O, duv);
+    }
     edge_rows_kernel<<<dim3(tiles, (C + kChannels - 1) / kChannels, B), kBlock, 0, stream>>>(x, C, N, rows);
     if (C <= 4)
         edge_neighbours_kernel<4><<<dim3(gathers, 1), kBlock, 0, stream>>>(rows, index, lists, B, N, K, C, st);
@@ -867,7 +987,7 @@ int tk3d_mlp_edge_backward_f32(const float *g, const float *extreme, const unsig
         edge_neighbours_kernel<64><<<dim3(gathers, (C + 63) / 64), kBlock, 0, stream>>>(rows, index, lists,
                                                                                         B, N, K, C, st);
     const EdgeGradOp grad{{}, x, st, w, coef, norm->mean, lists, duv, C, O, K, half, 2 * half, N};
-    int rc = launch_product(grad, B, stream);
+    rc = launch_product(grad, B, stream);
     if (rc == TK3D_OK && dx) {
         const EdgeInputOp input{{}, duv, w, dx, O, C, N};
         rc = launch_product(input, B, stream);
