@@ -103,3 +103,22 @@ def test_launches_of_many_queries_keep_their_kernels(cuda, k, n2):
     q, c = cloud("uniform", 5, 2, 20000), cloud("lattice", 6, 2, n2)
     same(knn_points(torch.from_numpy(q).to(cuda), torch.from_numpy(c).to(cuda), k),
          oracle.knn(q, c, k))
+
+
+@pytest.mark.parametrize("b,n1,n2,k", [  # either side of the lines up to which a query has a wave
+    (18, 1024, 1024, 3), (18, 1025, 1024, 3), (100, 256, 1025, 8), (100, 257, 1025, 8),
+    (50, 512, 4096, 16), (40, 512, 4097, 16), (40, 513, 4097, 16), (50, 513, 4096, 16), (100, 256, 4097, 17), (100, 257, 4097, 17),
+    (48, 1024, 200, 33), (48, 1025, 200, 33), (128, 1024, 2047, 64), (128, 1024, 2048, 64), (128, 1025, 2048, 64)])
+def test_both_sides_of_the_limits(cuda, b, n1, n2, k):
+    """A batch as a whole and a few clouds of it at a time, which have a wave per query, agree bit for bit; some of
+    the distances are equal (coordinates in steps of 1/16)."""
+    from torkit3d_amd import _C
+
+    g = torch.Generator().manual_seed(b + n1 + n2)
+    query = (torch.rand(b, n1, 3, generator=g) * 16).round().div(16).to(cuda)
+    key = (torch.rand(b, n2, 3, generator=g) * 16).round().div(16).to(cuda)
+    distance, index = _C.knn_distance_cuda(query, key, k, 1)
+    few = max(1, 8192 // n1)
+    for i in (0, b // 2, b - few):
+        d, j = _C.knn_distance_cuda(query[i:i + few].contiguous(), key[i:i + few].contiguous(), k, 1)
+        assert torch.equal(distance[i:i + few], d) and torch.equal(index[i:i + few], j)

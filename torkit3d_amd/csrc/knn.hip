@@ -503,8 +503,8 @@ __device__ __forceinline__ double knn_max_f64(double a, double b)
 // clouds unless said otherwise: 32 x 8192 queries on 2048 keys k = 3 69.6, 54.9 (in clusters 68.1, 66.0), k = 8 83.2, 70.1, k = 16
 // 128, 114 (on a sphere 130, 113); 16 x 16384 on 4096 k = 3 103, 75; 4 x 16384 on 16384 k = 16 249, 204; 20 x 1000 on 16384
 // k = 8 232, 160; 1 x 40000 on 40000 k = 16 546, 498; 32 slots, whose waves' boxes are of 256 queries, 24 x 8192 on 2048 k = 32
-// 212, 203, 32 x 2048 on 8192 208, 211; on 64 to 512 keys 0.9 to 1.02 of the time before; clouds of 128 queries, which
-// two waves have anyway, up to 1.12.
+// 212, 203, 32 x 2048 on 8192 208, 211; on 64 to 512 keys 0.9 to 1.02 of the time before; clouds of up to 128 queries,
+// which two waves have anyway, 0.9 where there are more of them than CUs, else up to 1.12.
 constexpr int knn_max4(int a, int b, int c, int d)
 {
     const int ab = a > b ? a : b, cd = c > d ? c : d;
@@ -1594,15 +1594,21 @@ __global__ __launch_bounds__(KNN_BLOCK, LONG ? 1 : 8) void knn_wave_kernel_f32(
 }
 
 // Where a wave per query wins: its time goes with the number of queries, that of the kernels of a lane per query hardly
-// does while they leave CUs idle. At the limits, 18432 queries, and 36864 with more than 32 neighbours, which the
-// others keep in a tree in LDS, it is the faster one throughout. us, it and the pre-filtered kernel, 18432 queries: on
-// 64 keys k = 3 9.7, 11.6, k = 8 12.7, 14.0, k = 16 15.6, 18.8, k = 32 16.6, 30.1; on 512 k = 3 14.8, 19.0, k = 8 22.1,
-// 24.0, k = 16 32.0, 34.6, k = 32 45.8, 64.0; on 16384 k = 3 152, 211, k = 16 171, 244, k = 32 197, 307. With the tree,
-// 36864 queries: on 64 keys k = 64 10.7, 37, on 16384 492, 1570. (Up to k = 16 the two are even at 20000 to 24000
-// queries, at 32 at 32000 to 40000.)
-inline bool knn_wave_pays(int64_t queries, int k)
+// does while they leave CUs idle. us, it and the pre-filtered kernel, 20480 queries in clouds of 4096: on 128 keys k = 3 12.0,
+// 13.6, k = 8 16.8, 16.3, k = 16 21.7, 21.6, k = 32 28.0, 33.1; on 1024 k = 3 17.8, 25.8, k = 16 38.6, 47.0, k = 32 58, 78;
+// on 16384 k = 3 147, 151, k = 16 153, 193, k = 32 164, 327. 24576 queries: on 128 keys k = 16 23.8, 22.6, k = 32 30.7, 34.5;
+// on 1024 k = 3 20.4, 26.2, k = 16 44.6, 46.3; on 4096 k = 3 49, 49, k = 16 71, 90; on 16384 k = 3 174, 153, k = 32 192, 325.
+// 25600 in clouds of 128, on 2048 keys k = 3 29.1, 38.5, k = 16 56.9, 62.3. 32768: on 128 k = 3 15.9, 12.6, on 4096 k = 3
+// 64.5, 52.7, k = 16 91, 91. With more than 32 neighbours the others keep a tree in LDS: 49152 queries on 128 keys k = 64 59,
+// 72, on 4096 301, 549; 65536 on 1024 253, 243; 131072 on 128 k = 40 146, 136, on 4096 k = 40 570, 985, k = 64 771, 1143.
+// Keys in the order of a coordinate, of which many more are inserted, take more of both and leave the order as it is (20480
+// queries on 16384 keys k = 3 214, 348, 98304 on 4096 k = 64 1208, 1979). On 1024 keys and fewer, up to 16 neighbours, the two
+// are close from 18432 queries on (on 512 k = 8 22.1, 24.0).
+inline bool knn_wave_pays(int64_t queries, int64_t keys, int k)
 {
-    return k <= 64 && queries <= (k <= 32 ? 18432 : 36864);
+    if (k > 32)
+        return k <= 64 && queries <= (keys >= 2048 ? 131072 : 49152);
+    return queries <= (keys <= 1024 ? 18432 : k <= 16 && keys > 4096 ? 20480 : 25600);
 }
 
 template <bool SOA, bool WEIGHTS>
@@ -1748,14 +1754,16 @@ int knn_filter_launch(const float *query, const float *key, float *distance, int
 {
     // 512 lanes: two workgroups (16 waves) per CU. A launch of few such workgroups leaves CUs
     // without one: 256 lanes then, unless there are keys enough for the boxes of 512 sorted queries to pay (us, 256 and 512
-    // lanes: 5 x 4096 queries on 512 keys k = 8 24.4, 28.0, 8 x 4096 on 1024 k = 3 26.2, 25.3, 2 x 16384 on 4096 k = 3 64, 49,
-    // 5 x 5000 on 1024 k = 16 46.5, 52.8, 3 x 8192 on 16384 k = 16 256, 191). 32 slots leave room for three waves per
+    // lanes: 8 x 4096 queries on 1024 keys k = 8 32.9, 34.8, on 2048 k = 3 39.0, 33.9, k = 16 62.9, 69.1, on 8192 k = 3 114, 78,
+    // k = 16 155, 129, 12 x 4096 on 4096 k = 8 76.4, 66.2, 2 x 16384 on 4096 k = 3 63, 50, 3 x 10000 on 16384 k = 16 280, 196;
+    // keys in the order of a coordinate, of which each is inserted, take fewer waves a SIMD better, 8 x 4096 on 8192 k = 16 342,
+    // 396, as before the boxes, 317). 32 slots leave room for three waves per
     // SIMD, twelve a CU: three workgroups of 256 lanes or one of 512.
     if (!(whatever_the_size || knn_filter_takes(B, n1, n2, k)))
         return TK3D_ERR_UNSUPPORTED;
     if constexpr (KMAX <= 16) {
         const int64_t bpb = ((int64_t)n1 + 511) / 512;
-        if (B * bpb > (KMAX <= 8 ? 128 : 160) || n2 >= (KMAX <= 8 ? 1024 : 2048))
+        if (B * bpb > (KMAX <= 8 ? 128 : 160) || n2 >= 512 * KMAX)
             return knn_filter_launch_as<KMAX, SOA, WEIGHTS, 512>(query, key, distance, index, weight,
                                                                  eps, B, n1, n2, k, s);
     }
@@ -1841,7 +1849,7 @@ int knn(const T *query, const T *key, int64_t B, int64_t N1, int64_t N2, int64_t
     hipStream_t s = (hipStream_t)stream;
     const int n1 = (int)N1, n2 = (int)N2, kk = (int)k;
     if constexpr (sizeof(T) == 4) {
-        if (knn_wave_pays(B * N1, kk))
+        if (knn_wave_pays(B * N1, N2, kk))
             return knn_wave_launch<false, false>(query, key, distance, index, nullptr, 0.0f, B, n1,
                                                  n2, kk, 0, 0, s);
     }
@@ -1939,7 +1947,7 @@ int knn_bcn(const T *query, const T *key, int64_t B, int64_t N1, int64_t N2, int
         return TK3D_ERR_NULL_POINTER;
     hipStream_t s = (hipStream_t)stream;
     if constexpr (sizeof(T) == 4) {
-        if (knn_wave_pays(B * N1, kk))
+        if (knn_wave_pays(B * N1, N2, kk))
             return knn_wave_launch<true, false>(query, key, distance, index, nullptr, 0.0f, B, n1, n2,
                                                 kk, 0, 0, s);
         if (k > 4 && !knn_filter_takes(B, n1, n2, kk)) {
@@ -1996,7 +2004,7 @@ int knn_ordered(const T *query, const T *key, bool channels_first, int64_t B, in
     if constexpr (sizeof(T) == 4) {
         if (B > 0 && N1 > 0 && k > 0 && k <= N2 && query && key && distance && index &&
             N1 <= TK_MAX_I32 / 4 && N2 <= TK_MAX_I32 / 4 && tk_fits(TK_MAX_ELEMS, B, N2, 3) &&
-            knn_wave_pays(B * N1, (int)k)) {
+            knn_wave_pays(B * N1, N2, (int)k)) {
             const auto launch = channels_first ? knn_wave_launch<true, false> : knn_wave_launch<false, false>;
             return launch(query, key, distance, index, nullptr, 0.0f, B, (int)N1, (int)N2, (int)k,
                           sorted, root, (hipStream_t)stream);
@@ -2030,7 +2038,7 @@ int three_nn(const T *query, const T *key, bool channels_first, int64_t B, int64
         return TK3D_ERR_UNSUPPORTED;
     hipStream_t s = (hipStream_t)stream;
     if constexpr (sizeof(T) == 4) {
-        if (knn_wave_pays(B * N1, 3)) {
+        if (knn_wave_pays(B * N1, N2, 3)) {
             const auto launch = channels_first ? knn_wave_launch<true, true> : knn_wave_launch<false, true>;
             return launch(query, key, distance, index, weight, (float)eps, B, (int)N1, (int)N2, 3, 0, 0,
                           s);
