@@ -239,7 +239,9 @@ def test_products_of_shared_tiles(cuda, monkeypatch, b, p, widths, pool, trainin
     if not training:  # infinities and NaN stay where they are
         x[0, 0, 0], x[-1, -1, -1] = float("inf"), float("nan")
         with torch.no_grad():
-            got, want = fused(mlp, x), reference(stock(mlp, torch.float32), x)
+            # (on the CPU: of the convolutions that the library picks between, some mix neighbouring positions,
+            # and a NaN then reaches those of a whole tile)
+            got, want = fused(mlp, x).cpu(), reference(stock(mlp, torch.float32).cpu(), x.cpu())
         assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
 
 
