@@ -105,3 +105,18 @@ def test_backward_of_planes_and_roots_with_infinite_gradients(cuda):
     # (the distances' gradients agree to the bit; sums of the same float32 terms in another order: a few of them a point)
     for g, w in zip(got, want):
         torch.testing.assert_close(g.transpose(1, 2), w, rtol=1e-5, atol=1e-5, equal_nan=True)
+
+
+@pytest.mark.parametrize("transpose,sqrt,more", [(False, False, 0), (True, False, 2), (False, True, 2), (True, True, 4)])
+@pytest.mark.parametrize("n1,n2", [(300, 700), (8193, 600)])
+def test_backward_allocates_no_more_than_it_needs(cuda, n1, n2, transpose, sqrt, more):
+    """Both gradients, and the copies of planes and the gradients of distances only where launches of their own
+    make them: what is allocated for a path that is then not taken is host time of every call."""
+    x, y = [(t.transpose(1, 2) if transpose else t).contiguous().to(cuda).requires_grad_() for t in clouds(1, n1, n2)]
+    grads = [torch.randn(1, n, device=cuda) for n in (n1, n2)]
+    out = chamfer_distance(x, y, transpose=transpose, sqrt=sqrt)
+    torch.autograd.grad(out, (x, y), grads, retain_graph=True)
+    before = torch.cuda.memory_stats()["allocation.all.allocated"]
+    result = torch.autograd.grad(out, (x, y), grads, retain_graph=True)
+    taken = torch.cuda.memory_stats()["allocation.all.allocated"] - before
+    assert len(result) == 2 and taken == 2 + (more if n1 > 8192 else 0)

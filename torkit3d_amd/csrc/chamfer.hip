@@ -4444,6 +4444,11 @@ int tk3d_chamfer_roots_f32(const float *dist1, const float *dist2, int64_t n1, i
     return tk_launch_status();
 }
 
+int tk3d_chamfer_distance_backward_takes_forms(int64_t N1, int64_t N2)
+{
+    return N1 <= CHAMFER_FORMS_POINTS && N2 <= CHAMFER_FORMS_POINTS;
+}
+
 int tk3d_chamfer_distance_backward_forms_f32(const float *grad1, const float *grad2, const float *xyz1,
                                              const float *xyz2, const int64_t *idx1, const int64_t *idx2,
                                              const float *dist1, const float *dist2, const float *root1,
@@ -4452,7 +4457,7 @@ int tk3d_chamfer_distance_backward_forms_f32(const float *grad1, const float *gr
                                              void *stream)
 {
     const bool roots = dist1 || dist2 || root1 || root2;
-    if (N1 > CHAMFER_FORMS_POINTS || N2 > CHAMFER_FORMS_POINTS)
+    if (!tk3d_chamfer_distance_backward_takes_forms(N1, N2))
         return TK3D_ERR_UNSUPPORTED;
     if (roots && ((B * N1 > 0 && (!dist1 || !root1)) || (B * N2 > 0 && (!dist2 || !root2))))
         return TK3D_ERR_NULL_POINTER;

@@ -325,14 +325,12 @@ std::vector<Tensor> chamfer_backward(const Tensor &grad1, const Tensor &grad2, c
 }
 
 // The same of what the forward call leaves, in one launch: clouds of either layout, and gradients of the distances or
-// of their roots (`of` then holds both distances and both roots). False, with nothing launched, for what the kernel
-// does not take.
-bool chamfer_backward_forms(const Tensor &grad1, const Tensor &grad2, const Tensor &xyz1, const Tensor &xyz2,
-                            const Tensor &idx1, const Tensor &idx2, const Tensor *of, double eps,
-                            bool channels_first, Tensor *grad_xyz1, Tensor *grad_xyz2)
+// of their roots (`of` then holds both distances and both roots). float32, sizes that
+// tk3d_chamfer_distance_backward_takes_forms() names.
+std::vector<Tensor> chamfer_backward_forms(const Tensor &grad1, const Tensor &grad2, const Tensor &xyz1,
+                                           const Tensor &xyz2, const Tensor &idx1, const Tensor &idx2,
+                                           const Tensor *of, double eps, bool channels_first, bool want1, bool want2)
 {
-    if (!is_f32(xyz1))
-        return false;
     check_contiguous_cuda("grad_dist1", grad1);
     check_contiguous_cuda("grad_dist2", grad2);
     check_contiguous_cuda("xyz1", xyz1);
@@ -358,24 +356,17 @@ bool chamfer_backward_forms(const Tensor &grad1, const Tensor &grad2, const Tens
         check(of[i].sizes() == (i % 2 ? grad2 : grad1).sizes(), "distances and grad_dist differ in shape.");
     }
     OnDeviceOf guard(xyz1.device());
-    Tensor g1, g2;
-    if (grad_xyz1)
-        g1 = like(xyz1, {b, n1, 3});
-    if (grad_xyz2)
-        g2 = like(xyz2, {b, n2, 3});
-    const int rc = tk3d_chamfer_distance_backward_forms_f32(
-        (const float *)ptr(grad1), (const float *)ptr(grad2), (const float *)ptr(xyz1), (const float *)ptr(xyz2),
-        ptr(idx1), ptr(idx2), of ? (const float *)ptr(of[0]) : nullptr, of ? (const float *)ptr(of[1]) : nullptr,
-        of ? (const float *)ptr(of[2]) : nullptr, of ? (const float *)ptr(of[3]) : nullptr, eps, channels_first, b, n1,
-        n2, grad_xyz1 ? (float *)ptr(g1) : nullptr, grad_xyz2 ? (float *)ptr(g2) : nullptr, stream_of(xyz1));
-    if (rc == TK3D_ERR_UNSUPPORTED)
-        return false;
-    done(rc, "tk3d_chamfer_distance_backward_forms_f32");
-    if (grad_xyz1)
-        *grad_xyz1 = g1;
-    if (grad_xyz2)
-        *grad_xyz2 = g2;
-    return true;
+    Tensor grad_xyz1, grad_xyz2;
+    if (want1)
+        grad_xyz1 = like(xyz1, {b, n1, 3});
+    if (want2)
+        grad_xyz2 = like(xyz2, {b, n2, 3});
+    done(tk3d_chamfer_distance_backward_forms_f32(
+             ptr(grad1), ptr(grad2), ptr(xyz1), ptr(xyz2), ptr(idx1), ptr(idx2), of ? ptr(of[0]) : Ptr{},
+             of ? ptr(of[1]) : Ptr{}, of ? ptr(of[2]) : Ptr{}, of ? ptr(of[3]) : Ptr{}, eps, channels_first, b, n1, n2,
+             ptr(grad_xyz1), ptr(grad_xyz2), stream_of(xyz1)),
+         "tk3d_chamfer_distance_backward_forms_f32");
+    return {grad_xyz1, grad_xyz2};
 }
 
 // Like the reference (which goes through at::gather) non-contiguous tensors are accepted.
@@ -539,7 +530,8 @@ struct ChamferNode : torch::autograd::Function<ChamferNode> {
         Tensor g1 = grads[0].contiguous(), g2 = grads[1].contiguous();
         Tensor a = saved[0], c = saved[1];
         OnDeviceOf guard(a.device());
-        const double eps = saved.size() > 4 ? ctx->saved_data["eps"].toDouble() : 0.0;
+        const bool roots = saved.size() > 4, want1 = (want & 1) != 0, want2 = (want & 2) != 0;
+        const double eps = roots ? ctx->saved_data["eps"].toDouble() : 0.0;
         const auto result = [&](std::vector<Tensor> g) {
             for (int i = 0; i < 2; ++i) {
                 if (!(want & (1 << i)))
@@ -549,16 +541,16 @@ struct ChamferNode : torch::autograd::Function<ChamferNode> {
             }
             return variable_list{g[0], g[1], Tensor(), Tensor(), Tensor()};
         };
-        std::vector<Tensor> g(2);
-        if (chamfer_backward_forms(g1, g2, a, c, saved[2], saved[3], saved.size() > 4 ? &saved[4] : nullptr, eps,
-                                   channels_first, want & 1 ? &g[0] : nullptr, want & 2 ? &g[1] : nullptr))
-            return result(std::move(g));
-        // (the other backward kernels work on [B,N,3] and gradients of distances)
         const int64_t b = a.size(0), n1 = g1.size(1), n2 = g2.size(1);
+        // (asked before anything is allocated: a call on few long clouds takes as long as its host work)
+        if (is_f32(a) && (channels_first || roots) && tk3d_chamfer_distance_backward_takes_forms(n1, n2))
+            return result(chamfer_backward_forms(g1, g2, a, c, saved[2], saved[3], roots ? &saved[4] : nullptr, eps,
+                                                 channels_first, want1, want2));
+        // (the other backward kernels work on [B,N,3] and gradients of distances)
         const Tensor a3 = channels_first ? like(a, {b, n1, 3}) : a;
         const Tensor c3 = channels_first ? like(c, {b, n2, 3}) : c;
         bool copied = !channels_first;
-        if (saved.size() > 4) {
+        if (roots) {
             const Tensor o1 = like(g1, g1.sizes()), o2 = like(g2, g2.sizes());
             if (channels_first && is_f32(a)) {
                 done(tk3d_chamfer_root_grads_rows_f32(ptr(g1), ptr(g2), ptr(saved[4]), ptr(saved[5]),
@@ -580,7 +572,7 @@ struct ChamferNode : torch::autograd::Function<ChamferNode> {
                       ptr(c3), stream_of(a));
         a = a3;
         c = c3;
-        return result(chamfer_backward(g1, g2, a, c, saved[2], saved[3], (want & 1) != 0, (want & 2) != 0));
+        return result(chamfer_backward(g1, g2, a, c, saved[2], saved[3], want1, want2));
     }
 };
 
