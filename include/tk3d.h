@@ -178,10 +178,10 @@ int tk3d_chamfer_distance_backward_f64(const double *grad_dist1,
 
 /* The same from what the forward calls leave: clouds as [B,N,3] or, channels_first, [B,3,N] (the gradients are [B,N,3]
  * in either case), and gradients of the distances or, with dist1 .. root2 not NULL, of their roots (as
- * tk3d_chamfer_root_grads_f32 takes them). TK3D_ERR_UNSUPPORTED, with nothing launched, beyond 8192 points a cloud,
- * where copies and gradients of the roots by launches of their own take less: tk3d_chamfer_distance_backward_takes_forms()
- * says whether it takes the sizes. */
-int tk3d_chamfer_distance_backward_takes_forms(int64_t N1, int64_t N2);
+ * tk3d_chamfer_root_grads_f32 takes them). TK3D_ERR_UNSUPPORTED, with nothing launched, where copies and gradients of
+ * the roots by launches of their own take less time on the GPU: beyond 8192 points a cloud, and roots of [B,3,N] clouds of
+ * more than 4096 points both. tk3d_chamfer_distance_backward_takes_forms() says whether it takes a call. */
+int tk3d_chamfer_distance_backward_takes_forms(int channels_first, int roots, int64_t N1, int64_t N2);
 int tk3d_chamfer_distance_backward_forms_f32(const float *grad1, const float *grad2, const float *xyz1,
                                              const float *xyz2, const int64_t *idx1, const int64_t *idx2,
                                              const float *dist1, const float *dist2, const float *root1,

@@ -212,6 +212,14 @@ pointer, i32 = ctypes.c_void_p, ctypes.c_int32
 IN_RAW, IN_GRAD, OUT_PLAIN, OUT_EVAL, OUT_MASK = 0, 3, 1, 3, 6
 
 
+@pytest.mark.parametrize("planes,roots,n1,n2,taken", [
+    (1, 0, 8192, 8192, True), (1, 0, 8193, 5, False), (0, 1, 8192, 8192, True), (0, 1, 5, 8193, False),
+    (1, 1, 8192, 4096, True), (1, 1, 4096, 8192, True), (1, 1, 4097, 4097, False), (1, 1, 8193, 1, False)])
+def test_chamfer_backward_reads_planes_and_roots_where_it_pays(lib, planes, roots, n1, n2, taken):
+    args = [ctypes.c_int(planes), ctypes.c_int(roots), ctypes.c_int64(n1), ctypes.c_int64(n2)]
+    assert bool(lib.tk3d_chamfer_distance_backward_takes_forms(*args)) is taken
+
+
 class Source(ctypes.Structure):
     _fields_ = [(n, pointer) for n in ("x", "y", "coef", "w")] + [("batch_stride", ctypes.c_int64)] + [
         (n, i32) for n in ("K", "wk", "wc")]

@@ -1332,12 +1332,20 @@ template <typename T> __device__ __forceinline__ T chamfer_root_grad(T g, T d, T
     return d >= eps ? of_root : (T)0;
 }
 
-// Up to two ranges a cloud: every range reads what it is sent anew, roots and distances as well, and points at random
-// places from three planes. (Kernels of a backward call in us, [B,3,N] with roots, with launches in front that copy the
-// clouds to rows and form the gradients, and without: 8 x 2500 x 3001 10.6 + 2.7, 13.5, and 4 to 7 us less of the
-// host's time; without roots 32 x 2048 x 2048 9.9 + 3.0, 10.8, 16 x 8192 x 8192 13.0 + 3.9, 17.6; 32 x 16384 x 16384 21.1 +
-// 9.0, 39.2, without roots 21.1 + 8.7, 31.0.)
-constexpr int64_t CHAMFER_FORMS_POINTS = 8192;
+// Every range reads what it is sent anew, roots and distances as well, and points at random places from three planes:
+// where that takes longer than launches in front that copy the clouds to rows and form the gradients, these stay. Kernels
+// of a backward call in us, with launches in front and without: planes and roots 8 x 2500 x 3001 12.9, 11.6, 8 x 4096 x 4096
+// 14.6, 13.5, 32 x 8192 x 1024 16.0, 14.0, 8 x 8192 x 4096 16.1, 16.5, but 8 x 6000 x 5000 15.5, 17.3, 16 x 8192 x 8192 18.3,
+// 20.3; planes 32 x 2048 x 2048 12.7, 10.7, 32 x 5000 x 5000 16.3, 15.5, 8 x 6000 x 5000 14.5, 15.5, 16 x 8192 x 8192 16.8,
+// 17.8, 64 x 8192 x 8192 25.7, 23.6; roots 8 x 2500 x 3001 12.5, 10.2, 16 x 8192 x 8192 16.5, 16.2. Of the host's time go 4 to
+// 7 us. 32 x 16384 x 16384, planes and roots 30.1, 39.2, planes 29.8, 31.0.
+constexpr int64_t CHAMFER_FORMS_POINTS = 8192, CHAMFER_BOTH_FORMS_POINTS = 4096;
+
+inline bool chamfer_takes_forms(bool planes, bool roots, int64_t N1, int64_t N2)
+{
+    const int64_t most = N1 > N2 ? N1 : N2, least = N1 > N2 ? N2 : N1;
+    return most <= CHAMFER_FORMS_POINTS && (!(planes && roots) || least <= CHAMFER_BOTH_FORMS_POINTS);
+}
 
 struct ChamferRootGrads {
     const float *dist[2], *root[2];
@@ -1443,14 +1451,21 @@ __global__ __launch_bounds__(NT) void chamfer_backward_fixed_kernel(
     // Sender u of a lane in round `round`: runs of NT consecutive senders, the rounds
     // interleaved so that each of them is spread over the whole cloud.
     auto sender = [&](int round, int u) { return tid + NT * (u * rounds + round); };
+    // Whether a run has senders at all (uniform). Not asked, a division and up to six loads for each of those that do not
+    // exist make roots slower here than behind launches in front (8 x 4096 x 4096, planes, 15.5 us, now 13.5); the
+    // loads alone are as fast without the question.
+    auto run_exists = [&](int round, int u) { return !ROOT || NT * (u * rounds + round) < ny; };
     // A sender's match as a position within the range, -1 when it lies outside.
     auto load_matches = [&](int round, int (&jj)[U]) {
         int64_t m64[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int i = sender(round, u);
-            m64[u] = load_i64(riY, (i < ny ? i : 0) * 8);
-            m64[u] = i < ny ? m64[u] : -1;
+            m64[u] = -1;
+            if (run_exists(round, u)) {
+                m64[u] = load_i64(riY, (i < ny ? i : 0) * 8);
+                m64[u] = i < ny ? m64[u] : -1;
+            }
         }
 #pragma unroll
         for (int u = 0; u < U; ++u)
@@ -1468,8 +1483,12 @@ __global__ __launch_bounds__(NT) void chamfer_backward_fixed_kernel(
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int is = jj[u] >= 0 ? sender(round, u) : 0;
-            g[u] = load_grad(rgY, rdY, rtY, is) * 2;
-            y[u] = load_point(rY, is, ny);
+            g[u] = 0.0f;
+            y[u] = f3{0.0f, 0.0f, 0.0f};
+            if (run_exists(round, u)) {
+                g[u] = load_grad(rgY, rdY, rtY, is) * 2;
+                y[u] = load_point(rY, is, ny);
+            }
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -4444,9 +4463,9 @@ int tk3d_chamfer_roots_f32(const float *dist1, const float *dist2, int64_t n1, i
     return tk_launch_status();
 }
 
-int tk3d_chamfer_distance_backward_takes_forms(int64_t N1, int64_t N2)
+int tk3d_chamfer_distance_backward_takes_forms(int channels_first, int roots, int64_t N1, int64_t N2)
 {
-    return N1 <= CHAMFER_FORMS_POINTS && N2 <= CHAMFER_FORMS_POINTS;
+    return chamfer_takes_forms(channels_first != 0, roots != 0, N1, N2);
 }
 
 int tk3d_chamfer_distance_backward_forms_f32(const float *grad1, const float *grad2, const float *xyz1,
@@ -4457,7 +4476,7 @@ int tk3d_chamfer_distance_backward_forms_f32(const float *grad1, const float *gr
                                              void *stream)
 {
     const bool roots = dist1 || dist2 || root1 || root2;
-    if (!tk3d_chamfer_distance_backward_takes_forms(N1, N2))
+    if (!chamfer_takes_forms(channels_first != 0, roots, N1, N2))
         return TK3D_ERR_UNSUPPORTED;
     if (roots && ((B * N1 > 0 && (!dist1 || !root1)) || (B * N2 > 0 && (!dist2 || !root2))))
         return TK3D_ERR_NULL_POINTER;

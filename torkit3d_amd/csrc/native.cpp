@@ -280,9 +280,8 @@ std::vector<Tensor> chamfer_forward(const Tensor &xyz1, const Tensor &xyz2, bool
     return {dist1, idx1, dist2, idx2};
 }
 
-std::vector<Tensor> chamfer_backward(const Tensor &grad1, const Tensor &grad2, const Tensor &xyz1,
-                                     const Tensor &xyz2, const Tensor &idx1, const Tensor &idx2,
-                                     bool want1 = true, bool want2 = true)
+void check_chamfer_backward(const Tensor &grad1, const Tensor &grad2, const Tensor &xyz1, const Tensor &xyz2,
+                            const Tensor &idx1, const Tensor &idx2, bool channels_first = false)
 {
     check_contiguous_cuda("grad_dist1", grad1);
     check_contiguous_cuda("grad_dist2", grad2);
@@ -296,10 +295,17 @@ std::vector<Tensor> chamfer_backward(const Tensor &grad1, const Tensor &grad2, c
     check(xyz1.dim() == 3 && xyz2.dim() == 3, "xyz1 and xyz2 must be 3-D tensors.");
     check_eq(xyz1.size(0), b, "xyz1.size(0) == bs");
     check_eq(xyz2.size(0), b, "xyz2.size(0) == bs");
-    check_eq(xyz1.size(1), n1, "xyz1.size(1) == n1");
-    check_eq(xyz2.size(1), n2, "xyz2.size(1) == n2");
-    check_eq(xyz1.size(2), 3, "xyz1.size(2) == 3");
-    check_eq(xyz2.size(2), 3, "xyz2.size(2) == 3");
+    if (channels_first) {
+        check_eq(xyz1.size(2), n1, "xyz1.size(2) == n1");
+        check_eq(xyz2.size(2), n2, "xyz2.size(2) == n2");
+        check_eq(xyz1.size(1), 3, "xyz1.size(1) == 3");
+        check_eq(xyz2.size(1), 3, "xyz2.size(1) == 3");
+    } else {
+        check_eq(xyz1.size(1), n1, "xyz1.size(1) == n1");
+        check_eq(xyz2.size(1), n2, "xyz2.size(1) == n2");
+        check_eq(xyz1.size(2), 3, "xyz1.size(2) == 3");
+        check_eq(xyz2.size(2), 3, "xyz2.size(2) == 3");
+    }
     check(idx1.dim() == 2 && idx2.dim() == 2, "idx1 and idx2 must be 2-D tensors.");
     check_eq(idx1.size(0), b, "idx1.size(0) == bs");
     check_eq(idx2.size(0), b, "idx2.size(0) == bs");
@@ -310,63 +316,95 @@ std::vector<Tensor> chamfer_backward(const Tensor &grad1, const Tensor &grad2, c
     check_same("grad_dist1", grad1, "xyz1", xyz1);
     check_same("grad_dist2", grad2, "xyz2", xyz2);
     check_same("xyz1", xyz1, "xyz2", xyz2);
-    OnDeviceOf guard(xyz1.device());
-    if (!is_f32(xyz1) || std::max(n1, n2) > (1 << 27))
+}
+
+// The gradients from clouds [B,N,3] and gradients of distances at `x` and `grad`; `xyz` says type and device.
+std::vector<Tensor> chamfer_gradients(const Tensor &xyz, int64_t b, const int64_t (&n)[2], const Ptr (&grad)[2],
+                                      const Ptr (&x)[2], const Tensor &idx1, const Tensor &idx2, bool want1, bool want2)
+{
+    if (!is_f32(xyz) || std::max(n[0], n[1]) > (1 << 27))
         want1 = want2 = true;  // (one gradient alone: the fp32 kernel)
     Tensor grad_xyz1, grad_xyz2;
     if (want1)
-        grad_xyz1 = like(xyz1, {b, n1, 3});
+        grad_xyz1 = like(xyz, {b, n[0], 3});
     if (want2)
-        grad_xyz2 = like(xyz1, {b, n2, 3});
-    TK3D_CALL(is_f32(xyz1), tk3d_chamfer_distance_backward, ptr(grad1), ptr(grad2), ptr(xyz1),
-              ptr(xyz2), ptr(idx1), ptr(idx2), b, n1, n2, ptr(grad_xyz1), ptr(grad_xyz2),
-              stream_of(xyz1));
+        grad_xyz2 = like(xyz, {b, n[1], 3});
+    TK3D_CALL(is_f32(xyz), tk3d_chamfer_distance_backward, grad[0], grad[1], x[0], x[1], ptr(idx1), ptr(idx2), b,
+              n[0], n[1], ptr(grad_xyz1), ptr(grad_xyz2), stream_of(xyz));
     return {grad_xyz1, grad_xyz2};
 }
 
-// The same of what the forward call leaves, in one launch: clouds of either layout, and gradients of the distances or
-// of their roots (`of` then holds both distances and both roots). float32, sizes that
-// tk3d_chamfer_distance_backward_takes_forms() names.
+std::vector<Tensor> chamfer_backward(const Tensor &grad1, const Tensor &grad2, const Tensor &xyz1,
+                                     const Tensor &xyz2, const Tensor &idx1, const Tensor &idx2)
+{
+    check_chamfer_backward(grad1, grad2, xyz1, xyz2, idx1, idx2);
+    OnDeviceOf guard(xyz1.device());
+    return chamfer_gradients(xyz1, grad1.size(0), {grad1.size(1), grad2.size(1)}, {ptr(grad1), ptr(grad2)},
+                             {ptr(xyz1), ptr(xyz2)}, idx1, idx2, true, true);
+}
+
+// The same of what the forward call leaves: clouds of either layout, and gradients of the distances or of their roots
+// (`of` then holds both distances and both roots).
 std::vector<Tensor> chamfer_backward_forms(const Tensor &grad1, const Tensor &grad2, const Tensor &xyz1,
                                            const Tensor &xyz2, const Tensor &idx1, const Tensor &idx2,
                                            const Tensor *of, double eps, bool channels_first, bool want1, bool want2)
 {
-    check_contiguous_cuda("grad_dist1", grad1);
-    check_contiguous_cuda("grad_dist2", grad2);
-    check_contiguous_cuda("xyz1", xyz1);
-    check_contiguous_cuda("xyz2", xyz2);
-    check_contiguous_cuda("idx1", idx1);
-    check_contiguous_cuda("idx2", idx2);
-    check(grad1.dim() == 2 && grad2.dim() == 2, "grad_dist must be 2-D tensors.");
-    check(xyz1.dim() == 3 && xyz2.dim() == 3, "xyz1 and xyz2 must be 3-D tensors.");
-    const int64_t b = grad1.size(0), n1 = grad1.size(1), n2 = grad2.size(1);
-    const int64_t points = channels_first ? 2 : 1, coords = 3 - points;
-    check(grad2.size(0) == b && xyz1.size(0) == b && xyz2.size(0) == b, "grad_dist and clouds differ in batch size.");
-    check(xyz1.size(points) == n1 && xyz2.size(points) == n2, "grad_dist and clouds differ in points.");
-    check(xyz1.size(coords) == 3 && xyz2.size(coords) == 3, "clouds must have three coordinates.");
-    check(idx1.sizes() == grad1.sizes() && idx2.sizes() == grad2.sizes(), "idx and grad_dist differ in shape.");
-    check_index("idx1", idx1);
-    check_index("idx2", idx2);
-    check_same("grad_dist1", grad1, "xyz1", xyz1);
-    check_same("grad_dist2", grad2, "xyz2", xyz2);
-    check_same("xyz1", xyz1, "xyz2", xyz2);
+    check_chamfer_backward(grad1, grad2, xyz1, xyz2, idx1, idx2, channels_first);
     for (int i = 0; of && i < 4; ++i) {
         check_contiguous_cuda("dist", of[i]);
         check_same("dist", of[i], "xyz1", xyz1);
         check(of[i].sizes() == (i % 2 ? grad2 : grad1).sizes(), "distances and grad_dist differ in shape.");
     }
     OnDeviceOf guard(xyz1.device());
-    Tensor grad_xyz1, grad_xyz2;
-    if (want1)
-        grad_xyz1 = like(xyz1, {b, n1, 3});
-    if (want2)
-        grad_xyz2 = like(xyz2, {b, n2, 3});
-    done(tk3d_chamfer_distance_backward_forms_f32(
-             ptr(grad1), ptr(grad2), ptr(xyz1), ptr(xyz2), ptr(idx1), ptr(idx2), of ? ptr(of[0]) : Ptr{},
-             of ? ptr(of[1]) : Ptr{}, of ? ptr(of[2]) : Ptr{}, of ? ptr(of[3]) : Ptr{}, eps, channels_first, b, n1, n2,
-             ptr(grad_xyz1), ptr(grad_xyz2), stream_of(xyz1)),
-         "tk3d_chamfer_distance_backward_forms_f32");
-    return {grad_xyz1, grad_xyz2};
+    const int64_t b = grad1.size(0), n[2] = {grad1.size(1), grad2.size(1)};
+    void *const stream = stream_of(xyz1);
+    // (asked before anything is allocated: a call on few long clouds takes as long as its host work)
+    if (is_f32(xyz1) && (channels_first || of) &&
+        tk3d_chamfer_distance_backward_takes_forms(channels_first, of != nullptr, n[0], n[1])) {
+        Tensor grad_xyz1, grad_xyz2;
+        if (want1)
+            grad_xyz1 = like(xyz1, {b, n[0], 3});
+        if (want2)
+            grad_xyz2 = like(xyz2, {b, n[1], 3});
+        done(tk3d_chamfer_distance_backward_forms_f32(
+                 ptr(grad1), ptr(grad2), ptr(xyz1), ptr(xyz2), ptr(idx1), ptr(idx2), of ? ptr(of[0]) : Ptr{},
+                 of ? ptr(of[1]) : Ptr{}, of ? ptr(of[2]) : Ptr{}, of ? ptr(of[3]) : Ptr{}, eps, channels_first, b, n[0],
+                 n[1], ptr(grad_xyz1), ptr(grad_xyz2), stream),
+             "tk3d_chamfer_distance_backward_forms_f32");
+        return {grad_xyz1, grad_xyz2};
+    }
+    // The other kernels work on [B,N,3] and gradients of distances: copies and gradients, all in one tensor.
+    Ptr x[2] = {ptr(xyz1), ptr(xyz2)}, g[2] = {ptr(grad1), ptr(grad2)};
+    Tensor work;
+    const int64_t points = b * (n[0] + n[1]);
+    if (points > 0 && (channels_first || of)) {
+        work = like(xyz1, {points * ((channels_first ? 3 : 0) + (of ? 1 : 0))});
+        char *at = static_cast<char *>(work.data_ptr());
+        const auto take = [&](int64_t elements) {
+            const Ptr p{at};
+            at += elements * (int64_t)work.element_size();
+            return p;
+        };
+        const Ptr rows[2] = {channels_first ? take(b * n[0] * 3) : Ptr{}, channels_first ? take(b * n[1] * 3) : Ptr{}};
+        const Ptr of_dist[2] = {of ? take(b * n[0]) : Ptr{}, of ? take(b * n[1]) : Ptr{}};
+        if (of && channels_first && is_f32(xyz1))
+            done(tk3d_chamfer_root_grads_rows_f32(g[0], g[1], ptr(of[0]), ptr(of[1]), ptr(of[2]), ptr(of[3]), x[0], x[1],
+                                                  b, n[0], n[1], eps, of_dist[0], of_dist[1], rows[0], rows[1], stream),
+                 "tk3d_chamfer_root_grads_rows_f32");
+        else {
+            if (of)
+                TK3D_CALL(is_f32(xyz1), tk3d_chamfer_root_grads, g[0], g[1], ptr(of[0]), ptr(of[1]), ptr(of[2]),
+                          ptr(of[3]), grad1.numel(), grad2.numel(), eps, of_dist[0], of_dist[1], stream);
+            if (channels_first)
+                TK3D_CALL(is_f32(xyz1), tk3d_chamfer_rows, x[0], x[1], 1, b, n[0], n[1], n[0], n[1], rows[0], rows[1],
+                          stream);
+        }
+        for (int i = 0; i < 2; ++i) {
+            x[i] = channels_first ? rows[i] : x[i];
+            g[i] = of ? of_dist[i] : g[i];
+        }
+    }
+    return chamfer_gradients(xyz1, b, n, g, x, idx1, idx2, want1, want2);
 }
 
 // Like the reference (which goes through at::gather) non-contiguous tensors are accepted.
@@ -527,52 +565,19 @@ struct ChamferNode : torch::autograd::Function<ChamferNode> {
         const variable_list saved = dense(ctx->get_saved_variables());
         const int64_t want = ctx->saved_data["want"].toInt();
         const bool channels_first = ctx->saved_data["channels_first"].toBool();
-        Tensor g1 = grads[0].contiguous(), g2 = grads[1].contiguous();
-        Tensor a = saved[0], c = saved[1];
-        OnDeviceOf guard(a.device());
-        const bool roots = saved.size() > 4, want1 = (want & 1) != 0, want2 = (want & 2) != 0;
-        const double eps = roots ? ctx->saved_data["eps"].toDouble() : 0.0;
-        const auto result = [&](std::vector<Tensor> g) {
-            for (int i = 0; i < 2; ++i) {
-                if (!(want & (1 << i)))
-                    g[i] = Tensor();
-                else if (channels_first)
-                    g[i] = g[i].transpose(1, 2);
-            }
-            return variable_list{g[0], g[1], Tensor(), Tensor(), Tensor()};
-        };
-        const int64_t b = a.size(0), n1 = g1.size(1), n2 = g2.size(1);
-        // (asked before anything is allocated: a call on few long clouds takes as long as its host work)
-        if (is_f32(a) && (channels_first || roots) && tk3d_chamfer_distance_backward_takes_forms(n1, n2))
-            return result(chamfer_backward_forms(g1, g2, a, c, saved[2], saved[3], roots ? &saved[4] : nullptr, eps,
-                                                 channels_first, want1, want2));
-        // (the other backward kernels work on [B,N,3] and gradients of distances)
-        const Tensor a3 = channels_first ? like(a, {b, n1, 3}) : a;
-        const Tensor c3 = channels_first ? like(c, {b, n2, 3}) : c;
-        bool copied = !channels_first;
-        if (roots) {
-            const Tensor o1 = like(g1, g1.sizes()), o2 = like(g2, g2.sizes());
-            if (channels_first && is_f32(a)) {
-                done(tk3d_chamfer_root_grads_rows_f32(ptr(g1), ptr(g2), ptr(saved[4]), ptr(saved[5]),
-                                                      ptr(saved[6]), ptr(saved[7]), ptr(a), ptr(c), b, n1,
-                                                      n2, eps, ptr(o1), ptr(o2), ptr(a3), ptr(c3),
-                                                      stream_of(g1)),
-                     "tk3d_chamfer_root_grads_rows_f32");
-                copied = true;
-            } else {
-                TK3D_CALL(is_f32(g1), tk3d_chamfer_root_grads, ptr(g1), ptr(g2), ptr(saved[4]),
-                          ptr(saved[5]), ptr(saved[6]), ptr(saved[7]), g1.numel(), g2.numel(), eps,
-                          ptr(o1), ptr(o2), stream_of(g1));
-            }
-            g1 = o1;
-            g2 = o2;
+        const Tensor g1 = grads[0].contiguous(), g2 = grads[1].contiguous();
+        const bool roots = saved.size() > 4;
+        std::vector<Tensor> g = chamfer_backward_forms(g1, g2, saved[0], saved[1], saved[2], saved[3],
+                                                       roots ? &saved[4] : nullptr,
+                                                       roots ? ctx->saved_data["eps"].toDouble() : 0.0, channels_first,
+                                                       (want & 1) != 0, (want & 2) != 0);
+        for (int i = 0; i < 2; ++i) {
+            if (!(want & (1 << i)))
+                g[i] = Tensor();
+            else if (channels_first)
+                g[i] = g[i].transpose(1, 2);
         }
-        if (!copied)
-            TK3D_CALL(is_f32(a), tk3d_chamfer_rows, ptr(a), ptr(c), 1, b, n1, n2, n1, n2, ptr(a3),
-                      ptr(c3), stream_of(a));
-        a = a3;
-        c = c3;
-        return result(chamfer_backward(g1, g2, a, c, saved[2], saved[3], want1, want2));
+        return {g[0], g[1], Tensor(), Tensor(), Tensor()};
     }
 };
 
