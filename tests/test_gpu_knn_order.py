@@ -1,0 +1,66 @@
+"""The pre-filtered KNN kernel on keys in an order, which launches of few workgroups look for: they then sweep every
+key instead of those in reach of a wave's box, half of the queries to a workgroup where CUs are free. Against the
+oracle's literal MinK, bit for bit."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from debug_abi import knn_filter
+
+pytestmark = pytest.mark.gpu
+
+
+def cloud(kind, b, n, seed):
+    g = np.random.default_rng(seed)
+    p = g.random((b, n, 3), dtype=np.float32)
+    if kind == "lattice by x":  # and equal distances everywhere
+        p = np.floor(p * 6).astype(np.float32)
+    if kind in ("by x", "lattice by x", "mixed", "not numbers"):
+        p = np.take_along_axis(p, np.argsort(p[:, :, :1], axis=1, kind="stable"), 1)
+    if kind == "mixed":  # ordered clouds and others in a launch
+        p[::2] = p[::2, g.permutation(n)]
+    elif kind == "flat":  # an axis without extent, keys by another
+        p = np.take_along_axis(p, np.argsort(p[:, :, 1:2], axis=1), 1)
+        p[:, :, 0] = 0.25
+    elif kind == "far key":  # in random order, but one key makes the cloud's box large
+        p[:, -1] = 1e3
+    elif kind == "not numbers":
+        p[:, : n // 3, 0] = np.nan
+        p[0, n - 2, 1] = np.nan
+    return p
+
+
+# k: the smallest and largest of 4, 8 and 16 slots; keys: the fewest that have boxes, a stage's edge, a remainder;
+# queries: around 256, 512 and their sums (the halves of a workgroup)
+@pytest.mark.parametrize("kind", ["by x", "lattice by x", "mixed", "flat", "far key", "not numbers"])
+@pytest.mark.parametrize("b,n1,n2,k", [
+    (2, 257, 2048, 1), (3, 511, 2049, 4), (2, 512, 2560, 3), (2, 513, 2048, 3), (3, 769, 2100, 4), (2, 1280, 2047, 4),
+    (2, 300, 4096, 5), (2, 768, 4097, 8), (1, 1025, 4095, 8), (2, 256, 4096, 8), (2, 129, 16384, 2), (2, 128, 16384, 2),
+    (1, 300, 8192, 9), (2, 770, 8705, 16), (2, 513, 8191, 16)])
+def test_few_workgroups(cuda, kind, b, n1, n2, k):
+    q, key = cloud("random", b, n1, n1), cloud(kind, b, n2, n2)
+    if kind == "not numbers":
+        q[0, 3, 2], q[-1, n1 - 1, 0] = np.nan, np.inf
+    got = knn_filter(torch.from_numpy(q).to(cuda), torch.from_numpy(key).to(cuda), k)
+    with np.errstate(invalid="ignore"):
+        want = oracle.knn(q, key, k)
+    assert np.array_equal(got[0].cpu().numpy(), want[0], equal_nan=True)
+    assert np.array_equal(got[1].cpu().numpy(), want[1])
+
+
+# either side of a workgroup to two CUs, and of one to one (256 CUs), beyond which order makes no difference
+@pytest.mark.parametrize("b,n2,k", [(128, 2048, 3), (129, 2048, 3), (256, 2048, 3), (257, 2048, 3), (257, 1024, 4),
+                                    (129, 3584, 16), (129, 3583, 16), (256, 2560, 8), (257, 1023, 12)])
+def test_workgroups_to_a_cu(cuda, b, n2, k):
+    q, key = cloud("random", b, 257, b), cloud("mixed", b, n2, n2)
+    got = knn_filter(torch.from_numpy(q).to(cuda), torch.from_numpy(key).to(cuda), k)
+    some = sorted({0, 1, b // 2, b - 2, b - 1})
+    want = oracle.knn(q[some], key[some], k)
+    assert np.array_equal(got[0].cpu().numpy()[some], want[0])
+    assert np.array_equal(got[1].cpu().numpy()[some], want[1])
+    # the rest against the same clouds a few at a time
+    few = 16
+    for at in range(0, b, few):
+        part = knn_filter(torch.from_numpy(q[at:at + few]).to(cuda), torch.from_numpy(key[at:at + few]).to(cuda), k)
+        assert torch.equal(got[0][at:at + few], part[0]) and torch.equal(got[1][at:at + few], part[1])

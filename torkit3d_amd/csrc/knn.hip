@@ -461,13 +461,26 @@ __device__ __forceinline__ double knn_max_f64(double a, double b)
 // from the centre (rescaled; thr would leave fp16's range) take every key as a candidate, key clouds
 // that are non-finite or huge the exact batched sweep.
 //
-// Boxes. From 1024 keys on the workgroup's queries are sorted along a Hilbert curve, so that a wave has
-// neighbours: its 64 queries' box is small, and a key whose distance to that box - by the operations of the canonical distance
-// on the per-axis gaps, each of which is monotone, hence a bound for every query in the box - is not below the
-// largest of the wave's maxima is a candidate of none of them. A lane tests a key, and what passes goes into the
-// wave's list in LDS, in key order; the sweep takes its chunks of 32 from there. Of 2048 keys 780 pass
-// for waves of 512 sorted queries at k = 3 and 1050 at k = 16 (sorted along a Morton curve 980 and 1190; 8192 queries
-// sorted together 300 and 470, but they take a kernel and a workspace of their own). Of fewer keys too many pass.
+// Boxes. In launches with keys enough (knn_filter_launch) the workgroup's 512 queries are sorted along a Hilbert
+// curve, so that a wave has neighbours: its 64 queries' box is small, and a key whose distance to that box - by the
+// operations of the canonical distance on the per-axis gaps, each of which is monotone, hence a bound for every query
+// in the box - is not below the largest of the wave's maxima is a candidate of none of them. A lane tests a key, and
+// what passes goes into the wave's list in LDS, in key order; the sweep takes its chunks of 32 from there. Of 2048
+// keys 780 pass for waves of 512 sorted queries at k = 3 and 1050 at k = 16 (sorted along a Morton curve 980 and
+// 1190; 8192 queries sorted together 300 and 470, but they take a kernel and a workspace of their own). Of fewer keys
+// too many pass, and of 256 sorted queries a wave's box is too large. Where every key is swept its own number is its
+// place in the list, which is then not written down.
+//
+// Keys in an order - scan lines, voxels - come near one wave of sorted queries at a time, and the others wait for it
+// at the barrier of each stage, with no second workgroup on the CU to use it. A workgroup that may be alone on its CU
+// therefore compares the box of the first stage's keys with that of all: in random order 512 of 2^16 normally
+// distributed keys reach over about 0.7 of the cloud, in the order of a coordinate or a space-filling curve 512 of
+// 1024 keys over half of an axis and of more over less. Under 0.6, it sweeps every key for its queries as they come
+// (and half of them, where CUs would be left without a workgroup: the other half has one of its own, which otherwise
+// ends there). us, 8 x 4096 queries, keys by x and by the voxels of a 16^3 grid along a Morton curve, without this
+// test, with it: 4096 keys k = 3 131, 101 and 332, 253, k = 8 177, 129 and 483, 336; 8192 keys k = 16 396, 288 and
+// 1206, 904; it takes 0 to 3 % of the time on keys in random order. Two workgroups to a CU fill each other's waits,
+// and are left with the boxes: 32 x 8192 on 4096 in voxels k = 3 422, every key 471, by x 194 and 194.
 //
 // The first keys behind the fill are below the maximum of half of the queries or more: up to 3 k (2 k with 32 slots) they
 // are put to all of them, without a sweep and a queue (a third less work than the steps they save: 142 -> 109 of
@@ -496,15 +509,16 @@ __device__ __forceinline__ double knn_max_f64(double a, double b)
 // position, a binary search, the nibbles' rotation), and 40 at k = 3 where slots in registers in their
 // own order took 112 (selects, a maximum, a scan for its first slot).
 //
-// Bound by vector issue, of which the steps are half to two thirds: a lane is a query whose
-// candidates are served in key order, so 59 % of the lanes are busy in a step at k = 16, a third at k =
-// 3. 512 lanes share the staged keys and the sort (up to 123 registers and 66 KB of LDS up to 16 slots: four waves
-// per SIMD); 32 slots run in 256, of which a CU holds three workgroups. us, all keys swept and this, uniform
-// clouds unless said otherwise: 32 x 8192 queries on 2048 keys k = 3 69.6, 54.9 (in clusters 68.1, 66.0), k = 8 83.2, 70.1, k = 16
-// 128, 114 (on a sphere 130, 113); 16 x 16384 on 4096 k = 3 103, 75; 4 x 16384 on 16384 k = 16 249, 204; 20 x 1000 on 16384
-// k = 8 232, 160; 1 x 40000 on 40000 k = 16 546, 498; 32 slots, whose waves' boxes are of 256 queries, 24 x 8192 on 2048 k = 32
-// 212, 203, 32 x 2048 on 8192 208, 211; on 64 to 512 keys 0.9 to 1.02 of the time before; clouds of up to 128 queries,
-// which two waves have anyway, 0.9 where there are more of them than CUs, else up to 1.12.
+// Bound by vector issue, of which the steps are half to two thirds: a lane is a query whose candidates are served in
+// key order, so 59 % of the lanes are busy in a step at k = 16, a third at k = 3. 512 lanes share the staged keys and
+// the sort (up to 126 registers and 66 KB of LDS, 50 without boxes: four waves per SIMD); 32 slots run in 256, of
+// which a CU holds three workgroups (with boxes of 256 queries they took up to 1.13 times as long: 80 x 250 on 16384
+// in clusters k = 20 328, 291 without). us, every key swept and none put
+// to all queries, and now: 32 x 8192 queries on 2048 keys k = 3 63.5, 49.5, k = 8 83, 69, k = 16 122, 110, k = 32 262, 246; 8 x
+// 4096 on 16384 k = 3 214, 139, k = 16 251, 198; 8 x 4096 on 256 k = 3 15.4, 11.9, k = 16 28.2, 25.4; 200 x 120 on
+// 4096 k = 8 66, 60.
+enum { KNN_EVERY_KEY, KNN_BOXES, KNN_BOXES_UNLESS_ORDERED };  // (what is passed over)
+
 constexpr int knn_max4(int a, int b, int c, int d)
 {
     const int ab = a > b ? a : b, cd = c > d ? c : d;
@@ -524,151 +538,104 @@ constexpr KnnCurve knn_make_curve()
 }
 __device__ constexpr KnnCurve knn_curve alignas(16) = knn_make_curve();
 
-template <int KMAX, bool SOA, bool WEIGHTS, int LANES>
-__global__ __launch_bounds__(LANES) void knn_filter_kernel_f32(
-    const float *__restrict__ query, const float *__restrict__ key,
-    float *__restrict__ distance, int64_t *__restrict__ index, float *__restrict__ weight,
-    float eps, int blocks_per_batch, int n1, int n2, int k)
-{
-    constexpr int BLOCK = LANES;
-    constexpr int NW = BLOCK / TK_WAVE;
-    constexpr int STAGE = KMAX > 16 ? 256 : 512;
-    constexpr int CHUNK = 32;
-    constexpr int TEST = KMAX > 16 ? 4 : 2;  // keys a lane tests against the box at once
-    constexpr int CAP = 4;
-    constexpr int T = 6;
-    constexpr int PER = STAGE > BLOCK ? STAGE / BLOCK : 1;
-    constexpr int RING = 2 * STAGE;  // a wave's list: it goes back to the first key of the stage before
-    using Slot = KnnSlot<KMAX>;
-    static_assert((STAGE % BLOCK == 0 || BLOCK % STAGE == 0) && STAGE % (TEST * TK_WAVE) == 0, "stage shape");
-    static_assert(!WEIGHTS || KMAX == 4, "weights of three neighbours");
-    // Two stage buffers of key terms, [key][half] x 16 bytes, then two of raw keys (x, y, z, 0) for the
+template <int KMAX, int LANES> struct KnnFilter {
+    static constexpr int BLOCK = LANES;
+    static constexpr int NW = BLOCK / TK_WAVE;
+    static constexpr int STAGE = KMAX > 16 ? 256 : 512;
+    static constexpr int PER = STAGE / BLOCK;
+    static constexpr int CHUNK = 32;
+    static constexpr int RING = 2 * STAGE;  // a wave's list: it goes back to the first key of the stage before
+    static constexpr int CELLS = 512;
+    // Two stage buffers of key terms, [key][half] x 16 bytes, then two of raw keys (x, y, z, number) for the
     // boxes' test and the service steps; before them the sort's counters, behind them the results.
-    constexpr int SCORE_FLOATS = 2 * STAGE * 8;
-    constexpr int STAGING_FLOATS = SCORE_FLOATS + 2 * STAGE * 4;
-    constexpr int CELLS = 512;
-    constexpr int PRUNE = 1024;
+    static constexpr int SCORE_FLOATS = 2 * STAGE * 8;
+    static constexpr int STAGING_FLOATS = SCORE_FLOATS + 2 * STAGE * 4;
+    static constexpr int SORT_FLOATS = CELLS + 4 + CELLS / 2 + 4 * BLOCK;
     // rows of results that leave together (36 KB of LDS with 8 slots, 40 at most)
-    constexpr int ROW = KMAX + 1;
-    constexpr int ROWS_FIT = KMAX == 4 ? 1024 : 4096 / KMAX;
-    constexpr int ROWS = ROWS_FIT < BLOCK ? ROWS_FIT : BLOCK;
-    constexpr int LDS_FLOATS = knn_max4(STAGING_FLOATS, ROWS * ROW * 2, CELLS + 4 + CELLS / 2 + 4 * BLOCK, KNN_STAGE * 4);
-    __shared__ __align__(16) float skey[LDS_FLOATS];
-    __shared__ __align__(16) unsigned short sring[NW][RING + CHUNK];  // (its beginning once more behind it)
-    float4 *const sraw = reinterpret_cast<float4 *>(skey + SCORE_FLOATS);
-    uint4 *const sterm = reinterpret_cast<uint4 *>(skey);
-    const int half = (threadIdx.x >> 5) & 1;
-    __shared__ float sred[NW][13];
-    const int tid = threadIdx.x;
-    const int lane = tid & (TK_WAVE - 1);
-    const int wave = __builtin_amdgcn_readfirstlane(tid / TK_WAVE);
-    const int b = blockIdx.x / blocks_per_batch;
-    const int qblock = blockIdx.x - b * blocks_per_batch;
-    const float *__restrict__ K = key + (int64_t)b * n2 * 3;
-    const float *__restrict__ Q = query + (int64_t)b * n1 * 3;
-    const float INF = __builtin_huge_valf();
+    static constexpr int ROW = KMAX + 1;
+    static constexpr int ROWS_FIT = KMAX == 4 ? 1024 : 4096 / KMAX;
+    static constexpr int ROWS = ROWS_FIT < BLOCK ? ROWS_FIT : BLOCK;
+    static constexpr int LDS_FLOATS = knn_max4(STAGING_FLOATS, ROWS * ROW * 2, SORT_FLOATS, KNN_STAGE * 4);
+    static constexpr int RED = 19;  // words a wave leaves to the others
+    static_assert(STAGE % BLOCK == 0, "stage shape");
+};
 
-    // ---- bounding boxes of the key cloud (its centre, and a bound of the centred norms) and of the
-    // workgroup's queries ----
-    const int mine0 = qblock * BLOCK + tid;
-    float ends[6] = {-INF, -INF, -INF, -INF, -INF, -INF};  // -lowest, highest
-    const auto reach_out = [&](float (&e)[6], const float (&v)[3]) {
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            e[a] = __builtin_fmaxf(e[a], -v[a]);
-            e[3 + a] = __builtin_fmaxf(e[3 + a], v[a]);
-        }
-    };
-    for (int j = tid; j < n2; j += BLOCK) {
-        const float v[3] = {knn_coord<SOA>(K, n2, j, 0), knn_coord<SOA>(K, n2, j, 1), knn_coord<SOA>(K, n2, j, 2)};
-        reach_out(ends, v);
-    }
-    const int nstages = (n2 + STAGE - 1) / STAGE;
-    float4 pre[PER];
-    auto fetch = [&](int st) {
-#pragma unroll
-        for (int r = 0; r < PER; ++r) {
-            const int kj = st * STAGE + r * BLOCK + tid;
-            pre[r] = make_float4(INF, INF, INF, __builtin_bit_cast(float, kj));  // (past the end: in no box's reach)
-            if (kj < n2 && (BLOCK <= STAGE || tid < STAGE))
-                pre[r] = make_float4(knn_coord<SOA>(K, n2, kj, 0), knn_coord<SOA>(K, n2, kj, 1),
-                                     knn_coord<SOA>(K, n2, kj, 2), __builtin_bit_cast(float, kj));
-        }
-    };
-    fetch(0);
-    float own[3] = {0.0f, 0.0f, 0.0f};  // (of a query that does not exist)
-    float qends[6] = {-INF, -INF, -INF, -INF, -INF, -INF};
-    if (mine0 < n1) {
-#pragma unroll
-        for (int a = 0; a < 3; ++a)
-            own[a] = knn_coord<SOA>(Q, n1, mine0, a);
-        reach_out(qends, own);
-    }
-    tk_wave_max_six<64>(ends);
-    tk_wave_max_six<64>(qends);
-    if (lane == TK_WAVE - 1) {
-#pragma unroll
-        for (int a = 0; a < 6; ++a) {
-            sred[wave][a] = ends[a];
-            sred[wave][6 + a] = qends[a];
-        }
-    }
-    unsigned *const cnt = reinterpret_cast<unsigned *>(skey);
-    unsigned short *const curve = reinterpret_cast<unsigned short *>(cnt + CELLS + 4);
-    if (tid < CELLS / 8)
-        reinterpret_cast<uint4 *>(curve)[tid] = reinterpret_cast<const uint4 *>(knn_curve.place)[tid];
-    for (int i = tid; i <= CELLS; i += BLOCK)
-        cnt[i] = 0u;
-    __syncthreads();
-    float cc[3], origin[3], cells[3];
-    float kmax2 = 0.0f;
+// -lowest and highest of each axis
+__device__ __forceinline__ void knn_reach_out(float (&e)[6], const float (&v)[3])
+{
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-        float l = -INF, h = -INF, ql = -INF, qh = -INF;
-#pragma unroll
-        for (int w = 0; w < NW; ++w) {
-            l = __builtin_fmaxf(l, sred[w][a]);
-            h = __builtin_fmaxf(h, sred[w][3 + a]);
-            ql = __builtin_fmaxf(ql, sred[w][6 + a]);
-            qh = __builtin_fmaxf(qh, sred[w][9 + a]);
-        }
-        cc[a] = 0.5f * h - 0.5f * l;
-        const float side = __builtin_fmaxf(h - cc[a], cc[a] + l);
-        // (the operations of a norm, each of which is monotone: no centred key is beyond it)
-        kmax2 = a == 0 ? side * side : __builtin_fmaf(side, side, kmax2);
-        origin[a] = -ql;
-        const float extent = qh + ql;
-        cells[a] = extent > 0.0f ? 7.99f / extent : 0.0f;  // also 0 for NaN / inf extents
+        e[a] = __builtin_fmaxf(e[a], -v[a]);
+        e[3 + a] = __builtin_fmaxf(e[3 + a], v[a]);
     }
-    const float c0 = cc[0], c1 = cc[1], c2 = cc[2];
-    bool safe = (c0 - c0 == 0.0f) && (c1 - c1 == 0.0f) && (c2 - c2 == 0.0f) && (kmax2 < 1e30f);
-    const float ext = __builtin_sqrtf(kmax2);
-    const int ebits = (int)((__builtin_bit_cast(unsigned, ext) >> 23) & 0xffu) - 127;
-    safe = safe && (ext == 0.0f || (ebits >= -40 && ebits <= 40));
-    // Half the box's diagonal comes to [2, 4): its largest side is 1/sqrt(3) of that or more, and a key on it.
-    const float scale = (!safe || ext == 0.0f) ? 1.0f
-                                               : __builtin_bit_cast(float, (unsigned)(128 - ebits) << 23);
+}
 
-    if (!safe) {  // uniform over the workgroup
-        knn_batched_body<KMAX, SOA, WEIGHTS>(query, key, distance, index, weight, eps, b,
-                                             qblock * BLOCK + tid, n1, n2, k, skey);
-        return;
+// The lane's keys of stage `st`. (Past the end: in no box's reach, and of no chunk's.)
+template <bool SOA, int PER, int BLOCK>
+__device__ __forceinline__ void knn_filter_fetch(float4 (&pre)[PER], const float *__restrict__ K, int n2, int st)
+{
+    const float INF = __builtin_huge_valf();
+#pragma unroll
+    for (int r = 0; r < PER; ++r) {
+        const int kj = (st * PER + r) * BLOCK + (int)threadIdx.x;
+        pre[r] = make_float4(INF, INF, INF, __builtin_bit_cast(float, kj));
+        if (kj < n2)
+            pre[r] = make_float4(knn_coord<SOA>(K, n2, kj, 0), knn_coord<SOA>(K, n2, kj, 1),
+                                 knn_coord<SOA>(K, n2, kj, 2), __builtin_bit_cast(float, kj));
     }
-    const float kmax = __builtin_sqrtf(kmax2) * scale * 1.000001f;
+}
+
+// What the kernel has found out before it comes to its queries.
+template <int PER> struct KnnFrame {
+    float centre[3], scale, kmax;   // of the keys; kmax bounds their rescaled norms
+    float origin[3], cells[3];      // of the grid that sorts the queries, with boxes
+    float own[3];                   // the lane's query before that
+    float4 pre[PER];                // the lane's keys of the first stage
+};
+
+// The queries base .. base + span - 1 of cloud b, a lane each; BOXES: sorted, keys outside a wave's box passed over.
+template <int KMAX, bool SOA, bool WEIGHTS, int LANES, bool BOXES>
+__device__ __forceinline__ void knn_filter_queries(
+    const float *__restrict__ Q, const float *__restrict__ K, float *__restrict__ distance,
+    int64_t *__restrict__ index, float *__restrict__ weight, float eps, int b, int base, int span, int n1, int n2, int k,
+    KnnFrame<KnnFilter<KMAX, LANES>::PER> &frame, float *skey, unsigned short *rings,
+    float (*sred)[KnnFilter<KMAX, LANES>::RED])
+{
+    using F = KnnFilter<KMAX, LANES>;
+    using Slot = KnnSlot<KMAX>;
+    constexpr int BLOCK = F::BLOCK, NW = F::NW, STAGE = F::STAGE, PER = F::PER, CHUNK = F::CHUNK, RING = F::RING;
+    constexpr int CELLS = F::CELLS, ROW = F::ROW, ROWS = F::ROWS;
+    constexpr int TEST = 2;  // keys a lane tests against the box at once
+    constexpr int CAP = 4;
+    constexpr int T = 6;
+    static_assert(!WEIGHTS || KMAX == 4, "weights of three neighbours");
+    static_assert(!BOXES || (3 * KMAX <= TK_WAVE && STAGE % (TEST * TK_WAVE) == 0 && CELLS == BLOCK), "boxes' shape");
+    float4 *const sraw = reinterpret_cast<float4 *>(skey + F::SCORE_FLOATS);
+    uint4 *const sterm = reinterpret_cast<uint4 *>(skey);
+    const int tid = threadIdx.x;
+    const int lane = tid & (TK_WAVE - 1);
+    const int half = (tid >> 5) & 1;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / TK_WAVE);
+    const float INF = __builtin_huge_valf();
+    const float c0 = frame.centre[0], c1 = frame.centre[1], c2 = frame.centre[2];
+    const float scale = frame.scale, kmax = frame.kmax;
     const float scale2 = scale * scale;  // <= 2^82
+    const int nstages = (n2 + STAGE - 1) / STAGE;
 
     // ---- the workgroup's queries in the order of their cells along a Hilbert curve, those that do not exist last
     // (a counting sort; the order within a cell is whatever the atomics give, which no result depends on) ----
     int mine = tid;
-    float qx = own[0], qy = own[1], qz = own[2];
-    const bool prune = n2 >= PRUNE && n1 > 128;  // uniform
-    if (prune) {
+    float qx = frame.own[0], qy = frame.own[1], qz = frame.own[2];
+    if constexpr (BOXES) {
+        unsigned *const cnt = reinterpret_cast<unsigned *>(skey);
+        const unsigned short *const curve = reinterpret_cast<const unsigned short *>(cnt + CELLS + 4);
+        float4 *const order = reinterpret_cast<float4 *>(cnt + CELLS + 4 + CELLS / 2);
         unsigned cell = CELLS;
-        if (mine0 < n1) {
+        if (base + tid < n1) {
             unsigned at = 0u;
 #pragma unroll
             for (int a = 0; a < 3; ++a) {
-                const float f = (own[a] - origin[a]) * cells[a];
+                const float f = (frame.own[a] - frame.origin[a]) * frame.cells[a];
                 // (a NaN or an out-of-range value lands in cell 0 or 7)
                 at = 8u * at + (unsigned)(int)__builtin_fminf(__builtin_fmaxf(f, 0.0f), 7.0f);
             }
@@ -676,14 +643,7 @@ __global__ __launch_bounds__(LANES) void knn_filter_kernel_f32(
         }
         const unsigned turn = atomicAdd(&cnt[cell], 1u);
         __syncthreads();
-        constexpr int RUN = CELLS / BLOCK;
-        static_assert(RUN * BLOCK == CELLS, "a run of cells to a lane");
-        unsigned c[RUN], sum = 0u;
-#pragma unroll
-        for (int i = 0; i < RUN; ++i) {
-            c[i] = cnt[tid * RUN + i];
-            sum += c[i];
-        }
+        const unsigned sum = cnt[tid];  // (a cell to a lane)
         unsigned incl = sum;
 #pragma unroll
         for (int o = 1; o < TK_WAVE; o <<= 1) {
@@ -691,22 +651,17 @@ __global__ __launch_bounds__(LANES) void knn_filter_kernel_f32(
             incl += lane >= o ? up : 0u;
         }
         if (lane == TK_WAVE - 1)
-            sred[wave][12] = __builtin_bit_cast(float, incl);
+            sred[wave][18] = __builtin_bit_cast(float, incl);
         __syncthreads();
-        unsigned start = incl - sum;
+        unsigned start = incl;
 #pragma unroll
         for (int w = 0; w < NW; ++w)
-            start += w < wave ? __builtin_bit_cast(unsigned, sred[w][12]) : 0u;
-#pragma unroll
-        for (int i = 0; i < RUN; ++i) {
-            cnt[tid * RUN + i] = start;
-            start += c[i];
-        }
+            start += w < wave ? __builtin_bit_cast(unsigned, sred[w][18]) : 0u;
+        cnt[tid] = start - sum;
         if (tid == BLOCK - 1)
             cnt[CELLS] = start;
         __syncthreads();
-        float4 *const order = reinterpret_cast<float4 *>(curve + CELLS);
-        order[cnt[cell] + turn] = make_float4(own[0], own[1], own[2], __builtin_bit_cast(float, tid));
+        order[cnt[cell] + turn] = make_float4(qx, qy, qz, __builtin_bit_cast(float, tid));
         __syncthreads();
         const float4 q = order[tid];
         qx = q.x;
@@ -716,19 +671,24 @@ __global__ __launch_bounds__(LANES) void knn_filter_kernel_f32(
     }
 
     // ---- the lane's query ----
-    const int qi = qblock * BLOCK + mine;
-    const bool active = qi < n1;
+    const int qi = base + mine;
+    const bool active = mine < span && qi < n1;
+    if (!BOXES && active) {
+        qx = knn_coord<SOA>(Q, n1, qi, 0);
+        qy = knn_coord<SOA>(Q, n1, qi, 1);
+        qz = knn_coord<SOA>(Q, n1, qi, 2);
+    }
     // the box of the wave's queries
     float box[6] = {-INF, -INF, -INF, -INF, -INF, -INF};
-    if (active) {
-        const float v[3] = {qx, qy, qz};
-        reach_out(box, v);
-    }
-    tk_wave_max_six<64>(box);
+    if constexpr (BOXES) {
+        if (active) {
+            const float v[3] = {qx, qy, qz};
+            knn_reach_out(box, v);
+        }
+        tk_wave_max_six<64>(box);
 #pragma unroll
-    for (int a = 0; a < 6; ++a) {
-        const int end = __builtin_amdgcn_readlane(__builtin_bit_cast(int, box[a]), TK_WAVE - 1);
-        box[a] = __builtin_bit_cast(float, prune ? end : 0x7f7fffff);  // (else all keys)
+        for (int a = 0; a < 6; ++a)
+            box[a] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, box[a]), TK_WAVE - 1));
     }
     float qn, slack_r;
     bool usable;
@@ -774,19 +734,21 @@ __global__ __launch_bounds__(LANES) void knn_filter_kernel_f32(
         v[s] = UNUSED;
     float max_key = 0.0f;
     // Pending chunk masks, oldest first (bit 31 = first key of the chunk), and the place in the wave's list
-    // of bit 31 of each. Named and no loops over the queue, so it stays in registers.
+    // of bit 31 of each, without a list the key. Named and no loops over the queue, so it stays in registers.
     static_assert(CAP == 4, "the queue is written out for four entries");
     unsigned m0 = 0u, m1 = 0u, m2 = 0u, m3 = 0u;
     int b0 = 0, b1 = 0, b2 = 0, b3 = 0;
     int qlen = 0, pending = 0;
 
-    // The wave's list: 16 times which key of the two buffers. (Zeros: a place that nothing was listed at is
-    // read where a query has no candidate.)
-    unsigned short *const ring = sring[wave];
+    // The wave's list: 16 times which key of the two buffers. Where boxes pass nothing over it has every key at its own
+    // number, and is not written down. (A place that nothing was listed at is read where a query has no candidate.)
+    unsigned short *const ring = rings + (BOXES ? wave * (RING + CHUNK) : 0);
     unsigned char *const lds_raw = reinterpret_cast<unsigned char *>(sraw);
     unsigned char *const lds_term = reinterpret_cast<unsigned char *>(sterm);
-    for (int i = lane; i < (RING + CHUNK) / 8; i += TK_WAVE)
-        reinterpret_cast<uint4 *>(ring)[i] = make_uint4(0u, 0u, 0u, 0u);
+    if constexpr (BOXES)
+        for (int i = lane; i < (RING + CHUNK) / 8; i += TK_WAVE)
+            reinterpret_cast<uint4 *>(ring)[i] = make_uint4(0u, 0u, 0u, 0u);
+    const auto listed = [&](int i) { return BOXES ? (int)ring[i] : 16 * (i & (RING - 1)); };
     int head = 0, tail = 0;  // places of the list: swept up to, filled up to (uniform)
 
     // Puts a key to the lane's query.
@@ -807,10 +769,6 @@ __global__ __launch_bounds__(LANES) void knn_filter_kernel_f32(
         max_key = ins ? __builtin_bit_cast(float, Slot::distance(v[0])) : max_key;
     };
 
-    // With 32 slots, one to three waves a SIMD: where the first candidate lies is looked up a step ahead, beside the insertion before it.
-    constexpr bool AHEAD = KMAX > 16 || LANES == 256;
-    unsigned coming = 0u;
-    auto look = [&]() { coming = ring[b0 + __builtin_clz(m0 | 1u)]; };
     // One service step: every query with a pending candidate takes its first one.
     auto service = [&]() {
         const bool has = qlen > 0;
@@ -818,7 +776,7 @@ __global__ __launch_bounds__(LANES) void knn_filter_kernel_f32(
         // below stays inside the buffer and nothing is inserted)
         const int bit = __builtin_clz(m0 | 1u);
         // resident: candidates are never older than the previous stage (see below)
-        const float4 raw = *reinterpret_cast<const float4 *>(lds_raw + (AHEAD ? coming : ring[b0 + bit]));
+        const float4 raw = *reinterpret_cast<const float4 *>(lds_raw + listed(b0 + bit));
         const int kj = __builtin_bit_cast(int, raw.w);
         const unsigned rest = m0 & ~(0x80000000u >> bit);
         const bool shift = has && rest == 0u;
@@ -831,8 +789,6 @@ __global__ __launch_bounds__(LANES) void knn_filter_kernel_f32(
         m3 = shift ? 0u : m3;
         qlen -= shift ? 1 : 0;
         pending -= has ? 1 : 0;
-        if constexpr (AHEAD)
-            look();
         put(raw, kj, has);
         // Keep the loop-carried state where it is: without this the register allocator
         // rotates some forty values through copies on every step.
@@ -849,12 +805,10 @@ __global__ __launch_bounds__(LANES) void knn_filter_kernel_f32(
 
     // ---- sweep: keys centred and staged in two LDS buffers, one barrier per stage ----
     auto stash = [&](int buf) {
-        if (BLOCK > STAGE && tid >= STAGE)
-            return;
 #pragma unroll
         for (int r = 0; r < PER; ++r) {
             const int j = buf * STAGE + r * BLOCK + tid;
-            const float ex = pre[r].x - c0, ey = pre[r].y - c1, ez = pre[r].z - c2;
+            const float ex = frame.pre[r].x - c0, ey = frame.pre[r].y - c1, ez = frame.pre[r].z - c2;
             const float x = ex * scale, y = ey * scale, z = ez * scale;
             const float n = __builtin_fmaf(ez, ez, __builtin_fmaf(ey, ey, ex * ex)) * scale2;
             const unsigned sx = tk_f16_split2(x), sy = tk_f16_split2(y), sz = tk_f16_split2(z);
@@ -863,7 +817,7 @@ __global__ __launch_bounds__(LANES) void knn_filter_kernel_f32(
             sterm[2 * j] = make_uint4(xh * 0x10001u, (sx >> 16) | (yh << 16), yh | (sy & 0xffff0000u),
                                       0x3c003c00u);
             sterm[2 * j + 1] = make_uint4(zh * 0x10001u, (sz >> 16) | (sn << 16), sn >> 16, 0x3c003c00u);
-            sraw[j] = pre[r];
+            sraw[j] = frame.pre[r];
         }
     };
     bool stale = true;    // the T terms do not belong to the maximum any more
@@ -875,7 +829,7 @@ __global__ __launch_bounds__(LANES) void knn_filter_kernel_f32(
     auto sweep = [&](int count) {
         tk_wave_fence();  // (the list is the wave's own)
         const int first = head & (RING - 1);  // (a chunk goes on into the ring's beginning behind its end)
-        const int at = ring[first + (row < count ? row : 0)];
+        const int at = listed(first + (row < count ? row : 0));
         const tk_f16x8 ka = *reinterpret_cast<const tk_f16x8 *>(lds_term + 2 * at + 16 * half);
         if (stale) {  // uniform
             const float m = max_key * scale2;  // rescaled units; slack 64 u R + 48 u M
@@ -919,8 +873,6 @@ __global__ __launch_bounds__(LANES) void knn_filter_kernel_f32(
         qlen += nz ? 1 : 0;
         pending += __builtin_popcount(m);
         head += count;
-        if constexpr (AHEAD)
-            look();
         // (two steps per trip: the loop-carried state is copied between registers once
         // per trip, some forty moves)
         while (must_serve()) {
@@ -960,48 +912,54 @@ __global__ __launch_bounds__(LANES) void knn_filter_kernel_f32(
         const float4 raw = sraw[j];
         put(raw, j, active);
     }
+    const bool idle = __builtin_amdgcn_ballot_w64(active) == 0;  // (a wave of queries that do not exist)
+    if (!BOXES)
+        head = tail = taken;
     for (int st = 0; st < nstages; ++st) {
         const int stage0 = st * STAGE, buf = (st & 1) * STAGE;
         if (st + 1 < nstages)
-            fetch(st + 1);
+            knn_filter_fetch<SOA, PER, BLOCK>(frame.pre, K, n2, st + 1);
         const int left = n2 - stage0;
         const int cnt = left < STAGE ? left : STAGE;
+        // (without boxes a stage at a time)
 #pragma unroll 1
-        for (int j0 = 0; j0 < cnt; j0 += TEST * TK_WAVE) {
-            if (moved) {  // uniform
-                reach = tk_wave_extreme<true>(active ? max_key : -INF);
-                moved = false;
-            }
-            float4 raw[TEST];
-            unsigned long long in[TEST];
-#pragma unroll
-            for (int u = 0; u < TEST; ++u)
-                raw[u] = sraw[buf + j0 + u * TK_WAVE + lane];
-#pragma unroll
-            for (int u = 0; u < TEST; ++u) {
-                // (box[a] is -lowest)
-                const float gx = __builtin_fmaxf(__builtin_fmaxf(-box[0] - raw[u].x, raw[u].x - box[3]), 0.0f);
-                const float gy = __builtin_fmaxf(__builtin_fmaxf(-box[1] - raw[u].y, raw[u].y - box[4]), 0.0f);
-                const float gz = __builtin_fmaxf(__builtin_fmaxf(-box[2] - raw[u].z, raw[u].z - box[5]), 0.0f);
-                const float bound = __builtin_fmaf(gz, gz, __builtin_fmaf(gy, gy, gx * gx));
-                in[u] = __builtin_amdgcn_ballot_w64(bound < reach);
-            }
-            if (st == 0 && j0 == 0) {  // uniform; these have been taken
-                in[0] = taken < TK_WAVE ? in[0] & (~0ull << taken) : 0ull;
-                in[1] = taken > TK_WAVE ? in[1] & (~0ull << (taken - TK_WAVE)) : in[1];
-            }
-#pragma unroll
-            for (int u = 0; u < TEST; ++u) {
-                const int below = __builtin_amdgcn_mbcnt_hi((unsigned)(in[u] >> 32),
-                                                            __builtin_amdgcn_mbcnt_lo((unsigned)in[u], 0));
-                if (__builtin_amdgcn_inverse_ballot_w64(in[u])) {
-                    const int to = (tail + below) & (RING - 1);
-                    const unsigned short key = (unsigned short)(16 * (buf + j0 + u * TK_WAVE + lane));
-                    ring[to] = key;
-                    if (to < CHUNK)
-                        ring[RING + to] = key;
+        for (int j0 = 0; j0 < cnt; j0 += BOXES ? TEST * TK_WAVE : STAGE) {
+            if constexpr (BOXES) {
+                if (moved) {  // uniform
+                    reach = tk_wave_extreme<true>(active ? max_key : -INF);
+                    moved = false;
                 }
-                tail += __builtin_popcountll(in[u]);
+                float4 raw[TEST];
+                unsigned long long in[TEST];
+#pragma unroll
+                for (int u = 0; u < TEST; ++u)
+                    raw[u] = sraw[buf + j0 + u * TK_WAVE + lane];
+#pragma unroll
+                for (int u = 0; u < TEST; ++u) {
+                    // (box[a] is -lowest)
+                    const float gx = __builtin_fmaxf(__builtin_fmaxf(-box[0] - raw[u].x, raw[u].x - box[3]), 0.0f);
+                    const float gy = __builtin_fmaxf(__builtin_fmaxf(-box[1] - raw[u].y, raw[u].y - box[4]), 0.0f);
+                    const float gz = __builtin_fmaxf(__builtin_fmaxf(-box[2] - raw[u].z, raw[u].z - box[5]), 0.0f);
+                    const float bound = __builtin_fmaf(gz, gz, __builtin_fmaf(gy, gy, gx * gx));
+                    in[u] = __builtin_amdgcn_ballot_w64(bound < reach);
+                }
+                if (st == 0 && j0 == 0)  // uniform; these have been taken
+                    in[0] = taken < TK_WAVE ? in[0] & (~0ull << taken) : 0ull;
+#pragma unroll
+                for (int u = 0; u < TEST; ++u) {
+                    const int below = __builtin_amdgcn_mbcnt_hi((unsigned)(in[u] >> 32),
+                                                                __builtin_amdgcn_mbcnt_lo((unsigned)in[u], 0));
+                    if (__builtin_amdgcn_inverse_ballot_w64(in[u])) {
+                        const int to = (tail + below) & (RING - 1);
+                        const unsigned short key = (unsigned short)(16 * (buf + j0 + u * TK_WAVE + lane));
+                        ring[to] = key;
+                        if (to < CHUNK)
+                            ring[RING + to] = key;
+                    }
+                    tail += __builtin_popcountll(in[u]);
+                }
+            } else if (!idle && stage0 + cnt > tail) {
+                tail = stage0 + cnt;
             }
             while (tail - head >= CHUNK)
                 sweep(CHUNK);
@@ -1034,8 +992,8 @@ __global__ __launch_bounds__(LANES) void knn_filter_kernel_f32(
     int *const ibuf = reinterpret_cast<int *>(skey + ROWS * ROW);
 #pragma unroll 1
     for (int part = 0; part < BLOCK / ROWS; ++part) {
-        const int row0 = qblock * BLOCK + part * ROWS;  // of the cloud's queries
-        int rows = n1 - row0;
+        const int row0 = base + part * ROWS;  // of the cloud's queries
+        int rows = (n1 - base < span ? n1 - base : span) - part * ROWS;
         if (rows <= 0)  // uniform
             break;
         rows = rows < ROWS ? rows : ROWS;
@@ -1084,6 +1042,144 @@ __global__ __launch_bounds__(LANES) void knn_filter_kernel_f32(
         }
     }
 }
+
+template <int KMAX, bool SOA, bool WEIGHTS, int LANES, int KIND>
+__global__ __launch_bounds__(LANES) void knn_filter_kernel_f32(
+    const float *__restrict__ query, const float *__restrict__ key,
+    float *__restrict__ distance, int64_t *__restrict__ index, float *__restrict__ weight,
+    float eps, int blocks_per_batch, int n1, int n2, int k)
+{
+    using F = KnnFilter<KMAX, LANES>;
+    constexpr int BLOCK = F::BLOCK, NW = F::NW, CELLS = F::CELLS;
+    constexpr bool BOXES = KIND != KNN_EVERY_KEY, ORDERED = KIND == KNN_BOXES_UNLESS_ORDERED;
+    __shared__ __align__(16) float skey[F::LDS_FLOATS];
+    // (a list's beginning comes once more behind it)
+    __shared__ __align__(16) unsigned short srings[BOXES ? NW * (F::RING + F::CHUNK) : 1];
+    __shared__ float sred[NW][F::RED];
+    const int tid = threadIdx.x;
+    const int lane = tid & (TK_WAVE - 1);
+    const int wave = tid / TK_WAVE;
+    const bool second = ORDERED && blockIdx.y > 0;
+    const int b = blockIdx.x / blocks_per_batch;
+    const int qblock = blockIdx.x - b * blocks_per_batch;
+    const float *__restrict__ K = key + (int64_t)b * n2 * 3;
+    const float *__restrict__ Q = query + (int64_t)b * n1 * 3;
+    const float INF = __builtin_huge_valf();
+
+    // ---- bounding boxes of the key cloud (its centre, and a bound of the centred norms) and of the
+    // workgroup's queries ----
+    const int base = qblock * BLOCK;
+    float ends[6] = {-INF, -INF, -INF, -INF, -INF, -INF};  // -lowest, highest
+    for (int j = tid; j < n2; j += BLOCK) {
+        const float v[3] = {knn_coord<SOA>(K, n2, j, 0), knn_coord<SOA>(K, n2, j, 1), knn_coord<SOA>(K, n2, j, 2)};
+        knn_reach_out(ends, v);
+    }
+    KnnFrame<F::PER> frame;
+    knn_filter_fetch<SOA, F::PER, BLOCK>(frame.pre, K, n2, 0);
+    float qends[6] = {-INF, -INF, -INF, -INF, -INF, -INF};
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+        frame.own[a] = 0.0f;  // (of a query that does not exist)
+    if (BOXES && base + tid < n1) {
+#pragma unroll
+        for (int a = 0; a < 3; ++a)
+            frame.own[a] = knn_coord<SOA>(Q, n1, base + tid, a);
+        knn_reach_out(qends, frame.own);
+    }
+    const auto box_of_wave = [&](float (&e)[6], int at) {
+        tk_wave_max_six<64>(e);
+        if (lane == TK_WAVE - 1) {
+#pragma unroll
+            for (int a = 0; a < 6; ++a)
+                sred[wave][at + a] = e[a];
+        }
+    };
+    box_of_wave(ends, 0);
+    if constexpr (BOXES)
+        box_of_wave(qends, 6);
+    if constexpr (ORDERED) {
+        float first[6] = {-INF, -INF, -INF, -INF, -INF, -INF};  // of the first stage's keys
+        if (tid < n2) {
+            const float v[3] = {frame.pre[0].x, frame.pre[0].y, frame.pre[0].z};
+            knn_reach_out(first, v);
+        }
+        box_of_wave(first, 12);
+    }
+    if constexpr (BOXES) {  // the sort's counters and its table
+        unsigned *const cnt = reinterpret_cast<unsigned *>(skey);
+        unsigned short *const curve = reinterpret_cast<unsigned short *>(cnt + CELLS + 4);
+        if (tid < CELLS / 8)
+            reinterpret_cast<uint4 *>(curve)[tid] = reinterpret_cast<const uint4 *>(knn_curve.place)[tid];
+        for (int i = tid; i <= CELLS; i += BLOCK)
+            cnt[i] = 0u;
+    }
+    __syncthreads();
+    // (a wave's values to a lane: read one after the other they took more than the reductions in the waves)
+    float all[6], queries[6], firsts[6];
+    const auto box_of_all = [&](float (&e)[6], int at) {
+#pragma unroll
+        for (int a = 0; a < 6; ++a)
+            e[a] = sred[lane & (NW - 1)][at + a];
+        tk_wave_max_six<8>(e);
+#pragma unroll
+        for (int a = 0; a < 6; ++a)
+            e[a] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, e[a]), 7));
+    };
+    box_of_all(all, 0);
+    if constexpr (BOXES)
+        box_of_all(queries, 6);
+    if constexpr (ORDERED)
+        box_of_all(firsts, 12);
+    float kmax2 = 0.0f;
+    bool ordered = false;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const float l = all[a], h = all[3 + a];
+        if (ORDERED)
+            ordered = ordered || firsts[3 + a] + firsts[a] < 0.6f * (h + l);
+        const float middle = 0.5f * h - 0.5f * l, side = __builtin_fmaxf(h - middle, middle + l);
+        frame.centre[a] = middle;
+        // (the operations of a norm, each of which is monotone: no centred key is beyond it)
+        kmax2 = a == 0 ? side * side : __builtin_fmaf(side, side, kmax2);
+        if (BOXES) {
+            frame.origin[a] = -queries[a];
+            const float extent = queries[3 + a] + queries[a];
+            frame.cells[a] = extent > 0.0f ? 7.99f / extent : 0.0f;  // also 0 for NaN / inf extents
+        }
+    }
+    const float c0 = frame.centre[0], c1 = frame.centre[1], c2 = frame.centre[2];
+    bool safe = (c0 - c0 == 0.0f) && (c1 - c1 == 0.0f) && (c2 - c2 == 0.0f) && (kmax2 < 1e30f);
+    const float ext = __builtin_sqrtf(kmax2);
+    const int ebits = (int)((__builtin_bit_cast(unsigned, ext) >> 23) & 0xffu) - 127;
+    safe = safe && (ext == 0.0f || (ebits >= -40 && ebits <= 40));
+    // Half the box's diagonal comes to [2, 4): its largest side is 1/sqrt(3) of that or more, and a key on it.
+    frame.scale = (!safe || ext == 0.0f) ? 1.0f : __builtin_bit_cast(float, (unsigned)(128 - ebits) << 23);
+    frame.kmax = __builtin_sqrtf(kmax2) * frame.scale * 1.000001f;
+
+    // (the same in all lanes, which the compiler cannot know)
+    const bool every = !BOXES || (ORDERED && __builtin_amdgcn_readfirstlane(ordered) != 0);
+    if (__builtin_amdgcn_readfirstlane(!safe || (second && !every))) {
+        if (!second)
+            knn_batched_body<KMAX, SOA, WEIGHTS>(query, key, distance, index, weight, eps, b, base + tid, n1, n2, k,
+                                                 skey);
+        return;
+    }
+    const auto run = [&](auto boxes, int from, int span) {
+        knn_filter_queries<KMAX, SOA, WEIGHTS, LANES, decltype(boxes)::value>(Q, K, distance, index, weight, eps, b, from,
+                                                                              span, n1, n2, k, frame, skey, srings, sred);
+    };
+    if constexpr (KIND == KNN_EVERY_KEY) {
+        run(std::false_type{}, base, BLOCK);
+    } else if constexpr (KIND == KNN_BOXES) {
+        run(std::true_type{}, base, BLOCK);
+    } else {
+        if (!every)
+            run(std::true_type{}, base, BLOCK);
+        else
+            run(std::false_type{}, second ? base + BLOCK / 2 : base, gridDim.y > 1 ? BLOCK / 2 : BLOCK);
+    }
+}
+
 
 // fp32 variant with the slots in LDS as a per-lane tournament tree.
 //
@@ -1737,12 +1833,12 @@ inline bool knn_filter_takes(int64_t B, int n1, int n2, int k)
     return k <= 32 && n2 >= 64 && (k <= 4 || n2 <= (k <= 16 ? 1 << 27 : 1 << 26)) && B * bpb <= TK_MAX_I32;
 }
 
-template <int KMAX, bool SOA, bool WEIGHTS, int LANES>
+template <int KMAX, bool SOA, bool WEIGHTS, int LANES, int KIND>
 int knn_filter_launch_as(const float *query, const float *key, float *distance, int64_t *index,
-                         float *weight, float eps, int64_t B, int n1, int n2, int k, hipStream_t s)
+                         float *weight, float eps, int64_t B, int n1, int n2, int k, hipStream_t s, bool halves = false)
 {
     const int64_t bpb = ((int64_t)n1 + LANES - 1) / LANES;
-    hipLaunchKernelGGL((knn_filter_kernel_f32<KMAX, SOA, WEIGHTS, LANES>), dim3((unsigned)(B * bpb)),
+    hipLaunchKernelGGL((knn_filter_kernel_f32<KMAX, SOA, WEIGHTS, LANES, KIND>), dim3((unsigned)(B * bpb), halves ? 2 : 1),
                        dim3(LANES), 0, s, query, key, distance, index, weight, eps, (int)bpb, n1, n2, k);
     return tk_launch_status();
 }
@@ -1752,23 +1848,43 @@ int knn_filter_launch(const float *query, const float *key, float *distance, int
                       float *weight, float eps, int64_t B, int n1, int n2, int k, hipStream_t s,
                       bool whatever_the_size = false)
 {
-    // 512 lanes: two workgroups (16 waves) per CU. A launch of few such workgroups leaves CUs
-    // without one: 256 lanes then, unless there are keys enough for the boxes of 512 sorted queries to pay (us, 256 and 512
-    // lanes: 8 x 4096 queries on 1024 keys k = 8 32.9, 34.8, on 2048 k = 3 39.0, 33.9, k = 16 62.9, 69.1, on 8192 k = 3 114, 78,
-    // k = 16 155, 129, 12 x 4096 on 4096 k = 8 76.4, 66.2, 2 x 16384 on 4096 k = 3 63, 50, 3 x 10000 on 16384 k = 16 280, 196;
-    // keys in the order of a coordinate, of which each is inserted, take fewer waves a SIMD better, 8 x 4096 on 8192 k = 16 342,
-    // 396, as before the boxes, 317). 32 slots leave room for three waves per
-    // SIMD, twelve a CU: three workgroups of 256 lanes or one of 512.
+    // 512 lanes: two workgroups (16 waves) per CU. A launch of few such workgroups leaves CUs without one: 256 lanes then,
+    // unless there are keys enough for boxes. The times of the instances over that of the same kernel
+    // without boxes and without keys put to all queries (256 lanes up to 128 or 160 workgroups of 512, else 512):
+    //   8 x 4096 queries, in launches of few     every key, 256 lanes   512   boxes, unless ordered
+    //     2048 keys in random order k = 3                 0.90           0.94          0.91
+    //     2048 k = 8                                      0.89           0.99          0.96
+    //     4096 k = 8                                      0.90           0.96          0.85
+    //     4096 k = 16                                     0.94           1.08          1.01
+    //     8192 k = 16                                     0.95           1.04          0.91
+    //   16 x 8192, a workgroup to a CU: 4096 k = 16       1.02           0.96          0.91
+    //     2048 k = 8                                      0.97           0.91          0.91 (in clusters 0.99, 0.92, 0.97)
+    //   32 x 8192, two: 1024 k = 3                        1.04           0.87          0.87 (boxes; voxels in order 0.73)
+    // Clouds of up to 256 queries have half of the 512 lanes to help with the staging, and one or two waves more to the
+    // boxes' one: 200 x 120 on 4096 k = 8 1.07, 0.94; 80 x 250 on 8192 k = 16 0.95, 0.86, boxes 0.95; from 16384 keys on
+    // boxes are even for k = 3, 0.89 and 0.83. 32 slots leave room for three waves per SIMD, twelve a CU: three workgroups of 256
+    // lanes or one of 512.
     if (!(whatever_the_size || knn_filter_takes(B, n1, n2, k)))
         return TK3D_ERR_UNSUPPORTED;
+    const auto as = [&](auto lanes, auto kind, bool halves = false) {
+        return knn_filter_launch_as<KMAX, SOA, WEIGHTS, decltype(lanes)::value, decltype(kind)::value>(
+            query, key, distance, index, weight, eps, B, n1, n2, k, s, halves);
+    };
+    using Wide = std::integral_constant<int, 512>;
+    using Narrow = std::integral_constant<int, 256>;
+    using EveryKey = std::integral_constant<int, KNN_EVERY_KEY>;
     if constexpr (KMAX <= 16) {
-        const int64_t bpb = ((int64_t)n1 + 511) / 512;
-        if (B * bpb > (KMAX <= 8 ? 128 : 160) || n2 >= 512 * KMAX)
-            return knn_filter_launch_as<KMAX, SOA, WEIGHTS, 512>(query, key, distance, index, weight,
-                                                                 eps, B, n1, n2, k, s);
+        const int64_t wide = B * (((int64_t)n1 + 511) / 512), cus = tk_cu_count();
+        const bool some = n1 > 256 || (n1 > 128 && n2 >= 4096 * KMAX);
+        if (some && wide > cus && n2 >= 1024)
+            return as(Wide{}, std::integral_constant<int, KNN_BOXES>{});
+        const bool half = 2 * wide <= cus;
+        if (some && wide <= cus && n2 >= (half ? 512 * KMAX : 128 * KMAX + 1536))
+            return as(Wide{}, std::integral_constant<int, KNN_BOXES_UNLESS_ORDERED>{}, half);
+        if (n1 <= 256 || wide > (KMAX <= 8 ? 128 : 160))
+            return as(Wide{}, EveryKey{});
     }
-    return knn_filter_launch_as<KMAX, SOA, WEIGHTS, 256>(query, key, distance, index, weight, eps, B,
-                                                         n1, n2, k, s);
+    return as(Narrow{}, EveryKey{});
 }
 
 // Rows of k <= 64 results in place: ascending distance (equal ones in slot order, NaNs last, as a

@@ -163,8 +163,8 @@ __device__ __forceinline__ float tk_min_of_halves(float v)
     return tk_min_f32(b.x, b.y);
 }
 
-// The maxima over the wave (LANES 64, left in lane 63) or over each half of it (32, in lanes 31 and 63) of six values
-// at once: the steps of one value are the wait between those of another, and a maximum takes its operand from the
+// The maxima over the wave (LANES 64, left in lane 63), over each half of it (32, in lanes 31 and 63) or over the first
+// eight lanes (8, in lane 7) of six values at once: the steps of one value are the wait between those of another, and a maximum takes its operand from the
 // other lane itself. One by one, through moves, the compiler makes it five instructions a step.
 template <int LANES> __device__ __forceinline__ void tk_wave_max_six(float (&v)[6])
 {
@@ -172,6 +172,15 @@ template <int LANES> __device__ __forceinline__ void tk_wave_max_six(float (&v)[
     "v_max_f32_dpp %0, %0, %0 " HOW "\n\tv_max_f32_dpp %1, %1, %1 " HOW      \
     "\n\tv_max_f32_dpp %2, %2, %2 " HOW "\n\tv_max_f32_dpp %3, %3, %3 " HOW \
     "\n\tv_max_f32_dpp %4, %4, %4 " HOW "\n\tv_max_f32_dpp %5, %5, %5 " HOW "\n\t"
+    if constexpr (LANES == 8) {
+        asm("s_nop 1\n\t"
+            TK_STEP("row_shr:1 row_mask:0xf bank_mask:0xf")
+            TK_STEP("row_shr:2 row_mask:0xf bank_mask:0xf")
+            TK_STEP("row_shr:4 row_mask:0xf bank_mask:0xf")
+            "s_nop 1"
+            : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]));
+        return;
+    }
     asm("s_nop 1\n\t"
         TK_STEP("row_shr:1 row_mask:0xf bank_mask:0xf")
         TK_STEP("row_shr:2 row_mask:0xf bank_mask:0xf")
