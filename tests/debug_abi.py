@@ -92,6 +92,16 @@ def knn_filter(query, key, k):
     return dist, idx
 
 
+def knn_wave_queries(keys, k):
+    """Up to how many queries float32 KNN gives each of them a wave."""
+    from torkit3d_amd import _lib
+    from torkit3d_amd._lib import i64
+
+    fn = getattr(_lib.lib(), "tk3d_debug_knn_wave_queries")
+    fn.restype = ctypes.c_int64
+    return fn(i64(keys), i64(k))
+
+
 def mfma_dot16(key_terms, query_terms):
     """scores [T,32,32] of one matrix instruction per tile; key_terms, query_terms: int16/uint16
     device tensors [T,32,16] of fp16 bit patterns."""

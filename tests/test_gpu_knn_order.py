@@ -6,7 +6,8 @@ import pytest
 import torch
 
 import oracle
-from debug_abi import knn_filter
+from debug_abi import knn_filter, knn_wave_queries
+from torkit3d_amd.ops.knn_points import knn_points
 
 pytestmark = pytest.mark.gpu
 
@@ -64,3 +65,19 @@ def test_workgroups_to_a_cu(cuda, b, n2, k):
     for at in range(0, b, few):
         part = knn_filter(torch.from_numpy(q[at:at + few]).to(cuda), torch.from_numpy(key[at:at + few]).to(cuda), k)
         assert torch.equal(got[0][at:at + few], part[0]) and torch.equal(got[1][at:at + few], part[1])
+
+
+# ---- either side of the lines up to which a query has a wave, whatever they are ----
+
+@pytest.mark.parametrize("n2,k", [(64, 2), (512, 3), (512, 8), (513, 8), (1024, 16), (1025, 1), (2048, 8), (4096, 5), (4097, 3),
+                                  (8192, 16), (8193, 9), (1024, 20), (4096, 32), (4097, 17), (32769, 24)])
+def test_both_sides_of_a_wave_to_a_query(cuda, n2, k):
+    """A cloud of as many queries as have a wave each, and of one more, which do not: the same rows."""
+    limit = knn_wave_queries(n2, k)
+    query, key = (torch.from_numpy(cloud(kind, 1, n, n)).to(cuda) for kind, n in (("random", limit + 1), ("by x", n2)))
+    few = knn_points(query[:, :limit].contiguous(), key, k)
+    many = knn_points(query, key, k)
+    assert torch.equal(few[0], many[0][:, :limit]) and torch.equal(few[1], many[1][:, :limit])
+    some = slice(limit - 40, limit + 1)
+    d, i = oracle.knn(query[:, some].cpu().numpy(), key.cpu().numpy(), k)
+    assert np.array_equal(many[0][:, some].cpu().numpy(), d) and np.array_equal(many[1][:, some].cpu().numpy(), i)

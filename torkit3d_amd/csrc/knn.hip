@@ -1689,23 +1689,38 @@ __global__ __launch_bounds__(KNN_BLOCK, LONG ? 1 : 8) void knn_wave_kernel_f32(
     }
 }
 
-// Where a wave per query wins: its time goes with the number of queries, that of the kernels of a lane per query hardly
-// does while they leave CUs idle. us, it and the pre-filtered kernel, 20480 queries in clouds of 4096: on 128 keys k = 3 12.0,
-// 13.6, k = 8 16.8, 16.3, k = 16 21.7, 21.6, k = 32 28.0, 33.1; on 1024 k = 3 17.8, 25.8, k = 16 38.6, 47.0, k = 32 58, 78;
-// on 16384 k = 3 147, 151, k = 16 153, 193, k = 32 164, 327. 24576 queries: on 128 keys k = 16 23.8, 22.6, k = 32 30.7, 34.5;
-// on 1024 k = 3 20.4, 26.2, k = 16 44.6, 46.3; on 4096 k = 3 49, 49, k = 16 71, 90; on 16384 k = 3 174, 153, k = 32 192, 325.
-// 25600 in clouds of 128, on 2048 keys k = 3 29.1, 38.5, k = 16 56.9, 62.3. 32768: on 128 k = 3 15.9, 12.6, on 4096 k = 3
-// 64.5, 52.7, k = 16 91, 91. With more than 32 neighbours the others keep a tree in LDS: 49152 queries on 128 keys k = 64 59,
-// 72, on 4096 301, 549; 65536 on 1024 253, 243; 131072 on 128 k = 40 146, 136, on 4096 k = 40 570, 985, k = 64 771, 1143.
-// Keys in the order of a coordinate, of which many more are inserted, take more of both and leave the order as it is (20480
-// queries on 16384 keys k = 3 214, 348, 98304 on 4096 k = 64 1208, 1979). On 1024 keys and fewer, up to 16 neighbours, the two
-// are close from 18432 queries on (on 512 k = 8 22.1, 24.0).
-inline bool knn_wave_pays(int64_t queries, int64_t keys, int k)
+// Up to how many queries a wave per query wins: its time goes with their number, that of the kernels of a lane per query
+// hardly does while they leave CUs idle. Its time over that of the pre-filtered kernel, keys in random order and in that of a
+// coordinate, clouds of 512 to 4096 queries:
+//   queries       keys    64         512        1024       2048       4096       8192       16384
+//   20480  k = 1       0.89 0.82  0.68 0.66  0.65 0.65  0.76 0.68  0.96 0.68  1.13 0.73  1.25 0.80
+//          k = 3       1.07 1.08  0.89 0.92  0.80 0.86  0.74 0.90  0.88 0.90  1.03 0.88  1.18 0.84
+//          k = 8       1.16 1.29  1.05 1.08  0.96 1.05  0.82 1.00  0.79 1.05  0.89 0.99  1.04 0.95
+//          k = 16      1.10 1.22  1.06 0.95  0.99 0.95  0.88 0.92  0.75 0.89  0.72 0.94  0.88 0.89
+//   24576  k = 1       1.03 0.91  0.79 0.75  0.75 0.73  0.90 0.76  1.12 0.78  1.36 0.85  1.48 0.94
+//          k = 3       1.22 1.24  1.03 1.00  0.92 0.97  0.86 1.03  1.04 1.02  1.24 1.01  1.37 0.99
+//          k = 8       1.34 1.44  1.20 1.21  1.11 1.18  0.95 1.12  0.92 1.19  1.07 1.14  1.26 1.09
+//          k = 16      1.26 1.37  1.22 1.07  1.16 1.07  1.01 1.03  0.87 1.01  0.85 1.06  1.04 1.01
+//          k = 32      0.92 0.96  0.96 0.85  0.98 0.85  0.92 0.82  0.83 0.82  0.74 0.79  0.69 0.76
+//   32768  k = 1       1.25 1.13  0.95 0.93  0.94 0.91  1.15 0.97  1.48 1.00  1.79 1.07  1.99 1.23
+//          k = 20      1.20 1.24  1.16 0.99  1.16 1.00  1.06 0.99  0.97 0.97  0.89 0.94  0.93 0.90
+//          k = 32      1.17 1.19  1.22 1.06  1.26 1.06  1.17 1.03  1.06 1.03  0.98 0.99  0.89 0.95
+// (on 65536, 32768 queries in clouds of 128 k = 20 1.06 1.29). With more than 32 neighbours the others keep a tree in LDS: us, the
+// wave and the tree, 49152 queries on 128 keys k = 64 59, 72, on 4096 301, 549; 65536 on 1024 253, 243; 131072 on 128 k = 40 146,
+// 136, on 4096 k = 40 570, 985, k = 64 771, 1143.
+inline int64_t knn_wave_queries(int64_t keys, int64_t k)
 {
     if (k > 32)
-        return k <= 64 && queries <= (keys >= 2048 ? 131072 : 49152);
-    return queries <= (keys <= 1024 ? 18432 : k <= 16 && keys > 4096 ? 20480 : 25600);
+        return k > 64 ? 0 : keys >= 2048 ? 131072 : 49152;
+    if (k > 16)
+        return keys <= 1024 ? 25600 : keys <= 4096 ? 28672 : keys <= 32768 ? 32768 : 25600;
+    if (keys <= 1024)
+        return k <= 2 ? 30720 : k <= 4 || keys > 512 ? 20480 : 18432;
+    if (keys <= 4096)
+        return k > 4 && k <= 8 ? 23552 : 25600;
+    return k > 8 && keys <= 8192 ? 25600 : 20480;
 }
+inline bool knn_wave_pays(int64_t queries, int64_t keys, int64_t k) { return queries <= knn_wave_queries(keys, k); }
 
 template <bool SOA, bool WEIGHTS>
 int knn_wave_launch(const float *query, const float *key, float *distance, int64_t *index,
@@ -2240,6 +2255,8 @@ int tk3d_knn_distance_ordered_f64(const double *query, const double *key, int ch
     return knn_ordered<double>(query, key, channels_first != 0, B, N1, N2, k, sorted, root, distance,
                                index, stream);
 }
+
+int64_t tk3d_debug_knn_wave_queries(int64_t keys, int64_t k) { return knn_wave_queries(keys, k); }
 
 int tk3d_debug_knn_wave_f32(const float *query, const float *key, int channels_first, int64_t B,
                             int64_t N1, int64_t N2, int64_t k, float *distance, int64_t *index,

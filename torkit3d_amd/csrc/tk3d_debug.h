@@ -70,6 +70,9 @@ int tk3d_debug_knn_wave_f32(const float *query, const float *key, int channels_f
                             int64_t N1, int64_t N2, int64_t k, float *distance, int64_t *index,
                             void *stream);
 
+/* Up to how many queries (of all clouds) fp32 KNN gives each of them a wave; 0 for k > 64. */
+int64_t tk3d_debug_knn_wave_queries(int64_t keys, int64_t k);
+
 /* tk3d_knn_distance_f32 through the pre-filtered kernel (knn_filter_kernel_f32, scores on
  * the matrix cores) whatever the launch size; k <= 32. */
 int tk3d_debug_knn_filter_f32(const float *query, const float *key, int64_t B, int64_t N1,
