@@ -273,7 +273,7 @@ def test_slot_order_of_the_hand_worked_mink_run(cuda, k, dtype):
 # in per-lane queues and are inserted later with the exact arithmetic. Whatever the input,
 # distances, indices and slot order must be MinK's: these cases aim at its error bound, its
 # queues, its stage boundaries and its fallbacks. (Sizes are inside the range where the dispatcher takes this
-# kernel: more than 18432 queries, 64 keys or more.) ----
+# kernel: more queries than knn_wave_queries in csrc/knn.hip says, at most 32768 here, 64 keys or more.) ----
 
 def _filter_case(kind, g, k, b=8, n1=8192 + 5, n2=2048 + 37):  # ragged: partial workgroup, partial chunk
     q, key = uniform_cloud(g, b, n1), uniform_cloud(g, b, n2)

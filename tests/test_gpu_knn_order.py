@@ -81,3 +81,23 @@ def test_both_sides_of_a_wave_to_a_query(cuda, n2, k):
     some = slice(limit - 40, limit + 1)
     d, i = oracle.knn(query[:, some].cpu().numpy(), key.cpu().numpy(), k)
     assert np.array_equal(many[0][:, some].cpu().numpy(), d) and np.array_equal(many[1][:, some].cpu().numpy(), i)
+
+
+@pytest.mark.parametrize("transpose", [False, True])
+@pytest.mark.parametrize("kind", ["random", "lattice by x"])
+@pytest.mark.parametrize("n2,k", [(40, 33), (200, 48), (300, 64), (2100, 40)])
+def test_more_than_32_neighbours_beyond_a_wave_to_a_query(cuda, kind, n2, k, transpose):
+    """The tree in LDS, rows and planes, and the kernel that puts its rows in order: the sizes follow the line."""
+    limit, b = knn_wave_queries(n2, k), 3
+    n1 = limit // b + 7
+    assert b * n1 > limit
+    few = cloud("random", b, 50, 5)
+    q, key = np.tile(few, (1, n1 // 50 + 1, 1))[:, :n1], cloud(kind, b, n2, n2)
+    d, i = (np.tile(t, (1, n1 // 50 + 1, 1))[:, :n1] for t in oracle.knn(few, key, k))
+    clouds = [torch.from_numpy(np.ascontiguousarray(t.transpose(0, 2, 1) if transpose else t)).to(cuda) for t in (q, key)]
+    got = knn_points(*clouds, k, transpose=transpose)
+    assert np.array_equal(got[0].cpu().numpy(), d) and np.array_equal(got[1].cpu().numpy(), i)
+    order = np.argsort(d, axis=2, kind="stable")
+    got = knn_points(*clouds, k, transpose=transpose, sorted=True, sqrt_distance=True)
+    assert np.array_equal(got[0].cpu().numpy(), np.sqrt(np.take_along_axis(d, order, 2)))
+    assert np.array_equal(got[1].cpu().numpy(), np.take_along_axis(i, order, 2))
