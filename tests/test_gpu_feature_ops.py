@@ -425,3 +425,32 @@ def test_long_row_scatter_at_the_edges_of_its_chunks(cuda, n1, b, n2):
     got = _C.group_points_backward_cuda(grad.to(cuda), index.to(cuda), n1).cpu()
     want = torch.zeros(b, c, n1).scatter_add_(2, index.view(b, 1, -1).expand(b, c, -1), grad.view(b, c, -1))
     assert torch.equal(got, want)
+
+
+# one channel a workgroup (chunks of 512 points) and two (of 256); as many jobs as workgroups, a number that no XCD
+# divides, and more than CUs: a workgroup's second job, whose first chunk is on its way
+@pytest.mark.parametrize("n1,chunk,b,c", [(8385, 512, 4, 32), (16384, 512, 4, 33), (16384, 512, 8, 40),
+                                          (4161, 256, 4, 63), (8384, 256, 8, 64)])
+@pytest.mark.parametrize("chunks,more", [(16, -1), (16, 0), (16, 1), (32, 1), (47, 3)])
+def test_long_row_scatter_beyond_a_chunk_to_a_wave(cuda, n1, chunk, b, c, chunks, more):
+    """Whole rows (no segments: 128 groups of channels or more) whose points are one chunk for each of the sixteen waves,
+    and some beyond. A term that its wave's first chunk, which sets the scale, does not see has the rows added again;
+    without that it would not fit. Whole numbers make every sum exact."""
+    from torkit3d_amd import _C
+
+    points = chunks * chunk + more
+    groups = b * (c if chunk == 512 else -(-c // 2))
+    assert groups >= 128  # (then the launch makes no segments)
+    per_wave = -(-(-(-points // chunk)) // 16)
+    assert (per_wave > 1) == (points > 16 * chunk)
+    g = gen(n1 + points)
+    index = torch.randint(0, n1, (b, points, 1), generator=g)
+    grad = torch.randint(-3, 4, (b, c, points, 1), generator=g).float()
+    if per_wave > 1:
+        unseen = (3 * per_wave + per_wave - 1) * chunk + 5  # in the last chunk of the fourth wave
+        assert unseen < points and unseen // chunk % per_wave > 0
+        grad[:, :: 3, unseen] = 4096.0  # (over eight times what the first chunks have)
+        grad[-1, -1, unseen] = -4096.0
+    got = _C.group_points_backward_cuda(grad.to(cuda), index.to(cuda), n1).cpu()
+    want = torch.zeros(b, c, n1).scatter_add_(2, index.view(b, 1, -1).expand(b, c, -1), grad.view(b, c, -1))
+    assert torch.equal(got, want)
