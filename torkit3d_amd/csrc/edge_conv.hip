@@ -300,7 +300,8 @@ __global__ void __launch_bounds__(kBlock)
 
 // The same from g, extreme and arg themselves: a workgroup has CH channels of a cloud, whose sums lie in LDS. kPart
 // points at a time, every lane finds the values of its points and the neighbours that they belong to; then one wave a
-// channel adds them, in the order of the points, so that every run adds in the same order. The two kernels above look
+// channel adds them, 64 points to an atomic. Lanes that meet at a neighbour are taken in their order, so that every run adds
+// in that of the points: the hardware's doing, which nothing here enforces and a test holds. The two kernels above look
 // at all K edges into a point for the few that count, 8 bytes a channel of each, and pass 8 bytes a value through
 // memory; here a value looks up its one neighbour. 8 x 2048 points, 20 neighbours, 64 channels: 26.4 us in two launches,
 // now 10.5, most of it the trips to g, to the neighbours and through LDS, one behind the other; 128 channels 40.8, 14.
