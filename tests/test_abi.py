@@ -304,3 +304,18 @@ class GroupedPool(ctypes.Structure):  # tk3d_mlp_grouped_pool
 def test_grouped_layers_that_share_a_launch(lib, widths, b, m, s, taken):
     sizes = GroupedPool(sizes=(67, b, 4 * m, m, s, *widths))
     assert bool(lib.tk3d_mlp_grouped_pool_supported(ctypes.byref(sizes))) is taken
+
+
+def test_edge_backward_workspace_has_the_selected_values_only_where_they_may_be_gathered(lib):
+    size = lib.tk3d_mlp_edge_backward_bytes
+    size.restype = ctypes.c_int64
+    b, o, c = 1, 64, 3
+
+    def bytes_of(n):
+        return size(*[ctypes.c_int(v) for v in (b, n, o, c)])
+
+    selected = 8 * b * o * 6144
+    assert bytes_of(6145) - bytes_of(6144) >= selected
+    # rows that are added in LDS: both halves of the gradient, the points as rows and their sums, and partial sums, which
+    # do not grow with the points beyond their parts
+    assert bytes_of(6144) - bytes_of(2048) < 4 * b * 4096 * (2 * o + 3 * c) + selected // 2

@@ -391,6 +391,9 @@ __global__ void __launch_bounds__(kOwners)
 
 int64_t owners_lds(int N, int channels) { return (int64_t)channels * (N * 8 + kPart * 8); }
 
+// Rows up to here are added in LDS whatever the device; what longer ones take depends on its CUs.
+bool may_gather(int N) { return N > 3 * kPart; }
+
 template <int CH>
 int edge_owners(const float *g, const float *extreme, const unsigned char *arg, const int64_t *index, int B, int N,
                 int K, int O, const tk3d_mlp_norm &norm, const float *coef, float *out, hipStream_t stream)
@@ -942,7 +945,7 @@ int64_t tk3d_mlp_edge_backward_bytes(int B, int N, int O, int C)
 {
     const int64_t partial = (int64_t)weight_runs(B, N, O, C).parts * 2 * tiles_of(O) * kTile * C * 8;
     const int64_t points = (int64_t)B * N * 4;
-    return partial + points * (2 * O + 2 * O + 3 * (int64_t)C);
+    return partial + points * ((may_gather(N) ? 2 * O : 0) + 2 * O + 3 * (int64_t)C);
 }
 
 int tk3d_mlp_edge_backward_f32(const float *g, const float *extreme, const unsigned char *arg,
@@ -955,10 +958,10 @@ int tk3d_mlp_edge_backward_f32(const float *g, const float *extreme, const unsig
     const hipStream_t stream = (hipStream_t)stream_;
     const WeightRuns r = weight_runs(B, N, O, C);
     const int half = tiles_of(O) * kTile;
-    // the workspace: partial sums, sel [B, N, O] of 8 bytes, duv [B, 2 O, N], rows [B, N, C], st [B, 2 C, N]
+    // the workspace: partial sums, sel [B, N, O] of 8 bytes if the sums may be gathered, duv [B, 2 O, N], rows [B, N, C], st [B, 2 C, N]
     double *partial = reinterpret_cast<double *>(workspace);
     int2 *sel = reinterpret_cast<int2 *>(partial + (int64_t)r.parts * 2 * half * C);
-    float *duv = reinterpret_cast<float *>(sel + (int64_t)B * N * O);
+    float *duv = reinterpret_cast<float *>(sel + (may_gather(N) ? (int64_t)B * N * O : 0));
     float *rows = duv + (int64_t)B * N * 2 * O, *st = rows + (int64_t)B * N * C;
     const int tiles = (N + kPoints - 1) / kPoints, blocks = (O + kChannels - 1) / kChannels;
     const int gathers = (N + kGather - 1) / kGather * B;
@@ -968,7 +971,7 @@ int tk3d_mlp_edge_backward_f32(const float *g, const float *extreme, const unsig
     // 16384 182.3, 174.8), as are rows that LDS does not hold. Two channels of a workgroup share the lines of the
     // neighbours, as long as that leaves every CU a workgroup (512 rows of 2048: 10.5 us, one channel 12.5).
     const int64_t channels = (int64_t)B * O;
-    if (owners_lds(N, 1) <= kOwnersLds && (channels * 2 >= tk_cu_count() || N <= 3 * kPart)) {
+    if (!may_gather(N) || (owners_lds(N, 1) <= kOwnersLds && channels * 2 >= tk_cu_count())) {
         const bool two = channels >= 2 * tk_cu_count() && owners_lds(N, 2) <= kOwnersLds;
         rc = two ? edge_owners<2>(g, extreme, arg, index, B, N, K, O, *norm, coef, duv, stream)
                  : edge_owners<1>(g, extreme, arg, index, B, N, K, O, *norm, coef, duv, stream);
