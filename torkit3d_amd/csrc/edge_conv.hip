@@ -212,8 +212,9 @@ __device__ __forceinline__ int point_of(int entry, int N)
 }
 
 // A thread's part of a tile of kChannels by kPoints: a point, and every kChannelStep-th channel. Its loads leave
-// together: one value after the other, each behind the trip of the one before, edge_select_kernel took
-// 11.2 us for 6.3 now, edge_rows_kernel 6.2 for 4.8 (8 x 2048 points, 64 channels).
+// together, of the channels that some thread has: one value after the other, each behind the trip of the one before,
+// edge_rows_kernel took 6.2 us for 4.8 now (8 x 2048 points, 64 channels), edge_select_kernel 11.2 for 6.3 on those
+// sizes, which no longer come to it.
 constexpr int kChannelStep = kBlock / kPoints, kOwn = kChannels / kChannelStep;
 
 // The sparse gradient, [B, N, O] of (a e, place), from g, extreme and arg [B, O, N].
@@ -225,18 +226,20 @@ __global__ void __launch_bounds__(kBlock)
     const int tid = threadIdx.x, b = blockIdx.z, first = blockIdx.x * kPoints;
     const int cbase = blockIdx.y * kChannels;
     const int p = tid % kPoints, ch0 = tid / kPoints;
-    float y[kOwn], gv[kOwn], a[kOwn];
-    int place[kOwn];
-    f32x4 ss[kOwn];
+    float y[kOwn] = {}, gv[kOwn] = {}, a[kOwn] = {};
+    int place[kOwn] = {};
+    f32x4 ss[kOwn] = {};
 #pragma unroll
     for (int i = 0; i < kOwn; ++i) {  // (what does not exist is read where something else is, and not written)
-        const int c = min(cbase + ch0 + i * kChannelStep, O - 1);
-        const int64_t at = ((int64_t)b * O + c) * N + min(first + p, N - 1);
-        y[i] = extreme[at];
-        gv[i] = g[at];
-        place[i] = arg[at];
-        ss[i] = constants_of(norm, c);
-        a[i] = coef[c * 4];
+        if (cbase + i * kChannelStep < O) {  // uniform
+            const int c = min(cbase + ch0 + i * kChannelStep, O - 1);
+            const int64_t at = ((int64_t)b * O + c) * N + min(first + p, N - 1);
+            y[i] = extreme[at];
+            gv[i] = g[at];
+            place[i] = arg[at];
+            ss[i] = constants_of(norm, c);
+            a[i] = coef[c * 4];
+        }
     }
 #pragma unroll
     for (int i = 0; i < kOwn; ++i)
@@ -413,10 +416,11 @@ __global__ void __launch_bounds__(kBlock) edge_rows_kernel(const float *x, int C
     const int tid = threadIdx.x, first = blockIdx.x * kPoints, cbase = blockIdx.y * kChannels;
     const int64_t b = blockIdx.z;
     const int p = tid % kPoints, ch0 = tid / kPoints;
-    float v[kOwn];
+    float v[kOwn] = {};
 #pragma unroll
     for (int i = 0; i < kOwn; ++i)
-        v[i] = x[(b * C + min(cbase + ch0 + i * kChannelStep, C - 1)) * N + min(first + p, N - 1)];
+        if (cbase + i * kChannelStep < C)  // uniform
+            v[i] = x[(b * C + min(cbase + ch0 + i * kChannelStep, C - 1)) * N + min(first + p, N - 1)];
 #pragma unroll
     for (int i = 0; i < kOwn; ++i)
         tile[p][ch0 + i * kChannelStep] = v[i];
