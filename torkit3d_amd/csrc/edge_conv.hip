@@ -216,6 +216,19 @@ __device__ __forceinline__ int point_of(int entry, int N)
 // edge_rows_kernel took 6.2 us for 4.8 now (8 x 2048 points, 64 channels), edge_select_kernel 11.2 for 6.3 on those
 // sizes, which no longer come to it.
 constexpr int kChannelStep = kBlock / kPoints, kOwn = kChannels / kChannelStep;
+template <typename F> __device__ __forceinline__ void for_own_channels(int cbase, int channels, const F &load)
+{
+    if (cbase + kChannels <= channels) {  // uniform, as the others are: a whole tile's loads without them in between
+#pragma unroll
+        for (int i = 0; i < kOwn; ++i)
+            load(i);
+    } else {
+#pragma unroll
+        for (int i = 0; i < kOwn; ++i)
+            if (cbase + i * kChannelStep < channels)
+                load(i);
+    }
+}
 
 // The sparse gradient, [B, N, O] of (a e, place), from g, extreme and arg [B, O, N].
 __global__ void __launch_bounds__(kBlock)
@@ -229,18 +242,15 @@ __global__ void __launch_bounds__(kBlock)
     float y[kOwn] = {}, gv[kOwn] = {}, a[kOwn] = {};
     int place[kOwn] = {};
     f32x4 ss[kOwn] = {};
-#pragma unroll
-    for (int i = 0; i < kOwn; ++i) {  // (what does not exist is read where something else is, and not written)
-        if (cbase + i * kChannelStep < O) {  // uniform
-            const int c = min(cbase + ch0 + i * kChannelStep, O - 1);
-            const int64_t at = ((int64_t)b * O + c) * N + min(first + p, N - 1);
-            y[i] = extreme[at];
-            gv[i] = g[at];
-            place[i] = arg[at];
-            ss[i] = constants_of(norm, c);
-            a[i] = coef[c * 4];
-        }
-    }
+    for_own_channels(cbase, O, [&](int i) {  // (what does not exist is read where something else is, and not written)
+        const int c = min(cbase + ch0 + i * kChannelStep, O - 1);
+        const int64_t at = ((int64_t)b * O + c) * N + min(first + p, N - 1);
+        y[i] = extreme[at];
+        gv[i] = g[at];
+        place[i] = arg[at];
+        ss[i] = constants_of(norm, c);
+        a[i] = coef[c * 4];
+    });
 #pragma unroll
     for (int i = 0; i < kOwn; ++i)
         tile[p][ch0 + i * kChannelStep] =
@@ -417,10 +427,9 @@ __global__ void __launch_bounds__(kBlock) edge_rows_kernel(const float *x, int C
     const int64_t b = blockIdx.z;
     const int p = tid % kPoints, ch0 = tid / kPoints;
     float v[kOwn] = {};
-#pragma unroll
-    for (int i = 0; i < kOwn; ++i)
-        if (cbase + i * kChannelStep < C)  // uniform
-            v[i] = x[(b * C + min(cbase + ch0 + i * kChannelStep, C - 1)) * N + min(first + p, N - 1)];
+    for_own_channels(cbase, C, [&](int i) {
+        v[i] = x[(b * C + min(cbase + ch0 + i * kChannelStep, C - 1)) * N + min(first + p, N - 1)];
+    });
 #pragma unroll
     for (int i = 0; i < kOwn; ++i)
         tile[p][ch0 + i * kChannelStep] = v[i];
