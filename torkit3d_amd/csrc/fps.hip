@@ -513,9 +513,19 @@ constexpr int FPS_CLAIM_MAX = 1024;
 __device__ __forceinline__ int fps_max(int a, int b) { return a > b ? a : b; }
 __device__ __forceinline__ int fps_min(int a, int b) { return a < b ? a : b; }
 
-// The places of all cells of a 16^3 grid. (Worked out for every point they took 150 operations, 13 us of
+// The places of all cells of a 16^3 grid, by 256 x + 16 y + z. (Worked out for every point they took 150 operations, 13 us of
 // the 612 at 8 x 16384 -> 4096 and 3 of the 155 at 16 x 4096 -> 1024.)
-__device__ constexpr TkCurve fps_curve alignas(16) = tk_make_curve();
+struct FpsCurve {
+    unsigned short place[4096];
+};
+constexpr FpsCurve fps_make_curve()
+{
+    FpsCurve t{};
+    for (unsigned i = 0; i < 4096u; ++i)
+        t.place[i] = (unsigned short)tk_hilbert(i >> 8, (i >> 4) & 15u, i & 15u);
+    return t;
+}
+__device__ constexpr FpsCurve fps_curve alignas(16) = fps_make_curve();
 
 // Adds to a counter in LDS, lane by lane, and returns what it held before. (As an atomicAdd the
 // compiler turns it into a scan over the lanes, for a handful of which it is.)
@@ -695,9 +705,9 @@ __device__ __forceinline__ void fps_band(const float *__restrict__ pts, int64_t 
         s_red[wave][6] = odd ? -1.0f : far;
     }
     // (the table where the list comes later, if there is room)
-    constexpr bool NEAR = S * 4 >= (int)sizeof(TkCurve);
+    constexpr bool NEAR = S * 4 >= (int)sizeof(FpsCurve);
     if constexpr (NEAR)
-        for (int i = tid; i < (int)sizeof(TkCurve) / 16; i += NT)
+        for (int i = tid; i < (int)sizeof(FpsCurve) / 16; i += NT)
             reinterpret_cast<uint4 *>(fps_band_lds)[i] = reinterpret_cast<const uint4 *>(&fps_curve)[i];
     const unsigned short *const curve =
         NEAR ? reinterpret_cast<const unsigned short *>(fps_band_lds) : fps_curve.place;

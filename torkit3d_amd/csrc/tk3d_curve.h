@@ -25,15 +25,3 @@ constexpr unsigned tk_hilbert(unsigned x, unsigned y, unsigned z)
             place = 2u * place + (((c[a] ^ gray) >> b) & 1u);
     return place;
 }
-
-// The places of all cells, by 256 x + 16 y + z.
-struct TkCurve {
-    unsigned short place[4096];
-};
-constexpr TkCurve tk_make_curve()
-{
-    TkCurve t{};
-    for (unsigned i = 0; i < 4096u; ++i)
-        t.place[i] = (unsigned short)tk_hilbert(i >> 8, (i >> 4) & 15u, i & 15u);
-    return t;
-}
