@@ -515,7 +515,7 @@ __device__ __forceinline__ double knn_max_f64(double a, double b)
 // which a CU holds three workgroups (with boxes of 256 queries they took up to 1.13 times as long: 80 x 250 on 16384
 // in clusters k = 20 328, 291 without). us, every key swept and none put
 // to all queries, and now: 32 x 8192 queries on 2048 keys k = 3 63.5, 49.5, k = 8 83, 69, k = 16 122, 110, k = 32 262, 246; 8 x
-// 4096 on 16384 k = 3 214, 139, k = 16 251, 198; 8 x 4096 on 256 k = 3 15.4, 11.9, k = 16 28.2, 25.4; 200 x 120 on
+// 4096 on 16384 k = 3 214, 139, k = 16 251, 198; 8 x 4096 on 256 k = 3 15.3, 12.9, k = 16 28.2, 25.4; 200 x 120 on
 // 4096 k = 8 66, 60.
 enum { KNN_EVERY_KEY, KNN_BOXES, KNN_BOXES_UNLESS_ORDERED };  // (what is passed over)
 
