@@ -1333,12 +1333,13 @@ template <typename T> __device__ __forceinline__ T chamfer_root_grad(T g, T d, T
 }
 
 // Every range reads what it is sent anew, roots and distances as well, and points at random places from three planes:
-// where that takes longer than launches in front that copy the clouds to rows and form the gradients, these stay. Kernels
-// of a backward call in us, with launches in front and without: planes and roots 8 x 2500 x 3001 12.9, 11.6, 8 x 4096 x 4096
-// 14.6, 13.5, 32 x 8192 x 1024 16.0, 14.0, 8 x 8192 x 4096 16.1, 16.5, but 8 x 6000 x 5000 15.5, 17.3, 16 x 8192 x 8192 18.3,
-// 20.3; planes 32 x 2048 x 2048 12.7, 10.7, 32 x 5000 x 5000 16.3, 15.5, 8 x 6000 x 5000 14.5, 15.5, 16 x 8192 x 8192 16.8,
-// 17.8, 64 x 8192 x 8192 25.7, 23.6; roots 8 x 2500 x 3001 12.5, 10.2, 16 x 8192 x 8192 16.5, 16.2. Of the host's time go 4 to
-// 7 us. 32 x 16384 x 16384, planes and roots 30.1, 39.2, planes 29.8, 31.0.
+// where that takes longer than launches in front that copy the clouds to rows and form the gradients, these stay.
+// Kernels of a backward call in us, with launches in front and without: planes and roots 8 x 2500 x 3001 12.9, 11.6,
+// 8 x 4096 x 4096 14.6, 13.5, 32 x 8192 x 1024 16.0, 14.0, 8 x 8192 x 4096 16.1, 16.5, but 8 x 6000 x 5000 15.5,
+// 17.3, 16 x 8192 x 8192 18.3, 20.3; planes 32 x 2048 x 2048 12.7, 10.7, 32 x 5000 x 5000 16.3, 15.5, 8 x 6000 x 5000
+// 14.5, 15.5, 16 x 8192 x 8192 16.8, 17.8, 64 x 8192 x 8192 25.7, 23.6; roots 8 x 2500 x 3001 12.5, 10.2, 16 x 8192 x
+// 8192 16.5, 16.2. Of the host's time go 4 to 7 us. 32 x 16384 x 16384, planes and roots 30.1, 39.2, planes 29.8,
+// 31.0.
 constexpr int64_t CHAMFER_FORMS_POINTS = 8192, CHAMFER_BOTH_FORMS_POINTS = 4096;
 
 inline bool chamfer_takes_forms(bool planes, bool roots, int64_t N1, int64_t N2)
@@ -1451,9 +1452,9 @@ __global__ __launch_bounds__(NT) void chamfer_backward_fixed_kernel(
     // Sender u of a lane in round `round`: runs of NT consecutive senders, the rounds
     // interleaved so that each of them is spread over the whole cloud.
     auto sender = [&](int round, int u) { return tid + NT * (u * rounds + round); };
-    // Whether a run has senders at all (uniform). Not asked, a division and up to six loads for each of those that do not
-    // exist make roots slower here than behind launches in front (8 x 4096 x 4096, planes, 15.5 us, now 13.5); the
-    // loads alone are as fast without the question.
+    // Whether a run has senders at all (uniform). Not asked, a division and up to six loads for each of those that do
+    // not exist make roots slower here than behind launches in front (8 x 4096 x 4096, planes, 15.5 us, now 13.5);
+    // the loads alone are as fast without the question.
     auto run_exists = [&](int round, int u) { return !ROOT || NT * (u * rounds + round) < ny; };
     // A sender's match as a position within the range, -1 when it lies outside.
     auto load_matches = [&](int round, int (&jj)[U]) {

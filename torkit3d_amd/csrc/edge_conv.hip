@@ -313,12 +313,12 @@ __global__ void __launch_bounds__(kBlock)
 
 // The same from g, extreme and arg themselves: a workgroup has CH channels of a cloud, whose sums lie in LDS. kPart
 // points at a time, every lane finds the values of its points and the neighbours that they belong to; then one wave a
-// channel adds them, 64 points to an atomic. Lanes that meet at a neighbour are taken in their order, so that every run adds
-// in that of the points: the hardware's doing, which nothing here enforces and a test holds. The two kernels above look
-// at all K edges into a point for the few that count, 8 bytes a channel of each, and pass 8 bytes a value through
-// memory; here a value looks up its one neighbour. 8 x 2048 points, 20 neighbours, 64 channels: 26.4 us in two launches,
-// now 10.5, most of it the trips to g, to the neighbours and through LDS, one behind the other; 128 channels 40.8, 14.
-// A step of DGCNN's training on them 74 us less.
+// channel adds them, 64 points to an atomic. Lanes that meet at a neighbour are taken in their order, so that every
+// run adds in that of the points: the hardware's doing, which nothing here enforces and a test holds. The two kernels
+// above look at all K edges into a point for the few that count, 8 bytes a channel of each, and pass 8 bytes a value
+// through memory; here a value looks up its one neighbour. 8 x 2048 points, 20 neighbours, 64 channels: 26.4 us in
+// two launches, now 10.5, most of it the trips to g, to the neighbours and through LDS, one behind the other; 128
+// channels 40.8, 14. A step of DGCNN's training on them 74 us less.
 template <int CH>
 __global__ void __launch_bounds__(kOwners)
     edge_owners_kernel(const float *__restrict__ g, const float *__restrict__ extreme,
@@ -971,7 +971,8 @@ int tk3d_mlp_edge_backward_f32(const float *g, const float *extreme, const unsig
     const hipStream_t stream = (hipStream_t)stream_;
     const WeightRuns r = weight_runs(B, N, O, C);
     const int half = tiles_of(O) * kTile;
-    // the workspace: partial sums, sel [B, N, O] of 8 bytes if the sums may be gathered, duv [B, 2 O, N], rows [B, N, C], st [B, 2 C, N]
+    // the workspace: partial sums, sel [B, N, O] of 8 bytes if the sums may be gathered, duv [B, 2 O, N], rows [B, N,
+    // C], st [B, 2 C, N]
     double *partial = reinterpret_cast<double *>(workspace);
     int2 *sel = reinterpret_cast<int2 *>(partial + (int64_t)r.parts * 2 * half * C);
     float *duv = reinterpret_cast<float *>(sel + (may_gather(N) ? (int64_t)B * N * O : 0));

@@ -513,8 +513,8 @@ constexpr int FPS_CLAIM_MAX = 1024;
 __device__ __forceinline__ int fps_max(int a, int b) { return a > b ? a : b; }
 __device__ __forceinline__ int fps_min(int a, int b) { return a < b ? a : b; }
 
-// The places of all cells of a 16^3 grid, by 256 x + 16 y + z. (Worked out for every point they took 150 operations, 13 us of
-// the 612 at 8 x 16384 -> 4096 and 3 of the 155 at 16 x 4096 -> 1024.)
+// The places of all cells of a 16^3 grid, by 256 x + 16 y + z. (Worked out for every point they took 150 operations,
+// 13 us of the 612 at 8 x 16384 -> 4096 and 3 of the 155 at 16 x 4096 -> 1024.)
 struct FpsCurve {
     unsigned short place[4096];
 };

@@ -514,9 +514,9 @@ __device__ __forceinline__ double knn_max_f64(double a, double b)
 // the sort (up to 126 registers and 66 KB of LDS, 50 without boxes: four waves per SIMD); 32 slots run in 256, of
 // which a CU holds three workgroups (with boxes of 256 queries they took up to 1.13 times as long: 80 x 250 on 16384
 // in clusters k = 20 328, 291 without). us, every key swept and none put
-// to all queries, and now: 32 x 8192 queries on 2048 keys k = 3 63.5, 49.5, k = 8 83, 69, k = 16 122, 110, k = 32 262, 246; 8 x
-// 4096 on 16384 k = 3 214, 139, k = 16 251, 198; 8 x 4096 on 256 k = 3 15.3, 12.9, k = 16 28.2, 25.4; 200 x 120 on
-// 4096 k = 8 66, 60.
+// to all queries, and now: 32 x 8192 queries on 2048 keys k = 3 63.5, 49.5, k = 8 83, 69, k = 16 122, 110, k = 32
+// 262, 246; 8 x 4096 on 16384 k = 3 214, 139, k = 16 251, 198; 8 x 4096 on 256 k = 3 15.3, 12.9, k = 16 28.2, 25.4;
+// 200 x 120 on 4096 k = 8 66, 60.
 enum { KNN_EVERY_KEY, KNN_BOXES, KNN_BOXES_UNLESS_ORDERED };  // (what is passed over)
 
 constexpr int knn_max4(int a, int b, int c, int d)
@@ -1689,9 +1689,9 @@ __global__ __launch_bounds__(KNN_BLOCK, LONG ? 1 : 8) void knn_wave_kernel_f32(
     }
 }
 
-// Up to how many queries a wave per query wins: its time goes with their number, that of the kernels of a lane per query
-// hardly does while they leave CUs idle. Its time over that of the pre-filtered kernel, keys in random order and in that of a
-// coordinate, clouds of 512 to 4096 queries:
+// Up to how many queries a wave per query wins: its time goes with their number, that of the kernels of a lane per
+// query hardly does while they leave CUs idle. Its time over that of the pre-filtered kernel, keys in random order
+// and in that of a coordinate, clouds of 512 to 4096 queries:
 //   queries       keys    64         512        1024       2048       4096       8192       16384
 //   20480  k = 1       0.89 0.82  0.68 0.66  0.65 0.65  0.76 0.68  0.96 0.68  1.13 0.73  1.25 0.80
 //          k = 3       1.07 1.08  0.89 0.92  0.80 0.86  0.74 0.90  0.88 0.90  1.03 0.88  1.18 0.84
@@ -1705,9 +1705,9 @@ __global__ __launch_bounds__(KNN_BLOCK, LONG ? 1 : 8) void knn_wave_kernel_f32(
 //   32768  k = 1       1.25 1.13  0.95 0.93  0.94 0.91  1.15 0.97  1.48 1.00  1.79 1.07  1.99 1.23
 //          k = 20      1.20 1.24  1.16 0.99  1.16 1.00  1.06 0.99  0.97 0.97  0.89 0.94  0.93 0.90
 //          k = 32      1.17 1.19  1.22 1.06  1.26 1.06  1.17 1.03  1.06 1.03  0.98 0.99  0.89 0.95
-// (on 65536, 32768 queries in clouds of 128 k = 20 1.06 1.29). With more than 32 neighbours the others keep a tree in LDS: us, the
-// wave and the tree, 49152 queries on 128 keys k = 64 59, 72, on 4096 301, 549; 65536 on 1024 253, 243; 131072 on 128 k = 40 146,
-// 136, on 4096 k = 40 570, 985, k = 64 771, 1143.
+// (on 65536, 32768 queries in clouds of 128 k = 20 1.06 1.29). With more than 32 neighbours the others keep a tree in
+// LDS: us, the wave and the tree, 49152 queries on 128 keys k = 64 59, 72, on 4096 301, 549; 65536 on 1024 253, 243;
+// 131072 on 128 k = 40 146, 136, on 4096 k = 40 570, 985, k = 64 771, 1143.
 inline int64_t knn_wave_queries(int64_t keys, int64_t k)
 {
     if (k > 32)
@@ -1863,9 +1863,9 @@ int knn_filter_launch(const float *query, const float *key, float *distance, int
                       float *weight, float eps, int64_t B, int n1, int n2, int k, hipStream_t s,
                       bool whatever_the_size = false)
 {
-    // 512 lanes: two workgroups (16 waves) per CU. A launch of few such workgroups leaves CUs without one: 256 lanes then,
-    // unless there are keys enough for boxes. The times of the instances over that of the same kernel
-    // without boxes and without keys put to all queries (256 lanes up to 128 or 160 workgroups of 512, else 512):
+    // 512 lanes: two workgroups (16 waves) per CU. A launch of few such workgroups leaves CUs without one: 256 lanes
+    // then, unless there are keys enough for boxes. The times of the instances over that of the same kernel without
+    // boxes and without keys put to all queries (256 lanes up to 128 or 160 workgroups of 512, else 512):
     //   8 x 4096 queries, in launches of few     every key, 256 lanes   512   boxes, unless ordered
     //     2048 keys in random order k = 3                 0.90           0.94          0.91
     //     2048 k = 8                                      0.89           0.99          0.96
@@ -1876,9 +1876,9 @@ int knn_filter_launch(const float *query, const float *key, float *distance, int
     //     2048 k = 8                                      0.97           0.91          0.91 (in clusters 0.99, 0.92, 0.97)
     //   32 x 8192, two: 1024 k = 3                        1.04           0.87          0.87 (boxes; voxels in order 0.73)
     // Clouds of up to 256 queries have half of the 512 lanes to help with the staging, and one or two waves more to the
-    // boxes' one: 200 x 120 on 4096 k = 8 1.07, 0.94; 80 x 250 on 8192 k = 16 0.95, 0.86, boxes 0.95; from 16384 keys on
-    // boxes are even for k = 3, 0.89 and 0.83. 32 slots leave room for three waves per SIMD, twelve a CU: three workgroups of 256
-    // lanes or one of 512.
+    // boxes' one: 200 x 120 on 4096 k = 8 1.07, 0.94; 80 x 250 on 8192 k = 16 0.95, 0.86, boxes 0.95; from 16384 keys
+    // on boxes are even for k = 3, 0.89 and 0.83. 32 slots leave room for three waves per SIMD, twelve a CU: three
+    // workgroups of 256 lanes or one of 512.
     if (!(whatever_the_size || knn_filter_takes(B, n1, n2, k)))
         return TK3D_ERR_UNSUPPORTED;
     const auto as = [&](auto lanes, auto kind, bool halves = false) {

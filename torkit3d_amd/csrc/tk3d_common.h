@@ -164,8 +164,9 @@ __device__ __forceinline__ float tk_min_of_halves(float v)
 }
 
 // The maxima over the wave (LANES 64, left in lane 63), over each half of it (32, in lanes 31 and 63) or over the first
-// eight lanes (8, in lane 7) of six values at once: the steps of one value are the wait between those of another, and a maximum takes its operand from the
-// other lane itself. One by one, through moves, the compiler makes it five instructions a step.
+// eight lanes (8, in lane 7) of six values at once: the steps of one value are the wait between those of another, and
+// a maximum takes its operand from the other lane itself. One by one, through moves, the compiler makes it five
+// instructions a step.
 template <int LANES> __device__ __forceinline__ void tk_wave_max_six(float (&v)[6])
 {
 #define TK_STEP(HOW)                                                           \
